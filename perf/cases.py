@@ -7,7 +7,7 @@ on, and three of the other decoders at the same layer sizes, their layers as the
 feed-forwards all dense; between them they run every kind of kernel: full, windowed and latent attention, state-space,
 delta-rule, retention, gated linear and RWKV-style recurrences, dense feed-forwards and experts). They have few enough
 layers that two correct implementations' roundings, which random weights amplify from layer to layer, stay comparable:
-16 layers for the headline, 8 at the 3B sizes and for Morulix, 4 for the others. Weights are random, in bfloat16, the type the
+12 of the headline's 16, 8 at the 3B sizes and for Morulix, 4 for the others. Weights are random, in bfloat16, the type the
 engine serves in (float32 is there to show faults). A case's numbers:
 
     model                 one of MODELS
@@ -78,7 +78,7 @@ def _kufolorn() -> dict:
     return {"architecture": "Kufolorn", "vocab": VOCAB, "width": WIDTH, "norm": {"eps": 1e-6}, "logit_softcap": 20.0, "layers": [delta, pair] * 2}
 
 
-MODELS = {"llama-1b": _llama(16, 2048, 32, 64), "llama-3b": _llama(8, 3072, 24, 128), "morulix": _morulix(),
+MODELS = {"llama-1b": _llama(12, 2048, 32, 64), "llama-3b": _llama(8, 3072, 24, 128), "morulix": _morulix(),
           "tegolix": _tegolix(), "kufolorn": _kufolorn()}
 
 
@@ -263,7 +263,7 @@ def work(case: dict) -> dict:
 def tolerance(case: dict) -> dict:
     """Logits of one model with its products in another order (prompts in 25 portions beside 2, or whole) differ by 0.006 of
     their norm for Morulix, 0.009 for Kufolorn, 0.006 for Tegolix (0.02 where a token's scores lie so close that it takes
-    another expert) and 0.019 to 0.028 for Llama, whose stream is bfloat16: as much as each differs from the 64-bit model."""
+    another expert) and 0.018 to 0.025 for Llama, whose stream is bfloat16: as much as each differs from the 64-bit model."""
     return {"rel": 0.025 if case["model"] == "morulix" else 0.03, "max": 0.4}
 
 

@@ -572,6 +572,36 @@ def test_tiled_product(m, n, k):
         hip().gemm_tiled(ad[:, :k], wd[:n - 1])
 
 
+@pytest.mark.parametrize("form,limit,slope,shift", [("silu_rounded", 0.0, 1.0, 0.0), ("sigmoid", 0.0, 1.0, 0.0), ("sigmoid", 0.7, 1.702, 1.0),
+                                                    ("relu", 0.0, 1.0, 0.0), ("gelu_tanh", 0.0, 1.0, 0.0)])
+@pytest.mark.parametrize("m,f,k", [(1, 8, 64), (129, 136, 128), (257, 1032, 192), (300, 8200, 64), (999, 8192, 320), (1100, 8200, 128), (2048, 2056, 64)])
+def test_gated_product_of_many_rows(m, f, k, form, limit, slope, shift):
+    """One, two, three and more k-steps, tiles of each size that hang over the last rows and columns, several tiles a
+    workgroup, rows that lie apart. The bound: 2^-8 (half a step of bfloat16) for the stored result and, where branches are rounded first, for each
+    of them (silu' stays below 1.1), beside what 32-bit sums of k products can be off."""
+    g = gen(m + f + k)
+    a, w = torch.randn(m, 2 * k, generator=g).bfloat16(), (torch.randn(2 * f, k, generator=g) * (2.0 / math.sqrt(k))).bfloat16()
+    ad, wd = a.to(dev()), w.to(dev())
+    sums = ad[:, :k].double() @ wd.double().T
+    size = ad[:, :k].double().abs() @ wd.double().abs().T * (k * 2.0 ** -24)
+    (gate, up), (dg, du) = sums.split(f, dim=1), size.split(f, dim=1)
+    if form == "silu_rounded":
+        dg, du = dg + gate.abs() * 2.0 ** -8, du + up.abs() * 2.0 ** -8
+    if limit > 0:
+        gate, up = gate.clamp(max=limit), up.clamp(-limit, limit)
+    up = up + shift
+    act = {"relu": torch.relu, "gelu_tanh": lambda z: torch.nn.functional.gelu(z, approximate="tanh")}.get(form, lambda z: z * torch.sigmoid(slope * z))
+    want = act(gate) * up
+    bound = 1.2 * (dg * up.abs() + du * act(gate).abs()) + 1.2 * dg * du + want.abs() * (2.0 ** -7.9) + 1e-6
+    out = hip().gemm_glu(ad[:, :k], wd, form, limit, slope, shift)
+    assert out.dtype == torch.bfloat16 and out.shape == (m, f)
+    assert bool(((out.double() - want).abs() <= bound).all()), float(((out.double() - want).abs() / bound).max())
+    assert torch.equal(hip().gemm_glu(ad[:, :k].contiguous(), wd, form, limit, slope, shift), out)
+    for bad in (lambda: hip().gemm_glu(ad[:, :k - 8], wd[:, :k - 8], form), lambda: hip().gemm_glu(ad[:, :k], wd[:2 * f - 8], form)):
+        with pytest.raises(hip().KernelError, match="gated product takes"):
+            bad()
+
+
 @pytest.mark.parametrize("m", [1, 3, 8, 16, 17, 32])
 @pytest.mark.parametrize("n,k", [(3072, 2048), (2048, 2048), (16384, 2048), (2048, 8192), (992, 512), (130, 3072), (64, 4096),
                                  (8192, 3072), (8256, 4096)])

@@ -64,6 +64,7 @@ def _declare(lib: ctypes.CDLL) -> None:
         "ts_feed_tokens": [p, p, p, i, i, p],
         "ts_gemm_library_bf16": [p, p, p, i, i, i, i64, i64, i64, i, i, p, ctypes.c_size_t, p],
         "ts_gemm_tiled_bf16": [p, p, p, i, i, i, i64, i64, i64, i, i, p],
+        "ts_gemm_glu_bf16": [p, p, p, i, i, i, i64, i64, i64, i, f, f, f, p],
         "ts_gemm_library_init": [],
         "ts_gemm_library_timing": [i],
         "ts_gemm_library_choices": [p, i],
@@ -1415,8 +1416,8 @@ _many_rows = "library"
 
 def many_rows_products(which: str | None = None) -> str:
     """Which kernel serves bfloat16 products of many rows: "library" (the vendor's, the faster one
-    and the default) or "tiled" (this repository's LDS-tiled matrix-core kernel, for the shapes it
-    takes). Sets it if `which` is given; returns the setting. It holds for the process."""
+    and the default; products that end in a gated unit go to `gemm_glu`, which takes the unit along) or
+    "tiled" (this repository's LDS-tiled matrix-core kernel, for the shapes it takes). Sets it if `which` is given; returns the setting. It holds for the process."""
     global _many_rows
     if which is not None:
         _need(which in MANY_ROWS_PRODUCTS, lambda: f"products of many rows are one of {MANY_ROWS_PRODUCTS}, not {which!r}")
@@ -1451,6 +1452,36 @@ def gemm_tiled(x: torch.Tensor, weight: torch.Tensor, glu: bool = False,
         _run("gemm_tiled", library().ts_gemm_tiled_bf16(_ptr(y), _ptr(x), _ptr(weight), M, N, K, x.stride(0),
                                                         weight.stride(0), y.stride(0), int(glu),
                                                         int(out_dtype == torch.float32), _stream()))
+    return y
+
+
+GLU_FORMS = {"silu_rounded": 0, "sigmoid": 1, "relu": 2, "gelu_tanh": 3}
+
+
+def glu_takes(x: torch.Tensor, weight: torch.Tensor) -> bool:
+    """Whether `gemm_glu` serves these operands (see gemm_glu.hip for the conditions)."""
+    n, k = weight.shape
+    return (x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and k % 64 == 0 and n % 16 == 0 and x.stride(1) == 1
+            and weight.stride(1) == 1 and x.stride(0) % 8 == 0 and weight.stride(0) % 8 == 0 and x.stride(0) >= k and weight.stride(0) >= k
+            and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0
+            and 2 * n * weight.stride(0) < 1 << 31 and 512 * x.stride(0) < 1 << 31)
+
+
+def gemm_glu(x: torch.Tensor, weight: torch.Tensor, form: str, limit: float = 0.0, slope: float = 1.0, up_shift: float = 0.0) -> torch.Tensor:
+    """The gated unit of bfloat16 x [M, K] against a weight [2 F, K] of F gate rows, then F up rows, as bfloat16 [M, F], in
+    one kernel for many rows (gemm_glu.hip). `form` "silu_rounded": silu(gate) up of branches rounded to bfloat16 first
+    (what `silu_mul` makes of a bfloat16 product); "sigmoid", "relu", "gelu_tanh": `capped_glu` of the 32-bit sums."""
+    _gpu(x, weight)
+    _need(form in GLU_FORMS, lambda: f"form {form!r}: one of {sorted(GLU_FORMS)}")
+    _need(x.dim() == 2 and weight.dim() == 2 and x.shape[1] == weight.shape[1], lambda: f"shapes {tuple(x.shape)} x {tuple(weight.shape)}^T")
+    _need(glu_takes(x, weight), "the gated product takes bfloat16 operands with dense, 16-byte aligned rows, a reduction that is a "
+          "multiple of 64, a unit's width that is a multiple of 8 and a weight below 2 GB")
+    M, K = x.shape
+    F = weight.shape[0] // 2
+    y = torch.empty((M, F), dtype=torch.bfloat16, device=x.device)
+    if M and F:
+        _run("gemm_glu", library().ts_gemm_glu_bf16(_ptr(y), _ptr(x), _ptr(weight), M, F, K, x.stride(0), weight.stride(0), F,
+                                                    GLU_FORMS[form], float(limit), float(slope), float(up_shift), _stream()))
     return y
 
 
@@ -1498,6 +1529,16 @@ def _skinny_serves(rows: int, n: int, k: int) -> bool:
     streams the rest faster."""
     return (rows <= SKINNY_MAX_ROWS and skinny_takes(rows, k) and k <= 4096
             and (rows <= SKINNY_FUSED_ROWS or n * k <= SKINNY_WIDE_ELEMENTS))
+
+
+def many_rows(x: torch.Tensor, weight: torch.Tensor, packed: "StreamingCopies | None" = None) -> bool:
+    """Whether a plain 32-bit product of these operands goes to a kernel for many rows (by `many_rows_products`) and to none
+    of the weight-streaming ones."""
+    rows, (n, k) = x.shape[0], weight.shape
+    if not (_dense_rows(x) and weight.is_contiguous() and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0):
+        return True
+    return not (skinny8_takes(rows, n, k) or _skinny_serves(rows, n, k)
+                or (packed is not None and packed.by16 is not None and rows64_takes(rows, n, k)))
 
 
 def linear_bf16(x: torch.Tensor, weight: torch.Tensor, out_dtype: torch.dtype = torch.bfloat16,

@@ -154,6 +154,8 @@ def linear(x: "torch.Tensor | DeferredNorm | hip.PackedRows8 | hip.SplitAttentio
         if (out_dtype in (None, torch.bfloat16) and hip.many_rows_products() == "tiled" and x.is_cuda
                 and hip.tiled_takes(x, weight, glu=True)):
             return hip.gemm_tiled(x, weight, glu=True)
+        if out_dtype in (None, torch.bfloat16) and hip.many_rows_products() == "library" and x.is_cuda and hip.glu_takes(x, weight):
+            return hip.gemm_glu(x, weight, "silu_rounded")
         return hip.silu_mul(linear(x, weight, out_dtype, packed=packed))
     if x.dtype == torch.float32:
         return hip.gemm_exact(x, weight, out_dtype)

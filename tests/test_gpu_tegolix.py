@@ -82,7 +82,7 @@ def test_two_mixers_sum_with_their_factors_and_the_gated_table_rows():
 
 # ---- decays, the scan, the token shift ---------------------------------------------------------------------------------
 
-def scan_case(read_first: bool, H: int, D: int, V: int, counts_by_step, slots, tau=3.0, seed=0, far=None):
+def scan_case(read_first: bool, H: int, D: int, V: int, counts_by_step, slots, tau=3.0, seed=0, far=None, chunked=False):
     """Requests fed in unequal portions over several steps, each on its state slot; returns (kernel rows, oracle rows) per
     request. `far` = (request, position): that token's k and v are made large and the decays near 1, and every later
     query of the request is aligned with that k, so what it reads is what the state has kept of one token far back."""
@@ -117,7 +117,8 @@ def scan_case(read_first: bool, H: int, D: int, V: int, counts_by_step, slots, t
         K = H * D
         o = h.decay_scan(fused[:, :K], fused[:, K:2 * K], fused[:, 2 * K:], cat(z), bias.to(DEV), state, dev(cu), dev([slots[r] for r in live]),
                          H, D, V, form="double_exponent" if read_first else "sigmoid_root", tau=tau, q_scale=1.0 if read_first else D ** -0.5,
-                         bonus=None if bonus is None else bonus.to(DEV), longest=max(step))
+                         bonus=None if bonus is None else bonus.to(DEV), longest=max(step),
+                         ctx=step_context([[0]] * len(live), 4096, [0] * len(live), [step[r] for r in live], slots=[slots[r] for r in live]) if chunked else None)
         for i, r in enumerate(live):
             got[r].append(o[cu[i]:cu[i + 1]].cpu())
             fed[r] += step[r]
@@ -153,11 +154,26 @@ def test_decay_scan_over_unequal_requests_in_unequal_portions(read_first, sizes)
 
 
 @pytest.mark.parametrize("read_first", [False, True])
-def test_a_token_far_back_is_still_in_the_state(read_first):
-    """Position 3 of 700 stands out; the request is fed in portions and then token by token. A state that is dropped between
+@pytest.mark.parametrize("sizes", [(3, 32, 64), (2, 64, 128), (5, 64, 64), (2, 128, 64), (1, 128, 256), (2, 32, 320)])
+def test_long_portions_in_chunks(read_first, sizes):
+    """Portions from the shortest that is worked in chunks on, whole chunks and ragged ends (one token, a block's edge), beside
+    requests that are walked, states handed from chunks to walk and back. The bound: a number is a sum of at most
+    D + 64 products beside what the state's 32-bit numbers carry, each rounding good to 2^-24."""
+    H, D, V = sizes
+    least = hip().DECAY_CHUNKS_FROM
+    steps = [[least, 3, 0], [1, least + 129, least + 16], [least + 63, 1, least + 47], [70, 0, 2]]
+    got, want = scan_case(read_first, H, D, V, steps, slots=[2, 0, 3], seed=D + V, chunked=True)
+    for g, w in zip(got, want):
+        torch.testing.assert_close(g.to(F64), w, atol=(D + 64) * 2.0 ** -24 * float(w.abs().max()), rtol=1e-5)
+
+
+@pytest.mark.parametrize("chunked", [False, True])
+@pytest.mark.parametrize("read_first", [False, True])
+def test_a_token_far_back_is_still_in_the_state(read_first, chunked):
+    """Position 3 of 700 (or 2,400) stands out; the request is fed in portions and then token by token. A state that is dropped between
     steps, decayed in the wrong order, or read from the wrong slot loses it."""
-    steps = [[300], [64], [2], [200]] + [[1]] * 134
-    got, want = scan_case(read_first, 2, 32, 48, steps, slots=[1], far=(0, 3), seed=5)
+    steps = [[1300 if chunked else 300], [64], [2], [900 if chunked else 200]] + [[1]] * 134
+    got, want = scan_case(read_first, 2, 32, 64 if chunked else 48, steps, slots=[1], far=(0, 3), seed=5, chunked=chunked)
     assert float(want[0][-1].abs().max()) > 50 * float(want[0][2].abs().max()), "the far token dominates the last read-out"
     torch.testing.assert_close(got[0].to(F64), want[0], atol=3e-4 * float(want[0].abs().max()), rtol=2e-4)
 

@@ -35,7 +35,7 @@ decay_scan_kernel(float* __restrict__ out, const float* __restrict__ q, int64_t 
                   int64_t w_stride, const float* __restrict__ bonus,
                   float* __restrict__ state, int64_t state_stride, const int32_t* __restrict__ cu_seqlens,
                   const int32_t* __restrict__ state_slots, int heads, int dim, int vdim,
-                  float q_scale, int block_tokens) {
+                  float q_scale, int at_most, int block_tokens) {
   extern __shared__ float lds[];
   constexpr int GROUPS = TS_WAVE / WC;
   const int threads = blockDim.x, waves = threads / TS_WAVE;
@@ -47,7 +47,7 @@ decay_scan_kernel(float* __restrict__ out, const float* __restrict__ q, int64_t 
   const int col = wave * WC + (lane % WC), grp = lane / WC;
   const bool live = v0 + col < vdim;
   const int t_begin = cu_seqlens[seq], t_end = cu_seqlens[seq + 1];
-  if (t_begin >= t_end) return;
+  if (t_begin >= t_end || t_end - t_begin > at_most) return;
   float* st = state + (int64_t)state_slots[seq] * state_stride + (int64_t)h * dim * vdim;
   float S[R4 * 4], U[READ_FIRST ? R4 * 4 : 1];
 #pragma unroll
@@ -151,7 +151,7 @@ decay_scan_pieces_kernel(float* __restrict__ out, const float* __restrict__ q, i
                          int64_t k_stride, const float* __restrict__ v, int64_t v_stride, const float* __restrict__ w,
                          int64_t w_stride, const float* __restrict__ bonus, float* __restrict__ state, int64_t state_stride,
                          const int32_t* __restrict__ cu_seqlens, const int32_t* __restrict__ state_slots, int heads, int dim,
-                         int vdim, float q_scale) {
+                         int vdim, float q_scale, int at_most) {
   extern __shared__ float lds[];
   constexpr int WC = WIDE ? TS_WAVE : TS_WAVE / GROUPS;     // columns of a wave
   constexpr int VG = WIDE ? GROUPS : 1;                     // shares of a column that a lane keeps
@@ -167,7 +167,7 @@ decay_scan_pieces_kernel(float* __restrict__ out, const float* __restrict__ q, i
   const int col = wave * WC + (lane % WC), grp = WIDE ? 0 : lane / WC;
   const bool live = v0 + col < vdim;
   const int t_begin = cu_seqlens[seq], t_end = cu_seqlens[seq + 1];
-  if (t_begin >= t_end) return;
+  if (t_begin >= t_end || t_end - t_begin > at_most) return;
   float* st = state + (int64_t)state_slots[seq] * state_stride + (int64_t)h * dim * vdim;
   float S[RG * VG * 4];
 #pragma unroll
@@ -333,11 +333,12 @@ static int ds_block_tokens(int threads, int in_size) {
 }
 
 // `wide`: a wave owns 64 columns instead of 16 (steps of few tokens a request: the state's rows are read and written
-// whole cache lines at a time, and nothing is exchanged between lanes); the result is the same bit for bit.
+// whole cache lines at a time, and nothing is exchanged between lanes); the result is the same bit for bit. Requests that feed
+// more than `at_most` tokens are left as they are (decay_chunks.hip has them).
 extern "C" int ts_decay_scan(float* out, const float* q, int64_t q_stride, const float* k, int64_t k_stride, const float* v,
                              int64_t v_stride, const float* w, int64_t w_stride, const float* bonus, float* state,
                              int64_t state_stride, const int32_t* cu_seqlens, const int32_t* state_slots, int num_seqs, int heads,
-                             int dim, int vdim, float q_scale, int read_first, int waves, int wide, hipStream_t stream) {
+                             int dim, int vdim, float q_scale, int read_first, int waves, int wide, int at_most, hipStream_t stream) {
   if (num_seqs <= 0) return TS_OK;
   if (heads <= 0 || heads > 65535 || dim <= 0 || dim > 1024 || vdim <= 0 || waves < 1 || waves > 4 || (read_first && !bonus) ||
       state_stride < (int64_t)heads * dim * vdim)
@@ -358,7 +359,7 @@ extern "C" int ts_decay_scan(float* out, const float* q, int64_t q_stride, const
     const int in_size = 3 * rg * groups * 4 + cols;
     dim3 grid(num_seqs, heads, slices);
 #define DS_FARGS out, q, q_stride, k, k_stride, v, v_stride, w, w_stride, bonus, state, state_stride, cu_seqlens, state_slots, heads, dim, \
-                 vdim, q_scale
+                 vdim, q_scale, at_most
 #define DS_FAST3(G, WD, RG, RF, NP, TB) \
     decay_scan_pieces_kernel<G, WD, RG, RF, NP, TB><<<grid, threads, (size_t)(2 * TB * in_size + rg * groups * 4) * sizeof(float), stream>>>(DS_FARGS)
 #define DS_FAST2(G, WD, RG, NP, TB) \
@@ -402,7 +403,7 @@ extern "C" int ts_decay_scan(float* out, const float* q, int64_t q_stride, const
   dim3 grid(num_seqs, heads, slices);
   const size_t lds = (size_t)2 * block_tokens * in_size * sizeof(float);
 #define DS_ARGS out, q, q_stride, k, k_stride, v, v_stride, w, w_stride, bonus, state, state_stride, cu_seqlens, state_slots, \
-                heads, dim, vdim, q_scale, block_tokens
+                heads, dim, vdim, q_scale, at_most, block_tokens
 #define DS_LAUNCH(WC, R4) \
   if (read_first) decay_scan_kernel<WC, R4, true><<<grid, waves * TS_WAVE, lds, stream>>>(DS_ARGS); \
   else decay_scan_kernel<WC, R4, false><<<grid, waves * TS_WAVE, lds, stream>>>(DS_ARGS)

@@ -122,7 +122,8 @@ def _declare(lib: ctypes.CDLL) -> None:
         "ts_mlstm_scan_chunks": [p, p, i64, p, p, p, p, p, p, p, p, p, i, i, i, i, i, f, f, p],
         "ts_mlstm_finish": [p, i, p, p, p, i64, i, i, i, f, i, i, p],
         "ts_moe_combine": [p, p, p, p, i, i, i, p, i, p, i, p, p],
-        "ts_decay_scan": [p, p, i64, p, i64, p, i64, p, i64, p, p, i64, p, p, i, i, i, i, f, i, i, i, p],
+        "ts_decay_scan": [p, p, i64, p, i64, p, i64, p, i64, p, p, i64, p, p, i, i, i, i, f, i, i, i, i, p],
+        "ts_decay_chunks": [p, p, i64, p, i64, p, i64, p, i64, p, p, p, i64, p, p, p, p, p, p, i, i, i, i, i, f, i, f, p],
         "ts_decay_factors": [p, p, i64, p, i, i, i, f, p],
         "ts_token_shift": [p, p, i, p, p, i64, p, p, p, i, i, i, p],
         "ts_token_shift_keep": [p, i64, p, i, p, p, i, i, p],
@@ -2521,12 +2522,18 @@ def mlstm_finish(o: torch.Tensor, weight: torch.Tensor | None, gate: torch.Tenso
 DECAY_FORMS = {"sigmoid_root": 0, "double_exponent": 1}
 DECAY_MAX_DIM = 1024
 DECAY_FULL_WORKGROUPS = 512      # workgroups of four waves from which a step keeps them (fewer: one wave each, four times as many)
+# Tokens of a request from which its portion is worked in chunks of 64. The walk takes 0.15 us a token and head group (32 heads of
+# 64 channels: 115 us for 512 tokens, 440 for 2,048; in chunks 30 and 68; 8 heads of 128 by 256 120 and 450 against 81 and 102), so
+# chunks are the faster from 128 (64 channels) or 320 tokens (128) on; short portions still walk, whose rows are the same bits
+# however a request's tokens are cut into steps.
+DECAY_CHUNKS_FROM = 768
+DECAY_CHUNK_DIMS = (32, 64, 128)
 DECAY_WIDE_UP_TO = 4             # tokens of a step's longest portion up to which a wave owns 64 value columns instead of 16
 
 
 def decay_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, z: torch.Tensor, z_bias: torch.Tensor, state: torch.Tensor,
                cu_seqlens: torch.Tensor, state_slots: torch.Tensor, heads: int, dim: int, vdim: int, *, form: str, tau: float = 1.0,
-               q_scale: float = 1.0, bonus: torch.Tensor | None = None, longest: int | None = None) -> torch.Tensor:
+               q_scale: float = 1.0, bonus: torch.Tensor | None = None, longest: int | None = None, ctx=None) -> torch.Tensor:
     """Linear attention with a decay per key channel over a packed step. q, k, z float32 [tokens, heads dim] and v
     float32 [tokens, heads vdim] are views whose rows may lie apart (columns of fused projections); z_bias float32
     [heads dim]. The decays are w = sigmoid(z + z_bias)^(1 / tau) (`form` "sigmoid_root") or exp(-exp(z + z_bias))
@@ -2534,7 +2541,10 @@ def decay_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, z: torch.Tenso
     o = (S + diag(bonus) k v^T)^T q first, then the same update. `state` float32 [slots, >= heads dim vdim]: each
     request's S lies at the start of its slot's row, is read there and written back. Returns o float32 [tokens, heads vdim].
     `longest`: the most tokens any request feeds in the step (None: unknown); steps of few tokens a request are cut into
-    fewer, wider slices of the value columns (the result is the same bit for bit)."""
+    fewer, wider slices of the value columns (the result is the same bit for bit). With `ctx` (the packed step's context, whose
+    requests these are) requests that feed at least `DECAY_CHUNKS_FROM` tokens are worked in chunks on the matrix cores where
+    the sizes allow it (`decay_chunks_take`): the same 32-bit sums in another order, so a request's rows then depend on how
+    its tokens are cut into steps."""
     _gpu(q, k, v, z, z_bias, state, cu_seqlens, state_slots, bonus)
     T = q.shape[0]
     _need(form in DECAY_FORMS, lambda: f"form {form!r}: one of {sorted(DECAY_FORMS)}")
@@ -2549,6 +2559,23 @@ def decay_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, z: torch.Tenso
     _need(cu_seqlens.dtype == torch.int32 and cu_seqlens.shape == (S + 1,) and state_slots.dtype == torch.int32, "cu_seqlens int32 [requests + 1], slots int32 [requests]")
     _need(0 < dim <= DECAY_MAX_DIM and tau > 0, lambda: f"heads of up to {DECAY_MAX_DIM} dimensions, a positive tau")
     out = torch.empty((T, heads * vdim), dtype=torch.float32, device=q.device)
+    at_most = 0x7fffffff
+    if ctx is not None and ctx.max_query_len >= DECAY_CHUNKS_FROM and decay_chunks_take(dim, vdim, state, bonus, (q, k, v, z)):
+        _check_step_requests(ctx)
+        _need(ctx.num_tokens == T and ctx.num_seqs == S, "the rows are the step's")
+        chunks, chunk_cu = _step_chunks(ctx, DECAY_CHUNKS_FROM, q.device)
+        C = chunks.shape[0]
+        buf = torch.empty((C, heads * dim * vdim), dtype=torch.float32, device=q.device)
+        totals = torch.empty((C, heads * dim), dtype=torch.float32, device=q.device)
+        logs = torch.empty((T, heads * dim), dtype=torch.float32, device=q.device)
+        _run("decay_chunks", library().ts_decay_chunks(
+            _ptr(out), _ptr(q), q.stride(0), _ptr(k), k.stride(0), _ptr(v), v.stride(0), _ptr(z), z.stride(0), _ptr(z_bias), _ptr(bonus), _ptr(state),
+            state.stride(0), _ptr(chunks), _ptr(chunk_cu), _ptr(state_slots), _ptr(buf), _ptr(totals), _ptr(logs), C, S, heads, dim, vdim, float(q_scale),
+            DECAY_FORMS[form], float(tau), _stream()))
+        if _all_in_chunks(ctx, DECAY_CHUNKS_FROM):
+            return out
+        at_most = DECAY_CHUNKS_FROM - 1
+        longest = max(n for n in (b - a for a, b in zip(ctx.host_cu_seqlens, ctx.host_cu_seqlens[1:])) if n <= at_most)
     w = torch.empty((T, heads * dim), dtype=torch.float32, device=q.device)
     _run("decay_factors", library().ts_decay_factors(_ptr(w), _ptr(z), z.stride(0), _ptr(z_bias), T, heads * dim, DECAY_FORMS[form], float(tau), _stream()))
     wide = longest is not None and longest <= DECAY_WIDE_UP_TO and vdim >= 64
@@ -2559,8 +2586,14 @@ def decay_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, z: torch.Tenso
     _run("decay_scan", library().ts_decay_scan(
         _ptr(out), _ptr(q), q.stride(0), _ptr(k), k.stride(0), _ptr(v), v.stride(0), _ptr(w), w.stride(0), _ptr(bonus),
         _ptr(state), state.stride(0), _ptr(cu_seqlens), _ptr(state_slots), S, heads, dim, vdim, float(q_scale), int(bonus is not None),
-        waves, int(wide), _stream()))
+        waves, int(wide), at_most, _stream()))
     return out
+
+
+def decay_chunks_take(dim: int, vdim: int, state: torch.Tensor, bonus: torch.Tensor | None, rows: "tuple[torch.Tensor, ...]") -> bool:
+    """Whether long portions of heads of these sizes, with q, k, v and z as `rows`, may be worked in chunks (decay_chunks.hip)."""
+    return (dim in DECAY_CHUNK_DIMS and vdim % 64 == 0 and vdim <= 65536 and state.stride(0) % 4 == 0 and state.data_ptr() % 16 == 0
+            and (bonus is None or bonus.data_ptr() % 16 == 0) and all(max(t.stride(0), t.shape[1]) <= 1 << 23 for t in rows))
 
 
 def token_shift(h: torch.Tensor, mu: torch.Tensor, kept: torch.Tensor, ctx) -> torch.Tensor:

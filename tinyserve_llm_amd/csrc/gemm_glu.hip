@@ -20,24 +20,7 @@
 // turn and fetches the next tile's first steps before it writes out the present one. The gate rows of a wave's columns
 // and their up rows lie side by side in the tile, so that a gate and its up meet in one lane; two lanes exchange halves so
 // that every store is 16 bytes (8-byte stores: 45 µs against 24 for the same product with K = 128).
-#include "attention_mfma.h"
-
-typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(3))) void* lds_ptr_t;
-
-static __device__ __forceinline__ float4_t mfma32v(u32x4_t a, u32x4_t b, float4_t acc) {
-  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), acc, 0, 0, 0);
-}
-
-// 1 KB from memory straight into LDS: lane l's 16 bytes at voffset + soffset land at lds + 16 l
-static __device__ __forceinline__ void load_to_lds(__amdgpu_buffer_rsrc_t rsrc, uint32_t lds, uint32_t voffset, uint32_t soffset) {
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_ptr_t)(uintptr_t)lds, 16, (int)voffset, (int)soffset, 0, 0);
-}
-
-// Waits until at most VM loads and LGKM reads of this wave are under way (vmcnt in bits 3:0 and 15:14, lgkmcnt in 11:8).
-template <int VM, int LGKM = 15> static __device__ __forceinline__ void wait_for() {
-  __builtin_amdgcn_s_waitcnt((VM & 15) | ((VM >> 4) << 14) | (7 << 4) | (LGKM << 8));
-}
+#include "lds_loads.h"
 
 // How a gate goes into the unit: as `silu_mul` of a bfloat16 product and `capped_glu` of 32-bit sums do it, so that the stored
 // units are the same (the hardware's 2^x and reciprocal throughout would take 10 of 130 µs off the sigmoid form).
@@ -91,7 +74,7 @@ __global__ __launch_bounds__(WM * WN * TS_WAVE, 2) void gemm_glu_kernel(const Gl
   __amdgpu_buffer_rsrc_t rsrc_x, rsrc_w;
   auto aim_x = [&](int turn) {
     const int m0 = (die * a.per_die + turn) % a.row_tiles * BM;
-    rsrc_x = __builtin_amdgcn_make_buffer_rsrc((void*)(a.x + (int64_t)m0 * a.ldx), 0, 0x7fffffff, 0x20000);
+    rsrc_x = load_base(a.x + (int64_t)m0 * a.ldx);
 #pragma unroll
     for (int q = 0; q < NX; ++q) {
       const int at = (wave * NX + q) * 8 + lane / 8;
@@ -100,7 +83,7 @@ __global__ __launch_bounds__(WM * WN * TS_WAVE, 2) void gemm_glu_kernel(const Gl
   };
   auto aim_w = [&](int turn) {
     const int c0 = (die * a.per_die + turn) / a.row_tiles * (BN / 2);
-    rsrc_w = __builtin_amdgcn_make_buffer_rsrc((void*)(a.w + (int64_t)c0 * a.ldw), 0, 0x7fffffff, 0x20000);
+    rsrc_w = load_base(a.w + (int64_t)c0 * a.ldw);
 #pragma unroll
     for (int q = 0; q < NW; ++q) {
       const int at = (wave * NW + q) * 8 + lane / 8, in = at % (2 * HALF);

@@ -16,7 +16,7 @@
 // Queries arrive 32-bit and are rounded to bfloat16 once, as the keys were. Scores, maxima, weights and sums are
 // 32-bit. Causal, with a sliding window or chunks (`ts_first_key`). Optionally a learned sink per head in the softmax's
 // denominator and a gate per head (sigmoid) on the result.
-#include "attention_mfma.h"
+#include "lds_loads.h"
 
 #define LM_WAVES 4
 #define LM_THREADS (LM_WAVES * TS_WAVE)
@@ -339,6 +339,202 @@ extern "C" int ts_paged_attention_latent_mfma(void* out, int out_dtype, const fl
   return ts_check_launch();
 }
 
+// ---- steps of many tokens ---------------------------------------------------------------------------------------
+// The same for steps that fill the chip with tiles of 128 rows (four tokens of 32 heads): a workgroup of eight waves, a wave
+// 16 rows with their queries and whole outputs in registers, and every 32-key step's keys and values shared by all of them
+// through LDS, where they go straight from memory, three steps in turn (one worked on, two under way). What bounds it: the
+// matrix cores, 48 products a wave and step of 256 numbers (16 for the scores, 32 for the weights' two bfloat16 terms),
+// beside the wave's softmax; the kernel above reads every token's keys from the second-level cache anew (2 GB for 2,048
+// tokens over 256 numbers: 577 us, this one 122). The reference maximum of a row is raised only where a score
+// exceeds it by 2^8, so that outputs are rarely rescaled. In LDS a key's 16-byte pieces are turned by the key's place among
+// the 16 that an operand takes, a value column's four by half the column's number: an operand's read then meets every bank once.
+#define LP_WAVES 8
+#define LP_ROWS (16 * LP_WAVES)
+#define LP_RING 3
+
+// CP: 32-wide pieces of a cached row, VB: 16-wide blocks of value columns, both rounded up to what is built.
+template <int CP, int VB, typename TO>
+__global__ void __launch_bounds__(LP_WAVES * TS_WAVE, 2)
+latent_attention_tiles_kernel(TO* __restrict__ out, const float* __restrict__ q, const bf16_t* __restrict__ k_cache,
+                              const bf16_t* __restrict__ v_cache, const int32_t* __restrict__ block_tables,
+                              const int32_t* __restrict__ seq_of_token, const int32_t* __restrict__ positions,
+                              const int32_t* __restrict__ tiles, int num_tiles, int heads_block, int nh, int rank, int row,
+                              int64_t kp, int64_t ks, int64_t vp, int64_t vd, int max_blocks, float scale_log2, int window,
+                              int page_run, const float* __restrict__ sinks, const float* __restrict__ gate, int64_t gate_token) {
+  constexpr int SL = (4 * CP + 15) / 16 * 16;               // 16-byte places of a key in LDS
+  constexpr int KBYTES = 32 * SL * 16, STEP = KBYTES + VB * 1024;
+  constexpr int NK = KBYTES / 1024 / LP_WAVES, NV = VB / LP_WAVES;       // kilobytes of a step that a wave fetches
+  static_assert(VB % LP_WAVES == 0 && KBYTES % (1024 * LP_WAVES) == 0, "whole kilobytes a wave");
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[LP_RING * STEP];
+  const int tile = num_tiles - 1 - blockIdx.x;              // (the list ascends by the keys to walk: the longest first)
+  const int t0 = tiles[2 * tile], count = tiles[2 * tile + 1], hb = blockIdx.y;
+  const int heads_here = min(nh - heads_block * hb, heads_block);
+  const int wave = wave_index(), lane = threadIdx.x & (TS_WAVE - 1), r = lane & 15, g = lane >> 4;
+  // this lane's row of the tile: token t0 + i / heads_here, head heads_block hb + i % heads_here
+  const int i_row = 16 * wave + r, tok = i_row / heads_here, head = heads_block * hb + i_row % heads_here;
+  const bool valid = tok < count;
+  const int pos0 = positions[t0], pos_max = pos0 + count - 1;
+  const int my_pos = valid ? pos0 + tok : pos_max, my_lo = ts_first_key(my_pos, window);
+  const int32_t* table = block_tables + (int64_t)seq_of_token[t0] * max_blocks;
+  const int kb0 = ts_first_key(pos0, window) & ~31, steps = ((pos_max - kb0) >> 5) + 1;
+  const int all_from = ts_first_key(pos_max, window);       // keys from here up to pos0 are seen by every row
+  auto page_of = [&](int step) -> int64_t {                  // a step lies inside one page of the pool (pages of 32 keys)
+    const int pg = (kb0 >> 5) + min(step, steps - 1);
+    return ((int64_t)table[pg >> page_run] << page_run) + (pg & ((1 << page_run) - 1));
+  };
+  // ---- the loading side ----
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_ptr_t)lds;
+  uint32_t koff[NK], voff[NV];
+#pragma unroll
+  for (int n = 0; n < NK; ++n) {
+    const int place = (wave * NK + n) * 64 + lane, key = place / SL, kr = 4 * (key >> 3) + (key & 3);
+    koff[n] = (uint32_t)(key * ks * 2) + min(8 * ((place % SL) ^ kr), row - 8) * 2;      // (past the row's end: zeros of the queries)
+  }
+#pragma unroll
+  for (int n = 0; n < NV; ++n) {
+    const int d = (wave * NV + n) * 16 + lane / 4;
+    voff[n] = (uint32_t)(min(d, rank - 1) * vd * 2) + ((lane % 4) ^ ((d >> 1) & 3)) * 16;
+  }
+  auto fetch = [&](int slot, int64_t page) {
+    const __amdgpu_buffer_rsrc_t kb = load_base(k_cache + page * kp), vb = load_base(v_cache + page * vp);
+    const uint32_t at = lds0 + slot * STEP;
+#pragma unroll
+    for (int n = 0; n < NK; ++n) load_to_lds(kb, at + (wave * NK + n) * 1024, koff[n], 0);
+#pragma unroll
+    for (int n = 0; n < NV; ++n) load_to_lds(vb, at + KBYTES + (wave * NV + n) * 1024, voff[n], 0);
+  };
+  fetch(0, page_of(0));
+  fetch(1, page_of(1));
+  int64_t page_next = page_of(2);
+  // the wave's queries, rounded once, zeros where there is no row or no dimension
+  u32x4_t qf[CP];
+  {
+    const float* src = q + ((int64_t)(t0 + (valid ? tok : 0)) * nh + (valid ? head : heads_block * hb)) * row;
+#pragma unroll
+    for (int c = 0; c < CP; ++c) {
+      const int d = 32 * c + 8 * g;
+      const float4 a = *(const float4*)(src + min(d, row - 8)), b = *(const float4*)(src + min(d, row - 8) + 4);
+      const bool in = valid && d < row;
+      qf[c] = in ? (u32x4_t){pack_bf16(a.x, a.y), pack_bf16(a.z, a.w), pack_bf16(b.x, b.y), pack_bf16(b.z, b.w)} : (u32x4_t){0, 0, 0, 0};
+    }
+  }
+  // ---- the multiplying side ----
+  uint32_t kat[4];                                          // this lane's place in a step for the pieces c, c + 4, ...
+#pragma unroll
+  for (int c = 0; c < 4; ++c) kat[c] = (uint32_t)((8 * (r >> 2) + (r & 3)) * SL * 16 + (((4 * c + g) ^ r) & 15) * 16);
+  const uint32_t vat = KBYTES + r * 64 + ((g ^ (r >> 1)) & 3) * 16;
+  float4_t acc[VB];
+#pragma unroll
+  for (int i = 0; i < VB; ++i) acc[i] = (float4_t){0.f, 0.f, 0.f, 0.f};
+  float m = -INFINITY, l = 0.f;
+  int slot = 0;
+  for (int step = 0; step < steps; ++step) {
+    // this step has landed (the next one's loads may be under way) and every wave is done with the step before
+    wait_for<NK + NV, 0>();
+    __builtin_amdgcn_s_barrier();
+    {
+      const int into = slot == 0 ? LP_RING - 1 : slot - 1;
+      fetch(into, page_next);
+      page_next = page_of(step + 3);
+    }
+    const unsigned char* at = lds + slot * STEP;
+    slot = slot + 1 == LP_RING ? 0 : slot + 1;
+    const int kb = kb0 + 32 * step;
+    float4_t st[2] = {(float4_t){0.f, 0.f, 0.f, 0.f}, (float4_t){0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+    for (int c = 0; c < CP; ++c)
+#pragma unroll
+      for (int tau = 0; tau < 2; ++tau)
+        st[tau] = mfma32v(*(const u32x4_t*)(at + kat[c & 3] + (c >> 2) * 256 + tau * (4 * SL * 16)), qf[c], st[tau]);
+    float s[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) s[j] = st[j >> 2][j & 3] * scale_log2;
+    if (kb < all_from || kb + 31 > pos0) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const int key = kb + 8 * g + j;
+        if (key < my_lo || key > my_pos) s[j] = -INFINITY;
+      }
+    }
+    float top = fmaxf(fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3])), fmaxf(fmaxf(s[4], s[5]), fmaxf(s[6], s[7])));
+    if (__any(top > m + 8.f)) {                              // (m = -inf: any key at all)
+      top = row_max(top);
+      const float m_new = top > m + 8.f ? top : m;
+      const float alpha = m_new == m ? 1.f : fast_exp2(m - m_new);
+      m = m_new;
+      l *= alpha;
+#pragma unroll
+      for (int i = 0; i < VB; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[i][j] *= alpha;
+    }
+    const float m_safe = m == -INFINITY ? 0.f : m;
+    u32x4_t hi, lo;
+    float sum = 0.f;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const float p0 = fast_exp2(s[2 * j] - m_safe), p1 = fast_exp2(s[2 * j + 1] - m_safe);
+      sum += p0 + p1;
+      hi[j] = pack_bf16(p0, p1);
+      lo[j] = pack_bf16(p0 - __uint_as_float(hi[j] << 16), p1 - __uint_as_float(hi[j] & 0xffff0000u));
+    }
+    l += sum;
+#pragma unroll
+    for (int i = 0; i < VB; ++i) {
+      const u32x4_t vf = *(const u32x4_t*)(at + vat + i * 1024);
+      acc[i] = mfma32v(vf, hi, acc[i]);
+      acc[i] = mfma32v(vf, lo, acc[i]);
+    }
+  }
+  wait_for<0>();                                            // (the steps fetched beyond the last land before the LDS is another's)
+  const float total = row_sum(l);                           // (every lane takes part, whatever its row)
+  if (!valid) return;
+  const float inv = lm_scale(m, total, sinks, head) * lm_gate(gate, (int64_t)(t0 + tok) * gate_token + head);
+  TO* dst = out + ((int64_t)(t0 + tok) * nh + head) * rank + 4 * g;
+#pragma unroll
+  for (int i = 0; i < VB; ++i)
+    if (16 * i < rank) {
+      if constexpr (sizeof(TO) == 4) *(float4_t*)(dst + 16 * i) = acc[i] * inv;
+      else *(uint2*)(dst + 16 * i) = make_uint2(pack_bf16(acc[i][0] * inv, acc[i][1] * inv), pack_bf16(acc[i][2] * inv, acc[i][3] * inv));
+    }
+}
+
+// Whether the kernel for steps of many tokens is built for these rows.
+extern "C" int ts_latent_tiles_takes(int rank, int row) { return ts_latent_mfma_takes(rank, row) && rank <= 256 && row <= 384; }
+
+// tiles as above, of at most LP_ROWS / min(heads, LP_ROWS) tokens.
+extern "C" int ts_paged_attention_latent_tiles(void* out, int out_dtype, const float* q, const void* k_cache, const void* v_cache,
+                                               const int32_t* block_tables, const int32_t* seq_of_token, const int32_t* positions,
+                                               const int32_t* tiles, int num_tiles, int tile_tokens, int num_tokens, int nh, int rank,
+                                               int rot, int page_size, int64_t kp, int64_t ks, int64_t vp, int64_t vd, int64_t v_slot,
+                                               int max_blocks, float scale, int window, int page_run, const float* sinks,
+                                               const float* gate, int64_t gate_token, hipStream_t stream) {
+  if (num_tiles <= 0 || num_tokens <= 0) return TS_OK;
+  const int row = rank + rot, heads_block = min(nh, LP_ROWS);
+  if (!ts_latent_tiles_takes(rank, row) || nh <= 0 || page_size != 32 || v_slot != 1 || kp % 8 || ks % 8 || vp % 8 || vd % 8 || ks < row ||
+      32 * ks >= (1 << 29) || rank * vd >= (1 << 29) || (((uintptr_t)k_cache | (uintptr_t)v_cache | (uintptr_t)q | (uintptr_t)out) & 15) ||
+      max_blocks <= 0 || page_run < 0 || page_run > 16 || !tiles || tile_tokens < 1 || tile_tokens * heads_block > LP_ROWS)
+    return TS_BAD_SHAPE;
+  const dim3 grid(num_tiles, (nh + heads_block - 1) / heads_block);
+  const float scale_log2 = scale * 1.4426950408889634f;
+#define LP_LAUNCH(CP, VB, TO) \
+  latent_attention_tiles_kernel<CP, VB, TO><<<grid, LP_WAVES * TS_WAVE, 0, stream>>>((TO*)out, q, (const bf16_t*)k_cache, (const bf16_t*)v_cache, \
+      block_tables, seq_of_token, positions, tiles, num_tiles, heads_block, nh, rank, row, kp, ks, vp, vd, max_blocks, scale_log2, window, \
+      page_run, sinks, gate, gate_token)
+#define LP_PICK(TO) \
+  do { \
+    if (row <= 128 && rank <= 128) LP_LAUNCH(4, 8, TO); \
+    else if (row <= 256) LP_LAUNCH(8, 16, TO); \
+    else LP_LAUNCH(12, 16, TO); \
+  } while (0)
+  if (out_dtype == 0) LP_PICK(float);
+  else if (out_dtype == 1) LP_PICK(bf16_t);
+  else return TS_BAD_DTYPE;
+#undef LP_PICK
+#undef LP_LAUNCH
+  return ts_check_launch();
+}
+
 // ---- products per head on the matrix cores ---------------------------------------------------------------------
 // y[t, h, n] = sum_k x[t, h, k] w[h][n][k] for bfloat16 matrices whose k runs along memory (a matrix stored [k, n]
 // comes as a transposed copy), x 32-bit (rounded to bfloat16 once, as a projection's operand is) or bfloat16, 32-bit
@@ -381,6 +577,23 @@ heads_gemm_mfma_kernel(TO* __restrict__ y, int64_t y_token, int64_t y_head, cons
     }
   }
   if (t >= num_tokens) return;
+  // whole fours of columns go out in one store (four of a number each: 51 µs against 36 for 2,048 tokens by 32 heads of 256)
+  TO* yrow = y + (int64_t)t * y_token + (int64_t)h * y_head;
+  if (N % 4 == 0 && ((y_token | y_head) & 3) == 0 && ((uintptr_t)y & (4 * sizeof(TO) - 1)) == 0) {
+#pragma unroll
+    for (int nb = 0; nb < HM_COLS / 16; ++nb) {
+      const int n = n0 + 16 * nb + 4 * g;
+      if (n >= N) continue;
+      float4_t v = acc[nb];
+      if (gate) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[j] = v[j] / (1.0f + expf(-gate[(int64_t)t * gate_token + (int64_t)h * N + n + j]));
+      }
+      if constexpr (sizeof(TO) == 4) *(float4_t*)(yrow + n) = v;
+      else *(uint2*)(yrow + n) = make_uint2(pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3]));
+    }
+    return;
+  }
 #pragma unroll
   for (int nb = 0; nb < HM_COLS / 16; ++nb)
 #pragma unroll
@@ -389,7 +602,7 @@ heads_gemm_mfma_kernel(TO* __restrict__ y, int64_t y_token, int64_t y_head, cons
       if (n >= N) continue;
       float v = acc[nb][j];
       if (gate) v = v / (1.0f + expf(-gate[(int64_t)t * gate_token + (int64_t)h * N + n]));
-      Num<TO>::st(y + (int64_t)t * y_token + (int64_t)h * y_head + n, v);
+      Num<TO>::st(yrow + n, v);
     }
 }
 

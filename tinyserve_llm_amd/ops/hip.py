@@ -104,6 +104,8 @@ def _declare(lib: ctypes.CDLL) -> None:
         "ts_heads_gemm_mfma": [p, i, i64, i64, p, i, i64, i64, p, i64, i64, i, i, i, i, p, i64, p],
         "ts_paged_attention_latent_mfma": [p, i, p, p, p, p, p, p, p, i, i, i, i, i, i, i, i64, i64, i64, i64, i64, i, f, i, i, i, p, p,
                                            p, p, i64, p],
+        "ts_latent_tiles_takes": [i, i],
+        "ts_paged_attention_latent_tiles": [p, i, p, p, p, p, p, p, p, i, i, i, i, i, i, i, i64, i64, i64, i64, i64, i, f, i, i, p, p, i64, p],
         "ts_rotate_heads": [p, i, i64, i64, p, i, i64, i64, i, i, i, p, f, p, i, i, p, i64, p],
         "ts_heads_gemm": [p, i, i64, i64, p, i, i64, i64, p, i, i64, i64, i64, i, i, i, i, p, i64, p],
         "ts_paged_attention_latent": [p, i, p, i, p, i, p, p, p, i, i, i, i, i, i64, i64, i, f, i, i, p, p, i64, p],
@@ -2345,6 +2347,8 @@ def heads_gemm(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, gate: torch.
 
 
 LATENT_TILE_ROWS = 32     # rows (token, head) of a workgroup of the matrix-core kernel
+LATENT_WIDE_TILE_ROWS = 128    # and of its form for steps of many tokens,
+LATENT_MANY_ROWS = 8192   # which takes portions of steps of at least so many rows
 LATENT_MAX_SPLITS = 16    # stretches a tile's keys may be cut into,
 LATENT_FEW_GROUPS = 512   # where the step has fewer workgroups than half of this
 
@@ -2357,6 +2361,17 @@ def latent_mfma_takes(q: torch.Tensor, cache: torch.Tensor, v_cache: torch.Tenso
             and cache.shape[1] == 32 and v_cache.stride(1) == 1 and bool(library().ts_latent_mfma_takes(rank, q.shape[2]))
             and all(st % 8 == 0 for st in (cache.stride(0), cache.stride(1), v_cache.stride(0), v_cache.stride(3)))
             and cache.data_ptr() % 16 == 0 and v_cache.data_ptr() % 16 == 0 and q.data_ptr() % 16 == 0)
+
+
+def _latent_tiles(ctx, tile_tokens: int, device) -> torch.Tensor:
+    """`attention_tiles` of a step on the device (int32 [tiles, 2]), made once and kept in the step's scratch."""
+    tiles = ctx.scratch.get(("latent_tiles", tile_tokens))
+    if tiles is None:
+        _need(not torch.cuda.is_current_stream_capturing(), "the tile list is made before a graph is recorded")
+        flat = attention_tiles(ctx.host_cu_seqlens, ctx.host_starts, tile_tokens)
+        tiles = torch.tensor(flat, dtype=torch.int32).view(-1, 2).to(device, non_blocking=True)
+        ctx.scratch[("latent_tiles", tile_tokens)] = tiles
+    return tiles
 
 
 def paged_attention_latent(q: torch.Tensor, cache: torch.Tensor, rank: int, ctx, space: int, scale: float, window: int = 0,
@@ -2386,16 +2401,21 @@ def paged_attention_latent(q: torch.Tensor, cache: torch.Tensor, rank: int, ctx,
     mask = -chunk_mask if chunk_mask else int(window)
     if latent_mfma_takes(q, cache, v_cache, rank) and out.dtype in (torch.float32, torch.bfloat16):
         _need(v_cache.shape == (*cache.shape[:3], rank), "the values' view must match the rows'")
+        if ctx.max_query_len > 1 and T * H >= LATENT_MANY_ROWS and out.data_ptr() % 16 == 0 and bool(library().ts_latent_tiles_takes(rank, row)):
+            # many tokens: tiles of four times as many rows, whose keys a workgroup reads once
+            tile_tokens = max(1, LATENT_WIDE_TILE_ROWS // H)
+            tiles = _latent_tiles(ctx, tile_tokens, q.device)
+            _run("paged_attention_latent_tiles", library().ts_paged_attention_latent_tiles(
+                _ptr(out), _code(out.dtype), _ptr(q), _ptr(cache), _ptr(v_cache), _ptr(tables), _ptr(ctx.seq_of_token), _ptr(ctx.positions),
+                _ptr(tiles), tiles.shape[0], tile_tokens, T, H, rank, row - rank, cache.shape[1], cache.stride(0),
+                cache.stride(1), v_cache.stride(0), v_cache.stride(3), v_cache.stride(1), tables.shape[1], float(scale), mask,
+                _page_run(table_page // cache.shape[1]), _ptr(sinks), _ptr(head_gate), gate_stride, _stream()))
+            return out
         tile_tokens = max(1, LATENT_TILE_ROWS // H)
         tiles, num_tiles = None, T
         if ctx.max_query_len > 1 and tile_tokens > 1:
             # (a token with 32 heads or more is a tile of its own: no list; else tiles of several tokens of one request)
-            tiles = ctx.scratch.get(("latent_tiles", tile_tokens))
-            if tiles is None:
-                _need(not torch.cuda.is_current_stream_capturing(), "the tile list is made before a graph is recorded")
-                flat = attention_tiles(ctx.host_cu_seqlens, ctx.host_starts, tile_tokens)
-                tiles = torch.tensor(flat, dtype=torch.int32).view(-1, 2).to(q.device, non_blocking=True)
-                ctx.scratch[("latent_tiles", tile_tokens)] = tiles
+            tiles = _latent_tiles(ctx, tile_tokens, q.device)
             num_tiles = tiles.shape[0]
         # few tiles (decoded tokens): a tile's keys in stretches, a workgroup each, and a second kernel that adds them up
         groups = num_tiles * -(-H // LATENT_TILE_ROWS)

@@ -602,6 +602,30 @@ def test_gated_product_of_many_rows(m, f, k, form, limit, slope, shift):
             bad()
 
 
+@pytest.mark.parametrize("unit", [("sigmoid", 0.0, 1.0, 0.0), ("sigmoid", 0.7, 1.702, 1.0), ("relu", 0.0, 1.0, 0.0), ("gelu_tanh", 0.5, 1.0, 0.25)])
+@pytest.mark.parametrize("m,f,k", [(1, 48, 256), (2, 512, 1024), (5, 8192, 2048), (8, 4096, 4096), (16, 4112, 512), (32, 1024, 2048), (33, 4096, 1024),
+                                   (40, 2064, 2048), (64, 8192, 2048)])
+def test_gated_unit_of_few_rows(m, f, k, unit):
+    """The unit on the product's way out has the bits of the unit of the same kernel's 32-bit sums: rows handed on as a matrix
+    and in the 8-row form's order, one wave and several, widths that hang over the last workgroup."""
+    from tinyserve_llm_amd.parts import linear as lin
+    g = gen(m + f + k)
+    x = torch.randn(m, k, generator=g).bfloat16().to(dev())
+    w, down = ((torch.randn(n, kk, generator=g) * (2.0 / math.sqrt(kk))).bfloat16().to(dev()) for n, kk in ((2 * f, k), (256, f)))
+    wide = hip().rows64_takes(m, 2 * f, k)
+    for copies in ([None] if not wide else []) + [lin.streaming_copy(w)]:
+        out = lin.few_rows_unit(x, w, copies, down, unit)
+        if m > 16 and not wide and 2 * f * k > hip().SKINNY_WIDE_ELEMENTS or m > 32 and not wide:
+            assert out is None, "no plain product of this shape goes to such a kernel"
+            continue
+        assert isinstance(out, hip().PackedRows8) == (2 <= m <= 8)
+        sums = (hip().gemm_rows64(x, copies.by16, torch.float32) if wide else hip().gemm_skinny(x, w, torch.float32)[0])
+        want = hip().capped_glu(sums, *unit[1:], torch.bfloat16, activation=unit[0])
+        assert torch.equal(out.rows() if isinstance(out, hip().PackedRows8) else out, want)
+    with pytest.raises(hip().KernelError, match="comes with the gate"):
+        hip().gemm_skinny(x, w, unit=unit)
+
+
 @pytest.mark.parametrize("m", [1, 3, 8, 16, 17, 32])
 @pytest.mark.parametrize("n,k", [(3072, 2048), (2048, 2048), (16384, 2048), (2048, 8192), (992, 512), (130, 3072), (64, 4096),
                                  (8192, 3072), (8256, 4096)])

@@ -20,28 +20,17 @@
 // turn and fetches the next tile's first steps before it writes out the present one. The gate rows of a wave's columns
 // and their up rows lie side by side in the tile, so that a gate and its up meet in one lane; two lanes exchange halves so
 // that every store is 16 bytes (8-byte stores: 45 µs against 24 for the same product with K = 128).
+#include "glu_unit.h"
 #include "lds_loads.h"
 
-// How a gate goes into the unit: as `silu_mul` of a bfloat16 product and `capped_glu` of 32-bit sums do it, so that the stored
-// units are the same (the hardware's 2^x and reciprocal throughout would take 10 of 130 µs off the sigmoid form).
-enum { GLU_SILU_ROUNDED, GLU_SIGMOID, GLU_RELU, GLU_GELU };
-static __device__ __forceinline__ float glu_sigmoid(float z) { return __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-1.44269504088896340736f * z)); }
+// The unit's forms (glu_unit.h; the hardware's 2^x and reciprocal throughout would take 10 of 130 µs off the sigmoid form).
 template <int ACT> static __device__ __forceinline__ float glu_unit(float g, float u, float limit, float slope, float up_shift) {
   if constexpr (ACT == GLU_SILU_ROUNDED) {          // both branches as a bfloat16 product leaves them
     const uint32_t both = pack_bf16(g, u);
     g = __uint_as_float(both << 16);
-    return g * glu_sigmoid(g) * __uint_as_float(both & 0xffff0000u);
+    return g * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-1.44269504088896340736f * g)) * __uint_as_float(both & 0xffff0000u);
   }
-  if (limit > 0.f) {
-    g = fminf(g, limit);
-    u = fminf(fmaxf(u, -limit), limit);
-  }
-  u += up_shift;
-  if constexpr (ACT == GLU_RELU) return fmaxf(g, 0.f) * u;
-  if constexpr (ACT == GLU_GELU) return 0.5f * g * (1.0f + tanhf(0.7978845608028654f * (g + 0.044715f * g * g * g))) * u;
-  // (g / d for d >= 1: the reciprocal's quotient and one correction, as good as a division here; d stays finite)
-  const float d = 1.0f + fminf(expf(-slope * g), 1e38f), inv = __builtin_amdgcn_rcpf(d), q = g * inv;
-  return fmaf(fmaf(-q, d, g), inv, q) * u;
+  return glu_capped(ACT, g, u, limit, slope, up_shift);
 }
 
 struct GluArgs {

@@ -32,6 +32,7 @@
 // gemm_skinny.hip does: the new residual, the next projection's operand and the rows' sums of squares
 // (whole: a workgroup of that kernel takes a row).
 #include <type_traits>
+#include "glu_unit.h"
 #include "skinny_ops.h"
 
 #define R64_CHUNK_STEPS 8         // 32-wide k steps per chunk of x in LDS
@@ -51,12 +52,14 @@ struct Rows64Args {
   const float* ssq_in;
   int ssq_parts;
   float eps;
+  float limit, slope, up_shift;      // of the unit (GLU > 1)
   int slices;            // the reduction in this many slices (gridDim.y); more than one: y is float [slices][M][ldy]
 };
 
 // BLOCKS: blocks of 16 rows of x, 4 (up to 64 rows) or 8 (up to 128: the compute waves then take a chunk's
 // steps one at a time instead of in pairs, for their registers' sake).
-template <bool GLU, typename OUT, int BLOCKS>
+// GLU: 0 none, 1 silu(gate) up, 1 + f the unit of form f of glu_unit.h.
+template <int GLU, typename OUT, int BLOCKS>
 __global__ void __launch_bounds__(512) gemm_rows64_kernel(const Rows64Args a) {
   // x as the B operands of the matrix instruction: [buffer][step][block of 16 rows][lane], lane r + 16 g
   // holding k = 8 g .. 8 g + 7 of row r (turned: sk_place)
@@ -205,13 +208,18 @@ __global__ void __launch_bounds__(512) gemm_rows64_kernel(const Rows64Args a) {
     acc[b] *= scale[b];
     u *= scale[b];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) Num<OUT>::st(y + (int64_t)m * a.ldy + n0 + j, GLU ? sk_silu(acc[b][j]) * u[j] : acc[b][j]);
+    for (int j = 0; j < 4; ++j) {
+      float v = acc[b][j];
+      if constexpr (GLU == 1) v = sk_silu(v) * u[j];
+      if constexpr (GLU > 1) v = glu_capped(GLU - 1, v, u[j], a.limit, a.slope, a.up_shift);
+      Num<OUT>::st(y + (int64_t)m * a.ldy + n0 + j, v);
+    }
   }
 }
 
 #define R64_MAX_ROWS 128
 
-template <bool GLU, typename OUT>
+template <int GLU, typename OUT>
 static int r64_launch(const Rows64Args& a, hipStream_t stream) {
   // 64 rows of W per workgroup; two buffers of a chunk of x in LDS: 64 KB for up to 64 rows, 128 KB beyond
   const dim3 grid(a.N / 64, a.slices);
@@ -227,18 +235,25 @@ static bool r64_operands_ok(const void* x, const void* w16, int M, int N, int K,
 
 // x [M <= 128, K] (row stride ldx), w16: W [N, K] as its 16-row packed copy, y [M, N] or, with glu, [M, N / 2]
 // (row stride ldy; out_f32: 32-bit sums instead of bfloat16). N a multiple of 64 (128 with glu), K of 1,024.
-// ssq_in [M, ssq_parts] and eps: the prepared norm's scale per row (null: none).
+// ssq_in [M, ssq_parts] and eps: the prepared norm's scale per row (null: none). glu: 1 silu(gate) up, 1 + f the unit of form f
+// of glu_unit.h with limit, slope and up_shift.
 extern "C" int ts_gemm_rows64_bf16(void* y, const void* x, const void* w16, int M, int N, int K, int64_t ldx, int64_t ldy,
-                                   int glu, int out_f32, const void* ssq_in, int ssq_parts, float eps, hipStream_t stream) {
+                                   int glu, int out_f32, const void* ssq_in, int ssq_parts, float eps, float limit, float slope,
+                                   float up_shift, hipStream_t stream) {
   if (M <= 0 || N <= 0) return TS_OK;
   if (N % (glu ? 128 : 64) || K % 1024 || !y || !r64_operands_ok(x, w16, M, N, K, ldx)) return TS_BAD_SHAPE;
   if (ldy < (glu ? N / 2 : N) || (((uintptr_t)y) & (out_f32 ? 3 : 1))) return TS_BAD_SHAPE;
   if (glu && out_f32) return TS_BAD_SHAPE;
   if (ssq_in && (ssq_parts <= 0 || (((uintptr_t)ssq_in) & 3))) return TS_BAD_SHAPE;
-  Rows64Args a = {(const bf16_t*)x, (const bf16_t*)w16, y, M, N, K, ldx, ldy, (const float*)ssq_in, ssq_parts, eps, 1};
-  if (glu) return r64_launch<true, bf16_t>(a, stream);
-  if (out_f32) return r64_launch<false, float>(a, stream);
-  return r64_launch<false, bf16_t>(a, stream);
+  Rows64Args a = {(const bf16_t*)x, (const bf16_t*)w16, y, M, N, K, ldx, ldy, (const float*)ssq_in, ssq_parts, eps, limit, slope, up_shift, 1};
+  switch (glu) {
+    case 0: return out_f32 ? r64_launch<0, float>(a, stream) : r64_launch<0, bf16_t>(a, stream);
+    case 1: return r64_launch<1, bf16_t>(a, stream);
+    case 1 + GLU_SIGMOID: return r64_launch<1 + GLU_SIGMOID, bf16_t>(a, stream);
+    case 1 + GLU_RELU: return r64_launch<1 + GLU_RELU, bf16_t>(a, stream);
+    case 1 + GLU_GELU: return r64_launch<1 + GLU_GELU, bf16_t>(a, stream);
+  }
+  return TS_BAD_SHAPE;
 }
 
 // ---- a product in slices of its reduction, and what finishes it
@@ -335,8 +350,8 @@ extern "C" int ts_gemm_rows64_sliced_bf16(void* y, void* parts, const void* x, c
   } else if (!y || (((uintptr_t)y) & 7)) {
     return TS_BAD_SHAPE;
   }
-  Rows64Args a = {(const bf16_t*)x, (const bf16_t*)w16, parts, M, N, K, ldx, (int64_t)N, nullptr, 0, 0.f, slices};
-  const int rc = r64_launch<false, float>(a, stream);
+  Rows64Args a = {(const bf16_t*)x, (const bf16_t*)w16, parts, M, N, K, ldx, (int64_t)N, nullptr, 0, 0.f, 0.f, 0.f, 0.f, slices};
+  const int rc = r64_launch<0, float>(a, stream);
   if (rc != TS_OK) return rc;
   const int threads = N / 4 >= R64_FINISH_THREADS ? R64_FINISH_THREADS : (N / 4 + TS_WAVE - 1) / TS_WAVE * TS_WAVE;
   if (next_nw) rows64_finish_kernel<true><<<M, threads, 0, stream>>>(f);
@@ -469,8 +484,8 @@ extern "C" int ts_gemm_rows64_sliced_rope_bf16(void* q_out, void* parts, const v
   if (ssq_in && (ssq_parts <= 0 || (((uintptr_t)ssq_in) & 3))) return TS_BAD_SHAPE;
   if (rotate && (!cos_sin || !positions)) return TS_BAD_SHAPE;
   if (k_cache && (!v_cache || !slots || (kp % 4) || (ks % 4) || (kh % 4) || (((uintptr_t)k_cache) & 7))) return TS_BAD_SHAPE;
-  Rows64Args a = {(const bf16_t*)x, (const bf16_t*)w16, parts, M, N, K, ldx, (int64_t)N, nullptr, 0, 0.f, slices};
-  const int rc = r64_launch<false, float>(a, stream);
+  Rows64Args a = {(const bf16_t*)x, (const bf16_t*)w16, parts, M, N, K, ldx, (int64_t)N, nullptr, 0, 0.f, 0.f, 0.f, 0.f, slices};
+  const int rc = r64_launch<0, float>(a, stream);
   if (rc != TS_OK) return rc;
   Rows64RopeArgs f = {(const float*)parts, slices, M, N, K, (const float*)ssq_in, ssq_parts, eps, cos_sin, positions, slots,
                       (bf16_t*)q_out, (bf16_t*)k_cache, (bf16_t*)v_cache, nh, nkv, hd, rotate, page_size,

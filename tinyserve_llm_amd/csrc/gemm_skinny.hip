@@ -23,12 +23,16 @@
 //              t^2 over the tile's columns; y itself is not stored
 //   EPI_GLU    W = [gate rows | up rows]; a workgroup takes matching rows of both and writes
 //              silu(gate) * up, y being [M, N / 2]
+//   EPI_UNIT   the same with a capped unit of the 32-bit sums in silu's place (glu_unit.h); its form and numbers
+//              travel in fields that only EPI_ROPE uses: nh the form, nkv, hd and rotate the bits of limit,
+//              slope and up_shift
 //   EPI_ROPE   W = [q heads | k heads | v heads] of head_dim columns each; a 16-row tile holds 8
 //              columns of the first half of a head (matrix rows r < 8) and the 8 that rotate with
 //              them (rows r >= 8: head_dim / 2 further on), so a workgroup of one tile has both
 //              halves of a rotation and a matrix of 3,072 columns gives 192 workgroups; it rounds the
 //              products as y would hold them, rotates q and k by the token's position, and writes q
 //              to its own tensor and k and v into their cache slots: y itself is never stored
+#include "glu_unit.h"
 #include "skinny_ops.h"
 
 struct SkinnyArgs {
@@ -79,7 +83,7 @@ struct SkinnyArgs {
 template <int RT, int CB, int STEPS, int MODE, int EPI, int MAXT, typename OUT>
 __global__ void __launch_bounds__(MAXT)
 gemm_skinny_kernel(const SkinnyArgs a) {
-  constexpr bool GLU = EPI == EPI_GLU, ROPE = EPI == EPI_ROPE, PAIRS = GLU || ROPE, NEXT = EPI == EPI_NEXT;
+  constexpr bool UNIT = EPI == EPI_UNIT, GLU = EPI == EPI_GLU || UNIT, ROPE = EPI == EPI_ROPE, PAIRS = GLU || ROPE, NEXT = EPI == EPI_NEXT;
   static_assert(MODE != MODE_NORM || CB == 1, "the fused norm serves one block of rows");
   static_assert(!GLU || RT % 2 == 0, "gate and up tiles come in pairs");
   // steps of x fetched at a time: fewer where more blocks of x, more row tiles of W or a larger workgroup leave fewer registers
@@ -221,7 +225,7 @@ gemm_skinny_kernel(const SkinnyArgs a) {
   // ---- EPI_NEXT: the residual and the next norm's weight of the four columns this thread will finish
   // are asked for right behind W (where every thread finishes at most one item and the columns are
   // whole), so that the way out does not wait for a trip to the cache
-  constexpr int NEXT_ITEMS = (EPI == EPI_GLU ? RT / 2 : RT) * CB * 64;
+  constexpr int NEXT_ITEMS = (GLU ? RT / 2 : RT) * CB * 64;
   const bool next_early = NEXT && NEXT_ITEMS <= (int)blockDim.x && a.N % 4 == 0;
   uint2 pre_res = make_uint2(0, 0), pre_nw = make_uint2(0, 0);
   if constexpr (NEXT) {
@@ -444,6 +448,10 @@ gemm_skinny_kernel(const SkinnyArgs a) {
   // part[.][t][b][m_local * 16 + n_local]: a thread sums 4 consecutive n of one m over the waves in order
   OUT* y = (OUT*)a.y;
   const int ncols = GLU ? half : a.N;
+  const auto gated = [&](float gate, float up) -> float {
+    if constexpr (UNIT) return glu_capped(a.nh, gate, up, __int_as_float(a.nkv), __int_as_float(a.hd), __int_as_float(a.rotate));
+    else return sk_silu(gate) * up;
+  };
   if constexpr (NEXT) {
     if (next_early) {                                   // every thread finishes at most one item, and has prepared it
       if ((int)threadIdx.x >= NEXT_ITEMS) return;       // (whole waves: an item's four threads stay together)
@@ -501,7 +509,7 @@ gemm_skinny_kernel(const SkinnyArgs a) {
       }
       float v[4];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) v[j] = sk_silu(s[j]) * u[j];
+      for (int j = 0; j < 4; ++j) v[j] = gated(s[j], u[j]);
       if (a.y_pack8) *(uint2*)way_dst = make_uint2(sk_round(v[0]) | (sk_round(v[1]) << 16), sk_round(v[2]) | (sk_round(v[3]) << 16));
       else *(uint2*)way_dst = make_uint2(f2bf(v[0]) | ((uint32_t)f2bf(v[1]) << 16), f2bf(v[2]) | ((uint32_t)f2bf(v[3]) << 16));
       return;
@@ -669,14 +677,14 @@ gemm_skinny_kernel(const SkinnyArgs a) {
         bf16_t* dst = (bf16_t*)a.y + (((int64_t)w * S + (in_half >> 5)) * 64 + m + 8 * hf + 16 * ((in_half & 31) >> 3)) * 8 + (n & 7);
         float v[4];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) v[j] = sk_silu(s[j]) * u[j];
+        for (int j = 0; j < 4; ++j) v[j] = gated(s[j], u[j]);
         *(uint2*)dst = make_uint2(sk_round(v[0]) | (sk_round(v[1]) << 16), sk_round(v[2]) | (sk_round(v[3]) << 16));
         continue;
       }
     }
 #pragma unroll
     for (int j = 0; j < 4; ++j)
-      if (n + j < ncols) Num<OUT>::st(y + (int64_t)m * a.ldy + n + j, GLU ? sk_silu(s[j]) * u[j] : s[j]);
+      if (n + j < ncols) Num<OUT>::st(y + (int64_t)m * a.ldy + n + j, GLU ? gated(s[j], u[j]) : s[j]);
   }
 }
 
@@ -700,8 +708,9 @@ static int sk_launch(const SkinnyArgs& a, hipStream_t stream) {
   // (the kilobytes through which a wave turns its rows of x, where it does: X_TURNED of the kernel)
   if (CB >= 2 && CB >= RT && MODE != MODE_NORM && nwaves <= 8 && (CB * STEPS + RT * STEPS) <= 48 && smem < (size_t)nwaves * STEPS * 1024)
     smem = (size_t)nwaves * STEPS * 1024;
-  constexpr int OT = GLU == EPI_GLU ? RT / 2 : RT;
-  const int ncols = GLU == EPI_GLU ? a.N / 2 : a.N;     // (EPI_ROPE: a 16-row tile of the matrix per 8 columns and their partners)
+  constexpr bool PAIRED = GLU == EPI_GLU || GLU == EPI_UNIT;
+  constexpr int OT = PAIRED ? RT / 2 : RT;
+  const int ncols = PAIRED ? a.N / 2 : a.N;     // (EPI_ROPE: a 16-row tile of the matrix per 8 columns and their partners)
   if (smem > sk_lds_limit()) return TS_BAD_SHAPE;       // (the largest instances ask for a little more than 64 KB)
   dim3 grid((ncols + 16 * OT - 1) / (16 * OT)), block(nwaves * TS_WAVE);
   if (nwaves <= 8) {
@@ -723,7 +732,7 @@ static int sk_launch(const SkinnyArgs& a, hipStream_t stream) {
 #endif
 template <int MODE, int EPI, typename OUT>
 static int sk_dispatch(const SkinnyArgs& a, hipStream_t stream) {
-  constexpr bool GLU = EPI == EPI_GLU, NORM = MODE == MODE_NORM;
+  constexpr bool GLU = EPI == EPI_GLU || EPI == EPI_UNIT, NORM = MODE == MODE_NORM;
   const int steps = (a.K % 256 == 0 && a.K / 256 <= 16) ? 8 : 16;
   if (a.K % (steps * SK_KSTEP) || a.K / (steps * SK_KSTEP) > 16) return TS_BAD_SHAPE;
   const int nwaves = a.K / (steps * SK_KSTEP);
@@ -1068,13 +1077,15 @@ extern "C" int ts_gemm_skinny8_act_bf16(void* y, const void* x, const void* w, i
 // (up to 8192), contiguous 16-byte aligned rows; mode 1 takes x, res, res_out as dense [M, K].
 // With next_nw (EPI_NEXT; modes 0 and 2 without glu, bfloat16) y is not written: next_res_out, next_op
 // [M, N] and ssq_out [M, tiles] are, tiles being the 16-column tiles the grid covers (ts_skinny_tiles).
+// glu > 1 (mode 0): the unit of form glu - 1 of glu_unit.h with limit, slope and up_shift in silu's place.
 // y_pack8 > 0 (glu, bfloat16, M <= 8, N / 2 a multiple of 64 y_pack8): y is not [M, N / 2] but the gated product in
 // the order the 8-row form of y_pack8 steps reads its x (SkinnyArgs::x_packed8): N / 2 / 8 pieces of 64 lanes.
 extern "C" int ts_gemm_skinny_bf16(void* y, const void* x, const void* w, const void* res, const void* nw,
                                    void* res_out, int M, int N, int K, int64_t ldx, int64_t ldw, int64_t ldy,
                                    float eps, int mode, int glu, int out_dtype, int packed, const void* ssq_in,
                                    int ssq_parts, const void* next_res, const void* next_nw, void* next_res_out,
-                                   void* next_op, void* ssq_out, int y_pack8, hipStream_t stream) {
+                                   void* next_op, void* ssq_out, int y_pack8, float limit, float slope, float up_shift,
+                                   hipStream_t stream) {
   if (M <= 0 || N <= 0) return TS_OK;
   // the gated product for the 8-row form: up to 8 rows, bfloat16, whole waves of the reader (64 y_pack8 of k each)
   if (y_pack8 && (!glu || out_dtype != 1 || M > 8 || (y_pack8 != 4 && y_pack8 != 8 && y_pack8 != 16) || (N / 2) % (64 * y_pack8))) return TS_BAD_SHAPE;
@@ -1096,7 +1107,12 @@ extern "C" int ts_gemm_skinny_bf16(void* y, const void* x, const void* w, const 
     if (mode == MODE_PLAIN) return sk_dispatch<MODE_PLAIN, EPI_NEXT, bf16_t>(a, stream);
     return sk_dispatch<MODE_PREP, EPI_NEXT, bf16_t>(a, stream);
   }
-  if (!y || ldy < (glu ? N / 2 : N)) return TS_BAD_SHAPE;
+  if (!y || ldy < (glu ? N / 2 : N) || glu < 0 || glu > 1 + GLU_GELU) return TS_BAD_SHAPE;
+  if (glu > 1) {
+    if (out_dtype != 1 || mode != MODE_PLAIN) return TS_BAD_DTYPE;
+    a.nh = glu - 1, a.nkv = __builtin_bit_cast(int, limit), a.hd = __builtin_bit_cast(int, slope), a.rotate = __builtin_bit_cast(int, up_shift);
+    return sk_dispatch<MODE_PLAIN, EPI_UNIT, bf16_t>(a, stream);
+  }
   if (out_dtype == 1) {
     if (mode == MODE_PLAIN && !glu) return sk_dispatch<MODE_PLAIN, EPI_NONE, bf16_t>(a, stream);
     if (mode == MODE_PLAIN && glu) return sk_dispatch<MODE_PLAIN, EPI_GLU, bf16_t>(a, stream);

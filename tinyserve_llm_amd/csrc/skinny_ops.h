@@ -14,6 +14,7 @@ typedef float float4_t __attribute__((ext_vector_type(4)));
 #define EPI_GLU 1
 #define EPI_ROPE 2
 #define EPI_NEXT 3
+#define EPI_UNIT 4      // EPI_GLU with one of the capped units of glu_unit.h in silu's place
 
 // acc + A · B over 32 k: lane (r, g) gives k = 8 g .. 8 g + 7 of row r of A and of column r of B
 static __device__ __forceinline__ float4_t sk_mfma(const uint4& a, const uint4& b, float4_t acc) {

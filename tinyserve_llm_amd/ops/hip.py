@@ -69,10 +69,10 @@ def _declare(lib: ctypes.CDLL) -> None:
         "ts_gemm_library_timing": [i],
         "ts_gemm_library_choices": [p, i],
         "ts_paged_attention_prefill": [p, p, p, p, p, p, p, p, i, i, i, i, i, i, i, i64, i64, i64, i64, i64, i64, i, f, i, i, i, i, i, p, p, i, p],
-        "ts_gemm_skinny_bf16": [p, p, p, p, p, p, i, i, i, i64, i64, i64, f, i, i, i, i, p, i, p, p, p, p, p, i, p],
+        "ts_gemm_skinny_bf16": [p, p, p, p, p, p, i, i, i, i64, i64, i64, f, i, i, i, i, p, i, p, p, p, p, p, i, f, f, f, p],
         "ts_gemm_skinny8_bf16": [p, p, p, i, i, i, i64, i64, i64, i, i, p, p, p, p, p, i, p, p, p, i, i, i, i, p],
         "ts_gemm_skinny8_act_bf16": [p, p, p, i, i, i, i64, i64, i64, i, i, p, i, p],
-        "ts_gemm_rows64_bf16": [p, p, p, i, i, i, i64, i64, i, i, p, i, f, p],
+        "ts_gemm_rows64_bf16": [p, p, p, i, i, i, i64, i64, i, i, p, i, f, f, f, f, p],
         "ts_gemm_rows64_sliced_bf16": [p, p, p, p, i, i, i, i64, i, p, p, p, p, p, i64, p],
         "ts_gemm_rows64_sliced_rope_bf16": [p, p, p, p, i, i, i64, i, p, i, f, p, p, p, p, p, i, i, i, i, i, i64, i64, i64, i64, i64,
                                             i64, i64, p],
@@ -1107,10 +1107,15 @@ def skinny_fuses(rows: int, k: int, norm: bool, glu: bool) -> bool:
     return rows <= SKINNY_EPILOGUE_ROWS and k <= SKINNY_EPILOGUE_WIDE_K
 
 
+def _unit_code(glu: bool, unit) -> int:
+    """The few-rows kernels' `glu` argument: none, silu(gate) up, or which of the units of `capped_glu`."""
+    return int(glu) if unit is None else 1 + GLU_FORMS[unit[0]]
+
+
 def gemm_skinny(x: torch.Tensor, weight: torch.Tensor, out_dtype: torch.dtype = torch.bfloat16, *,
                 residual: torch.Tensor | None = None, norm_weight: torch.Tensor | None = None, eps: float = 0.0,
                 glu: bool = False, packed: torch.Tensor | None = None, squares: torch.Tensor | None = None,
-                next_norm=None, pack8_steps: int = 0) -> "tuple[torch.Tensor | PreparedNorm | PackedRows8, torch.Tensor | None]":
+                next_norm=None, pack8_steps: int = 0, unit: "tuple[str, float, float, float] | None" = None) -> "tuple[torch.Tensor | PreparedNorm | PackedRows8, torch.Tensor | None]":
     """bfloat16 e(f(x) [M <= 32, K] · weight [N, K]^T) by the weight-streaming MFMA kernel (up to 64
     rows over reductions of up to 2048). With `norm_weight`: f = RMSNorm(x + residual) * norm_weight,
     and x + residual comes back as the second result. With `squares` (and `eps`): x is the operand of
@@ -1119,7 +1124,8 @@ def gemm_skinny(x: torch.Tensor, weight: torch.Tensor, out_dtype: torch.dtype = 
     With `packed` (= pack_weight(weight)) the kernel reads that copy. With `next_norm` = (residual or
     None, weight of the norm that follows) the first result is a `PreparedNorm` instead of the product.
     With `pack8_steps` (and `glu`, up to 8 rows) the gated product comes back as a `PackedRows8` for a
-    reader of that many steps."""
+    reader of that many steps. `unit` (with `glu` and a plain x): (form, limit, slope, up_shift) of the unit of
+    `capped_glu` in silu's place."""
     _gpu(x, weight, residual, norm_weight)
     _need(x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16, "gemm_skinny takes bfloat16")
     _need(x.dim() == 2 and weight.dim() == 2 and x.shape[1] == weight.shape[1],
@@ -1137,6 +1143,7 @@ def gemm_skinny(x: torch.Tensor, weight: torch.Tensor, out_dtype: torch.dtype = 
     _check_squares(squares, M)
     _need(squares is None or not norm, "a norm is either prepared by the kernel before or made here")
     mode = 1 if norm else 2 if squares is not None else 0
+    _need(unit is None or (glu and mode == 0 and unit[0] in GLU_ACTIVATIONS), lambda: f"a unit {unit} comes with the gate and a plain x")
     if next_norm is not None:
         _need(not glu and not norm and out_dtype == torch.bfloat16, "a prepared norm follows a plain bfloat16 product")
         prepared, nres, nw = _next_norm_outputs(x, N, library().ts_skinny_tiles(M, N, K), next_norm)
@@ -1144,7 +1151,7 @@ def gemm_skinny(x: torch.Tensor, weight: torch.Tensor, out_dtype: torch.dtype = 
             None, _ptr(x), _ptr(weight if packed is None else packed), None, None, None, M, N, K, x.stride(0),
             weight.stride(0), N, float(eps), mode, 0, 1, int(packed is not None), _ptr(squares),
             0 if squares is None else squares.shape[1], _ptr(nres), _ptr(nw), _ptr(prepared.summed), _ptr(prepared.operand),
-            _ptr(prepared.squares), 0, _stream()))
+            _ptr(prepared.squares), 0, 0.0, 0.0, 0.0, _stream()))
         return prepared, None
     res_out = None
     if norm:
@@ -1170,8 +1177,9 @@ def gemm_skinny(x: torch.Tensor, weight: torch.Tensor, out_dtype: torch.dtype = 
     _run("gemm_skinny", library().ts_gemm_skinny_bf16(
         _ptr(out), _ptr(x), _ptr(weight if packed is None else packed), _ptr(residual), _ptr(norm_weight),
         _ptr(res_out) if residual is not None else None, M, N, K, x.stride(0), weight.stride(0), ldy,
-        float(eps), mode, int(glu), _code(out_dtype), int(packed is not None), _ptr(squares),
-        0 if squares is None else squares.shape[1], None, None, None, None, None, int(pack8_steps), _stream()))
+        float(eps), mode, _unit_code(glu, unit), _code(out_dtype), int(packed is not None), _ptr(squares),
+        0 if squares is None else squares.shape[1], None, None, None, None, None, int(pack8_steps),
+        *((0.0, 0.0, 0.0) if unit is None else map(float, unit[1:])), _stream()))
     return (PackedRows8(out, M, N // 2, pack8_steps) if pack8_steps else out), res_out
 
 
@@ -1194,11 +1202,13 @@ def rows64_takes(rows: int, n: int, k: int, glu: bool = False) -> bool:
 
 
 def gemm_rows64(x: torch.Tensor, packed: torch.Tensor, out_dtype: torch.dtype = torch.bfloat16, *,
-                glu: bool = False, squares: torch.Tensor | None = None, eps: float = 0.0) -> torch.Tensor:
+                glu: bool = False, squares: torch.Tensor | None = None, eps: float = 0.0,
+                unit: "tuple[str, float, float, float] | None" = None) -> torch.Tensor:
     """bfloat16 e(x [M <= 128, K] · W [N, K]^T) for a wide W given as `packed` = pack_weight(W), by the
     kernel that shares x among 64 rows of W through LDS (gemm_rows64.hip). With `glu`, W holds gate
     rows then up rows and the result is silu(gate) * up, [M, N / 2]. With `squares` (and `eps`) x is
-    the operand of a `PreparedNorm` and the rows' scales multiply the finished sums."""
+    the operand of a `PreparedNorm` and the rows' scales multiply the finished sums. `unit` (with `glu`, a plain
+    x): (form, limit, slope, up_shift) of the unit of `capped_glu` in silu's place."""
     _gpu(x, packed)
     _need(x.dtype == torch.bfloat16 and packed.dtype == torch.bfloat16 and x.dim() == 2 and packed.dim() == 4
           and packed.shape[2:] == (64, 8) and packed.is_contiguous(), "gemm_rows64 takes bfloat16 x [M, K] and pack_weight(W)")
@@ -1211,10 +1221,12 @@ def gemm_rows64(x: torch.Tensor, packed: torch.Tensor, out_dtype: torch.dtype = 
     _need(x.stride(1) == 1 and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0, "rows of x must be dense and 16-byte aligned")
     _need(out_dtype == torch.bfloat16 or (out_dtype == torch.float32 and not glu), "32-bit output comes without the gate")
     _check_squares(squares, M)
+    _need(unit is None or (glu and squares is None and unit[0] in GLU_ACTIVATIONS), lambda: f"a unit {unit} comes with the gate and a plain x")
     out = _gated_output(M, N // 2, x.device) if glu else torch.empty((M, N), dtype=out_dtype, device=x.device)
     _run("gemm_rows64", library().ts_gemm_rows64_bf16(
-        _ptr(out), _ptr(x), _ptr(packed), M, N, K, x.stride(0), out.stride(0), int(glu), int(out_dtype == torch.float32),
-        _ptr(squares), 0 if squares is None else squares.shape[1], float(eps), _stream()))
+        _ptr(out), _ptr(x), _ptr(packed), M, N, K, x.stride(0), out.stride(0), _unit_code(glu, unit), int(out_dtype == torch.float32),
+        _ptr(squares), 0 if squares is None else squares.shape[1], float(eps),
+        *((0.0, 0.0, 0.0) if unit is None else map(float, unit[1:])), _stream()))
     return out
 
 

@@ -7,7 +7,7 @@ import torch
 
 from tinyserve_llm_amd.ops import hip
 from tinyserve_llm_amd.parts.base import FeedForward, ParamSpec, StepContext, register
-from tinyserve_llm_amd.parts.linear import linear, streaming_copy
+from tinyserve_llm_amd.parts.linear import few_rows_unit, linear, streaming_copy
 
 
 @register("feed_forward", "gated_mlp")
@@ -117,13 +117,14 @@ class CappedGLU(FeedForward):
         return sum(c.nbytes() for c in (self.gate_up_packed, self.down_packed) if c is not None)
 
     def forward(self, x: torch.Tensor, ctx: StepContext) -> torch.Tensor:
-        if (hip.many_rows_products() == "library" and x.is_cuda and hip.glu_takes(x, self.gate_up)
-                and hip.many_rows(x, self.gate_up, self.gate_up_packed)):
+        unit = few_rows_unit(x, self.gate_up, self.gate_up_packed, self.down, (self.activation, self.limit, self.slope, self.up_shift))
+        if unit is None and (hip.many_rows_products() == "library" and x.is_cuda and hip.glu_takes(x, self.gate_up)
+                             and hip.many_rows(x, self.gate_up, self.gate_up_packed)):
             # many rows: the unit rides on the product's way out and the 32-bit sums stay where they are made
             unit = hip.gemm_glu(x, self.gate_up, self.activation, self.limit, self.slope, self.up_shift)
-            return linear(unit, self.down, out_dtype=torch.float32, packed=self.down_packed)
-        sums = linear(x, self.gate_up, out_dtype=torch.float32, packed=self.gate_up_packed)
-        unit = hip.capped_glu(sums, self.limit, self.slope, self.up_shift, x.dtype, activation=self.activation)
+        if unit is None:
+            sums = linear(x, self.gate_up, out_dtype=torch.float32, packed=self.gate_up_packed)
+            unit = hip.capped_glu(sums, self.limit, self.slope, self.up_shift, x.dtype, activation=self.activation)
         return linear(unit, self.down, out_dtype=torch.float32, packed=self.down_packed)
 
 

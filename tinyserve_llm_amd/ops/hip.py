@@ -10,6 +10,7 @@ from __future__ import annotations
 
 import contextlib
 import ctypes
+import functools
 import threading
 
 import torch
@@ -259,21 +260,20 @@ def _check_cache(k_cache: torch.Tensor, v_cache: torch.Tensor, dtype: torch.dtyp
     """A layer's caches are addressed as [pages, page_size, kv_heads, head_dim]. Keys: head_dim
     dense, the other three strided in any order. Values: all four strided in any order (the
     engine's pools keep a head's slots of one dimension together, i.e. pages transposed)."""
-    for name, c in (("key", k_cache), ("value", v_cache)):
-        _need(c.dim() == 4 and c.shape[2] == nkv and c.shape[3] == hd,
-              lambda: f"{name} cache view must be [pages, page_size, {nkv}, {hd}], got {tuple(c.shape)}")
-        _need(c.dtype == dtype, "cache and activations differ in storage type")
-        # no two elements may overlap: sort the strides and check each spans the dimensions below it
+    ks, vs, shape = k_cache.stride(), v_cache.stride(), k_cache.shape
+    _need(len(shape) == 4 and shape[2] == nkv and shape[3] == hd and k_cache.dtype == dtype and v_cache.dtype == dtype and v_cache.shape == shape,
+          lambda: f"key and value cache views must be {dtype} [pages, page_size, {nkv}, {hd}], got {k_cache.dtype} {tuple(k_cache.shape)} "
+                  f"and {v_cache.dtype} {tuple(v_cache.shape)}")
+    # no two elements may overlap: sort the strides and check each spans the dimensions below it
+    for name, strides in (("key", ks), ("value", vs)):
         span = 1
-        for stride, size in sorted(zip(c.stride(), c.shape)):
+        for stride, size in sorted(zip(strides, shape)):
             if size > 1:
-                _need(stride >= span, lambda: f"{name} cache elements overlap")
+                if stride < span:
+                    raise KernelError(f"{name} cache elements overlap")
                 span = stride * size
-    _need(k_cache.shape == v_cache.shape, "key and value caches differ in shape")
-    _need(k_cache.stride(3) == 1, "head_dim must be contiguous in the key cache")
-    itemsize = k_cache.element_size()
-    _need(all((k_cache.stride(i) * itemsize) % 16 == 0 for i in range(3)) and k_cache.data_ptr() % 16 == 0,
-          "key rows must be 16-byte aligned")
+    _need(ks[3] == 1, "head_dim must be contiguous in the key cache")
+    _need(((ks[0] | ks[1] | ks[2]) * k_cache.element_size()) % 16 == 0 and k_cache.data_ptr() % 16 == 0, "key rows must be 16-byte aligned")
 
 
 def _page_run(pages_per_entry: int) -> int:
@@ -395,12 +395,13 @@ def decode_plan(num_tokens: int, nkv: int, group: int, hd: int, capacity: int) -
 
 def decode_kernel_takes(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor) -> bool:
     """Whether the matrix-core decode kernel serves these operands (else the wave kernel does)."""
-    nh, hd = q.shape[1], q.shape[2]
-    nkv, page = k_cache.shape[2], k_cache.shape[1]
-    return (q.dtype == torch.bfloat16 and hd in DECODE_HEAD_DIMS and nh // nkv <= 16 and (nh // nkv) * hd <= 2048
-            and page % 8 == 0 and v_cache.stride(1) == 1
-            and all(st % 8 == 0 for st in (*k_cache.stride()[:3], v_cache.stride(0), v_cache.stride(2), v_cache.stride(3)))
-            and v_cache.data_ptr() % 16 == 0)
+    _, nh, hd = q.shape
+    _, page, nkv, _ = k_cache.shape
+    if not (q.dtype == torch.bfloat16 and hd in DECODE_HEAD_DIMS and nh // nkv <= 16 and (nh // nkv) * hd <= 2048 and page % 8 == 0):
+        return False
+    k0, k1, k2, _ = k_cache.stride()
+    v0, v1, v2, v3 = v_cache.stride()
+    return v1 == 1 and (k0 | k1 | k2 | v0 | v2 | v3) % 8 == 0 and v_cache.data_ptr() % 16 == 0
 
 
 def paged_attention_decode(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, block_tables: torch.Tensor,
@@ -749,6 +750,33 @@ def paged_attention_prefill(q: torch.Tensor, k_cache: torch.Tensor, v_cache: tor
     return out
 
 
+def _prefill_plan(q: torch.Tensor, k_cache: torch.Tensor, ctx, decode_ok: bool) -> tuple:
+    """How a step's rows are dealt to the matrix-core kernels, from its lengths and the heads' sizes: (leading one-token
+    requests, which go to the split-key kernel; tokens per tile; waves; tiles; chunks; keys per chunk). Every layer of one kind
+    asks for the same plan, so a step makes it once."""
+    (rows, nh, hd), nkv = q.shape, k_cache.shape[2]
+    key = ("attention_plan", rows, nh, nkv, hd, decode_ok)
+    plan = ctx.scratch.get(key)
+    if plan is not None:
+        return plan
+    cu, starts = ctx.host_cu_seqlens, ctx.host_starts
+    lead = 0
+    while decode_ok and lead + 1 < len(cu) and cu[lead + 1] - cu[lead] == 1:
+        lead += 1
+    walked = sum((cu[i + 1] - cu[i]) * (starts[i] + (cu[i + 1] - cu[i] + 1) / 2) for i in range(lead, len(cu) - 1))
+    mean_keys = walked / max(1, rows - lead)
+    tile_tokens = prefill_tile_tokens(rows - lead, nkv, nh // nkv, hd, mean_keys)
+    waves = prefill_waves(tile_tokens, nh // nkv, hd, mean_keys)
+    tiles = ctx.scratch.get(("attention_tiles", tile_tokens, lead))
+    if tiles is None:
+        flat = attention_tiles(cu, starts, tile_tokens, lead)
+        tiles = torch.tensor(flat, dtype=torch.int32).view(-1, 2).to(q.device, non_blocking=True)
+        ctx.scratch[("attention_tiles", tile_tokens, lead)] = tiles
+    splits, chunk = prefill_splits(tiles.shape[0] * nkv, max(ctx.host_context_lens[lead:], default=0))
+    plan = ctx.scratch[key] = (lead, tile_tokens, waves, tiles, splits, chunk)
+    return plan
+
+
 def paged_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, ctx, space: int,
                     scale: float, window: int = 0, leave_split: bool = False, softcap: float = 0.0,
                     sink: bool = False, sinks: torch.Tensor | None = None, slopes: torch.Tensor | None = None,
@@ -783,30 +811,15 @@ def paged_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
         if ctx.max_query_len == 1 and decode_ok:
             return paged_attention_decode(q, k_cache, v_cache, tables, ctx.seq_of_token, ctx.positions, scale, window,
                                           pages_per_entry=per_entry, leave_split=leave_split and gate is None, gate=gate, **extra)
-        # the one-token requests that lead the step go to the split-key kernel, the rest to the tiles
-        cu = ctx.host_cu_seqlens
-        lead = 0
-        while decode_ok and lead + 1 < len(cu) and cu[lead + 1] - cu[lead] == 1:
-            lead += 1
-        nkv = k_cache.shape[2]
-        walked = sum((cu[i + 1] - cu[i]) * (ctx.host_starts[i] + (cu[i + 1] - cu[i] + 1) / 2) for i in range(lead, len(cu) - 1))
-        mean_keys = walked / max(1, q.shape[0] - lead)
-        tile_tokens = prefill_tile_tokens(q.shape[0] - lead, nkv, q.shape[1] // nkv, q.shape[2], mean_keys)
-        waves = prefill_waves(tile_tokens, q.shape[1] // nkv, q.shape[2], mean_keys)
-        tiles = ctx.scratch.get(("attention_tiles", tile_tokens, lead))
-        if tiles is None:
-            flat = attention_tiles(cu, ctx.host_starts, tile_tokens, lead)
-            tiles = torch.tensor(flat, dtype=torch.int32).view(-1, 2).to(q.device, non_blocking=True)
-            ctx.scratch[("attention_tiles", tile_tokens, lead)] = tiles
+        lead, tile_tokens, waves, tiles, splits, chunk = _prefill_plan(q, k_cache, ctx, decode_ok)
         out = torch.empty_like(q)
         if lead:
             paged_attention_decode(q[:lead], k_cache, v_cache, tables, ctx.seq_of_token[:lead], ctx.positions[:lead],
                                    scale, window, out=out[:lead], pages_per_entry=per_entry,
                                    gate=None if gate is None else gate[:lead], **extra)
-        splits, chunk = prefill_splits(tiles.shape[0] * nkv, max(ctx.host_context_lens[lead:], default=0))
         return paged_attention_prefill(q, k_cache, v_cache, tables, ctx.seq_of_token, ctx.positions, tiles, scale,
                                        window, tile_tokens=tile_tokens, out=out, num_splits=splits, chunk=chunk,
-                                       first_token=cu[lead], waves=waves, pages_per_entry=per_entry, gate=gate, **extra)
+                                       first_token=ctx.host_cu_seqlens[lead], waves=waves, pages_per_entry=per_entry, gate=gate, **extra)
     if general or k_cache.shape[3] != v_cache.shape[3]:
         return paged_attention_general(q, k_cache, v_cache, tables, ctx.seq_of_token, ctx.positions, scale, softcap=softcap,
                                        sink=sink, window=window, pages_per_entry=per_entry, sinks=sinks, slopes=slopes, gate=gate)
@@ -854,7 +867,7 @@ def _gated_output(rows: int, width: int, device) -> torch.Tensor:
     `OPERAND_ROW_SKEW` elements further apart than they are long (the down projection over 8,192 of
     8 rows 10.2 -> 9.8 µs, of 64 rows 15.4 -> 15.0; up to 4 rows the dense form is as fast)."""
     skew = OPERAND_ROW_SKEW if rows >= GATED_SKEW_MIN_ROWS else 0
-    return torch.empty((rows, width + skew), dtype=torch.bfloat16, device=device)[:, :width]
+    return torch.empty_strided((rows, width), (width + skew, 1), dtype=torch.bfloat16, device=device)
 
 
 def _next_norm_outputs(x: torch.Tensor, n: int, parts: int, next_norm, skew: int = 0,
@@ -871,9 +884,10 @@ def _next_norm_outputs(x: torch.Tensor, n: int, parts: int, next_norm, skew: int
     if residual is not None:
         _need(residual.dtype == torch.bfloat16 and residual.shape == (M, n) and residual.is_contiguous(),
               lambda: f"the residual must be bfloat16 [{M}, {n}]")
-    out = PreparedNorm(torch.empty((M, n), dtype=torch.bfloat16, device=x.device),
-                       torch.empty((M, n + skew), dtype=torch.bfloat16, device=x.device)[:, :n],
-                       torch.empty((M, parts), dtype=torch.float32, device=x.device))
+    device = x.device
+    out = PreparedNorm(torch.empty((M, n), dtype=torch.bfloat16, device=device),
+                       torch.empty_strided((M, n), (n + skew, 1), dtype=torch.bfloat16, device=device),
+                       torch.empty((M, parts), dtype=torch.float32, device=device))
     return out, residual, weight
 
 
@@ -1245,6 +1259,12 @@ def rows64_slices(rows: int, n: int, k: int) -> int:
     14.1 against 18.9, 17.3 against 21.6, 27.5 against 38.3; 64 rows 15.5 against 22.0 + 7 at 2,048."""
     if not (ROWS64_SLICED_MIN_ROWS <= rows <= ROWS64_MAX_ROWS) or n % 64 or n >= ROWS64_MIN_WIDTH or k % ROWS64_SLICE_K:
         return 0
+    return _filling_slices(n, k)
+
+
+@functools.lru_cache(maxsize=256)
+def _filling_slices(n: int, k: int) -> int:
+    """The fewest of up to 16 slices of a reduction of `k` whose workgroups of 64 of `n` rows of W fill the chip, else the most."""
     fits = [s for s in range(1, 17) if (k // ROWS64_SLICE_K) % s == 0]
     enough = [s for s in fits if (n // 64) * s >= ROWS64_WORKGROUPS]
     return enough[0] if enough else fits[-1]
@@ -1381,9 +1401,7 @@ def qkv_rope_sliced_slices(x: torch.Tensor, weight: torch.Tensor, head_dim: int,
     rows, (n, k) = x.shape[0], weight.shape
     if not (QKV_SLICED_MIN_ROWS <= rows <= ROWS64_MAX_ROWS) or rows <= qkv_rope_max_rows(k) or n % 64 or k % ROWS64_SLICE_K:
         return 0
-    fits = [s for s in range(1, 17) if (k // ROWS64_SLICE_K) % s == 0]
-    enough = [s for s in fits if (n // 64) * s >= ROWS64_WORKGROUPS]
-    return enough[0] if enough else fits[-1]
+    return _filling_slices(n, k)
 
 
 def qkv_rope_store_sliced(x: torch.Tensor, packed_rope: torch.Tensor, slices: int, cos_sin: torch.Tensor | None,
@@ -1511,15 +1529,30 @@ class StreamingCopies:
         return sum(t.numel() * t.element_size() for t in (self.by16, self.by8) if t is not None)
 
 
-def next_norm_fuses(x: "torch.Tensor | PackedRows8", weight: torch.Tensor, packed: "StreamingCopies | None" = None) -> bool:
-    """Whether `linear_bf16(x, weight, next_norm=...)` has a kernel that leaves a `PreparedNorm`."""
+def _next_norm_route(x: "torch.Tensor | PackedRows8", weight: torch.Tensor, packed: "StreamingCopies | None") -> int:
+    """Where `linear_bf16` gives a product that leaves a `PreparedNorm`: -1 the weight-streaming kernels, n > 0 the shared-x
+    kernel in n slices; 0: no kernel leaves one."""
     if isinstance(x, PackedRows8):          # (made for the 8-row form, which does)
-        return True
+        return -1
     if not (x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and x.is_cuda and x.dim() == 2 and weight.dim() == 2
             and _dense_rows(x) and weight.is_contiguous() and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0):
-        return False
+        return 0
     rows, (n, k) = x.shape[0], weight.shape
-    return skinny8_takes(rows, n, k) or _skinny_serves(rows, n, k) or _sliced_serves(rows, n, k, packed) > 0
+    return _sliced_serves(rows, n, k, packed) or (-1 if skinny8_takes(rows, n, k) or _skinny_serves(rows, n, k) else 0)
+
+
+def next_norm_fuses(x: "torch.Tensor | PackedRows8", weight: torch.Tensor, packed: "StreamingCopies | None" = None) -> bool:
+    """Whether `linear_bf16(x, weight, next_norm=...)` has a kernel that leaves a `PreparedNorm`."""
+    return _next_norm_route(x, weight, packed) != 0
+
+
+def linear_into_norm(x: "torch.Tensor | PackedRows8", weight: torch.Tensor, packed: "StreamingCopies | None", next_norm) -> PreparedNorm | None:
+    """x · weight^T finished into `next_norm` = (residual or None, weight of the norm that follows) by the kernel that
+    `linear_bf16` gives such a product to; None where that kernel leaves no prepared norm."""
+    route = _next_norm_route(x, weight, packed)
+    if route > 0 and x.shape[1] == weight.shape[1]:
+        return gemm_rows64_sliced(x, packed.by16, route, next_norm=next_norm)
+    return linear_bf16(x, weight, torch.bfloat16, packed, next_norm=next_norm) if route else None
 
 
 ROWS64_PLAIN_MAX_WIDTH = 4096  # widest product that takes the sliced kernel when nothing rides on its finishing kernel
@@ -1530,11 +1563,15 @@ def _sliced_serves(rows: int, n: int, k: int, packed: "StreamingCopies | None", 
     `finishing`: the second kernel also makes the residual sum and the next norm's first half, and
     so saves a kernel; without that the parts' trip through memory only pays for narrow products (32
     rows against a weight of 5,120 x 3,072: 14.5 µs, the library 11)."""
-    if packed is None or packed.by16 is None or skinny8_takes(rows, n, k) or _skinny_serves(rows, n, k):
+    if packed is None or packed.by16 is None or not finishing and n > ROWS64_PLAIN_MAX_WIDTH:
         return 0
-    if not finishing and n > ROWS64_PLAIN_MAX_WIDTH:
-        return 0
-    return rows64_slices(rows, n, k)
+    return _sliced_route(rows, n, k)
+
+
+@functools.lru_cache(maxsize=4096)
+def _sliced_route(rows: int, n: int, k: int) -> int:
+    """The slices for a product that neither form of the weight-streaming kernel serves; 0: those do, or the slices do not fit."""
+    return 0 if skinny8_takes(rows, n, k) or _skinny_serves(rows, n, k) else rows64_slices(rows, n, k)
 
 
 def _skinny_serves(rows: int, n: int, k: int) -> bool:

@@ -134,10 +134,11 @@ def linear(x: "torch.Tensor | DeferredNorm | hip.PackedRows8 | hip.SplitAttentio
         residual = then.residual()
         if isinstance(x, DeferredNorm):
             x = x.materialize()
-        if (out_dtype in (None, torch.bfloat16) and then.weight.dtype == torch.bfloat16 and hip.next_norm_fuses(x, weight, packed)
+        if (out_dtype in (None, torch.bfloat16) and then.weight.dtype == torch.bfloat16
                 and (residual is None or (residual.is_contiguous() and residual.dtype == torch.bfloat16))):
-            prepared = hip.linear_bf16(x, weight, torch.bfloat16, packed, next_norm=(residual, then.weight))
-            return DeferredNorm(None, None, then.weight, then.eps, prepared)
+            prepared = hip.linear_into_norm(x, weight, packed, (residual, then.weight))
+            if prepared is not None:
+                return DeferredNorm(None, None, then.weight, then.eps, prepared)
         return DeferredNorm(linear(x, weight, out_dtype, packed=packed), residual, then.weight, then.eps)
     by16 = None if packed is None else packed.by16
     rows = x.rows if isinstance(x, DeferredNorm) else x.shape[0]

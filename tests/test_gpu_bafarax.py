@@ -104,6 +104,36 @@ def test_heads_turn_in_halves_with_an_amplitude_and_reach_the_cache(dtype, shape
         torch.testing.assert_close(v[s // page, s % page].cpu().to(F64), r[i, (H + G) * D:].reshape(G, V), **tol)
 
 
+@pytest.mark.parametrize("shape", [(1, 1, 32, 16, 32, False), (4, 2, 64, 64, 64, False), (8, 2, 64, 32, 48, True), (5, 1, 96, 128, 64, False),
+                                   (2, 1, 256, 256, 256, True), (3, 1, 40, 8, 0, False), (16, 16, 24, 32, 6, True)])
+@pytest.mark.parametrize("few", [1, 3, 23, 127])
+def test_a_step_of_few_tokens_finishes_like_one_of_many(few, shape):
+    """The kernel for few tokens against the one for many on the same rows: every head, tokens that share a workgroup, a last
+    workgroup that is not full. The same 32-bit operations; a product and a sum may be contracted in either order, half a
+    step of the larger term each, beside the root's."""
+    h = hip()
+    H, G, D, V, rot, inter = shape
+    page, many = 16, 1100
+    gen = torch.Generator().manual_seed(few + D)
+    rows = torch.randn(many, (H + G) * D + G * V, generator=gen).to(DEV)
+    positions = torch.randint(0, 90000, (many,), generator=gen, dtype=torch.int32).to(DEV)
+    slots = torch.randperm(70 * page, generator=gen)[:many].to(torch.int32)
+    slots[1::7] = -1                                                       # (rows that leave nothing in the cache)
+    slots = slots.to(DEV)
+    freqs = plain.rotary_frequencies(rot, 9000.0, None)[0].to(DEV) if rot else None
+    found = []
+    for n in (few, many):
+        k, v = paged(70, page, G, D, V, torch.float32)
+        k.zero_(), v.zero_()
+        q = h.qkv_finish(rows[:n], freqs, positions[:n].contiguous(), slots[:n].contiguous(), k, v, H, G, D, V, torch.float32,
+                         interleaved=inter, qk_norm_eps=1e-5 if D != 96 else None, amplitude=1.25)
+        at = slots[:few][slots[:few] >= 0].long()
+        found.append((q[:few], k[at // page, at % page], v[at // page, at % page], k.count_nonzero() if n == few else None))
+    for a, b in zip(found[0][:3], found[1][:3]):
+        torch.testing.assert_close(a, b, rtol=0.0, atol=2.0 ** -21 * 8)
+    assert int(found[0][3]) <= found[0][1].numel(), "nothing but the step's own slots is written"
+
+
 # ---- attention inside chunks with learned sinks -----------------------------------------------------
 
 def chunk_case(dtype, H, G, D, V, page, length, queries, stand_out, scale, chunk, seed=0, sink_value=None, portion_from=None):

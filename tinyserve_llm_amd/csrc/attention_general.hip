@@ -94,9 +94,8 @@ qkv_finish_kernel(TO* __restrict__ q_out, TO* __restrict__ k_cache, TO* __restri
 
 // The same for heads whose sizes are multiples of eight: a thread holds a piece of eight consecutive elements
 // of a head (whole pairs of the interleaved layout; for the halves layout the partner piece is fetched as well), GS threads side by side hold a head (GS the power of two that covers the larger head size),
-// and a thread takes every `slices`-th head of its token: 16 slices for steps of many tokens, so that a token's
-// angles are taken 16 times and not once per head; a slice per head for steps of few, which have threads to spare
-// and no time for one head after the other. All of a thread's loads for a head go out together.
+// and a thread takes every `slices`-th head of its token, so that a token's angles are taken AG_SLICES times and not
+// once per head. All of a thread's loads for a head go out together. (Steps of few tokens: qkv_finish_few_kernel.)
 #define AG_SLICES 16
 template <typename T> struct Piece8;
 template <> struct Piece8<float> {
@@ -234,6 +233,83 @@ qkv_finish_pieces_kernel(TO* __restrict__ q_out, TO* __restrict__ k_cache, TO* _
   }
 }
 
+// The same for steps of few tokens (below the line at which heads are dealt out in AG_SLICES slices): a thread holds one piece of
+// one head of one token. Such a launch is bound by its chain of latencies, and the longest link was the angles: eight sine and
+// cosine calls a thread, one after the other, in code that every wave fetches anew. Here a workgroup's threads take the angles
+// of its tokens once, side by side, and leave them in LDS while the pieces are on their way (5 to 48 tokens: 10 to 11 µs -> 5,
+// about what an empty launch takes).
+#define AG_FEW_ANGLES 640      // (a workgroup of 256 threads spans at most 85 / GS + 2 tokens of three or more heads, of up to 4 GS pairs each)
+template <typename TI, typename TO, int GS>
+__global__ void __launch_bounds__(AG_WAVES * TS_WAVE)
+qkv_finish_few_kernel(TO* __restrict__ q_out, TO* __restrict__ k_cache, TO* __restrict__ v_cache, const TI* __restrict__ qkv,
+                      const double* __restrict__ freqs, const int32_t* __restrict__ positions, const int32_t* __restrict__ slots,
+                      int num_tokens, int nh, int nkv, int hd, int vd_size, int rot, int interleaved, int qk_norm, float qk_eps,
+                      int v_norm, float v_eps, int page_size, int64_t kp, int64_t ks, int64_t kh, int64_t vp, int64_t vs, int64_t vh,
+                      int64_t vd, int with_values, float amplitude, int64_t row, int heads) {
+  static_assert(AG_WAVES * TS_WAVE == 256, "AG_FEW_ANGLES is counted for 256 threads");
+  __shared__ float2 turn_s[AG_FEW_ANGLES];
+  const int per_token = GS * heads, first_thread = (int)blockIdx.x * 256, gid = first_thread + (int)threadIdx.x;   // (below 65,536 x heads / 16)
+  const int piece = gid % GS, h = gid / GS % heads, t_of = gid / per_token;
+  const bool live = t_of < num_tokens;                     // (lanes beyond the step go along for the shuffles and store nothing)
+  const int t = live ? t_of : num_tokens - 1, d0 = 8 * piece, pairs = rot / 2;
+  const bool is_q = h < nh, is_v = h >= nh + nkv;
+  const int size = is_v ? vd_size : hd;
+  const bool mine = d0 < size, turns_here = !is_v && mine && d0 < rot;
+  const TI* src = qkv + (int64_t)t * row + (is_v ? (int64_t)(nh + nkv) * hd + (int64_t)(h - nh - nkv) * vd_size : (int64_t)h * hd) + d0;
+  float x[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, w[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  if (mine) Piece8<TI>::ld(src, x);
+  if (turns_here && !interleaved) Piece8<TI>::ld(src + (d0 < pairs ? pairs : -pairs), w);      // (rot a multiple of 16: whole pieces)
+  const int slot = slots && k_cache && live && !is_q ? slots[t] : -1;
+  const int t_first = first_thread / per_token, t_last = min((first_thread + 255) / per_token, num_tokens - 1);
+  for (int i = threadIdx.x; i < (t_last - t_first + 1) * pairs; i += 256) {
+    const int tl = i / pairs, pair = i - tl * pairs;
+    // the angle in 64-bit, brought to [-pi, pi] before the 32-bit sine and cosine
+    const double angle = (double)positions[t_first + tl] * freqs[pair];
+    const double turns = rint(angle * 0.15915494309189535);
+    float sn, cs;
+    sincosf((float)fma(-turns, 6.283185307179586, angle), &sn, &cs);
+    turn_s[i] = make_float2(cs * amplitude, sn * amplitude);
+  }
+  __syncthreads();
+  const float2* turn = turn_s + (t - t_first) * pairs;
+  float y[8], squares = 0.f;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    float v = x[e];
+    const int d = d0 + e;
+    if (turns_here && d < rot) {
+      const float2 c = turn[interleaved ? d >> 1 : (d < pairs ? d : d - pairs)];
+      const float partner = interleaved ? x[e ^ 1] : w[e];
+      const bool first = interleaved ? !(e & 1) : d0 < pairs;
+      v = first ? v * c.x - partner * c.y : v * c.x + partner * c.y;
+    }
+    y[e] = v;
+    squares = fmaf(v, v, squares);
+  }
+  float scale = 1.0f;
+  if (is_v ? v_norm : qk_norm) {                             // (the same for all threads of a head: they shuffle together)
+#pragma unroll
+    for (int o = GS / 2; o > 0; o >>= 1) squares += __shfl_xor(squares, o, TS_WAVE);
+    scale = 1.0f / sqrtf(squares / (float)size + (is_v ? v_eps : qk_eps));
+  }
+#pragma unroll
+  for (int e = 0; e < 8; ++e) y[e] *= scale;
+  if (!mine || !live) return;
+  if (is_q) {
+    Piece8<TO>::st(q_out + ((int64_t)t * nh + h) * hd + d0, y);
+    return;
+  }
+  if (slot < 0) return;
+  const int page = slot / page_size, off = slot - page * page_size;
+  if (!is_v) {
+    Piece8<TO>::st(k_cache + page * kp + off * ks + (int64_t)(h - nh) * kh + d0, y);
+    return;
+  }
+  TO* dst = v_cache + page * vp + off * vs + (int64_t)(h - nh - nkv) * vh + (int64_t)d0 * vd;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) Num<TO>::st(dst + (int64_t)e * vd, y[e]);
+}
+
 // The values of AG_VTOK consecutive tokens of one key/value head, through LDS: rows are read along their
 // dimensions, normalised, and written with the lanes along the tokens, so that tokens in consecutive slots
 // of a page (whose values lie side by side there, pages holding values transposed) leave in whole segments.
@@ -297,18 +373,23 @@ extern "C" int ts_qkv_finish(void* q_out, void* k_cache, void* v_cache, const vo
   int gs = 4;
   while (gs * 8 < (hd > vd_size ? hd : vd_size)) gs *= 2;
   const int all_heads = nh + (v_tiles ? 1 : 2) * nkv;
-  const int slices = (int64_t)num_tokens * AG_SLICES * gs >= 65536 ? AG_SLICES : all_heads;
+  // few: fewer threads in AG_SLICES slices than the chip has lanes for (256 compute units of 4 waves); a piece of one head a thread then
+  const bool few = (int64_t)num_tokens * AG_SLICES * gs < 65536;
+  const int slices = few ? all_heads : AG_SLICES;
   const int64_t piece_threads = (int64_t)num_tokens * slices * gs;
   const unsigned piece_blocks = (unsigned)((piece_threads + AG_WAVES * TS_WAVE - 1) / (AG_WAVES * TS_WAVE));
 #define QF_ARGS(TI, TO) \
       (TO*)q_out, (TO*)k_cache, (TO*)v_cache, (const TI*)qkv, freqs, positions, slots, num_tokens, nh, nkv, hd, vd_size, rot, \
       interleaved, qk_norm, qk_eps, v_norm, v_eps, page_size, kp, ks, kh, vp, vs, vh, vd, !v_tiles, amplitude, row
+#define QF_PIECES(TI, TO, GS) \
+  if (few) qkv_finish_few_kernel<TI, TO, GS><<<piece_blocks, AG_WAVES * TS_WAVE, 0, stream>>>(QF_ARGS(TI, TO), slices); \
+  else qkv_finish_pieces_kernel<TI, TO, GS><<<piece_blocks, AG_WAVES * TS_WAVE, 0, stream>>>(QF_ARGS(TI, TO), slices)
 #define QF_LAUNCH(TI, TO) \
   if (!pieces) qkv_finish_kernel<TI, TO><<<(unsigned)blocks, AG_WAVES * TS_WAVE, 0, stream>>>(QF_ARGS(TI, TO)); \
-  else if (gs == 4) qkv_finish_pieces_kernel<TI, TO, 4><<<piece_blocks, AG_WAVES * TS_WAVE, 0, stream>>>(QF_ARGS(TI, TO), slices); \
-  else if (gs == 8) qkv_finish_pieces_kernel<TI, TO, 8><<<piece_blocks, AG_WAVES * TS_WAVE, 0, stream>>>(QF_ARGS(TI, TO), slices); \
-  else if (gs == 16) qkv_finish_pieces_kernel<TI, TO, 16><<<piece_blocks, AG_WAVES * TS_WAVE, 0, stream>>>(QF_ARGS(TI, TO), slices); \
-  else qkv_finish_pieces_kernel<TI, TO, 32><<<piece_blocks, AG_WAVES * TS_WAVE, 0, stream>>>(QF_ARGS(TI, TO), slices); \
+  else if (gs == 4) { QF_PIECES(TI, TO, 4); } \
+  else if (gs == 8) { QF_PIECES(TI, TO, 8); } \
+  else if (gs == 16) { QF_PIECES(TI, TO, 16); } \
+  else { QF_PIECES(TI, TO, 32); } \
   if (v_tiles) v_finish_kernel<TI, TO><<<v_grid, AG_WAVES * TS_WAVE, 0, stream>>>( \
       (TO*)v_cache, (const TI*)qkv, slots, num_tokens, row, (int64_t)(nh + nkv) * hd, vd_size, v_norm, v_eps, page_size, vp, vs, vh, vd)
   if (in_dtype == 0 && out_dtype == 0) { QF_LAUNCH(float, float); }
@@ -316,6 +397,7 @@ extern "C" int ts_qkv_finish(void* q_out, void* k_cache, void* v_cache, const vo
   else if (in_dtype == 1 && out_dtype == 1) { QF_LAUNCH(bf16_t, bf16_t); }
   else return TS_BAD_DTYPE;
 #undef QF_LAUNCH
+#undef QF_PIECES
 #undef QF_ARGS
   return ts_check_launch();
 }

@@ -374,6 +374,29 @@ def test_router_grouping_and_experts(dtype, sizes):
     torch.testing.assert_close(out.cpu().to(F64), want, **(dict(atol=1e-4, rtol=1e-4) if dtype == torch.float32 else dict(atol=2e-2, rtol=1e-2)))
 
 
+@pytest.mark.parametrize("sizes", [(3, 64, 40, 5), (2, 128, 131, 300), (5, 192, 260, 700), (1, 320, 512, 257), (70, 64, 96, 900)])
+@pytest.mark.parametrize("tile_rows", [128, 256])
+def test_tiles_through_lds_give_the_narrower_tiles_sums(sizes, tile_rows):
+    """One, two, three and more k-steps, widths that hang over the last workgroup's columns and are no whole 16 bytes, experts
+    without rows, tiles with few rows, more tiles than lanes; an identity expert's pairs are left alone. Every row's sums run
+    over k in ascending order whatever the tile, so they are the same bits."""
+    h = hip()
+    E, K, N, n = sizes
+    gen = torch.Generator().manual_seed(n)
+    x = torch.randn(n, K, generator=gen).bfloat16().to(DEV)
+    w = (torch.randn(E, 2 * N, K, generator=gen) * K ** -0.5).bfloat16().to(DEV)
+    ids = (torch.rand(n, 2, generator=gen) ** 2 * (E + 1)).to(torch.int32).to(DEV)      # (E: the identity expert)
+    taken = ids.view(-1) < E
+    found = []
+    for rows in (64, tile_rows):
+        grouped = h.moe_group(ids, E, rows)
+        found.append([h.moe_gemm(x, w, grouped, torch.bfloat16, per_token=True, glu=(1.2, 1.702, 1.0)),
+                      h.moe_gemm(x, w, grouped, torch.float32, per_token=True),
+                      h.moe_gemm(x, w, grouped, torch.bfloat16, per_token=True, activation="relu2")])
+    for a, b in zip(*found):
+        assert torch.equal(a[taken], b[taken])
+
+
 # ---- whole models through trace replay ---------------------------------------------------------------
 
 LENGTHS = {"P": [1, 23, 97, 200], "Q": [1, 30, 75, 150], "R": [2, 19, 66, 131], "S": [1, 40, 140]}

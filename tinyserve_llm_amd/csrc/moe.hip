@@ -19,7 +19,7 @@
 //     expert's row, times a gate per token if there is one). A choice at or beyond `real` is an identity expert: it
 //     has no matrices, `ts_moe_group` leaves its pairs out of every tile, and its row is the token's input itself.
 // float32 runs 32-bit multiply-adds; bfloat16 operands go through the matrix cores with 32-bit sums.
-#include "common.h"
+#include "lds_loads.h"
 
 #define MOE_THREADS 256
 #define MOE_ROUTE_TOKENS 4
@@ -500,150 +500,155 @@ moe_gemm_stream_kernel(TO* __restrict__ out, const bf16_t* __restrict__ x, const
   moe_store4(orow + c0, y, N - c0);
 }
 
-// Tiles of 128 rows, for steps that give an expert hundreds of rows: both operands go through LDS, fetched a whole
-// 128-byte line of a row by eight threads side by side and read from LDS as the matrix instruction wants them (lane
-// (r, g) of block b and half h: row 16 b + r, elements 32 h + 8 g .. + 7),
-// 64 of K at a time, two k-steps in flight (one in an LDS buffer being multiplied, the next in registers on its way
-// into the other buffer), as in the engine's tiled product for plain matrices; here the rows of x are gathered by
-// pair, the matrix is the tile's expert's, and the rows of y go to their pairs' places. A workgroup of WM x WN
-// waves takes 128 rows by 128 columns (with GLU: 64 gate and 64 up columns, whose sums meet in one lane). K is a
-// multiple of 64.
-template <int WM, int WN, bool GLU, typename TO>
-__global__ void __launch_bounds__(WM * WN * TS_WAVE)
+// Tiles of 128 or 256 rows, for steps that give an expert hundreds of rows: the gated product's scheme (gemm_glu.hip) with the
+// rows of x gathered by pair, the matrix the tile's expert's, and the rows of y stored at their pairs' places. A workgroup of
+// eight waves takes BM rows by 256 rows of W (with GLU 128 gate and 128 up rows, whose sums meet in one lane), 64 of K at a
+// time, K a multiple of 64. What bounds it is the matrix cores and a compute unit's path to memory: operands go from memory
+// straight into LDS, two steps of x and three of W, pieces turned by (row / 2) % 8 against bank conflicts, and loads, operand
+// reads and products are dealt out evenly. 7,300 pairs of 16 experts over 2,048 against 2 x 1,024, and back over 1,024: 71 and
+// 49 µs with tiles of 128 rows, 68 and 42 with 256 (111 and 85 where operands passed through registers on their way to LDS,
+// 128 rows by 128 of W a workgroup, and the dies took eighths of the whole table).
+template <int BM, bool GLU, typename TO>
+__global__ void __launch_bounds__(512, 2)
 moe_gemm_lds_kernel(TO* __restrict__ out, const bf16_t* __restrict__ x, const bf16_t* __restrict__ w,
                     const int32_t* __restrict__ sorted, const int32_t* __restrict__ tiles, int num_tiles, int col_blocks,
                     int src_div, int N, int K, float limit, float slope, float shift, int act) {
-  constexpr int BM = 128, BN = 128;
-  constexpr int THREADS = WM * WN * TS_WAVE;
-  constexpr int FX = BM / 16 * 2, FW = BN / 16 * 2;       // fragments (a kilobyte each) of a k-step of 64
-  constexpr int TM = BM / WM / 16, TN = BN / WN / 16;     // 16 x 16 blocks of a wave
-  constexpr int LX = FX * 64 / THREADS, LW = FW * 64 / THREADS;
-  static_assert(!GLU || WN == 1, "a gate sum and its up sum must meet in one wave");
-  __shared__ moe_u32x4 lds[2][(FX + FW) * 64];
+  constexpr int BN = 256, WM = 2, WN = 4, WAVES = WM * WN, TM = BM / WM / 16, TN = BN / WN / 16, HALF = BN / WN / 2;
+  constexpr int NX = BM / 8 / WAVES, NW = BN / 8 / WAVES;      // kilobytes of a step that a wave fetches
+  constexpr int XS = BM * 128, WS = BN * 128;                  // bytes of a step of x and of W
+  static_assert(NW * 8 == HALF, "a wave fetches gate rows or up rows");
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[2 * XS + 3 * WS];
   // Workgroups go to the chip's eight dies in turn, each die with a cache of its own: die d takes the d-th eighth
   // of the (tile, column block) list, column blocks innermost and tiles in the experts' order, so that the
-  // workgroups a die runs at one time share a few tiles' rows and one expert's columns in its cache.
-  const int per_die = gridDim.x / MOE_DIES;
-  const int item = (blockIdx.x % MOE_DIES) * per_die + blockIdx.x / MOE_DIES;
-  if (item >= num_tiles * col_blocks) return;
+  // workgroups a die runs at one time share a few tiles' rows and one expert's columns in its cache. The eighths are those
+  // of the tiles that hold rows, which lead the table: it is made for the worst case, and eighths of all of it leave two
+  // of the eight dies without work (the products above then take 98 and 63 µs with tiles of 128 rows).
+  const int lane = threadIdx.x % TS_WAVE, r = lane % 16, g = lane / 16;
+  int used = 0;
+  for (int t0 = 0; t0 < num_tiles; t0 += TS_WAVE) used += __popcll(__ballot(t0 + lane < num_tiles && tiles[3 * min(t0 + lane, num_tiles - 1) + 2] > 0));
+  const int per_die = (used * col_blocks + MOE_DIES - 1) / MOE_DIES, turn = blockIdx.x / MOE_DIES;
+  const int item = __builtin_amdgcn_readfirstlane((blockIdx.x % MOE_DIES) * per_die + turn);
+  if (turn >= per_die || item >= used * col_blocks) return;
   const int tile = item / col_blocks;
   const int rows = tiles[3 * tile + 2];
-  if (rows == 0) return;
   const int e = tiles[3 * tile], first = tiles[3 * tile + 1];
-  // (with GLU a workgroup's 128 columns of the product are 64 columns of y)
   const int n0 = (item - tile * col_blocks) * (GLU ? BN / 2 : BN);
-  const int t = threadIdx.x, lane = t % TS_WAVE, r = lane % 16, g = lane / 16;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / TS_WAVE), wm = wave % WM, wn = wave / WM;
-  const bf16_t* we = w + (int64_t)e * (GLU ? 2 : 1) * N * K;
-  const bf16_t* xp[LX];
-  const bf16_t* wp[LW];
-  // (fetching: eight threads side by side take the eight 16-byte pieces of one row's 64 k, a whole line of memory)
-  int place[LX > LW ? LX : LW];
+  const int wave = wave_index(), wm = wave % WM, wn = wave / WM;
+  const int steps = K / 64;
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_ptr_t)lds;
+
+  // ---- the loading side (a row past the tile's, or a column past the matrix's last: the last one again) ----
+  const bf16_t* xp[NX];
+  uint32_t woff[NW];
 #pragma unroll
-  for (int i = 0; i < LX; ++i) {
-    const int row = (t + THREADS * i) / 8, piece = (t + THREADS * i) % 8;
-    const int pair = sorted[first + min(row, rows - 1)];
-    xp[i] = x + (int64_t)(pair / src_div) * K + 8 * piece;
+  for (int q = 0; q < NX; ++q) {
+    const int at = (wave * NX + q) * 8 + lane / 8;
+    xp[q] = x + (int64_t)(sorted[first + min(at, rows - 1)] / src_div) * K + ((lane % 8) ^ ((at >> 1) & 7)) * 8;
   }
+  const int ups = GLU && wave % 2 ? N : 0;                     // (odd waves fetch up rows)
+  const __amdgpu_buffer_rsrc_t rsrc_w = load_base(w + ((int64_t)e * (GLU ? 2 : 1) * N + n0 + ups) * K);
 #pragma unroll
-  for (int i = 0; i < LW; ++i) {
-    const int row = (t + THREADS * i) / 8, piece = (t + THREADS * i) % 8;
-    int col = row;
-    if (GLU) col = min(n0 + col % (BN / 2), N - 1) + (col >= BN / 2 ? N : 0);
-    else col = min(n0 + col, N - 1);
-    wp[i] = we + (int64_t)col * K + 8 * piece;
+  for (int q = 0; q < NW; ++q) {
+    const int at = (wave * NW + q) * 8 + lane / 8;
+    woff[q] = (uint32_t)(min(GLU ? at / (2 * HALF) * HALF + at % HALF : at, N - 1 - n0) * K * 2) + ((lane % 8) ^ ((at >> 1) & 7)) * 16;
   }
-  // (in LDS row R keeps its piece c at place c ^ (R % 8): the eight threads that store a row fill its 128 bytes, and the
-  // lanes that read one piece of eight rows in a row for the matrix instruction find them in eight different places)
-  static_assert(LX == LW, "as many pieces of x as of the matrix a thread");
+  const uint32_t xfirst = lds0 + wave * NX * 1024, wfirst = lds0 + 2 * XS + wave * NW * 1024;
+  uint32_t xslot = xfirst, wslot = wfirst;
+  int xk = 0, wk = 0;
+  auto fetch_x = [&]() {
 #pragma unroll
-  for (int i = 0; i < LX; ++i) {
-    const int row = (t + THREADS * i) / 8, piece = (t + THREADS * i) % 8;
-    place[i] = row * 8 + (piece ^ (row & 7));
-  }
-  moe_u32x4 sx0[LX], sw0[LW], sx1[LX], sw1[LW];
-  moe_f32x4 acc[TN][TM];
+    for (int q = 0; q < NX; ++q) row_to_lds(xp[q] + xk * 64, xslot + q * 1024);
+  };
+  auto fetch_w = [&]() {
+#pragma unroll
+    for (int q = 0; q < NW; ++q) load_to_lds(rsrc_w, wslot + q * 1024, woff[q], (uint32_t)wk * 128);
+  };
+  // (past the last step its loads are made again: a few, in bounds and never read)
+  auto next_x = [&]() { xslot = xslot == xfirst ? xfirst + XS : xfirst, xk = min(xk + 1, steps - 1); };
+  auto next_w = [&]() { wslot = wslot == wfirst + 2 * WS ? wfirst : wslot + WS, wk = min(wk + 1, steps - 1); };
+
+  // ---- the multiplying side ----
+  const uint32_t rd0 = (uint32_t)(r * 128 + (g ^ (r >> 1)) * 16), rd1 = rd0 ^ 64;      // a step's two halves of K
+  const unsigned char* rx = lds + wm * TM * 2048;
+  const unsigned char* rw = lds + 2 * XS + wn * TN * 2048;
+  uint32_t xc = 0, wc = 0;
+  u32x4_t fw[2][TN], fx[2][TM];
+  float4_t acc[TN][TM];
 #pragma unroll
   for (int j = 0; j < TN; ++j)
 #pragma unroll
-    for (int i = 0; i < TM; ++i) acc[j][i] = (moe_f32x4){0.f, 0.f, 0.f, 0.f};
-#define MOE_FETCH(S, k0)                                                                                  \
-  do {                                                                                                    \
-    _Pragma("unroll") for (int i = 0; i < LX; ++i) sx##S[i] = *(const moe_u32x4*)(xp[i] + (k0));          \
-    _Pragma("unroll") for (int i = 0; i < LW; ++i) sw##S[i] = *(const moe_u32x4*)(wp[i] + (k0));          \
-  } while (0)
-#define MOE_STASH(S)                                                                                      \
-  do {                                                                                                    \
-    _Pragma("unroll") for (int i = 0; i < LX; ++i) lds[S][place[i]] = sx##S[i];                           \
-    _Pragma("unroll") for (int i = 0; i < LW; ++i) lds[S][FX * 64 + place[i]] = sw##S[i];                 \
-  } while (0)
-#define MOE_MULTIPLY(S)                                                                                   \
-  _Pragma("unroll") for (int h = 0; h < 2; ++h) {                                                         \
-    moe_u32x4 fx[TM], fw[TN];                                                                             \
-    _Pragma("unroll") for (int i = 0; i < TM; ++i)                                                        \
-      fx[i] = lds[S][((wm * TM + i) * 16 + r) * 8 + ((4 * h + g) ^ (r & 7))];                             \
-    _Pragma("unroll") for (int j = 0; j < TN; ++j)                                                        \
-      fw[j] = lds[S][FX * 64 + ((wn * TN + j) * 16 + r) * 8 + ((4 * h + g) ^ (r & 7))];                   \
-    _Pragma("unroll") for (int j = 0; j < TN; ++j)                                                        \
-      _Pragma("unroll") for (int i = 0; i < TM; ++i) acc[j][i] = moe_mfma(fw[j], fx[i], acc[j][i]);       \
-  }
-  const int steps = K / 64;
-  MOE_FETCH(0, 0);
-  if (steps == 1) {
-    MOE_STASH(0);
-    __syncthreads();
+    for (int i = 0; i < TM; ++i) acc[j][i] = (float4_t){0.f, 0.f, 0.f, 0.f};
+  fetch_x(), next_x();
+  fetch_w(), next_w();
+  fetch_w(), next_w();
+  fetch_x(), next_x();
+  wait_for<NW + NX>();
+  __builtin_amdgcn_s_barrier();
+#define MOE_READ(S, RD)                                                                                        \
+  _Pragma("unroll") for (int j = 0; j < TN; ++j) fw[S][j] = *(const u32x4_t*)(rw + (RD + wc) + j * 2048);      \
+  _Pragma("unroll") for (int i = 0; i < TM; ++i) fx[S][i] = *(const u32x4_t*)(rx + (RD + xc) + i * 2048);
+#define MOE_MULTIPLY(S)                                                                                        \
+  _Pragma("unroll") for (int i = 0; i < TM; ++i)                                                               \
+      _Pragma("unroll") for (int j = 0; j < TN; ++j) acc[j][i] = mfma32v(fw[S][j], fx[S][i], acc[j][i]);
+// the order of a half step: TM TN products, among their first two thirds the TM + TN operand reads, among all the loads
+#define MOE_DEAL(LOADS)                                                                                        \
+  _Pragma("unroll") for (int q = 0; q < TM * TN; ++q) {                                                        \
+    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                                                         \
+    if ((q + 1) * (TM + TN) * 3 / 2 / (TM * TN) > q * (TM + TN) * 3 / 2 / (TM * TN)) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0); \
+    if ((q + 1) * LOADS / (TM * TN) > q * LOADS / (TM * TN)) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0); \
+  }                                                                                                            \
+  __builtin_amdgcn_sched_barrier(0);
+  MOE_READ(0, rd0)
+  for (int s = 0; s < steps; ++s) {
+    __builtin_amdgcn_sched_barrier(0);
+    fetch_w();
+    MOE_READ(1, rd1)
     MOE_MULTIPLY(0)
-  } else {
-    MOE_FETCH(1, 64);
-    MOE_STASH(0);
-    __syncthreads();
-    int s = 0;
-    for (; s + 3 < steps; s += 2) {
-      MOE_FETCH(0, 64 * (s + 2));
-      MOE_MULTIPLY(0)
-      MOE_STASH(1);
-      __syncthreads();
-      MOE_FETCH(1, 64 * (s + 3));
-      MOE_MULTIPLY(1)
-      MOE_STASH(0);
-      __syncthreads();
-    }
-    // two or three steps are left: step s in buffer 0, step s + 1 in register set 1
-    if (steps - s == 3) {
-      MOE_FETCH(0, 64 * (s + 2));
-      MOE_MULTIPLY(0)
-      MOE_STASH(1);
-      __syncthreads();
-      MOE_MULTIPLY(1)
-      MOE_STASH(0);
-      __syncthreads();
-      MOE_MULTIPLY(0)
-    } else {
-      MOE_MULTIPLY(0)
-      MOE_STASH(1);
-      __syncthreads();
-      MOE_MULTIPLY(1)
-    }
+    MOE_DEAL(NW)
+    next_w();
+    xc = XS - xc;
+    wc = wc == 2 * WS ? 0 : wc + WS;
+    // every wave has read the last of this step's x and of W (so their places may be filled), and the next step has
+    // landed: x was asked for half a step later than W, so all but the newest NW loads are done
+    wait_for<NW, 0>();
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    fetch_x();
+    MOE_READ(0, rd0)
+    MOE_MULTIPLY(1)
+    MOE_DEAL(NX)
+    next_x();
   }
-#undef MOE_FETCH
-#undef MOE_STASH
+#undef MOE_READ
 #undef MOE_MULTIPLY
+#undef MOE_DEAL
   // lane (r, g) of block (j, i): row 16 (wm TM + i) + r of the tile, columns .. + 4 g .. + 3
+  int pair[TM];
+#pragma unroll
+  for (int i = 0; i < TM; ++i) pair[i] = sorted[first + min((wm * TM + i) * 16 + r, rows - 1)];
 #pragma unroll
   for (int i = 0; i < TM; ++i) {
-    const int m = (wm * TM + i) * 16 + r;
-    if (m >= rows) continue;
-    TO* orow = out + (int64_t)sorted[first + m] * N;
+    TO* orow = out + (int64_t)pair[i] * N;
+    const bool mine = (wm * TM + i) * 16 + r < rows;
     if constexpr (GLU) {
+      const int c0 = n0 + wn * HALF;
+      float y[TN / 2][4];
 #pragma unroll
-      for (int j = 0; j < TN / 2; ++j) {
-        const int n = n0 + j * 16 + 4 * g;
-        float y[4];
+      for (int j = 0; j < TN / 2; ++j)
 #pragma unroll
-        for (int c = 0; c < 4; ++c) y[c] = moe_unit(acc[j][i][c], acc[j + TN / 2][i][c], limit, slope, shift);
-        moe_store4(orow + n, y, N - n);
+        for (int c = 0; c < 4; ++c) y[j][c] = moe_unit(acc[j][i][c], acc[j + TN / 2][i][c], limit, slope, shift);
+      if (sizeof(TO) == 2 && N % 8 == 0 && ((uintptr_t)out & 15) == 0) {
+        // lanes g and g ^ 1 exchange halves so that each has eight columns in a row
+        static_assert(TN == 4, "two blocks of columns a wave");
+        const auto lo = __builtin_amdgcn_permlane16_swap(pack_bf16(y[0][0], y[0][1]), pack_bf16(y[1][0], y[1][1]), false, false);
+        const auto hi = __builtin_amdgcn_permlane16_swap(pack_bf16(y[0][2], y[0][3]), pack_bf16(y[1][2], y[1][3]), false, false);
+        const int c = c0 + (g & 1) * 16 + (g >> 1) * 8;
+        if (mine && c < N) *(u32x4_t*)((bf16_t*)orow + c) = (u32x4_t){lo[0], hi[0], lo[1], hi[1]};
+      } else if (mine) {
+#pragma unroll
+        for (int j = 0; j < TN / 2; ++j) moe_store4(orow + c0 + j * 16 + 4 * g, y[j], N - (c0 + j * 16 + 4 * g));
       }
-    } else {
+    } else if (mine) {
 #pragma unroll
       for (int j = 0; j < TN; ++j) {
         const int n = n0 + (wn * TN + j) * 16 + 4 * g;
@@ -652,6 +657,7 @@ moe_gemm_lds_kernel(TO* __restrict__ out, const bf16_t* __restrict__ x, const bf
       }
     }
   }
+  wait_for<0>();      // what was fetched beyond the end lands before the workgroup's LDS is another's
 }
 
 extern "C" int ts_moe_gemm(void* out, int out_dtype, const void* x, int x_dtype, const void* w, const int32_t* sorted,
@@ -659,21 +665,25 @@ extern "C" int ts_moe_gemm(void* out, int out_dtype, const void* x, int x_dtype,
                            float slope, float shift, int act, hipStream_t stream) {
   if (max_tiles <= 0) return TS_OK;
   if (act < 0 || act > 1 || (glu && act)) return TS_BAD_SHAPE;
-  if (N <= 0 || K <= 0 || src_div <= 0 || (tile_rows != 16 && tile_rows != 64 && tile_rows != 128)) return TS_BAD_SHAPE;
+  if (N <= 0 || K <= 0 || src_div <= 0 || (tile_rows != 16 && tile_rows != 64 && tile_rows != 128 && tile_rows != 256)) return TS_BAD_SHAPE;
   const bool mfma = x_dtype == 1 && K % 32 == 0 && (((uintptr_t)x | (uintptr_t)w) & 15) == 0;
-  if (tile_rows == 128) {
-    if (!mfma || K % 64) return TS_BAD_SHAPE;
-    const int col_blocks = glu ? (N + 63) / 64 : (N + 127) / 128;
+  if (tile_rows >= 128) {
+    if (!mfma || K % 64 || K > (1 << 22)) return TS_BAD_SHAPE;                 // (byte offsets within 256 rows of W)
+    const int col_blocks = glu ? (N + 127) / 128 : (N + 255) / 256;
     const int64_t items = (int64_t)max_tiles * col_blocks;
     if (items > 0x3fffffff) return TS_BAD_SHAPE;
     const unsigned grid = (unsigned)((items + MOE_DIES - 1) / MOE_DIES * MOE_DIES);
-#define MOE_LDS(WM, WN, GLU, TO) \
-    moe_gemm_lds_kernel<WM, WN, GLU, TO><<<grid, WM * WN * TS_WAVE, 0, stream>>>((TO*)out, (const bf16_t*)x, (const bf16_t*)w, sorted, \
-                                                                                  tiles, max_tiles, col_blocks, src_div, N, K, limit, slope, shift, act)
-    if (glu && out_dtype == 1) MOE_LDS(4, 1, true, bf16_t);
-    else if (!glu && out_dtype == 0) MOE_LDS(2, 2, false, float);
-    else if (!glu && out_dtype == 1) MOE_LDS(2, 2, false, bf16_t);
+#define MOE_LDS(BM, GLU, TO) \
+    moe_gemm_lds_kernel<BM, GLU, TO><<<grid, 512, 0, stream>>>((TO*)out, (const bf16_t*)x, (const bf16_t*)w, sorted, tiles, max_tiles, \
+                                                               col_blocks, src_div, N, K, limit, slope, shift, act)
+#define MOE_LDS_ROWS(GLU, TO) \
+    if (tile_rows == 256) MOE_LDS(256, GLU, TO); \
+    else MOE_LDS(128, GLU, TO)
+    if (glu && out_dtype == 1) { MOE_LDS_ROWS(true, bf16_t); }
+    else if (!glu && out_dtype == 0) { MOE_LDS_ROWS(false, float); }
+    else if (!glu && out_dtype == 1) { MOE_LDS_ROWS(false, bf16_t); }
     else return TS_BAD_DTYPE;
+#undef MOE_LDS_ROWS
 #undef MOE_LDS
     return ts_check_launch();
   }

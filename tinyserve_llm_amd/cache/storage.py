@@ -140,5 +140,5 @@ class KVStorage:
             t[dst_slot].copy_(t[src_slot])
 
     def reset_state(self, slot: int) -> None:
-        for t in self.states.values():
-            t[slot].zero_()
+        if self.states:            # (one launch for all of a request's states)
+            torch._foreach_zero_([t[slot] for t in self.states.values()])

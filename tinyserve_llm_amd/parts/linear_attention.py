@@ -115,6 +115,10 @@ class ShiftedDecayRecurrence(Mixer):
         # S of every head, then the previous token's input row
         return StateSpec((self.size * self.head_dim + self.hidden_size,), torch.float32)
 
+    def widest_activation(self) -> int:
+        # (a long portion's chunks of 64 tokens each keep a state; the projections of GatedLinearAttention are wider than that)
+        return max(super().widest_activation(), -(-self.size * self.head_dim // hip.SSD_CHUNK))
+
     def keep_streaming_copies(self) -> int:
         self.packed = {n: streaming_copy(getattr(self, n)) for n in ("r", "k", "v", "g", "o")}
         return sum(c.nbytes() for c in self.packed.values() if c is not None)

@@ -238,6 +238,22 @@ def test_token_shift_reads_the_kept_row_and_leaves_the_last(dtype):
     assert torch.equal(kept[[0, 3, 5]], before[[0, 3, 5]])
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("n,width,mixes", [(65540, 8, 1), (7400, 72, 5), (523, 1024, 3), (259, 2056, 5)])
+def test_token_shift_in_whole_pieces(dtype, n, width, mixes):
+    """Many rows of whole 16-byte pieces take eight elements a thread; kept rows that begin elsewhere take one. The same bits."""
+    from types import SimpleNamespace
+    h = hip()
+    mu = torch.rand(mixes, width, device=DEV)
+    wide = torch.randn(6, width + 8, device=DEV)
+    apart = torch.empty(6, width + 8, device=DEV)
+    apart[:, 3:3 + width] = wide[:, 4:4 + width]
+    x, _ = rounded(torch.randn(n, width), dtype)
+    ints = lambda t: torch.tensor(t, dtype=torch.int32, device=DEV)
+    ctx = SimpleNamespace(cu_seqlens=ints([0, 1, n - 7, n]), seq_of_token=ints([0] + [1] * (n - 8) + [2] * 7), state_slots=ints([4, 1, 2]))
+    assert torch.equal(h.token_shift(x, mu, wide[:, 4:4 + width], ctx), h.token_shift(x, mu, apart[:, 3:3 + width], ctx))
+
+
 @pytest.mark.parametrize("shared", [True, False])
 def test_heads_norm_weight_and_silu_gate(shared):
     h = hip()

@@ -2176,10 +2176,10 @@ class ExpertTiles:
 
 
 def moe_tile_rows(pairs: int, experts: int, dtype: torch.dtype, k_sizes: "tuple[int, ...]" = ()) -> int:
-    """Rows of a tile for a step of `pairs` (token, expert) pairs: the wide tile where the matrix-core kernel
-    runs (bfloat16, reductions that are multiples of 32) and an expert has that many rows on average, so
-    that an expert's matrix is read once per 64 rows and not once per 16."""
-    if dtype == torch.bfloat16 and all(k % 64 == 0 for k in k_sizes) and pairs >= MOE_LDS_FROM * experts:
+    """Rows of a tile for a step of `pairs` (token, expert) pairs whose products run over `k_sizes`: wider tiles where a
+    matrix-core kernel runs (bfloat16; reductions that are multiples of 64 through LDS, of 32 otherwise) and an expert has
+    enough rows on average, so that its matrix is read once per tile of them and not once per 16."""
+    if dtype == torch.bfloat16 and all(k % 64 == 0 for k in k_sizes) and pairs >= (MOE_LDS_FROM if k_sizes else MOE_LDS_TILE_ROWS) * experts:
         wide = pairs >= MOE_LDS_WIDE_FROM * experts and min(k_sizes, default=0) >= MOE_LDS_WIDE_MIN_K
         return MOE_LDS_WIDE_TILE_ROWS if wide else MOE_LDS_TILE_ROWS
     wide = dtype == torch.bfloat16 and all(k % 32 == 0 for k in k_sizes) and pairs >= MOE_WIDE_TILE_ROWS * experts

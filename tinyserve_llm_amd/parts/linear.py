@@ -3,7 +3,8 @@
 float32 runs the engine's own exact kernel (32-bit multiply-adds, ascending k, independent of the
 batch). bfloat16 uses the weight-streaming kernel for few rows and the vendor matrix library for
 many, as the reference uses a vendor library for every projection (or, if
-`hip.many_rows_products("tiled")` says so, the engine's own tiled kernel, which is slower).
+`hip.many_rows_products("tiled")` says so, the engine's own tiled kernel, which is slower); a
+gate|up projection of many rows goes to the engine's own kernel, which takes the unit along.
 
 With few rows a step's time goes to launching kernels and to waiting for memory, so what
 precedes or follows a projection can ride along with it: a norm may hand its input over as a

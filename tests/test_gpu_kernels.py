@@ -626,6 +626,34 @@ def test_gated_unit_of_few_rows(m, f, k, unit):
         hip().gemm_skinny(x, w, unit=unit)
 
 
+@pytest.mark.parametrize("unit", [("sigmoid", 0.0, 1.0, 0.0), ("sigmoid", 7.0, 1.702, 1.0), ("relu", 0.0, 1.0, 0.0), ("gelu_tanh", 0.0, 1.0, 0.0),
+                                  ("silu_rounded", 0.0, 1.0, 0.0)])
+def test_gated_units_at_the_ends_of_their_range(unit):
+    """Gates that are infinite, no number, zero, or so far below zero that the sigmoid vanishes: a product that takes the unit along
+    stores what the unit's own kernel makes of the same 32-bit sums (each a single term here, so exact), bit for bit."""
+    from tinyserve_llm_amd.parts import linear as lin
+    form, *numbers = unit
+    f, k = 4096, 1024
+    left = torch.tensor([1.0, -1.0, 2.0 ** 100, -2.0 ** 100, 3e38, -3e38, math.nan]).bfloat16().float()
+    gates = torch.tensor([0.0, 0.5, 5.0, 20.0, 60.0, 84.0, 87.0, 88.0, 89.0, 90.0, 96.0, 104.0, 130.0, 1e5, 1e30, 3e38]).bfloat16().float().repeat(f // 16)
+    ups = torch.tensor([1.0, -3.0, 0.0]).repeat(f)[:f]
+    for rows in (7, 40):
+        x, w = torch.zeros(rows, k), torch.zeros(2 * f, k)
+        x[:, 0], x[:, 1] = left.repeat(6)[:rows], 1.0
+        w[:f, 0], w[f:, 1] = gates, ups
+        sums = torch.cat([x[:, :1] * gates, (x[:, :1] * 0.0) + ups], dim=1).to(dev())
+        x, w = x.bfloat16().to(dev()), w.bfloat16().to(dev())
+        want = hip().silu_mul(sums.bfloat16()) if form == "silu_rounded" else hip().capped_glu(sums, *numbers, torch.bfloat16, activation=form)
+        assert bool(want.isinf().any()) == (numbers[0] == 0.0) and bool(want.isnan().any())
+        found = [hip().gemm_glu(x, w, *unit)]
+        if form != "silu_rounded":
+            few = lin.few_rows_unit(x, w, lin.streaming_copy(w), torch.empty(256, f, dtype=torch.bfloat16, device=dev()), unit)
+            found.append(few.rows() if isinstance(few, hip().PackedRows8) else few)
+        for out in found:
+            assert torch.equal(out.isnan(), want.isnan())
+            assert torch.equal(out.nan_to_num(0.0, math.inf, -math.inf), want.nan_to_num(0.0, math.inf, -math.inf))
+
+
 @pytest.mark.parametrize("m", [1, 3, 8, 16, 17, 32])
 @pytest.mark.parametrize("n,k", [(3072, 2048), (2048, 2048), (16384, 2048), (2048, 8192), (992, 512), (130, 3072), (64, 4096),
                                  (8192, 3072), (8256, 4096)])

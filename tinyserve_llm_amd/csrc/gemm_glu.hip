@@ -5,7 +5,7 @@
 // vendor library's rate (2,048 rows, F 8,192, K 2,048: 1.2 to 1.3 PFLOP/s either way, at the clocks such products hold);
 // what is gained is the trip of the product through memory and the launch that read it again. Measured with the weights
 // coming from memory, against the library's product followed by the unit's kernel: 2,048 rows 120 µs against 134 (bfloat16
-// product) and 171 (32-bit product: 125 with relu, 133 with the sigmoid), 999 rows 59 against 65 and 77, 512 rows 35 against 42,
+// product) and 171 (32-bit product: 125 with relu, 135 with the sigmoid), 999 rows 59 against 65 and 77, 512 rows 35 against 42,
 // 160 rows 23 against 31.
 //
 // A workgroup of 8 waves computes BM rows by BN rows of W (BN / 2 columns of the unit), 64 of K at a time. Slices of x
@@ -23,7 +23,7 @@
 #include "glu_unit.h"
 #include "lds_loads.h"
 
-// The unit's forms (glu_unit.h; the hardware's 2^x and reciprocal throughout would take 10 of 130 µs off the sigmoid form).
+// The unit's forms (glu_unit.h; the hardware's 2^x and reciprocal throughout would take 12 of 135 µs off the sigmoid form).
 template <int ACT> static __device__ __forceinline__ float glu_unit(float g, float u, float limit, float slope, float up_shift) {
   if constexpr (ACT == GLU_SILU_ROUNDED) {          // both branches as a bfloat16 product leaves them
     const uint32_t both = pack_bf16(g, u);

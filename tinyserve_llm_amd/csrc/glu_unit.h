@@ -14,7 +14,5 @@ static __device__ __forceinline__ float glu_capped(int act, float g, float u, fl
   u += up_shift;
   if (act == GLU_RELU) return fmaxf(g, 0.f) * u;
   if (act == GLU_GELU) return 0.5f * g * (1.0f + tanhf(0.7978845608028654f * (g + 0.044715f * g * g * g))) * u;
-  // (g / d for d >= 1: the reciprocal's quotient and one correction, as good as a division here; d stays finite)
-  const float d = 1.0f + fminf(expf(-slope * g), 1e38f), inv = __builtin_amdgcn_rcpf(d), q = g * inv;
-  return fmaf(fmaf(-q, d, g), inv, q) * u;
+  return g / (1.0f + expf(-slope * g)) * u;
 }

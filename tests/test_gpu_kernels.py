@@ -654,6 +654,32 @@ def test_gated_units_at_the_ends_of_their_range(unit):
             assert torch.equal(out.nan_to_num(0.0, math.inf, -math.inf), want.nan_to_num(0.0, math.inf, -math.inf))
 
 
+@pytest.mark.parametrize("m,f,k,along", [(1, 1024, 8192, False), (4, 256, 5120, False), (17, 1024, 4096, False), (32, 4096, 3072, False), (32, 256, 576, True),
+                                         (96, 512, 2048, False), (160, 1024, 4096, False), (160, 512, 512, True), (700, 2048, 1024, True)])
+def test_where_gated_projections_go(m, f, k, along, monkeypatch):
+    """Through the parts: a projection whose unit does not pay to be taken along is the plain product and the unit's kernel."""
+    from tinyserve_llm_amd.parts import linear as lin
+    from tinyserve_llm_amd.parts.mlp import CappedGLU
+    g = gen(m + f + k)
+    x, w = torch.randn(m, k, generator=g).bfloat16().to(dev()), (torch.randn(2 * f, k, generator=g) * k ** -0.5).bfloat16().to(dev())
+    went, plain = [], hip().gemm_glu
+    monkeypatch.setattr(hip(), "gemm_glu", lambda *a, **k: went.append(a[2]) or plain(*a, **k))
+    copies = lin.streaming_copy(w)
+    out = lin.linear(x, w, glu=True, packed=copies)
+    assert went == (["silu_rounded"] if along else [])
+    if not along:
+        assert torch.equal(out, hip().silu_mul(hip().linear_bf16(x, w, torch.bfloat16, copies)))
+    part = CappedGLU(k, f, limit=0.0, slope=1.0, up_shift=0.0, activation="relu")
+    part.gate_up, part.gate_up_packed, part.down = w, copies, torch.eye(f, device=dev()).bfloat16()
+    went.clear()
+    got = part.forward(x, None)
+    if m > 32:
+        assert went == (["relu"] if along else [])
+    if m > 16 and not along:
+        assert went == []
+        assert torch.equal(got, hip().capped_glu(hip().linear_bf16(x, w, torch.float32, copies), 0.0, 1.0, 0.0, torch.bfloat16, activation="relu").float())
+
+
 @pytest.mark.parametrize("m", [1, 3, 8, 16, 17, 32])
 @pytest.mark.parametrize("n,k", [(3072, 2048), (2048, 2048), (16384, 2048), (2048, 8192), (992, 512), (130, 3072), (64, 4096),
                                  (8192, 3072), (8256, 4096)])

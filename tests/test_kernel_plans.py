@@ -129,3 +129,27 @@ def test_which_narrow_products_have_their_reduction_cut_into_slices():
     assert hip._sliced_serves(40, 2048, 8192, None) == 0, "no packed copy: the library"
     assert hip._sliced_serves(24, 5120, 3072, copies) == 3 and hip._sliced_serves(24, 5120, 3072, copies, finishing=False) == 0
     assert hip._sliced_serves(24, 4096, 14336, copies, finishing=False) == 4
+
+
+def test_gated_products_take_the_unit_along_where_that_is_faster():
+    """Both ways were timed at these sizes (rows, unit's width, reduction); the slower one costs 1.1 times the other or more."""
+    apart = [(1, 1024, 8192), (16, 1024, 8192), (17, 8192, 3072), (32, 8192, 3072), (17, 4096, 4096), (128, 3072, 5120), (129, 1024, 2048),
+             (160, 2048, 4096), (512, 1024, 4096), (320, 13824, 5120), (16, 14336, 8192), (65, 1024, 2048)]
+    along = [(1, 1536, 576), (64, 2560, 960), (129, 512, 512), (256, 8192, 3072), (512, 13824, 5120), (1024, 2560, 960), (1024, 8192, 3072),
+             (2048, 1024, 2048), (2048, 8192, 3072), (1024, 14336, 4096)]
+    for rows, width, k in apart:
+        assert not hip.glu_pays(rows, 2 * width, k), (rows, width, k)
+    for rows, width, k in along:
+        assert hip.glu_pays(rows, 2 * width, k), (rows, width, k)
+    # 32-bit branches: the separate unit reads twice as much
+    assert not hip.glu_pays(17, 16384, 2048, 4) and not hip.glu_pays(64, 2048, 1024, 4) and not hip.glu_pays(1024, 10240, 5120, 4)
+    assert hip.glu_pays(256, 16384, 2048, 4) and hip.glu_pays(2048, 16384, 2048, 4) and hip.glu_pays(512, 8192, 2048, 4)
+
+
+def test_gated_product_tiles_follow_the_rounds():
+    assert [hip.glu_plan(m, 16384)[0] for m in (256, 999, 1514, 2048)] == [2, 0, 1, 0]
+    for rows in (1, 128, 129, 300, 5000):
+        for n in (16, 256, 9000):
+            tile, cost = hip.glu_plan(rows, n)
+            bm, bn, us = hip.GLU_TILES[tile]
+            assert cost == us * -(-(-(-rows // bm) * -(-n // bn)) // 256) == min(u * -(-(-(-rows // a) * -(-n // b)) // 256) for a, b, u in hip.GLU_TILES)

@@ -214,20 +214,18 @@ static int launch_glu(GluArgs a, int act, hipStream_t stream) {
 }
 
 // x [M, K], w [2 F, K], y [M, F] bfloat16, 16-byte aligned, rows ldx, ldw, ldy elements apart (multiples of 8); K a
-// multiple of 64, F of 8. act: 0 silu(gate) up with both branches rounded to bfloat16 first (limit, slope and up_shift
+// multiple of 64, F of 8. tile: rows of x by rows of W of a workgroup, 0 256 x 256, 1 128 x 256, 2 128 x 128. act: 0 silu(gate) up with both branches rounded to bfloat16 first (limit, slope and up_shift
 // unused); 1, 2, 3: the capped unit from the 32-bit sums with the gate through a sigmoid of slope, relu or gelu's tanh form.
 extern "C" int ts_gemm_glu_bf16(void* y, const void* x, const void* w, int M, int F, int K, int64_t ldx, int64_t ldw, int64_t ldy,
-                                int act, float limit, float slope, float up_shift, hipStream_t stream) {
+                                int tile, int act, float limit, float slope, float up_shift, hipStream_t stream) {
   if (M <= 0 || F <= 0) return TS_OK;
-  if (K <= 0 || K % 64 || F % 8 || ldx < K || ldw < K || ldy < F || ldx % 8 || ldw % 8 || ldy % 8 || act < 0 || act > 3) return TS_BAD_SHAPE;
+  if (K <= 0 || K % 64 || F % 8 || ldx < K || ldw < K || ldy < F || ldx % 8 || ldw % 8 || ldy % 8 || act < 0 || act > 3 || tile < 0 || tile > 2) return TS_BAD_SHAPE;
   if (((uintptr_t)x | (uintptr_t)w | (uintptr_t)y) & 15) return TS_BAD_SHAPE;
   if (!x || !w || !y || 2 * (int64_t)F * ldw * 2 >= (1ll << 31) || 256 * ldx * 2 >= (1ll << 31)) return TS_TOO_LARGE;   // (byte offsets from a tile's start)
-  // The tile with the cheapest rounds of one workgroup a compute unit: for K = 2,048 a round takes 60 µs with 256 x 256,
-  // 36 with 128 x 256 and 23 with 128 x 128 (1,514 rows of F 8,192: 124, 108 and 128 µs; 999: 60, 68, 84; 256: 48, 34, 25).
-  const auto rounds = [&](int bm, int bn) { return ((int64_t)((M + bm - 1) / bm) * ((2 * F + bn - 1) / bn) + 255) / 256; };
   const GluArgs a = {(bf16_t*)y, (const bf16_t*)x, (const bf16_t*)w, M, F, K, 0, 0, 0, ldx, ldw, ldy, limit, slope, up_shift};
-  const int64_t big = 60 * rounds(256, 256), mid = 36 * rounds(128, 256), small = 23 * rounds(128, 128);
-  if (big <= mid && big <= small) return launch_glu<256, 256, 2, 4>(a, act, stream);
-  if (mid <= small) return launch_glu<128, 256, 2, 4>(a, act, stream);
-  return launch_glu<128, 128, 2, 4>(a, act, stream);
+  switch (tile) {
+    case 0: return launch_glu<256, 256, 2, 4>(a, act, stream);
+    case 1: return launch_glu<128, 256, 2, 4>(a, act, stream);
+    default: return launch_glu<128, 128, 2, 4>(a, act, stream);
+  }
 }

@@ -65,7 +65,7 @@ def _declare(lib: ctypes.CDLL) -> None:
         "ts_feed_tokens": [p, p, p, i, i, p],
         "ts_gemm_library_bf16": [p, p, p, i, i, i, i64, i64, i64, i, i, p, ctypes.c_size_t, p],
         "ts_gemm_tiled_bf16": [p, p, p, i, i, i, i64, i64, i64, i, i, p],
-        "ts_gemm_glu_bf16": [p, p, p, i, i, i, i64, i64, i64, i, f, f, f, p],
+        "ts_gemm_glu_bf16": [p, p, p, i, i, i, i64, i64, i64, i, i, f, f, f, p],
         "ts_gemm_library_init": [],
         "ts_gemm_library_timing": [i],
         "ts_gemm_library_choices": [p, i],
@@ -1449,7 +1449,7 @@ _many_rows = "library"
 
 def many_rows_products(which: str | None = None) -> str:
     """Which kernel serves bfloat16 products of many rows: "library" (the vendor's, the faster one
-    and the default; products that end in a gated unit go to `gemm_glu`, which takes the unit along) or
+    and the default; products that end in a gated unit go to `gemm_glu`, which takes the unit along, where `glu_pays`) or
     "tiled" (this repository's LDS-tiled matrix-core kernel, for the shapes it takes). Sets it if `which` is given; returns the setting. It holds for the process."""
     global _many_rows
     if which is not None:
@@ -1500,6 +1500,36 @@ def glu_takes(x: torch.Tensor, weight: torch.Tensor) -> bool:
             and 2 * n * weight.stride(0) < 1 << 31 and 512 * x.stride(0) < 1 << 31)
 
 
+# Tiles of `gemm_glu` (rows of x by rows of W) and the µs a round of one workgroup a compute unit takes of them over a reduction of 2,048
+GLU_TILES = ((256, 256, 60), (128, 256, 36), (128, 128, 23))
+COMPUTE_UNITS = 256
+
+
+@functools.lru_cache(maxsize=4096)
+def glu_plan(rows: int, n: int) -> tuple[int, int]:
+    """The tile of `gemm_glu` (its place in `GLU_TILES`) with the cheapest rounds for `rows` rows of x against a weight of
+    `n` rows, and the µs they take over a reduction of 2,048 (1,514 rows, n 16,384: 124, 108 and 128 by tile; 999: 60, 68, 84;
+    256: 48, 34, 25)."""
+    costs = [us * -(-(-(-rows // bm) * -(-n // bn)) // COMPUTE_UNITS) for bm, bn, us in GLU_TILES]
+    return costs.index(min(costs)), min(costs)
+
+
+@functools.lru_cache(maxsize=4096)
+def glu_pays(rows: int, n: int, k: int, branch_bytes: int = 2) -> bool:
+    """Whether `gemm_glu` is the faster way to the unit of `rows` rows against a weight [n, k] than a plain product (its branches
+    stored in `branch_bytes` each) and the unit's kernel. Its least work is a round of whole tiles over all of k, however few
+    they are, where the library cuts the reduction and has smaller tiles; what it saves is a launch and the branches' trip
+    through memory. Both sides are estimated as they measured, in µs, with the weights coming from memory: here the plan's
+    rounds; there 11 (10 for 32-bit branches, whose reading is counted apart) beside the longer of the weight's reading at
+    6.5 TB/s and the full tiles' products at 1 / 1.15 of the rate here, and the branches' trip at 3 TB/s. Over 589 points (1 to 2,048 rows, n
+    1,024 to 28,672, k 512 to 8,192) what this takes is at most 1.05 times the slower route's time where it errs. Apart and
+    here: F = n / 2 of 8,192, k 3,072: 17 rows 25 and 34, 160 rows 39 and 36, 320 rows 47 and 50, 2,048 rows 171 and 151; F 1,024, k 8,192: 16 rows 15
+    and 64, 1,024 rows 54 and 70, 2,048 rows 78 and 77; F 1,536, k 576: 1 row 8.9 and 7.6, 1,024 rows 15.8 and 9.2."""
+    full = 60 * rows * n / (256 * 256 * COMPUTE_UNITS) * k / 2048
+    apart = (11 if branch_bytes == 2 else 10) + max(2 * n * k / 6.5e6, 1.15 * full) + rows * n * (branch_bytes + 1) / 3e6
+    return 1.5 + glu_plan(rows, n)[1] * k / 2048 < apart
+
+
 def gemm_glu(x: torch.Tensor, weight: torch.Tensor, form: str, limit: float = 0.0, slope: float = 1.0, up_shift: float = 0.0) -> torch.Tensor:
     """The gated unit of bfloat16 x [M, K] against a weight [2 F, K] of F gate rows, then F up rows, as bfloat16 [M, F], in
     one kernel for many rows (gemm_glu.hip). `form` "silu_rounded": silu(gate) up of branches rounded to bfloat16 first
@@ -1514,7 +1544,7 @@ def gemm_glu(x: torch.Tensor, weight: torch.Tensor, form: str, limit: float = 0.
     y = torch.empty((M, F), dtype=torch.bfloat16, device=x.device)
     if M and F:
         _run("gemm_glu", library().ts_gemm_glu_bf16(_ptr(y), _ptr(x), _ptr(weight), M, F, K, x.stride(0), weight.stride(0), F,
-                                                    GLU_FORMS[form], float(limit), float(slope), float(up_shift), _stream()))
+                                                    glu_plan(M, 2 * F)[0], GLU_FORMS[form], float(limit), float(slope), float(up_shift), _stream()))
     return y
 
 

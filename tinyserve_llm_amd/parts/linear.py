@@ -4,7 +4,8 @@ float32 runs the engine's own exact kernel (32-bit multiply-adds, ascending k, i
 batch). bfloat16 uses the weight-streaming kernel for few rows and the vendor matrix library for
 many, as the reference uses a vendor library for every projection (or, if
 `hip.many_rows_products("tiled")` says so, the engine's own tiled kernel, which is slower); a
-gate|up projection of many rows goes to the engine's own kernel, which takes the unit along.
+gate|up projection of many rows goes to the engine's own kernel, which takes the unit along, where
+that is the faster way (`hip.glu_pays`).
 
 With few rows a step's time goes to launching kernels and to waiting for memory, so what
 precedes or follows a projection can ride along with it: a norm may hand its input over as a
@@ -176,7 +177,8 @@ def linear(x: "torch.Tensor | DeferredNorm | hip.PackedRows8 | hip.SplitAttentio
         if (out_dtype in (None, torch.bfloat16) and hip.many_rows_products() == "tiled" and x.is_cuda
                 and hip.tiled_takes(x, weight, glu=True)):
             return hip.gemm_tiled(x, weight, glu=True)
-        if out_dtype in (None, torch.bfloat16) and hip.many_rows_products() == "library" and x.is_cuda and hip.glu_takes(x, weight):
+        if (out_dtype in (None, torch.bfloat16) and hip.many_rows_products() == "library" and x.is_cuda and hip.glu_takes(x, weight)
+                and hip.glu_pays(x.shape[0], *weight.shape)):
             return hip.gemm_glu(x, weight, "silu_rounded")
         return hip.silu_mul(linear(x, weight, out_dtype, packed=packed))
     if x.dtype == torch.float32:

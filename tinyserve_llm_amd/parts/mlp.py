@@ -119,7 +119,8 @@ class CappedGLU(FeedForward):
     def forward(self, x: torch.Tensor, ctx: StepContext) -> torch.Tensor:
         unit = few_rows_unit(x, self.gate_up, self.gate_up_packed, self.down, (self.activation, self.limit, self.slope, self.up_shift))
         if unit is None and (hip.many_rows_products() == "library" and x.is_cuda and hip.glu_takes(x, self.gate_up)
-                             and hip.many_rows(x, self.gate_up, self.gate_up_packed)):
+                             and hip.many_rows(x, self.gate_up, self.gate_up_packed)
+                             and hip.glu_pays(x.shape[0], *self.gate_up.shape, branch_bytes=4)):
             # many rows: the unit rides on the product's way out and the 32-bit sums stay where they are made
             unit = hip.gemm_glu(x, self.gate_up, self.activation, self.limit, self.slope, self.up_shift)
         if unit is None:

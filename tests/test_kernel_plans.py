@@ -2,6 +2,8 @@
 
 import random
 
+import torch
+
 from tinyserve_llm_amd.ops import hip
 
 
@@ -153,3 +155,18 @@ def test_gated_product_tiles_follow_the_rounds():
             tile, cost = hip.glu_plan(rows, n)
             bm, bn, us = hip.GLU_TILES[tile]
             assert cost == us * -(-(-(-rows // bm) * -(-n // bn)) // 256) == min(u * -(-(-(-rows // a) * -(-n // b)) // 256) for a, b, u in hip.GLU_TILES)
+
+
+def test_expert_tiles_are_the_fastest_that_were_timed():
+    """(experts, width, experts' width, pairs an expert) with the tiles whose time was within 1.05 of the fastest, weights from memory."""
+    bf = torch.bfloat16
+    timed = [((8, 512, 256, 32), {16}), ((8, 512, 256, 48), {16}), ((8, 1024, 512, 32), {16}), ((4, 2048, 1024, 32), {16, 128}),
+             ((4, 2048, 1024, 128), {128}), ((4, 2048, 1024, 512), {128}), ((8, 1024, 512, 128), {128}), ((16, 2048, 1024, 64), {128}),
+             ((16, 2048, 1024, 256), {256}), ((16, 2048, 1024, 512), {128}), ((8, 4096, 1536, 512), {256}), ((32, 1024, 512, 1024), {128, 256}),
+             ((128, 2048, 256, 1024), {256}), ((64, 2048, 768, 1024), {256}), ((8, 2048, 5632, 128), {128})]
+    for (experts, width, inner, each), good in timed:
+        assert hip.moe_tile_rows(each * experts, experts, bf, (width, inner)) in good, (experts, width, inner, each)
+    # few pairs an expert, 32-bit rows and odd reductions as before
+    assert hip.moe_tile_rows(31 * 16, 16, bf, (2048, 1024)) == 16 and hip.moe_tile_rows(4096, 4, torch.float32, (2048, 1024)) == 16
+    assert hip.moe_tile_rows(4096, 4, bf, (2048, 96)) == 64 and hip.moe_tile_rows(4096, 4, bf, (2048, 40)) == 16
+    assert hip.moe_tile_rows(4096, 4, bf) == 128

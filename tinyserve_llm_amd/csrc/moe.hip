@@ -525,23 +525,24 @@ moe_gemm_stream_kernel(TO* __restrict__ out, const bf16_t* __restrict__ x, const
   moe_store4(orow + c0, y, N - c0);
 }
 
-// Tiles of 128 or 256 rows, for steps that give an expert hundreds of rows: the gated product's scheme (gemm_glu.hip) with the
-// rows of x gathered by pair, the matrix the tile's expert's, and the rows of y stored at their pairs' places. A workgroup of
-// eight waves takes BM rows by 256 rows of W (with GLU 128 gate and 128 up rows, whose sums meet in one lane), 64 of K at a
-// time, K a multiple of 64. What bounds it is the matrix cores and a compute unit's path to memory: operands go from memory
+// Tiles of 128 or 256 rows, for steps that give an expert dozens or hundreds of rows: the gated product's scheme (gemm_glu.hip)
+// with the rows of x gathered by pair, the matrix the tile's expert's, and the rows of y stored at their pairs' places. A
+// workgroup of eight waves takes BM rows by as many rows of W (with GLU half gate, half up rows, whose sums meet in one lane), 64
+// of K at a time, K a multiple of 64. What bounds it is the matrix cores and a compute unit's path to memory: operands go from memory
 // straight into LDS, two steps of x and three of W, pieces turned by (row / 2) % 8 against bank conflicts, and loads, operand
-// reads and products are dealt out evenly. 7,300 pairs of 16 experts over 2,048 against 2 x 1,024, and back over 1,024: 71 and
-// 49 µs with tiles of 128 rows, 68 and 42 with 256 (111 and 85 where operands passed through registers on their way to LDS,
-// 128 rows by 128 of W a workgroup, and the dies took eighths of the whole table).
+// reads and products are dealt out evenly. Of the smaller tile two workgroups share a compute unit, one waiting while the other
+// multiplies: 128 x 128 is as fast as 128 x 256 at any size and faster where tiles are few. Both products of 16 experts over
+// 2,048, 2 x 1,024 and back over 1,024, weights from memory: 64 pairs each 55 µs (128 x 256: 72, tiles of 64 rows without LDS 172), 128 each 81, 256
+// each 112 (256 x 256: 99), 512 each 165 (184), 1,024 each 295 (274; where operands passed through registers on their way to LDS 342).
 template <int BM, bool GLU, typename TO>
-__global__ void __launch_bounds__(512, 2)
+__global__ void __launch_bounds__(512, BM == 128 ? 4 : 2)
 moe_gemm_lds_kernel(TO* __restrict__ out, const bf16_t* __restrict__ x, const bf16_t* __restrict__ w,
                     const int32_t* __restrict__ sorted, const int32_t* __restrict__ tiles, int num_tiles, int col_blocks,
                     int src_div, int N, int K, float limit, float slope, float shift, int act) {
-  constexpr int BN = 256, WM = 2, WN = 4, WAVES = WM * WN, TM = BM / WM / 16, TN = BN / WN / 16, HALF = BN / WN / 2;
+  constexpr int BN = BM, WN = BN / 64, WM = 8 / WN, WAVES = WM * WN, TM = BM / WM / 16, TN = BN / WN / 16, HALF = BN / WN / 2;
   constexpr int NX = BM / 8 / WAVES, NW = BN / 8 / WAVES;      // kilobytes of a step that a wave fetches
   constexpr int XS = BM * 128, WS = BN * 128;                  // bytes of a step of x and of W
-  static_assert(NW * 8 == HALF, "a wave fetches gate rows or up rows");
+  static_assert(HALF % (NW * 8) == 0, "a wave fetches gate rows or up rows");
   __shared__ __attribute__((aligned(1024))) unsigned char lds[2 * XS + 3 * WS];
   // Workgroups go to the chip's eight dies in turn, each die with a cache of its own: die d takes the d-th eighth
   // of the (tile, column block) list, column blocks innermost and tiles in the experts' order, so that the
@@ -570,7 +571,7 @@ moe_gemm_lds_kernel(TO* __restrict__ out, const bf16_t* __restrict__ x, const bf
     const int at = (wave * NX + q) * 8 + lane / 8;
     xp[q] = x + (int64_t)(sorted[first + min(at, rows - 1)] / src_div) * K + ((lane % 8) ^ ((at >> 1) & 7)) * 8;
   }
-  const int ups = GLU && wave % 2 ? N : 0;                     // (odd waves fetch up rows)
+  const int ups = GLU && wave * NW * 8 / HALF % 2 ? N : 0;     // (the waves whose rows of the tile are up rows)
   const __amdgpu_buffer_rsrc_t rsrc_w = load_base(w + ((int64_t)e * (GLU ? 2 : 1) * N + n0 + ups) * K);
 #pragma unroll
   for (int q = 0; q < NW; ++q) {
@@ -694,7 +695,7 @@ extern "C" int ts_moe_gemm(void* out, int out_dtype, const void* x, int x_dtype,
   const bool mfma = x_dtype == 1 && K % 32 == 0 && (((uintptr_t)x | (uintptr_t)w) & 15) == 0;
   if (tile_rows >= 128) {
     if (!mfma || K % 64 || K > (1 << 22)) return TS_BAD_SHAPE;                 // (byte offsets within 256 rows of W)
-    const int col_blocks = glu ? (N + 127) / 128 : (N + 255) / 256;
+    const int per_block = glu ? tile_rows / 2 : tile_rows, col_blocks = (N + per_block - 1) / per_block;
     const int64_t items = (int64_t)max_tiles * col_blocks;
     if (items > 0x3fffffff) return TS_BAD_SHAPE;
     const unsigned grid = (unsigned)((items + MOE_DIES - 1) / MOE_DIES * MOE_DIES);

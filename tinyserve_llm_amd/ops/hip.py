@@ -11,6 +11,7 @@ from __future__ import annotations
 import contextlib
 import ctypes
 import functools
+import math
 import threading
 
 import torch
@@ -2155,12 +2156,10 @@ def conv_state_update(state: torch.Tensor, proj: torch.Tensor, ctx) -> None:
 
 MOE_TILE_ROWS = 16        # rows of a tile of the experts' products,
 MOE_WIDE_TILE_ROWS = 64   # or, in bfloat16, where the experts have this many rows each on average,
-MOE_LDS_TILE_ROWS = 128   # tiles of the kernel whose operands both go through LDS (reductions that are multiples of 64),
-MOE_LDS_FROM = 32         # taken from this many pairs an expert on: 16 experts over 2,048, 2 x 1,024 and back, 32 pairs each: 50 µs
-                          # (112 with tiles of 16 rows, 120 of 64); 64 each: 52 (150, 139); 128 each: 56 (294, 199)
-MOE_LDS_WIDE_TILE_ROWS = 256      # and its larger tiles,
-MOE_LDS_WIDE_FROM = 512           # from this many pairs an expert on where both reductions have MOE_LDS_WIDE_MIN_K: 512 each 110 µs
-MOE_LDS_WIDE_MIN_K = 1024         # (119 with 128 rows), 1,024 each 186 (228), 256 each 84 (60); 32 experts of 1,024 and 512, 512 each: 107 (102)
+MOE_LDS_TILE_ROWS = 128   # or tiles of the kernel whose operands both go through LDS (reductions that are multiples of 64),
+MOE_LDS_WIDE_TILE_ROWS = 256
+MOE_LDS_ROUND_US = {128: 21, 256: 60}     # µs of a round of one such tile, by as many rows of W, a compute unit over a reduction of 2,048
+MOE_LDS_FROM = 32         # pairs an expert below which the narrow tiles stay, whose rows have the same bits in a batch of any size
 MOE_MAX_EXPERTS = 1024
 MOE_MAX_TOP = 32
 MOE_MAX_GROUPS = 64
@@ -2205,13 +2204,31 @@ class ExpertTiles:
         self.sorted, self.tiles, self.top, self.experts, self.tile_rows = sorted_pairs, tiles, top, experts, tile_rows
 
 
-def moe_tile_rows(pairs: int, experts: int, dtype: torch.dtype, k_sizes: "tuple[int, ...]" = ()) -> int:
-    """Rows of a tile for a step of `pairs` (token, expert) pairs whose products run over `k_sizes`: wider tiles where a
-    matrix-core kernel runs (bfloat16; reductions that are multiples of 64 through LDS, of 32 otherwise) and an expert has
-    enough rows on average, so that its matrix is read once per tile of them and not once per 16."""
-    if dtype == torch.bfloat16 and all(k % 64 == 0 for k in k_sizes) and pairs >= (MOE_LDS_FROM if k_sizes else MOE_LDS_TILE_ROWS) * experts:
-        wide = pairs >= MOE_LDS_WIDE_FROM * experts and min(k_sizes, default=0) >= MOE_LDS_WIDE_MIN_K
-        return MOE_LDS_WIDE_TILE_ROWS if wide else MOE_LDS_TILE_ROWS
+@functools.lru_cache(maxsize=4096)
+def moe_tile_rows(pairs: int, experts: int, dtype: torch.dtype, k_sizes: "tuple[int, ...]" = (), gated: bool = True) -> int:
+    """Rows of a tile for a step of `pairs` (token, expert) pairs whose two products run over `k_sizes` = (the width, the experts'
+    width; `gated`: the first product makes twice that), so that an expert's matrix is read once per tile of them and not once
+    per 16. Where the matrix-core kernels run (bfloat16; reductions that are multiples of 64 through LDS, of 32 otherwise) and an expert has enough
+    rows on average, the tile with the least estimated µs is taken, pairs lying evenly over the experts: of 16 rows, every tile
+    reads its expert's matrices, at 4.5 TB/s; through LDS, rounds of whole tiles and at least the matrices once at 4.6 TB/s. Of the
+    108 sizes of at least 32 pairs an expert that were timed (4 to 128 experts, widths 512 to 4,096 and 256 to 5,632, up to 1,024 pairs an expert) each was within 1.05 of its
+    fastest tile: 8 experts of 512 and 256, 32 each: 9 µs (13 and 30 with 128 and 256 rows), 128 each: 15 (16 rows 16, 256 rows 33); 4 of 2,048 and 1,024, 32 each: 34 of
+    either (256 rows 74), 512 each: 52 (16 rows 295, 256 rows 84), 1,024 each: 84 of 256 (128 rows 85); 16 of them, 256 each: 99 of 256 (112, 16 rows 607)."""
+    if dtype == torch.bfloat16 and all(k % 64 == 0 for k in k_sizes):
+        if len(k_sizes) == 2 and pairs >= MOE_LDS_FROM * experts:
+            width, inner = k_sizes
+            ups = 2 * inner if gated else inner
+            matrices = 2 * (ups + inner) * width            # bytes of an expert
+            costs = {}
+            if pairs < MOE_LDS_TILE_ROWS * experts:         # (whole tiles of 128: never the slower ones)
+                costs[MOE_TILE_ROWS] = 5 + experts * (pairs / experts / MOE_TILE_ROWS + 0.5) * matrices / 4.5e6
+            for rows, us in MOE_LDS_ROUND_US.items():
+                tiles = experts * max(1.0, pairs / experts / rows + 0.5)
+                rounds = [math.ceil(tiles * -(-n // rows) / COMPUTE_UNITS) * k / 2048 for n, k in ((ups, width), (width, inner))]
+                costs[rows] = 5 + max(us * sum(rounds), experts * matrices / 4.6e6)
+            return min(costs, key=costs.get)
+        if not k_sizes and pairs >= MOE_LDS_TILE_ROWS * experts:
+            return MOE_LDS_TILE_ROWS
     wide = dtype == torch.bfloat16 and all(k % 32 == 0 for k in k_sizes) and pairs >= MOE_WIDE_TILE_ROWS * experts
     return MOE_WIDE_TILE_ROWS if wide else MOE_TILE_ROWS
 

@@ -125,7 +125,7 @@ class RoutedDenseExperts(FeedForward):
     def forward(self, x: torch.Tensor, ctx: StepContext) -> torch.Tensor:
         experts, weights = hip.moe_route(x, self.router, None, self.top, self.router_scale, True,
                                          softmax_chosen=self.scoring == "softmax_chosen")
-        tile_rows = hip.moe_tile_rows(experts.numel(), self.num_experts, x.dtype, (self.hidden_size, self.intermediate_size))
+        tile_rows = hip.moe_tile_rows(experts.numel(), self.num_experts, x.dtype, (self.hidden_size, self.intermediate_size), gated=False)
         grouped = hip.moe_group(experts, self.num_experts, tile_rows)
         act = hip.moe_gemm(x, self.up, grouped, x.dtype, per_token=True, activation=self.activation)
         rows = hip.moe_gemm(act, self.down, grouped, torch.float32, per_token=False)

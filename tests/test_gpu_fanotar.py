@@ -397,6 +397,26 @@ def test_tiles_through_lds_give_the_narrower_tiles_sums(sizes, tile_rows):
         assert torch.equal(a[taken], b[taken])
 
 
+@pytest.mark.parametrize("tile_rows", [128, 256])
+def test_wide_tiles_over_a_reduction_beyond_32_bit_offsets(tile_rows):
+    """Rows of more than 2^22 elements (256 of them lie further apart than 31 bits of bytes): the narrower tiles' bits, and in size
+    what 64 bits give, at the ends of the row as in its middle."""
+    h = hip()
+    K, N, n = (1 << 22) + 64, 8, 70
+    gen = torch.Generator().manual_seed(tile_rows)
+    x, w = torch.zeros(2, K, dtype=torch.bfloat16, device=DEV), torch.zeros(1, 2 * N, K, dtype=torch.bfloat16, device=DEV)
+    spots = torch.tensor([0, 1, 63, 64, 1 << 21, (1 << 22) - 1, 1 << 22, K - 1], device=DEV)
+    x[:, spots], w[:, :, spots] = torch.randn(2, 8, generator=gen).bfloat16().to(DEV), torch.randn(1, 2 * N, 8, generator=gen).bfloat16().to(DEV)
+    ids = torch.zeros(2, n, dtype=torch.int32, device=DEV)                   # (a token chosen many times over: 140 pairs in 2 rows of x)
+    sums = x[:, spots].double() @ w[0][:, spots].double().T
+    want = sums.repeat_interleave(n, dim=0)
+    found = [h.moe_gemm(x, w, h.moe_group(ids, 1, rows), torch.float32, per_token=True) for rows in (64, tile_rows)]
+    assert torch.equal(*found)
+    torch.testing.assert_close(found[1].double(), want, rtol=0.0, atol=8 * 2.0 ** -23 * float(want.abs().max()) * 8)
+    unit = [h.moe_gemm(x, w, h.moe_group(ids, 1, rows), torch.bfloat16, per_token=True, glu=(1.2, 1.702, 1.0)) for rows in (64, tile_rows)]
+    assert torch.equal(*unit)
+
+
 # ---- whole models through trace replay ---------------------------------------------------------------
 
 LENGTHS = {"P": [1, 23, 97, 200], "Q": [1, 30, 75, 150], "R": [2, 19, 66, 131], "S": [1, 40, 140]}

@@ -383,13 +383,13 @@ static __device__ __forceinline__ void moe_store4(bf16_t* p, const float (&y)[4]
 template <int TM, int TN, bool GLU, typename TO>
 __global__ void __launch_bounds__(MOE_THREADS)
 moe_gemm_mfma_kernel(TO* __restrict__ out, const bf16_t* __restrict__ x, const bf16_t* __restrict__ w,
-                     const int32_t* __restrict__ sorted, const int32_t* __restrict__ tiles, int src_div, int N, int K,
+                     const int32_t* __restrict__ sorted, const int32_t* __restrict__ tiles, int parts, int src_div, int N, int K,
                      float limit, float slope, float shift, int act) {
   constexpr int SETS = GLU ? 2 : 1;
-  const int tile = blockIdx.x;
-  const int rows = tiles[3 * tile + 2];
-  if (rows == 0) return;
-  const int e = tiles[3 * tile], first = tiles[3 * tile + 1];
+  const int tile = blockIdx.x / parts, at = blockIdx.x % parts * TM * 16;     // (wider tiles in parts of so many rows)
+  const int rows = min(tiles[3 * tile + 2] - at, TM * 16);
+  if (rows <= 0) return;
+  const int e = tiles[3 * tile], first = tiles[3 * tile + 1] + at;
   const int wave = threadIdx.x / TS_WAVE, lane = threadIdx.x & (TS_WAVE - 1);
   const int r = lane & 15, g = lane >> 4;
   const int n0 = (blockIdx.y * 4 + wave) * TN * 16;
@@ -693,8 +693,8 @@ extern "C" int ts_moe_gemm(void* out, int out_dtype, const void* x, int x_dtype,
   if (act < 0 || act > 1 || (glu && act)) return TS_BAD_SHAPE;
   if (N <= 0 || K <= 0 || src_div <= 0 || (tile_rows != 16 && tile_rows != 64 && tile_rows != 128 && tile_rows != 256)) return TS_BAD_SHAPE;
   const bool mfma = x_dtype == 1 && K % 32 == 0 && (((uintptr_t)x | (uintptr_t)w) & 15) == 0;
-  if (tile_rows >= 128) {
-    if (!mfma || K % 64 || K > (1 << 22)) return TS_BAD_SHAPE;                 // (byte offsets within 256 rows of W)
+  if (tile_rows >= 128 && (!mfma || K % 64)) return TS_BAD_SHAPE;
+  if (tile_rows >= 128 && K <= (1 << 22)) {                 // (byte offsets within 256 rows of W; longer reductions by 64-bit addresses below)
     const int per_block = glu ? tile_rows / 2 : tile_rows, col_blocks = (N + per_block - 1) / per_block;
     const int64_t items = (int64_t)max_tiles * col_blocks;
     if (items > 0x3fffffff) return TS_BAD_SHAPE;
@@ -728,11 +728,12 @@ extern "C" int ts_moe_gemm(void* out, int out_dtype, const void* x, int x_dtype,
       return ts_check_launch();
     }
     // (a wave takes 32 columns of all the tile's rows; with the gate, 32 gate and 32 up columns)
-    dim3 grid(max_tiles, (N + 127) / 128);
-    if (grid.y > 65535) return TS_BAD_SHAPE;
+    const int parts = tile_rows / 64;
+    dim3 grid((unsigned)max_tiles * parts, (N + 127) / 128);
+    if (grid.y > 65535 || max_tiles > 0x3fffffff / parts) return TS_BAD_SHAPE;
 #define MOE_MFMA(TM, GLU, TO) \
     moe_gemm_mfma_kernel<TM, 2, GLU, TO><<<grid, MOE_THREADS, 0, stream>>>((TO*)out, (const bf16_t*)x, (const bf16_t*)w, sorted, \
-                                                                           tiles, src_div, N, K, limit, slope, shift, act)
+                                                                           tiles, parts, src_div, N, K, limit, slope, shift, act)
     if (glu && out_dtype == 1) MOE_MFMA(4, true, bf16_t);
     else if (!glu && out_dtype == 0) MOE_MFMA(4, false, float);
     else if (!glu && out_dtype == 1) MOE_MFMA(4, false, bf16_t);

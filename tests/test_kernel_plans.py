@@ -2,6 +2,7 @@
 
 import random
 
+import pytest
 import torch
 
 from tinyserve_llm_amd.ops import hip
@@ -170,3 +171,19 @@ def test_expert_tiles_are_the_fastest_that_were_timed():
     assert hip.moe_tile_rows(31 * 16, 16, bf, (2048, 1024)) == 16 and hip.moe_tile_rows(4096, 4, torch.float32, (2048, 1024)) == 16
     assert hip.moe_tile_rows(4096, 4, bf, (2048, 96)) == 64 and hip.moe_tile_rows(4096, 4, bf, (2048, 40)) == 16
     assert hip.moe_tile_rows(4096, 4, bf) == 128
+
+
+def test_each_fault_of_a_cache_is_named():
+    def caches(pages=3, page=16, kv=2, hd=32, dtype=torch.float32):
+        return torch.zeros(pages, page, kv, hd, dtype=dtype)
+    ok = caches()
+    hip._check_cache(ok, ok.clone(), torch.float32, 2, 32)
+    faults = [(caches(kv=3), ok, "key cache view must be"), (ok, caches(hd=16), "value cache view must be"), (ok[0], ok, "key cache view must be"),
+              (caches(dtype=torch.bfloat16), ok, "storage type: the key"), (ok, caches(dtype=torch.bfloat16), "storage type: the value"),
+              (ok, caches(pages=4), "differ in shape"), (ok[:1].expand(3, 16, 2, 32), ok, "key cache elements overlap"),
+              (ok, ok[:1].expand(3, 16, 2, 32), "value cache elements overlap"),
+              (ok.transpose(1, 3).contiguous().transpose(1, 3), ok, "head_dim must be contiguous"),
+              (torch.zeros(3, 16, 2, 33)[..., :32], ok, "16-byte aligned")]
+    for k, v, message in faults:
+        with pytest.raises(hip.KernelError, match=message):
+            hip._check_cache(k, v, torch.float32, 2, 32)

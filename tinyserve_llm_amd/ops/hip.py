@@ -263,8 +263,7 @@ def _check_cache(k_cache: torch.Tensor, v_cache: torch.Tensor, dtype: torch.dtyp
     engine's pools keep a head's slots of one dimension together, i.e. pages transposed)."""
     ks, vs, shape = k_cache.stride(), v_cache.stride(), k_cache.shape
     _need(len(shape) == 4 and shape[2] == nkv and shape[3] == hd and k_cache.dtype == dtype and v_cache.dtype == dtype and v_cache.shape == shape,
-          lambda: f"key and value cache views must be {dtype} [pages, page_size, {nkv}, {hd}], got {k_cache.dtype} {tuple(k_cache.shape)} "
-                  f"and {v_cache.dtype} {tuple(v_cache.shape)}")
+          lambda: _cache_fault(k_cache, v_cache, dtype, nkv, hd))
     # no two elements may overlap: sort the strides and check each spans the dimensions below it
     for name, strides in (("key", ks), ("value", vs)):
         span = 1
@@ -275,6 +274,16 @@ def _check_cache(k_cache: torch.Tensor, v_cache: torch.Tensor, dtype: torch.dtyp
                 span = stride * size
     _need(ks[3] == 1, "head_dim must be contiguous in the key cache")
     _need(((ks[0] | ks[1] | ks[2]) * k_cache.element_size()) % 16 == 0 and k_cache.data_ptr() % 16 == 0, "key rows must be 16-byte aligned")
+
+
+def _cache_fault(k_cache: torch.Tensor, v_cache: torch.Tensor, dtype: torch.dtype, nkv: int, hd: int) -> str:
+    """What is wrong with caches whose shapes or types do not fit."""
+    for name, c in (("key", k_cache), ("value", v_cache)):
+        if c.dim() != 4 or c.shape[2] != nkv or c.shape[3] != hd:
+            return f"{name} cache view must be [pages, page_size, {nkv}, {hd}], got {tuple(c.shape)}"
+        if c.dtype != dtype:
+            return f"cache and activations differ in storage type: the {name} cache is {c.dtype}, the activations are {dtype}"
+    return f"key and value caches differ in shape: {tuple(k_cache.shape)} and {tuple(v_cache.shape)}"
 
 
 def _page_run(pages_per_entry: int) -> int:

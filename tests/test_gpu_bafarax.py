@@ -377,6 +377,50 @@ def test_latent_attention_window_edges(dtype, window, sizes, form, page):
             assert not decides(want[queries.index(q), 0], v[key]), (q, key)
 
 
+@pytest.mark.parametrize("mask", [("full", 0), ("window", 100), ("chunk", 128)])
+@pytest.mark.parametrize("sizes", [(32, 256, 0), (16, 256, 128), (40, 96, 24), (130, 64, 16), (32, 128, 0)])
+def test_latent_attention_of_several_requests_in_wide_tiles(sizes, mask, monkeypatch):
+    """Requests of uneven lengths and starts in one list of tiles of 128 rows, decoded tokens beside them, tiles cut at the requests'
+    borders, heads beyond 128, pages of the pool in runs, sinks and a gate per head. Scores spread over +-10, so that a key
+    more or less at an edge shows. The same requests with many more decoded tokens are the other kernel's where heads are few."""
+    h = hip()
+    (H, rank, rot), (kind, size) = sizes, mask
+    row, page, scale = rank + rot, 64, 3.0 * (rank + rot) ** -0.5
+    gen = torch.Generator().manual_seed(H + row + size)
+    ran, plain_run = [], h._run
+    monkeypatch.setattr(h, "_run", lambda name, code: ran.append(name) or plain_run(name, code))
+    for decoding in (3, 1200):
+        starts = [40, 333, 700] * (decoding // 3) + [0, 77, 500, 0, 130]
+        counts = [1] * decoding + [290, 129, 1, 5, 160]
+        ends = [a + b for a, b in zip(starts, counts)]
+        pages = [-(-n // page) for n in ends]
+        order = torch.randperm(sum(pages) + 5, generator=gen).tolist()
+        tables = [order[sum(pages[:i]):sum(pages[:i + 1])] for i in range(len(pages))]
+        cache = torch.zeros(2 * len(order), 32, 1, row, dtype=torch.bfloat16, device=DEV)
+        values = torch.zeros(2 * len(order), 1, rank, 32, dtype=torch.bfloat16, device=DEV).permute(0, 3, 1, 2)
+        kept = []
+        for table, n in zip(tables, ends):
+            rows, at = torch.randn(n, row, generator=gen).bfloat16().to(DEV), torch.arange(n)
+            pg, off = (2 * torch.tensor(table)[at // page] + at % page // 32).to(DEV), (at % 32).to(DEV)
+            cache[pg, off, 0], values[pg, off, 0] = rows, rows[:, :rank]
+            kept.append(rows.cpu().to(F64))
+        q = torch.randn(sum(counts), H, row, generator=gen).bfloat16().float().to(DEV)
+        sinks, gates = torch.linspace(-3.0, 8.0, H, device=DEV), torch.randn(sum(counts), H + 3, generator=gen).to(DEV)
+        ctx = step_context(tables, page, starts, counts)
+        ran.clear()
+        out = h.paged_attention_latent(q, cache, rank, ctx, 0, scale, size if kind == "window" else 0, size if kind == "chunk" else 0,
+                                       out_dtype=torch.float32, v_cache=values, sinks=sinks, head_gate=gates[:, 1:1 + H])
+        assert ran == ["paged_attention_latent_tiles" if decoding == 3 or H > 32 else "paged_attention_latent_mfma"]
+        picked = range(len(counts)) if decoding == 3 else [0, 1, decoding - 1, decoding, decoding + 4]
+        for i in picked:
+            mine = slice(sum(counts[:i]), sum(counts[:i + 1]))
+            positions = torch.arange(starts[i], ends[i])
+            want = plain.masked_attention(q[mine].cpu().to(F64), kept[i][:, None], kept[i][:, None, :rank], positions, scale, kind, size, sinks.cpu().to(F64))
+            want = want * torch.sigmoid(gates[mine, 1:1 + H].cpu().to(F64))[:, :, None]
+            # (weights are kept as two bfloat16 terms, 2^-16 of each; scores of up to 15 good to 2^-21 of that over 384 products)
+            torch.testing.assert_close(out[mine].cpu().to(F64), want, atol=1e-4, rtol=1e-4)
+
+
 @pytest.mark.parametrize("form", sorted(FORMS))
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("page", [16, 32])

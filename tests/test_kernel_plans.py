@@ -187,3 +187,14 @@ def test_each_fault_of_a_cache_is_named():
     for k, v, message in faults:
         with pytest.raises(hip.KernelError, match=message):
             hip._check_cache(k, v, torch.float32, 2, 32)
+
+
+def test_wide_latent_tiles_where_they_are_full_and_their_walks_long():
+    def step(portion, decoding=0):
+        return list(range(decoding)) + [decoding, decoding + portion]
+    wide = hip.latent_wide_tiles
+    assert wide(step(2048), 32, 2048) and wide(step(256), 32, 256) and not wide(step(255), 32, 255)
+    assert not wide(step(64), 128, 64) and wide(step(96), 128, 64) and wide(step(64), 128, 300)
+    # decoded tokens of few heads: tiles that are mostly padding
+    assert not wide(step(2, 300), 32, 1000) and not wide(step(128, 300), 32, 1000) and wide(step(256, 256), 32, 1000) and wide(step(1024, 16), 32, 8000)
+    assert wide(step(2, 300), 48, 1000) and wide(step(2, 300), 128, 1000) and wide(step(2, 300), 200, 1000) and not wide(step(2, 2000), 8, 1000)

@@ -2459,7 +2459,10 @@ def heads_gemm(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, gate: torch.
 
 LATENT_TILE_ROWS = 32     # rows (token, head) of a workgroup of the matrix-core kernel
 LATENT_WIDE_TILE_ROWS = 128    # and of its form for steps of many tokens,
-LATENT_MANY_ROWS = 8192   # which takes portions of steps of at least so many rows
+LATENT_MANY_ROWS = 8192   # which takes steps of at least so many rows: from here the kernel of 32 rows has 256 workgroups and cuts no keys
+LATENT_MANY_SHORT_ROWS = 12288 # (or so many, where nobody reads more than
+LATENT_SHORT_REACH = 64        # so many keys: 128 heads, 64 tokens 12.9 µs and with wide tiles 14.8, 96 tokens 20.2 and 16.9),
+LATENT_WIDE_FILL = 0.35        # and whose wide tiles are this full on average (a decoded token is a tile of its own)
 LATENT_MAX_SPLITS = 16    # stretches a tile's keys may be cut into,
 LATENT_FEW_GROUPS = 512   # where the step has fewer workgroups than half of this
 
@@ -2472,6 +2475,29 @@ def latent_mfma_takes(q: torch.Tensor, cache: torch.Tensor, v_cache: torch.Tenso
             and cache.shape[1] == 32 and v_cache.stride(1) == 1 and bool(library().ts_latent_mfma_takes(rank, q.shape[2]))
             and all(st % 8 == 0 for st in (cache.stride(0), cache.stride(1), v_cache.stride(0), v_cache.stride(3)))
             and cache.data_ptr() % 16 == 0 and v_cache.data_ptr() % 16 == 0 and q.data_ptr() % 16 == 0)
+
+
+def latent_wide_tiles(cu_seqlens: "list[int]", heads: int, reach: int) -> bool:
+    """Whether a step of more than decoded tokens (request i feeds cu_seqlens[i + 1] - cu_seqlens[i]), nobody of which sees more
+    than `reach` keys, is the faster in tiles of `LATENT_WIDE_TILE_ROWS` rows: eight waves share a tile's keys where the
+    kernel of 32 rows reads them anew for each, but a tile of a token of few heads is mostly padding. Rows of 256 numbers,
+    narrow and wide: 32 heads, 2,048 tokens 557 and 115 µs, 256 tokens 24.3 and 20.7, 300 decoded tokens (contexts of 1,000) beside a
+    prompt of 2 89 and 99, of 128 92 and 101, 256 beside one of 256 87 and 75; 48 heads, 300 beside one of 2 145 and 100; 128 heads 229 and 112."""
+    rows = cu_seqlens[-1] * heads
+    if rows < (LATENT_MANY_ROWS if reach > LATENT_SHORT_REACH else LATENT_MANY_SHORT_ROWS):
+        return False
+    tokens = max(1, LATENT_WIDE_TILE_ROWS // heads)
+    tiles = sum(-(-(b - a) // tokens) for a, b in zip(cu_seqlens, cu_seqlens[1:])) * -(-heads // LATENT_WIDE_TILE_ROWS)
+    return rows >= LATENT_WIDE_FILL * tiles * LATENT_WIDE_TILE_ROWS
+
+
+def _latent_wide(ctx, heads: int, mask: int) -> bool:
+    """`latent_wide_tiles` of a step, worked out once for every layer of a kind."""
+    key = ("latent_wide", heads, mask)
+    if key not in ctx.scratch:
+        reach = max(ctx.host_context_lens)
+        ctx.scratch[key] = latent_wide_tiles(ctx.host_cu_seqlens, heads, min(reach, abs(mask)) if mask else reach)
+    return ctx.scratch[key]
 
 
 def _latent_tiles(ctx, tile_tokens: int, device) -> torch.Tensor:
@@ -2512,7 +2538,7 @@ def paged_attention_latent(q: torch.Tensor, cache: torch.Tensor, rank: int, ctx,
     mask = -chunk_mask if chunk_mask else int(window)
     if latent_mfma_takes(q, cache, v_cache, rank) and out.dtype in (torch.float32, torch.bfloat16):
         _need(v_cache.shape == (*cache.shape[:3], rank), "the values' view must match the rows'")
-        if ctx.max_query_len > 1 and T * H >= LATENT_MANY_ROWS and out.data_ptr() % 16 == 0 and bool(library().ts_latent_tiles_takes(rank, row)):
+        if ctx.max_query_len > 1 and _latent_wide(ctx, H, mask) and out.data_ptr() % 16 == 0 and bool(library().ts_latent_tiles_takes(rank, row)):
             # many tokens: tiles of four times as many rows, whose keys a workgroup reads once
             tile_tokens = max(1, LATENT_WIDE_TILE_ROWS // H)
             tiles = _latent_tiles(ctx, tile_tokens, q.device)

@@ -2679,10 +2679,12 @@ def mlstm_finish(o: torch.Tensor, weight: torch.Tensor | None, gate: torch.Tenso
 DECAY_FORMS = {"sigmoid_root": 0, "double_exponent": 1}
 DECAY_MAX_DIM = 1024
 DECAY_FULL_WORKGROUPS = 512      # workgroups of four waves from which a step keeps them (fewer: one wave each, four times as many)
-# Tokens of a request from which its portion is worked in chunks of 64. The walk takes 0.15 us a token and head group (32 heads of
-# 64 channels: 115 us for 512 tokens, 440 for 2,048; in chunks 30 and 68; 8 heads of 128 by 256 120 and 450 against 81 and 102), so
-# chunks are the faster from 128 (64 channels) or 320 tokens (128) on; short portions still walk, whose rows are the same bits
-# however a request's tokens are cut into steps.
+# Tokens of a request from which its portion is worked in chunks of 64. One request, walked and in chunks, µs: 32 heads of 64 channels 128
+# tokens 34 and 25, 512 115 and 30, 768 169 and 39, 2,048 438 and 70; 8 heads of 128 by 256 values 320 tokens 78 and 78, 512 119 and 87, 768
+# 173 and 88, 2,048 442 and 106 (16 requests of 1,024 together: 877 and 472; 1,722 and 620). So chunks are the faster from 128 (up to 64 channels) or
+# 320 tokens (128) on. But they add in another order, and a model with routed experts shows it: with the contexts of 48 decoded requests (350
+# to 700 tokens) in chunks, one row in six runs of 48 took another expert at a near tie and moved by 0.13 of its norm. So
+# a portion keeps the walk's bits, which do not depend on how a request is cut into steps, until chunks take half the time or less at every head size.
 DECAY_CHUNKS_FROM = 768
 DECAY_CHUNK_DIMS = (32, 64, 128)
 DECAY_WIDE_UP_TO = 4             # tokens of a step's longest portion up to which a wave owns 64 value columns instead of 16

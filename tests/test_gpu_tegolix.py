@@ -167,6 +167,38 @@ def test_long_portions_in_chunks(read_first, sizes):
         torch.testing.assert_close(g.to(F64), w, atol=(D + 64) * 2.0 ** -24 * float(w.abs().max()), rtol=1e-5)
 
 
+@pytest.mark.parametrize("read_first", [False, True])
+@pytest.mark.parametrize("sizes", [(8, 64, 64), (4, 128, 128), (2, 128, 256)])
+def test_chunks_are_no_further_from_64_bits_than_the_walk(read_first, sizes):
+    """Read-outs and states of both against the recurrence in 64 bits from the same 32-bit inputs, root mean square: the
+    chunks' order of sums costs no precision."""
+    h = hip()
+    H, D, V = sizes
+    n, gen = 1030, torch.Generator().manual_seed(D + V)
+    rand = lambda *shape: torch.randn(*shape, generator=gen).to(DEV)
+    q, k, v, z, bias, start = rand(n, H * D), rand(n, H * D), rand(n, H * V), rand(n, H * D) * 1.5, rand(H * D) + (-1.0 if read_first else 2.0), rand(1, H * D * V)
+    bonus, q_scale = (rand(H, D) * 0.5, 1.0) if read_first else (None, D ** -0.5)
+    zz = (z + bias).to(F64)
+    w = (torch.exp(-torch.exp(zz)) if read_first else torch.exp(torch.nn.functional.logsigmoid(zz) / 16.0)).view(n, H, D, 1)
+    S, rows = start.to(F64).view(H, D, V), []
+    for t in range(n):
+        kv = k[t].to(F64).view(H, D, 1) * v[t].to(F64).view(H, 1, V)
+        if not read_first:
+            S = w[t] * S + kv
+        read = S + bonus.to(F64)[:, :, None] * kv if read_first else S
+        rows.append((q[t].to(F64).view(H, 1, D) * q_scale @ read).view(-1))
+        if read_first:
+            S = w[t] * S + kv
+    want, off = torch.stack(rows), []
+    for ctx in (None, step_context([[0]], 4096, [0], [n], slots=[0])):
+        state, dev = start.clone(), lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+        out = h.decay_scan(q, k, v, z, bias, state, dev([0, n]), dev([0]), H, D, V, form="double_exponent" if read_first else "sigmoid_root", tau=16.0,
+                           q_scale=q_scale, bonus=bonus, longest=n, ctx=ctx)
+        off.append([float((a.to(F64) - b).norm() / b.norm()) for a, b in ((out, want), (state.view(H, D, V), S))])
+    (walk, walk_state), (chunks, chunk_state) = off
+    assert 0.0 < chunks <= walk and 0.0 < chunk_state <= walk_state, off      # (the walk is the measure; a state's error grows with its memory)
+
+
 @pytest.mark.parametrize("chunked", [False, True])
 @pytest.mark.parametrize("read_first", [False, True])
 def test_a_token_far_back_is_still_in_the_state(read_first, chunked):

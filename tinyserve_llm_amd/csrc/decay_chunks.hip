@@ -1,5 +1,5 @@
-// Linear attention with a decay per key channel over long portions, in chunks of 64 tokens on the matrix cores, all of it in
-// 32 bits (the walk token by token is in decay_scan.hip, with the two orders of decay and read). With W(s, t] the product of
+// Linear attention with a decay per key channel over long portions, in chunks of 64 tokens on the matrix cores, in
+// 32 bits or more (the walk token by token is in decay_scan.hip, with the two orders of decay and read). With W(s, t] the product of
 // the decays of a channel over the tokens after s up to t, S0 the state before the chunk and tokens counted in the chunk:
 //     o_t = sum_d q_td W(start, t] S0_d + sum_{s <= t} A_ts v_s,   A_ts = sum_d q_td k_sd W(s, t]
 //     S   = W(start, end] S0 + sum_s (k_s W(s, end]) v_s^T
@@ -12,13 +12,15 @@
 // blocks between, from the start of t's block: all at most 1); pairs in one block are walked, the running k_s W(s, t] kept in
 // registers, as the token-by-token kernel does it.
 // What bounds it: the walk is a chain of tokens, 150 ns each however few heads there are (two
-// requests of 2,048 tokens together: 301 µs for 8 heads of 128 x 256, 258 µs for 32 of 64 x 64, and 12 µs for the decays; in
-// chunks 126 and 85 µs). The same tokens in chunks are 3 and 2 GFLOP of 32-bit matrix instructions (157 TFLOP/s) beside the
+// requests of 2,048 tokens together: 532 µs for 8 heads of 128 x 256, 444 µs for 32 of 64 x 64; in
+// chunks 130 and 130 µs). The same tokens in chunks are 3 and 2 GFLOP of 32-bit matrix instructions (157 TFLOP/s) beside the
 // states' trips through memory (34 and 17 MB, three times): what is left is the chain of a workgroup's phases. Error against
-// 64 bits (root mean square, 2,048 tokens): 2.0e-7 for the first heads (the walk: 7.0e-7), 1.05e-7 for the second (0.91e-7),
+// 64 bits (root mean square, 2,048 tokens): 1.7e-7 for the first heads (the walk: 7.0e-7), 0.81e-7 for the second (0.91e-7),
 // of the states 1.5e-7 (7.8e-7) and 5.6e-8 (5.8e-8). A 32-bit instruction takes one number a lane
 // and operand, so operands are fetched as 16 bytes of four steps where the order of the sum allows it, and a wave keeps all
 // 64 tokens of its value columns so that every number of the state is read once.
+#include <type_traits>
+
 #include "chunk_ops.h"
 
 #define DC_THREADS 256
@@ -34,6 +36,9 @@ struct DecayChunks {
 };
 
 static __device__ __forceinline__ float4_t mfma_f32(float a, float b, float4_t acc) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, acc, 0, 0, 0); }
+
+static __device__ __forceinline__ float dc_fma(float a, float b, float c) { return fmaf(a, b, c); }
+static __device__ __forceinline__ double dc_fma(float a, float b, double c) { return fma((double)a, (double)b, c); }
 
 // The logarithm of one token's decay: of sigmoid(z)^(1 / tau) or exp(-exp(z)) (0 past a chunk's end, where q, k and v count as 0). A decay near 1 loses most of what tells it from 1 when it is stored in 32 bits; its logarithm does not,
 // so products of decays are exponentials of sums of these (all of one sign: nothing cancels).
@@ -181,7 +186,11 @@ __global__ void __launch_bounds__(DC_THREADS) decay_chunk_scan_kernel(const Deca
 template <int D, int VT, bool READ_FIRST>
 __global__ void __launch_bounds__(DC_THREADS, 2) decay_chunk_out_kernel(const DecayChunks a) {
   constexpr int DH = D < 64 ? D : 64, ROW = DH + 4, AROW = SS_L + 4;      // (16 rows of 16-byte pieces in different banks)
-  constexpr int SETS = VT == 4 ? 2 : 4;                     // running sums of an output, added at the end
+  // Sums are cut short: 32-bit products run one after the other through a matrix instruction's accumulator, and a long run loses
+  // more than the walk's sums over a few channels a lane. So every 16 channels (or tokens) have PARTS sums that start
+  // from nothing, which are added to one of SETS totals (in runs of 32 products: 1.05e-7, the walk 0.91e-7).
+  constexpr int SETS = VT == 4 ? 1 : 2, PARTS = VT == 4 ? 1 : 2;
+  constexpr float4_t NONE = {0.f, 0.f, 0.f, 0.f};
   __shared__ __attribute__((aligned(16))) float q_s[SS_L][ROW], k_s[SS_L][ROW], w_s[SS_L][ROW], a_s[SS_L][AROW], p_s[4][DH];
   const int c = blockIdx.x, h = blockIdx.y, tok0 = a.chunks[4 * c], len = a.chunks[4 * c + 1];
   const int lane = threadIdx.x % TS_WAVE, wave = wave_index();
@@ -256,8 +265,11 @@ __global__ void __launch_bounds__(DC_THREADS, 2) decay_chunk_out_kernel(const De
         }
         own = (part.x + part.y) + (part.z + part.w);
       }
+      // (read first: these pairs and `own` are most of a row, and the walk's sums of a few channels a lane are good to 0.91e-7; in
+      // 64 bits the rows are good to 0.81e-7, in 32 to 0.98e-7)
+      using sum_t = std::conditional_t<READ_FIRST, double, float>;
       for (int t = 0; t < DC_BLOCK; ++t) {
-        float4 part = make_float4(0.f, 0.f, 0.f, 0.f);
+        sum_t part[4] = {0, 0, 0, 0};
         const bool later = t > r;
 #pragma unroll
         for (int i = 0; i < DH / 16; ++i) {
@@ -266,15 +278,15 @@ __global__ void __launch_bounds__(DC_THREADS, 2) decay_chunk_out_kernel(const De
           const float4 y = make_float4(x.x * w4.x, x.y * w4.y, x.z * w4.z, x.w * w4.w);
           const float4 then = later ? y : x;
           if constexpr (!READ_FIRST) x = then;
-          part.x = fmaf(q4.x, x.x, part.x), part.y = fmaf(q4.y, x.y, part.y);
-          part.z = fmaf(q4.z, x.z, part.z), part.w = fmaf(q4.w, x.w, part.w);
+          part[0] = dc_fma(q4.x, x.x, part[0]), part[1] = dc_fma(q4.y, x.y, part[1]);
+          part[2] = dc_fma(q4.z, x.z, part[2]), part[3] = dc_fma(q4.w, x.w, part[3]);
           if constexpr (READ_FIRST) x = then;
         }
-        float sum = (part.x + part.y) + (part.z + part.w);
+        sum_t sum = (part[0] + part[1]) + (part[2] + part[3]);
         if (READ_FIRST && t == r) sum = own;
         sum += __shfl_xor(sum, 16, TS_WAVE);
         sum += __shfl_xor(sum, 32, TS_WAVE);
-        if (g == 0) a_s[t0 + t][t0 + r] = t >= r ? (d0 > 0 ? a_s[t0 + t][t0 + r] : 0.f) + sum : 0.f;
+        if (g == 0) a_s[t0 + t][t0 + r] = t >= r ? (d0 > 0 ? a_s[t0 + t][t0 + r] : 0.f) + (float)sum : 0.f;
       }
     }
     __syncthreads();
@@ -294,25 +306,26 @@ __global__ void __launch_bounds__(DC_THREADS, 2) decay_chunk_out_kernel(const De
     // A of pairs in different blocks: six blocks of 16 x 16, two a wave for the first two waves and one for the others
     for (int n = wave; n < 6; n += 4) {
       const int jb = n < 3 ? 3 : n < 5 ? 2 : 1, ib = n < 3 ? n : n < 5 ? n - 3 : 0;      // (3,0) (3,1) (3,2) (2,0) (2,1) (1,0)
-      float4_t part[2] = {(float4_t){0.f, 0.f, 0.f, 0.f}, (float4_t){0.f, 0.f, 0.f, 0.f}};
+      float4_t part[DH / 8];
 #pragma unroll
       for (int i = 0; i < DH / 16; ++i) {
-        float4_t& acc = part[i & 1];
         const float4 q4 = *(const float4*)&q_s[jb * DC_BLOCK + r][16 * i + 4 * g];
         float4 k4 = *(const float4*)&k_s[ib * DC_BLOCK + r][16 * i + 4 * g];
         for (int m = ib + 1; m < jb; ++m) {
           const float4 p4 = *(const float4*)&p_s[m][16 * i + 4 * g];
           k4.x *= p4.x, k4.y *= p4.y, k4.z *= p4.z, k4.w *= p4.w;
         }
-        acc = mfma_f32(q4.x, k4.x, acc);
-        acc = mfma_f32(q4.y, k4.y, acc);
-        acc = mfma_f32(q4.z, k4.z, acc);
-        acc = mfma_f32(q4.w, k4.w, acc);
+        part[2 * i] = mfma_f32(q4.y, k4.y, mfma_f32(q4.x, k4.x, NONE));
+        part[2 * i + 1] = mfma_f32(q4.w, k4.w, mfma_f32(q4.z, k4.z, NONE));
       }
+#pragma unroll
+      for (int n2 = DH / 16; n2 > 0; n2 /= 2)
+#pragma unroll
+        for (int i = 0; i < n2; ++i) part[i] += part[i + n2];
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         float& x = a_s[jb * DC_BLOCK + 4 * g + e][ib * DC_BLOCK + r];
-        x = (d0 > 0 ? x : 0.f) + (part[0][e] + part[1][e]);
+        x = (d0 > 0 ? x : 0.f) + part[0][e];
       }
     }
     // the state's share, 16 channels a round
@@ -323,10 +336,16 @@ __global__ void __launch_bounds__(DC_THREADS, 2) decay_chunk_out_kernel(const De
       for (int t = 0; t < 4; ++t) {
         const float4 q4 = *(const float4*)&q_s[t * DC_BLOCK + r][16 * i + 4 * g];
         const float qq[4] = {q4.x * upto.x, q4.y * upto.y, q4.z * upto.z, q4.w * upto.w};
+        float4_t part[PARTS][VT];
 #pragma unroll
         for (int e = 0; e < 4; ++e)
 #pragma unroll
-          for (int j = 0; j < VT; ++j) o[i & 1][t][j] = mfma_f32(qq[e], sv[i % AHEAD][e][j], o[i & 1][t][j]);
+          for (int j = 0; j < VT; ++j) {
+            float4_t& acc = part[e * PARTS / 4][j];
+            acc = mfma_f32(qq[e], sv[i % AHEAD][e][j], e * PARTS % 4 ? acc : NONE);
+          }
+#pragma unroll
+        for (int j = 0; j < VT; ++j) o[i % SETS][t][j] += PARTS == 2 ? part[0][j] + part[PARTS - 1][j] : part[0][j];
         const float4 p4 = *(const float4*)&p_s[t][16 * i + 4 * g];
         upto.x *= p4.x, upto.y *= p4.y, upto.z *= p4.z, upto.w *= p4.w;
       }
@@ -347,11 +366,16 @@ __global__ void __launch_bounds__(DC_THREADS, 2) decay_chunk_out_kernel(const De
     for (int t = s; t < 4; ++t) {
       const float4 a4 = *(const float4*)&a_s[t * DC_BLOCK + r][s * DC_BLOCK + 4 * g];
       const float aa[4] = {a4.x, a4.y, a4.z, a4.w};
-      constexpr int FIRST = SETS - 2;
+      float4_t part[PARTS][VT];
 #pragma unroll
       for (int e = 0; e < 4; ++e)
 #pragma unroll
-        for (int j = 0; j < VT; ++j) o[FIRST + (s & 1)][t][j] = mfma_f32(aa[e], vv[s & 1][e][j], o[FIRST + (s & 1)][t][j]);
+        for (int j = 0; j < VT; ++j) {
+          float4_t& acc = part[e * PARTS / 4][j];
+          acc = mfma_f32(aa[e], vv[s & 1][e][j], e * PARTS % 4 ? acc : NONE);
+        }
+#pragma unroll
+      for (int j = 0; j < VT; ++j) o[s % SETS][t][j] += PARTS == 2 ? part[0][j] + part[PARTS - 1][j] : part[0][j];
     }
   }
   float* dst = a.out + (int64_t)tok0 * a.heads * a.vdim + h * a.vdim + v0 + r;
@@ -363,9 +387,7 @@ __global__ void __launch_bounds__(DC_THREADS, 2) decay_chunk_out_kernel(const De
       if (at < len)
 #pragma unroll
         for (int j = 0; j < VT; ++j) {
-          float y = o[0][t][j][e] + o[1][t][j][e];
-          if constexpr (SETS == 4) y += o[2][t][j][e] + o[3][t][j][e];
-          dst[(int64_t)at * a.heads * a.vdim + 16 * j] = y;
+          dst[(int64_t)at * a.heads * a.vdim + 16 * j] = SETS == 2 ? o[0][t][j][e] + o[SETS - 1][t][j][e] : o[0][t][j][e];
         }
     }
 }

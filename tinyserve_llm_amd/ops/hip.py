@@ -2680,11 +2680,12 @@ DECAY_FORMS = {"sigmoid_root": 0, "double_exponent": 1}
 DECAY_MAX_DIM = 1024
 DECAY_FULL_WORKGROUPS = 512      # workgroups of four waves from which a step keeps them (fewer: one wave each, four times as many)
 # Tokens of a request from which its portion is worked in chunks of 64. One request, walked and in chunks, µs: 32 heads of 64 channels 128
-# tokens 34 and 25, 512 115 and 30, 768 169 and 39, 2,048 438 and 70; 8 heads of 128 by 256 values 320 tokens 78 and 78, 512 119 and 87, 768
-# 173 and 88, 2,048 442 and 106 (16 requests of 1,024 together: 877 and 472; 1,722 and 620). So chunks are the faster from 128 (up to 64 channels) or
+# tokens 33 and 27, 512 115 and 32, 768 170 and 42, 2,048 440 and 77; 8 heads of 128 by 256 values 320 tokens 77 and 72, 512 118 and 76, 768
+# 174 and 78, 2,048 442 and 94 (16 requests of 1,024 together: 882 and 503; 1,721 and 536). So chunks are the faster from 128 (up to 64 channels) or
 # 320 tokens (128) on. But they add in another order, and a model with routed experts shows it: with the contexts of 48 decoded requests (350
 # to 700 tokens) in chunks, one row in six runs of 48 took another expert at a near tie and moved by 0.13 of its norm. So
-# a portion keeps the walk's bits, which do not depend on how a request is cut into steps, until chunks take half the time or less at every head size.
+# a portion keeps the walk's bits, which do not depend on how a request is cut into steps, until chunks take half the time or less of one request's
+# walk at every head size.
 DECAY_CHUNKS_FROM = 768
 DECAY_CHUNK_DIMS = (32, 64, 128)
 DECAY_WIDE_UP_TO = 4             # tokens of a step's longest portion up to which a wave owns 64 value columns instead of 16
@@ -2702,7 +2703,7 @@ def decay_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, z: torch.Tenso
     `longest`: the most tokens any request feeds in the step (None: unknown); steps of few tokens a request are cut into
     fewer, wider slices of the value columns (the result is the same bit for bit). With `ctx` (the packed step's context, whose
     requests these are) requests that feed at least `DECAY_CHUNKS_FROM` tokens are worked in chunks on the matrix cores where
-    the sizes allow it (`decay_chunks_take`): the same 32-bit sums in another order, so a request's rows then depend on how
+    the sizes allow it (`decay_chunks_take`): the same sums in another order, no further from 64 bits, so a request's rows then depend on how
     its tokens are cut into steps."""
     _gpu(q, k, v, z, z_bias, state, cu_seqlens, state_slots, bonus)
     T = q.shape[0]

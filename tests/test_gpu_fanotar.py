@@ -397,6 +397,22 @@ def test_tiles_through_lds_give_the_narrower_tiles_sums(sizes, tile_rows):
         assert torch.equal(a[taken], b[taken])
 
 
+@pytest.mark.parametrize("sizes", [(3, 512, 40, 200), (2, 768, 131, 300), (5, 1024, 260, 700), (16, 2048, 64, 640)])
+def test_tiles_of_128_rows_are_as_good_as_the_narrow_ones(sizes):
+    """Where the rule takes tiles of 128 rows in the place of those of 16, the sums are the same bits; against 64 bits the other
+    wide tiles are further off."""
+    h = hip()
+    E, K, N, n = sizes
+    gen = torch.Generator().manual_seed(K)
+    x, w = torch.randn(n, K, generator=gen).bfloat16().to(DEV), (torch.randn(E, 2 * N, K, generator=gen) * K ** -0.5).bfloat16().to(DEV)
+    ids = torch.randint(0, E, (n, 1), generator=gen, dtype=torch.int32).to(DEV)
+    out = {rows: h.moe_gemm(x, w, h.moe_group(ids, E, rows), torch.float32, per_token=True) for rows in (16, 64, 128)}
+    assert torch.equal(out[16], out[128])
+    assert torch.equal(*(h.moe_gemm(x, w, h.moe_group(ids, E, rows), torch.bfloat16, per_token=True, glu=(1.2, 1.702, 1.0)) for rows in (16, 128)))
+    want = torch.stack([x[t].double() @ w[int(e)].double().T for t, e in enumerate(ids[:, 0].tolist())])
+    assert float((out[128].double() - want).norm()) < float((out[64].double() - want).norm())
+
+
 @pytest.mark.parametrize("tile_rows", [128, 256])
 def test_wide_tiles_over_a_reduction_beyond_32_bit_offsets(tile_rows):
     """Rows of more than 2^22 elements (256 of them lie further apart than 31 bits of bytes): the narrower tiles' bits, and in size

@@ -171,6 +171,9 @@ def test_expert_tiles_are_the_fastest_that_were_timed():
     assert hip.moe_tile_rows(31 * 16, 16, bf, (2048, 1024)) == 16 and hip.moe_tile_rows(4096, 4, torch.float32, (2048, 1024)) == 16
     assert hip.moe_tile_rows(4096, 4, bf, (2048, 96)) == 64 and hip.moe_tile_rows(4096, 4, bf, (2048, 40)) == 16
     assert hip.moe_tile_rows(4096, 4, bf) == 128
+    # up to 63 pairs an expert only tiles whose sums are the narrow tiles' bits join them
+    assert hip.moe_tile_rows(40 * 16, 16, bf, (2048, 1024)) == 128 and hip.moe_tile_rows(40 * 16, 16, bf, (2048, 960)) == 16
+    assert hip.moe_tile_rows(40 * 64, 64, bf, (2048, 256)) == 16 and hip.moe_tile_rows(64 * 64, 64, bf, (2048, 256)) == 128
 
 
 def test_each_fault_of_a_cache_is_named():

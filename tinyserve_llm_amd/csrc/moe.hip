@@ -14,7 +14,9 @@
 //     matrix; with `glu` the matrix holds gate rows, then up rows, and the capped gated unit
 //     g = min(gate, L), u = clamp(up, -L, L), y = g sigmoid(slope g) (u + shift) leaves instead of the sums.
 //     Without `glu`, `act` 1 squares the sums' positive parts on their way out (experts of the form W_down relu(W_up h)^2).
-//     Every row's sums run over k in ascending order whatever the tile it lands in.
+//     Every row's sums run over k in ascending order whatever the tile it lands in, in one stretch (tiles of 64 and 256 rows) or
+//     four that are then added in order (16 rows; 128 where the reduction is 512 or more in multiples of 256): the same bits
+//     within either kind, and 2.7e-7 and 1.3e-7 from 64 bits over 2,048.
 //   * `ts_moe_combine`: out[token] = sum over its choices, in order, of weight * the pair's row (+ a shared
 //     expert's row, times a gate per token if there is one). A choice at or beyond `real` is an identity expert: it
 //     has no matrices, `ts_moe_group` leaves its pairs out of every tile, and its row is the token's input itself.
@@ -525,6 +527,9 @@ moe_gemm_stream_kernel(TO* __restrict__ out, const bf16_t* __restrict__ x, const
   moe_store4(orow + c0, y, N - c0);
 }
 
+// Steps of 64 of k in a stretch of the tiles of 128 rows (a whole number of stretches).
+static __device__ __forceinline__ int moe_stretch(int K) { return K >= 512 && K % 256 == 0 ? K / 256 : K / 64; }
+
 // Tiles of 128 or 256 rows, for steps that give an expert dozens or hundreds of rows: the gated product's scheme (gemm_glu.hip)
 // with the rows of x gathered by pair, the matrix the tile's expert's, and the rows of y stored at their pairs' places. A
 // workgroup of eight waves takes BM rows by as many rows of W (with GLU half gate, half up rows, whose sums meet in one lane), 64
@@ -604,6 +609,16 @@ moe_gemm_lds_kernel(TO* __restrict__ out, const bf16_t* __restrict__ x, const bf
   for (int j = 0; j < TN; ++j)
 #pragma unroll
     for (int i = 0; i < TM; ++i) acc[j][i] = (float4_t){0.f, 0.f, 0.f, 0.f};
+  // (tiles of 128 rows have the registers for it: four stretches of k, so that the sums are as good as the narrow tiles')
+  constexpr bool STRETCHES = BM == 128;
+  const int stretch = moe_stretch(K);
+  float4_t total[STRETCHES ? TN : 1][STRETCHES ? TM : 1];
+  int left = stretch;
+  if constexpr (STRETCHES)
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int i = 0; i < TM; ++i) total[j][i] = (float4_t){0.f, 0.f, 0.f, 0.f};
   fetch_x(), next_x();
   fetch_w(), next_w();
   fetch_w(), next_w();
@@ -644,7 +659,20 @@ moe_gemm_lds_kernel(TO* __restrict__ out, const bf16_t* __restrict__ x, const bf
     MOE_MULTIPLY(1)
     MOE_DEAL(NX)
     next_x();
+    if constexpr (STRETCHES)
+      if (--left == 0) {
+        left = stretch;
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+          for (int i = 0; i < TM; ++i) total[j][i] += acc[j][i], acc[j][i] = (float4_t){0.f, 0.f, 0.f, 0.f};
+      }
   }
+  if constexpr (STRETCHES)
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int i = 0; i < TM; ++i) acc[j][i] = total[j][i];
 #undef MOE_READ
 #undef MOE_MULTIPLY
 #undef MOE_DEAL

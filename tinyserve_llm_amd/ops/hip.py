@@ -2168,7 +2168,8 @@ MOE_WIDE_TILE_ROWS = 64   # or, in bfloat16, where the experts have this many ro
 MOE_LDS_TILE_ROWS = 128   # or tiles of the kernel whose operands both go through LDS (reductions that are multiples of 64),
 MOE_LDS_WIDE_TILE_ROWS = 256
 MOE_LDS_ROUND_US = {128: 21, 256: 60}     # µs of a round of one such tile, by as many rows of W, a compute unit over a reduction of 2,048
-MOE_LDS_FROM = 32         # pairs an expert below which the narrow tiles stay, whose rows have the same bits in a batch of any size
+MOE_LDS_FROM = 32         # pairs an expert below which the narrow tiles stay, whose rows have the same bits in a batch of any size; up to twice
+                          # as many only tiles of 128 rows join them, where their sums are the same bits (moe.hip)
 MOE_MAX_EXPERTS = 1024
 MOE_MAX_TOP = 32
 MOE_MAX_GROUPS = 64
@@ -2224,7 +2225,8 @@ def moe_tile_rows(pairs: int, experts: int, dtype: torch.dtype, k_sizes: "tuple[
     fastest tile: 8 experts of 512 and 256, 32 each: 9 µs (13 and 30 with 128 and 256 rows), 128 each: 15 (16 rows 16, 256 rows 33); 4 of 2,048 and 1,024, 32 each: 34 of
     either (256 rows 74), 512 each: 52 (16 rows 295, 256 rows 84), 1,024 each: 84 of 256 (128 rows 85); 16 of them, 256 each: 99 of 256 (112, 16 rows 607)."""
     if dtype == torch.bfloat16 and all(k % 64 == 0 for k in k_sizes):
-        if len(k_sizes) == 2 and pairs >= MOE_LDS_FROM * experts:
+        few = pairs < 2 * MOE_LDS_FROM * experts
+        if len(k_sizes) == 2 and pairs >= MOE_LDS_FROM * experts and not (few and any(k < 512 or k % 256 for k in k_sizes)):
             width, inner = k_sizes
             ups = 2 * inner if gated else inner
             matrices = 2 * (ups + inner) * width            # bytes of an expert
@@ -2232,6 +2234,8 @@ def moe_tile_rows(pairs: int, experts: int, dtype: torch.dtype, k_sizes: "tuple[
             if pairs < MOE_LDS_TILE_ROWS * experts:         # (whole tiles of 128: never the slower ones)
                 costs[MOE_TILE_ROWS] = 5 + experts * (pairs / experts / MOE_TILE_ROWS + 0.5) * matrices / 4.5e6
             for rows, us in MOE_LDS_ROUND_US.items():
+                if few and rows != MOE_LDS_TILE_ROWS:
+                    continue
                 tiles = experts * max(1.0, pairs / experts / rows + 0.5)
                 rounds = [math.ceil(tiles * -(-n // rows) / COMPUTE_UNITS) * k / 2048 for n, k in ((ups, width), (width, inner))]
                 costs[rows] = 5 + max(us * sum(rounds), experts * matrices / 4.6e6)

@@ -421,6 +421,29 @@ def test_latent_attention_of_several_requests_in_wide_tiles(sizes, mask, monkeyp
             torch.testing.assert_close(out[mine].cpu().to(F64), want, atol=1e-4, rtol=1e-4)
 
 
+@pytest.mark.parametrize("sizes", [(32, 256, 0), (16, 256, 32), (40, 128, 64)])
+@pytest.mark.parametrize("sharp", [1.0, 3.0])
+def test_wide_latent_tiles_are_as_close_to_64_bits_as_narrow_ones(sizes, sharp, monkeypatch):
+    """Softmaxes that a few keys decide as well as flat ones: the error's root mean square is that of the kernel of 32 rows (the
+    same scores and weights; the sums of the weights are made in another order: a hundredth of it)."""
+    h = hip()
+    H, rank, rot = sizes
+    row, n = rank + rot, 520
+    gen = torch.Generator().manual_seed(H + rot)
+    rows = torch.randn(544, row, generator=gen).bfloat16().to(DEV)
+    cache, values = rows.view(17, 32, 1, row), rows[:, :rank].reshape(17, 32, 1, rank).permute(0, 2, 3, 1).contiguous().permute(0, 3, 1, 2)
+    q = torch.randn(n, H, row, generator=gen).bfloat16().float().to(DEV)
+    scores = torch.einsum("thd,kd->htk", q.double().cpu(), rows.double().cpu()) * (sharp * row ** -0.5)
+    scores = scores.masked_fill(torch.arange(544)[None, None] > torch.arange(n)[None, :, None], float("-inf"))
+    want = torch.einsum("htk,kd->thd", torch.softmax(scores, dim=-1), rows[:, :rank].double().cpu())
+    off = []
+    for wide in (False, True):
+        monkeypatch.setattr(h, "latent_wide_tiles", lambda *a: wide)
+        out = h.paged_attention_latent(q, cache, rank, step_context([list(range(17))], 32, [0], [n]), 0, sharp * row ** -0.5, out_dtype=torch.float32, v_cache=values)
+        off.append(float((out.cpu().double() - want).norm() / want.norm()))
+    assert 0.0 < off[1] <= 1.01 * off[0] < 1e-5, off
+
+
 @pytest.mark.parametrize("form", sorted(FORMS))
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("page", [16, 32])

@@ -345,8 +345,7 @@ extern "C" int ts_paged_attention_latent_mfma(void* out, int out_dtype, const fl
 // through LDS, where they go straight from memory, three steps in turn (one worked on, two under way). What bounds it: the
 // matrix cores, 48 products a wave and step of 256 numbers (16 for the scores, 32 for the weights' two bfloat16 terms),
 // beside the wave's softmax; the kernel above reads every token's keys from the second-level cache anew (2 GB for 2,048
-// tokens over 256 numbers: 577 us, this one 122). The reference maximum of a row is raised only where a score
-// exceeds it by 2^8, so that outputs are rarely rescaled. In LDS a key's 16-byte pieces are turned by the key's place among
+// tokens over 256 numbers: 560 us, this one 128). In LDS a key's 16-byte pieces are turned by the key's place among
 // the 16 that an operand takes, a value column's four by half the column's number: an operand's read then meets every bank once.
 #define LP_WAVES 8
 #define LP_ROWS (16 * LP_WAVES)
@@ -440,12 +439,17 @@ latent_attention_tiles_kernel(TO* __restrict__ out, const float* __restrict__ q,
     const unsigned char* at = lds + slot * STEP;
     slot = slot + 1 == LP_RING ? 0 : slot + 1;
     const int kb = kb0 + 32 * step;
-    float4_t st[2] = {(float4_t){0.f, 0.f, 0.f, 0.f}, (float4_t){0.f, 0.f, 0.f, 0.f}};
+    // (a score's pieces in four sums, added in the order of the kernel above, whose scores these are bit for bit: in one sum
+    // of all its pieces the rows were 1.9e-6 from 64 bits instead of 1.1e-6)
+    float4_t st[2], piece[4][2];
 #pragma unroll
     for (int c = 0; c < CP; ++c)
 #pragma unroll
       for (int tau = 0; tau < 2; ++tau)
-        st[tau] = mfma32v(*(const u32x4_t*)(at + kat[c & 3] + (c >> 2) * 256 + tau * (4 * SL * 16)), qf[c], st[tau]);
+        piece[c & 3][tau] = mfma32v(*(const u32x4_t*)(at + kat[c & 3] + (c >> 2) * 256 + tau * (4 * SL * 16)), qf[c],
+                                    c < 4 ? (float4_t){0.f, 0.f, 0.f, 0.f} : piece[c & 3][tau]);
+#pragma unroll
+    for (int tau = 0; tau < 2; ++tau) st[tau] = piece[0][tau] + piece[1][tau] + piece[2][tau] + piece[3][tau];
     float s[8];
 #pragma unroll
     for (int j = 0; j < 8; ++j) s[j] = st[j >> 2][j & 3] * scale_log2;
@@ -457,12 +461,13 @@ latent_attention_tiles_kernel(TO* __restrict__ out, const float* __restrict__ q,
       }
     }
     float top = fmaxf(fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3])), fmaxf(fmaxf(s[4], s[5]), fmaxf(s[6], s[7])));
-    if (__any(top > m + 8.f)) {                              // (m = -inf: any key at all)
-      top = row_max(top);
-      const float m_new = top > m + 8.f ? top : m;
-      const float alpha = m_new == m ? 1.f : fast_exp2(m - m_new);
+    // (the reference is the row's largest score so far, whose weight of 1 is exact in the first of its two terms: raised only
+    // where a score exceeded it by 2^8, it cost rows that one key decides half as much precision again, 2.0e-6 for 1.3e-6)
+    float alpha = 1.f;
+    if (__any(top > m)) {                                    // (m = -inf: any key at all)
+      const float m_new = fmaxf(m, row_max(top));
+      alpha = m_new == -INFINITY ? 1.f : fast_exp2(m - m_new);
       m = m_new;
-      l *= alpha;
 #pragma unroll
       for (int i = 0; i < VB; ++i)
 #pragma unroll
@@ -478,7 +483,7 @@ latent_attention_tiles_kernel(TO* __restrict__ out, const float* __restrict__ q,
       hi[j] = pack_bf16(p0, p1);
       lo[j] = pack_bf16(p0 - __uint_as_float(hi[j] << 16), p1 - __uint_as_float(hi[j] & 0xffff0000u));
     }
-    l += sum;
+    l = l * alpha + sum;
 #pragma unroll
     for (int i = 0; i < VB; ++i) {
       const u32x4_t vf = *(const u32x4_t*)(at + vat + i * 1024);

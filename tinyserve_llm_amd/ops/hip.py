@@ -2464,8 +2464,8 @@ def heads_gemm(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, gate: torch.
 LATENT_TILE_ROWS = 32     # rows (token, head) of a workgroup of the matrix-core kernel
 LATENT_WIDE_TILE_ROWS = 128    # and of its form for steps of many tokens,
 LATENT_MANY_ROWS = 8192   # which takes steps of at least so many rows: from here the kernel of 32 rows has 256 workgroups and cuts no keys
-LATENT_MANY_SHORT_ROWS = 12288 # (or so many, where nobody reads more than
-LATENT_SHORT_REACH = 64        # so many keys: 128 heads, 64 tokens 12.9 µs and with wide tiles 14.8, 96 tokens 20.2 and 16.9),
+LATENT_MANY_SHORT_ROWS = 9216  # (or so many, more than a round of that kernel, where nobody reads more than
+LATENT_SHORT_REACH = 128       # so many keys: 128 heads, 64 tokens 12.7 µs and with wide tiles 13.4, 80 tokens 19.1 and 15.2),
 LATENT_WIDE_FILL = 0.35        # and whose wide tiles are this full on average (a decoded token is a tile of its own)
 LATENT_MAX_SPLITS = 16    # stretches a tile's keys may be cut into,
 LATENT_FEW_GROUPS = 512   # where the step has fewer workgroups than half of this
@@ -2485,8 +2485,8 @@ def latent_wide_tiles(cu_seqlens: "list[int]", heads: int, reach: int) -> bool:
     """Whether a step of more than decoded tokens (request i feeds cu_seqlens[i + 1] - cu_seqlens[i]), nobody of which sees more
     than `reach` keys, is the faster in tiles of `LATENT_WIDE_TILE_ROWS` rows: eight waves share a tile's keys where the
     kernel of 32 rows reads them anew for each, but a tile of a token of few heads is mostly padding. Rows of 256 numbers,
-    narrow and wide: 32 heads, 2,048 tokens 557 and 115 µs, 256 tokens 24.3 and 20.7, 300 decoded tokens (contexts of 1,000) beside a
-    prompt of 2 89 and 99, of 128 92 and 101, 256 beside one of 256 87 and 75; 48 heads, 300 beside one of 2 145 and 100; 128 heads 229 and 112."""
+    narrow and wide: 32 heads, 2,048 tokens 560 and 128 µs, 256 tokens 24.8 and 22.5, 300 decoded tokens (contexts of 1,000) beside a
+    prompt of 2 89 and 102, of 128 90 and 105, 256 beside one of 256 87 and 79; 48 heads, 300 beside one of 2 145 and 105; 128 heads 232 and 123."""
     rows = cu_seqlens[-1] * heads
     if rows < (LATENT_MANY_ROWS if reach > LATENT_SHORT_REACH else LATENT_MANY_SHORT_ROWS):
         return False

@@ -134,6 +134,14 @@ def test_a_step_of_few_tokens_finishes_like_one_of_many(few, shape):
     assert int(found[0][3]) <= found[0][1].numel(), "nothing but the step's own slots is written"
 
 
+@pytest.mark.parametrize("few", [256, 257, 700, 1023])
+@pytest.mark.parametrize("shape", [(1, 1, 32, 32, 32, False), (1, 1, 24, 32, 24, True), (2, 1, 32, 8, 16, False)])
+def test_steps_of_few_tokens_whose_values_leave_apart(few, shape):
+    """From 256 tokens on the values leave through their own kernel, and a token of one query and one key head gives a
+    workgroup of the kernel for few tokens 32 tokens' angles at once, the most that its table must hold."""
+    test_a_step_of_few_tokens_finishes_like_one_of_many(few, shape)
+
+
 # ---- attention inside chunks with learned sinks -----------------------------------------------------
 
 def chunk_case(dtype, H, G, D, V, page, length, queries, stand_out, scale, chunk, seed=0, sink_value=None, portion_from=None):

@@ -238,7 +238,10 @@ qkv_finish_pieces_kernel(TO* __restrict__ q_out, TO* __restrict__ k_cache, TO* _
 // cosine calls a thread, one after the other, in code that every wave fetches anew. Here a workgroup's threads take the angles
 // of its tokens once, side by side, and leave them in LDS while the pieces are on their way (5 to 48 tokens: 10 to 11 µs -> 5,
 // about what an empty launch takes).
-#define AG_FEW_ANGLES 640      // (a workgroup of 256 threads spans at most 85 / GS + 2 tokens of three or more heads, of up to 4 GS pairs each)
+// Angles of a workgroup of 256 threads: with three or more heads it spans at most 85 / GS + 2 tokens of up to 4 GS pairs each (340 + 8 GS,
+// 596 for the largest head); with two, the fewest (a query and a key head, where the values leave through the tile kernel), a token's 2 GS
+// threads divide 256 and it spans 128 / GS whole tokens: 512.
+#define AG_FEW_ANGLES 640
 template <typename TI, typename TO, int GS>
 __global__ void __launch_bounds__(AG_WAVES * TS_WAVE)
 qkv_finish_few_kernel(TO* __restrict__ q_out, TO* __restrict__ k_cache, TO* __restrict__ v_cache, const TI* __restrict__ qkv,

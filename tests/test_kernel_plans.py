@@ -149,6 +149,13 @@ def test_gated_products_take_the_unit_along_where_that_is_faster():
     assert hip.glu_pays(256, 16384, 2048, 4) and hip.glu_pays(2048, 16384, 2048, 4) and hip.glu_pays(512, 8192, 2048, 4)
 
 
+def test_units_of_few_rows_ride_along_where_that_is_faster():
+    along = [(1, 1024, 512), (8, 2048, 1024), (1, 4096, 2048), (8, 16384, 2048), (16, 2048, 2048), (4, 8192, 3072), (8, 28672, 4096), (16, 28672, 4096), (1, 8192, 4096)]
+    apart = [(1, 1024, 2560), (8, 1024, 3072), (4, 2048, 3072), (1, 1024, 4096), (16, 1024, 4096), (8, 4096, 4096), (4, 28672, 4096), (1, 16384, 4096)]
+    assert [hip.few_rows_unit_pays(*c) for c in along] == [True] * len(along)
+    assert [hip.few_rows_unit_pays(*c) for c in apart] == [False] * len(apart)
+
+
 def test_gated_product_tiles_follow_the_rounds():
     assert [hip.glu_plan(m, 16384)[0] for m in (256, 999, 1514, 2048)] == [2, 0, 1, 0]
     for rows in (1, 128, 129, 300, 5000):

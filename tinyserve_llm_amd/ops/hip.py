@@ -1623,6 +1623,16 @@ def _skinny_serves(rows: int, n: int, k: int) -> bool:
             and (rows <= SKINNY_FUSED_ROWS or n * k <= SKINNY_WIDE_ELEMENTS))
 
 
+def few_rows_unit_pays(rows: int, n: int, k: int) -> bool:
+    """Whether up to 16 rows of a capped gated unit against [n, k] are the faster with the unit on the 16-row form's way out (n / 32
+    workgroups) than as a plain product, up to 8 rows by the 8-row form (n / 8), and the unit's kernel. Measured with the down projection
+    behind it, apart and here, µs: n 2,048, k 1,024 8.1 and 7.5, k 2,048 9.0 and 9.4, k 4,096 11.3 and 13.3 (9 rows 14.1 and 14.6); n 4,096, k 2,048
+    11.3 and 10.7, k 4,096 15.5 and 16.5; n 8,192, k 4,096 23.9 and 23.6; n 28,672, k 4,096 1 row 67.7 and 72.0, 8 rows 78.4 and 76.0."""
+    if k >= 4096:
+        return n > 4096 and (rows > SKINNY8_FEW_ROWS or n < 16384)
+    return rows > SKINNY8_MAX_ROWS or k < 2048 or n >= 4096
+
+
 def many_rows(x: torch.Tensor, weight: torch.Tensor, packed: "StreamingCopies | None" = None) -> bool:
     """Whether a plain 32-bit product of these operands goes to a kernel for many rows (by `many_rows_products`) and to none
     of the weight-streaming ones."""

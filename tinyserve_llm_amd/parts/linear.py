@@ -87,15 +87,16 @@ def few_rows_unit(x: torch.Tensor, weight: torch.Tensor, packed: hip.StreamingCo
                   unit: tuple[str, float, float, float]) -> "torch.Tensor | hip.PackedRows8 | None":
     """The gated unit (form, limit, slope, up_shift: `hip.capped_glu`) of few rows of x against W = [gate rows | up rows] by
     the kernel that makes the product, which takes it from its 32-bit sums on the way out; `feeds` as for `linear`. None: no
-    such kernel serves the operands. Above the rows of the 8-row form it is the kernel that a plain product goes to as well, so the unit has the bits of the
-    two calls; the few rows that leave the 8-row form for this get a launch less (4 to 5 µs of a decode step's layer)."""
+    such kernel serves the operands, or it would be the slower way (`hip.few_rows_unit_pays`). Above the rows of the 8-row form it is
+    the kernel that a plain product goes to as well, so the unit has the bits of the two calls."""
     if not (_streams(x, weight) and weight.shape[0] % 32 == 0):
         return None
     rows, (n, k) = x.shape[0], weight.shape
     by16 = None if packed is None else packed.by16
     if by16 is not None and hip.rows64_takes(rows, n, k) and n % 128 == 0:
         return hip.gemm_rows64(x, by16, glu=True, unit=unit)
-    if hip.skinny_fuses(rows, k, False, True) and (rows <= hip.SKINNY_FUSED_ROWS or hip._skinny_serves(rows, n, k)):
+    if (hip.skinny_fuses(rows, k, False, True) and (rows <= hip.SKINNY_FUSED_ROWS or hip._skinny_serves(rows, n, k))
+            and hip.few_rows_unit_pays(rows, n, k)):
         pack8 = hip.rows8_reader_steps(rows, feeds) if PACKED_ROWS_MIN <= rows <= 8 else 0
         if pack8 and (n // 2) % (64 * pack8):
             pack8 = 0

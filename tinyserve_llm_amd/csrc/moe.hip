@@ -31,7 +31,9 @@
 #define MOE_ROUTE_CHUNK 2048      // elements of a token's row that lie in LDS at a time
 #define MOE_ROUTE_THREADS 1024    // sixteen waves: an expert each at a time, so that a step of few tokens has all its loads in flight at once
 
-template <typename TX>
+// BY4: the router's rows are read in 16-byte pieces (a width that is a multiple of 4, from an aligned start); other widths have a
+// kernel of their own, whose loads the pieces' registers would hold up (64 tokens over 2,049, 18 rows: 13.4 µs, 16.7 in one kernel).
+template <typename TX, bool BY4>
 __global__ void __launch_bounds__(MOE_ROUTE_THREADS)
 moe_route_kernel(int32_t* __restrict__ ids_out, float* __restrict__ w_out, const TX* __restrict__ x,
                  const float* __restrict__ router, const float* __restrict__ correction, int num_tokens, int K, int E, int top,
@@ -46,19 +48,18 @@ moe_route_kernel(int32_t* __restrict__ ids_out, float* __restrict__ w_out, const
   const int t0 = blockIdx.x * MOE_ROUTE_TOKENS;
   const int nt = min(MOE_ROUTE_TOKENS, num_tokens - t0);
   for (int i = threadIdx.x; i < MOE_ROUTE_TOKENS * rows; i += MOE_ROUTE_THREADS) s_s[i] = 0.f;
-  const bool by4 = K % 4 == 0 && ((uintptr_t)router & 15) == 0;     // (rows of the router in 16-byte pieces)
   constexpr int PER = 16 / sizeof(TX);                              // elements of a 16-byte piece of x
   const bool whole = K % PER == 0 && ((uintptr_t)x & 15) == 0;
   // A stretch of the rows into LDS, then every wave takes experts in turn: a lane reads the router's row side by
   // side with its neighbours, all of a stretch's pieces asked for before the first is used. A step of few tokens is bound
   // by the chain of these trips: a wave's first row of the router is on its way while the tokens' rows are, and each
   // further one while the sums of the one before go through the wave (48 tokens over 2,048, 18 rows: 12.0 -> 9.5 µs; 2,048 tokens 22.0 -> 19.2).
-  constexpr int PIECES = MOE_ROUTE_CHUNK / (4 * TS_WAVE);
+  constexpr int PIECES = BY4 ? MOE_ROUTE_CHUNK / (4 * TS_WAVE) : 1;
   float4 w[PIECES];
   for (int k0 = 0; k0 < K; k0 += MOE_ROUTE_CHUNK) {
     const int kn = min(MOE_ROUTE_CHUNK, K - k0);
     const auto ask = [&](int e) {
-      if (!by4 || e >= rows) return;
+      if (!BY4 || e >= rows) return;
 #pragma unroll
       for (int i = 0; i < PIECES; ++i) {
         const int k = 4 * (lane + TS_WAVE * i);
@@ -93,7 +94,7 @@ moe_route_kernel(int32_t* __restrict__ ids_out, float* __restrict__ w_out, const
       float acc[MOE_ROUTE_TOKENS];
 #pragma unroll
       for (int r = 0; r < MOE_ROUTE_TOKENS; ++r) acc[r] = 0.f;
-      if (by4) {
+      if constexpr (BY4) {
 #pragma unroll
         for (int i = 0; i < PIECES; ++i) {
           const int k = 4 * (lane + TS_WAVE * i);
@@ -209,13 +210,16 @@ extern "C" int ts_moe_route(int32_t* ids_out, float* w_out, const void* x, int x
     return TS_BAD_SHAPE;
   const unsigned blocks = (num_tokens + MOE_ROUTE_TOKENS - 1) / MOE_ROUTE_TOKENS;
   const size_t lds = (size_t)MOE_ROUTE_TOKENS * (2 * (E + extras) + MOE_ROUTE_CHUNK) * sizeof(float);
-  if (x_dtype == 0)
-    moe_route_kernel<float><<<blocks, MOE_ROUTE_THREADS, lds, stream>>>(ids_out, w_out, (const float*)x, router, correction,
-                                                                        num_tokens, K, E, top, scale, normalize, scoring, extras, extra_out, groups, keep);
-  else if (x_dtype == 1)
-    moe_route_kernel<bf16_t><<<blocks, MOE_ROUTE_THREADS, lds, stream>>>(ids_out, w_out, (const bf16_t*)x, router, correction,
-                                                                         num_tokens, K, E, top, scale, normalize, scoring, extras, extra_out, groups, keep);
+  const bool by4 = K % 4 == 0 && ((uintptr_t)router & 15) == 0;
+#define MOE_ROUTE(TX, BY4) \
+  moe_route_kernel<TX, BY4><<<blocks, MOE_ROUTE_THREADS, lds, stream>>>(ids_out, w_out, (const TX*)x, router, correction, num_tokens, K, E, top, \
+                                                                        scale, normalize, scoring, extras, extra_out, groups, keep)
+  if (x_dtype == 0 && by4) MOE_ROUTE(float, true);
+  else if (x_dtype == 0) MOE_ROUTE(float, false);
+  else if (x_dtype == 1 && by4) MOE_ROUTE(bf16_t, true);
+  else if (x_dtype == 1) MOE_ROUTE(bf16_t, false);
   else return TS_BAD_DTYPE;
+#undef MOE_ROUTE
   return ts_check_launch();
 }
 

@@ -286,6 +286,12 @@ def test_token_shift_in_whole_pieces(dtype, n, width, mixes):
     assert torch.equal(h.token_shift(x, mu, wide[:, 4:4 + width], ctx), h.token_shift(x, mu, apart[:, 3:3 + width], ctx))
 
 
+@pytest.mark.parametrize("n,width,mixes", [(76804, 8, 1), (8540, 72, 5), (601, 1024, 3), (300, 2056, 5)])
+def test_token_shift_of_enough_pieces(n, width, mixes):
+    """The least numbers of rows that go in pieces (76,800 of them in bfloat16), a last workgroup that is not full."""
+    test_token_shift_in_whole_pieces(torch.bfloat16, n, width, mixes)
+
+
 @pytest.mark.parametrize("shared", [True, False])
 def test_heads_norm_weight_and_silu_gate(shared):
     h = hip()

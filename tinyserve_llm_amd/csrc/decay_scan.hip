@@ -463,20 +463,19 @@ token_shift_kernel(T* __restrict__ out, const T* __restrict__ h, const float* __
     Num<T>::st(out + ((int64_t)s * num_tokens + t) * width + i, fmaf(before - x, mu[s * width + i], x));
 }
 
-// The same for rows in whole 16-byte pieces: a thread per (token, eight elements). Bound by the mixes' way to memory: five of
-// 2,048 tokens of 2,048 are 42 MB (an element a thread 22.6 µs, 12.4 now). Steps that make fewer threads than the chip holds
-// four waves a compute unit of stay with an element a thread (48 tokens: 2.9 µs against 4.1).
-#define SHIFT_PIECES_FROM 65536
-template <typename T>
+// The same for bfloat16 rows in whole 16-byte pieces: a thread per (token, eight elements). Bound by the mixes' way to memory: five of
+// 2,048 tokens of 2,048 are 42 MB (an element a thread 22.6 µs, 12.4 now; 512 tokens 7.1 and 6.2, 300 5.3 and 5.1). Steps of fewer pieces stay with
+// an element a thread (256 tokens: 4.5 µs against 4.9, 48 2.9 against 4.1), and so do 32-bit rows (1,024 tokens 12.6 against 13.6).
+#define SHIFT_PIECES_FROM 76800
 __global__ void __launch_bounds__(256)
-token_shift_pieces_kernel(T* __restrict__ out, const T* __restrict__ h, const float* __restrict__ mu, const float* __restrict__ kept,
+token_shift_pieces_kernel(bf16_t* __restrict__ out, const bf16_t* __restrict__ h, const float* __restrict__ mu, const float* __restrict__ kept,
                           int64_t kept_stride, const int32_t* __restrict__ cu_seqlens, const int32_t* __restrict__ seq_of_token,
                           const int32_t* __restrict__ state_slots, int num_tokens, int width, int mixes) {
   const int pieces = width / 8, at = blockIdx.x * 256 + threadIdx.x;
   if (at >= num_tokens * pieces) return;
   const int t = at / pieces, i = 8 * (at - t * pieces);
   const int seq = seq_of_token[t];
-  const T* row = h + (int64_t)t * width + i;
+  const bf16_t* row = h + (int64_t)t * width + i;
   float x[8], step[8];
   const auto load8 = [](const auto* p, float (&v)[8]) {
     if constexpr (sizeof(*p) == 4) {
@@ -499,14 +498,9 @@ token_shift_pieces_kernel(T* __restrict__ out, const T* __restrict__ h, const fl
     load8(mu + s * width + i, y);
 #pragma unroll
     for (int k = 0; k < 8; ++k) y[k] = fmaf(step[k], y[k], x[k]);
-    T* to = out + ((int64_t)s * num_tokens + t) * width + i;
-    if constexpr (sizeof(T) == 4) {
-      *(float4*)to = make_float4(y[0], y[1], y[2], y[3]);
-      *(float4*)(to + 4) = make_float4(y[4], y[5], y[6], y[7]);
-    } else {
-      *(uint4*)to = make_uint4((uint32_t)f2bf(y[0]) | ((uint32_t)f2bf(y[1]) << 16), (uint32_t)f2bf(y[2]) | ((uint32_t)f2bf(y[3]) << 16),
-                               (uint32_t)f2bf(y[4]) | ((uint32_t)f2bf(y[5]) << 16), (uint32_t)f2bf(y[6]) | ((uint32_t)f2bf(y[7]) << 16));
-    }
+    *(uint4*)(out + ((int64_t)s * num_tokens + t) * width + i) =
+        make_uint4((uint32_t)f2bf(y[0]) | ((uint32_t)f2bf(y[1]) << 16), (uint32_t)f2bf(y[2]) | ((uint32_t)f2bf(y[3]) << 16),
+                   (uint32_t)f2bf(y[4]) | ((uint32_t)f2bf(y[5]) << 16), (uint32_t)f2bf(y[6]) | ((uint32_t)f2bf(y[7]) << 16));
   }
 }
 
@@ -528,15 +522,11 @@ extern "C" int ts_token_shift(void* out, const void* h, int dtype, const float* 
   if (width <= 0 || mixes <= 0 || kept_stride < width) return TS_BAD_SHAPE;
   const int64_t blocks = ((int64_t)num_tokens * width + 255) / 256;
   if (blocks > 0x7fffffff) return TS_BAD_SHAPE;
-  if (width % 8 == 0 && kept_stride % 4 == 0 && (((uintptr_t)out | (uintptr_t)h | (uintptr_t)mu | (uintptr_t)kept) & 15) == 0 &&
-      (int64_t)num_tokens * width / 8 >= SHIFT_PIECES_FROM && (int64_t)num_tokens * width <= 0x7ffff800 && (dtype | 1) == 1) {
+  if (dtype == 1 && width % 8 == 0 && kept_stride % 4 == 0 && (((uintptr_t)out | (uintptr_t)h | (uintptr_t)mu | (uintptr_t)kept) & 15) == 0 &&
+      (int64_t)num_tokens * width / 8 >= SHIFT_PIECES_FROM && (int64_t)num_tokens * width <= 0x7ffff800) {
     const unsigned grid = (unsigned)(((int64_t)num_tokens * (width / 8) + 255) / 256);
-    if (dtype == 0)
-      token_shift_pieces_kernel<float><<<grid, 256, 0, stream>>>((float*)out, (const float*)h, mu, kept, kept_stride, cu_seqlens, seq_of_token,
-                                                                 state_slots, num_tokens, width, mixes);
-    else
-      token_shift_pieces_kernel<bf16_t><<<grid, 256, 0, stream>>>((bf16_t*)out, (const bf16_t*)h, mu, kept, kept_stride, cu_seqlens, seq_of_token,
-                                                                  state_slots, num_tokens, width, mixes);
+    token_shift_pieces_kernel<<<grid, 256, 0, stream>>>((bf16_t*)out, (const bf16_t*)h, mu, kept, kept_stride, cu_seqlens, seq_of_token, state_slots,
+                                                        num_tokens, width, mixes);
     return ts_check_launch();
   }
   if (dtype == 0)

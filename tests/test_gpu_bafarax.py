@@ -452,6 +452,36 @@ def test_wide_latent_tiles_are_as_close_to_64_bits_as_narrow_ones(sizes, sharp, 
     assert 0.0 < off[1] <= 1.01 * off[0] < 1e-5, off
 
 
+@pytest.mark.parametrize("listed", [False, True])
+def test_a_step_recorded_before_its_wide_tiles_are_listed(listed, monkeypatch):
+    """From 32 heads on the kernel of 32 rows needs no list of tiles, so a step is recorded as its context comes; where an eager step
+    listed the wide tiles before, they are recorded. Replays with the inputs changed and eager work in between."""
+    h = hip()
+    H, rank, n = 32, 128, 300
+    gen = torch.Generator().manual_seed(5)
+    rows = torch.randn(320, rank, generator=gen).bfloat16().to(DEV)
+    cache, values = rows.view(10, 32, 1, rank), rows.reshape(10, 32, 1, rank).permute(0, 2, 3, 1).contiguous().permute(0, 3, 1, 2)
+    queries = [torch.randn(n, H, rank, generator=gen).bfloat16().float().to(DEV) for _ in range(4)]
+    attend = lambda q, ctx: h.paged_attention_latent(q, cache, rank, ctx, 0, 0.1, out_dtype=torch.float32, v_cache=values)
+    ctx, q = step_context([list(range(10))], 32, [0], [n]), queries[0].clone()
+    if listed:
+        attend(q, ctx)
+    ran, plain_run = [], h._run
+    monkeypatch.setattr(h, "_run", lambda name, code: ran.append(name) or plain_run(name, code))
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = attend(q, ctx)
+    assert ran == ["paged_attention_latent_tiles" if listed else "paged_attention_latent_mfma"]
+    monkeypatch.setattr(h, "latent_wide_tiles", lambda *a: listed)
+    for given in queries:
+        want = attend(given, step_context([list(range(10))], 32, [0], [n]))
+        q.copy_(given)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
+
+
 @pytest.mark.parametrize("form", sorted(FORMS))
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("page", [16, 32])

@@ -2506,12 +2506,16 @@ def latent_wide_tiles(cu_seqlens: "list[int]", heads: int, reach: int) -> bool:
 
 
 def _latent_wide(ctx, heads: int, mask: int) -> bool:
-    """`latent_wide_tiles` of a step, worked out once for every layer of a kind."""
+    """`latent_wide_tiles` of a step, worked out once for every layer of a kind. A step without the host's lists, or recorded into
+    a graph before its tiles were listed, stays with the kernel of 32 rows (which needs no list from 32 heads on)."""
     key = ("latent_wide", heads, mask)
     if key not in ctx.scratch:
+        if not len(ctx.host_context_lens) == len(ctx.host_starts) == ctx.num_seqs:
+            return False
         reach = max(ctx.host_context_lens)
         ctx.scratch[key] = latent_wide_tiles(ctx.host_cu_seqlens, heads, min(reach, abs(mask)) if mask else reach)
-    return ctx.scratch[key]
+    return ctx.scratch[key] and (("latent_tiles", max(1, LATENT_WIDE_TILE_ROWS // heads)) in ctx.scratch
+                                 or not torch.cuda.is_current_stream_capturing())
 
 
 def _latent_tiles(ctx, tile_tokens: int, device) -> torch.Tensor:

@@ -229,6 +229,34 @@ def test_the_bonus_is_for_the_current_token_only_and_tau_roots_the_decay():
     assert float(o) == pytest.approx(8.0 * math.sqrt(0.5), rel=1e-6), "sigmoid(0)^(1/2), applied before the read-out"
 
 
+@pytest.mark.parametrize("listed", [False, True])
+def test_a_step_recorded_before_its_chunks_are_listed(listed):
+    """A long portion is recorded as its context comes, as the walk; where an eager step listed the chunks before, as the
+    chunks. Replays from fresh states with the inputs changed and eager work in between."""
+    h = hip()
+    H, D, V, n = 2, 64, 64, 800
+    gen = torch.Generator().manual_seed(3)
+    rand = lambda *shape: torch.randn(*shape, generator=gen).to(DEV)
+    k, v, z, bias, start = rand(n, H * D), rand(n, H * V), rand(n, H * D), rand(H * D) + 2.0, rand(1, H * D * V)
+    queries, cu, slots = [rand(n, H * D) for _ in range(4)], dev([0, n]), dev([0])
+    scan = lambda q, state, ctx: h.decay_scan(q, k, v, z, bias, state, cu, slots, H, D, V, form="sigmoid_root", tau=2.0, longest=n, ctx=ctx)
+    ctx, q, state = step_context([[0]], 4096, [0], [n], slots=[0]), queries[0].clone(), start.clone()
+    if listed:
+        scan(q, start.clone(), ctx)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = scan(q, state, ctx)
+    for given in queries:
+        want_state = start.clone()
+        want = scan(given, want_state, step_context([[0]], 4096, [0], [n], slots=[0]) if listed else None)
+        q.copy_(given)
+        state.copy_(start)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want) and torch.equal(state, want_state)
+
+
 @pytest.mark.parametrize("read_first", [False, True])
 @pytest.mark.parametrize("sizes", [(2, 64, 128), (3, 20, 64), (1, 256, 256), (2, 128, 72)])
 def test_wide_and_narrow_slices_of_the_columns_give_the_same_bits(read_first, sizes):

@@ -2738,7 +2738,9 @@ def decay_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, z: torch.Tenso
     _need(0 < dim <= DECAY_MAX_DIM and tau > 0, lambda: f"heads of up to {DECAY_MAX_DIM} dimensions, a positive tau")
     out = torch.empty((T, heads * vdim), dtype=torch.float32, device=q.device)
     at_most = 0x7fffffff
-    if ctx is not None and ctx.max_query_len >= DECAY_CHUNKS_FROM and decay_chunks_take(dim, vdim, state, bonus, (q, k, v, z)):
+    # (a step recorded into a graph before its chunks were listed is walked, which takes the lengths from the device)
+    if (ctx is not None and ctx.max_query_len >= DECAY_CHUNKS_FROM and decay_chunks_take(dim, vdim, state, bonus, (q, k, v, z))
+            and (("ssd_chunks", DECAY_CHUNKS_FROM) in ctx.scratch or not torch.cuda.is_current_stream_capturing())):
         _check_step_requests(ctx)
         _need(ctx.num_tokens == T and ctx.num_seqs == S, "the rows are the step's")
         chunks, chunk_cu = _step_chunks(ctx, DECAY_CHUNKS_FROM, q.device)

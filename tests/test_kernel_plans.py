@@ -208,3 +208,11 @@ def test_wide_latent_tiles_where_they_are_full_and_their_walks_long():
     # decoded tokens of few heads: tiles that are mostly padding
     assert not wide(step(2, 300), 32, 1000) and not wide(step(128, 300), 32, 1000) and wide(step(256, 256), 32, 1000) and wide(step(1024, 16), 32, 8000)
     assert wide(step(2, 300), 48, 1000) and wide(step(2, 300), 128, 1000) and wide(step(2, 300), 200, 1000) and not wide(step(2, 2000), 8, 1000)
+
+
+def test_wide_latent_tiles_leave_caches_beyond_their_offsets_to_the_narrow_kernel():
+    def caches(key, dim):
+        return (torch.empty_strided((4, 32, 1, 256), (32 * key, key, key, 1), dtype=torch.bfloat16, device="meta"),
+                torch.empty_strided((4, 32, 1, 128), (128 * dim, 1, 128 * dim, dim), dtype=torch.bfloat16, device="meta"))
+    assert hip.latent_wide_reaches(*caches(256, 32)) and hip.latent_wide_reaches(*caches((1 << 24) - 8, (1 << 22) - 8))
+    assert not hip.latent_wide_reaches(*caches(1 << 24, 32)) and not hip.latent_wide_reaches(*caches(256, 1 << 22))

@@ -2505,6 +2505,12 @@ def latent_wide_tiles(cu_seqlens: "list[int]", heads: int, reach: int) -> bool:
     return rows >= LATENT_WIDE_FILL * tiles * LATENT_WIDE_TILE_ROWS
 
 
+def latent_wide_reaches(cache: torch.Tensor, v_cache: torch.Tensor) -> bool:
+    """Whether a page's keys and values lie close enough for the wide tiles' 31-bit byte offsets from its start (the kernel of
+    32 rows goes by 64-bit addresses)."""
+    return cache.shape[1] * cache.stride(1) < 1 << 29 and v_cache.shape[3] * v_cache.stride(3) < 1 << 29
+
+
 def _latent_wide(ctx, heads: int, mask: int) -> bool:
     """`latent_wide_tiles` of a step, worked out once for every layer of a kind. A step without the host's lists, or recorded into
     a graph before its tiles were listed, stays with the kernel of 32 rows (which needs no list from 32 heads on)."""
@@ -2556,7 +2562,8 @@ def paged_attention_latent(q: torch.Tensor, cache: torch.Tensor, rank: int, ctx,
     mask = -chunk_mask if chunk_mask else int(window)
     if latent_mfma_takes(q, cache, v_cache, rank) and out.dtype in (torch.float32, torch.bfloat16):
         _need(v_cache.shape == (*cache.shape[:3], rank), "the values' view must match the rows'")
-        if ctx.max_query_len > 1 and _latent_wide(ctx, H, mask) and out.data_ptr() % 16 == 0 and bool(library().ts_latent_tiles_takes(rank, row)):
+        if (ctx.max_query_len > 1 and _latent_wide(ctx, H, mask) and out.data_ptr() % 16 == 0 and latent_wide_reaches(cache, v_cache)
+                and bool(library().ts_latent_tiles_takes(rank, row))):
             # many tokens: tiles of four times as many rows, whose keys a workgroup reads once
             tile_tokens = max(1, LATENT_WIDE_TILE_ROWS // H)
             tiles = _latent_tiles(ctx, tile_tokens, q.device)

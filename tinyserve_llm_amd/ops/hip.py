@@ -11,6 +11,8 @@ from __future__ import annotations
 import contextlib
 import ctypes
 import functools
+import importlib.machinery
+import importlib.util
 import math
 import threading
 
@@ -19,6 +21,7 @@ import torch
 from tinyserve_llm_amd.csrc import build as _build
 
 _lib = None
+_calls = None         # the library's own module (calls.cpp): launches of plain operands in one call
 _lock = threading.Lock()
 
 _DTYPE_CODE = {torch.float32: 0, torch.bfloat16: 1}
@@ -32,15 +35,28 @@ class KernelError(RuntimeError):
 
 def library() -> ctypes.CDLL:
     """The kernel library; built on first use if no current build exists. Never a fallback."""
-    global _lib
+    global _lib, _calls
     if _lib is None:
         with _lock:
             if _lib is None:
                 path = _build.find_current() or _build.build(force=True)
                 lib = ctypes.CDLL(path)
                 _declare(lib)
+                loader = importlib.machinery.ExtensionFileLoader("tinyserve_hip_calls", path)
+                module = importlib.util.module_from_spec(importlib.util.spec_from_loader(loader.name, loader))
+                loader.exec_module(module)
+                _calls = module
                 _lib = lib
     return _lib
+
+
+def _native():
+    """The library's own module. Its functions serve the plain case of the functions of the same names here, with
+    everything between Python and the launch made in C++, and give None where something is another way: the function here
+    then goes on by itself, and says what is wrong if something is."""
+    if _calls is None:
+        library()
+    return _calls
 
 
 def _declare(lib: ctypes.CDLL) -> None:
@@ -202,6 +218,9 @@ def rmsnorm(x: torch.Tensor, weight: torch.Tensor, eps: float, residual: torch.T
             ) -> tuple[torch.Tensor, torch.Tensor | None]:
     """(norm(x + residual) * weight, x + residual). With `rows` (int32) only those rows are
     normalised, in that order, and no residual is returned."""
+    done = _native().rmsnorm(x, weight, eps, residual, want_residual) if rows is None else None
+    if done is not None:
+        return done
     _gpu(x, weight, residual, rows)
     _need(x.dim() == 2 and x.is_contiguous(), "rmsnorm input must be contiguous [rows, hidden]")
     hidden = x.shape[1]
@@ -232,6 +251,9 @@ def rope_store(qkv: torch.Tensor, cos_sin: torch.Tensor | None, positions: torch
     layer's view [pages, page_size, nkv, hd] (may be strided over pages and slots); None = no write.
     `cos_sin` None = no rotation; a table narrower than head_dim ([positions, rot], rot even) turns
     the first rot dimensions of every head (j with j + rot / 2) and lets the others pass."""
+    q = _native().rope_store(qkv, cos_sin, positions, slots, k_cache, v_cache, num_heads, num_kv_heads, head_dim)
+    if q is not None:
+        return q
     _gpu(qkv, cos_sin, positions, slots, k_cache, v_cache)
     T = qkv.shape[0]
     row = (num_heads + 2 * num_kv_heads) * head_dim
@@ -807,9 +829,19 @@ def paged_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
     _need(chunk_mask >= 0 and window >= 0 and not (chunk_mask and window), "a sliding window or chunks, both counted in positions")
     if chunk_mask:
         window = -chunk_mask
+    tables = ctx.block_tables[space]
+    key = ("attention_step", q.shape, k_cache.shape, tables.shape)
+    step = ctx.scratch.get(key)
+
+    def planned(step) -> torch.Tensor | None:
+        return _native().attention_step(q, k_cache, v_cache, tables, ctx.seq_of_token, ctx.positions, step[0], scale, window, softcap, sink,
+                                        sinks, slopes, gate, *step[1])
+    if step is not None:         # (an earlier layer of the step has made the plan for these sizes)
+        out = planned(step)
+        if out is not None:
+            return out
     general = softcap > 0 or sink or sinks is not None or slopes is not None or gate is not None
     extra = dict(softcap=softcap, sink=sink, sinks=sinks, slopes=slopes)
-    tables = ctx.block_tables[space]
     # (the tables count in pages of ctx.page_size tokens; the pools may be cut into shorter ones)
     table_page = getattr(ctx, "page_size", 0) or k_cache.shape[1]
     _need(table_page % k_cache.shape[1] == 0, lambda: f"block tables in pages of {table_page} over a cache in pages of {k_cache.shape[1]}")
@@ -822,6 +854,12 @@ def paged_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
             return paged_attention_decode(q, k_cache, v_cache, tables, ctx.seq_of_token, ctx.positions, scale, window,
                                           pages_per_entry=per_entry, leave_split=leave_split and gate is None, gate=gate, **extra)
         lead, tile_tokens, waves, tiles, splits, chunk = _prefill_plan(q, k_cache, ctx, decode_ok)
+        nkv = k_cache.shape[2]
+        split_walk = decode_plan(lead, nkv, q.shape[1] // nkv, q.shape[2], capacity) if lead else (0, 0)
+        ctx.scratch[key] = (tiles, (per_entry, lead, *split_walk, tile_tokens, waves, splits, chunk, ctx.host_cu_seqlens[lead]))
+        out = planned(ctx.scratch[key])
+        if out is not None:
+            return out
         out = torch.empty_like(q)
         if lead:
             paged_attention_decode(q[:lead], k_cache, v_cache, tables, ctx.seq_of_token[:lead], ctx.positions[:lead],
@@ -1233,6 +1271,11 @@ def gemm_rows64(x: torch.Tensor, packed: torch.Tensor, out_dtype: torch.dtype = 
     rows then up rows and the result is silu(gate) * up, [M, N / 2]. With `squares` (and `eps`) x is
     the operand of a `PreparedNorm` and the rows' scales multiply the finished sums. `unit` (with `glu`, a plain
     x): (form, limit, slope, up_shift) of the unit of `capped_glu` in silu's place."""
+    if unit is None or (glu and unit[0] in GLU_ACTIVATIONS):
+        out = _native().gemm_rows64(x, packed, out_dtype is torch.float32, _unit_code(glu, unit), squares, eps,
+                                    *((0.0, 0.0, 0.0) if unit is None else unit[1:])) if out_dtype in _DTYPE_CODE else None
+        if out is not None:
+            return out
     _gpu(x, packed)
     _need(x.dtype == torch.bfloat16 and packed.dtype == torch.bfloat16 and x.dim() == 2 and packed.dim() == 4
           and packed.shape[2:] == (64, 8) and packed.is_contiguous(), "gemm_rows64 takes bfloat16 x [M, K] and pack_weight(W)")
@@ -1285,6 +1328,10 @@ def gemm_rows64_sliced(x: torch.Tensor, packed: torch.Tensor, slices: int, next_
     shared-x kernel with the reduction in `slices` slices (K / slices a multiple of 512), whose 32-bit
     parts a second kernel adds in ascending order. With `next_norm` = (residual or None, weight of the
     norm that follows) the product is not stored: a `PreparedNorm` comes back."""
+    residual, nw = (None, None) if next_norm is None else next_norm
+    done = _native().gemm_rows64_sliced(x, packed, slices, residual, nw) if next_norm is None or nw is not None else None
+    if done is not None:
+        return done if next_norm is None else PreparedNorm(*done)
     _gpu(x, packed)
     _need(x.dtype == torch.bfloat16 and packed.dtype == torch.bfloat16 and x.dim() == 2 and packed.dim() == 4
           and packed.shape[2:] == (64, 8) and packed.is_contiguous(), "gemm_rows64_sliced takes bfloat16 x [M, K] and pack_weight(W)")
@@ -1422,6 +1469,10 @@ def qkv_rope_store_sliced(x: torch.Tensor, packed_rope: torch.Tensor, slices: in
     second kernel that adds the parts, rotates and writes the cache: q [tokens, nh, hd] comes back.
     `packed_rope` = pack_weight_rope(weight, head_dim). With `squares` (and `eps`) x is the operand of
     a `PreparedNorm` and the rows' scales multiply the finished sums."""
+    q = _native().qkv_rope_store_sliced(x, packed_rope, slices, cos_sin, positions, slots, k_cache, v_cache, num_heads, num_kv_heads,
+                                        head_dim, eps, squares)
+    if q is not None:
+        return q
     _gpu(x, packed_rope, cos_sin, positions, slots, k_cache, v_cache)
     _check_squares(squares, x.shape[0])
     M, K = x.shape
@@ -1544,6 +1595,9 @@ def gemm_glu(x: torch.Tensor, weight: torch.Tensor, form: str, limit: float = 0.
     """The gated unit of bfloat16 x [M, K] against a weight [2 F, K] of F gate rows, then F up rows, as bfloat16 [M, F], in
     one kernel for many rows (gemm_glu.hip). `form` "silu_rounded": silu(gate) up of branches rounded to bfloat16 first
     (what `silu_mul` makes of a bfloat16 product); "sigmoid", "relu", "gelu_tanh": `capped_glu` of the 32-bit sums."""
+    y = _native().gemm_glu(x, weight, glu_plan(x.shape[0], weight.shape[0])[0], GLU_FORMS[form], limit, slope, up_shift) if form in GLU_FORMS else None
+    if y is not None:
+        return y
     _gpu(x, weight)
     _need(form in GLU_FORMS, lambda: f"form {form!r}: one of {sorted(GLU_FORMS)}")
     _need(x.dim() == 2 and weight.dim() == 2 and x.shape[1] == weight.shape[1], lambda: f"shapes {tuple(x.shape)} x {tuple(weight.shape)}^T")
@@ -1609,6 +1663,15 @@ def _sliced_serves(rows: int, n: int, k: int, packed: "StreamingCopies | None", 
 
 
 @functools.lru_cache(maxsize=4096)
+def _library_serves(rows: int, n: int, k: int, packed16: bool, out_f32: bool) -> bool:
+    """Whether `linear_bf16` gives a product of these sizes that nothing rides on to the matrix library, with `packed16` where the
+    weight's 16-row copy is there: no kernel of this library takes it, and its rows are whole 16-byte pieces."""
+    if k % 8 or n < 8 or skinny8_takes(rows, n, k) or _skinny_serves(rows, n, k):
+        return False
+    return not (packed16 and (rows64_takes(rows, n, k) or (not out_f32 and n <= ROWS64_PLAIN_MAX_WIDTH and rows64_slices(rows, n, k))))
+
+
+@functools.lru_cache(maxsize=4096)
 def _sliced_route(rows: int, n: int, k: int) -> int:
     """The slices for a product that neither form of the weight-streaming kernel serves; 0: those do, or the slices do not fit."""
     return 0 if skinny8_takes(rows, n, k) or _skinny_serves(rows, n, k) else rows64_slices(rows, n, k)
@@ -1651,6 +1714,13 @@ def linear_bf16(x: torch.Tensor, weight: torch.Tensor, out_dtype: torch.dtype = 
     if isinstance(x, PackedRows8):
         _need(rows8_reader_steps(x.shape[0], weight) == x.steps, "packed rows go to the projection they were made for")
         return gemm_skinny8(x, weight, out_dtype, None if packed is None else packed.by8, next_norm=next_norm)
+    if next_norm is None and _many_rows == "library" and _library_tuning is None and x.dim() == 2 and out_dtype in _DTYPE_CODE:
+        rows, k = x.shape
+        if (_library_serves(rows, weight.shape[0], k, packed is not None and packed.by16 is not None, out_dtype is torch.float32)
+                and x.stride(0) % 8 == 0 and weight.stride(0) % 8 == 0):
+            y = _native().gemm_library(x, weight, out_dtype is torch.float32)
+            if y is not None:
+                return y
     _gpu(x, weight)
     _need(x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16, "linear_bf16 takes bfloat16")
     _need(x.dim() == 2 and weight.dim() == 2 and x.shape[1] == weight.shape[1],
@@ -1735,6 +1805,10 @@ def gemm_library(x: torch.Tensor, weight: torch.Tensor, out_dtype: torch.dtype =
     """bfloat16 x [M, K] · weight [N, K]^T by the vendor's matrix library, called directly with the
     algorithm kept for the shape (see gemm_library.hip). Rows may be strided. The result is bfloat16,
     or the 32-bit sums themselves with `out_dtype` float32."""
+    if _library_tuning is None and out_dtype in _DTYPE_CODE:
+        y = _native().gemm_library(x, weight, out_dtype is torch.float32)
+        if y is not None:
+            return y
     _need(x.stride(1) == 1 and weight.stride(1) == 1, "rows of x and of the weight must be dense")
     _need(out_dtype in (torch.bfloat16, torch.float32), "the library product comes out as bfloat16 or float32")
     M, K = x.shape
@@ -1800,6 +1874,10 @@ def stream_update_norm(x: torch.Tensor, a: torch.Tensor | None = None, b: torch.
     for each given weight norm(x) * weight of the updated rows comes back in `out_dtype` (both norms
     share the row's mean square). With `rows` (int32) nothing is updated and only those rows are
     normalised, in that order."""
+    if rows is None and bias is None and weights[0] is not None and weights[1] is None and out_dtype in _DTYPE_CODE:
+        out = _native().stream_update_norm(x, a, b, mult, weights[0], eps, _DTYPE_CODE[out_dtype])
+        if out is not None:
+            return out, None
     _gpu(x, a, b, bias, rows, *weights)
     _need(x.dtype == torch.float32 and x.dim() == 2 and x.is_contiguous(), "the stream must be contiguous float32 [tokens, width]")
     tokens, width = x.shape
@@ -1924,6 +2002,11 @@ def qkv_finish(qkv: torch.Tensor, freqs: torch.Tensor | None, positions: torch.T
     k turn in their first rot dimensions by position * freqs[i], pair i being dimensions (2i, 2i+1) if
     `interleaved`, else (i, i + rot/2), cosine and sine times `amplitude`. `qk_norm_eps` / `v_norm_eps`: each q
     and k head, and each value head, is then divided by its root mean square (eps inside the root); None: not."""
+    if out_dtype in _DTYPE_CODE:
+        q = _native().qkv_finish(qkv, freqs, positions, slots, k_cache, v_cache, num_heads, num_kv_heads, head_dim, value_dim,
+                                 _DTYPE_CODE[out_dtype], interleaved, qk_norm_eps, v_norm_eps, amplitude)
+        if q is not None:
+            return q
     _gpu(qkv, freqs, positions, slots, k_cache, v_cache)
     T = qkv.shape[0]
     row = (num_heads + num_kv_heads) * head_dim + num_kv_heads * value_dim
@@ -2081,6 +2164,10 @@ def capped_glu(gate_up: torch.Tensor, limit: float, slope: float, up_shift: floa
     """From rows [gate | up] (float32 or `out_dtype`): g = min(gate, limit), u = clamp(up, -limit, limit)
     (limit <= 0: no cap), y = act(g) (u + up_shift) in 32-bit, stored as `out_dtype`; act(g) is g sigmoid(slope g)
     ("sigmoid"), max(g, 0) ("relu") or gelu in its tanh form ("gelu_tanh")."""
+    if activation in GLU_ACTIVATIONS and out_dtype in _DTYPE_CODE:
+        out = _native().capped_glu(gate_up, limit, slope, up_shift, _DTYPE_CODE[out_dtype], GLU_ACTIVATIONS[activation])
+        if out is not None:
+            return out
     _gpu(gate_up)
     _need(activation in GLU_ACTIVATIONS, lambda: f"activation {activation!r}: one of {sorted(GLU_ACTIVATIONS)}")
     _need(gate_up.dim() == 2 and gate_up.shape[1] % 2 == 0 and gate_up.stride(1) == 1 and gate_up.stride(0) >= gate_up.shape[1],
@@ -2687,6 +2774,10 @@ def mlstm_finish(o: torch.Tensor, weight: torch.Tensor | None, gate: torch.Tenso
     """Each head's row of o (float32 [tokens, heads vdim]) divided by its root mean square, times `weight` (float32
     [heads vdim], or [vdim]: one weight that all heads share; None: none), times sigmoid(gate) (float32 [tokens, heads vdim], rows
     may lie apart; with `silu_gate` times gate sigmoid(gate)), as `out_dtype`."""
+    if out_dtype in _DTYPE_CODE:
+        out = _native().mlstm_finish(o, weight, gate, heads, vdim, eps, _DTYPE_CODE[out_dtype], silu_gate)
+        if out is not None:
+            return out
     _gpu(o, weight, gate)
     T = o.shape[0]
     _need(o.dtype == torch.float32 and o.shape == (T, heads * vdim) and o.is_contiguous(), "o must be contiguous float32 [tokens, heads vdim]")
@@ -2813,6 +2904,10 @@ def stream_post_norm(x: torch.Tensor, a: torch.Tensor, post_weight: torch.Tensor
     """The float32 stream x [tokens, width] takes x += a / sqrt(mean(a^2) + post_eps) * post_weight * scale in place (a
     float32, what a branch has made; `scale` float32 [width] or None). With `out_dtype`, the updated rows come back in
     that type: normalised and times `weight` (x / sqrt(mean(x^2) + eps) * weight), or as they are if `weight` is None."""
+    if out_dtype in _DTYPE_CODE:
+        out = _native().stream_post_norm(x, a, post_weight, scale, post_eps, weight, eps, _DTYPE_CODE[out_dtype])
+        if out is not None:
+            return out
     _gpu(x, a, post_weight, scale, weight)
     _need(x.dtype == torch.float32 and x.dim() == 2 and x.is_contiguous() and a.dtype == torch.float32 and a.shape == x.shape and a.is_contiguous(),
           "the stream and the branch's rows must be contiguous float32 [tokens, width]")

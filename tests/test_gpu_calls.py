@@ -70,6 +70,11 @@ def forms():
         for out_dtype in (BF, F32):
             add(f"linear-{m}-{n}-{k}-{skew}-{out_dtype}", hip.linear_bf16, lambda m=m, n=n, k=k, skew=skew, out_dtype=out_dtype: ((rows(m, k, skew=skew), rows(n, k), out_dtype), {}))
             add(f"library-{m}-{n}-{k}-{skew}-{out_dtype}", hip.gemm_library, lambda m=m, n=n, k=k, skew=skew, out_dtype=out_dtype: ((rows(m, k, skew=skew), rows(n, k), out_dtype), {}))
+    for m, n, k, skew in ((130, 1024, 2048, 0), (200, 2048, 4096, 16), (40, 72, 384, 8)):
+        for out_dtype, norm in ((BF, None), (F32, None), (BF, True), (BF, False), (F32, True)):
+            add(f"slices-{m}-{n}-{k}-{skew}-{out_dtype}-{norm}", hip.gemm_slices, lambda m=m, n=n, k=k, skew=skew, out_dtype=out_dtype, norm=norm: (
+                (rows(m, k, skew=skew), rows(n, k), 4, 2, out_dtype, None if norm is None else (rows(m, n) if norm else None, vec(n), 1e-5)), {}))
+        add(f"linear-deep-{m}-{n}-{k}", hip.linear_bf16, lambda m=m, n=n, k=k, skew=skew: ((rows(m, k, skew=skew), rows(n, k), F32), {}))
     add("linear-odd-k", hip.linear_bf16, lambda: ((rows(50, 100), rows(40, 100)), {}))
     add("linear-odd-stride", hip.linear_bf16, lambda: ((rows(50, 64, skew=3), rows(40, 64)), {}))
     add("linear-shapes", hip.linear_bf16, lambda: ((rows(50, 64), rows(40, 72)), {}))

@@ -1,0 +1,117 @@
+"""Products of many rows with the reduction in slices (gemm_slices.hip) against the same product in 64 bits, their endings against
+the kernels they stand in for, and the rule that chooses them."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from tinyserve_llm_amd.ops import hip
+from tinyserve_llm_amd.parts.linear import DeferredNorm, NormRequest, linear
+
+BF = torch.bfloat16
+
+
+def operands(rows, n, k, seed=0, x_skew=0):
+    g = torch.Generator().manual_seed(1000 * rows + n + k + seed)
+    x = torch.randn(rows, k + x_skew, generator=g).to(BF).cuda()[:, :k]
+    return x, (torch.randn(n, k, generator=g) * k ** -0.5).to(BF).cuda()
+
+
+# (edges of the tiles' rows and columns, uneven slices, the fewest steps a slice, one slice, rows of x apart)
+FORMS = [(t, s, rows, n, k, skew) for t, (bm, bn, *_) in enumerate(hip.SLICES_TILES)
+         for s, rows, n, k, skew in ((3, bm, bn, 640, 0), (2, bm + 1, bn + 8, 448, 8), (1, 1, 8, 192, 0), (5, 2 * bm - 1, 2 * bn - 8, 1024, 64),
+                                     (16, 37, bn + 64, 3072, 0))]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tile, slices, rows, n, k, skew", FORMS)
+def test_a_product_in_slices(tile, slices, rows, n, k, skew):
+    """32-bit sums of k products: (k + slices) 2^-24 of the sum of their sizes at most; in bfloat16 half a unit in the last place more."""
+    x, w = operands(rows, n, k, x_skew=skew)
+    want, sizes = x.double() @ w.double().T, x.double().abs() @ w.double().abs().T
+    wide = hip.gemm_slices(x, w, tile, slices, torch.float32)
+    bound = (k + slices) * 2.0 ** -24 * sizes
+    assert wide.shape == want.shape and bool(((wide.double() - want).abs() <= bound).all())
+    assert torch.equal(hip.gemm_slices(x, w, tile, slices), wide.to(BF))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows, n, residual", [(129, 2048, True), (3, 8192, True), (200, 1032, False), (33, 264, True)])
+def test_the_norm_that_follows_has_the_bits_of_its_own_kernel(rows, n, residual):
+    x, w = operands(rows, n, 512)
+    g = torch.Generator().manual_seed(n)
+    res = torch.randn(rows, n, generator=g).to(BF).cuda() if residual else None
+    nw = torch.randn(n, generator=g).to(BF).cuda()
+    got, total = hip.gemm_slices(x, w, 0, 2, next_norm=(res, nw, 1e-5))
+    product = hip.gemm_slices(x, w, 0, 2)
+    want, want_total = hip.rmsnorm(product, nw, 1e-5, res)
+    assert torch.equal(got, want) and torch.equal(total, want_total)
+
+
+@pytest.mark.gpu
+def test_numbers_that_are_none_stay_in_their_rows_and_columns():
+    x, w = operands(150, 1024, 2048)
+    x[7, 2000], w[5, 3] = float("nan"), float("inf")
+    y = hip.gemm_slices(x, w, 4, 4, torch.float32)
+    odd = torch.zeros_like(y, dtype=torch.bool)
+    odd[7], odd[:, 5] = True, True
+    assert bool((~torch.isfinite(y) == odd).all())
+
+
+@pytest.mark.gpu
+def test_linear_takes_the_slices_where_the_rule_says_so_and_hands_the_norm_on(monkeypatch):
+    rows, n, k = 160, 2048, 8192
+    assert hip.slices_plan(rows, n, k, "bf16") and hip.slices_plan(rows, n, k, "norm")
+    x, w = operands(rows, n, k)
+    res, nw = torch.randn(rows, n, device="cuda").to(BF), torch.randn(n, device="cuda").to(BF)
+    plan = hip.slices_plan(rows, n, k, "f32")
+    assert torch.equal(linear(x, w, torch.float32), hip.gemm_slices(x, w, *plan, torch.float32))
+    d = linear(x, w, then=NormRequest(nw, 1e-5, res))
+    assert isinstance(d, DeferredNorm) and d.done is not None and d.rows == rows
+    want, total = hip.gemm_slices(x, w, *hip.slices_plan(rows, n, k, "norm"), next_norm=(res, nw, 1e-5))
+    assert torch.equal(d.materialize(), want) and torch.equal(d.residual_out, total)
+    narrow = torch.randn(64, n, device="cuda").to(BF)
+    assert torch.equal(linear(d, narrow), linear(want, narrow))
+
+
+@pytest.mark.gpu
+def test_what_the_slices_do_not_take_is_refused_before_anything_runs():
+    x, w = operands(130, 1024, 2048)
+    nw, res = torch.ones(1024, dtype=BF, device="cuda"), torch.zeros(130, 1024, dtype=BF, device="cuda")
+    for args, kwargs in [((x[:, :2000], w[:, :2000], 0, 2), {}), ((x, w, 5, 2), {}), ((x, w, 0, 11), {}), ((x, w, 0, 0), {}), ((x.float(), w, 0, 2), {}),
+                         ((x, w[:1020], 0, 2), {}), ((x[:, 1:], w[:, 1:], 0, 2), {}), ((x, w, 0, 2, torch.float16), {}),
+                         ((x, w, 0, 2, torch.float32), {"next_norm": (res, nw, 1e-5)}), ((x, w, 0, 2), {"next_norm": (res[:129], nw, 1e-5)}),
+                         ((x, w, 0, 2), {"next_norm": (res, None, 1e-5)}), ((x, w, 0, 2), {"next_norm": (res, nw.float(), 1e-5)})]:
+        with pytest.raises(hip.KernelError):
+            hip.gemm_slices(*args, **kwargs)
+
+
+@pytest.mark.gpu
+def test_a_recorded_product_in_slices_is_replayed():
+    x, w = operands(140, 1024, 2048)
+    want = hip.gemm_slices(operands(140, 1024, 2048, seed=1)[0], w, 0, 4)
+    hip.gemm_slices(x, w, 0, 4)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        got = hip.gemm_slices(x, w, 0, 4)
+    x.copy_(operands(140, 1024, 2048, seed=1)[0])
+    for _ in range(3):
+        got.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(got, want)
+
+
+def test_the_rule_keeps_to_what_was_measured():
+    for ending in ("bf16", "f32", "norm"):
+        for rows, n, k in ((128, 2048, 8192), (2049, 2048, 8192), (256, 8192, 8192), (256, 512, 8192), (256, 2048, 1024), (256, 2048, 8160), (256, 2044, 8192)):
+            assert hip.slices_plan(rows, n, k, ending) is None
+        for rows in range(129, 2049, 37):
+            for n in (1024, 2048, 3072, 4096):
+                for k in (2048, 4096, 8192, 14336):
+                    plan = hip.slices_plan(rows, n, k, ending)
+                    if plan is not None:
+                        bm, bn = hip.SLICES_TILES[plan[0]][:2]
+                        assert k // 64 // plan[1] >= hip.SLICES_MIN_STEPS and -(-rows // bm) * -(-n // bn) * plan[1] <= hip.COMPUTE_UNITS

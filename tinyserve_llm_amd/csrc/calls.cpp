@@ -193,6 +193,26 @@ PyObject* gemm_library(Args a) {      // x, weight, 32-bit out -> y
   return wrap(y);
 }
 
+PyObject* gemm_slices(Args a) {      // x, weight, tile, slices, 32-bit out, residual, norm weight, eps -> y, or with a norm weight (norm, sum)
+  const Tensor *x = a.tensor(), *w = a.tensor();
+  const int tile = a.i32(), slices = a.i32();
+  const bool wide = a.i32();
+  const Tensor *res = a.maybe(), *nw = a.maybe();
+  const float eps = a.number();
+  if (!a.done() || x->dim() != 2 || w->dim() != 2 || !bf16(*x) || !bf16(*w) || x->size(1) != w->size(1) || !pieces(*x) || !pieces(*w)) return none();
+  const int64_t M = x->size(0), K = x->size(1), N = w->size(0);
+  if (!M || !N || !fits(M) || !fits(N) || !fits(K) || x->stride(0) < K || w->stride(0) < K || slices < 1 || slices > 64 || (res && !nw)) return none();
+  if (nw && (wide || !vector(*nw, at::kBFloat16, N) || !aligned(*nw))) return none();
+  if (res && !(bf16(*res) && matrix(*res, M, N) && res->is_contiguous() && aligned(*res))) return none();
+  if (N % 8 || K % 64) return none();
+  Tensor parts = make(*x, {slices, M, N}, at::kFloat), y = make(*x, {M, N}, wide ? at::kFloat : at::kBFloat16), sum;
+  if (nw) sum = make(*x, {M, N}, at::kBFloat16);
+  if (ts_gemm_slices_bf16(ptr(&y), nw ? ptr(&sum) : nullptr, ptr(&parts), ptr(x), ptr(w), M, N, K, x->stride(0), w->stride(0), tile, slices, wide, ptr(res), ptr(nw),
+                          eps, stream()))
+    return none();
+  return nw ? Py_BuildValue("(NN)", wrap(y), wrap(sum)) : wrap(y);
+}
+
 PyObject* gemm_glu(Args a) {      // x, weight, tile, form's number, limit, slope, up_shift -> y
   const Tensor *x = a.tensor(), *w = a.tensor();
   const int tile = a.i32(), form = a.i32();
@@ -445,6 +465,7 @@ PyMethodDef calls[] = {TS_CALL(rmsnorm),
                        TS_CALL(stream_post_norm),
                        TS_CALL(stream_update_norm),
                        TS_CALL(gemm_library),
+                       TS_CALL(gemm_slices),
                        TS_CALL(gemm_glu),
                        TS_CALL(gemm_rows64),
                        TS_CALL(gemm_rows64_sliced),

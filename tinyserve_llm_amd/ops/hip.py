@@ -90,6 +90,7 @@ def _declare(lib: ctypes.CDLL) -> None:
         "ts_gemm_skinny_bf16": [p, p, p, p, p, p, i, i, i, i64, i64, i64, f, i, i, i, i, p, i, p, p, p, p, p, i, f, f, f, p],
         "ts_gemm_skinny8_bf16": [p, p, p, i, i, i, i64, i64, i64, i, i, p, p, p, p, p, i, p, p, p, i, i, i, i, p],
         "ts_gemm_skinny8_act_bf16": [p, p, p, i, i, i, i64, i64, i64, i, i, p, i, p],
+        "ts_gemm_slices_bf16": [p, p, p, p, p, i, i, i, i64, i64, i, i, i, p, p, f, p],
         "ts_gemm_rows64_bf16": [p, p, p, i, i, i, i64, i64, i, i, p, i, f, f, f, f, p],
         "ts_gemm_rows64_sliced_bf16": [p, p, p, p, i, i, i, i64, i, p, p, p, p, p, i64, p],
         "ts_gemm_rows64_sliced_rope_bf16": [p, p, p, p, i, i, i64, i, p, i, f, p, p, p, p, p, i, i, i, i, i, i64, i64, i64, i64, i64,
@@ -1612,6 +1613,106 @@ def gemm_glu(x: torch.Tensor, weight: torch.Tensor, form: str, limit: float = 0.
     return y
 
 
+# Tiles of `gemm_slices` (rows of x by rows of W); for each, with the plain ending and with the norm's: the µs that do not depend
+# on the sizes, those of a step of 64 of K, of a million numbers of the parts and of a million of W
+SLICES_TILES = ((128, 128, (8.0, 0.42, 1.28, 0.16), (10.8, 0.45, 1.23, 0.15)),
+                (128, 256, (10.8, 0.59, 0.80, 0.18), (13.0, 0.63, 1.00, 0.16)),
+                (192, 256, (12.7, 0.78, 0.75, 0.14), (14.0, 0.80, 1.19, 0.13)),
+                (256, 256, (11.8, 1.09, 0.89, 0.12), (12.5, 1.10, 1.42, 0.10)),
+                (64, 128, (4.2, 0.23, 2.36, 0.34), (7.0, 0.25, 1.84, 0.36)))
+# what the matrix library takes (with the norm: and the norm's kernel): fixed, a thousand of K, that times the root of the rows over 32,
+# and a million products (of a thousand each), numbers of W and of y
+SLICES_LIBRARY = {"bf16": (4.7, 0.33, 1.24, 1.16, 0.55, 0.10), "f32": (3.9, 0.29, 1.46, 1.07, 0.63, 0.57), "norm": (7.7, 0.25, 1.20, 1.15, 0.61, 1.58)}
+SLICES_MIN_ROWS, SLICES_MAX_ROWS = 129, 2048       # fewer rows: the kernels that share x; more: whole reductions fill the chip
+SLICES_MIN_WIDTH, SLICES_MAX_WIDTH = 1024, 4096    # columns (wider: whole reductions fill the chip as well)
+SLICES_MAX, SLICES_MIN_STEPS = 16, 3               # slices, and steps of 64 in each
+SLICES_NORM_MAX_WIDTH = 8192                       # the norm's kernel keeps a row in its workgroup's registers
+
+
+@functools.lru_cache(maxsize=4096)
+def slices_plan(rows: int, n: int, k: int, ending: str) -> tuple[int, int] | None:
+    """The tile of `gemm_slices` and the slices for `rows` rows of x against a weight [n, k], all workgroups in one round; None where
+    the matrix library (and, with the ending "norm", the norm's kernel) is estimated to be within 5 % of it. Both sides are
+    estimates in µs fitted to 143 measured points with weights from memory (129 to 2,048 rows, n 1,024 to 4,096, k 2,048 to
+    14,336; 5 to 8 % root mean square). What it takes is 0.83 to 0.88 of the other way's time on average and at most 1.13 times it.
+    n 2,048, library and here: k 8,192 160 rows 25.8 and 18.8, 512 rows 33.7 and 29.1, 1,024 rows 49.3 and 41.4, with the norm 1,514
+    rows 61.3 and 57.8; k 4,096 300 rows 18.0 and 15.3, 1,024 rows 24.4 and 26.0; k 2,048 160 rows 9.6 and 11.3, with the norm
+    12.8 and 13.4."""
+    if not SLICES_MIN_ROWS <= rows <= SLICES_MAX_ROWS or not SLICES_MIN_WIDTH <= n <= SLICES_MAX_WIDTH or n % 8 or k % 64 or k < 2048:
+        return None
+    steps, best = k // 64, None
+    for tile, (bm, bn, *costs) in enumerate(SLICES_TILES):
+        fixed, step, part, weight = costs[ending == "norm"]
+        tiles = -(-rows // bm) * -(-n // bn)
+        for slices in range(2, min(SLICES_MAX, steps // SLICES_MIN_STEPS, COMPUTE_UNITS // tiles) + 1):
+            us = fixed + step * -(-steps // slices) + (part * slices * rows * n + weight * n * k) * 1e-6
+            if best is None or us < best[0]:
+                best = (us, tile, slices)
+    fixed, chain, rooted, work, weight, out = SLICES_LIBRARY[ending]
+    library = fixed + (chain + rooted * math.sqrt(rows) / 32) * k / 1024 + (work * rows * n * k * 1e-3 + weight * n * k + out * rows * n) * 1e-6
+    return best[1:] if best is not None and best[0] < 0.95 * library else None
+
+
+def slices_takes(x: torch.Tensor, weight: torch.Tensor) -> bool:
+    """Whether `gemm_slices` takes these operands (whatever the rule by sizes says of them)."""
+    return (x.dim() == 2 and weight.dim() == 2 and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16
+            and x.stride(1) == 1 and weight.stride(1) == 1 and x.stride(0) % 8 == 0 and weight.stride(0) % 8 == 0
+            and x.stride(0) >= x.shape[1] and weight.stride(0) >= weight.shape[1]
+            and x.shape[1] % 64 == 0 and weight.shape[0] % 8 == 0 and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0
+            and 512 * x.stride(0) < 1 << 31 and 512 * weight.stride(0) < 1 << 31)
+
+
+def gemm_slices(x: torch.Tensor, weight: torch.Tensor, tile: int, slices: int, out_dtype: torch.dtype = torch.bfloat16,
+                next_norm: "tuple[torch.Tensor | None, torch.Tensor, float] | None" = None) -> "torch.Tensor | tuple[torch.Tensor, torch.Tensor]":
+    """bfloat16 x [M, K] · weight [N, K]^T with the reduction cut into `slices`, whose 32-bit parts a second kernel adds up, the
+    first slice first (gemm_slices.hip); `tile` by its place in `SLICES_TILES`. With `next_norm` = (residual or None, weight,
+    eps): (`rmsnorm` of the product in bfloat16 plus the residual, that sum)."""
+    residual, nw, eps = next_norm if next_norm is not None else (None, None, 0.0)
+    done = _native().gemm_slices(x, weight, tile, slices, out_dtype is torch.float32, residual, nw, eps) if out_dtype in (torch.float32, torch.bfloat16) else None
+    if done is not None:
+        return done
+    _gpu(x, weight, residual, nw)
+    _need(x.dim() == 2 and weight.dim() == 2 and x.shape[1] == weight.shape[1], lambda: f"shapes {tuple(x.shape)} x {tuple(weight.shape)}^T")
+    _need(out_dtype in (torch.bfloat16, torch.float32), lambda: f"bfloat16 products come out as bfloat16 or float32, not {out_dtype}")
+    _need(slices_takes(x, weight), "the product in slices takes bfloat16 operands with dense, 16-byte aligned rows, a reduction that is a "
+          "multiple of 64 and a width that is a multiple of 8")
+    M, K = x.shape
+    N = weight.shape[0]
+    _need(0 <= tile < len(SLICES_TILES) and 1 <= slices <= 64 and K // 64 // slices >= SLICES_MIN_STEPS,
+          lambda: f"tile {tile}, {slices} slices of a reduction of {K}: at least {SLICES_MIN_STEPS} steps of 64 in each")
+    if nw is not None:
+        _need(out_dtype is torch.bfloat16 and N <= SLICES_NORM_MAX_WIDTH and nw.dtype == torch.bfloat16 and nw.shape == (N,) and nw.is_contiguous()
+              and nw.data_ptr() % 16 == 0, lambda: f"the norm that follows has a bfloat16 weight of {N} numbers, at most {SLICES_NORM_MAX_WIDTH}")
+        _need(residual is None or (residual.dtype == torch.bfloat16 and residual.shape == (M, N) and residual.is_contiguous() and residual.data_ptr() % 16 == 0),
+              "the residual has the product's shape and type")
+    else:
+        _need(residual is None, "a residual goes with a norm")
+    y = torch.empty((M, N), dtype=out_dtype, device=x.device)
+    total = torch.empty((M, N), dtype=torch.bfloat16, device=x.device) if nw is not None else None
+    if M and N:
+        parts = torch.empty((slices, M, N), dtype=torch.float32, device=x.device)
+        _run("gemm_slices", library().ts_gemm_slices_bf16(
+            _ptr(y), _ptr(total), _ptr(parts), _ptr(x), _ptr(weight), M, N, K, x.stride(0), weight.stride(0), tile, slices,
+            int(out_dtype is torch.float32), _ptr(residual), _ptr(nw), float(eps), _stream()))
+    return y if nw is None else (y, total)
+
+
+def linear_through_norm(x: torch.Tensor, weight: torch.Tensor, packed: "StreamingCopies | None", residual: torch.Tensor | None,
+                        norm_weight: torch.Tensor, eps: float) -> "tuple[torch.Tensor, torch.Tensor] | None":
+    """(`rmsnorm` of x · weight^T plus the residual, that sum) of many rows by the product in slices, where `linear_bf16` would
+    give the product to the matrix library and the slices are the faster way; None where not."""
+    if _many_rows != "library" or x.dim() != 2 or x.dtype != torch.bfloat16 or norm_weight.dtype != torch.bfloat16:
+        return None
+    rows, k = x.shape
+    n = weight.shape[0]
+    plan = slices_plan(rows, n, k, "norm")
+    if (plan is None or not _library_serves(rows, n, k, packed is not None and packed.by16 is not None, False) or not slices_takes(x, weight)
+            or norm_weight.data_ptr() % 16 or not norm_weight.is_contiguous()
+            or residual is not None and (residual.data_ptr() % 16 or not residual.is_contiguous() or residual.dtype != torch.bfloat16)):
+        return None
+    return gemm_slices(x, weight, *plan, next_norm=(residual, norm_weight, eps))
+
+
 class StreamingCopies:
     """A weight once more in the orders the weight-streaming kernels read it: `by16` for the form
     with 16-row tiles (`pack_weight`), `by8` for the 8-row form (`pack_weight8`); either may be None."""
@@ -1718,7 +1819,9 @@ def linear_bf16(x: torch.Tensor, weight: torch.Tensor, out_dtype: torch.dtype = 
         rows, k = x.shape
         if (_library_serves(rows, weight.shape[0], k, packed is not None and packed.by16 is not None, out_dtype is torch.float32)
                 and x.stride(0) % 8 == 0 and weight.stride(0) % 8 == 0):
-            y = _native().gemm_library(x, weight, out_dtype is torch.float32)
+            wide = out_dtype is torch.float32
+            plan = slices_plan(rows, weight.shape[0], k, "f32" if wide else "bf16")
+            y = _native().gemm_library(x, weight, wide) if plan is None else _native().gemm_slices(x, weight, *plan, wide, None, None, 0.0)
             if y is not None:
                 return y
     _gpu(x, weight)
@@ -1747,6 +1850,9 @@ def linear_bf16(x: torch.Tensor, weight: torch.Tensor, out_dtype: torch.dtype = 
         # rows that are no whole 16-byte pieces: the library has no algorithm for every such shape; the
         # exact kernel takes any (32-bit multiply-adds, slower, for sizes no real model has)
         return gemm_exact(x, weight, out_dtype)
+    plan = slices_plan(x.shape[0], weight.shape[0], x.shape[1], "f32" if out_dtype == torch.float32 else "bf16") if _many_rows == "library" else None
+    if plan is not None and slices_takes(x, weight):
+        return gemm_slices(x, weight, *plan, out_dtype)
     return gemm_library(x, weight, out_dtype)
 
 

@@ -76,6 +76,8 @@ class Attention(Mixer):
                                                  self.num_kv_heads, self.head_dim, eps=d.eps, squares=d.prepared.squares)
             return hip.qkv_rope_store(rows, self.qkv, table, positions, slots, k_store, v_store, self.num_heads,
                                       self.num_kv_heads, self.head_dim, eps=d.eps, packed=by16, squares=d.prepared.squares)[0]
+        if d is not None and d.done is not None:         # (made beside a product of many rows: more than are fused here)
+            return None
         rows = d.x if d is not None else x
         if not (rows.is_cuda and hip.qkv_rope_fuses(rows, self.qkv, self.head_dim, k_store, table=table)):
             slices = 0 if by16 is None or not rows.is_cuda else hip.qkv_rope_sliced_slices(rows, self.qkv, self.head_dim, k_store, table)

@@ -28,18 +28,21 @@ class DeferredNorm:
     """norm(x + residual) * weight, not yet computed: the first projection that takes it either
     fuses it or materialises it. Either way `residual_out` then holds x + residual. With `prepared`
     (what the projection that made x has left: `hip.PreparedNorm`) the sum is there already and
-    `x`, `residual` are not given."""
+    `x`, `residual` are not given; with `done` (the norm and the sum, by the projection of many rows that made x) nothing is left to do."""
 
     def __init__(self, x: torch.Tensor | None, residual: torch.Tensor | None, weight: torch.Tensor, eps: float,
-                 prepared: hip.PreparedNorm | None = None) -> None:
+                 prepared: hip.PreparedNorm | None = None, done: tuple[torch.Tensor, torch.Tensor] | None = None) -> None:
         self.x, self.residual, self.weight, self.eps, self.prepared = x, residual, weight, eps, prepared
-        self.residual_out: torch.Tensor | None = None if prepared is None else prepared.summed
+        self.done = None if done is None else done[0]
+        self.residual_out: torch.Tensor | None = prepared.summed if prepared is not None else None if done is None else done[1]
 
     @property
     def rows(self) -> int:
-        return (self.x if self.prepared is None else self.prepared.operand).shape[0]
+        return (self.done if self.done is not None else self.x if self.prepared is None else self.prepared.operand).shape[0]
 
     def materialize(self) -> torch.Tensor:
+        if self.done is not None:
+            return self.done
         if self.prepared is not None:
             return hip.rmsnorm(self.prepared.summed, self.weight, self.eps, want_residual=False)[0]
         out, self.residual_out = hip.rmsnorm(self.x, self.weight, self.eps, self.residual)
@@ -144,6 +147,10 @@ def linear(x: "torch.Tensor | DeferredNorm | hip.PackedRows8 | hip.SplitAttentio
             prepared = hip.linear_into_norm(x, weight, packed, (residual, then.weight))
             if prepared is not None:
                 return DeferredNorm(None, None, then.weight, then.eps, prepared)
+            if x.is_cuda:
+                done = hip.linear_through_norm(x, weight, packed, residual, then.weight, then.eps)
+                if done is not None:
+                    return DeferredNorm(None, None, then.weight, then.eps, done=done)
         return DeferredNorm(linear(x, weight, out_dtype, packed=packed), residual, then.weight, then.eps)
     by16 = None if packed is None else packed.by16
     rows = x.rows if isinstance(x, DeferredNorm) else x.shape[0]
@@ -163,7 +170,7 @@ def linear(x: "torch.Tensor | DeferredNorm | hip.PackedRows8 | hip.SplitAttentio
         x = d.materialize()
     if isinstance(x, DeferredNorm):
         d = x
-        if (out_dtype in (None, torch.bfloat16) and _streams(d.x, weight) and d.weight.dtype == torch.bfloat16
+        if (d.done is None and out_dtype in (None, torch.bfloat16) and _streams(d.x, weight) and d.weight.dtype == torch.bfloat16
                 and (d.residual is None or d.residual.is_contiguous())
                 and hip.skinny_fuses(d.x.shape[0], weight.shape[1], True, glu) and (not glu or weight.shape[0] % 32 == 0)):
             y, d.residual_out = hip.gemm_skinny(d.x, weight, residual=d.residual, norm_weight=d.weight, eps=d.eps, glu=glu,

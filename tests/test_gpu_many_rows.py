@@ -1,4 +1,4 @@
-"""Products of many rows with the reduction in slices (gemm_slices.hip) against the same product in 64 bits, their endings against
+"""Products of many rows: with the reduction in slices (gemm_slices.hip) against the same product in 64 bits, their endings against
 the kernels they stand in for, and the rule that chooses them."""
 
 from __future__ import annotations
@@ -115,3 +115,17 @@ def test_the_rule_keeps_to_what_was_measured():
                     if plan is not None:
                         bm, bn = hip.SLICES_TILES[plan[0]][:2]
                         assert k // 64 // plan[1] >= hip.SLICES_MIN_STEPS and -(-rows // bm) * -(-n // bn) * plan[1] <= hip.COMPUTE_UNITS
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tile", range(len(hip.GLU_TILES)))
+@pytest.mark.parametrize("over", [-1, 0, 1])
+def test_the_gated_product_is_the_same_in_every_tile(tile, over, monkeypatch):
+    """A row more and less than one and two tiles, columns that hang over: each sum adds up in the order of K in every tile."""
+    rows, f, k = 2 * hip.GLU_TILES[tile][0] + over, 136, 192
+    x, w = operands(rows, 2 * f, k)
+    want = [hip.gemm_glu(x, w, form, 5.0, 1.5, 0.5) for form in ("silu_rounded", "sigmoid")]
+    one = hip.gemm_glu(x[:hip.GLU_TILES[tile][0] + over], w, "relu")
+    monkeypatch.setattr(hip, "glu_plan", lambda rows, n: (tile, 0))
+    assert all(torch.equal(hip.gemm_glu(x, w, form, 5.0, 1.5, 0.5), y) for form, y in zip(("silu_rounded", "sigmoid"), want))
+    assert torch.equal(hip.gemm_glu(x[:hip.GLU_TILES[tile][0] + over], w, "relu"), one)

@@ -8,6 +8,11 @@
 // product) and 171 (32-bit product: 125 with relu, 135 with the sigmoid), 999 rows 59 against 65 and 77, 512 rows 35 against 42,
 // 160 rows 23 against 31.
 //
+// The tile is the one whose rounds of one workgroup a compute unit cost least (hip.glu_plan): a round of 256 x 256 is the chip's best
+// rate, and other heights fill the last round where that one would not. F 8,192, weights from memory, in tiles of 256, 192 and
+// 128 x 256: K 2,048, 700 rows 48.5, 43.7 and 57.5 µs, 1,514 rows 96.0, 81.7 and 87.7, 2,048 rows 104.8, 117.3 and 118.9; K 3,072,
+// 1,514 rows 138, 117 and 135.
+//
 // A workgroup of 8 waves computes BM rows by BN rows of W (BN / 2 columns of the unit), 64 of K at a time. Slices of x
 // and W go from memory straight into LDS, a kilobyte (8 rows of 128 bytes) an instruction; a row's eight 16-byte pieces
 // are turned by (row / 2) % 8, which frees the operand reads of bank conflicts: a 16-byte read of a wave is served in four
@@ -214,18 +219,20 @@ static int launch_glu(GluArgs a, int act, hipStream_t stream) {
 }
 
 // x [M, K], w [2 F, K], y [M, F] bfloat16, 16-byte aligned, rows ldx, ldw, ldy elements apart (multiples of 8); K a
-// multiple of 64, F of 8. tile: rows of x by rows of W of a workgroup, 0 256 x 256, 1 128 x 256, 2 128 x 128. act: 0 silu(gate) up with both branches rounded to bfloat16 first (limit, slope and up_shift
+// multiple of 64, F of 8. tile: rows of x by rows of W of a workgroup, 0 256 x 256, 1 192 x 256, 2 128 x 128,
+// 3 128 x 256. act: 0 silu(gate) up with both branches rounded to bfloat16 first (limit, slope and up_shift
 // unused); 1, 2, 3: the capped unit from the 32-bit sums with the gate through a sigmoid of slope, relu or gelu's tanh form.
 extern "C" int ts_gemm_glu_bf16(void* y, const void* x, const void* w, int M, int F, int K, int64_t ldx, int64_t ldw, int64_t ldy,
                                 int tile, int act, float limit, float slope, float up_shift, hipStream_t stream) {
   if (M <= 0 || F <= 0) return TS_OK;
-  if (K <= 0 || K % 64 || F % 8 || ldx < K || ldw < K || ldy < F || ldx % 8 || ldw % 8 || ldy % 8 || act < 0 || act > 3 || tile < 0 || tile > 2) return TS_BAD_SHAPE;
+  if (K <= 0 || K % 64 || F % 8 || ldx < K || ldw < K || ldy < F || ldx % 8 || ldw % 8 || ldy % 8 || act < 0 || act > 3 || tile < 0 || tile > 3) return TS_BAD_SHAPE;
   if (((uintptr_t)x | (uintptr_t)w | (uintptr_t)y) & 15) return TS_BAD_SHAPE;
   if (!x || !w || !y || 2 * (int64_t)F * ldw * 2 >= (1ll << 31) || 256 * ldx * 2 >= (1ll << 31)) return TS_TOO_LARGE;   // (byte offsets from a tile's start)
   const GluArgs a = {(bf16_t*)y, (const bf16_t*)x, (const bf16_t*)w, M, F, K, 0, 0, 0, ldx, ldw, ldy, limit, slope, up_shift};
   switch (tile) {
     case 0: return launch_glu<256, 256, 2, 4>(a, act, stream);
-    case 1: return launch_glu<128, 256, 2, 4>(a, act, stream);
-    default: return launch_glu<128, 128, 2, 4>(a, act, stream);
+    case 1: return launch_glu<192, 256, 2, 4>(a, act, stream);
+    case 2: return launch_glu<128, 128, 2, 4>(a, act, stream);
+    default: return launch_glu<128, 256, 2, 4>(a, act, stream);
   }
 }

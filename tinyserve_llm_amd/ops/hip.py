@@ -1562,16 +1562,17 @@ def glu_takes(x: torch.Tensor, weight: torch.Tensor) -> bool:
             and 2 * n * weight.stride(0) < 1 << 31 and 512 * x.stride(0) < 1 << 31)
 
 
-# Tiles of `gemm_glu` (rows of x by rows of W) and the µs a round of one workgroup a compute unit takes of them over a reduction of 2,048
-GLU_TILES = ((256, 256, 60), (128, 256, 36), (128, 128, 23))
+# Tiles of `gemm_glu` (rows of x by rows of W) and the µs a round of one workgroup a compute unit counts for over a reduction of 2,048: what
+# the slowest measured (the fastest: 46, 38, 18 and 28), 192 x 256 a tenth more, so that it is not taken for a gain within what rounds differ by
+GLU_TILES = ((256, 256, 60), (192, 256, 54), (128, 128, 23), (128, 256, 36))
 COMPUTE_UNITS = 256
 
 
 @functools.lru_cache(maxsize=4096)
 def glu_plan(rows: int, n: int) -> tuple[int, int]:
     """The tile of `gemm_glu` (its place in `GLU_TILES`) with the cheapest rounds for `rows` rows of x against a weight of
-    `n` rows, and the µs they take over a reduction of 2,048 (1,514 rows, n 16,384: 124, 108 and 128 by tile; 999: 60, 68, 84;
-    256: 48, 34, 25)."""
+    `n` rows, and the µs they take over a reduction of 2,048. Measured, n 16,384, by tile: 1,514 rows 96, 82, 119 and 88; 1,000 rows 55,
+    76, 81 and 62; 700 rows 49, 44, 59 and 58; 256 rows 47, 38, 26 and 33."""
     costs = [us * -(-(-(-rows // bm) * -(-n // bn)) // COMPUTE_UNITS) for bm, bn, us in GLU_TILES]
     return costs.index(min(costs)), min(costs)
 

@@ -129,3 +129,30 @@ def test_the_gated_product_is_the_same_in_every_tile(tile, over, monkeypatch):
     monkeypatch.setattr(hip, "glu_plan", lambda rows, n: (tile, 0))
     assert all(torch.equal(hip.gemm_glu(x, w, form, 5.0, 1.5, 0.5), y) for form, y in zip(("silu_rounded", "sigmoid"), want))
     assert torch.equal(hip.gemm_glu(x[:hip.GLU_TILES[tile][0] + over], w, "relu"), one)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("heads, dim", [(2, 64), (8, 128), (3, 80)])
+@pytest.mark.parametrize("portions", [
+    [(40, 0)], [(13, None), (50, 0)], [(5, None), (3, 13), (20, 21), (9, 7)], [(17, 5), (1, -1), (30, 8)], [(7, 1), (8, 8), (8, 15), (16, 16)], [(9, -1), (23, 6)]])
+def test_values_reach_their_slots_wherever_a_run_of_eight_begins(heads, dim, portions):
+    """Steps of portions (tokens, their first slot on a page of its own; None: single tokens on pages of their own; -1: no slots):
+    aligned, behind decoding requests, ends of portions, over a page's edge. Every slot holds its token, all others stay."""
+    page, slots, next_page = 16, [], 0
+    for n, first in portions:
+        if first is None:
+            slots += [(next_page + i) * page + (5 * i) % page for i in range(n)]
+            next_page += n
+        else:
+            slots += [-1 if first < 0 else next_page * page + first + i for i in range(n)]
+            next_page += 0 if first < 0 else -(-(first + n) // page)
+    g = torch.Generator().manual_seed(len(slots))
+    qkv = torch.randn(len(slots), 3 * heads * dim, generator=g).to(BF).cuda()
+    k, v = torch.zeros(next_page, page, heads, dim, dtype=BF, device="cuda"), torch.full((next_page, heads, dim, page), 7.0, dtype=BF, device="cuda")
+    where = torch.tensor(slots, dtype=torch.int32, device="cuda")
+    hip.rope_store(qkv, None, torch.zeros_like(where), where, k, v.permute(0, 3, 1, 2), heads, heads, dim)
+    want = torch.full((next_page * page, heads, dim), 7.0, dtype=BF)
+    for t, s in enumerate(slots):
+        if s >= 0:
+            want[s] = qkv[t, 2 * heads * dim:].view(heads, dim).cpu()
+    assert torch.equal(v.permute(0, 3, 1, 2).reshape(-1, heads, dim).cpu(), want)

@@ -156,3 +156,68 @@ def test_values_reach_their_slots_wherever_a_run_of_eight_begins(heads, dim, por
         if s >= 0:
             want[s] = qkv[t, 2 * heads * dim:].view(heads, dim).cpu()
     assert torch.equal(v.permute(0, 3, 1, 2).reshape(-1, heads, dim).cpu(), want)
+
+
+def attended(q, k, v, starts, lens, scale, window, softcap):
+    """float64, one request after the other; k, v [requests][keys, kv heads, dim]."""
+    out, at = [], 0
+    for i, n in enumerate(lens):
+        group = q.shape[1] // k[i].shape[1]
+        x, kk, vv = q[at:at + n].double(), k[i].double().repeat_interleave(group, 1), v[i].double().repeat_interleave(group, 1)
+        score = torch.einsum("thd,shd->hts", x.cpu(), kk.cpu()).cuda() * scale
+        if softcap:
+            score = softcap * torch.tanh(score / softcap)
+        gap = (torch.arange(n, device="cuda") + starts[i])[:, None] - torch.arange(k[i].shape[0], device="cuda")[None]
+        score = score.masked_fill((gap < 0) | ((gap >= window) if window else False), float("-inf"))
+        p = torch.softmax(score, -1)
+        out.append(torch.stack([p[h] @ vv[:, h] for h in range(q.shape[1])], 1))
+        at += n
+    return torch.cat(out)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("heads, kv, dim, waves, tiles", [(8, 2, 64, 4, 1), (8, 2, 64, 8, 1), (4, 4, 64, 4, 4), (6, 2, 128, 4, 1), (6, 2, 128, 8, 1), (4, 1, 96, 4, 2),
+                                                          (2, 2, 32, 4, 1), (4, 2, 64, 8, 2)])
+@pytest.mark.parametrize("page, lens, starts, window, softcap", [(32, (300, 5, 77), (0, 40, 31), 0, 0.0), (64, (33, 257), (600, 1), 100, 0.0),
+                                                                 (256, (31, 190), (8500, 0), 0, 20.0), (32, (1, 64), (0, 9000), 8400, 0.0)])
+def test_prompts_attend_to_their_keys(heads, kv, dim, waves, tiles, page, lens, starts, window, softcap):
+    """Tiles in several rounds and a partial one, walks of fewer steps than LDS holds and of more than the ring of places, steps that
+    begin inside a window; slots past a request's last hold numbers that must not count (and no number at all in a page's keys)."""
+    g = torch.Generator().manual_seed(dim + sum(lens))
+    pages = [-(-(s + n) // page) for s, n in zip(starts, lens)]
+    total = sum(lens)
+    q = torch.randn(total, heads, dim, generator=g).to(BF).cuda()
+    k_pool = torch.full((sum(pages), page, kv, dim), float("nan"), dtype=BF, device="cuda")
+    v_pool = torch.full((sum(pages), kv, dim, page), 1e4, dtype=BF, device="cuda")
+    tables = torch.zeros(len(lens), max(pages), dtype=torch.int32)
+    order, at, ks, vs = torch.randperm(sum(pages), generator=g), 0, [], []
+    for i, (s, n) in enumerate(zip(starts, lens)):
+        mine = order[at:at + pages[i]]
+        at += pages[i]
+        tables[i, :pages[i]] = mine.int()
+        ks.append(torch.randn(s + n, kv, dim, generator=g).to(BF).cuda())
+        vs.append(torch.randn(s + n, kv, dim, generator=g).to(BF).cuda())
+        for t0 in range(0, s + n, page):
+            cut = ks[i][t0:t0 + page]
+            k_pool[mine[t0 // page], :cut.shape[0]] = cut
+            v_pool[mine[t0 // page], :, :, :cut.shape[0]] = vs[i][t0:t0 + page].permute(1, 2, 0)
+    cu = [0]
+    for n in lens:
+        cu.append(cu[-1] + n)
+    tokens = waves * tiles * (16 // (heads // kv))
+    where = torch.tensor(hip.attention_tiles(cu, list(starts), tokens), dtype=torch.int32).view(-1, 2).cuda()
+    seq = torch.cat([torch.full((n,), i) for i, n in enumerate(lens)]).int().cuda()
+    pos = torch.cat([torch.arange(s, s + n) for s, n in zip(starts, lens)]).int().cuda()
+    got = hip.paged_attention_prefill(q, k_pool, v_pool.permute(0, 3, 1, 2), tables.cuda(), seq, pos, where, dim ** -0.5, window, tile_tokens=tokens, waves=waves, softcap=softcap)
+    want = attended(q, ks, vs, starts, lens, dim ** -0.5, window, softcap)
+    # weights and output in bfloat16: 2^-8 of the values' size a weight (they add up to 1), 2^-8 of the output
+    bound = (2.0 ** -7) * max(float(v.abs().max()) for v in vs)
+    assert bool(((got.double() - want).abs() <= bound).all()), float((got.double() - want).abs().max())
+    assert float((got.double() - want).norm() / want.norm()) < 0.01
+
+
+def test_heads_of_128_take_eight_waves_where_these_fill_the_chip_and_the_general_variant_keeps_single_tiles():
+    shape = hip.prefill_shape
+    assert shape(1501, 20, 4, 8, 3, 128, 500.0, False) == (40, 8) and shape(1024, 20, 4, 8, 3, 128, 512.0, False) == (20, 4)
+    assert shape(1501, 20, 4, 8, 3, 128, 2000.0, False) == (20, 4) and shape(1501, 20, 4, 8, 3, 128, 500.0, True) == (20, 4)
+    assert shape(2048, 32, 8, 8, 4, 64, 1024.0, True) == (16, 4) and shape(2048, 32, 8, 8, 4, 64, 1024.0, False) == (32, 8)

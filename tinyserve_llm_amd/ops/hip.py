@@ -783,12 +783,30 @@ def paged_attention_prefill(q: torch.Tensor, k_cache: torch.Tensor, v_cache: tor
     return out
 
 
-def _prefill_plan(q: torch.Tensor, k_cache: torch.Tensor, ctx, decode_ok: bool) -> tuple:
+PREFILL_EIGHT_WAVES_WIDE_WORKGROUPS = 288      # heads of 128 take eight waves from this many workgroups of theirs on
+
+
+def prefill_shape(tokens: int, tile_tokens: int, waves: int, nkv: int, group: int, head_dim: int, mean_keys: float, general: bool) -> tuple[int, int]:
+    """(tokens per tile, waves) of the prefill kernel from what `prefill_tile_tokens` and `prefill_waves` make of the step. Heads
+    of 64 in the general variant keep tiles of one row tile a wave where eight waves would take two (their softmax, twice as
+    long, is what bounds them: 2,048 tokens 48.8 µs against 56.3, 819 and 1,229 together 31.2 against 36.8); heads of 128 take eight waves over
+    a short walk as soon as these fill the chip (1,501 tokens in two requests 24.6 µs against 27.0, 1,500 in one 34.9 against 38.1,
+    but 1,024 26.2 against 23.7)."""
+    one = PREFILL_WAVES * (16 // group)
+    if general and head_dim == 64 and waves == 2 * PREFILL_WAVES:
+        return one, PREFILL_WAVES
+    if (head_dim == 128 and not general and tile_tokens == one and waves == PREFILL_WAVES and 0.0 < mean_keys < PREFILL_EIGHT_WAVES_MEAN_KEYS
+            and -(-tokens // (2 * one)) * nkv >= PREFILL_EIGHT_WAVES_WIDE_WORKGROUPS):
+        return 2 * one, 2 * PREFILL_WAVES
+    return tile_tokens, waves
+
+
+def _prefill_plan(q: torch.Tensor, k_cache: torch.Tensor, ctx, decode_ok: bool, general: bool = False) -> tuple:
     """How a step's rows are dealt to the matrix-core kernels, from its lengths and the heads' sizes: (leading one-token
     requests, which go to the split-key kernel; tokens per tile; waves; tiles; chunks; keys per chunk). Every layer of one kind
     asks for the same plan, so a step makes it once."""
     (rows, nh, hd), nkv = q.shape, k_cache.shape[2]
-    key = ("attention_plan", rows, nh, nkv, hd, decode_ok)
+    key = ("attention_plan", rows, nh, nkv, hd, decode_ok, general)
     plan = ctx.scratch.get(key)
     if plan is not None:
         return plan
@@ -800,6 +818,7 @@ def _prefill_plan(q: torch.Tensor, k_cache: torch.Tensor, ctx, decode_ok: bool) 
     mean_keys = walked / max(1, rows - lead)
     tile_tokens = prefill_tile_tokens(rows - lead, nkv, nh // nkv, hd, mean_keys)
     waves = prefill_waves(tile_tokens, nh // nkv, hd, mean_keys)
+    tile_tokens, waves = prefill_shape(rows - lead, tile_tokens, waves, nkv, nh // nkv, hd, mean_keys, general)
     tiles = ctx.scratch.get(("attention_tiles", tile_tokens, lead))
     if tiles is None:
         flat = attention_tiles(cu, starts, tile_tokens, lead)
@@ -831,7 +850,8 @@ def paged_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
     if chunk_mask:
         window = -chunk_mask
     tables = ctx.block_tables[space]
-    key = ("attention_step", q.shape, k_cache.shape, tables.shape)
+    general = softcap > 0 or sink or sinks is not None or slopes is not None or gate is not None
+    key = ("attention_step", q.shape, k_cache.shape, tables.shape, general)
     step = ctx.scratch.get(key)
 
     def planned(step) -> torch.Tensor | None:
@@ -841,7 +861,6 @@ def paged_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
         out = planned(step)
         if out is not None:
             return out
-    general = softcap > 0 or sink or sinks is not None or slopes is not None or gate is not None
     extra = dict(softcap=softcap, sink=sink, sinks=sinks, slopes=slopes)
     # (the tables count in pages of ctx.page_size tokens; the pools may be cut into shorter ones)
     table_page = getattr(ctx, "page_size", 0) or k_cache.shape[1]
@@ -854,7 +873,7 @@ def paged_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
         if ctx.max_query_len == 1 and decode_ok:
             return paged_attention_decode(q, k_cache, v_cache, tables, ctx.seq_of_token, ctx.positions, scale, window,
                                           pages_per_entry=per_entry, leave_split=leave_split and gate is None, gate=gate, **extra)
-        lead, tile_tokens, waves, tiles, splits, chunk = _prefill_plan(q, k_cache, ctx, decode_ok)
+        lead, tile_tokens, waves, tiles, splits, chunk = _prefill_plan(q, k_cache, ctx, decode_ok, general)
         nkv = k_cache.shape[2]
         split_walk = decode_plan(lead, nkv, q.shape[1] // nkv, q.shape[2], capacity) if lead else (0, 0)
         ctx.scratch[key] = (tiles, (per_entry, lead, *split_walk, tile_tokens, waves, splits, chunk, ctx.host_cu_seqlens[lead]))

@@ -221,3 +221,48 @@ def test_heads_of_128_take_eight_waves_where_these_fill_the_chip_and_the_general
     assert shape(1501, 20, 4, 8, 3, 128, 500.0, False) == (40, 8) and shape(1024, 20, 4, 8, 3, 128, 512.0, False) == (20, 4)
     assert shape(1501, 20, 4, 8, 3, 128, 2000.0, False) == (20, 4) and shape(1501, 20, 4, 8, 3, 128, 500.0, True) == (20, 4)
     assert shape(2048, 32, 8, 8, 4, 64, 1024.0, True) == (16, 4) and shape(2048, 32, 8, 8, 4, 64, 1024.0, False) == (32, 8)
+
+
+def test_chunks_are_walked_where_their_states_are_many():
+    def z(heads, vp, np):
+        return type("Z", (), dict(np=np, matrix=heads * vp * np))
+    assert hip.ssd_walks(32, 32, z(64, 64, 128)) and hip.ssd_walks(5, 5, z(64, 64, 128)) and hip.ssd_walks(17, 7, z(16, 128, 128))
+    assert hip.ssd_walks(80, 5, z(4, 64, 128)) and hip.ssd_walks(1, 1, z(4, 64, 32))
+    assert not hip.ssd_walks(32, 32, z(4, 64, 128)) and not hip.ssd_walks(32, 32, z(16, 128, 128)) and not hip.ssd_walks(32, 32, z(64, 64, 160))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("heads, vdim, groups, places", [(2, 16, 1, 32), (3, 37, 3, 64), (4, 64, 2, 96), (8, 80, 4, 128), (1, 130, 1, 100)])
+@pytest.mark.parametrize("lengths", [[64], [1, 65, 130], [200, 37, 300], [128, 448]])
+@pytest.mark.parametrize("one_decay", [False, True])
+def test_a_walk_over_the_chunks_leaves_what_the_chunks_do(heads, vdim, groups, places, lengths, one_decay, monkeypatch):
+    """The same states, bit for bit (the sums are the same), and outputs a rounding apart: two 32-bit sums of at most 64 and `places`
+    terms that are added once more, so 2^-22 of what goes into them; channels that are no fours, places of none, a chunk's rest."""
+    g = torch.Generator().manual_seed(sum(lengths) + heads)
+    z = hip.SsdSizes(heads, vdim, groups, places, 4)
+    total, slots = sum(lengths), list(range(len(lengths)))[::-1]
+    mixed = torch.zeros(total, z.row)
+    x, bc = mixed[:, :heads * z.vp].view(total, heads, z.vp), mixed[:, heads * z.vp:].view(total, 2 * groups, z.np)
+    x[:, :, :vdim] = torch.randn(total, heads, vdim, generator=g)
+    bc[:, :, :places] = torch.randn(total, 2 * groups, places, generator=g)
+    shape = (heads,) if one_decay else (total, heads)
+    steps, logs = (torch.rand(shape, generator=g) + 0.1).cuda(), -(torch.rand(shape, generator=g) ** 4 * 30).cuda()
+    skip, start = torch.randn(heads, generator=g).cuda(), torch.randn(len(lengths), z.matrix + z.kept, generator=g).cuda()
+    start[:, :z.matrix].view(-1, heads, z.vp, z.np)[:, :, vdim:] = 0.0
+    mixed = mixed.to(BF).cuda()
+    cu = [0]
+    for n in lengths:
+        cu.append(cu[-1] + n)
+    found = []
+    for walks in (True, False):
+        ctx = type("Ctx", (), dict(num_seqs=len(lengths), num_tokens=total, max_query_len=max(lengths), host_cu_seqlens=cu, scratch={},
+                                   cu_seqlens=torch.tensor(cu, dtype=torch.int32).cuda(), state_slots=torch.tensor(slots, dtype=torch.int32).cuda(),
+                                   seq_of_token=torch.cat([torch.full((n,), i) for i, n in enumerate(lengths)]).int().cuda()))
+        monkeypatch.setattr(hip, "ssd_walks", lambda *a, w=walks: w)
+        state = start.clone()
+        y = hip.ssd_scan(mixed, steps, logs, skip, state, ctx, z, chunks_from=1, keeps=torch.exp(logs) if one_decay else None)
+        found.append((y, state))
+    (y, state), (want, want_state) = found
+    assert torch.equal(state, want_state)
+    size = float(want.abs().max()) + float(start.abs().max()) * places ** 0.5 + 64.0
+    assert float((y - want).abs().max()) <= 2.0 ** -22 * 8 * size

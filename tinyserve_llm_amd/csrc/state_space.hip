@@ -25,6 +25,7 @@
 #define SS_THREADS 256
 #define SS_WAVES (SS_THREADS / TS_WAVE)
 #define SS_MAX_TAPS 16
+#define SS_TABLE (2 * SS_L + 4)     // floats of a chunk and head: every token's decay since the chunk's start, the weights of what it adds, the whole decay
 
 struct SsSizes { int heads, vdim, vp, groups, state, np, taps; };
 
@@ -407,9 +408,11 @@ ssd_chunk_scan_kernel(float* __restrict__ buf, const float* __restrict__ totals,
 // One workgroup per (chunk, head, slice of 64 channels): first each wave makes the second sum's weights of its 16 tokens
 // (keys as the product's rows, so that the weights come out in the order the next product reads), then each wave the
 // outputs of its 16 channels for all tokens.
-template <int NQ>
+// STATE: with the state before the chunk, out of buf. Without: the second sum alone, and what the walk needs of the decays goes
+// into `tables` (SS_TABLE floats a chunk and head).
+template <int NQ, bool STATE>
 __global__ void __launch_bounds__(SS_THREADS)
-ssd_chunk_out_kernel(float* __restrict__ out, const float* __restrict__ buf, const bf16_t* __restrict__ mixed,
+ssd_chunk_out_kernel(float* __restrict__ out, const float* __restrict__ buf, float* __restrict__ tables, const bf16_t* __restrict__ mixed,
                      const float* __restrict__ steps, const float* __restrict__ logs, const float* __restrict__ skip, int token_stride,
                      const int32_t* __restrict__ chunks, int heads, int vdim, int vp, int groups) {
   constexpr int np = 32 * NQ;
@@ -425,8 +428,19 @@ ssd_chunk_out_kernel(float* __restrict__ out, const float* __restrict__ buf, con
   const bf16_t* b_rows = rows + heads * vp + g * np + 8 * q;
   const bf16_t* c_rows = b_rows + groups * np;
   if (threadIdx.x < TS_WAVE) {
-    b_s[lane] = ss_running(logs, tok0, len, token_stride, h);
-    d_s[lane] = lane < len ? steps[(int64_t)(tok0 + lane) * token_stride + h] : 0.f;
+    const double b = ss_running(logs, tok0, len, token_stride, h);
+    const float d = lane < len ? steps[(int64_t)(tok0 + lane) * token_stride + h] : 0.f;
+    b_s[lane] = b;
+    d_s[lane] = d;
+    if constexpr (!STATE) {
+      const double total = __shfl(b, TS_WAVE - 1, TS_WAVE);
+      float* table = tables + ((int64_t)chunk * heads + h) * SS_TABLE;
+      if (blockIdx.z == 0) {
+        table[lane] = expf((float)b);
+        table[SS_L + lane] = lane < len ? expf((float)(total - b)) * d : 0.f;
+        if (lane == 0) table[2 * SS_L] = expf((float)total);
+      }
+    }
   }
   ss_turn<false>(x_s, nullptr, mixed + h * vp + v0, row, tok0, len, vp - v0, nullptr);
   const int t = 16 * wave + r;                               // (this lane's token of the first product)
@@ -476,9 +490,9 @@ ssd_chunk_out_kernel(float* __restrict__ out, const float* __restrict__ buf, con
   float4_t acc[4];
 #pragma unroll
   for (int tb = 0; tb < 4; ++tb) acc[tb] = (float4_t){0.f, 0.f, 0.f, 0.f};
-  const float* s_row = buf + ((int64_t)chunk * heads + h) * vp * np + (int64_t)(v0 + 16 * wave + r) * np + 8 * q;
+  const float* s_row = STATE ? buf + ((int64_t)chunk * heads + h) * vp * np + (int64_t)(v0 + 16 * wave + r) * np + 8 * q : nullptr;
 #pragma unroll
-  for (int i = 0; i < NQ; ++i) {
+  for (int i = 0; i < (STATE ? NQ : 0); ++i) {
     float s[8];
     ss_load4(s_row + 32 * i, *(float (*)[4])&s[0]);
     ss_load4(s_row + 32 * i + 4, *(float (*)[4])&s[4]);
@@ -502,9 +516,11 @@ ssd_chunk_out_kernel(float* __restrict__ out, const float* __restrict__ buf, con
 #pragma unroll
   for (int tb = 0; tb < 4; ++tb) {
     const int tok = 16 * tb + r;
-    const float decay = expf((float)b_s[tok]);
+    if constexpr (STATE) {
+      const float decay = expf((float)b_s[tok]);
 #pragma unroll
-    for (int j = 0; j < 4; ++j) acc[tb][j] *= decay;
+      for (int j = 0; j < 4; ++j) acc[tb][j] *= decay;
+    }
 #pragma unroll
     for (int k = 0; k < 2; ++k)
       if (32 * k <= 16 * tb + 15) {
@@ -546,13 +562,255 @@ extern "C" int ts_ssd_chunks(float* out, const void* mixed, const float* steps, 
                                                                                        groups, np);
   ssd_chunk_scan_kernel<<<dim3(num_seqs, heads, scan_blocks), SS_THREADS, 0, stream>>>(buf, totals, states, slot_stride, chunk_cu, state_slots,
                                                                                       heads, (int)per_head);
-#define SS_OUT(NQ) case NQ: ssd_chunk_out_kernel<NQ><<<dim3(num_chunks, heads, slices), SS_THREADS, 0, stream>>>( \
-    out, buf, m, steps, logs, skip, token_stride, chunks, heads, vdim, vp, groups); break;
+#define SS_OUT(NQ) case NQ: ssd_chunk_out_kernel<NQ, true><<<dim3(num_chunks, heads, slices), SS_THREADS, 0, stream>>>( \
+    out, buf, nullptr, m, steps, logs, skip, token_stride, chunks, heads, vdim, vp, groups); break;
   switch (np / 32) {
     SS_OUT(1) SS_OUT(2) SS_OUT(3) SS_OUT(4) SS_OUT(5) SS_OUT(6) SS_OUT(7) SS_OUT(8) SS_OUT(9) SS_OUT(10) SS_OUT(11) SS_OUT(12)
     SS_OUT(13) SS_OUT(14) SS_OUT(15) SS_OUT(16)
   }
 #undef SS_OUT
+  return ts_check_launch();
+}
+
+// ---- the same without the states' trips through memory: a walk over a request's chunks ----
+
+// What bounds the chunks above is the states between them: written, scanned and read they are four times chunks x heads x vp x np
+// numbers of memory (2,048 tokens, 64 heads of 64 x 128: 268 MB). Here a workgroup keeps 16 channels of a head's state over all of a
+// request's chunks, and adds to the second sums that `ssd_chunk_out_kernel` has left in `out`: y += exp(b_t) S C_t, then S = exp(b_L) S + sum_j x_j B_j^T
+// weighted as before. A wave keeps every fourth 32 places of the state in the registers its products leave them in, and
+// puts them into LDS as two bfloat16 terms for all four, each of which reads the state out for 16 of the chunk's tokens. The next
+// chunk's B (turned) and weighted x go into LDS meanwhile by four other waves, those of the chunks after it are on their way: one barrier a chunk.
+// What bounds it then is the walk, 0.9 to 1.3 µs a chunk, most of it the loads' rows (C's 16 rows a load); with one set of waves for both
+// halves 1.5 to 1.8. Measured, chunks and walk, µs: 64 heads of 64 x 128, 304 tokens 33.0 and 22.7, 2,048 92.7 and 73.7, 16 requests
+// of 300 249 and 159; 16 heads of 128 x 128, three requests of 999 tokens 40.4 and 33.1, one of 2,048 55.6 and 57.7; 4 heads, 2,048
+// 26.3 and 43.5 (where the chunks stay). The same states, bit for bit; the outputs 6.5e-8 apart.
+template <int NQ, bool FOURS>
+__global__ void __launch_bounds__(2 * SS_THREADS)
+ssd_walk_kernel(float* __restrict__ out, const float* __restrict__ tables, const bf16_t* __restrict__ mixed, float* __restrict__ states,
+                int64_t slot_stride, const int32_t* __restrict__ chunks, const int32_t* __restrict__ chunk_cu,
+                const int32_t* __restrict__ state_slots, int heads, int vdim, int vp, int groups) {
+  constexpr int np = 32 * NQ, MINE = (NQ + 3) / 4;                           // (32 places of a wave at a time)
+  __shared__ __attribute__((aligned(16))) bf16_t b_s[2][np][SS_PAD];         // B, turned: [state][token]
+  __shared__ __attribute__((aligned(16))) bf16_t x_s[2][2][16][SS_PAD];      // weighted x, turned, two terms: [channel][token]
+  __shared__ uint4 s_s[2][NQ][2][TS_WAVE];                                   // the state, two terms: [32 places][lane]
+  // (consecutive workgroups go to different dies: a die takes a run of heads, which share B and C)
+  const int items = gridDim.x, item = items % 8 ? blockIdx.x : blockIdx.x % 8 * (items / 8) + blockIdx.x / 8;
+  const int slices = vp / 16, h = item / slices, v0 = (item - h * slices) * 16, seq = blockIdx.y;
+  const int begin = chunk_cu[seq], end = chunk_cu[seq + 1];
+  if (begin >= end) return;
+  const int first = chunks[4 * begin], past = chunks[4 * (end - 1)] + chunks[4 * (end - 1) + 1];      // the request's tokens
+  const int row = heads * vp + 2 * groups * np, g = h / (heads / groups);
+  if (wave_index() >= SS_WAVES) {
+    // Four waves bring the chunks' B and x into LDS. Nothing is asked for behind a test, so that every wait is for what it needs
+    // alone: chunks past the last are the last one again and never used, a token past a chunk's end is its last one and counts as 0.
+    // Neighbouring lanes take neighbouring pieces of a row (a load in 32 rows at once takes four times as long as one in 4), and
+    // two neighbouring tokens each; a column's blocks of 8 tokens change places with its piece, or all pieces would meet in few banks.
+    const int thread = threadIdx.x - SS_THREADS;
+    // (of B: a row's pieces of eight places, and a thread's pairs of tokens; where 32 pairs are not whole rounds of threads some
+    // take one again)
+    constexpr int PIECES = 4 * NQ, PAIRS = (NQ + 1) / 2;
+    const int x_piece = thread & 7, x_pair = thread >> 3;
+    const bf16_t* const b_cols = mixed + heads * vp + g * np;
+    auto piece_of = [&](int k) { return (thread + k * SS_THREADS) % PIECES; };
+    auto token_of = [&](int k) { return 2 * ((thread + k * SS_THREADS) / PIECES & 31); };
+    const bf16_t* const x_cols = mixed + h * vp + v0 + 2 * x_piece;
+    struct Rows { uint4 b[PAIRS][2]; uint32_t x[2]; float weight[2]; };
+    auto fetch = [&](int c, Rows& t) {
+      const int at = min(c, end - 1), tok0 = first + (at - begin) * SS_L, len = min(SS_L, past - tok0);
+#pragma unroll
+      for (int k = 0; k < PAIRS; ++k) {
+        const int ta = token_of(k), col = 8 * piece_of(k);
+        t.b[k][0] = *(const uint4*)(b_cols + (int64_t)(tok0 + min(ta, len - 1)) * row + col);
+        t.b[k][1] = *(const uint4*)(b_cols + (int64_t)(tok0 + min(ta + 1, len - 1)) * row + col);
+      }
+      t.x[0] = *(const uint32_t*)(x_cols + (int64_t)(tok0 + min(2 * x_pair, len - 1)) * row);
+      t.x[1] = *(const uint32_t*)(x_cols + (int64_t)(tok0 + min(2 * x_pair + 1, len - 1)) * row);
+      const float* weight = tables + ((int64_t)at * heads + h) * SS_TABLE + SS_L;
+      t.weight[0] = weight[2 * x_pair], t.weight[1] = weight[2 * x_pair + 1];      // (0 past the chunk's end)
+    };
+    auto put = [&](int c, const Rows& t, int to) {
+      const int len = min(SS_L, past - first - (min(c, end - 1) - begin) * SS_L);
+#pragma unroll
+      for (int k = 0; k < PAIRS; ++k) {
+        const int ta = token_of(k), piece = piece_of(k), at = 8 * ((ta >> 3) ^ (piece & 7)) + (ta & 7);
+        const uint32_t keep_a = ta < len ? 0xffffffffu : 0u, keep_b = ta + 1 < len ? 0xffffffffu : 0u;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const uint32_t x = (&t.b[k][0].x)[e >> 1] & keep_a, y = (&t.b[k][1].x)[e >> 1] & keep_b;
+          *(uint32_t*)&b_s[to][8 * piece + e][at] = e & 1 ? (x >> 16) | (y & 0xffff0000u) : (x & 0xffffu) | (y << 16);
+        }
+      }
+      const uint32_t xw = 2 * x_pair < len ? t.x[0] : 0u, yw = 2 * x_pair + 1 < len ? t.x[1] : 0u;
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        const float x = __uint_as_float(e ? xw & 0xffff0000u : xw << 16) * t.weight[0], y = __uint_as_float(e ? yw & 0xffff0000u : yw << 16) * t.weight[1];
+        const uint32_t hi = pack_bf16(x, y);
+        *(uint32_t*)&x_s[to][0][2 * x_piece + e][2 * x_pair] = hi;
+        *(uint32_t*)&x_s[to][1][2 * x_piece + e][2 * x_pair] = ss_rest(hi, x, y);
+      }
+    };
+    Rows rows[2];
+    fetch(begin, rows[0]);
+    __builtin_amdgcn_sched_barrier(0);
+    fetch(begin + 1, rows[1]);
+    __builtin_amdgcn_sched_barrier(0);
+    put(begin, rows[0], 0);
+    fetch(begin + 2, rows[0]);
+    __syncthreads();
+    auto work = [&](int c, Rows& after, int p) {
+      put(c + 1, after, 1 - p);                              // (that half was read before the last barrier)
+      __builtin_amdgcn_sched_barrier(0);
+      fetch(c + 3, after);
+      __syncthreads();
+    };
+    for (int c = begin;; c += 2) {
+      work(c, rows[1], 0);
+      if (c + 1 >= end) break;
+      work(c + 1, rows[0], 1);
+      if (c + 2 >= end) break;
+    }
+    return;
+  }
+  const int wave = wave_index(), lane = threadIdx.x & (TS_WAVE - 1), r = lane & 15, q = lane >> 4;
+  const bf16_t* const c_cols = mixed + heads * vp + (groups + g) * np + 8 * q;
+  const int v = v0 + 4 * q;
+  float* st = states + (int64_t)state_slots[seq] * slot_stride + (int64_t)h * vp * np + (int64_t)(v0 + r) * np + 8 * q;
+  float S[MINE][8];                                          // places 32 i + 8 q .. + 7 of channel v0 + r, i = wave + 4 m
+#pragma unroll
+  for (int m = 0; m < MINE; ++m) {
+    const int i = wave + 4 * m;
+    if (i < NQ) {
+      ss_load4(st + 32 * i, *(float (*)[4])&S[m][0]);
+      ss_load4(st + 32 * i + 4, *(float (*)[4])&S[m][4]);
+    }
+  }
+  auto put_state = [&](int to) {
+#pragma unroll
+    for (int m = 0; m < MINE; ++m) {
+      const int i = wave + 4 * m;
+      if (i < NQ) {
+        uint4 hi, lo;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          (&hi.x)[j] = pack_bf16(S[m][2 * j], S[m][2 * j + 1]);
+          (&lo.x)[j] = ss_rest((&hi.x)[j], S[m][2 * j], S[m][2 * j + 1]);
+        }
+        s_s[to][i][0][lane] = hi;
+        s_s[to][i][1][lane] = lo;
+      }
+    }
+  };
+  // what a lane reads out: a token's C, its decay and the second sum that is there already
+  struct Token { uint4 c[NQ]; float decay, keep, y[4]; };
+  auto token_at = [&](int c) { return min(first + (min(c, end - 1) - begin) * SS_L + 16 * wave + r, past - 1); };
+  auto fetch_c = [&](int c, Token& t) {
+    const bf16_t* src = c_cols + (int64_t)token_at(c) * row;
+#pragma unroll
+    for (int i = 0; i < NQ; ++i) t.c[i] = *(const uint4*)(src + 32 * i);
+  };
+  auto fetch_y = [&](int c, Token& t) {
+    const float* table = tables + ((int64_t)min(c, end - 1) * heads + h) * SS_TABLE;
+    t.decay = table[16 * wave + r], t.keep = table[2 * SS_L];
+    const float* src = out + ((int64_t)token_at(c) * heads + h) * vdim;
+    if constexpr (FOURS) ss_load4(src + min(v, vdim - 4), t.y);
+    else {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) t.y[j] = src[min(v + j, vdim - 1)];
+    }
+  };
+  Token tokens[2];
+  fetch_c(begin, tokens[0]), fetch_y(begin, tokens[0]);
+  __builtin_amdgcn_sched_barrier(0);
+  fetch_c(begin + 1, tokens[1]), fetch_y(begin + 1, tokens[1]);
+  __builtin_amdgcn_sched_barrier(0);
+  put_state(0);
+  __syncthreads();
+  auto work = [&](int c, Token& now, int p) {                // chunk c, whose half of LDS is p
+    // the state's next value first: the other waves wait for it
+    uint4 xf[2][2];
+#pragma unroll
+    for (int k = 0; k < 2; ++k)
+#pragma unroll
+      for (int e = 0; e < 2; ++e) xf[k][e] = *(const uint4*)&x_s[p][e][r][32 * k + 8 * q];
+#pragma unroll
+    for (int m = 0; m < MINE; ++m) {
+      const int i = wave + 4 * m;
+      if (i < NQ) {
+#pragma unroll
+        for (int tau = 0; tau < 2; ++tau) {
+          float4_t add = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int k = 0; k < 2; ++k) {
+            const int n = 32 * i + 8 * (r >> 2) + 4 * tau + (r & 3);
+            const uint4 bf = *(const uint4*)&b_s[p][n][8 * ((4 * k + q) ^ ((n >> 3) & 7))];
+            add = mfma32(bf, xf[k][0], add);
+            add = mfma32(bf, xf[k][1], add);
+          }
+#pragma unroll
+          for (int j = 0; j < 4; ++j) S[m][4 * tau + j] = fmaf(now.keep, S[m][4 * tau + j], add[j]);
+        }
+      }
+    }
+    float4_t acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < NQ; ++i) {
+      acc = mfma32(s_s[p][i][0][lane], now.c[i], acc);
+      acc = mfma32(s_s[p][i][1][lane], now.c[i], acc);
+    }
+    put_state(1 - p);                                        // (that half was read before the last barrier)
+    fetch_c(c + 2, now);
+    const int tok = first + (c - begin) * SS_L + 16 * wave + r;
+    float y[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) y[j] = fmaf(now.decay, acc[j], now.y[j]);
+    if (tok < past) {
+      float* dst = out + ((int64_t)tok * heads + h) * vdim + v;
+      if constexpr (FOURS) {
+        if (v < vdim) ss_store4(dst, y);
+      } else {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          if (v + j < vdim) dst[j] = y[j];
+      }
+    }
+    fetch_y(c + 2, now);                                     // (other tokens than any that have been written)
+    __syncthreads();
+  };
+  for (int c = begin;; c += 2) {
+    work(c, tokens[0], 0);
+    if (c + 1 >= end) break;
+    work(c + 1, tokens[1], 1);
+    if (c + 2 >= end) break;
+  }
+#pragma unroll
+  for (int m = 0; m < MINE; ++m) {
+    const int i = wave + 4 * m;
+    if (i < NQ) {
+      ss_store4(st + 32 * i, *(float (*)[4])&S[m][0]);
+      ss_store4(st + 32 * i + 4, *(float (*)[4])&S[m][4]);
+    }
+  }
+}
+
+// As ts_ssd_chunks, but np at most 128, and a request's chunks are of 64 neighbouring tokens each but the last; tables float32 [chunks, heads, 132] is scratch.
+extern "C" int ts_ssd_walk(float* out, const void* mixed, const float* steps, const float* logs, const float* skip, int token_stride,
+                           float* states, int64_t slot_stride, const int32_t* chunks, const int32_t* chunk_cu, const int32_t* state_slots,
+                           float* tables, int num_chunks, int num_seqs, int heads, int vdim, int vp, int groups, int np, hipStream_t stream) {
+  if (num_chunks <= 0 || num_seqs <= 0) return TS_OK;
+  const int64_t per_head = (int64_t)vp * np;
+  if (heads <= 0 || heads > 65535 || num_seqs > 65535 || groups <= 0 || heads % groups || vdim <= 0 || vp < vdim || vp % 16 || np <= 0 || np % 32 || np > 128 ||
+      per_head > (1 << 24) || (int64_t)heads * (vp / 16) > 0x7fffffff || slot_stride < heads * per_head || slot_stride % 4 ||
+      (((uintptr_t)states | (uintptr_t)mixed | (uintptr_t)out) & 15) || ((uintptr_t)tables & 3) || (token_stride != 0 && token_stride < heads))
+    return TS_BAD_SHAPE;
+  const bf16_t* m = (const bf16_t*)mixed;
+  const dim3 sums(num_chunks, heads, (vp + 63) / 64), walks(heads * (vp / 16), num_seqs);
+#define SS_WALK(NQ) case NQ: \
+    ssd_chunk_out_kernel<NQ, false><<<sums, SS_THREADS, 0, stream>>>(out, nullptr, tables, m, steps, logs, skip, token_stride, chunks, heads, vdim, vp, groups); \
+    if (vdim % 4 == 0) ssd_walk_kernel<NQ, true><<<walks, 2 * SS_THREADS, 0, stream>>>(out, tables, m, states, slot_stride, chunks, chunk_cu, state_slots, heads, vdim, vp, groups); \
+    else ssd_walk_kernel<NQ, false><<<walks, 2 * SS_THREADS, 0, stream>>>(out, tables, m, states, slot_stride, chunks, chunk_cu, state_slots, heads, vdim, vp, groups); \
+    break;
+  switch (np / 32) { SS_WALK(1) SS_WALK(2) SS_WALK(3) SS_WALK(4) }
+#undef SS_WALK
   return ts_check_launch();
 }
 

@@ -132,6 +132,7 @@ def _declare(lib: ctypes.CDLL) -> None:
         "ts_ssd_prepare": [p, i, p, p, p, i64, p, p, p, i64, p, p, p, p, p, i, i, i, i, i, i, i, i, i, p],
         "ts_ssd_conv_keep": [p, i64, p, i64, p, p, i, i, i, i, i, i, i, i, p],
         "ts_ssd_step": [p, p, i, p, p, p, p, i, p, i64, p, p, i, i, i, i, i, i, i, p],
+        "ts_ssd_walk": [p, p, p, p, p, i, p, i64, p, p, p, p, i, i, i, i, i, i, i, p],
         "ts_ssd_chunks": [p, p, p, p, p, i, p, i64, p, p, p, p, p, i, i, i, i, i, i, i, p],
         "ts_retention_prepare": [p, i, p, i64, p, p, i, i, i, i, i, i, i, p],
         "ts_delta_prepare": [p, i, p, p, p, p, i64, p, p, i64, p, p, p, p, p, i, i, i, i, i, i, i, i, f, i, p],
@@ -3204,6 +3205,19 @@ def _all_in_chunks(ctx, from_tokens: int) -> bool:
     return all(b - a >= from_tokens for a, b in zip(ctx.host_cu_seqlens, ctx.host_cu_seqlens[1:]))
 
 
+SSD_TABLE = 132             # floats of a chunk and head that the chunks' second sums leave for the walk
+SSD_WALK_MAX_PLACES = 128   # places of the state that the walk keeps in a workgroup
+
+
+def ssd_walks(chunks: int, longest: int, z: SsdSizes) -> bool:
+    """Whether a step's chunks are walked (their states stay in a workgroup) or worked all at once with the states between them
+    in memory. A walk takes 0.85 µs a chunk of the longest request (`longest` chunks of `chunks` in all); what it saves is fitted to
+    what both ways measured, 2.5 µs and 0.05 a chunk, 2.6 more for a million numbers of the state. Chunks and walk, µs: 64 heads of 64 x
+    128, 2,048 tokens 92.7 and 73.7; 16 of 128 x 128, 999 tokens in three requests 40.4 and 33.1, 2,048 in one 55.6 and 57.7; 4 of 64 x
+    128, 16 requests of 300 tokens 32.5 and 22.5, one of 2,048 26.3 and 43.5."""
+    return z.np <= SSD_WALK_MAX_PLACES and 0.85 * longest < 2.5 + chunks * (0.05 + 2.6e-6 * z.matrix)
+
+
 def ssd_scan(mixed: torch.Tensor, steps: torch.Tensor, logs: torch.Tensor, skip: torch.Tensor | None, state: torch.Tensor, ctx,
              sizes: SsdSizes, chunks_from: int = SSD_CHUNKS_FROM, keeps: torch.Tensor | None = None) -> torch.Tensor:
     """The recurrence over a packed step: per head S <- exp(log) S + step x B^T, y = S C + skip x, each request from and to
@@ -3231,11 +3245,17 @@ def ssd_scan(mixed: torch.Tensor, steps: torch.Tensor, logs: torch.Tensor, skip:
     if chunked:
         chunks, chunk_cu = _step_chunks(ctx, chunks_from, mixed.device)
         C = chunks.shape[0]
-        buf = torch.empty((C, z.matrix), dtype=torch.float32, device=mixed.device)
-        totals = torch.empty((C, z.heads), dtype=torch.float32, device=mixed.device)
-        _run("ssd_chunks", library().ts_ssd_chunks(
-            _ptr(out), _ptr(mixed), _ptr(steps), _ptr(logs), _ptr(skip), token_stride, _ptr(state), state.stride(0), _ptr(chunks), _ptr(chunk_cu),
-            _ptr(ctx.state_slots), _ptr(buf), _ptr(totals), C, S, z.heads, z.vdim, z.vp, z.groups, z.np, _stream()))
+        if ssd_walks(C, -(-ctx.max_query_len // SSD_CHUNK), z):
+            tables = torch.empty((C, z.heads, SSD_TABLE), dtype=torch.float32, device=mixed.device)
+            _run("ssd_walk", library().ts_ssd_walk(
+                _ptr(out), _ptr(mixed), _ptr(steps), _ptr(logs), _ptr(skip), token_stride, _ptr(state), state.stride(0), _ptr(chunks), _ptr(chunk_cu),
+                _ptr(ctx.state_slots), _ptr(tables), C, S, z.heads, z.vdim, z.vp, z.groups, z.np, _stream()))
+        else:
+            buf = torch.empty((C, z.matrix), dtype=torch.float32, device=mixed.device)
+            totals = torch.empty((C, z.heads), dtype=torch.float32, device=mixed.device)
+            _run("ssd_chunks", library().ts_ssd_chunks(
+                _ptr(out), _ptr(mixed), _ptr(steps), _ptr(logs), _ptr(skip), token_stride, _ptr(state), state.stride(0), _ptr(chunks), _ptr(chunk_cu),
+                _ptr(ctx.state_slots), _ptr(buf), _ptr(totals), C, S, z.heads, z.vdim, z.vp, z.groups, z.np, _stream()))
         if _all_in_chunks(ctx, chunks_from):
             return out
     _run("ssd_step", library().ts_ssd_step(

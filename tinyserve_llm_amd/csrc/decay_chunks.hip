@@ -60,56 +60,51 @@ static __device__ __forceinline__ void dc_log_column(float (&l)[DC_BLOCK], float
   for (int t = 0; t < DC_BLOCK; ++t) l[t] = b * DC_BLOCK + t < len ? dc_log(l[t] + bias, form, inv_tau) : 0.f;
 }
 
-// VT: 16-column tiles of a wave (four waves side by side).
+// VT: 16-column tiles of a wave (four waves side by side). A workgroup takes DP of the head's channels: with all 128 in one, two
+// requests of 2,048 tokens together were a workgroup a compute unit, whose loads and logarithms nothing hid (8 heads of
+// 128 x 256: 45.6 µs, and 37.7 in halves, each element's sums in the same order; heads of 64 x 64 are one workgroup as before).
 template <int D, int VT>
 __global__ void __launch_bounds__(DC_THREADS) decay_chunk_sums_kernel(const DecayChunks a) {
-  constexpr int ROW = D + 16;                               // (four neighbouring tokens' rows 16 banks apart)
-  __shared__ float k_s[SS_L][ROW], p_s[4][D];
+  constexpr int DP = D < 64 ? D : 64, PARTS = D / DP;
+  constexpr int ROW = DP + 16;                              // (four neighbouring tokens' rows 16 banks apart)
+  __shared__ float k_s[SS_L][ROW], p_s[4][DP];
+  const int d0 = blockIdx.z % PARTS * DP, vz = blockIdx.z / PARTS;
   const int c = blockIdx.x, h = blockIdx.y, tok0 = a.chunks[4 * c], len = a.chunks[4 * c + 1];
   // a thread takes a channel of a block (or two): the block's sum of logarithms, then k W(s, end] from the chunk's end back
-  constexpr int ITEMS = 4 * D, PER = (ITEMS + DC_THREADS - 1) / DC_THREADS;
-  float l[PER][DC_BLOCK], kk[PER][DC_BLOCK];
+  constexpr int ITEMS = 4 * DP;
+  static_assert(ITEMS <= DC_THREADS, "a channel of a block a thread");
+  const int d = threadIdx.x % DP, b0 = threadIdx.x / DP;
+  const bool takes = threadIdx.x < ITEMS;
+  float l[DC_BLOCK], kk[DC_BLOCK];
+  dc_column(l, a.z + (int64_t)tok0 * a.z_stride + h * D + d0, (int)a.z_stride, d, b0 % 4, len);
+  dc_column(kk, a.k + (int64_t)tok0 * a.k_stride + h * D + d0, (int)a.k_stride, d, b0 % 4, len);
+  if (takes) {
+    dc_log_column(l, a.z_bias[h * D + d0 + d], a.form, a.inv_tau, b0, len);
+    float all = 0.f;
 #pragma unroll
-  for (int i = 0; i < PER; ++i) {
-    const int item = threadIdx.x + i * DC_THREADS, d = item % D, b = item / D % 4;
-    dc_column(l[i], a.z + (int64_t)tok0 * a.z_stride + h * D, (int)a.z_stride, d, b, len);
-    dc_column(kk[i], a.k + (int64_t)tok0 * a.k_stride + h * D, (int)a.k_stride, d, b, len);
-  }
-#pragma unroll
-  for (int i = 0; i < PER; ++i) {
-    const int item = threadIdx.x + i * DC_THREADS, d = item % D, b = item / D;
-    if (item < ITEMS) {
-      dc_log_column(l[i], a.z_bias[h * D + d], a.form, a.inv_tau, b, len);
-      float all = 0.f;
-#pragma unroll
-      for (int t = DC_BLOCK - 1; t >= 0; --t) {
-        all += l[i][t];
-        if (blockIdx.z == 0 && b * DC_BLOCK + t < len) a.logs[((int64_t)(tok0 + b * DC_BLOCK + t) * a.heads + h) * D + d] = l[i][t];
-      }
-      p_s[b][d] = all;
+    for (int t = DC_BLOCK - 1; t >= 0; --t) {
+      all += l[t];
+      if (vz == 0 && b0 * DC_BLOCK + t < len) a.logs[((int64_t)(tok0 + b0 * DC_BLOCK + t) * a.heads + h) * D + d0 + d] = l[t];
     }
+    p_s[b0][d] = all;
   }
   __syncthreads();
+  if (takes) {
+    float after = 0.f;
+    for (int m = 3; m > b0; --m) after += p_s[m][d];
 #pragma unroll
-  for (int i = 0; i < PER; ++i) {
-    const int item = threadIdx.x + i * DC_THREADS, d = item % D, b = item / D;
-    if (item < ITEMS) {
-      float after = 0.f;
-      for (int m = 3; m > b; --m) after += p_s[m][d];
-#pragma unroll
-      for (int t = DC_BLOCK - 1; t >= 0; --t) {
-        k_s[b * DC_BLOCK + t][d] = kk[i][t] * expf(after);
-        after += l[i][t];
-      }
-      if (b == 0 && blockIdx.z == 0) a.totals[((int64_t)c * a.heads + h) * D + d] = expf(after);
+    for (int t = DC_BLOCK - 1; t >= 0; --t) {
+      k_s[b0 * DC_BLOCK + t][d] = kk[t] * expf(after);
+      after += l[t];
     }
+    if (b0 == 0 && vz == 0) a.totals[((int64_t)c * a.heads + h) * D + d0 + d] = expf(after);
   }
   __syncthreads();
   const int lane = threadIdx.x % TS_WAVE, r = lane % 16, g = lane / 16, wave = wave_index();
-  const int v0 = blockIdx.z * (64 * VT) + wave * (16 * VT);
-  float4_t acc[D / 16][VT];
+  const int v0 = vz * (64 * VT) + wave * (16 * VT);
+  float4_t acc[DP / 16][VT];
 #pragma unroll
-  for (int i = 0; i < D / 16; ++i)
+  for (int i = 0; i < DP / 16; ++i)
 #pragma unroll
     for (int j = 0; j < VT; ++j) acc[i][j] = (float4_t){0.f, 0.f, 0.f, 0.f};
   const float* v = a.v + (int64_t)tok0 * a.v_stride + h * a.vdim + v0 + r;
@@ -132,15 +127,15 @@ __global__ void __launch_bounds__(DC_THREADS) decay_chunk_sums_kernel(const Deca
 #pragma unroll
     for (int s = 0; s < 4; ++s)
 #pragma unroll
-      for (int i = 0; i < D / 16; ++i) {
+      for (int i = 0; i < DP / 16; ++i) {
         const float ka = k_s[b * DC_BLOCK + 4 * s + g][16 * i + r];
 #pragma unroll
         for (int j = 0; j < VT; ++j) acc[i][j] = mfma_f32(ka, vv[b & 1][s][j], acc[i][j]);
       }
   }
-  float* dst = a.buf + ((int64_t)c * a.heads + h) * D * a.vdim + v0 + r;
+  float* dst = a.buf + (((int64_t)c * a.heads + h) * D + d0) * a.vdim + v0 + r;
 #pragma unroll
-  for (int i = 0; i < D / 16; ++i)
+  for (int i = 0; i < DP / 16; ++i)
 #pragma unroll
     for (int e = 0; e < 4; ++e)
 #pragma unroll
@@ -395,7 +390,7 @@ __global__ void __launch_bounds__(DC_THREADS, 2) decay_chunk_out_kernel(const De
 template <int D, int VT>
 static int launch_decay_chunks(const DecayChunks& a, int num_chunks, int num_seqs, hipStream_t stream) {
   const dim3 grid(num_chunks, a.heads, a.vdim / (64 * VT));
-  decay_chunk_sums_kernel<D, VT><<<grid, DC_THREADS, 0, stream>>>(a);
+  decay_chunk_sums_kernel<D, VT><<<dim3(num_chunks, a.heads, grid.z * (D < 64 ? 1 : D / 64)), DC_THREADS, 0, stream>>>(a);
   decay_chunk_scan_kernel<<<dim3(num_seqs, a.heads, (D * a.vdim / 4 + DC_THREADS - 1) / DC_THREADS), DC_THREADS, 0, stream>>>(a, D);
   if (a.bonus) decay_chunk_out_kernel<D, VT, true><<<grid, DC_THREADS, 0, stream>>>(a);
   else decay_chunk_out_kernel<D, VT, false><<<grid, DC_THREADS, 0, stream>>>(a);

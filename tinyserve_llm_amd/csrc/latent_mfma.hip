@@ -345,11 +345,16 @@ extern "C" int ts_paged_attention_latent_mfma(void* out, int out_dtype, const fl
 // through LDS, where they go straight from memory, three steps in turn (one worked on, two under way). What bounds it: the
 // matrix cores, 48 products a wave and step of 256 numbers (16 for the scores, 32 for the weights' two bfloat16 terms),
 // beside the wave's softmax; the kernel above reads every token's keys from the second-level cache anew (2 GB for 2,048
-// tokens over 256 numbers: 560 us, this one 128). In LDS a key's 16-byte pieces are turned by the key's place among
-// the 16 that an operand takes, a value column's four by half the column's number: an operand's read then meets every bank once.
+// tokens over 256 numbers: 560 us, this one 112). The operands are read LP_AHEAD ahead of the products that take them, the
+// first values ahead of the softmax: with each pair of reads waited for, as the compiler lays them out, it took 129 (heads of
+// 320 numbers 118 and now 100, 130 heads of 80 388 and 351; 6 and 8 ahead the same). Waves of 32 rows, four to a workgroup and
+// two workgroups to a unit, read half as much from LDS and took 138 to 160: no registers are left to read ahead into.
+// In LDS a key's 16-byte pieces are turned by the key's place among the 16 that an operand takes, a value column's four by
+// half the column's number: an operand's read then meets every bank once.
 #define LP_WAVES 8
 #define LP_ROWS (16 * LP_WAVES)
 #define LP_RING 3
+#define LP_AHEAD 4
 
 // CP: 32-wide pieces of a cached row, VB: 16-wide blocks of value columns, both rounded up to what is built.
 template <int CP, int VB, typename TO>
@@ -442,14 +447,29 @@ latent_attention_tiles_kernel(TO* __restrict__ out, const float* __restrict__ q,
     // (a score's pieces in four sums, added in the order of the kernel above, whose scores these are bit for bit: in one sum
     // of all its pieces the rows were 1.9e-6 from 64 bits instead of 1.1e-6)
     float4_t st[2], piece[4][2];
+    u32x4_t held[LP_AHEAD];                                 // (first keys, then values)
+    auto key_piece = [&](int n) {
+      const int c = n >> 1, tau = n & 1;
+      return *(const u32x4_t*)(at + kat[c & 3] + (c >> 2) * 256 + tau * (4 * SL * 16));
+    };
 #pragma unroll
-    for (int c = 0; c < CP; ++c)
+    for (int n = 0; n < LP_AHEAD; ++n) held[n] = key_piece(n);
 #pragma unroll
-      for (int tau = 0; tau < 2; ++tau)
-        piece[c & 3][tau] = mfma32v(*(const u32x4_t*)(at + kat[c & 3] + (c >> 2) * 256 + tau * (4 * SL * 16)), qf[c],
-                                    c < 4 ? (float4_t){0.f, 0.f, 0.f, 0.f} : piece[c & 3][tau]);
+    for (int n = 0; n < 2 * CP; ++n) {
+      const int c = n >> 1, tau = n & 1;
+      piece[c & 3][tau] = mfma32v(held[n % LP_AHEAD], qf[c], c < 4 ? (float4_t){0.f, 0.f, 0.f, 0.f} : piece[c & 3][tau]);
+      if (n + LP_AHEAD < 2 * CP) held[n % LP_AHEAD] = key_piece(n + LP_AHEAD);
+    }
+    __builtin_amdgcn_sched_group_barrier(0x100, LP_AHEAD, 0);
+#pragma unroll
+    for (int n = 0; n < 2 * CP; ++n) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      if (n + LP_AHEAD < 2 * CP) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+    }
 #pragma unroll
     for (int tau = 0; tau < 2; ++tau) st[tau] = piece[0][tau] + piece[1][tau] + piece[2][tau] + piece[3][tau];
+#pragma unroll
+    for (int i = 0; i < LP_AHEAD; ++i) held[i] = *(const u32x4_t*)(at + vat + i * 1024);
     float s[8];
 #pragma unroll
     for (int j = 0; j < 8; ++j) s[j] = st[j >> 2][j & 3] * scale_log2;
@@ -486,9 +506,14 @@ latent_attention_tiles_kernel(TO* __restrict__ out, const float* __restrict__ q,
     l = l * alpha + sum;
 #pragma unroll
     for (int i = 0; i < VB; ++i) {
-      const u32x4_t vf = *(const u32x4_t*)(at + vat + i * 1024);
-      acc[i] = mfma32v(vf, hi, acc[i]);
-      acc[i] = mfma32v(vf, lo, acc[i]);
+      acc[i] = mfma32v(held[i % LP_AHEAD], hi, acc[i]);
+      acc[i] = mfma32v(held[i % LP_AHEAD], lo, acc[i]);
+      if (i + LP_AHEAD < VB) held[i % LP_AHEAD] = *(const u32x4_t*)(at + vat + (i + LP_AHEAD) * 1024);
+    }
+#pragma unroll
+    for (int i = 0; i < VB; ++i) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 2, 1);
+      if (i + LP_AHEAD < VB) __builtin_amdgcn_sched_group_barrier(0x100, 1, 1);
     }
   }
   wait_for<0>();                                            // (the steps fetched beyond the last land before the LDS is another's)

@@ -2709,7 +2709,8 @@ def latent_wide_tiles(cu_seqlens: "list[int]", heads: int, reach: int) -> bool:
     """Whether a step of more than decoded tokens (request i feeds cu_seqlens[i + 1] - cu_seqlens[i]), nobody of which sees more
     than `reach` keys, is the faster in tiles of `LATENT_WIDE_TILE_ROWS` rows: eight waves share a tile's keys where the
     kernel of 32 rows reads them anew for each, but a tile of a token of few heads is mostly padding. Rows of 256 numbers,
-    narrow and wide: 32 heads, 2,048 tokens 560 and 128 µs, 256 tokens 24.8 and 22.5, 300 decoded tokens (contexts of 1,000) beside a
+    narrow and wide: 32 heads, 2,048 tokens 560 and 112 µs, 256 tokens 24.8 and 21.8; before the wide tiles' operands were read
+    ahead, which took a fourteenth to an eighth off them since: 300 decoded tokens (contexts of 1,000) beside a
     prompt of 2 89 and 102, of 128 90 and 105, 256 beside one of 256 87 and 79; 48 heads, 300 beside one of 2 145 and 105; 128 heads 232 and 123."""
     rows = cu_seqlens[-1] * heads
     if rows < (LATENT_MANY_ROWS if reach > LATENT_SHORT_REACH else LATENT_MANY_SHORT_ROWS):

@@ -1,5 +1,6 @@
-"""Products of many rows: with the reduction in slices (gemm_slices.hip) against the same product in 64 bits, their endings against
-the kernels they stand in for, and the rule that chooses them."""
+"""Steps of many rows: products with the reduction in slices (gemm_slices.hip) against 64 bits, their endings against the kernels
+they stand in for and the rule that chooses them; the gated product in every tile; values on their way into transposed pages;
+prompts' attention; walks over chunks of the state-space recurrence."""
 
 from __future__ import annotations
 

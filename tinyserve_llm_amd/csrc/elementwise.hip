@@ -341,7 +341,7 @@ __global__ void rope_store_kernel(T* __restrict__ q_out, T* __restrict__ k_cache
     // writes 8 tokens as one 16-byte piece of a transposed page, for every 8 neighbouring tokens whose slots are consecutive
     // and begin at a multiple of 8, wherever in the step such a run begins: the workgroup in whose group it does writes
     // it whole, up to 7 tokens of the next group with it. (With runs counted from the group's own start a prompt behind 13
-    // decoding requests went a store a token: 1,514 tokens, 8 value heads of 128, 20.5 us and now 9.)
+    // decoding requests went a store a token: 1,514 tokens, 8 value heads of 128, 20.5 us and now 12.7.)
     constexpr int VP = 16 / sizeof(T);                // elements of a 16-byte piece
     static_assert(VP == 8 || sizeof(T) == 4, "runs of 8 tokens are pieces of bfloat16");
     constexpr int RUN = 8, ROWS = ROPE_TOK + RUN - 1;

@@ -1,6 +1,6 @@
 """Steps of many rows: products with the reduction in slices (gemm_slices.hip) against 64 bits, their endings against the kernels
 they stand in for and the rule that chooses them; the gated product in every tile; values on their way into transposed pages;
-prompts' attention; walks over chunks of the state-space recurrence."""
+prompts' attention; walks over chunks of the state-space recurrence; products per head."""
 
 from __future__ import annotations
 
@@ -267,3 +267,32 @@ def test_a_walk_over_the_chunks_leaves_what_the_chunks_do(heads, vdim, groups, p
     assert torch.equal(state, want_state)
     size = float(want.abs().max()) + float(start.abs().max()) * places ** 0.5 + 64.0
     assert float((y - want).abs().max()) <= 2.0 ** -22 * 8 * size
+
+
+# (tokens at the edges of two and four blocks of 16 a wave, a block that ends early; columns in fours or not; a ragged reduction)
+@pytest.mark.gpu
+@pytest.mark.parametrize("gated", [False, True])
+@pytest.mark.parametrize("heads, k, n", [(32, 72, 100), (32, 64, 256), (128, 128, 62)])
+@pytest.mark.parametrize("x_type, y_type", [(torch.float32, torch.float32), (torch.float32, BF), (BF, torch.float32), (BF, BF)])
+@pytest.mark.parametrize("tokens", [257, 512, 1000, 2065])
+def test_products_per_head_are_the_same_bits_whatever_the_tokens(tokens, x_type, y_type, heads, k, n, gated):
+    """Against the same rows 48 at a time (one block of tokens a wave), and against 64 bits: sums of k products good to k 2^-24 of the
+    sum of their sizes, the gate to 2^-21, in bfloat16 half a unit in the last place more. Rows lie apart, what is beside them stays."""
+    g = torch.Generator().manual_seed(tokens + n)
+    x = torch.randn(tokens, heads, k, generator=g).to(x_type).cuda()
+    w = (torch.randn(heads, n, k, generator=g) * k ** -0.5).to(BF).cuda().transpose(1, 2)
+    gate = torch.randn(tokens, heads * n + 4, generator=g).cuda()[:, :heads * n] if gated else None
+    kept = torch.full((tokens + 1, heads, n + 4), 7.0, dtype=y_type, device="cuda")
+    out = hip.heads_gemm(x, w, kept[:tokens, :, :n], gate)
+    few = torch.empty(tokens, heads, n, dtype=y_type, device="cuda")
+    for a in range(0, tokens, 48):
+        hip.heads_gemm(x[a:a + 48], w, few[a:a + 48], None if gate is None else gate[a:a + 48])
+    assert torch.equal(out, few) and torch.all(kept[tokens] == 7.0) and torch.all(kept[:, :, n:] == 7.0)
+    picked = [0, tokens // 2, tokens - 17, tokens - 1]
+    xs, ws = x[picked].to(BF).double().cpu().transpose(0, 1), w.double().cpu()
+    want, size = torch.bmm(xs, ws.contiguous()).transpose(0, 1), torch.bmm(xs.abs(), ws.abs().contiguous()).transpose(0, 1)
+    if gated:
+        turn = torch.sigmoid(gate[picked].double().cpu().view(len(picked), heads, n))
+        want, size = want * turn, size * turn
+    bound = size * (k * 2.0 ** -24 + (2.0 ** -21 if gated else 0.0)) + (want.abs() * 2.0 ** -8 if y_type == BF else 0.0)
+    assert torch.all((out[picked].double().cpu() - want).abs() <= bound + 1e-30)

@@ -568,14 +568,17 @@ extern "C" int ts_paged_attention_latent_tiles(void* out, int out_dtype, const f
 // ---- products per head on the matrix cores ---------------------------------------------------------------------
 // y[t, h, n] = sum_k x[t, h, k] w[h][n][k] for bfloat16 matrices whose k runs along memory (a matrix stored [k, n]
 // comes as a transposed copy), x 32-bit (rounded to bfloat16 once, as a projection's operand is) or bfloat16, 32-bit
-// sums, times sigmoid(gate) on the way out if there is one. A workgroup makes 64 tokens by 64 columns of one head, a
-// wave 16 tokens: the matrix's rows are the instruction's rows, so that a lane ends with four adjacent columns of
-// one token. Operands come straight from memory in 16-byte pieces; pieces past K are zeros of x against the
-// matrix's last piece.
+// sums, times sigmoid(gate) on the way out if there is one. A wave makes RT blocks of 16 tokens by 64 columns of one head, a
+// workgroup four waves' tokens: the matrix's rows are the instruction's rows, so that a lane ends with four adjacent columns of
+// one token. Operands come straight from memory in 16-byte pieces; pieces past K are zeros of x against the matrix's last piece.
+// What bounds it is loads and stores of 64 bytes of each of 16 rows: results are turned through shared memory into rows of 64
+// columns (a twentieth less), and where that leaves enough waves a wave's pieces of the matrix serve two or four blocks of tokens.
+// 2,048 tokens, 32 heads, 1, 2 and 4 blocks: K 64 by 256, 32-bit rows in and out 29.9, 26.9 and 23.6 us (31.3 before), K 256 by 64, bfloat16 23.6,
+// 17.6 and 15.9 (24.0), of 32-bit rows 27.2, 21.7 and 27.3 (27.9); 300 tokens 7.7, 8.8 and 11.3. Every result is the same bits.
 #define HM_TOKENS 64
 #define HM_COLS 64
 
-template <typename TX, typename TO>
+template <int RT, typename TX, typename TO>
 __global__ void __launch_bounds__(LM_THREADS)
 heads_gemm_mfma_kernel(TO* __restrict__ y, int64_t y_token, int64_t y_head, const TX* __restrict__ x, int64_t x_token,
                        int64_t x_head, const bf16_t* __restrict__ w, int64_t w_head, int64_t w_n, int num_tokens, int N, int K,
@@ -583,57 +586,80 @@ heads_gemm_mfma_kernel(TO* __restrict__ y, int64_t y_token, int64_t y_head, cons
   const int wave = wave_index(), lane = threadIdx.x & (TS_WAVE - 1);
   const int r = lane & 15, g = lane >> 4;
   const int h = blockIdx.y, n0 = blockIdx.z * HM_COLS;
-  const int t = blockIdx.x * HM_TOKENS + 16 * wave + r;
-  const TX* xrow = x + (int64_t)min(t, num_tokens - 1) * x_token + (int64_t)h * x_head;
-  const bf16_t* wh = w + (int64_t)h * w_head;
-  float4_t acc[HM_COLS / 16];
+  const int t0 = RT * (blockIdx.x * HM_TOKENS + 16 * wave);
+  const TX* xrow[RT];
 #pragma unroll
-  for (int nb = 0; nb < HM_COLS / 16; ++nb) acc[nb] = (float4_t){0.f, 0.f, 0.f, 0.f};
+  for (int rt = 0; rt < RT; ++rt) xrow[rt] = x + (int64_t)min(t0 + 16 * rt + r, num_tokens - 1) * x_token + (int64_t)h * x_head;
+  const bf16_t* wh = w + (int64_t)h * w_head;
+  float4_t acc[RT][HM_COLS / 16];
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+    for (int nb = 0; nb < HM_COLS / 16; ++nb) acc[rt][nb] = (float4_t){0.f, 0.f, 0.f, 0.f};
 #pragma unroll 4
   for (int k0 = 0; k0 < K; k0 += 32) {
     const int k = k0 + 8 * g, kc = min(k, K - 8);
-    uint4 b;
-    if constexpr (sizeof(TX) == 4) {
-      const float4 lo = *(const float4*)(xrow + kc), hi = *(const float4*)(xrow + kc + 4);
-      b = make_uint4(pack_bf16(lo.x, lo.y), pack_bf16(lo.z, lo.w), pack_bf16(hi.x, hi.y), pack_bf16(hi.z, hi.w));
-    } else {
-      b = *(const uint4*)(xrow + kc);
+    uint4 b[RT];
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) {
+      if constexpr (sizeof(TX) == 4) {
+        const float4 lo = *(const float4*)(xrow[rt] + kc), hi = *(const float4*)(xrow[rt] + kc + 4);
+        b[rt] = make_uint4(pack_bf16(lo.x, lo.y), pack_bf16(lo.z, lo.w), pack_bf16(hi.x, hi.y), pack_bf16(hi.z, hi.w));
+      } else {
+        b[rt] = *(const uint4*)(xrow[rt] + kc);
+      }
+      if (k >= K) b[rt] = make_uint4(0, 0, 0, 0);
     }
-    if (k >= K) b = make_uint4(0, 0, 0, 0);
 #pragma unroll
     for (int nb = 0; nb < HM_COLS / 16; ++nb) {
       const int n = min(n0 + 16 * nb + r, N - 1);
-      acc[nb] = mfma32(*(const uint4*)(wh + (int64_t)n * w_n + kc), b, acc[nb]);
+      const uint4 a = *(const uint4*)(wh + (int64_t)n * w_n + kc);
+#pragma unroll
+      for (int rt = 0; rt < RT; ++rt) acc[rt][nb] = mfma32(a, b[rt], acc[rt][nb]);
     }
   }
-  if (t >= num_tokens) return;
-  // whole fours of columns go out in one store (four of a number each: 51 µs against 36 for 2,048 tokens by 32 heads of 256)
-  TO* yrow = y + (int64_t)t * y_token + (int64_t)h * y_head;
+  // whole fours of columns go out in one store of a lane, 16 lanes side by side, which the wave turns through shared memory
   if (N % 4 == 0 && ((y_token | y_head) & 3) == 0 && ((uintptr_t)y & (4 * sizeof(TO) - 1)) == 0) {
+    __shared__ __attribute__((aligned(16))) float4_t turn[LM_WAVES][16][HM_COLS / 4 + 1];
 #pragma unroll
-    for (int nb = 0; nb < HM_COLS / 16; ++nb) {
-      const int n = n0 + 16 * nb + 4 * g;
-      if (n >= N) continue;
-      float4_t v = acc[nb];
-      if (gate) {
+    for (int rt = 0; rt < RT; ++rt) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) v[j] = v[j] / (1.0f + expf(-gate[(int64_t)t * gate_token + (int64_t)h * N + n + j]));
+      for (int nb = 0; nb < HM_COLS / 16; ++nb) turn[wave][r][4 * nb + g] = acc[rt][nb];
+      __builtin_amdgcn_wave_barrier();
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int at = 4 * i + g, to = t0 + 16 * rt + at, n = n0 + 4 * r;
+        float4_t v = turn[wave][at][r];
+        if (to >= num_tokens || n >= N) continue;
+        if (gate) {
+          const float* gr = gate + (int64_t)to * gate_token + (int64_t)h * N + n;
+#pragma unroll
+          for (int j = 0; j < 4; ++j) v[j] = v[j] / (1.0f + expf(-gr[j]));
+        }
+        TO* yrow = y + (int64_t)to * y_token + (int64_t)h * y_head + n;
+        if constexpr (sizeof(TO) == 4) *(float4_t*)yrow = v;
+        else *(uint2*)yrow = make_uint2(pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3]));
       }
-      if constexpr (sizeof(TO) == 4) *(float4_t*)(yrow + n) = v;
-      else *(uint2*)(yrow + n) = make_uint2(pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3]));
+      __builtin_amdgcn_wave_barrier();
     }
     return;
   }
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt) {
+    const int t = t0 + 16 * rt + r;
+    if (t >= num_tokens) continue;
+    TO* yrow = y + (int64_t)t * y_token + (int64_t)h * y_head;
 #pragma unroll
   for (int nb = 0; nb < HM_COLS / 16; ++nb)
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const int n = n0 + 16 * nb + 4 * g + j;
       if (n >= N) continue;
-      float v = acc[nb][j];
+      float v = acc[rt][nb][j];
       if (gate) v = v / (1.0f + expf(-gate[(int64_t)t * gate_token + (int64_t)h * N + n]));
       Num<TO>::st(yrow + n, v);
     }
+  }
 }
 
 // w: bfloat16 [heads][N][K] with K along memory (stride w_n between rows, a multiple of 8; K a multiple of 8);
@@ -646,15 +672,26 @@ extern "C" int ts_heads_gemm_mfma(void* y, int y_dtype, int64_t y_token, int64_t
   if (heads <= 0 || heads > 65535 || N <= 0 || K < 8 || K % 8 || w_n % 8 || w_head % 8 || ((uintptr_t)w & 15) ||
       ((uintptr_t)x & 15) || (x_token * x_size) % 16 || (x_head * x_size) % 16 || (N + HM_COLS - 1) / HM_COLS > 65535)
     return TS_BAD_SHAPE;
-  dim3 grid((num_tokens + HM_TOKENS - 1) / HM_TOKENS, heads, (N + HM_COLS - 1) / HM_COLS);
-#define HM_LAUNCH(TX, TO) \
-  heads_gemm_mfma_kernel<TX, TO><<<grid, LM_THREADS, 0, stream>>>((TO*)y, y_token, y_head, (const TX*)x, x_token, x_head, \
+  // blocks of 16 tokens a wave: two from 512 workgroups of one on, four from 2,048 (of bfloat16 rows, whose loads are half as many,
+  // from 1,024); reductions below 64, whose waves are over at once, keep one (40 by 100, 24 heads, 1,000 tokens 6.6 us, 7.2 and 8.6)
+  const int64_t groups = (int64_t)((num_tokens + HM_TOKENS - 1) / HM_TOKENS) * heads * ((N + HM_COLS - 1) / HM_COLS);
+  const int blocks = K < 64 || groups < 512 ? 1 : groups >= 2048 || (groups >= 1024 && x_dtype == 1) ? 4 : 2;
+  const dim3 grid((num_tokens + blocks * HM_TOKENS - 1) / (blocks * HM_TOKENS), heads, (N + HM_COLS - 1) / HM_COLS);
+#define HM_GO(RT, TX, TO) \
+  heads_gemm_mfma_kernel<RT, TX, TO><<<grid, LM_THREADS, 0, stream>>>((TO*)y, y_token, y_head, (const TX*)x, x_token, x_head, \
       (const bf16_t*)w, w_head, w_n, num_tokens, N, K, gate, gate_token)
+#define HM_LAUNCH(TX, TO) \
+  do { \
+    if (blocks == 1) HM_GO(1, TX, TO); \
+    else if (blocks == 2) HM_GO(2, TX, TO); \
+    else HM_GO(4, TX, TO); \
+  } while (0)
   if (x_dtype == 0 && y_dtype == 0) HM_LAUNCH(float, float);
   else if (x_dtype == 0 && y_dtype == 1) HM_LAUNCH(float, bf16_t);
   else if (x_dtype == 1 && y_dtype == 0) HM_LAUNCH(bf16_t, float);
   else if (x_dtype == 1 && y_dtype == 1) HM_LAUNCH(bf16_t, bf16_t);
   else return TS_BAD_DTYPE;
 #undef HM_LAUNCH
+#undef HM_GO
   return ts_check_launch();
 }

@@ -1,0 +1,145 @@
+"""The library's own module (calls.cpp) over launchers that only answer: what it does with each answer, on tensors in host memory."""
+
+from __future__ import annotations
+
+import ctypes
+import importlib.machinery
+import importlib.util
+import os
+import re
+import subprocess
+
+import pytest
+import torch
+
+from tinyserve_llm_amd.csrc import build
+from tinyserve_llm_amd.ops import hip
+
+BF, F32, I32 = torch.bfloat16, torch.float32, torch.int32
+OK, BAD_DTYPE, BAD_SHAPE, LAUNCH_FAILED, TOO_LARGE = range(5)
+
+STUB = """
+#include <map>
+#include <string>
+namespace c10::hip { struct NoStream { hipStream_t stream() const { return nullptr; } }; inline NoStream no_stream() { return {}; } }
+#define is_cuda is_cpu
+#define getCurrentHIPStream no_stream
+static std::map<std::string, int> answers;
+static std::string called;
+static int answer(const char* name) { called += std::string(name) + " "; return answers[name]; }
+extern "C" void stub_answer(const char* name, int rc) { answers[name] = rc; }
+extern "C" const char* stub_called() { static std::string last; last = called; called.clear(); return last.c_str(); }
+"""
+
+
+@pytest.fixture(scope="session")
+def stub(tmp_path_factory):
+    """(the module, answer(launcher, rc), called() -> the launchers called since it was last asked)."""
+    folder = tmp_path_factory.mktemp("calls")
+    with open(os.path.join(build.HERE, "calls.cpp")) as f:
+        source = f.read()
+    with open(os.path.join(build.HERE, "entry_points.h")) as f:
+        points = re.findall(r"^int (ts_\w+)(\([^;]*\));", f.read(), re.M)
+    headers = re.findall(r'^#include .*$', source, re.M)
+    launchers = [f'extern "C" int {name}{parameters} {{ return answer("{name}"); }}' for name, parameters in points]
+    code, lib = folder / "stub.cpp", folder / "stub.so"
+    code.write_text("\n".join([*headers, STUB, *launchers, f'#include "{build.HERE}/calls.cpp"\n']))
+    links = [flag for flag in build.LINK if flag != "-lhipblaslt"]
+    subprocess.run([build._hipcc(), *build._compile_flags("calls.cpp"), f"-I{build.HERE}", "-shared", "-Wl,-Bsymbolic", str(code), "-x", "none",
+                    f"-L{build._torch_folder()}/lib", *links, "-o", str(lib)], check=True)
+    loader = importlib.machinery.ExtensionFileLoader("tinyserve_hip_calls", str(lib))
+    module = importlib.util.module_from_spec(importlib.util.spec_from_loader(loader.name, loader))
+    loader.exec_module(module)
+    c = ctypes.CDLL(str(lib))
+    c.stub_called.restype = ctypes.c_char_p
+    return module, lambda name, rc: c.stub_answer(name.encode(), rc), lambda: c.stub_called().decode().split()
+
+
+def ints(*values):
+    return torch.tensor(values, dtype=I32)
+
+
+def caches(pages=4, page=32, heads=2, dim=64):
+    return torch.zeros(pages, page, heads, dim, dtype=BF), torch.zeros(pages, heads, dim, page, dtype=BF).permute(0, 3, 1, 2)
+
+
+def bf(*shape):
+    return torch.zeros(*shape, dtype=BF)
+
+
+def step(lead, softcap=0.0):
+    """`attention_step` of `lead` decoding requests beside a prompt of 40 tokens; a few keys a workgroup of the decoding part."""
+    T = lead + 40
+    k, v = caches()
+    return (bf(T, 4, 64), k, v, torch.zeros(lead + 1, 2, dtype=I32), torch.zeros(T, dtype=I32), torch.zeros(T, dtype=I32), torch.zeros(5, 2, dtype=I32), 0.125, 0,
+            softcap, False, None, None, None, 1, lead, 64 if lead else 0, 2 if lead else 0, 32, 4, 1, 0, lead)
+
+
+# a plain call of every function, and the launchers that it makes
+PLAIN = {
+    "rmsnorm": (lambda: (bf(3, 64), bf(64), 1e-5, bf(3, 64), True), ["ts_rmsnorm"]),
+    "stream_post_norm": (lambda: (torch.zeros(3, 64), torch.zeros(3, 64), torch.zeros(64), None, 1e-6, torch.zeros(64), 1e-5, 1), ["ts_stream_post_norm"]),
+    "stream_update_norm": (lambda: (torch.zeros(3, 64), bf(3, 64), None, 0.5, bf(64), 1e-5, 1), ["ts_stream_update_norm"]),
+    "gemm_library": (lambda: (bf(9, 64), bf(16, 64), True), ["ts_gemm_library_bf16"]),
+    "gemm_slices": (lambda: (bf(9, 384), bf(16, 384), 0, 2, False, bf(9, 16), bf(16), 1e-5), ["ts_gemm_slices_bf16"]),
+    "gemm_glu": (lambda: (bf(9, 64), bf(32, 64), 0, 0, 0.0, 1.0, 0.0), ["ts_gemm_glu_bf16"]),
+    "gemm_rows64": (lambda: (bf(9, 1024), bf(8, 32, 64, 8), False, 1, None, 0.0, 0.0, 0.0, 0.0), ["ts_gemm_rows64_bf16"]),
+    "gemm_rows64_sliced": (lambda: (bf(9, 1024), bf(4, 32, 64, 8), 2, None, bf(64)), ["ts_gemm_rows64_sliced_bf16"]),
+    "rope_store": (lambda: (bf(3, 8 * 64), torch.zeros(9, 64), ints(0, 1, 2), ints(0, 1, 2), *caches(), 4, 2, 64), ["ts_rope_store"]),
+    "qkv_rope_store_sliced": (lambda: (bf(3, 1024), bf(32, 32, 64, 8), 2, torch.zeros(9, 64), ints(0, 1, 2), ints(0, 1, 2), *caches(), 4, 2, 64, 0.0, None),
+                              ["ts_gemm_rows64_sliced_rope_bf16"]),
+    "qkv_finish": (lambda: (torch.zeros(3, 8 * 64), torch.zeros(16, dtype=torch.float64), ints(0, 1, 2), ints(0, 1, 2), *caches(), 4, 2, 64, 64, 1, False, None, 1e-6, 1.0),
+                   ["ts_qkv_finish"]),
+    "attention_step": (lambda: step(0), ["ts_paged_attention_prefill"]),
+    "capped_glu": (lambda: (torch.zeros(3, 64), 3.0, 1.0, 0.0, 1, 0), ["ts_capped_glu"]),
+    "mlstm_finish": (lambda: (torch.zeros(3, 64), None, torch.zeros(3, 64), 2, 32, 1e-6, 1, False), ["ts_mlstm_finish"]),
+}
+
+
+def test_every_function_is_here(stub):
+    assert sorted(PLAIN) == sorted(n for n in dir(stub[0]) if not n.startswith("_"))
+
+
+@pytest.mark.parametrize("name", PLAIN)
+def test_a_refusal_is_left_to_the_general_function_and_a_failed_launch_is_raised(stub, name):
+    """A launch that failed may have run, and written to what it updates in place: it is not to be made once more."""
+    module, answer, called = stub
+    args, launchers = PLAIN[name]
+    assert getattr(module, name)(*args()) is not None and called() == launchers
+    for rc in (BAD_DTYPE, BAD_SHAPE, TOO_LARGE):
+        answer(launchers[0], rc)
+        assert getattr(module, name)(*args()) is None and called() == launchers
+    answer(launchers[0], LAUNCH_FAILED)
+    with pytest.raises(hip.KernelError, match=hip._ERRORS[LAUNCH_FAILED]):
+        getattr(module, name)(*args())
+    assert called() == launchers
+    answer(launchers[0], OK)
+
+
+@pytest.mark.parametrize("softcap", [0.0, 20.0])
+def test_a_step_whose_decoding_part_has_run_is_not_made_again(stub, softcap):
+    module, answer, called = stub
+    general = "_general" if softcap else ""
+    decode, prefill = f"ts_paged_attention_decode{general}", f"ts_paged_attention_prefill{general}"
+    assert module.attention_step(*step(2, softcap)) is not None and called() == [decode, prefill]
+    answer(decode, BAD_SHAPE)
+    assert module.attention_step(*step(2, softcap)) is None and called() == [decode]
+    answer(decode, OK)
+    for rc in (BAD_SHAPE, LAUNCH_FAILED):
+        answer(prefill, rc)
+        with pytest.raises(hip.KernelError, match=f"paged_attention_prefill{general}: {re.escape(hip._ERRORS[rc])}"):
+            module.attention_step(*step(2, softcap))
+        assert called() == [decode, prefill]
+    answer(prefill, BAD_SHAPE)
+    assert module.attention_step(*step(0, softcap)) is None and called() == [prefill]
+    answer(prefill, OK)
+
+
+def test_a_stream_is_updated_by_one_launch(stub, monkeypatch):
+    module, answer, called = stub
+    monkeypatch.setattr(hip, "_native", lambda: module)
+    answer("ts_stream_update_norm", LAUNCH_FAILED)
+    with pytest.raises(hip.KernelError, match="stream_update_norm"):
+        hip.stream_update_norm(torch.zeros(3, 64), bf(3, 64), weights=(bf(64), None), eps=1e-5, out_dtype=BF)
+    assert called() == ["ts_stream_update_norm"]
+    answer("ts_stream_update_norm", OK)

@@ -6,7 +6,9 @@
 // Every function here serves the plain case of the function of the same name in ops/hip.py, whose arguments it takes in
 // order, and answers None where anything is another way (a type, a stride, an alignment, a tensor that is not on a GPU) or
 // the launcher refuses: that function then goes its own, general way, which also says what is wrong. Nothing has been
-// launched by then. Like all of ops/hip.py, calls go to the current device's current stream.
+// launched by then: a launch that failed, and a refusal behind a launch of the same call, are raised as `_run` of ops/hip.py raises
+// them (what has run may have written to its operands, and is not to run twice). Like all of ops/hip.py, calls go to the
+// current device's current stream.
 #include <Python.h>
 
 #include <ATen/core/Tensor.h>
@@ -99,6 +101,20 @@ bool pieces(const Tensor& x) { return x.dim() == 2 && x.stride(1) == 1 && x.stri
 
 Tensor make(const Tensor& like, at::IntArrayRef sizes, at::ScalarType type) { return at::empty(sizes, like.options().dtype(type)); }
 
+// Whether a launcher has refused its operands, which it does before it launches anything. An error where it is more than that: a failed
+// launch (or an earlier one's failure, found only now), or a refusal `behind` a launch of this call.
+template <class F> bool refused(const char* name, const F& launch, bool behind = false) {
+  const int rc = launch();
+  if (rc == TS_OK) return false;
+  if (rc != TS_LAUNCH_FAILED && !behind) return true;
+  PyObject* hip = PyImport_ImportModule("tinyserve_llm_amd.ops.hip");
+  PyObject* none = hip ? PyObject_CallMethod(hip, "_run", "si", name, rc) : nullptr;      // (raises for every answer but TS_OK)
+  Py_XDECREF(hip);
+  Py_XDECREF(none);
+  throw python_error();
+}
+#define TS_REFUSED(NAME, CALL, ...) refused(NAME, [&] { return CALL; }, ##__VA_ARGS__)
+
 PyObject* wrap(const Tensor& t) { return THPVariable_Wrap(t); }
 PyObject* none() { Py_RETURN_NONE; }
 
@@ -139,7 +155,9 @@ PyObject* rmsnorm(Args a) {      // x, weight, eps, residual, want_residual -> (
   if (!fits(x->size(0)) || !fits(x->size(1))) return none();
   Tensor out = make(*x, x->sizes(), x->scalar_type()), sum;
   if (res && want) sum = make(*x, x->sizes(), x->scalar_type());
-  if (ts_rmsnorm(ptr(&out), sum.defined() ? ptr(&sum) : nullptr, ptr(x), ptr(res), ptr(w), nullptr, x->size(0), x->size(1), eps, code(*x), code(*w), stream()))
+  if (TS_REFUSED("rmsnorm",
+                 ts_rmsnorm(ptr(&out), sum.defined() ? ptr(&sum) : nullptr, ptr(x), ptr(res), ptr(w), nullptr, x->size(0), x->size(1), eps, code(*x), code(*w),
+                            stream())))
     return none();
   PyObject* second = !want ? none() : wrap(res ? sum : *x);
   return Py_BuildValue("(NN)", wrap(out), second);
@@ -157,7 +175,9 @@ PyObject* stream_post_norm(Args a) {      // x, a, post weight, scale, post eps,
   for (const Tensor* v : {post, scale, w})
     if (v && !vector(*v, at::kFloat, width)) return none();
   Tensor out = make(*x, {n, width}, out_code ? at::kBFloat16 : at::kFloat);
-  if (ts_stream_post_norm(typed<float>(x), typed<float>(b), typed<float>(post), typed<float>(scale), post_eps, ptr(&out), out_code, typed<float>(w), eps, n, width, stream()))
+  if (TS_REFUSED("stream_post_norm",
+                 ts_stream_post_norm(typed<float>(x), typed<float>(b), typed<float>(post), typed<float>(scale), post_eps, ptr(&out), out_code, typed<float>(w),
+                                     eps, n, width, stream())))
     return none();
   return wrap(out);
 }
@@ -174,8 +194,9 @@ PyObject* stream_update_norm(Args a) {      // x, a, b, mult, weight, eps, out c
     if (t && !(matrix(*t, n, width) && t->is_contiguous() && code(*t) >= 0)) return none();
   if (code(*w) < 0 || !vector(*w, w->scalar_type(), width) || !fits(n) || !fits(width)) return none();
   Tensor out = make(*x, {n, width}, out_code ? at::kBFloat16 : at::kFloat);
-  if (ts_stream_update_norm(typed<float>(x), ptr(b1), b1 ? code(*b1) : 0, ptr(b2), b2 ? code(*b2) : 0, nullptr, 0, mult, ptr(&out), nullptr,
-                            out_code, ptr(w), nullptr, code(*w), eps, nullptr, n, width, stream()))
+  if (TS_REFUSED("stream_update_norm",
+                 ts_stream_update_norm(typed<float>(x), ptr(b1), b1 ? code(*b1) : 0, ptr(b2), b2 ? code(*b2) : 0, nullptr, 0, mult, ptr(&out), nullptr,
+                                       out_code, ptr(w), nullptr, code(*w), eps, nullptr, n, width, stream())))
     return none();
   return wrap(out);
 }
@@ -189,7 +210,9 @@ PyObject* gemm_library(Args a) {      // x, weight, 32-bit out -> y
   const int64_t M = x->size(0), K = x->size(1), N = w->size(0);
   if (!M || !N || !fits(M) || !fits(N) || !fits(K)) return none();
   Tensor y = make(*x, {M, N}, wide ? at::kFloat : at::kBFloat16);
-  if (ts_gemm_library_bf16(ptr(&y), ptr(x), ptr(w), M, N, K, x->stride(0), w->stride(0), N, wide, 0, nullptr, 0, stream())) return none();
+  if (TS_REFUSED("gemm_library",
+                 ts_gemm_library_bf16(ptr(&y), ptr(x), ptr(w), M, N, K, x->stride(0), w->stride(0), N, wide, 0, nullptr, 0, stream())))
+    return none();
   return wrap(y);
 }
 
@@ -207,8 +230,9 @@ PyObject* gemm_slices(Args a) {      // x, weight, tile, slices, 32-bit out, res
   if (N % 8 || K % 64) return none();
   Tensor parts = make(*x, {slices, M, N}, at::kFloat), y = make(*x, {M, N}, wide ? at::kFloat : at::kBFloat16), sum;
   if (nw) sum = make(*x, {M, N}, at::kBFloat16);
-  if (ts_gemm_slices_bf16(ptr(&y), nw ? ptr(&sum) : nullptr, ptr(&parts), ptr(x), ptr(w), M, N, K, x->stride(0), w->stride(0), tile, slices, wide, ptr(res), ptr(nw),
-                          eps, stream()))
+  if (TS_REFUSED("gemm_slices",
+                 ts_gemm_slices_bf16(ptr(&y), nw ? ptr(&sum) : nullptr, ptr(&parts), ptr(x), ptr(w), M, N, K, x->stride(0), w->stride(0), tile, slices, wide,
+                                     ptr(res), ptr(nw), eps, stream())))
     return none();
   return nw ? Py_BuildValue("(NN)", wrap(y), wrap(sum)) : wrap(y);
 }
@@ -221,7 +245,9 @@ PyObject* gemm_glu(Args a) {      // x, weight, tile, form's number, limit, slop
   const int64_t M = x->size(0), K = x->size(1), F = w->size(0) / 2;
   if (!M || !F || !fits(M) || !fits(w->size(0)) || w->size(0) % 16 || K % 64 || x->stride(0) < K || w->stride(0) < K) return none();
   Tensor y = make(*x, {M, F}, at::kBFloat16);
-  if (ts_gemm_glu_bf16(ptr(&y), ptr(x), ptr(w), M, F, K, x->stride(0), w->stride(0), F, tile, form, limit, slope, shift, stream())) return none();
+  if (TS_REFUSED("gemm_glu",
+                 ts_gemm_glu_bf16(ptr(&y), ptr(x), ptr(w), M, F, K, x->stride(0), w->stride(0), F, tile, form, limit, slope, shift, stream())))
+    return none();
   return wrap(y);
 }
 
@@ -241,7 +267,9 @@ PyObject* gemm_rows64(Args a) {      // x, packed, 32-bit out, unit's number (0:
   if (M < 1 || M > ROWS64_MAX_ROWS || N % (unit ? 128 : 64) || K % 1024 || !squares_fit(sq, M) || !fits(N) || !fits(K)) return none();
   const int64_t skew = M >= GATED_SKEW_MIN_ROWS ? ROW_SKEW : 0;
   Tensor y = unit ? at::empty_strided({M, N / 2}, {N / 2 + skew, 1}, x->options()) : make(*x, {M, N}, wide ? at::kFloat : at::kBFloat16);
-  if (ts_gemm_rows64_bf16(ptr(&y), ptr(x), ptr(p), M, N, K, x->stride(0), y.stride(0), unit, wide, ptr(sq), sq ? sq->size(1) : 0, eps, limit, slope, shift, stream()))
+  if (TS_REFUSED("gemm_rows64",
+                 ts_gemm_rows64_bf16(ptr(&y), ptr(x), ptr(p), M, N, K, x->stride(0), y.stride(0), unit, wide, ptr(sq), sq ? sq->size(1) : 0, eps, limit, slope,
+                                     shift, stream())))
     return none();
   return wrap(y);
 }
@@ -258,13 +286,16 @@ PyObject* gemm_rows64_sliced(Args a) {      // x, packed, slices, residual, norm
   Tensor parts = make(*x, {slices, M, N}, at::kFloat);
   if (!nw) {
     Tensor y = make(*x, {M, N}, at::kBFloat16);
-    if (ts_gemm_rows64_sliced_bf16(ptr(&y), ptr(&parts), ptr(x), ptr(p), M, N, K, x->stride(0), slices, nullptr, nullptr, nullptr, nullptr, nullptr, 0, stream()))
+    if (TS_REFUSED("gemm_rows64_sliced",
+                   ts_gemm_rows64_sliced_bf16(ptr(&y), ptr(&parts), ptr(x), ptr(p), M, N, K, x->stride(0), slices, nullptr, nullptr, nullptr, nullptr, nullptr,
+                                              0, stream())))
       return none();
     return wrap(y);
   }
   Tensor sum = make(*x, {M, N}, at::kBFloat16), operand = at::empty_strided({M, N}, {N + ROW_SKEW, 1}, x->options()), squares = make(*x, {M, 1}, at::kFloat);
-  if (ts_gemm_rows64_sliced_bf16(nullptr, ptr(&parts), ptr(x), ptr(p), M, N, K, x->stride(0), slices, ptr(res), ptr(nw), ptr(&sum), ptr(&operand), ptr(&squares),
-                                 operand.stride(0), stream()))
+  if (TS_REFUSED("gemm_rows64_sliced",
+                 ts_gemm_rows64_sliced_bf16(nullptr, ptr(&parts), ptr(x), ptr(p), M, N, K, x->stride(0), slices, ptr(res), ptr(nw), ptr(&sum), ptr(&operand),
+                                            ptr(&squares), operand.stride(0), stream())))
     return none();
   return Py_BuildValue("(NNN)", wrap(sum), wrap(operand), wrap(squares));
 }
@@ -295,8 +326,10 @@ PyObject* rope_store(Args a) {      // qkv, table, positions, slots, k, v, heads
   if (table && !(f32(*table) && table->dim() == 2 && table->is_contiguous() && table->size(1) >= 2 && table->size(1) <= hd && table->size(1) % 2 == 0)) return none();
   if (!s.take(T, x->scalar_type(), nkv, hd, hd)) return none();
   Tensor q = make(*x, {T, nh, hd}, x->scalar_type());
-  if (ts_rope_store(ptr(&q), ptr(s.k), ptr(s.v), ptr(x), typed<float>(table), typed<int32_t>(pos), typed<int32_t>(s.slots), T, nh, nkv, hd,
-                    table ? table->size(1) : hd, table != nullptr, s.page, s.ks[0], s.ks[1], s.ks[2], s.vs[0], s.vs[1], s.vs[2], s.vs[3], code(*x), stream()))
+  if (TS_REFUSED("rope_store",
+                 ts_rope_store(ptr(&q), ptr(s.k), ptr(s.v), ptr(x), typed<float>(table), typed<int32_t>(pos), typed<int32_t>(s.slots), T, nh, nkv, hd, table ?
+                               table->size(1) : hd, table != nullptr, s.page, s.ks[0], s.ks[1], s.ks[2], s.vs[0], s.vs[1], s.vs[2], s.vs[3], code(*x),
+                               stream())))
     return none();
   return wrap(q);
 }
@@ -316,9 +349,10 @@ PyObject* qkv_rope_store_sliced(Args a) {      // x, packed, slices, table, posi
   if (table && !(f32(*table) && table->dim() == 2 && table->size(1) == hd && table->is_contiguous())) return none();
   if (!s.take(M, at::kBFloat16, nkv, hd, hd)) return none();
   Tensor parts = make(*x, {slices, M, N}, at::kFloat), q = make(*x, {M, nh, hd}, at::kBFloat16);
-  if (ts_gemm_rows64_sliced_rope_bf16(ptr(&q), ptr(&parts), ptr(x), ptr(p), M, K, x->stride(0), slices, ptr(sq), sq ? sq->size(1) : 0, eps, typed<float>(table),
-                                      typed<int32_t>(pos), typed<int32_t>(s.slots), ptr(s.k), ptr(s.v), nh, nkv, hd, table != nullptr, s.page, s.ks[0], s.ks[1],
-                                      s.ks[2], s.vs[0], s.vs[1], s.vs[2], s.vs[3], stream()))
+  if (TS_REFUSED("qkv_rope_store_sliced",
+                 ts_gemm_rows64_sliced_rope_bf16(ptr(&q), ptr(&parts), ptr(x), ptr(p), M, K, x->stride(0), slices, ptr(sq), sq ? sq->size(1) : 0, eps,
+                                                 typed<float>(table), typed<int32_t>(pos), typed<int32_t>(s.slots), ptr(s.k), ptr(s.v), nh, nkv, hd, table !=
+                                                 nullptr, s.page, s.ks[0], s.ks[1], s.ks[2], s.vs[0], s.vs[1], s.vs[2], s.vs[3], stream())))
     return none();
   return wrap(q);
 }
@@ -341,9 +375,10 @@ PyObject* qkv_finish(Args a) {      // qkv, freqs, positions, slots, k, v, heads
   if (freqs && !(is(*freqs, at::kDouble) && freqs->dim() == 1 && freqs->is_contiguous() && 2 * freqs->size(0) <= hd)) return none();
   if (!s.take(T, out_type, nkv, hd, vd)) return none();
   Tensor q = make(*x, {T, nh, hd}, out_type);
-  if (ts_qkv_finish(ptr(&q), ptr(s.k), ptr(s.v), ptr(x), typed<double>(freqs), typed<int32_t>(pos), typed<int32_t>(s.slots), T, nh, nkv, hd, vd,
-                    freqs ? 2 * freqs->size(0) : 0, interleaved, normed[0], eps[0], normed[1], eps[1], s.page, s.ks[0], s.ks[1], s.ks[2], s.vs[0], s.vs[1], s.vs[2],
-                    s.vs[3], code(*x), out_code, amplitude, x->size(1), stream()))
+  if (TS_REFUSED("qkv_finish",
+                 ts_qkv_finish(ptr(&q), ptr(s.k), ptr(s.v), ptr(x), typed<double>(freqs), typed<int32_t>(pos), typed<int32_t>(s.slots), T, nh, nkv, hd, vd,
+                               freqs ? 2 * freqs->size(0) : 0, interleaved, normed[0], eps[0], normed[1], eps[1], s.page, s.ks[0], s.ks[1], s.ks[2], s.vs[0],
+                               s.vs[1], s.vs[2], s.vs[3], code(*x), out_code, amplitude, x->size(1), stream())))
     return none();
   return wrap(q);
 }
@@ -410,20 +445,29 @@ PyObject* attention_step(Args a) {
   const int32_t *tb = typed<int32_t>(tables), *sq = typed<int32_t>(seq), *ps = typed<int32_t>(pos), *tl = typed<int32_t>(tiles);
   const int64_t k0 = k->stride(0), k1 = k->stride(1), k2 = k->stride(2), v0 = v->stride(0), v2 = v->stride(2), v3 = v->stride(3);
   const float *sk = typed<float>(sinks), *sl = typed<float>(slopes), *gt = typed<float>(gate);
-  hipStream_t st = stream();
-  int rc = 0;
-  if (lead && general)
-    rc = ts_paged_attention_decode_general(ptr(&out), dpof, dpmf, ptr(q), ptr(k), ptr(v), tb, sq, ps, lead, nh, nkv, hd, page, k0, k1, k2, v0, v2, v3, blocks, dsplits,
-                                           dchunk, dwaves, scale, window, run, softcap, sink, sk, sl, gt, gstride, st);
-  else if (lead)
-    rc = ts_paged_attention_decode(ptr(&out), dpof, dpmf, ptr(q), ptr(k), ptr(v), tb, sq, ps, lead, nh, nkv, hd, page, k0, k1, k2, v0, v2, v3, blocks, dsplits, dchunk,
-                                   dwaves, scale, window, run, 1, st);
-  if (rc) return none();
-  rc = general ? ts_paged_attention_prefill_general(ptr(&out), ptr(q), ptr(k), ptr(v), tb, sq, ps, tl, tiles->size(0), tile_tokens, waves, nh, nkv, hd, page, k0, k1, k2,
-                                                    v0, v2, v3, blocks, scale, window, first, T, splits, chunk, pof, pmf, run, softcap, sink, sk, sl, gt, gstride, st)
-               : ts_paged_attention_prefill(ptr(&out), ptr(q), ptr(k), ptr(v), tb, sq, ps, tl, tiles->size(0), tile_tokens, waves, nh, nkv, hd, page, k0, k1, k2, v0, v2,
-                                            v3, blocks, scale, window, first, T, splits, chunk, pof, pmf, run, st);
-  return rc ? none() : wrap(out);
+  if (lead && general) {
+    if (TS_REFUSED("paged_attention_decode_general",
+                   ts_paged_attention_decode_general(ptr(&out), dpof, dpmf, ptr(q), ptr(k), ptr(v), tb, sq, ps, lead, nh, nkv, hd, page, k0, k1, k2, v0, v2, v3, blocks,
+                                                     dsplits, dchunk, dwaves, scale, window, run, softcap, sink, sk, sl, gt, gstride, stream())))
+      return none();
+  } else if (lead) {
+    if (TS_REFUSED("paged_attention_decode", ts_paged_attention_decode(ptr(&out), dpof, dpmf, ptr(q), ptr(k), ptr(v), tb, sq, ps, lead, nh, nkv, hd, page, k0, k1, k2, v0,
+                                                                       v2, v3, blocks, dsplits, dchunk, dwaves, scale, window, run, 1, stream())))
+      return none();
+  }
+  const bool behind = lead > 0;
+  if (general) {
+    if (TS_REFUSED("paged_attention_prefill_general",
+                   ts_paged_attention_prefill_general(ptr(&out), ptr(q), ptr(k), ptr(v), tb, sq, ps, tl, tiles->size(0), tile_tokens, waves, nh, nkv, hd, page, k0, k1,
+                                                      k2, v0, v2, v3, blocks, scale, window, first, T, splits, chunk, pof, pmf, run, softcap, sink, sk, sl, gt, gstride,
+                                                      stream()), behind))
+      return none();
+  } else if (TS_REFUSED("paged_attention_prefill",
+                        ts_paged_attention_prefill(ptr(&out), ptr(q), ptr(k), ptr(v), tb, sq, ps, tl, tiles->size(0), tile_tokens, waves, nh, nkv, hd, page, k0, k1, k2, v0,
+                                                   v2, v3, blocks, scale, window, first, T, splits, chunk, pof, pmf, run, stream()), behind)) {
+    return none();
+  }
+  return wrap(out);
 }
 
 // ---- units ----
@@ -435,7 +479,9 @@ PyObject* capped_glu(Args a) {      // gate|up, limit, slope, up_shift, out code
   if (!a.done() || out_code < 0 || out_code > 1 || code(*x) < 0 || x->dim() != 2 || x->size(1) % 2 || x->stride(1) != 1 || x->stride(0) < x->size(1)) return none();
   if (!fits(x->size(0)) || !fits(x->size(1))) return none();
   Tensor y = make(*x, {x->size(0), x->size(1) / 2}, out_code ? at::kBFloat16 : at::kFloat);
-  if (ts_capped_glu(ptr(&y), out_code, ptr(x), code(*x), x->stride(0), x->size(0), x->size(1) / 2, limit, slope, shift, act, stream())) return none();
+  if (TS_REFUSED("capped_glu",
+                 ts_capped_glu(ptr(&y), out_code, ptr(x), code(*x), x->stride(0), x->size(0), x->size(1) / 2, limit, slope, shift, act, stream())))
+    return none();
   return wrap(y);
 }
 
@@ -449,7 +495,9 @@ PyObject* mlstm_finish(Args a) {      // o, weight, gate, heads, value size, eps
   if (o->size(1) != width || !fits(T) || !fits(width) || (w && !vector(*w, at::kFloat, width) && !vector(*w, at::kFloat, vdim))) return none();
   if (!f32(*g) || !matrix(*g, T, width) || g->stride(1) != 1 || g->stride(0) < width) return none();
   Tensor y = make(*o, {T, width}, out_code ? at::kBFloat16 : at::kFloat);
-  if (ts_mlstm_finish(ptr(&y), out_code, typed<float>(o), typed<float>(w), typed<float>(g), g->stride(0), T, heads, vdim, eps, w && w->size(0) == width ? vdim : 0, silu, stream()))
+  if (TS_REFUSED("mlstm_finish",
+                 ts_mlstm_finish(ptr(&y), out_code, typed<float>(o), typed<float>(w), typed<float>(g), g->stride(0), T, heads, vdim, eps, w && w->size(0) ==
+                                 width ? vdim : 0, silu, stream())))
     return none();
   return wrap(y);
 }

@@ -4,6 +4,13 @@
 #include <stddef.h>
 #include <stdint.h>
 
+// Error codes returned by the extern "C" launchers (0 = launched).
+#define TS_OK 0
+#define TS_BAD_DTYPE 1
+#define TS_BAD_SHAPE 2
+#define TS_LAUNCH_FAILED 3
+#define TS_TOO_LARGE 4
+
 typedef struct ihipStream_t* hipStream_t;
 
 extern "C" {

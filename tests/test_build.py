@@ -33,3 +33,28 @@ def test_a_fallback_folder_must_be_the_users_own(tmp_path, monkeypatch):
 
 def test_the_source_folder_is_taken_as_it_is():
     assert build.candidate_dirs()[0] == build.HERE and build._usable(build.HERE, create=False)
+
+
+def test_a_library_of_another_torch_or_python_is_stale(tmp_path, monkeypatch):
+    """calls.cpp takes torch's tensors and Python's objects as their headers lay them out: a library built against others is not loaded."""
+    first, second = tmp_path / "torch", tmp_path / "other" / "torch"
+    for folder in (first, second):
+        folder.mkdir(parents=True)
+        (folder / "version.py").write_text("__version__ = '2.10.0'\ngit_version = 'a1'\n")
+    monkeypatch.setattr(build, "_torch_folder", lambda: str(first))
+    monkeypatch.setattr(build, "candidate_dirs", lambda: [str(tmp_path)])
+    monkeypatch.setattr(build, "_usable", lambda folder, create: True)
+    (tmp_path / build.LIB_NAME).write_bytes(b"")
+    (tmp_path / (build.LIB_NAME + ".hash")).write_text(build.source_hash())
+    assert build.find_current() == str(tmp_path / build.LIB_NAME)
+    (first / "version.py").write_text("__version__ = '2.10.0'\ngit_version = 'b2'\n")
+    assert build.find_current() is None
+    (first / "version.py").write_text("__version__ = '2.10.0'\ngit_version = 'a1'\n")
+    assert build.find_current() is not None
+    with monkeypatch.context() as m:
+        m.setattr(build, "_torch_folder", lambda: str(second))
+        assert build.find_current() is None
+    with monkeypatch.context() as m:
+        m.setattr(build.sysconfig, "get_config_var", lambda name: "cpython-399-x86_64-linux-gnu")
+        assert build.find_current() is None
+    assert build.find_current() is not None

@@ -5,8 +5,8 @@ launcher that takes raw device pointers and a stream, and Python calls them thro
 Python module inside the same library, calls those that a step of a prompt is made of itself, with
 operands and outputs taken as torch tensors. The library is written next
 to the sources; if that folder is read-only, to a per-user folder under the system's temporary
-directory (made with mode 0700, and used only if it is this user's own and closed to everyone else). A sidecar file records a hash of the sources and flags so that a stale library is
-rebuilt and a current one is loaded as it is.
+directory (made with mode 0700, and used only if it is this user's own and closed to everyone else). A sidecar file records a hash of the sources, the
+flags and the torch and Python they were compiled against, so that a stale library is rebuilt and a current one is loaded as it is.
 """
 
 from __future__ import annotations
@@ -64,9 +64,17 @@ def _compile_flags(src: str) -> list[str]:
     return HOST_FLAGS + [f"-I{headers}", f"-I{os.path.join(headers, 'torch', 'csrc', 'api', 'include')}", f"-I{sysconfig.get_paths()['include']}"]
 
 
+def _compiled_against() -> list[str]:
+    """What of torch and Python `calls.cpp` is compiled and linked against: the C interface's name (its version and build), torch's
+    folder and its version file, which holds its version and commit."""
+    folder = os.path.realpath(_torch_folder())
+    with open(os.path.join(folder, "version.py")) as f:
+        return [str(sysconfig.get_config_var("SOABI")), sys.version.split()[0], folder, f.read()]
+
+
 def source_hash() -> str:
     h = hashlib.sha256()
-    h.update(" ".join(FLAGS + HOST_FLAGS + LINK).encode())
+    h.update("\0".join(FLAGS + HOST_FLAGS + LINK + _compiled_against()).encode())
     for name in sorted(f for f in os.listdir(HERE) if f.endswith((".hip", ".h", ".cpp"))):
         h.update(name.encode())
         with open(os.path.join(HERE, name), "rb") as f:

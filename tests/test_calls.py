@@ -26,7 +26,9 @@ namespace c10::hip { struct NoStream { hipStream_t stream() const { return nullp
 #define getCurrentHIPStream no_stream
 static std::map<std::string, int> answers;
 static std::string called;
-static int answer(const char* name) { called += std::string(name) + " "; return answers[name]; }
+static int locked = 0;
+static int answer(const char* name) { locked += PyGILState_Check(); called += std::string(name) + " "; return answers[name]; }
+extern "C" int stub_locked() { const int n = locked; locked = 0; return n; }
 extern "C" void stub_answer(const char* name, int rc) { answers[name] = rc; }
 extern "C" const char* stub_called() { static std::string last; last = called; called.clear(); return last.c_str(); }
 """
@@ -34,7 +36,7 @@ extern "C" const char* stub_called() { static std::string last; last = called; c
 
 @pytest.fixture(scope="session")
 def stub(tmp_path_factory):
-    """(the module, answer(launcher, rc), called() -> the launchers called since it was last asked)."""
+    """(the module, answer(launcher, rc), called() -> the launchers called since it was last asked), none of them with Python's lock held."""
     folder = tmp_path_factory.mktemp("calls")
     with open(os.path.join(build.HERE, "calls.cpp")) as f:
         source = f.read()
@@ -52,7 +54,10 @@ def stub(tmp_path_factory):
     loader.exec_module(module)
     c = ctypes.CDLL(str(lib))
     c.stub_called.restype = ctypes.c_char_p
-    return module, lambda name, rc: c.stub_answer(name.encode(), rc), lambda: c.stub_called().decode().split()
+    def called():
+        assert c.stub_locked() == 0
+        return c.stub_called().decode().split()
+    return module, lambda name, rc: c.stub_answer(name.encode(), rc), called
 
 
 def ints(*values):

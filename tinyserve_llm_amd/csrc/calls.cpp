@@ -99,12 +99,30 @@ bool matrix(const Tensor& t, int64_t rows, int64_t columns) { return t.dim() == 
 // rows that lie apart in whole 16-byte pieces, dense and aligned
 bool pieces(const Tensor& x) { return x.dim() == 2 && x.stride(1) == 1 && x.stride(0) % 8 == 0 && aligned(x); }
 
-Tensor make(const Tensor& like, at::IntArrayRef sizes, at::ScalarType type) { return at::empty(sizes, like.options().dtype(type)); }
+// Python's lock, let go of: memory may have to be waited for, and so may a full queue, another thread's product or the timing of a
+// product's algorithms, while other threads have work in Python. (ctypes lets go of it for a launcher, torch for a new tensor.)
+struct Unlocked {
+  PyThreadState* state = PyEval_SaveThread();
+  ~Unlocked() { PyEval_RestoreThread(state); }
+};
+
+Tensor make(const Tensor& like, at::IntArrayRef sizes, at::ScalarType type) {
+  Unlocked unlocked;
+  return at::empty(sizes, like.options().dtype(type));
+}
+// rows of n numbers `skew` apart from each other
+Tensor make_rows(const Tensor& like, int64_t rows, int64_t n, int64_t skew) {
+  Unlocked unlocked;
+  return at::empty_strided({rows, n}, {n + skew, 1}, like.options());
+}
 
 // Whether a launcher has refused its operands, which it does before it launches anything. An error where it is more than that: a failed
 // launch (or an earlier one's failure, found only now), or a refusal `behind` a launch of this call.
 template <class F> bool refused(const char* name, const F& launch, bool behind = false) {
-  const int rc = launch();
+  const int rc = [&] {
+    Unlocked unlocked;
+    return launch();
+  }();
   if (rc == TS_OK) return false;
   if (rc != TS_LAUNCH_FAILED && !behind) return true;
   PyObject* hip = PyImport_ImportModule("tinyserve_llm_amd.ops.hip");
@@ -266,7 +284,7 @@ PyObject* gemm_rows64(Args a) {      // x, packed, 32-bit out, unit's number (0:
   const int64_t M = x->size(0), K = x->size(1), N = p->size(0) * 16;
   if (M < 1 || M > ROWS64_MAX_ROWS || N % (unit ? 128 : 64) || K % 1024 || !squares_fit(sq, M) || !fits(N) || !fits(K)) return none();
   const int64_t skew = M >= GATED_SKEW_MIN_ROWS ? ROW_SKEW : 0;
-  Tensor y = unit ? at::empty_strided({M, N / 2}, {N / 2 + skew, 1}, x->options()) : make(*x, {M, N}, wide ? at::kFloat : at::kBFloat16);
+  Tensor y = unit ? make_rows(*x, M, N / 2, skew) : make(*x, {M, N}, wide ? at::kFloat : at::kBFloat16);
   if (TS_REFUSED("gemm_rows64",
                  ts_gemm_rows64_bf16(ptr(&y), ptr(x), ptr(p), M, N, K, x->stride(0), y.stride(0), unit, wide, ptr(sq), sq ? sq->size(1) : 0, eps, limit, slope,
                                      shift, stream())))
@@ -292,7 +310,7 @@ PyObject* gemm_rows64_sliced(Args a) {      // x, packed, slices, residual, norm
       return none();
     return wrap(y);
   }
-  Tensor sum = make(*x, {M, N}, at::kBFloat16), operand = at::empty_strided({M, N}, {N + ROW_SKEW, 1}, x->options()), squares = make(*x, {M, 1}, at::kFloat);
+  Tensor sum = make(*x, {M, N}, at::kBFloat16), operand = make_rows(*x, M, N, ROW_SKEW), squares = make(*x, {M, 1}, at::kFloat);
   if (TS_REFUSED("gemm_rows64_sliced",
                  ts_gemm_rows64_sliced_bf16(nullptr, ptr(&parts), ptr(x), ptr(p), M, N, K, x->stride(0), slices, ptr(res), ptr(nw), ptr(&sum), ptr(&operand),
                                             ptr(&squares), operand.stride(0), stream())))

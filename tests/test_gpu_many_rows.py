@@ -296,3 +296,27 @@ def test_products_per_head_are_the_same_bits_whatever_the_tokens(tokens, x_type,
         want, size = want * turn, size * turn
     bound = size * (k * 2.0 ** -24 + (2.0 ** -21 if gated else 0.0)) + (want.abs() * 2.0 ** -8 if y_type == BF else 0.0)
     assert torch.all((out[picked].double().cpu() - want).abs() <= bound + 1e-30)
+
+
+def test_the_blocks_of_tokens_a_wave_takes_are_blocks_that_have_tokens():
+    """Sizes that were measured on both sides of the rule's lines (latent_mfma.hip): few tokens of many heads keep one block a wave."""
+    blocks = hip.library().ts_heads_gemm_blocks
+    for x_type in (0, 1):
+        assert [blocks(t, 128, 512, 128, x_type) for t in (1, 5, 48, 64)] == [1] * 4
+        assert [blocks(t, 32, 256, 64, x_type) for t in (8, 64, 129, 200, 304)] == [1, 1, 1, 2, 2]
+        assert blocks(1000, 24, 100, 40, x_type) == 1 and blocks(2048, 32, 256, 64, x_type) == 4
+        assert blocks(100, 128, 512, 128, x_type) == 4 and blocks(2048, 32, 64, 256, x_type) == (4 if x_type else 2)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("x_type, y_type", [(torch.float32, torch.float32), (BF, BF), (BF, torch.float32)])
+@pytest.mark.parametrize("tokens", [1, 17, 63, 64, 65])
+def test_products_per_head_of_few_tokens_are_stored_as_those_of_many(tokens, x_type, y_type):
+    """Results stored as they are (below 64 tokens, and 16-bit ones of one block) and turned: the same bits, nothing beside them."""
+    g = torch.Generator().manual_seed(tokens)
+    x = torch.randn(320, 64, 64, generator=g).to(x_type).cuda()
+    w = (torch.randn(64, 132, 64, generator=g) / 8).to(BF).cuda().transpose(1, 2)
+    whole, few = (torch.full((n + 1, 64, 136), 7.0, dtype=y_type, device="cuda") for n in (320, tokens))
+    hip.heads_gemm(x, w, whole[:320, :, :132])
+    hip.heads_gemm(x[:tokens], w, few[:tokens, :, :132])
+    assert torch.equal(few[:tokens], whole[:tokens]) and torch.all(few[tokens] == 7.0) and torch.all(few[:, :, 132:] == 7.0)

@@ -618,28 +618,35 @@ heads_gemm_mfma_kernel(TO* __restrict__ y, int64_t y_token, int64_t y_head, cons
       for (int rt = 0; rt < RT; ++rt) acc[rt][nb] = mfma32(a, b[rt], acc[rt][nb]);
     }
   }
-  // whole fours of columns go out in one store of a lane, 16 lanes side by side, which the wave turns through shared memory
+  // whole fours of columns go out in one store of a lane; 16 lanes' side by side, turned through shared memory by the wave, where
+  // that pays (below: 16 tokens, 32 heads of 64 by 256 3.9 us as they are and 4.0 turned, 200 tokens, 24 of 40 by 100 with bfloat16
+  // results 4.0 and 4.1, 32-bit ones 4.2 and 4.1)
   if (N % 4 == 0 && ((y_token | y_head) & 3) == 0 && ((uintptr_t)y & (4 * sizeof(TO) - 1)) == 0) {
+    auto put = [&](int t, int n, float4_t v) {
+      if (t >= num_tokens || n >= N) return;
+      if (gate) {
+        const float* gr = gate + (int64_t)t * gate_token + (int64_t)h * N + n;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[j] = v[j] / (1.0f + expf(-gr[j]));
+      }
+      TO* yrow = y + (int64_t)t * y_token + (int64_t)h * y_head + n;
+      if constexpr (sizeof(TO) == 4) *(float4_t*)yrow = v;
+      else *(uint2*)yrow = make_uint2(pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3]));
+    };
     __shared__ __attribute__((aligned(16))) float4_t turn[LM_WAVES][16][HM_COLS / 4 + 1];
+    const bool turned = RT > 1 || (sizeof(TO) == 4 && num_tokens >= HM_TOKENS);
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) {
+      if (!turned) {
+#pragma unroll
+        for (int nb = 0; nb < HM_COLS / 16; ++nb) put(t0 + 16 * rt + r, n0 + 16 * nb + 4 * g, acc[rt][nb]);
+        continue;
+      }
 #pragma unroll
       for (int nb = 0; nb < HM_COLS / 16; ++nb) turn[wave][r][4 * nb + g] = acc[rt][nb];
       __builtin_amdgcn_wave_barrier();
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int at = 4 * i + g, to = t0 + 16 * rt + at, n = n0 + 4 * r;
-        float4_t v = turn[wave][at][r];
-        if (to >= num_tokens || n >= N) continue;
-        if (gate) {
-          const float* gr = gate + (int64_t)to * gate_token + (int64_t)h * N + n;
-#pragma unroll
-          for (int j = 0; j < 4; ++j) v[j] = v[j] / (1.0f + expf(-gr[j]));
-        }
-        TO* yrow = y + (int64_t)to * y_token + (int64_t)h * y_head + n;
-        if constexpr (sizeof(TO) == 4) *(float4_t*)yrow = v;
-        else *(uint2*)yrow = make_uint2(pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3]));
-      }
+      for (int i = 0; i < 4; ++i) put(t0 + 16 * rt + 4 * i + g, n0 + 4 * r, turn[wave][4 * i + g][r]);
       __builtin_amdgcn_wave_barrier();
     }
     return;
@@ -662,6 +669,16 @@ heads_gemm_mfma_kernel(TO* __restrict__ y, int64_t y_token, int64_t y_head, cons
   }
 }
 
+// The blocks of 16 tokens that a wave takes: two from 512 workgroups of one on, four from 2,048 (of bfloat16 rows, whose loads are
+// half as many, from 1,024); one for reductions below 64, whose waves are over at once (40 by 100, 24 heads, 1,000 tokens 6.6 us, 7.2
+// and 8.6), and for tokens that one workgroup of one holds, most of whose waves would have none (128 heads of 128 by 512, bfloat16
+// rows, 5 tokens 10.4 us and in four blocks 12.7, 64 tokens 13.9 and 15.8, 100 tokens 24.1 and 17.2).
+extern "C" int ts_heads_gemm_blocks(int num_tokens, int heads, int N, int K, int x_dtype) {
+  const int64_t groups = (int64_t)((num_tokens + HM_TOKENS - 1) / HM_TOKENS) * heads * ((N + HM_COLS - 1) / HM_COLS);
+  if (K < 64 || num_tokens <= HM_TOKENS || groups < 512) return 1;
+  return groups >= 2048 || (groups >= 1024 && x_dtype == 1) ? 4 : 2;
+}
+
 // w: bfloat16 [heads][N][K] with K along memory (stride w_n between rows, a multiple of 8; K a multiple of 8);
 // x rows 16-byte aligned.
 extern "C" int ts_heads_gemm_mfma(void* y, int y_dtype, int64_t y_token, int64_t y_head, const void* x, int x_dtype,
@@ -672,10 +689,7 @@ extern "C" int ts_heads_gemm_mfma(void* y, int y_dtype, int64_t y_token, int64_t
   if (heads <= 0 || heads > 65535 || N <= 0 || K < 8 || K % 8 || w_n % 8 || w_head % 8 || ((uintptr_t)w & 15) ||
       ((uintptr_t)x & 15) || (x_token * x_size) % 16 || (x_head * x_size) % 16 || (N + HM_COLS - 1) / HM_COLS > 65535)
     return TS_BAD_SHAPE;
-  // blocks of 16 tokens a wave: two from 512 workgroups of one on, four from 2,048 (of bfloat16 rows, whose loads are half as many,
-  // from 1,024); reductions below 64, whose waves are over at once, keep one (40 by 100, 24 heads, 1,000 tokens 6.6 us, 7.2 and 8.6)
-  const int64_t groups = (int64_t)((num_tokens + HM_TOKENS - 1) / HM_TOKENS) * heads * ((N + HM_COLS - 1) / HM_COLS);
-  const int blocks = K < 64 || groups < 512 ? 1 : groups >= 2048 || (groups >= 1024 && x_dtype == 1) ? 4 : 2;
+  const int blocks = ts_heads_gemm_blocks(num_tokens, heads, N, K, x_dtype);
   const dim3 grid((num_tokens + blocks * HM_TOKENS - 1) / (blocks * HM_TOKENS), heads, (N + HM_COLS - 1) / HM_COLS);
 #define HM_GO(RT, TX, TO) \
   heads_gemm_mfma_kernel<RT, TX, TO><<<grid, LM_THREADS, 0, stream>>>((TO*)y, y_token, y_head, (const TX*)x, x_token, x_head, \

@@ -121,6 +121,7 @@ def _declare(lib: ctypes.CDLL) -> None:
         "ts_latent_finish": [p, p, i, p, i64, i, i, i, i, i, p, p, f, p, f, p, p, i, i64, i64, p, i64, i64, i, p],
         "ts_latent_mfma_takes": [i, i],
         "ts_heads_gemm_mfma": [p, i, i64, i64, p, i, i64, i64, p, i64, i64, i, i, i, i, p, i64, p],
+        "ts_heads_gemm_blocks": [i, i, i, i, i],
         "ts_paged_attention_latent_mfma": [p, i, p, p, p, p, p, p, p, i, i, i, i, i, i, i, i64, i64, i64, i64, i64, i, f, i, i, i, p, p,
                                            p, p, i64, p],
         "ts_latent_tiles_takes": [i, i],

@@ -4,6 +4,8 @@ prompts' attention; walks over chunks of the state-space recurrence; products pe
 
 from __future__ import annotations
 
+import types
+
 import pytest
 import torch
 
@@ -222,6 +224,23 @@ def test_heads_of_128_take_eight_waves_where_these_fill_the_chip_and_the_general
     assert shape(1501, 20, 4, 8, 3, 128, 500.0, False) == (40, 8) and shape(1024, 20, 4, 8, 3, 128, 512.0, False) == (20, 4)
     assert shape(1501, 20, 4, 8, 3, 128, 2000.0, False) == (20, 4) and shape(1501, 20, 4, 8, 3, 128, 500.0, True) == (20, 4)
     assert shape(2048, 32, 8, 8, 4, 64, 1024.0, True) == (16, 4) and shape(2048, 32, 8, 8, 4, 64, 1024.0, False) == (32, 8)
+
+
+def test_wide_tiles_of_eight_waves_are_for_long_walks_and_whole_tiles_and_are_not_cut():
+    """Steps that were measured (24 heads of 128 over 8, and 16 over 2): a short window, requests whose ends leave the wide tiles
+    open, and a context long enough that so few workgroups would have their keys cut in chunks."""
+    def plan(nh, nkv, lens, window=0):
+        cu = [0]
+        for n in lens:
+            cu.append(cu[-1] + n)
+        ctx = types.SimpleNamespace(scratch={}, host_cu_seqlens=cu, host_starts=[0] * len(lens), host_context_lens=lens)
+        lead, tile_tokens, waves, _, splits, _ = hip._prefill_plan(torch.empty(cu[-1], nh, 128, dtype=BF), torch.empty(1, 32, nkv, 128, dtype=BF), ctx, True, False, window)
+        assert lead == 0
+        return tile_tokens, waves, splits
+    assert plan(24, 8, [600, 901]) == plan(24, 8, [1500], 1024) == (40, 8, 1)
+    assert plan(24, 8, [1500], 128) == plan(24, 8, [1500], 512) == plan(24, 8, [1500], -2048) == (20, 4, 1)
+    assert plan(24, 8, [100] * 16) == (20, 4, 1) and plan(16, 16, [300] * 8) == (64, 4, 1)
+    assert plan(16, 2, [3000]) == (16, 8, 1) and plan(16, 2, [2000]) == (8, 4, 1)
 
 
 def test_chunks_are_walked_where_their_states_are_many():

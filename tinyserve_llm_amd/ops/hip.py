@@ -785,30 +785,42 @@ def paged_attention_prefill(q: torch.Tensor, k_cache: torch.Tensor, v_cache: tor
     return out
 
 
-PREFILL_EIGHT_WAVES_WIDE_WORKGROUPS = 288      # heads of 128 take eight waves from this many workgroups of theirs on
+PREFILL_EIGHT_WAVES_WIDE_WORKGROUPS = 288      # heads of 128 take eight waves from this many workgroups of theirs on,
+PREFILL_EIGHT_WAVES_WIDE_WINDOW = 1024         # without a window or with one of at least this many keys,
+PREFILL_EIGHT_WAVES_WIDE_FILL = 0.9            # and where this much of their tiles' places has tokens
 
 
-def prefill_shape(tokens: int, tile_tokens: int, waves: int, nkv: int, group: int, head_dim: int, mean_keys: float, general: bool) -> tuple[int, int]:
+def prefill_shape(tokens: int, tile_tokens: int, waves: int, nkv: int, group: int, head_dim: int, mean_keys: float, general: bool,
+                  long_walk: bool = True, wide_tiles: int = 0) -> tuple[int, int]:
     """(tokens per tile, waves) of the prefill kernel from what `prefill_tile_tokens` and `prefill_waves` make of the step. Heads
     of 64 in the general variant keep tiles of one row tile a wave where eight waves would take two (their softmax, twice as
-    long, is what bounds them: 2,048 tokens 48.8 µs against 56.3, 819 and 1,229 together 31.2 against 36.8); heads of 128 take eight waves over
-    a short walk as soon as these fill the chip (1,501 tokens in two requests 24.6 µs against 27.0, 1,500 in one 34.9 against 38.1,
-    but 1,024 26.2 against 23.7)."""
+    long, is what bounds them: 2,048 tokens 48.8 µs against 56.3, 819 and 1,229 together 31.2 against 36.8). Heads of 128 take eight waves
+    over a short walk as soon as these fill the chip. Measured over groups of 1 to 16 heads, four waves and eight: from 264 to 284 workgroups
+    of eight waves (24 heads over 8: 1,300 tokens 30.1 µs and 31.3, 1,400 34.1 and 33.4; 16 over 2: 2,000 tokens 37.8 and 43.9, 2,300 50.0 and 49.4)
+    the two cross, at 304 eight take 0.88 to 0.92 of the time, at 376 0.80. Not over a window of 512 keys or fewer (`long_walk`: 128 keys, 24 over 8,
+    1,500 tokens 19.1 and 22.8; 512 keys 26.5 and 26.5, behind 700 more 35.3 and 39.8; 1,024 keys 33.9 and 29.2), and not where the wide
+    tiles (`wide_tiles` of them, if not as many as the tokens make in one piece) are left open by the requests' ends (16 requests of 100
+    tokens in tiles of 40 14.0 and 15.6)."""
     one = PREFILL_WAVES * (16 // group)
     if general and head_dim == 64 and waves == 2 * PREFILL_WAVES:
         return one, PREFILL_WAVES
-    if (head_dim == 128 and not general and tile_tokens == one and waves == PREFILL_WAVES and 0.0 < mean_keys < PREFILL_EIGHT_WAVES_MEAN_KEYS
-            and -(-tokens // (2 * one)) * nkv >= PREFILL_EIGHT_WAVES_WIDE_WORKGROUPS):
+    if (head_dim == 128 and not general and long_walk and tile_tokens == one and waves == PREFILL_WAVES and 0.0 < mean_keys < PREFILL_EIGHT_WAVES_MEAN_KEYS
+            and -(-tokens // (2 * one)) * nkv >= PREFILL_EIGHT_WAVES_WIDE_WORKGROUPS and tokens >= PREFILL_EIGHT_WAVES_WIDE_FILL * wide_tiles * 2 * one):
         return 2 * one, 2 * PREFILL_WAVES
     return tile_tokens, waves
 
 
-def _prefill_plan(q: torch.Tensor, k_cache: torch.Tensor, ctx, decode_ok: bool, general: bool = False) -> tuple:
+def _long_walk(window: int) -> bool:
+    """Whether a window (0: none; below 0: chunks) leaves the walks of a prompt long, as `prefill_shape` counts them."""
+    return window == 0 or window >= PREFILL_EIGHT_WAVES_WIDE_WINDOW
+
+
+def _prefill_plan(q: torch.Tensor, k_cache: torch.Tensor, ctx, decode_ok: bool, general: bool = False, window: int = 0) -> tuple:
     """How a step's rows are dealt to the matrix-core kernels, from its lengths and the heads' sizes: (leading one-token
     requests, which go to the split-key kernel; tokens per tile; waves; tiles; chunks; keys per chunk). Every layer of one kind
     asks for the same plan, so a step makes it once."""
     (rows, nh, hd), nkv = q.shape, k_cache.shape[2]
-    key = ("attention_plan", rows, nh, nkv, hd, decode_ok, general)
+    key = ("attention_plan", rows, nh, nkv, hd, decode_ok, general, _long_walk(window))
     plan = ctx.scratch.get(key)
     if plan is not None:
         return plan
@@ -820,13 +832,17 @@ def _prefill_plan(q: torch.Tensor, k_cache: torch.Tensor, ctx, decode_ok: bool, 
     mean_keys = walked / max(1, rows - lead)
     tile_tokens = prefill_tile_tokens(rows - lead, nkv, nh // nkv, hd, mean_keys)
     waves = prefill_waves(tile_tokens, nh // nkv, hd, mean_keys)
-    tile_tokens, waves = prefill_shape(rows - lead, tile_tokens, waves, nkv, nh // nkv, hd, mean_keys, general)
+    narrow, wide = (tile_tokens, waves), 2 * tile_tokens
+    tile_tokens, waves = prefill_shape(rows - lead, *narrow, nkv, nh // nkv, hd, mean_keys, general, _long_walk(window),
+                                       sum(-(-(b - a) // wide) for a, b in zip(cu[lead:], cu[lead + 1:])))
     tiles = ctx.scratch.get(("attention_tiles", tile_tokens, lead))
     if tiles is None:
         flat = attention_tiles(cu, starts, tile_tokens, lead)
         tiles = torch.tensor(flat, dtype=torch.int32).view(-1, 2).to(q.device, non_blocking=True)
         ctx.scratch[("attention_tiles", tile_tokens, lead)] = tiles
-    splits, chunk = prefill_splits(tiles.shape[0] * nkv, max(ctx.host_context_lens[lead:], default=0))
+    # (tiles made wider for eight waves are not cut: there were enough of the narrow ones)
+    longest = max(ctx.host_context_lens[lead:], default=0)
+    splits, chunk = prefill_splits(tiles.shape[0] * nkv, longest) if tile_tokens <= narrow[0] else (1, 0)
     plan = ctx.scratch[key] = (lead, tile_tokens, waves, tiles, splits, chunk)
     return plan
 
@@ -853,7 +869,7 @@ def paged_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
         window = -chunk_mask
     tables = ctx.block_tables[space]
     general = softcap > 0 or sink or sinks is not None or slopes is not None or gate is not None
-    key = ("attention_step", q.shape, k_cache.shape, tables.shape, general)
+    key = ("attention_step", q.shape, k_cache.shape, tables.shape, general, _long_walk(window))
     step = ctx.scratch.get(key)
 
     def planned(step) -> torch.Tensor | None:
@@ -875,7 +891,7 @@ def paged_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
         if ctx.max_query_len == 1 and decode_ok:
             return paged_attention_decode(q, k_cache, v_cache, tables, ctx.seq_of_token, ctx.positions, scale, window,
                                           pages_per_entry=per_entry, leave_split=leave_split and gate is None, gate=gate, **extra)
-        lead, tile_tokens, waves, tiles, splits, chunk = _prefill_plan(q, k_cache, ctx, decode_ok, general)
+        lead, tile_tokens, waves, tiles, splits, chunk = _prefill_plan(q, k_cache, ctx, decode_ok, general, window)
         nkv = k_cache.shape[2]
         split_walk = decode_plan(lead, nkv, q.shape[1] // nkv, q.shape[2], capacity) if lead else (0, 0)
         ctx.scratch[key] = (tiles, (per_entry, lead, *split_walk, tile_tokens, waves, splits, chunk, ctx.host_cu_seqlens[lead]))

@@ -243,6 +243,16 @@ def test_wide_tiles_of_eight_waves_are_for_long_walks_and_whole_tiles_and_are_no
     assert plan(16, 2, [3000]) == (16, 8, 1) and plan(16, 2, [2000]) == (8, 4, 1)
 
 
+def test_requests_of_few_chunks_are_walked_only_where_the_chip_holds_them_at_once():
+    """Sizes measured on both sides: 16 requests of a chunk each, of five, one and two requests; states of 32 places."""
+    def walks(heads, vp, np, lens):
+        chunks = [-(-n // 64) for n in lens]
+        return hip.ssd_walks(sum(chunks), max(chunks), type("Z", (), dict(np=np, matrix=heads * vp * np)), len(lens))
+    assert not walks(64, 64, 128, [64] * 16) and not walks(32, 128, 32, [64] * 16) and not walks(32, 128, 32, [128] * 8) and not walks(16, 64, 32, [30] * 24)
+    assert walks(64, 64, 128, [300] * 16) and walks(64, 64, 128, [64]) and walks(64, 64, 128, [64] * 2) and walks(16, 64, 32, [64] * 8)
+    assert not walks(32, 128, 32, [300] * 16) and walks(32, 128, 32, [304]) and walks(4, 64, 128, [300] * 16) and not walks(4, 64, 128, [2048])
+
+
 def test_chunks_are_walked_where_their_states_are_many():
     def z(heads, vp, np):
         return type("Z", (), dict(np=np, matrix=heads * vp * np))

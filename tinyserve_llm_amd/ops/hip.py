@@ -3219,21 +3219,38 @@ def _step_chunks(ctx, from_tokens: int, device) -> "tuple[torch.Tensor, torch.Te
     return kept
 
 
+def _requests_in_chunks(ctx, from_tokens: int) -> int:
+    key = ("requests_in_chunks", from_tokens)
+    if key not in ctx.scratch:
+        ctx.scratch[key] = sum(b - a >= from_tokens for a, b in zip(ctx.host_cu_seqlens, ctx.host_cu_seqlens[1:]))
+    return ctx.scratch[key]
+
+
 def _all_in_chunks(ctx, from_tokens: int) -> bool:
-    return all(b - a >= from_tokens for a, b in zip(ctx.host_cu_seqlens, ctx.host_cu_seqlens[1:]))
+    return _requests_in_chunks(ctx, from_tokens) == ctx.num_seqs
 
 
 SSD_TABLE = 132             # floats of a chunk and head that the chunks' second sums leave for the walk
 SSD_WALK_MAX_PLACES = 128   # places of the state that the walk keeps in a workgroup
 
 
-def ssd_walks(chunks: int, longest: int, z: SsdSizes) -> bool:
-    """Whether a step's chunks are walked (their states stay in a workgroup) or worked all at once with the states between them
-    in memory. A walk takes 0.85 µs a chunk of the longest request (`longest` chunks of `chunks` in all); what it saves is fitted to
-    what both ways measured, 2.5 µs and 0.05 a chunk, 2.6 more for a million numbers of the state. Chunks and walk, µs: 64 heads of 64 x
-    128, 2,048 tokens 92.7 and 73.7; 16 of 128 x 128, 999 tokens in three requests 40.4 and 33.1, 2,048 in one 55.6 and 57.7; 4 of 64 x
-    128, 16 requests of 300 tokens 32.5 and 22.5, one of 2,048 26.3 and 43.5."""
-    return z.np <= SSD_WALK_MAX_PLACES and 0.85 * longest < 2.5 + chunks * (0.05 + 2.6e-6 * z.matrix)
+SSD_WALK_GROUPS = 512       # workgroups of the walk that the chip holds at once
+
+
+def ssd_walks(chunks: int, longest: int, z: SsdSizes, requests: int = 1) -> bool:
+    """Whether a step's chunks (of `requests` requests) are walked, their states kept in a workgroup, or worked all at once with the states
+    between them in memory. A walk is counted as 0.85 µs a chunk of the longest request (`longest` chunks of `chunks` in all; it is 0.9 to 1.3 by
+    itself, and takes work off the chunks' kernels), what it saves as 2.5 µs and 0.05 a chunk, 2.6 more for a million numbers of the state:
+    weights fitted to what both ways measured. A workgroup's start, its state and first chunks fetched, is worth two chunks or so: where
+    requests have fewer than three, the walk is for what the chip holds at once, and for states of 32 places, which are hardly dearer in
+    memory, half of that at any length. Chunks and walk, µs: 64 heads of 64 x 128, 2,048 tokens 92.7 and 73.7, 16 requests of 64 62.3 and 74.8, of
+    300 249 and 159; 16 of 128 x 128, 999 tokens in three requests 40.4 and 33.1, 2,048 in one 55.6 and 57.7; 4 of 64 x 128, 16 requests of 300 tokens
+    32.5 and 22.5, one of 2,048 26.3 and 43.5; 32 of 128 x 32, one request of 304 18.1 and 16.4, 16 of 300 88.0 and 95.8, of 64 27.8 and 43.4. Over 1,173
+    points (1 to 64 requests of 24 to 4,096 tokens, 4 to 128 heads) what it takes is 0.80 of the chunks' time on average and at most 1.05."""
+    if z.np > SSD_WALK_MAX_PLACES or 0.85 * longest >= 2.5 + chunks * (0.05 + 2.6e-6 * z.matrix):
+        return False
+    groups = requests * z.matrix // (16 * z.np)
+    return groups <= SSD_WALK_GROUPS if chunks < 3 * requests else z.np > 32 or groups <= SSD_WALK_GROUPS // 2
 
 
 def ssd_scan(mixed: torch.Tensor, steps: torch.Tensor, logs: torch.Tensor, skip: torch.Tensor | None, state: torch.Tensor, ctx,
@@ -3263,7 +3280,7 @@ def ssd_scan(mixed: torch.Tensor, steps: torch.Tensor, logs: torch.Tensor, skip:
     if chunked:
         chunks, chunk_cu = _step_chunks(ctx, chunks_from, mixed.device)
         C = chunks.shape[0]
-        if ssd_walks(C, -(-ctx.max_query_len // SSD_CHUNK), z):
+        if ssd_walks(C, -(-ctx.max_query_len // SSD_CHUNK), z, _requests_in_chunks(ctx, chunks_from)):
             tables = torch.empty((C, z.heads, SSD_TABLE), dtype=torch.float32, device=mixed.device)
             _run("ssd_walk", library().ts_ssd_walk(
                 _ptr(out), _ptr(mixed), _ptr(steps), _ptr(logs), _ptr(skip), token_stride, _ptr(state), state.stride(0), _ptr(chunks), _ptr(chunk_cu),

@@ -121,13 +121,10 @@ def test_the_rule_keeps_to_what_was_measured():
 
 
 def test_the_rule_leaves_to_the_library_what_the_library_is_faster_at():
-    """Products that slices took 1.04 to 1.15 times the library's time for: they go to the library, or to a plan that takes 0.86 to 0.89 of
-    it; and some that take 0.72 to 0.93 of it."""
-    for rows, n, k, ending in ((1999, 4096, 4096, "norm"), (2048, 4096, 4096, "norm"), (450, 2048, 6144, "bf16"), (1514, 4096, 3072, "norm"),
-                               (320, 3072, 6144, "bf16"), (1501, 4096, 4096, "f32"), (2048, 4096, 5120, "bf16")):
+    """Products that slices took 1.04 to 1.15 times the library's time for, and some that they take 0.72 to 0.95 of it for."""
+    for rows, n, k, ending in ((513, 1536, 8192, "bf16"), (900, 1024, 8192, "bf16"), (850, 1024, 8192, "bf16"), (1999, 4096, 4096, "norm"), (2048, 4096, 4096, "norm"),
+                               (450, 2048, 6144, "bf16"), (1514, 4096, 3072, "norm"), (320, 3072, 6144, "bf16"), (1501, 4096, 4096, "f32"), (2048, 4096, 5120, "bf16")):
         assert hip.slices_plan(rows, n, k, ending) is None
-    for rows, n, k in ((513, 1536, 8192), (850, 1024, 8192), (900, 1024, 8192)):
-        assert hip.slices_plan(rows, n, k, "bf16") == (0, 4)
     for rows, n, k, ending in ((160, 2048, 8192, "bf16"), (512, 2048, 8192, "f32"), (1514, 3072, 8192, "norm"), (2048, 2048, 8192, "norm"), (300, 2048, 4096, "norm"),
                                (160, 2048, 4096, "norm")):
         assert hip.slices_plan(rows, n, k, ending) is not None

@@ -1651,18 +1651,18 @@ def gemm_glu(x: torch.Tensor, weight: torch.Tensor, form: str, limit: float = 0.
     return y
 
 
-# Tiles of `gemm_slices` (rows of x by rows of W); for each, with the plain ending and with the norm's: the µs that do not depend on the
-# sizes, those of a million numbers of the parts and of a million of W, of a step of 64 of K, and what a step takes longer on a full chip
-SLICES_TILES = ((128, 128, (5.9, 1.91, 0.124, 0.455, 0.0), (8.0, 2.09, 0.148, 0.461, 0.0)),
-                (128, 256, (10.8, 0.89, 0.117, 0.594, 0.080), (13.4, 0.98, 0.123, 0.587, 0.130)),
-                (192, 256, (14.1, 0.62, 0.055, 0.663, 0.302), (15.6, 1.00, 0.071, 0.690, 0.259)),
-                (256, 256, (14.6, 0.70, 0.0, 0.871, 0.448), (15.8, 1.15, 0.020, 0.889, 0.387)),
-                (64, 128, (3.7, 2.40, 0.267, 0.315, 0.0), (5.3, 2.66, 0.325, 0.312, 0.0)))
+# Tiles of `gemm_slices` (rows of x by rows of W); for each, with the plain ending and with the norm's: the µs that do not depend
+# on the sizes, those of a step of 64 of K, of a million numbers of the parts and of a million of W
+SLICES_TILES = ((128, 128, (8.0, 0.42, 1.28, 0.16), (10.8, 0.45, 1.23, 0.15)),
+                (128, 256, (10.8, 0.59, 0.80, 0.18), (13.0, 0.63, 1.00, 0.16)),
+                (192, 256, (12.7, 0.78, 0.75, 0.14), (14.0, 0.80, 1.19, 0.13)),
+                (256, 256, (11.8, 1.09, 0.89, 0.12), (12.5, 1.10, 1.42, 0.10)),
+                (64, 128, (4.2, 0.23, 2.36, 0.34), (7.0, 0.25, 1.84, 0.36)))
 # what the matrix library takes (with the norm: and the norm's kernel): fixed, a thousand of K, that times the root of the rows over 32,
 # and a million products (of a thousand each), numbers of W and of y
-SLICES_LIBRARY = {"bf16": (4.75, 0.45, 1.46, 1.27, 0.52, 0.13), "f32": (4.22, 0.30, 1.88, 1.12, 0.62, 0.52), "norm": (7.63, 0.34, 1.57, 1.15, 0.60, 1.78)}
-SLICES_GAIN = {2: 0.86}                            # the slices' share of the library's time, as estimated, up to which they are taken (others than
-SLICES_GAIN_OTHERS, SLICES_GAIN_US = 0.97, 1.0     # two slices), and the µs that they have to gain beyond
+SLICES_LIBRARY = {"bf16": (4.7, 0.33, 1.24, 1.16, 0.55, 0.10), "f32": (3.9, 0.29, 1.46, 1.07, 0.63, 0.57), "norm": (7.7, 0.25, 1.20, 1.15, 0.61, 1.58)}
+# the share of the library's time, both as estimated, up to which the slices are taken: two of them in each tile, and more
+SLICES_TWO_SHARE, SLICES_SHARE = (0.95, 0.92, 0.91, 0.80, 0.80), 0.94
 SLICES_MIN_ROWS, SLICES_MAX_ROWS = 129, 2048       # fewer rows: the kernels that share x; more: whole reductions fill the chip
 SLICES_MIN_WIDTH, SLICES_MAX_WIDTH = 1024, 4096    # columns (wider: whole reductions fill the chip as well)
 SLICES_MAX, SLICES_MIN_STEPS = 16, 3               # slices, and steps of 64 in each
@@ -1672,11 +1672,12 @@ SLICES_NORM_MAX_WIDTH = 8192                       # the norm's kernel keeps a r
 @functools.lru_cache(maxsize=4096)
 def slices_plan(rows: int, n: int, k: int, ending: str) -> tuple[int, int] | None:
     """The tile of `gemm_slices` and the slices for `rows` rows of x against a weight [n, k], all workgroups in one round; None where
-    the matrix library (and, with the ending "norm", the norm's kernel) may well be as fast. Both sides are estimates in µs, fitted to what every
-    plan and the library took at 1,944 points with weights from memory (129 to 2,048 rows, n 1,024 to 4,096, k 2,048 to 14,336; 4 to 8 % root mean
-    square), and what is left to gain is asked to be more than they err by: two slices gain the least and are misjudged the most. Over 4,536
-    points (28 numbers of rows, 6 of n, 9 of k, the three endings) the rule takes 2,123, at 0.78 of the other way's time on average; 9 of them are
-    slower by more than 2 % and none by more than 5 (2,048 rows, n 4,096, k 8,192 122.4 and 127.1; 140 rows, n 1,536, k 3,072 with the norm 13.1 and 13.6).
+    the matrix library (and, with the ending "norm", the norm's kernel) may well be as fast. Both sides are estimates in µs fitted to 143
+    measured points with weights from memory (129 to 2,048 rows, n 1,024 to 4,096, k 2,048 to 14,336; 5 to 8 % root mean square). They know
+    nothing of how full the chip is: two slices, whose chains are the longest, take up to a fifth more than estimated in tiles of 256 x 256 and 64 x
+    128 (513 rows, n 1,536, k 8,192 estimated 26.9, measured 35.0, the library 30.5), so these have to promise more. Over 4,536
+    points (28 numbers of rows, 6 of n, 9 of k, the three endings) the rule takes 1,912, at 0.77 of the other way's time on average; 4 of them are
+    slower by more than 2 %: 257 rows, n 3,072, k 8,192 31.5 and 34.8, 1,501 rows, n 4,096, k 4,096 with the norm 67.4 and 69.6, k 5,120 67.9 and 69.6.
     n 2,048, library and here: k 8,192 160 rows 26.6 and 19.2, 512 rows 34.1 and 29.9, 1,024 rows 53.4 and 44.7, with the norm 1,514
     rows 66.5 and 61.9; k 4,096 with the norm 300 rows 25.2 and 20.4, 2,048 rows 50.0 and 49.9; k 2,048 160 rows 9.6 and 11.3, with the norm
     12.8 and 13.4."""
@@ -1684,16 +1685,18 @@ def slices_plan(rows: int, n: int, k: int, ending: str) -> tuple[int, int] | Non
         return None
     steps, best = k // 64, None
     for tile, (bm, bn, *costs) in enumerate(SLICES_TILES):
-        fixed, part, weight, step, crowd = costs[ending == "norm"]
+        fixed, step, part, weight = costs[ending == "norm"]
         tiles = -(-rows // bm) * -(-n // bn)
         for slices in range(2, min(SLICES_MAX, steps // SLICES_MIN_STEPS, COMPUTE_UNITS // tiles) + 1):
-            us = fixed + (step + crowd * tiles * slices / COMPUTE_UNITS) * -(-steps // slices) + (part * slices * rows * n + weight * n * k) * 1e-6
-            us = us / SLICES_GAIN.get(slices, SLICES_GAIN_OTHERS) + SLICES_GAIN_US
+            us = fixed + step * -(-steps // slices) + (part * slices * rows * n + weight * n * k) * 1e-6
             if best is None or us < best[0]:
                 best = (us, tile, slices)
+    if best is None:
+        return None
+    us, tile, slices = best
     fixed, chain, rooted, work, weight, out = SLICES_LIBRARY[ending]
     library = fixed + (chain + rooted * math.sqrt(rows) / 32) * k / 1024 + (work * rows * n * k * 1e-3 + weight * n * k + out * rows * n) * 1e-6
-    return best[1:] if best is not None and best[0] < library else None
+    return (tile, slices) if us < (SLICES_TWO_SHARE[tile] if slices == 2 else SLICES_SHARE) * library else None
 
 
 def slices_takes(x: torch.Tensor, weight: torch.Tensor) -> bool:

@@ -4,10 +4,11 @@
 // up to 4 RT such tiles of consecutive tokens (RT per wave) and walks the request's keys from the
 // first position any of its rows may see to the last, 32 keys at a time. Each step's keys and
 // values are fetched from the pages once per workgroup, straight into LDS in the order the lanes use them, each wave
-// its share of the operand registers, and all waves read the whole step back from there. Heads of up to 64 have four steps in
-// LDS, three of them under way, larger ones three: through registers, a step ahead, every step waited for its loads
-// (measured before and after, µs, heads of 64: 90 tokens 7.2 and 6.2, 512 11.9 and 10.0, 2,048 38.8 and 33 to 36; 24 heads of
-// 128: 2,048 tokens 52.3 and 46.4). Beyond that the vector work of the softmax bounds it, next to LDS's reads. (Pages that are
+// its share of the operand registers, and all waves read the whole step back from there. Three steps are in LDS, two of them under
+// way: through registers, a step ahead, every step waited for its loads (measured before and after, µs, heads of 64: 90 tokens 7.3
+// and 6.4, 1,024 19.8 and 16.0, 2,048 36.1 and 32.3; 24 heads of 128: 2,048 tokens 52.5 and 45.7). With a fourth step for heads of 64
+// a unit holds a workgroup fewer, which short turns behind long contexts feel: 100 tokens behind 8,000 31.8 before, 32.6 with four and
+// 31.4 with three, 400 behind 16,000 125.7, 130.5 and 129.2. Beyond that the vector work of the softmax bounds it, next to LDS's reads. (Pages that are
 // no multiple of 32 keys, whose steps lie in several, still go through registers.) A row masks the keys beyond its own
 // position (and before its window); steps that lie wholly inside every row's range skip the masks.
 // Normally nothing is split and nothing is combined: a row's sums run over the keys in ascending
@@ -34,7 +35,7 @@
 #define PRE_PLACES 256
 template <int HD, bool WHOLE>
 struct PrefillLds {
-  static constexpr int STAGES = WHOLE ? (HD <= 64 ? 4 : 3) : 2;
+  static constexpr int STAGES = WHOLE ? 3 : 2;
   uint4 stage[STAGES][HD / 8][TS_WAVE];   // steps of operand registers, [register][lane]
   int range[4][PRE_MAX_WAVES];
   int64_t place[2][PRE_PLACES];      // [keys | values][step mod PRE_PLACES], in elements

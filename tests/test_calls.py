@@ -148,3 +148,12 @@ def test_a_stream_is_updated_by_one_launch(stub, monkeypatch):
         hip.stream_update_norm(torch.zeros(3, 64), bf(3, 64), weights=(bf(64), None), eps=1e-5, out_dtype=BF)
     assert called() == ["ts_stream_update_norm"]
     answer("ts_stream_update_norm", OK)
+
+
+def test_the_limits_are_those_of_the_general_functions():
+    """The numbers that calls.cpp holds for itself, by which it takes or leaves a call."""
+    with open(os.path.join(build.HERE, "calls.cpp")) as f:
+        held = dict(re.findall(r"\b([A-Z][A-Z0-9_]+) = (\d+)[,;]", f.read()))
+    assert {name: int(value) for name, value in held.items()} == {
+        "DECODE_MAX_TOKENS": hip.MAX_DECODE_TOKENS, "MAX_SPLITS": hip.MAX_DECODE_SPLITS, "ROWS64_MAX_ROWS": hip.ROWS64_MAX_ROWS, "ROWS64_SLICE_K": hip.ROWS64_SLICE_K,
+        "ROW_SKEW": hip.OPERAND_ROW_SKEW, "GATED_SKEW_MIN_ROWS": hip.GATED_SKEW_MIN_ROWS}

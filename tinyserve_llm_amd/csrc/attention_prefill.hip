@@ -340,7 +340,7 @@ attn_prefill_mfma_kernel(bf16_t* __restrict__ out, const bf16_t* __restrict__ q,
   // many groups of `heads_per_group`; a group's (tile, head) pairs go round its dies, long tiles first.
   // A die's workgroups go round its 32 compute units. Where two of them fit a unit, those of a short prompt run all at once, and
   // every other round takes its tiles in the opposite order, so that the unit with the longest walk of one round has the
-  // shortest of the next (heads of 64: 1,024 tokens 18.2 and now 16.2 µs, 2,048 33.8 and 32.9; of 128 with eight waves, one
+  // shortest of the next (heads of 64: 1,024 tokens 18.2 and now 16.0 µs, 2,048 33.8 and 32.3; of 128 with eight waves, one
   // workgroup a unit, 46.0 and 54.2: longest first there).
   constexpr bool PAIRS = PRE_WAVES == 4 ? RT * HD <= 256 : HD <= 64;
   const int die = blockIdx.x % 8, place = blockIdx.x / 8, round = place / 32;

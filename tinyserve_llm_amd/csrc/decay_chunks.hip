@@ -68,7 +68,8 @@ static __device__ __forceinline__ void dc_log_column(float (&l)[DC_BLOCK], float
 
 // VT: 16-column tiles of a wave (four waves side by side). A workgroup takes DP of the head's channels: with all 128 in one, two
 // requests of 2,048 tokens together were a workgroup a compute unit, whose loads and logarithms nothing hid (8 heads of
-// 128 x 256: 45.6 µs, and 37.7 in halves, each element's sums in the same order; heads of 64 x 64 are one workgroup as before).
+// 128 x 256: 45.6 µs, 37.7 in halves and 35.1 since these ask for both their columns at once, each element's sums in the same order; heads of
+// 64 x 64 are one workgroup as before).
 template <int D, int VT>
 __global__ void __launch_bounds__(DC_THREADS) decay_chunk_sums_kernel(const DecayChunks a) {
   constexpr int DP = D < 64 ? D : 64, PARTS = D / DP;

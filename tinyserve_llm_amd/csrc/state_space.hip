@@ -583,7 +583,7 @@ extern "C" int ts_ssd_chunks(float* out, const void* mixed, const float* steps, 
 // What bounds it then is the walk, 0.9 to 1.3 µs a chunk, most of it the loads' rows (C's 16 rows a load); with one set of waves for both
 // halves 1.5 to 1.8. Measured, chunks and walk, µs: 64 heads of 64 x 128, 304 tokens 33.0 and 22.7, 2,048 92.7 and 73.7, 16 requests
 // of 300 249 and 159; 16 heads of 128 x 128, three requests of 999 tokens 40.4 and 33.1, one of 2,048 55.6 and 57.7; 4 heads, 2,048
-// 26.3 and 43.5 (where the chunks stay). The same states, bit for bit; the outputs 6.5e-8 apart.
+// 26.3 and 43.5 (where the chunks stay, as they do for batches of short requests: hip.ssd_walks). The same states, bit for bit; the outputs 6.5e-8 apart.
 template <int NQ, bool FOURS>
 __global__ void __launch_bounds__(2 * SS_THREADS)
 ssd_walk_kernel(float* __restrict__ out, const float* __restrict__ tables, const bf16_t* __restrict__ mixed, float* __restrict__ states,

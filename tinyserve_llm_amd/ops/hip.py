@@ -1599,8 +1599,9 @@ def glu_takes(x: torch.Tensor, weight: torch.Tensor) -> bool:
             and 2 * n * weight.stride(0) < 1 << 31 and 512 * x.stride(0) < 1 << 31)
 
 
-# Tiles of `gemm_glu` (rows of x by rows of W) and the µs a round of one workgroup a compute unit counts for over a reduction of 2,048: what
-# the slowest measured (the fastest: 46, 38, 18 and 28), 192 x 256 a tenth more, so that it is not taken for a gain within what rounds differ by
+# Tiles of `gemm_glu` (rows of x by rows of W) and the µs a round of one workgroup a compute unit counts for over a reduction of 2,048: weights for
+# the choice, within what whole rounds measured (46 to 63, 38 to 49, 18 to 26 and 28 to 36), 192 x 256 the dearest within its range, so that it is
+# not taken for a gain within what rounds differ by
 GLU_TILES = ((256, 256, 60), (192, 256, 54), (128, 128, 23), (128, 256, 36))
 COMPUTE_UNITS = 256
 
@@ -1622,7 +1623,10 @@ def glu_pays(rows: int, n: int, k: int, branch_bytes: int = 2) -> bool:
     through memory. Both sides are estimated as they measured, in µs, with the weights coming from memory: here the plan's
     rounds; there 11 (10 for 32-bit branches, whose reading is counted apart) beside the longer of the weight's reading at
     6.5 TB/s and the full tiles' products at 1 / 1.15 of the rate here, and the branches' trip at 3 TB/s. Over 589 points (1 to 2,048 rows, n
-    1,024 to 28,672, k 512 to 8,192) what this takes is at most 1.05 times the slower route's time where it errs. Apart and
+    1,024 to 28,672, k 512 to 8,192) what this takes is at most 1.05 times the slower route's time where it errs; more often it errs by
+    leaving a gain, where a tile's height has just been passed (n 16,384, apart and here: k 2,048 129 to 161 rows 30 and 24, 257 to 316 36 and
+    33, 513 to 531 48 and 41, 1,025 to 1,175 88 and 79; k 3,072 129 to 212 39 and 35, 513 to 608 67 and 59, 1,025 to 1,298 123 and 114, but 257 to
+    378 46 and 49). Apart and
     here: F = n / 2 of 8,192, k 3,072: 17 rows 25 and 34, 160 rows 39 and 36, 320 rows 47 and 50, 2,048 rows 171 and 151; F 1,024, k 8,192: 16 rows 15
     and 64, 1,024 rows 54 and 70, 2,048 rows 78 and 77; F 1,536, k 576: 1 row 8.9 and 7.6, 1,024 rows 15.8 and 9.2."""
     full = 60 * rows * n / (256 * 256 * COMPUTE_UNITS) * k / 2048

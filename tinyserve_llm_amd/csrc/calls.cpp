@@ -246,10 +246,11 @@ PyObject* gemm_slices(Args a) {      // x, weight, tile, slices, 32-bit out, res
   if (nw && (wide || !vector(*nw, at::kBFloat16, N) || !aligned(*nw))) return none();
   if (res && !(bf16(*res) && matrix(*res, M, N) && res->is_contiguous() && aligned(*res))) return none();
   if (N % 8 || K % 64) return none();
-  Tensor parts = make(*x, {slices, M, N}, at::kFloat), y = make(*x, {M, N}, wide ? at::kFloat : at::kBFloat16), sum;
+  Tensor parts, y = make(*x, {M, N}, wide ? at::kFloat : at::kBFloat16), sum;
+  if (nw || slices > 1) parts = make(*x, {slices, M, N}, at::kFloat);
   if (nw) sum = make(*x, {M, N}, at::kBFloat16);
   if (TS_REFUSED("gemm_slices",
-                 ts_gemm_slices_bf16(ptr(&y), nw ? ptr(&sum) : nullptr, ptr(&parts), ptr(x), ptr(w), M, N, K, x->stride(0), w->stride(0), tile, slices, wide,
+                 ts_gemm_slices_bf16(ptr(&y), nw ? ptr(&sum) : nullptr, parts.defined() ? ptr(&parts) : nullptr, ptr(x), ptr(w), M, N, K, x->stride(0), w->stride(0), tile, slices, wide,
                                      ptr(res), ptr(nw), eps, stream())))
     return none();
   return nw ? Py_BuildValue("(NN)", wrap(y), wrap(sum)) : wrap(y);
@@ -352,7 +353,9 @@ PyObject* rope_store(Args a) {      // qkv, table, positions, slots, k, v, heads
   return wrap(q);
 }
 
-PyObject* qkv_rope_store_sliced(Args a) {      // x, packed, slices, table, positions, slots, k, v, heads, kv heads, head size, eps, squares -> q
+// x, packed, slices, table, positions, slots, k, v, heads, kv heads, head size, eps, squares -> q; or, for `qkv_rope_store_whole`, the weight as it is
+// in the packed one's place and the tile in the slices'
+PyObject* qkv_rope_store_sliced(Args a) {
   const Tensor *x = a.tensor(), *p = a.tensor();
   const int slices = a.i32();
   const Tensor *table = a.maybe(), *pos = a.tensor();
@@ -360,8 +363,22 @@ PyObject* qkv_rope_store_sliced(Args a) {      // x, packed, slices, table, posi
   const int nh = a.i32(), nkv = a.i32(), hd = a.i32();
   const float eps = a.number();
   const Tensor* sq = a.maybe();
-  if (!a.done() || x->dim() != 2 || !bf16(*x) || !pieces(*x) || !packed16(*p, x->size(1)) || !aligned(*p) || nh <= 0 || nkv < 0 || hd <= 0 || hd % 32) return none();
-  const int64_t M = x->size(0), K = x->size(1), N = p->size(0) * 16;
+  if (!a.done() || x->dim() != 2 || !bf16(*x) || !pieces(*x) || nh <= 0 || nkv < 0 || hd <= 0 || hd % 32) return none();
+  const int64_t M = x->size(0), K = x->size(1);
+  if (p->dim() == 2) {
+    const int64_t N = (nh + 2 * (int64_t)nkv) * hd;
+    if (!bf16(*p) || !pieces(*p) || !matrix(*p, N, K) || sq || !M || !fits(M) || !fits(N) || !fits(K) || x->stride(0) < K || p->stride(0) < K) return none();
+    if (!vector(*pos, at::kInt, M) || !s.take(M, at::kBFloat16, nkv, hd, hd)) return none();
+    if (table && !(f32(*table) && table->dim() == 2 && table->size(1) == hd && table->is_contiguous())) return none();
+    Tensor q = make(*x, {M, nh, hd}, at::kBFloat16);
+    if (TS_REFUSED("qkv_rope_store_whole",
+                   ts_gemm_whole_rope_bf16(ptr(&q), ptr(x), ptr(p), M, K, x->stride(0), p->stride(0), typed<float>(table), typed<int32_t>(pos), typed<int32_t>(s.slots),
+                                           ptr(s.k), ptr(s.v), nh, nkv, hd, s.page, s.ks[0], s.ks[1], s.ks[2], s.vs[0], s.vs[1], s.vs[2], s.vs[3], slices, stream())))
+      return none();
+    return wrap(q);
+  }
+  if (!packed16(*p, K) || !aligned(*p)) return none();
+  const int64_t N = p->size(0) * 16;
   if (N != (nh + 2 * (int64_t)nkv) * hd || M < 1 || M > ROWS64_MAX_ROWS || N % 64 || slices < 1 || slices > 64 || K % (ROWS64_SLICE_K * slices)) return none();
   if (!vector(*pos, at::kInt, M) || !squares_fit(sq, M) || !fits(N) || !fits(K)) return none();
   if (table && !(f32(*table) && table->dim() == 2 && table->size(1) == hd && table->is_contiguous())) return none();

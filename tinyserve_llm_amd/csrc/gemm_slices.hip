@@ -10,13 +10,9 @@
 // kernel: 160 rows 14.4 µs (26.8), 256 rows 16.3 (27.5), 512 rows 23.0 (34.0), 1,024 rows 34.5 (51.1), 2,048 rows 61.5
 // (75.1); K 2,048: 256 rows 7.6 (12.4), 512 rows 10.4 (13.2).
 //
-// Operands go from memory straight into LDS, 64 of K a step, as gemm_glu.hip lays them out (a row's eight 16-byte pieces
-// turned by (row / 2) % 8), and like there x has XN = 2 steps in LDS, W three, and a step one barrier, in its middle (three and five
-// steps of both: the same within a tenth, but with tiles of 64 x 128, whose steps are short: 300 rows, N 2,048, K 4,096 19.6 and 17.5 µs with the norm). A workgroup computes one tile and ends: the last two steps are written out
-// apart, so that no load is made that nothing reads. Tiles that share a slice of W run on one die.
-#include "lds_loads.h"
+// The tile itself is tile_product.h's. A workgroup computes one and ends. Tiles that share a slice of W run on one die.
+#include "tile_product.h"
 
-#define GS_MIN_STEPS 3          // steps of 64 that a slice has at least
 #define GS_THREADS 256
 #define GS_HELD 4               // 8-column pieces of a row that a thread of the norm's kernel keeps
 
@@ -29,112 +25,35 @@ struct SlicesArgs {
 
 template <int BM, int BN, int WM, int WN, int XN>
 __global__ __launch_bounds__(WM * WN * TS_WAVE, 2) void gemm_slices_kernel(const SlicesArgs a) {
-  constexpr int WAVES = WM * WN, TM = BM / WM / 16, TN = BN / WN / 16;
-  constexpr int NX = BM / 8 / WAVES, NW = BN / 8 / WAVES;      // kilobytes of a step that a wave fetches
-  constexpr int XS = BM * 128, WS = BN * 128;                  // bytes of a step of x and of W
-  static_assert(BM % (8 * WAVES) == 0 && BN % (8 * WAVES) == 0, "whole kilobytes a wave");
-  __shared__ __attribute__((aligned(1024))) unsigned char lds[XN * XS + 3 * WS];
-  const int lane = threadIdx.x % TS_WAVE, r = lane % 16, g = lane / 16;
-  const int wave = wave_index(), wm = wave % WM, wn = wave / WM;
+  using Tile = TileProduct<BM, BN, WM, WN, XN>;
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[Tile::LDS];
   // consecutive workgroups go to different dies: a die takes a run of tiles, those of one slice of W's rows side by side
   const int item = blockIdx.x % 8 * a.per_die + blockIdx.x / 8;
   if (item >= a.items) return;
   const int m0 = item % a.row_tiles * BM, c0 = item / a.row_tiles % a.col_tiles * BN, slice = item / (a.row_tiles * a.col_tiles);
   const int base = a.steps / a.slices, longer = a.steps % a.slices;      // (the first slices take a step more where they are uneven)
-  const int steps = base + (slice < longer ? 1 : 0);
   const int64_t k0 = 64 * ((int64_t)slice * base + min(slice, longer));
-  const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_ptr_t)lds;
-  uint32_t xoff[NX], woff[NW];
-  const __amdgpu_buffer_rsrc_t rsrc_x = load_base(a.x + (int64_t)m0 * a.ldx + k0), rsrc_w = load_base(a.w + (int64_t)c0 * a.ldw + k0);
+  uint32_t xoff[Tile::NX], woff[Tile::NW];
 #pragma unroll
-  for (int q = 0; q < NX; ++q) {
-    const int at = (wave * NX + q) * 8 + lane / 8;
-    xoff[q] = (uint32_t)(min(at, a.M - 1 - m0) * a.ldx * 2) + ((lane % 8) ^ ((at >> 1) & 7)) * 16;      // (rows past the end: the last one again)
+  for (int q = 0; q < Tile::NX; ++q) {
+    const int at = Tile::x_row(q);
+    xoff[q] = (uint32_t)(min(at, a.M - 1 - m0) * a.ldx * 2) + Tile::piece(at);      // (rows past the end: the last one again)
   }
 #pragma unroll
-  for (int q = 0; q < NW; ++q) {
-    const int at = (wave * NW + q) * 8 + lane / 8;
-    woff[q] = (uint32_t)(min(at, a.N - 1 - c0) * a.ldw * 2) + ((lane % 8) ^ ((at >> 1) & 7)) * 16;
+  for (int q = 0; q < Tile::NW; ++q) {
+    const int at = Tile::w_row(q);
+    woff[q] = (uint32_t)(min(at, a.N - 1 - c0) * a.ldw * 2) + Tile::piece(at);
   }
-  const uint32_t xfirst = lds0 + wave * NX * 1024, wfirst = lds0 + XN * XS + wave * NW * 1024;
-  auto fetch_x = [&](int step, uint32_t place) {
-#pragma unroll
-    for (int q = 0; q < NX; ++q) load_to_lds(rsrc_x, xfirst + place + q * 1024, xoff[q], (uint32_t)step * 128);
-  };
-  auto fetch_w = [&](int step, uint32_t place) {
-#pragma unroll
-    for (int q = 0; q < NW; ++q) load_to_lds(rsrc_w, wfirst + place + q * 1024, woff[q], (uint32_t)step * 128);
-  };
-  const uint32_t rd0 = (uint32_t)(r * 128 + (g ^ (r >> 1)) * 16), rd1 = rd0 ^ 64;      // a step's two halves of K
-  const unsigned char* rx = lds + wm * TM * 2048;
-  const unsigned char* rw = lds + XN * XS + wn * TN * 2048;
-  u32x4_t fw[2][TN], fx[2][TM];
-  float4_t acc[TN][TM];
-#pragma unroll
-  for (int j = 0; j < TN; ++j)
-#pragma unroll
-    for (int i = 0; i < TM; ++i) acc[j][i] = (float4_t){0.f, 0.f, 0.f, 0.f};
-  fetch_x(0, 0), fetch_w(0, 0), fetch_w(1, WS), fetch_x(1, XS);
-  if constexpr (XN == 3) fetch_x(2, 2 * XS);
-  wait_for<NW + NX * (XN - 1)>();
-  __builtin_amdgcn_s_barrier();
-  uint32_t xc = 0, wc = 0, wfree = 2 * WS;      // the places of the step that is multiplied, and of the next one of W to come
-#define TS_READ(S, RD)                                                                                         \
-  _Pragma("unroll") for (int j = 0; j < TN; ++j) fw[S][j] = *(const u32x4_t*)(rw + (RD + wc) + j * 2048);      \
-  _Pragma("unroll") for (int i = 0; i < TM; ++i) fx[S][i] = *(const u32x4_t*)(rx + (RD + xc) + i * 2048);
-#define TS_MULTIPLY(S)                                                                                         \
-  _Pragma("unroll") for (int i = 0; i < TM; ++i)                                                               \
-      _Pragma("unroll") for (int j = 0; j < TN; ++j) acc[j][i] = mfma32v(fw[S][j], fx[S][i], acc[j][i]);
-// the order of a half step: TM TN products, among their first two thirds the TM + TN operand reads, among all the loads
-#define TS_DEAL(LOADS)                                                                                         \
-  _Pragma("unroll") for (int q = 0; q < TM * TN; ++q) {                                                        \
-    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                                                         \
-    if ((q + 1) * (TM + TN) * 3 / 2 / (TM * TN) > q * (TM + TN) * 3 / 2 / (TM * TN)) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0); \
-    if ((q + 1) * (LOADS) / (TM * TN) > q * (LOADS) / (TM * TN)) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0); \
-  }                                                                                                            \
-  __builtin_amdgcn_sched_barrier(0);
-// A step that another follows, with (where W, X) the loads of W's step after the next one and of x's XN steps on. At its
-// barrier every wave has read the last of the step's x and of W (so their places may be filled), and the next step has
-// landed once at most LATER loads are under way: W's step after it and x's XN - 2 steps after it.
-#define TS_STEP(W, X, LATER)                                                                                   \
-  __builtin_amdgcn_sched_barrier(0);                                                                           \
-  if constexpr (W) fetch_w(s + 2, wfree);                                                                      \
-  TS_READ(1, rd1)                                                                                              \
-  TS_MULTIPLY(0)                                                                                               \
-  TS_DEAL(W ? NW : 0)                                                                                          \
-  const uint32_t xfree = xc;                                                                                   \
-  wfree = wc;                                                                                                  \
-  xc = xc == (XN - 1) * XS ? 0 : xc + XS;                                                                      \
-  wc = wc == 2 * WS ? 0 : wc + WS;                                                                             \
-  wait_for<LATER, 0>();                                                                                        \
-  __builtin_amdgcn_s_barrier();                                                                                \
-  __builtin_amdgcn_sched_barrier(0);                                                                           \
-  if constexpr (X) fetch_x(s + XN, xfree);                                                                     \
-  TS_READ(0, rd0)                                                                                              \
-  TS_MULTIPLY(1)                                                                                               \
-  TS_DEAL(X ? NX : 0)
-  TS_READ(0, rd0)
-  int s = 0;
-  for (; s < steps - XN; ++s) { TS_STEP(true, true, NW + NX * (XN - 2)) }
-  if constexpr (XN == 3) {
-    TS_STEP(true, false, NW + NX)
-    ++s;
-  }
-  { TS_STEP(false, false, 0) }
-  TS_READ(1, rd1)
-  TS_MULTIPLY(0)
-  TS_MULTIPLY(1)
-#undef TS_READ
-#undef TS_MULTIPLY
-#undef TS_DEAL
-#undef TS_STEP
+  float4_t acc[Tile::TN][Tile::TM];
+  Tile::run(lds, load_base(a.x + (int64_t)m0 * a.ldx + k0), load_base(a.w + (int64_t)c0 * a.ldw + k0), xoff, woff, base + (slice < longer ? 1 : 0), acc);
+  const int lane = threadIdx.x % TS_WAVE, r = lane % 16, g = lane / 16, wm = wave_index() % WM, wn = wave_index() / WM;
   float* y = a.parts + (int64_t)slice * a.M * a.N;
 #pragma unroll
-  for (int i = 0; i < TM; ++i) {
-    const int m = m0 + (wm * TM + i) * 16 + r;
+  for (int i = 0; i < Tile::TM; ++i) {
+    const int m = m0 + (wm * Tile::TM + i) * 16 + r;
 #pragma unroll
-    for (int j = 0; j < TN; ++j) {
-      const int c = c0 + (wn * TN + j) * 16 + 4 * g;
+    for (int j = 0; j < Tile::TN; ++j) {
+      const int c = c0 + (wn * Tile::TN + j) * 16 + 4 * g;
       if (m < a.M && c < a.N) *(float4_t*)(y + (int64_t)m * a.N + c) = acc[j][i];
     }
   }
@@ -233,11 +152,13 @@ static int launch_slices(SlicesArgs a, hipStream_t stream) {
 // x [M, K] and w [N, K] bfloat16, 16-byte aligned, rows ldx and ldw elements apart (multiples of 8); K a multiple of 64 with at
 // least 3 steps of 64 a slice, N a multiple of 8. parts: float32 [slices][M][N], scratch that the call fills and reads. tile (rows of x by
 // rows of W of a workgroup): 0 128 x 128, 1 128 x 256, 2 192 x 256, 3 256 x 256, 4 64 x 128. y [M, N] contiguous, 32-bit or bfloat16; or, with
-// norm_w [N]: y the norm of (the product in bfloat16 plus res [M, N], which may be null), sum [M, N] that sum; N at most 8,192.
+// norm_w [N]: y the norm of (the product in bfloat16 plus res [M, N], which may be null), sum [M, N] that sum; N at most 8,192. One slice without
+// a norm needs no parts (null): its workgroups store y themselves (gemm_whole.hip).
 extern "C" int ts_gemm_slices_bf16(void* y, void* sum, void* parts, const void* x, const void* w, int M, int N, int K, int64_t ldx, int64_t ldw,
                                    int tile, int slices, int out_f32, const void* res, const void* norm_w, float eps, hipStream_t stream) {
   if (M <= 0 || N <= 0) return TS_OK;
-  if (K <= 0 || K % 64 || N % 8 || ldx < K || ldw < K || ldx % 8 || ldw % 8 || tile < 0 || tile > 4 || slices < 1 || slices > 64 || K / 64 / slices < GS_MIN_STEPS) return TS_BAD_SHAPE;
+  if (K <= 0 || K % 64 || N % 8 || ldx < K || ldw < K || ldx % 8 || ldw % 8 || tile < 0 || tile > 4 || slices < 1 || slices > 64 || K / 64 / slices < TileProduct<64, 128, 1, 4, 3>::MIN_STEPS) return TS_BAD_SHAPE;
+  if (slices == 1 && !norm_w) return ts_gemm_whole_bf16(1, &y, &x, &w, &N, M, K, ldx, ldw, tile, out_f32, stream);
   if (!x || !w || !y || !parts || (((uintptr_t)x | (uintptr_t)w | (uintptr_t)y | (uintptr_t)parts) & 15)) return TS_BAD_SHAPE;
   if ((int64_t)M * N >= (1ll << 40) || 256 * ldx * 2 >= (1ll << 31) || 256 * ldw * 2 >= (1ll << 31)) return TS_TOO_LARGE;      // (byte offsets from a tile's start)
   if (norm_w && (out_f32 || !sum || N > 8 * GS_THREADS * GS_HELD || (((uintptr_t)sum | (uintptr_t)res | (uintptr_t)norm_w) & 15))) return TS_BAD_SHAPE;

@@ -91,6 +91,8 @@ def _declare(lib: ctypes.CDLL) -> None:
         "ts_gemm_skinny8_bf16": [p, p, p, i, i, i, i64, i64, i64, i, i, p, p, p, p, p, i, p, p, p, i, i, i, i, p],
         "ts_gemm_skinny8_act_bf16": [p, p, p, i, i, i, i64, i64, i64, i, i, p, i, p],
         "ts_gemm_slices_bf16": [p, p, p, p, p, i, i, i, i64, i64, i, i, i, p, p, f, p],
+        "ts_gemm_whole_bf16": [i, p, p, p, p, i, i, i64, i64, i, i, p],
+        "ts_gemm_whole_rope_bf16": [p, p, p, i, i, i64, i64, p, p, p, p, p, i, i, i, i, i64, i64, i64, i64, i64, i64, i64, i, p],
         "ts_gemm_rows64_bf16": [p, p, p, i, i, i, i64, i64, i, i, p, i, f, f, f, f, p],
         "ts_gemm_rows64_sliced_bf16": [p, p, p, p, i, i, i, i64, i, p, p, p, p, p, i64, p],
         "ts_gemm_rows64_sliced_rope_bf16": [p, p, p, p, i, i, i64, i, p, i, f, p, p, p, p, p, i, i, i, i, i, i64, i64, i64, i64, i64,
@@ -1715,7 +1717,7 @@ def slices_takes(x: torch.Tensor, weight: torch.Tensor) -> bool:
 def gemm_slices(x: torch.Tensor, weight: torch.Tensor, tile: int, slices: int, out_dtype: torch.dtype = torch.bfloat16,
                 next_norm: "tuple[torch.Tensor | None, torch.Tensor, float] | None" = None) -> "torch.Tensor | tuple[torch.Tensor, torch.Tensor]":
     """bfloat16 x [M, K] · weight [N, K]^T with the reduction cut into `slices`, whose 32-bit parts a second kernel adds up, the
-    first slice first (gemm_slices.hip); `tile` by its place in `SLICES_TILES`. With `next_norm` = (residual or None, weight,
+    first slice first (gemm_slices.hip), or whole in one slice (gemm_whole.hip); `tile` by its place in `SLICES_TILES`. With `next_norm` = (residual or None, weight,
     eps): (`rmsnorm` of the product in bfloat16 plus the residual, that sum)."""
     residual, nw, eps = next_norm if next_norm is not None else (None, None, 0.0)
     done = _native().gemm_slices(x, weight, tile, slices, out_dtype is torch.float32, residual, nw, eps) if out_dtype in (torch.float32, torch.bfloat16) else None
@@ -1740,11 +1742,128 @@ def gemm_slices(x: torch.Tensor, weight: torch.Tensor, tile: int, slices: int, o
     y = torch.empty((M, N), dtype=out_dtype, device=x.device)
     total = torch.empty((M, N), dtype=torch.bfloat16, device=x.device) if nw is not None else None
     if M and N:
-        parts = torch.empty((slices, M, N), dtype=torch.float32, device=x.device)
+        parts = torch.empty((slices, M, N), dtype=torch.float32, device=x.device) if nw is not None or slices > 1 else None
         _run("gemm_slices", library().ts_gemm_slices_bf16(
             _ptr(y), _ptr(total), _ptr(parts), _ptr(x), _ptr(weight), M, N, K, x.stride(0), weight.stride(0), tile, slices,
             int(out_dtype is torch.float32), _ptr(residual), _ptr(nw), float(eps), _stream()))
     return y if nw is None else (y, total)
+
+
+WHOLE_PRODUCTS = 8                                                             # products of one launch
+
+
+def gemm_whole(xs: "Sequence[torch.Tensor]", weights: "Sequence[torch.Tensor]", tile: int, out_dtype: torch.dtype = torch.bfloat16) -> "tuple[torch.Tensor, ...]":
+    """bfloat16 x [M, K] · weight [N, K]^T of up to 8 products of the same M, K and strides in one launch, each tile's reduction in one
+    workgroup (gemm_whole.hip); `tile` by its place in `SLICES_TILES`."""
+    _need(1 <= len(xs) == len(weights) <= WHOLE_PRODUCTS, lambda: f"{len(xs)} operands and {len(weights)} weights: one to {WHOLE_PRODUCTS} products")
+    _gpu(*xs, *weights)
+    _need(out_dtype in (torch.bfloat16, torch.float32), lambda: f"bfloat16 products come out as bfloat16 or float32, not {out_dtype}")
+    _need(0 <= tile < len(SLICES_TILES), lambda: f"tile {tile}: one of {len(SLICES_TILES)}")
+    for x, w in zip(xs, weights):
+        _need(x.dim() == 2 and w.dim() == 2 and x.shape == xs[0].shape and x.stride() == xs[0].stride() and w.shape[1] == x.shape[1]
+              and w.stride() == weights[0].stride(), lambda: f"shapes {tuple(x.shape)} x {tuple(w.shape)}^T beside {tuple(xs[0].shape)}")
+        _need(whole_takes(x, w), "products of whole tiles take bfloat16 operands with dense, 16-byte aligned rows, a reduction that is a "
+              f"multiple of 64 from {64 * WHOLE_MIN_STEPS} on and widths that are multiples of 8")
+    M, K = xs[0].shape
+    ys = tuple(torch.empty((M, w.shape[0]), dtype=out_dtype, device=w.device) for w in weights)
+    if M:
+        n = len(ys)
+        pointers = [(ctypes.c_void_p * n)(*(t.data_ptr() for t in ts)) for ts in (ys, xs, weights)]
+        _run("gemm_whole", library().ts_gemm_whole_bf16(n, *pointers, (ctypes.c_int * n)(*(w.shape[0] for w in weights)), M, K, xs[0].stride(0),
+                                                        weights[0].stride(0), tile, int(out_dtype is torch.float32), _stream()))
+    return ys
+
+
+WHOLE_MIN_STEPS = 3      # steps of 64 that a tile's reduction has at least
+
+
+def whole_takes(x: torch.Tensor, weight: torch.Tensor) -> bool:
+    """Whether `gemm_whole` takes these operands (whatever the rule by sizes says of them)."""
+    return slices_takes(x, weight) and x.shape[1] >= 64 * WHOLE_MIN_STEPS and weight.shape[0] >= 8
+
+
+# Tiles of `qkv_rope_store_whole` (rows of x by rows of W, workgroups that a compute unit holds of it); for each the µs that do not depend on the
+# sizes, those of a step of 64 of K for a workgroup a compute unit (and for two, where it holds two), of a million numbers of W and of a million of the product
+WHOLE_ROPE_TILES = ((128, 128, 2, (3.97, 0.474, 0.748, 0.12, 1.17)), (128, 256, 1, (4.40, 0.723, 0.0, 0.06, 0.92)),
+                    (192, 256, 1, (6.50, 0.906, 0.0, 0.0, 0.96)), (64, 128, 2, (3.15, 0.324, 0.537, 0.20, 0.84)))
+# what the product (by the matrix library or in slices) and the rotation's kernel take: fixed, a thousand of K, that times the root of the rows over 32,
+# and a million products (of a thousand each), numbers of W and of the product
+WHOLE_ROPE_APART = (9.89, 1.506, 0.309, 1.233, 0.323, 1.167)
+WHOLE_ROPE_SHARE, WHOLE_ROPE_SURE_SHARE = 0.97, 0.9      # the share of that, both as estimated, up to which one kernel is taken; the second one up to
+WHOLE_ROPE_FEW, WHOLE_ROPE_LARGE = 192, 1 << 24          # these rows and beyond these numbers of W, where the estimates err more
+WHOLE_ROPE_MIN_ROWS, WHOLE_ROPE_MAX_ROWS = 129, 3072      # fewer rows: the kernels that share x
+
+
+@functools.lru_cache(maxsize=4096)
+def qkv_rope_whole_plan(rows: int, n: int, k: int) -> int | None:
+    """The tile of `qkv_rope_store_whole` for `rows` rows of x against a q|k|v weight [n, k]; None where a product of its own and `rope_store` may
+    well be as fast. Both sides are estimates fitted to 224 measured points with weights from memory (129 to 6,000 rows, n 1,152 to 12,288, k 896 to
+    5,120; 5 to 10 % root mean square here, 7 % there). Of these the rule takes 152, at 0.80 of the other way's time on average; 4 of them are
+    slower by more than 2 %: n 5,120, k 3,072 513 rows 32.1 and 32.9 µs, 3,000 rows 96.0 and 101.3, n 7,168, k 5,120 2,300 rows 151.3 and 157.7, n 12,288, k 4,096 1,280
+    rows 116.6 and 119.2 (inside a pass, where the library's choices are made among a few timed runs, none of 34 sizes of these two Llama
+    shapes was: whole passes at 0.95 to 1.00 of their time). Apart and here: n 3,072, k 2,048 192 rows
+    20.9 and 13.8, 513 rows 20.9 and 14.2, 1,024 rows 26.6 and 22.8, 2,048 rows 37.0 and 32.4, 3,000 rows 50.5 and 46.0; n 5,120, k 3,072
+    192 rows (left apart) 32.3 and 27.8, 720 rows 39.9 and 34.4, 1,514 rows 59.5 and 49.4, 2,048 rows 72.4 and 59.6."""
+    if not WHOLE_ROPE_MIN_ROWS <= rows <= WHOLE_ROPE_MAX_ROWS or k % 64 or k < 64 * WHOLE_MIN_STEPS:
+        return None
+    steps, costs = k // 64, []
+    for bm, bn, held, (fixed, one, two, weight, out) in WHOLE_ROPE_TILES:
+        rounds = -(-(-(-rows // bm) * -(-n // bn)) // COMPUTE_UNITS)
+        chain = one * (rounds % 2) + two * (rounds // 2) if held == 2 else one * rounds
+        costs.append(fixed + steps * chain + (weight * k + out * rows) * n * 1e-6)
+    fixed, chain, rooted, work, weight, out = WHOLE_ROPE_APART
+    apart = fixed + (chain + rooted * math.sqrt(rows) / 32) * k / 1024 + (work * rows * k * 1e-3 + weight * k + out * rows) * n * 1e-6
+    share = WHOLE_ROPE_SURE_SHARE if rows <= WHOLE_ROPE_FEW or n * k > WHOLE_ROPE_LARGE else WHOLE_ROPE_SHARE
+    return costs.index(min(costs)) if min(costs) < share * apart else None
+
+
+def qkv_rope_whole_takes(x: torch.Tensor, weight: torch.Tensor, head_dim: int, k_cache: torch.Tensor | None, table: torch.Tensor | None) -> bool:
+    """Whether `qkv_rope_store_whole` takes these operands (whatever the rule by sizes says of them): whole heads that turn as a whole."""
+    return (whole_takes(x, weight) and x.is_cuda and head_dim % 64 == 0 and weight.shape[0] * weight.stride(0) < 1 << 30
+            and (k_cache is None or k_cache.dtype == torch.bfloat16)
+            and (table is None or (table.dim() == 2 and table.shape[1] == head_dim and table.is_contiguous() and table.data_ptr() % 16 == 0)))
+
+
+def qkv_rope_whole_tile(x: "torch.Tensor", weight: torch.Tensor, packed: "StreamingCopies | None", head_dim: int, k_cache: torch.Tensor | None,
+                        table: torch.Tensor | None) -> int | None:
+    """The tile in which `qkv_rope_store_whole` should serve these operands, where `linear_bf16` would give the product to a kernel for many
+    rows; None if it should not."""
+    if _many_rows != "library" or x.dim() != 2:
+        return None
+    rows, k = x.shape
+    tile = qkv_rope_whole_plan(rows, weight.shape[0], k)
+    if (tile is None or not _library_serves(rows, weight.shape[0], k, packed is not None and packed.by16 is not None, False)
+            or not qkv_rope_whole_takes(x, weight, head_dim, k_cache, table)):
+        return None
+    return tile
+
+
+def qkv_rope_store_whole(x: torch.Tensor, weight: torch.Tensor, tile: int, cos_sin: torch.Tensor | None, positions: torch.Tensor, slots: torch.Tensor | None,
+                         k_cache: torch.Tensor | None, v_cache: torch.Tensor | None, num_heads: int, num_kv_heads: int, head_dim: int) -> torch.Tensor:
+    """`rope_store(x · weight^T in bfloat16, ...)` for many rows of x in one kernel (gemm_whole.hip), whole heads of a multiple of 64;
+    `tile` by its place in `WHOLE_ROPE_TILES`."""
+    q = _native().qkv_rope_store_sliced(x, weight, tile, cos_sin, positions, slots, k_cache, v_cache, num_heads, num_kv_heads, head_dim, 0.0, None)
+    if q is not None:
+        return q
+    _gpu(x, weight, cos_sin, positions, slots, k_cache, v_cache)
+    T, N = x.shape[0], (num_heads + 2 * num_kv_heads) * head_dim
+    _need(x.dim() == 2 and weight.shape == (N, x.shape[1]) and whole_takes(x, weight) and N * weight.stride(0) < 1 << 30 and head_dim % 64 == 0,
+          lambda: f"qkv_rope_store_whole takes bfloat16 x [M, K] with dense, aligned rows, heads of a multiple of 64 and a weight [{N}, K]")
+    _need(0 <= tile < len(WHOLE_ROPE_TILES), lambda: f"tile {tile}: one of {len(WHOLE_ROPE_TILES)}")
+    _need(positions.dtype == torch.int32 and positions.shape == (T,) and positions.is_contiguous(), "positions must be int32 [tokens]")
+    _need(cos_sin is None or (cos_sin.dtype == torch.float32 and cos_sin.dim() == 2 and cos_sin.shape[1] == head_dim and cos_sin.is_contiguous()
+                              and cos_sin.data_ptr() % 16 == 0), lambda: f"the rotation table must be float32 [positions, {head_dim}], 16-byte aligned")
+    page_size, kst, vst = 1, (0, 0, 0), (0, 0, 0, 0)
+    if k_cache is not None:
+        _need(v_cache is not None and slots is not None, "a cache write needs k, v and the slots")
+        _need(slots.dtype == torch.int32 and slots.shape == (T,) and slots.is_contiguous(), "slots must be int32 [tokens]")
+        _check_cache(k_cache, v_cache, x.dtype, num_kv_heads, head_dim)
+        page_size, kst, vst = k_cache.shape[1], k_cache.stride()[:3], v_cache.stride()
+    q = torch.empty((T, num_heads, head_dim), dtype=x.dtype, device=x.device)
+    _run("qkv_rope_store_whole", library().ts_gemm_whole_rope_bf16(
+        _ptr(q), _ptr(x), _ptr(weight), T, x.shape[1], x.stride(0), weight.stride(0), _ptr(cos_sin), _ptr(positions), _ptr(slots), _ptr(k_cache), _ptr(v_cache),
+        num_heads, num_kv_heads, head_dim, page_size, *kst, *vst, tile, _stream()))
+    return q
 
 
 def linear_through_norm(x: torch.Tensor, weight: torch.Tensor, packed: "StreamingCopies | None", residual: torch.Tensor | None,

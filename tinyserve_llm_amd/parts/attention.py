@@ -99,6 +99,15 @@ class Attention(Mixer):
                                                norm_weight=d.weight, eps=d.eps, packed=by16)
         return q
 
+    def _project_whole(self, x: torch.Tensor, table, positions, slots, k_store, v_store) -> torch.Tensor:
+        """The same for many rows: one kernel where that is the faster way (`hip.qkv_rope_whole_plan`), a product and `rope_store` where not."""
+        tile = hip.qkv_rope_whole_tile(x, self.qkv, self.qkv_packed, self.head_dim, k_store, table)
+        if tile is not None:
+            return hip.qkv_rope_store_whole(x, self.qkv, tile, table, positions, slots, k_store, v_store, self.num_heads, self.num_kv_heads,
+                                            self.head_dim)
+        return hip.rope_store(linear(x, self.qkv, packed=self.qkv_packed), table, positions, slots, k_store, v_store, self.num_heads,
+                              self.num_kv_heads, self.head_dim)
+
     def param_specs(self) -> dict[str, ParamSpec]:
         return {"qkv": ParamSpec((self.q_size + 2 * self.kv_size, self.hidden_size)),
                 "o": ParamSpec((self.hidden_size, self.q_size))}
@@ -112,9 +121,13 @@ class Attention(Mixer):
         k_store, v_store = (mem.k_cache, mem.v_cache) if mem.store else (None, None)
         q = self._project_fused(x, table, ctx.positions, slots, k_store, v_store)
         if q is None:
-            qkv = linear(x, self.qkv, packed=self.qkv_packed)
-            q = hip.rope_store(qkv, table, ctx.positions, slots, k_store, v_store, self.num_heads, self.num_kv_heads,
-                               self.head_dim)
+            if isinstance(x, DeferredNorm) and x.prepared is None and x.rows >= hip.WHOLE_ROPE_MIN_ROWS:
+                x = x.materialize()              # (`linear` runs the norm by its own kernel as well with so many rows)
+            if isinstance(x, DeferredNorm):
+                q = hip.rope_store(linear(x, self.qkv, packed=self.qkv_packed), table, ctx.positions, slots, k_store, v_store, self.num_heads,
+                                   self.num_kv_heads, self.head_dim)
+            else:
+                q = self._project_whole(x, table, ctx.positions, slots, k_store, v_store)
         # (a single token: the o projection adds the chunks of a split walk up itself, on its way in)
         o = hip.paged_attention(q, mem.k_cache, mem.v_cache, ctx, mem.space, self.scale, self.window,
                                 leave_split=hip.split_attention_fuses(ctx.num_tokens, self.o))

@@ -156,3 +156,22 @@ def test_the_rule_keeps_to_what_was_measured():
         assert tiles[plan(rows, n, k)] == tile
     assert plan(128, 3072, 2048) is None and plan(3073, 3072, 2048) is None and plan(170, 5120, 3072) is None
     assert plan(512, 3072, 2080) is None and plan(512, 1536, 128) is None
+
+
+def test_whole_tiles_are_taken_where_they_were_the_faster_way():
+    for rows, n, k, ending, tile in ((999, 12352, 2048, "f32", (256, 256)), (2048, 10304, 2048, "f32", (192, 256)), (2048, 2048, 2048, "bf16", (128, 128)), (720, 2048, 2048, "f32", (64, 128))):
+        plan, slices = hip.many_rows_plan(rows, n, k, ending)
+        assert hip.SLICES_TILES[plan][:2] == tile and slices == 1
+    for rows, n, k in ((257, 2048, 2048), (128, 12352, 2048), (3073, 12352, 2048), (999, 16384, 2048), (999, 1024, 2048), (999, 12352, 960), (999, 12356, 2048)):
+        assert hip.many_rows_plan(rows, n, k, "f32") is None
+    assert hip.many_rows_plan(1024, 2048, 8192, "f32") == hip.slices_plan(1024, 2048, 8192, "f32") != None      # noqa: E711 (a long reduction is cut as before)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows, n, k, out", [(720, 2048, 2048, torch.float32), (999, 12352, 2048, BF)])
+def test_linear_takes_them_by_the_module_and_by_the_general_function(rows, n, k, out, monkeypatch):
+    x, w = operands(rows, n, k)
+    want = hip.gemm_whole([x], [w], hip.whole_plan(rows, n, k, "f32" if out is torch.float32 else "bf16"), out)[0]
+    assert torch.equal(hip.linear_bf16(x, w, out), want)
+    monkeypatch.setattr(hip, "_native", lambda: types.SimpleNamespace(gemm_slices=lambda *a: None, gemm_library=lambda *a: None))
+    assert torch.equal(hip.linear_bf16(x, w, out), want)

@@ -1749,6 +1749,66 @@ def gemm_slices(x: torch.Tensor, weight: torch.Tensor, tile: int, slices: int, o
     return y if nw is None else (y, total)
 
 
+# For the tiles of `gemm_whole` (`SLICES_TILES`), by the type that comes out: workgroups that a compute unit holds; the µs that do not depend on the sizes;
+# those of a step of 64 of K in a round that fills the chip, in a last round that gives every compute unit at most one workgroup, in a fuller one, and
+# of its fill; of a million numbers of W; of a million of y
+WHOLE_TILES = {"bf16": ((2, 3.37, 0.894, 0.374, 0.555, 0.314, 0.124, 0.303), (1, 4.60, 0.823, 0.533, 0.0, 0.207, 0.216, 0.188),
+                        (1, 5.50, 1.053, 0.740, 0.0, 0.204, 0.147, 0.414), (1, 6.52, 1.335, 0.939, 0.0, 0.284, 0.094, 0.447),
+                        (2, 3.77, 0.649, 0.214, 0.370, 0.172, 0.271, 0.0)),
+               "f32": ((2, 4.12, 0.922, 0.378, 0.578, 0.273, 0.148, 0.769), (1, 6.34, 0.860, 0.533, 0.0, 0.197, 0.232, 0.440),
+                       (1, 8.37, 1.132, 0.733, 0.0, 0.268, 0.127, 0.486), (1, 9.98, 1.453, 0.938, 0.0, 0.353, 0.067, 0.533),
+                       (2, 4.52, 0.696, 0.207, 0.378, 0.170, 0.292, 0.142))}
+# what the matrix library takes: fixed, a thousand of K, that times the root of the rows over 32, and a million products (of a thousand each), numbers
+# of W and of y
+WHOLE_LIBRARY = {"bf16": (6.10, 0.431, 1.371, 1.152, 0.418, 0.329), "f32": (5.25, 0.551, 1.564, 1.093, 0.432, 0.862)}
+# the share of that, both as estimated, up to which whole tiles are taken: of few rows (inside a pass bfloat16 products of 500 to 650 rows were 1 % of the
+# pass slower than timed by themselves), of more, and of many in 32 bits with a wide W
+WHOLE_FEW_SHARE, WHOLE_SHARE, WHOLE_WIDE_SHARE = 0.92, 0.98, 1.03
+WHOLE_FEW, WHOLE_MANY, WHOLE_WIDE = {"bf16": 960, "f32": 450}, 960, 8192
+WHOLE_MIN_ROWS, WHOLE_MAX_ROWS = 129, 3072      # fewer rows: the kernels that share x
+WHOLE_MIN_WIDTH, WHOLE_MAX_WIDTH, WHOLE_MIN_K = 2048, 12800, 1024
+
+
+def _whole_cost(rows: int, widths: "tuple[int, ...]", k: int, ending: str) -> tuple[float, int]:
+    """(µs, tile) of the products of `rows` rows against weights [width, k] in one launch by the tile estimated to be the fastest."""
+    costs, total = [], sum(widths)
+    for (bm, bn, *_), (held, fixed, full, one, two, fill, weight, out) in zip(SLICES_TILES, WHOLE_TILES[ending]):
+        rounds, rest = divmod(-(-rows // bm) * sum(-(-n // bn) for n in widths), held * COMPUTE_UNITS)
+        chain = full * rounds + (0.0 if rest == 0 else two if rest > COMPUTE_UNITS else one) + fill * rest / (held * COMPUTE_UNITS)
+        costs.append(fixed + k // 64 * chain + (weight * k + out * rows) * total * 1e-6)
+    return min(costs), costs.index(min(costs))
+
+
+def _whole_library(rows: int, n: int, k: int, ending: str) -> float:
+    """µs that the matrix library's product is estimated to take."""
+    fixed, chain, rooted, work, weight, out = WHOLE_LIBRARY[ending]
+    return fixed + (chain + rooted * math.sqrt(rows) / 32) * k / 1024 + (work * rows * k * 1e-3 + weight * k + out * rows) * n * 1e-6
+
+
+@functools.lru_cache(maxsize=4096)
+def whole_plan(rows: int, n: int, k: int, ending: str) -> int | None:
+    """The tile of `gemm_whole` for `rows` rows of x against a weight [n, k]; None where the matrix library may well be as fast. Both sides are estimates
+    fitted to 836 measured points with weights from memory (129 to 6,000 rows, n 256 to 16,384, k 256 to 5,120; 3 to 9 % root mean square within these limits). Of 530 of
+    them that lie within these limits and are not for slices, the rule takes 137, at 0.93 of the library's time on average; 7 of them are slower by more than 2 %, all in
+    bfloat16 and wide: n 8,192, k 2,048, 2,048 rows 52.5 and 56.8 µs the most. Library and here: bfloat16, n 12,352, k 2,048, 999 rows 58.4 and 50.6; 32 bits, the same
+    62.7 and 55.3, n 10,304, k 2,048, 2,048 rows 98.2 and 88.4, n 2,048, k 2,048, 720 rows 14.8 and 13.9, 257 rows (left to the library) 11.6 and 13.0."""
+    if (not WHOLE_MIN_ROWS <= rows <= WHOLE_MAX_ROWS or not WHOLE_MIN_WIDTH <= n <= WHOLE_MAX_WIDTH or n % 8 or k % 64 or k < WHOLE_MIN_K):
+        return None
+    us, tile = _whole_cost(rows, (n,), k, ending)
+    share = WHOLE_FEW_SHARE if rows < WHOLE_FEW[ending] else WHOLE_WIDE_SHARE if rows >= WHOLE_MANY and n >= WHOLE_WIDE and ending == "f32" else WHOLE_SHARE
+    return tile if us < share * _whole_library(rows, n, k, ending) else None
+
+
+@functools.lru_cache(maxsize=4096)
+def many_rows_plan(rows: int, n: int, k: int, ending: str) -> tuple[int, int] | None:
+    """The tile and the slices of `gemm_slices` for a product that would go to the matrix library: in slices, or whole in one; None: the library's."""
+    plan = slices_plan(rows, n, k, ending)
+    if plan is None:
+        tile = whole_plan(rows, n, k, ending)
+        plan = None if tile is None else (tile, 1)
+    return plan
+
+
 WHOLE_PRODUCTS = 8                                                             # products of one launch
 
 
@@ -1989,7 +2049,7 @@ def linear_bf16(x: torch.Tensor, weight: torch.Tensor, out_dtype: torch.dtype = 
         if (_library_serves(rows, weight.shape[0], k, packed is not None and packed.by16 is not None, out_dtype is torch.float32)
                 and x.stride(0) % 8 == 0 and weight.stride(0) % 8 == 0):
             wide = out_dtype is torch.float32
-            plan = slices_plan(rows, weight.shape[0], k, "f32" if wide else "bf16")
+            plan = many_rows_plan(rows, weight.shape[0], k, "f32" if wide else "bf16")
             y = _native().gemm_library(x, weight, wide) if plan is None else _native().gemm_slices(x, weight, *plan, wide, None, None, 0.0)
             if y is not None:
                 return y
@@ -2019,7 +2079,7 @@ def linear_bf16(x: torch.Tensor, weight: torch.Tensor, out_dtype: torch.dtype = 
         # rows that are no whole 16-byte pieces: the library has no algorithm for every such shape; the
         # exact kernel takes any (32-bit multiply-adds, slower, for sizes no real model has)
         return gemm_exact(x, weight, out_dtype)
-    plan = slices_plan(x.shape[0], weight.shape[0], x.shape[1], "f32" if out_dtype == torch.float32 else "bf16") if _many_rows == "library" else None
+    plan = many_rows_plan(x.shape[0], weight.shape[0], x.shape[1], "f32" if out_dtype == torch.float32 else "bf16") if _many_rows == "library" else None
     if plan is not None and slices_takes(x, weight):
         return gemm_slices(x, weight, *plan, out_dtype)
     return gemm_library(x, weight, out_dtype)

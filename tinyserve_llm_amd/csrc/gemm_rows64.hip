@@ -38,6 +38,7 @@
 #define R64_CHUNK_STEPS 8         // 32-wide k steps per chunk of x in LDS
 #define R64_RING 16               // steps of W a compute wave has under way (two chunks): with 32 the chip had 32 MB under way and
                                   // every load, x's among them, came back some 5 us later (the gate|up product of 64 rows 20.7 us, 19.7 with 16)
+#define R64_STRETCH 4             // steps whose products a group's sums take together
 #define R64_STAGE_LOADS 8          // loads of a staging wave per chunk: two rows of its block each
 
 struct Rows64Args {
@@ -56,11 +57,27 @@ struct Rows64Args {
   int slices;            // the reduction in this many slices (gridDim.y); more than one: y is float [slices][M][ldy]
 };
 
+// Several products of the same rows and reduction in one launch, each with its x and its 32-bit y, their packed copies one behind the other:
+// the workgroups from first[p] on are product p's.
+#define R64_PRODUCTS 8
+struct Rows64GroupArgs : Rows64Args {
+  int products, first[R64_PRODUCTS], width[R64_PRODUCTS], tile0[R64_PRODUCTS];      // (tile0: the first 16-row tile of its copy)
+  const bf16_t* xs[R64_PRODUCTS];      // [M, K], rows ldx apart
+  float* ys[R64_PRODUCTS];             // [M, width]
+};
+
 // BLOCKS: blocks of 16 rows of x, 4 (up to 64 rows) or 8 (up to 128: the compute waves then take a chunk's
 // steps one at a time instead of in pairs, for their registers' sake).
 // GLU: 0 none, 1 silu(gate) up, 1 + f the unit of form f of glu_unit.h.
-template <int GLU, typename OUT, int BLOCKS>
-__global__ void __launch_bounds__(512) gemm_rows64_kernel(const Rows64Args a) {
+// With a group's arguments the sums are added up in stretches of 128 of K, with up to 64 rows in pairs of them, so that they are as near to 64 bits as
+// those of the kernels for a product of its own, which share a reduction out to their waves (over 2,048: 0.9e-7 up to 8 rows, 1.0e-7 up to 32, 1.3e-7 up to
+// 64, the library's beyond 2.7e-7). A product of a few million numbers of W is a launch, a trip of x to LDS and as few workgroups as it has columns for
+// 64 each: five of them (2,048 columns four times and 64, K 2,048) took 18 us apart and take 10.5 here with 1 row, 20 and 10.7 with 8, 28 and 11.3 with
+// 32, 50 and 11.8 with 48.
+template <int GLU, typename OUT, int BLOCKS, typename ARGS>
+__global__ void __launch_bounds__(512) gemm_rows64_kernel(const ARGS a) {
+  constexpr bool GROUP = std::is_same_v<ARGS, Rows64GroupArgs>;
+  static_assert(!GROUP || (GLU == 0 && std::is_same_v<OUT, float>), "products of a group are plain and 32-bit");
   // x as the B operands of the matrix instruction: [buffer][step][block of 16 rows][lane], lane r + 16 g
   // holding k = 8 g .. 8 g + 7 of row r (turned: sk_place)
   extern __shared__ __align__(16) uint4 xs_all[];
@@ -70,6 +87,12 @@ __global__ void __launch_bounds__(512) gemm_rows64_kernel(const Rows64Args a) {
   const int slice = blockIdx.y;
   const int nsteps = a.K / SK_KSTEP / a.slices, nchunks = nsteps / R64_CHUNK_STEPS;   // (steps: a multiple of the ring, chunks: even)
   const int64_t kfirst = (int64_t)slice * nsteps * SK_KSTEP;                  // the slice's first k
+  int which = 0;                                                              // the group's product
+  const bf16_t* x = a.x;
+  if constexpr (GROUP) {
+    while (which + 1 < a.products && (int)blockIdx.x >= a.first[which + 1]) ++which;
+    x = a.xs[which];
+  }
 
   if (wave >= 4) {
     // ---- staging waves: wave sw brings block sw of 16 rows, all the steps of every chunk. It asks for
@@ -91,7 +114,7 @@ __global__ void __launch_bounds__(512) gemm_rows64_kernel(const Rows64Args a) {
     auto ask = [&](int c, uint4 (&t)[LOADS]) {
       const int k0 = c * R64_CHUNK_STEPS * SK_KSTEP;      // first k of the chunk
 #pragma unroll
-      for (int j = 0; j < LOADS; ++j) t[j] = *(const uint4*)(a.x + xoff[j] + k0);
+      for (int j = 0; j < LOADS; ++j) t[j] = *(const uint4*)(x + xoff[j] + k0);
     };
     auto put = [&](int c, const uint4 (&t)[LOADS]) {
       uint4* buf = xs(c & 1, 0, 0);
@@ -114,7 +137,12 @@ __global__ void __launch_bounds__(512) gemm_rows64_kernel(const Rows64Args a) {
   }
 
   // ---- compute waves
-  const int tile = GLU ? (wave < 2 ? 2 * blockIdx.x + wave : a.N / 32 + 2 * blockIdx.x + (wave - 2)) : 4 * blockIdx.x + wave;
+  int tile = GLU ? (wave < 2 ? 2 * blockIdx.x + wave : a.N / 32 + 2 * blockIdx.x + (wave - 2)) : 4 * blockIdx.x + wave;
+  int column = 0;                                        // of a group: the first of this wave's in its product (past the last: computed again, not stored)
+  if constexpr (GROUP) {
+    column = 16 * (tile - 4 * a.first[which]);
+    tile = a.tile0[which] + min(column, a.width[which] - 16) / 16;
+  }
   const bf16_t* wp = a.w16 + (((int64_t)tile * a.slices + slice) * nsteps * 64 + lane) * 8;      // the slice's step s at wp + 512 s
   uint4 wr[R64_RING];
   // (in this order and no other: the ring is used oldest first, and a wait is for the oldest load only if the
@@ -127,6 +155,12 @@ __global__ void __launch_bounds__(512) gemm_rows64_kernel(const Rows64Args a) {
   float4_t acc[BLOCKS];
 #pragma unroll
   for (int b = 0; b < BLOCKS; ++b) acc[b] = (float4_t){0.f, 0.f, 0.f, 0.f};
+  constexpr bool PAIRS = BLOCKS == 4;                    // (more rows have no registers for it, and were the library's, which has no stretches)
+  float4_t total[GROUP ? BLOCKS : 1], held[GROUP && PAIRS ? BLOCKS : 1];
+  if constexpr (GROUP) {
+#pragma unroll
+    for (int b = 0; b < BLOCKS; ++b) total[b] = (float4_t){0.f, 0.f, 0.f, 0.f};
+  }
   int at[4];                    // where this lane's piece of a step lies in a block, by the step's last two bits
 #pragma unroll
   for (int i = 0; i < 4; ++i) at[i] = sk_place(r, i, g);
@@ -176,7 +210,17 @@ __global__ void __launch_bounds__(512) gemm_rows64_kernel(const Rows64Args a) {
         for (int i = 0; i < PER; ++i) {
           const int sl = R64_CHUNK_STEPS * h + PER * q + i;
 #pragma unroll
-          for (int b = 0; b < BLOCKS; ++b) acc[b] = sk_mfma(wr[sl], xb[q & 1][i][b], acc[b]);
+          for (int b = 0; b < BLOCKS; ++b) acc[b] = sk_mfma(wr[sl], xb[q & 1][i][b], GROUP && sl % R64_STRETCH == 0 ? (float4_t){0.f, 0.f, 0.f, 0.f} : acc[b]);
+          if constexpr (GROUP) {
+            if (sl % R64_STRETCH == R64_STRETCH - 1) {
+#pragma unroll
+              for (int b = 0; b < BLOCKS; ++b) {
+                if (!PAIRS) total[b] += acc[b];
+                else if (sl % (2 * R64_STRETCH) < R64_STRETCH) held[b] = acc[b];
+                else total[b] += held[b] + acc[b];
+              }
+            }
+          }
           if (decltype(more)::value) wr[sl] = *(const uint4*)(wp + (int64_t)(base + R64_RING + sl) * 512);
         }
         __builtin_amdgcn_sched_barrier(0);
@@ -188,6 +232,13 @@ __global__ void __launch_bounds__(512) gemm_rows64_kernel(const Rows64Args a) {
   for (; base + R64_RING < nsteps; base += R64_RING) ring(base, std::true_type{});
   ring(base, std::false_type{});
   // acc[b][j] = sum over k of W[row 16 tile + 4 g + j, k] * x[16 b + r, k]
+  if constexpr (GROUP) {
+    float* const to = a.ys[which] + column + 4 * g;
+#pragma unroll
+    for (int b = 0; b < BLOCKS; ++b)
+      if (16 * b + r < a.M && column < a.width[which]) *(float4_t*)(to + (int64_t)(16 * b + r) * a.width[which]) = total[b];
+    return;
+  }
   float4_t* ex = (float4_t*)xs_all;                      // [2 up waves][blocks][lane]; every read of x is behind the last barrier
   if (GLU) {
     if (wave >= 2) {
@@ -223,8 +274,8 @@ template <int GLU, typename OUT>
 static int r64_launch(const Rows64Args& a, hipStream_t stream) {
   // 64 rows of W per workgroup; two buffers of a chunk of x in LDS: 64 KB for up to 64 rows, 128 KB beyond
   const dim3 grid(a.N / 64, a.slices);
-  if (a.M <= 64) gemm_rows64_kernel<GLU, OUT, 4><<<grid, 512, 2 * R64_CHUNK_STEPS * 4 * TS_WAVE * sizeof(uint4), stream>>>(a);
-  else gemm_rows64_kernel<GLU, OUT, 8><<<grid, 512, 2 * R64_CHUNK_STEPS * 8 * TS_WAVE * sizeof(uint4), stream>>>(a);
+  if (a.M <= 64) gemm_rows64_kernel<GLU, OUT, 4, Rows64Args><<<grid, 512, 2 * R64_CHUNK_STEPS * 4 * TS_WAVE * sizeof(uint4), stream>>>(a);
+  else gemm_rows64_kernel<GLU, OUT, 8, Rows64Args><<<grid, 512, 2 * R64_CHUNK_STEPS * 8 * TS_WAVE * sizeof(uint4), stream>>>(a);
   return ts_check_launch();
 }
 
@@ -254,6 +305,26 @@ extern "C" int ts_gemm_rows64_bf16(void* y, const void* x, const void* w16, int 
     case 1 + GLU_GELU: return r64_launch<1 + GLU_GELU, bf16_t>(a, stream);
   }
   return TS_BAD_SHAPE;
+}
+
+// `products` of them in one launch (1 to 8): x[i] [M <= 128, K] with rows ldx apart, y[i] float32 [M, N[i]] contiguous, 16-byte aligned; w16 the
+// packed copies of their W [N[i], K], one behind the other; N[i] multiples of 16, K of 1,024.
+extern "C" int ts_gemm_rows64_group_bf16(int products, void* const* y, const void* const* x, const void* w16, const int* N, int M, int K, int64_t ldx,
+                                         hipStream_t stream) {
+  if (M <= 0) return TS_OK;
+  if (products < 1 || products > R64_PRODUCTS || !y || !x || !N || K % 1024) return TS_BAD_SHAPE;
+  Rows64GroupArgs a = {};
+  a.w16 = (const bf16_t*)w16, a.M = M, a.K = K, a.ldx = ldx, a.slices = 1, a.products = products;
+  int64_t groups = 0, tiles = 0;
+  for (int i = 0; i < products; ++i) {
+    if (N[i] <= 0 || N[i] % 16 || !y[i] || ((uintptr_t)y[i] & 15) || !r64_operands_ok(x[i], w16, M, N[i], K, ldx)) return TS_BAD_SHAPE;
+    a.first[i] = (int)groups, a.width[i] = N[i], a.tile0[i] = (int)tiles, a.xs[i] = (const bf16_t*)x[i], a.ys[i] = (float*)y[i];
+    groups += (N[i] + 63) / 64, tiles += N[i] / 16;
+    if (tiles > (1 << 24)) return TS_TOO_LARGE;
+  }
+  if (M <= 64) gemm_rows64_kernel<0, float, 4, Rows64GroupArgs><<<(unsigned)groups, 512, 2 * R64_CHUNK_STEPS * 4 * TS_WAVE * sizeof(uint4), stream>>>(a);
+  else gemm_rows64_kernel<0, float, 8, Rows64GroupArgs><<<(unsigned)groups, 512, 2 * R64_CHUNK_STEPS * 8 * TS_WAVE * sizeof(uint4), stream>>>(a);
+  return ts_check_launch();
 }
 
 // ---- a product in slices of its reduction, and what finishes it

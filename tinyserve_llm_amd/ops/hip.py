@@ -94,6 +94,7 @@ def _declare(lib: ctypes.CDLL) -> None:
         "ts_gemm_whole_bf16": [i, p, p, p, p, i, i, i64, i64, i, i, p],
         "ts_gemm_whole_rope_bf16": [p, p, p, i, i, i64, i64, p, p, p, p, p, i, i, i, i, i64, i64, i64, i64, i64, i64, i64, i, p],
         "ts_gemm_rows64_bf16": [p, p, p, i, i, i, i64, i64, i, i, p, i, f, f, f, f, p],
+        "ts_gemm_rows64_group_bf16": [i, p, p, p, p, i, i, i64, p],
         "ts_gemm_rows64_sliced_bf16": [p, p, p, p, i, i, i, i64, i, p, p, p, p, p, i64, p],
         "ts_gemm_rows64_sliced_rope_bf16": [p, p, p, p, i, i, i64, i, p, i, f, p, p, p, p, p, i, i, i, i, i, i64, i64, i64, i64, i64,
                                             i64, i64, p],
@@ -1337,6 +1338,29 @@ def gemm_rows64(x: torch.Tensor, packed: torch.Tensor, out_dtype: torch.dtype = 
     return out
 
 
+ROWS64_PRODUCTS = 8            # products of one launch
+
+
+def gemm_rows64_group(xs: "Sequence[torch.Tensor]", packed: torch.Tensor, widths: "Sequence[int]") -> "tuple[torch.Tensor, ...]":
+    """float32 x [M <= 128, K] · W [N, K]^T of up to 8 products of the same M, K and strides in one launch; `packed` holds the `pack_weight` copies
+    of their weights (of `widths` rows, multiples of 16) one behind the other."""
+    _need(1 <= len(xs) == len(widths) <= ROWS64_PRODUCTS, lambda: f"{len(xs)} operands and {len(widths)} weights: one to {ROWS64_PRODUCTS} products")
+    _gpu(*xs, packed)
+    x = xs[0]
+    M, K = x.shape
+    _need(all(t.dtype == torch.bfloat16 and t.shape == x.shape and t.stride() == x.stride() and t.data_ptr() % 16 == 0 for t in xs) and x.stride(1) == 1
+          and x.stride(0) % 8 == 0, "operands of a group are bfloat16, of one shape, with dense, 16-byte aligned rows as far apart")
+    _need(packed.dtype == torch.bfloat16 and packed.dim() == 4 and packed.shape[1] * 32 == K and packed.shape[2:] == (64, 8) and packed.is_contiguous()
+          and packed.shape[0] * 16 == sum(widths) and all(n > 0 and n % 16 == 0 for n in widths),
+          lambda: f"the packed copies of weights of {list(widths)} rows (multiples of 16) over {K}")
+    _need(1 <= M <= ROWS64_MAX_ROWS and K % 1024 == 0, lambda: f"gemm_rows64_group takes up to {ROWS64_MAX_ROWS} rows and K in steps of 1024, not {M} x {K}")
+    ys = tuple(torch.empty((M, n), dtype=torch.float32, device=x.device) for n in widths)
+    n = len(ys)
+    pointers = [(ctypes.c_void_p * n)(*(t.data_ptr() for t in ts)) for ts in (ys, xs)]
+    _run("gemm_rows64_group", library().ts_gemm_rows64_group_bf16(n, *pointers, _ptr(packed), (ctypes.c_int * n)(*widths), M, K, x.stride(0), _stream()))
+    return ys
+
+
 ROWS64_SLICE_K = 512           # a slice of the reduction is a multiple of this (one turn of a compute wave's ring of W)
 ROWS64_SLICED_MIN_ROWS = 5     # (fewer rows are the 8-row form's at any width; where the weight-streaming kernels serve a shape, they come first)
 ROWS64_WORKGROUPS = 192        # workgroups from which the chip's 256 compute units count as filled
@@ -1832,6 +1856,47 @@ def gemm_whole(xs: "Sequence[torch.Tensor]", weights: "Sequence[torch.Tensor]", 
         _run("gemm_whole", library().ts_gemm_whole_bf16(n, *pointers, (ctypes.c_int * n)(*(w.shape[0] for w in weights)), M, K, xs[0].stride(0),
                                                         weights[0].stride(0), tile, int(out_dtype is torch.float32), _stream()))
     return ys
+
+
+GROUP_FEW_ROWS = 64            # rows up to which a group goes to the kernel that streams W past x, beyond to whole tiles
+GROUP_SURE_ROWS, GROUP_SURE_WIDTH, GROUP_MIN_ROWS = 9, 8192, 5      # two products of few rows: from these rows on, or, with so many columns, from those
+
+
+@functools.lru_cache(maxsize=4096)
+def group_plan(rows: int, widths: "tuple[int, ...]", k: int, packed: bool) -> int | None:
+    """How `gemm_group` makes the products of `rows` rows against weights [width, k]: -1 by `gemm_rows64_group` (with `packed`: their packed copies are
+    there), a tile of `gemm_whole`, or None: one by one, which may well be as fast. Measured, µs, one by one and together: widths 2,048 four times and 64, k
+    2,048: 1 row 18.4 and 11.1, 8 rows 20.4 and 11.1, 48 rows 50.5 and 12.7, 128 rows 43.0 and 14.6, 600 rows 62.5 and 30.5, 2,048 rows 109.6 and 85.3; 2,048
+    twice: 1 row (left) 7.3 and 8.9, 16 rows 10.0 and 9.3, 48 rows 17.2 and 9.5, 1,024 rows 29.0 and 23.0; 3,104 and 8,192: 4 rows (left) 13.4 and 13.1, 8 rows 14.1 and 13.2, 48
+    rows 24.0 and 14.8, 1,024 rows 62.6 and 53.3, 1,500 rows (left) 77.6 and 86.0."""
+    if len(widths) < 2 or len(widths) > min(ROWS64_PRODUCTS, WHOLE_PRODUCTS):
+        return None
+    if rows <= GROUP_FEW_ROWS:
+        pays = len(widths) > 2 or rows >= GROUP_SURE_ROWS or (rows >= GROUP_MIN_ROWS and sum(widths) >= GROUP_SURE_WIDTH)
+        return -1 if packed and pays and k % 1024 == 0 and all(n % 16 == 0 for n in widths) else None
+    if rows > WHOLE_MAX_ROWS or k % 64 or k < WHOLE_MIN_K or any(n % 8 for n in widths):
+        return None
+    us, tile = _whole_cost(rows, widths, k, "f32")
+    apart = 0.0
+    for n in widths:
+        taken = many_rows_plan(rows, n, k, "f32")
+        alone = _whole_library(rows, n, k, "f32")
+        apart += min(alone, _whole_cost(rows, (n,), k, "f32")[0]) if taken is not None else alone
+    return tile if us < apart else None
+
+
+def gemm_group(xs: "Sequence[torch.Tensor]", weights: "Sequence[torch.Tensor]", packed: torch.Tensor | None) -> "tuple[torch.Tensor, ...] | None":
+    """float32 x · weight^T of several bfloat16 products of the same rows and reduction in one launch, where that is the faster way (`group_plan`); None
+    where not, or where their operands are another way. `packed`: the `pack_weight` copies of all the weights, one behind the other, if they are kept."""
+    x, w = xs[0], weights[0]
+    if _many_rows != "library" or x.dim() != 2 or not x.is_cuda or not all(
+            t.shape == x.shape and t.stride() == x.stride() and v.stride() == w.stride() and whole_takes(t, v) for t, v in zip(xs, weights)):
+        return None
+    rows, k = x.shape
+    plan = group_plan(rows, tuple(v.shape[0] for v in weights), k, packed is not None)
+    if rows == 0 or plan is None:
+        return None
+    return gemm_rows64_group(xs, packed, [v.shape[0] for v in weights]) if plan < 0 else gemm_whole(xs, weights, plan, torch.float32)
 
 
 WHOLE_MIN_STEPS = 3      # steps of 64 that a tile's reduction has at least

@@ -15,7 +15,7 @@ import torch
 
 from tinyserve_llm_amd.ops import hip
 from tinyserve_llm_amd.parts.base import KVSpec, LayerMemory, Mixer, ParamSpec, StateSpec, StepContext, register
-from tinyserve_llm_amd.parts.linear import DeferredNorm, linear, streaming_copy
+from tinyserve_llm_amd.parts.linear import DeferredNorm, in_three_steps, linear, streaming_copy
 
 
 @register("mixer", "attention")
@@ -151,6 +151,7 @@ class GeneralAttention(Mixer):
     in 32-bit and carry the weights into the products in two bfloat16 terms."""
 
     graph_safe = True
+    in_three = True
 
     def __init__(self, hidden_size: int, num_heads: int, num_kv_heads: int, head_dim: int, value_dim: int | None = None,
                  position: str | None = None, scale: float | None = None, softcap: float = 0.0, sink: bool = False,
@@ -252,12 +253,18 @@ class GeneralAttention(Mixer):
         self.qkv_packed, self.o_packed = streaming_copy(self.qkv), streaming_copy(self.o)
         return sum(c.nbytes() for c in (self.qkv_packed, self.o_packed) if c is not None)
 
-    def forward(self, x: torch.Tensor, ctx: StepContext, mem: LayerMemory) -> torch.Tensor:
+    def first_weights(self) -> list:
+        return [(self.qkv, self.qkv_packed)] + ([(self.gate, None)] if self.head_gate and not self.gate_inside else [])
+
+    def first_rows(self, x: torch.Tensor, ctx: StepContext, mem: LayerMemory) -> list[torch.Tensor]:
+        return [x] * len(self.first_weights())
+
+    def between(self, sums: list[torch.Tensor], x: torch.Tensor, ctx: StepContext, mem: LayerMemory) -> torch.Tensor:
         enc = ctx.position_encodings[self.position] if self.position else None
         slots = ctx.slot_mapping[mem.space] if mem.store else None
         k_store, v_store = (mem.k_cache, mem.v_cache) if mem.store else (None, None)
         gate_at = self.q_size + self.k_size + self.v_size
-        qkv = linear(x, self.qkv, out_dtype=torch.float32, packed=self.qkv_packed)
+        qkv = sums[0]
         if self.projection_norm_eps is not None:         # in place, each over its whole stretch of the row
             hip.segment_rmsnorm_pair(qkv, (0, self.q_size, self.q_norm), (self.q_size, self.k_size, self.k_norm), self.projection_norm_eps,
                                      bias=self.qkv_bias, rest=(self.q_size + self.k_size, self.v_size) if self.has_bias else (0, 0))
@@ -275,10 +282,12 @@ class GeneralAttention(Mixer):
         o = hip.paged_attention(q, mem.k_cache, mem.v_cache, ctx, mem.space, self.scale, self.window, softcap=self.softcap,
                                 sink=self.sink, sinks=self.sinks, chunk_mask=self.chunk, gate=qkv[:, gate_at:gate_at + self.num_heads] if self.gate_inside else None)
         if value_enc is not None:                         # each head's sum turned back by its own position, then its gate
-            gate = linear(x, self.gate, out_dtype=torch.float32) if self.head_gate else None
+            gate = sums[1] if self.head_gate else None
             hip.rotate_heads(o, o, value_enc.frequencies(), 1.0, ctx.positions, interleaved=value_enc.interleaved, back=True, gate=gate)
-        return linear(o.view(ctx.num_tokens, self.num_heads * self.value_dim), self.o, out_dtype=torch.float32,
-                      packed=self.o_packed)
+        return o.view(ctx.num_tokens, self.num_heads * self.value_dim)
+
+    def forward(self, x: torch.Tensor, ctx: StepContext, mem: LayerMemory) -> torch.Tensor:
+        return in_three_steps(self, x, ctx, mem)
 
 
 @register("mixer", "attention_conv")

@@ -178,6 +178,12 @@ class Mixer(Part):
     # True if forward() takes `then=` (a request of the norm that follows: Norm.request), hands it to
     # the `linear()` call that makes its result, and returns what that call returns
     finishes_into_norm = False
+    # True if forward() is 32-bit products of rows that follow from x alone, something between, and one product with the weight `o`, and the
+    # mixer offers these apart, so that two mixers side by side share launches: `first_weights()` [(weight, its streaming copy or None)],
+    # `first_rows(x, ctx, mem)` the rows each of them multiplies, `between(sums, x, ctx, mem)` the last product's rows, `o` and `o_packed`. (`alone`: a
+    # mixer beside another leaves the copies that several products share to the pair.)
+    in_three = False
+    alone = True
 
     def kv_spec(self) -> KVSpec | None:
         return None

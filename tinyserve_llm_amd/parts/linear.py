@@ -83,6 +83,37 @@ def streaming_copy(weight: torch.Tensor) -> hip.StreamingCopies | None:
     return hip.StreamingCopies(by16, by8) if by16 is not None or by8 is not None else None
 
 
+def packed_together(pairs: "list[tuple[torch.Tensor, hip.StreamingCopies | None]]") -> tuple[torch.Tensor | None, int]:
+    """(The `hip.pack_weight` copies of several (weight, `streaming_copy` of it or None) one behind the other, for `products`, and the bytes they hold
+    besides the copies given, whose 16-row forms become parts of them); (None, 0) where the kernel that reads them does not take the weights."""
+    if not all(w.is_cuda and w.dtype == torch.bfloat16 and w.dim() == 2 and w.is_contiguous() and w.shape[0] % 16 == 0 and w.shape[1] % 1024 == 0
+               and w.shape[1] == pairs[0][0].shape[1] for w, _ in pairs):
+        return None, 0
+    together = torch.cat([c.by16 if c is not None and c.by16 is not None else hip.pack_weight(w) for w, c in pairs])
+    at = more = 0
+    for w, c in pairs:
+        end = at + w.shape[0] // 16
+        if c is not None and c.by16 is not None:
+            c.by16 = together[at:end]
+        else:
+            more += w.numel() * w.element_size()
+        at = end
+    return together, more
+
+
+def products(operands: "list[tuple[torch.Tensor, torch.Tensor, hip.StreamingCopies | None]]", together: torch.Tensor | None) -> "list[torch.Tensor]":
+    """32-bit x · Wᵀ of several (x, weight, `streaming_copy` of it or None), in one launch where that is the faster way (`hip.group_plan`), else one
+    by one. `together`: `packed_together` of the weights, if it is kept."""
+    ys = hip.gemm_group([x for x, _, _ in operands], [w for _, w, _ in operands], together) if len(operands) > 1 else None
+    return list(ys) if ys is not None else [linear(x, w, out_dtype=torch.float32, packed=c) for x, w, c in operands]
+
+
+def in_three_steps(mixer, x: torch.Tensor, ctx, mem, together: torch.Tensor | None = None) -> torch.Tensor:
+    """forward() of a mixer that offers its products apart (`Mixer.in_three`)."""
+    firsts = [(rows, w, c) for rows, (w, c) in zip(mixer.first_rows(x, ctx, mem), mixer.first_weights())]
+    return linear(mixer.between(products(firsts, together), x, ctx, mem), mixer.o, out_dtype=torch.float32, packed=mixer.o_packed)
+
+
 PACKED_ROWS_MIN = 2      # rows from which a gated product is handed on in the 8-row form's order (one row is read whole anyway)
 
 

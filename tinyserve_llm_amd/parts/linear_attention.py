@@ -20,7 +20,7 @@ import torch
 
 from tinyserve_llm_amd.ops import hip
 from tinyserve_llm_amd.parts.base import LayerMemory, Mixer, ParamSpec, StateSpec, StepContext, register
-from tinyserve_llm_amd.parts.linear import linear, streaming_copy
+from tinyserve_llm_amd.parts.linear import in_three_steps, linear, packed_together, streaming_copy
 
 
 @register("mixer", "gated_linear_attention")
@@ -81,6 +81,7 @@ SHIFT_MIXES = ("r", "k", "v", "g", "w")      # the order of the rows of `mu`
 @register("mixer", "shifted_decay_recurrence")
 class ShiftedDecayRecurrence(Mixer):
     graph_safe = True
+    in_three = True
 
     def __init__(self, hidden_size: int, num_heads: int, head_dim: int, decay_rank: int, norm_eps: float) -> None:
         if min(num_heads, head_dim, decay_rank) <= 0 or head_dim > hip.DECAY_MAX_DIM:
@@ -95,6 +96,8 @@ class ShiftedDecayRecurrence(Mixer):
         self.norm: torch.Tensor | None = None
         self.o: torch.Tensor | None = None
         self.packed: dict[str, hip.StreamingCopies | None] = {}
+        self.together: torch.Tensor | None = None      # the first products' packed copies, one behind the other
+        self.alone = True                              # (a mixer beside another leaves them to the pair)
 
     @property
     def size(self) -> int:
@@ -121,18 +124,30 @@ class ShiftedDecayRecurrence(Mixer):
 
     def keep_streaming_copies(self) -> int:
         self.packed = {n: streaming_copy(getattr(self, n)) for n in ("r", "k", "v", "g", "o")}
-        return sum(c.nbytes() for c in self.packed.values() if c is not None)
+        held = sum(c.nbytes() for c in self.packed.values() if c is not None)
+        self.together, more = packed_together(self.first_weights()) if self.alone else (None, 0)
+        return held + more
 
-    def forward(self, x: torch.Tensor, ctx: StepContext, mem: LayerMemory) -> torch.Tensor:
-        H, D = self.num_heads, self.head_dim
-        kept = mem.state[:, self.size * D:]
+    @property
+    def o_packed(self) -> "hip.StreamingCopies | None":
+        return self.packed.get("o")
+
+    def first_weights(self) -> list:
+        return [(getattr(self, n), self.packed.get(n)) for n in SHIFT_MIXES[:4]] + [(self.decay_down, None)]
+
+    def first_rows(self, x: torch.Tensor, ctx: StepContext, mem: LayerMemory) -> list[torch.Tensor]:
+        kept = mem.state[:, self.size * self.head_dim:]
         mixes = hip.token_shift(x, self.mu, kept, ctx)
         hip.token_shift_keep(kept, x, ctx)
-        r, k, v, g = (linear(mixes[i], getattr(self, n), out_dtype=torch.float32, packed=self.packed.get(n))
-                      for i, n in enumerate(SHIFT_MIXES[:4]))
-        low = linear(mixes[4], self.decay_down, out_dtype=torch.float32)
+        return list(mixes)
+
+    def between(self, sums: list[torch.Tensor], x: torch.Tensor, ctx: StepContext, mem: LayerMemory) -> torch.Tensor:
+        H, D = self.num_heads, self.head_dim
+        r, k, v, g, low = sums
         z = linear(hip.bias_activation(low, None, "tanh", x.dtype), self.decay_up, out_dtype=torch.float32)
         o = hip.decay_scan(r, k, v, z, self.decay_bias, mem.state, ctx.cu_seqlens, ctx.state_slots, H, D, D,
                            form="double_exponent", bonus=self.bonus, longest=ctx.max_query_len, ctx=ctx if x.dtype == torch.bfloat16 else None)
-        gated = hip.mlstm_finish(o, self.norm, g, H, D, self.norm_eps, x.dtype, silu_gate=True)
-        return linear(gated, self.o, out_dtype=torch.float32, packed=self.packed.get("o"))
+        return hip.mlstm_finish(o, self.norm, g, H, D, self.norm_eps, x.dtype, silu_gate=True)
+
+    def forward(self, x: torch.Tensor, ctx: StepContext, mem: LayerMemory) -> torch.Tensor:
+        return in_three_steps(self, x, ctx, mem, self.together)

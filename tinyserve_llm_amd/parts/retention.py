@@ -16,12 +16,13 @@ import torch
 
 from tinyserve_llm_amd.ops import hip
 from tinyserve_llm_amd.parts.base import LayerMemory, Mixer, ParamSpec, StateSpec, StepContext, register
-from tinyserve_llm_amd.parts.linear import linear, streaming_copy
+from tinyserve_llm_amd.parts.linear import in_three_steps, streaming_copy
 
 
 @register("mixer", "retention")
 class Retention(Mixer):
     graph_safe = True
+    in_three = True
 
     def __init__(self, hidden_size: int, num_heads: int, head_dim: int, value_dim: int, decay: Sequence[float], norm_eps: float,
                  position: str | None = None) -> None:
@@ -63,11 +64,18 @@ class Retention(Mixer):
         self.proj_packed, self.o_packed = streaming_copy(self.proj), streaming_copy(self.o)
         return sum(c.nbytes() for c in (self.proj_packed, self.o_packed) if c is not None)
 
-    def forward(self, x: torch.Tensor, ctx: StepContext, mem: LayerMemory) -> torch.Tensor:
-        z = self.sizes
+    def first_weights(self) -> list:
+        return [(self.proj, self.proj_packed)]
+
+    def first_rows(self, x: torch.Tensor, ctx: StepContext, mem: LayerMemory) -> list[torch.Tensor]:
+        return [x]
+
+    def between(self, sums: list[torch.Tensor], x: torch.Tensor, ctx: StepContext, mem: LayerMemory) -> torch.Tensor:
+        z, (proj,) = self.sizes, sums
         enc = ctx.position_encodings[self.position] if self.position else None
-        proj = linear(x, self.proj, out_dtype=torch.float32, packed=self.proj_packed)
         mixed = hip.retention_prepare(proj, enc.frequencies() if enc is not None else None, ctx.positions, z, x.dtype)
         o = hip.ssd_scan(mixed, self._steps, self._logs, None, mem.state, ctx, z, keeps=self._keeps)
-        gated = hip.mlstm_finish(o, None, proj[:, z.channels:z.channels + z.inner], z.heads, z.vdim, self.norm_eps, x.dtype, silu_gate=True)
-        return linear(gated, self.o, out_dtype=torch.float32, packed=self.o_packed)
+        return hip.mlstm_finish(o, None, proj[:, z.channels:z.channels + z.inner], z.heads, z.vdim, self.norm_eps, x.dtype, silu_gate=True)
+
+    def forward(self, x: torch.Tensor, ctx: StepContext, mem: LayerMemory) -> torch.Tensor:
+        return in_three_steps(self, x, ctx, mem)

@@ -157,3 +157,27 @@ def test_the_limits_are_those_of_the_general_functions():
     assert {name: int(value) for name, value in held.items()} == {
         "DECODE_MAX_TOKENS": hip.MAX_DECODE_TOKENS, "MAX_SPLITS": hip.MAX_DECODE_SPLITS, "ROWS64_MAX_ROWS": hip.ROWS64_MAX_ROWS, "ROWS64_SLICE_K": hip.ROWS64_SLICE_K,
         "ROW_SKEW": hip.OPERAND_ROW_SKEW, "GATED_SKEW_MIN_ROWS": hip.GATED_SKEW_MIN_ROWS}
+
+
+def test_a_group_of_products(stub):
+    """`gemm_slices` with tuples of operands: in whole tiles, or with packed copies by the kernel that streams them; anything another way is left alone."""
+    module, answer, called = stub
+    xs, ws, packed = (bf(9, 1024), bf(9, 1024)), (bf(64, 1024), bf(32, 1024)), bf(6, 32, 64, 8)
+    for copies, launcher in ((None, "ts_gemm_whole_bf16"), (packed, "ts_gemm_rows64_group_bf16")):
+        ys = module.gemm_slices(xs, ws, 0, copies)
+        assert [(y.dtype, tuple(y.shape)) for y in ys] == [(F32, (9, 64)), (F32, (9, 32))] and called() == [launcher]
+        answer(launcher, BAD_SHAPE)
+        assert module.gemm_slices(xs, ws, 0, copies) is None and called() == [launcher]
+        answer(launcher, LAUNCH_FAILED)
+        with pytest.raises(hip.KernelError, match=hip._ERRORS[LAUNCH_FAILED]):
+            module.gemm_slices(xs, ws, 0, copies)
+        answer(launcher, OK)
+        called()
+        for other in ((list(xs), ws), (xs, ws[:1]), ((), ()), (xs * 5, ws * 5), ((xs[0], None), ws), ((xs[0], bf(8, 1024)), ws), ((xs[0], xs[1].float()), ws),
+                      ((xs[0], bf(9, 1032)[:, :1024]), ws), ((xs[0], bf(9 * 1024 + 1)[1:].view(9, 1024)), ws), (xs, (ws[0], bf(1024, 32).t())), (xs, (ws[0], bf(28, 1024))),
+                      (xs, (ws[0], bf(32, 512))), (tuple(x[:0] for x in xs), ws), (tuple(x[:, :128] for x in xs), tuple(w[:, :128] for w in ws))):
+            assert module.gemm_slices(*other, 0, copies) is None and called() == []
+    many = tuple(bf(129, 1024) for _ in xs)
+    assert module.gemm_slices(many, ws, 0, None) is not None and called() and module.gemm_slices(many, ws, 0, packed) is None
+    for other in (bf(6, 16, 64, 8), bf(5, 32, 64, 8), packed.float()):
+        assert module.gemm_slices(xs, ws, 0, other) is None and called() == []

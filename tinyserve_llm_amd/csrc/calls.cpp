@@ -234,7 +234,57 @@ PyObject* gemm_library(Args a) {      // x, weight, 32-bit out -> y
   return wrap(y);
 }
 
-PyObject* gemm_slices(Args a) {      // x, weight, tile, slices, 32-bit out, residual, norm weight, eps -> y, or with a norm weight (norm, sum)
+bool packed16(const Tensor& p, int64_t K) {
+  return bf16(p) && p.dim() == 4 && p.size(1) * 32 == K && p.size(2) == 64 && p.size(3) == 8 && p.is_contiguous();
+}
+
+// The products of a group (`gemm_group` of ops/hip.py), 32 bits on their way out: by the kernel that streams W past x where `packed` is given (the copies
+// of all the weights one behind the other), else in whole tiles.
+PyObject* group(PyObject* xs, PyObject* ws, const Tensor* packed, int tile) {
+  constexpr Py_ssize_t most{8};
+  if (!PyTuple_Check(xs) || !PyTuple_Check(ws)) return none();
+  const Py_ssize_t n = PyTuple_GET_SIZE(xs);
+  if (n < 1 || n > most || PyTuple_GET_SIZE(ws) != n) return none();
+  const Tensor *x[most], *w[most];
+  const void *xp[most], *wp[most];
+  void* yp[most];
+  int widths[most];
+  int64_t N = 0;
+  for (Py_ssize_t i = 0; i < n; ++i) {
+    PyObject *px = PyTuple_GET_ITEM(xs, i), *pw = PyTuple_GET_ITEM(ws, i);
+    if (!THPVariable_Check(px) || !THPVariable_Check(pw)) return none();
+    x[i] = &THPVariable_Unpack(px), w[i] = &THPVariable_Unpack(pw);
+    if (!x[i]->is_cuda() || !w[i]->is_cuda() || w[i]->dim() != 2 || !bf16(*x[i]) || !bf16(*w[i]) || !pieces(*x[i]) || !pieces(*w[i])) return none();
+    if (x[i]->sizes() != x[0]->sizes() || x[i]->strides() != x[0]->strides() || w[i]->strides() != w[0]->strides()) return none();
+    if (w[i]->size(1) != x[0]->size(1) || w[i]->size(0) < 8 || w[i]->size(0) % 8 || !fits(w[i]->size(0))) return none();
+    widths[i] = w[i]->size(0), xp[i] = ptr(x[i]), wp[i] = ptr(w[i]), N += widths[i];
+  }
+  const int64_t M = x[0]->size(0), K = x[0]->size(1), ldx = x[0]->stride(0), ldw = w[0]->stride(0);
+  if (M < 1 || !fits(M) || !fits(K) || K % 64 || K < 192 || ldx < K || ldw < K || 512 * ldx >= 1LL << 31 || 512 * ldw >= 1LL << 31) return none();
+  if (packed) {
+    if (!packed16(*packed, K) || packed->size(0) * 16 != N || M > ROWS64_MAX_ROWS || K % 1024) return none();
+    for (Py_ssize_t i = 0; i < n; ++i)
+      if (widths[i] % 16) return none();
+  }
+  Tensor y[most];
+  for (Py_ssize_t i = 0; i < n; ++i) y[i] = make(*x[0], {M, widths[i]}, at::kFloat), yp[i] = ptr(&y[i]);
+  if (packed ? TS_REFUSED("gemm_rows64_group", ts_gemm_rows64_group_bf16(n, yp, xp, ptr(packed), widths, M, K, ldx, stream()))
+             : TS_REFUSED("gemm_whole", ts_gemm_whole_bf16(n, yp, xp, wp, widths, M, K, ldx, ldw, tile, 1, stream())))
+    return none();
+  PyObject* out = PyTuple_New(n);
+  for (Py_ssize_t i = 0; out && i < n; ++i) PyTuple_SET_ITEM(out, i, wrap(y[i]));
+  return out;
+}
+
+// x, weight, tile, slices, 32-bit out, residual, norm weight, eps -> y, or with a norm weight (norm, sum); or, with tuples of operands: operands,
+// weights, tile, packed copies -> the products of a `group`
+PyObject* gemm_slices(Args a) {
+  if (a.left == 4) {
+    PyObject *xs = a.next(), *ws = a.next();
+    const int tile = a.i32();
+    const Tensor* packed = a.maybe();
+    return a.done() ? group(xs, ws, packed, tile) : none();
+  }
   const Tensor *x = a.tensor(), *w = a.tensor();
   const int tile = a.i32(), slices = a.i32();
   const bool wide = a.i32();
@@ -270,9 +320,6 @@ PyObject* gemm_glu(Args a) {      // x, weight, tile, form's number, limit, slop
   return wrap(y);
 }
 
-bool packed16(const Tensor& p, int64_t K) {
-  return bf16(p) && p.dim() == 4 && p.size(1) * 32 == K && p.size(2) == 64 && p.size(3) == 8 && p.is_contiguous();
-}
 bool squares_fit(const Tensor* s, int64_t rows) { return !s || (f32(*s) && s->dim() == 2 && s->size(0) == rows && s->size(1) >= 1 && s->is_contiguous()); }
 
 PyObject* gemm_rows64(Args a) {      // x, packed, 32-bit out, unit's number (0: none), squares, eps, limit, slope, up_shift -> y

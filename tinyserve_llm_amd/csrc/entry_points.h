@@ -32,6 +32,8 @@ int ts_gemm_glu_bf16(void* y, const void* x, const void* w, int M, int F, int K,
                      float limit, float slope, float up_shift, hipStream_t stream);
 int ts_gemm_rows64_bf16(void* y, const void* x, const void* w16, int M, int N, int K, int64_t ldx, int64_t ldy, int glu, int out_f32,
                         const void* ssq_in, int ssq_parts, float eps, float limit, float slope, float up_shift, hipStream_t stream);
+int ts_gemm_rows64_group_bf16(int products, void* const* y, const void* const* x, const void* w16, const int* N, int M, int K, int64_t ldx,
+                              hipStream_t stream);
 int ts_gemm_rows64_sliced_bf16(void* y, void* parts, const void* x, const void* w16, int M, int N, int K, int64_t ldx, int slices,
                                const void* next_res, const void* next_nw, void* next_res_out, void* next_op, void* ssq_out, int64_t ld_op,
                                hipStream_t stream);

@@ -1889,14 +1889,19 @@ def gemm_group(xs: "Sequence[torch.Tensor]", weights: "Sequence[torch.Tensor]", 
     """float32 x · weight^T of several bfloat16 products of the same rows and reduction in one launch, where that is the faster way (`group_plan`); None
     where not, or where their operands are another way. `packed`: the `pack_weight` copies of all the weights, one behind the other, if they are kept."""
     x, w = xs[0], weights[0]
-    if _many_rows != "library" or x.dim() != 2 or not x.is_cuda or not all(
-            t.shape == x.shape and t.stride() == x.stride() and v.stride() == w.stride() and whole_takes(t, v) for t, v in zip(xs, weights)):
+    if _many_rows != "library" or x.dim() != 2 or not x.is_cuda:
         return None
     rows, k = x.shape
-    plan = group_plan(rows, tuple(v.shape[0] for v in weights), k, packed is not None)
+    widths = tuple([v.shape[0] for v in weights])
+    plan = group_plan(rows, widths, k, packed is not None)
     if rows == 0 or plan is None:
         return None
-    return gemm_rows64_group(xs, packed, [v.shape[0] for v in weights]) if plan < 0 else gemm_whole(xs, weights, plan, torch.float32)
+    done = _native().gemm_slices(tuple(xs), tuple(weights), plan, packed if plan < 0 else None)
+    if done is not None:
+        return done
+    if not all(t.shape == x.shape and t.stride() == x.stride() and v.stride() == w.stride() and whole_takes(t, v) for t, v in zip(xs, weights)):
+        return None
+    return gemm_rows64_group(xs, packed, widths) if plan < 0 else gemm_whole(xs, weights, plan, torch.float32)
 
 
 WHOLE_MIN_STEPS = 3      # steps of 64 that a tile's reduction has at least

@@ -30,6 +30,13 @@ template <> struct Num<bf16_t> {
   static __device__ __forceinline__ float round(float v) { return bf2f(f2bf(v)); }
 };
 
+// 16 bytes that one workgroup reads once and no other soon after (a weight's, a cache's): told so, the caches do not put other lines out for them.
+typedef uint32_t stream_u32x4_t __attribute__((ext_vector_type(4)));
+template <typename V = uint4> __device__ __forceinline__ V load_once(const void* p) {
+  static_assert(sizeof(V) == 16, "16 bytes");
+  return __builtin_bit_cast(V, __builtin_nontemporal_load((const stream_u32x4_t*)p));
+}
+
 // A kernel's arguments lie in memory that no cache holds when the kernel starts, and the compiler fetches them
 // as the code comes to need them: a long argument block is then waited for two or three times, a trip to
 // memory each, before the first load of the operands can go out. This asks for one word of each 64 bytes of

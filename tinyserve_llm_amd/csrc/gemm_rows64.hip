@@ -5,8 +5,8 @@
 // once per 32 rows of W, which is twice the bytes of W itself. Here a workgroup owns 64 rows of W and
 // splits the work between two kinds of wave:
 //   four compute waves, one 16-row tile of W each over the whole of K: the tile streams from memory
-//   straight into MFMA operands, 16 steps of 32 k under way at any time (a step's register is asked for
-//   again as soon as it has been used), and the four 16-row blocks of x come out of LDS;
+//   straight into MFMA operands, 8 steps of 32 k under way at any time (a step's register is asked for
+//   again as soon as it has been used), and the 16-row blocks of x come out of LDS;
 //   four staging waves, which bring x into LDS in chunks of 256 k, one chunk ahead of the compute waves
 //   (two buffers, a barrier per chunk). A staging wave takes a block of 16 rows, and each of its loads
 //   512 contiguous bytes of two rows (an instruction that gathered 64 bytes of each of 16 rows, the
@@ -14,7 +14,9 @@
 //   and 7.5 of 62 at the 8B widths); the pieces go into LDS where the compute lanes look for them, with
 //   the place inside a block of 16 rows turned by the piece's step and part of k so that neither the
 //   writes nor the reads meet in a bank. Their loads hit the cache; in waves of their own they do not
-//   queue behind the loads of W (a wave's loads come back in the order it asked).
+//   queue behind the loads of W (a wave's loads come back in the order it asked). They do wait behind what all waves have
+//   under way to the caches, and a chunk takes as long as they wait: so no more of W is under way than memory needs to be
+//   kept busy, and W goes by the caches (load_once), where it put out the lines of x that every other workgroup of the die reads.
 // The gate can ride along as in gemm_skinny.hip:
 //   GLU   W = [gate rows | up rows]: waves 0 and 1 take two gate tiles, waves 2 and 3 the up tiles
 //         N / 2 rows below them, and y [M, N / 2] = silu(gate) * up
@@ -36,8 +38,11 @@
 #include "skinny_ops.h"
 
 #define R64_CHUNK_STEPS 8         // 32-wide k steps per chunk of x in LDS
-#define R64_RING 16               // steps of W a compute wave has under way (two chunks): with 32 the chip had 32 MB under way and
-                                  // every load, x's among them, came back some 5 us later (the gate|up product of 64 rows 20.7 us, 19.7 with 16)
+#define R64_RING 8                // steps of W a compute wave has under way (a chunk). With them, W by the caches and 2 or 6 blocks of x where 4 or 8 were
+                                  // taken, against 16 steps through the caches, us: gate|up of 16,384 x 2,048, 32 rows 13.6 and 16.7, 64 rows
+                                  // 15.0 and 17.7, 90 rows 16.8 and 21.1, 128 rows 20.6 and 23.1; a head of 128,256 x 2,048, 64 rows 100.8 and 110.2;
+                                  // in slices, with the finishing kernel, 2,048 x 8,192, 32 rows 12.6 and 14.0, 64 rows 14.0 and 14.8, 90 rows 15.6 and
+                                  // 17.5, 3,072 x 3,072, 90 rows 16.6 and 19.9. (The ring alone 0.2 to 1.5 of it, the blocks 0.5 to 1.5, the caches the rest.)
 #define R64_STRETCH 4             // steps whose products a group's sums take together
 #define R64_STAGE_LOADS 8          // loads of a staging wave per chunk: two rows of its block each
 
@@ -66,8 +71,8 @@ struct Rows64GroupArgs : Rows64Args {
   float* ys[R64_PRODUCTS];             // [M, width]
 };
 
-// BLOCKS: blocks of 16 rows of x, 4 (up to 64 rows) or 8 (up to 128: the compute waves then take a chunk's
-// steps one at a time instead of in pairs, for their registers' sake).
+// BLOCKS: blocks of 16 rows of x, 2, 4, 6 or 8 (beyond 64 rows the compute waves take a chunk's steps one at a time
+// instead of in pairs, for their registers' sake).
 // GLU: 0 none, 1 silu(gate) up, 1 + f the unit of form f of glu_unit.h.
 // With a group's arguments the sums are added up in stretches of 128 of K, with up to 64 rows in pairs of them, so that they are as near to 64 bits as
 // those of the kernels for a product of its own, which share a reduction out to their waves (over 2,048: 0.9e-7 up to 8 rows, 1.0e-7 up to 32, 1.3e-7 up to
@@ -98,15 +103,15 @@ __global__ void __launch_bounds__(512) gemm_rows64_kernel(const ARGS a) {
     // ---- staging waves: wave sw brings block sw of 16 rows, all the steps of every chunk. It asks for
     // the next chunk before it puts this one into LDS, so that a chunk costs the compute waves a barrier
     // and not a trip to the cache.
-    const int sw = wave - 4;                              // this wave's blocks of 16 rows: sw BLOCKS / 4 ..
-    constexpr int MINE = BLOCKS / 4, LOADS = R64_STAGE_LOADS * MINE;
+    const int sw = wave - 4;                              // this wave's quarter of the rows
+    constexpr int LOADS = R64_STAGE_LOADS * BLOCKS / 4;
     const int half = lane >> 5, kl = lane & 31;           // the row of a load's two, and the piece of its 256 k
     bool ok[LOADS];
     int64_t xoff[LOADS];
     int slot[LOADS];
 #pragma unroll
     for (int j = 0; j < LOADS; ++j) {
-      const int block = sw * MINE + j / R64_STAGE_LOADS, r = 2 * (j % R64_STAGE_LOADS) + half, m = 16 * block + r;
+      const int block = (sw * LOADS + j) / R64_STAGE_LOADS, r = 2 * ((sw * LOADS + j) % R64_STAGE_LOADS) + half, m = 16 * block + r;
       ok[j] = m < a.M;                                    // rows past M read row 0 and count as zeros
       xoff[j] = (int64_t)(ok[j] ? m : 0) * a.ldx + kfirst + 8 * kl;
       slot[j] = ((kl >> 2) * BLOCKS + block) * TS_WAVE + sk_place(r, kl >> 2, kl & 3);      // in a buffer's [step][block][64]
@@ -149,13 +154,13 @@ __global__ void __launch_bounds__(512) gemm_rows64_kernel(const ARGS a) {
   // compiler sees the first loads come in the order of their use)
 #pragma unroll
   for (int s = 0; s < R64_RING; ++s) {
-    wr[s] = *(const uint4*)(wp + (int64_t)s * 512);
+    wr[s] = load_once(wp + (int64_t)s * 512);
     __builtin_amdgcn_sched_barrier(0);
   }
   float4_t acc[BLOCKS];
 #pragma unroll
   for (int b = 0; b < BLOCKS; ++b) acc[b] = (float4_t){0.f, 0.f, 0.f, 0.f};
-  constexpr bool PAIRS = BLOCKS == 4;                    // (more rows have no registers for it, and were the library's, which has no stretches)
+  constexpr bool PAIRS = BLOCKS <= 4;                    // (more rows have no registers for it, and were the library's, which has no stretches)
   float4_t total[GROUP ? BLOCKS : 1], held[GROUP && PAIRS ? BLOCKS : 1];
   if constexpr (GROUP) {
 #pragma unroll
@@ -190,7 +195,7 @@ __global__ void __launch_bounds__(512) gemm_rows64_kernel(const ARGS a) {
       // a chunk in batches of steps (pairs; single steps with 8 blocks of x): the next batch's operands leave
       // LDS while this batch's products run (left to itself the compiler reads two operands, waits,
       // multiplies, and so on)
-      constexpr int PER = BLOCKS == 4 ? 2 : 1, BATCHES = R64_CHUNK_STEPS / PER;
+      constexpr int PER = BLOCKS <= 4 ? 2 : 1, BATCHES = R64_CHUNK_STEPS / PER;
       const int buf = (base / R64_CHUNK_STEPS + h) & 1;
       uint4 xb[2][PER][BLOCKS];
 #pragma unroll
@@ -221,7 +226,7 @@ __global__ void __launch_bounds__(512) gemm_rows64_kernel(const ARGS a) {
               }
             }
           }
-          if (decltype(more)::value) wr[sl] = *(const uint4*)(wp + (int64_t)(base + R64_RING + sl) * 512);
+          if (decltype(more)::value) wr[sl] = load_once(wp + (int64_t)(base + R64_RING + sl) * 512);
         }
         __builtin_amdgcn_sched_barrier(0);
       }
@@ -270,12 +275,19 @@ __global__ void __launch_bounds__(512) gemm_rows64_kernel(const ARGS a) {
 
 #define R64_MAX_ROWS 128
 
+// Blocks of 16 rows of x that a workgroup takes; two buffers of a chunk of them in LDS.
+static int r64_blocks(int M) { return M <= 32 ? 2 : M <= 64 ? 4 : M <= 96 ? 6 : 8; }
+static size_t r64_lds(int blocks) { return 2 * R64_CHUNK_STEPS * blocks * TS_WAVE * sizeof(uint4); }
+
 template <int GLU, typename OUT>
 static int r64_launch(const Rows64Args& a, hipStream_t stream) {
-  // 64 rows of W per workgroup; two buffers of a chunk of x in LDS: 64 KB for up to 64 rows, 128 KB beyond
   const dim3 grid(a.N / 64, a.slices);
-  if (a.M <= 64) gemm_rows64_kernel<GLU, OUT, 4, Rows64Args><<<grid, 512, 2 * R64_CHUNK_STEPS * 4 * TS_WAVE * sizeof(uint4), stream>>>(a);
-  else gemm_rows64_kernel<GLU, OUT, 8, Rows64Args><<<grid, 512, 2 * R64_CHUNK_STEPS * 8 * TS_WAVE * sizeof(uint4), stream>>>(a);
+  switch (r64_blocks(a.M)) {
+    case 2: gemm_rows64_kernel<GLU, OUT, 2, Rows64Args><<<grid, 512, r64_lds(2), stream>>>(a); break;
+    case 4: gemm_rows64_kernel<GLU, OUT, 4, Rows64Args><<<grid, 512, r64_lds(4), stream>>>(a); break;
+    case 6: gemm_rows64_kernel<GLU, OUT, 6, Rows64Args><<<grid, 512, r64_lds(6), stream>>>(a); break;
+    default: gemm_rows64_kernel<GLU, OUT, 8, Rows64Args><<<grid, 512, r64_lds(8), stream>>>(a);
+  }
   return ts_check_launch();
 }
 
@@ -322,8 +334,12 @@ extern "C" int ts_gemm_rows64_group_bf16(int products, void* const* y, const voi
     groups += (N[i] + 63) / 64, tiles += N[i] / 16;
     if (tiles > (1 << 24)) return TS_TOO_LARGE;
   }
-  if (M <= 64) gemm_rows64_kernel<0, float, 4, Rows64GroupArgs><<<(unsigned)groups, 512, 2 * R64_CHUNK_STEPS * 4 * TS_WAVE * sizeof(uint4), stream>>>(a);
-  else gemm_rows64_kernel<0, float, 8, Rows64GroupArgs><<<(unsigned)groups, 512, 2 * R64_CHUNK_STEPS * 8 * TS_WAVE * sizeof(uint4), stream>>>(a);
+  switch (r64_blocks(M)) {
+    case 2: gemm_rows64_kernel<0, float, 2, Rows64GroupArgs><<<(unsigned)groups, 512, r64_lds(2), stream>>>(a); break;
+    case 4: gemm_rows64_kernel<0, float, 4, Rows64GroupArgs><<<(unsigned)groups, 512, r64_lds(4), stream>>>(a); break;
+    case 6: gemm_rows64_kernel<0, float, 6, Rows64GroupArgs><<<(unsigned)groups, 512, r64_lds(6), stream>>>(a); break;
+    default: gemm_rows64_kernel<0, float, 8, Rows64GroupArgs><<<(unsigned)groups, 512, r64_lds(8), stream>>>(a);
+  }
   return ts_check_launch();
 }
 

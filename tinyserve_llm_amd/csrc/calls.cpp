@@ -322,20 +322,24 @@ PyObject* gemm_glu(Args a) {      // x, weight, tile, form's number, limit, slop
 
 bool squares_fit(const Tensor* s, int64_t rows) { return !s || (f32(*s) && s->dim() == 2 && s->size(0) == rows && s->size(1) >= 1 && s->is_contiguous()); }
 
-PyObject* gemm_rows64(Args a) {      // x, packed, 32-bit out, unit's number (0: none), squares, eps, limit, slope, up_shift -> y
+PyObject* gemm_rows64(Args a) {      // x, packed, 32-bit out, unit's number (0: none), squares, eps, limit, slope, up_shift, `few` of the launcher if it is there -> y
   const Tensor *x = a.tensor(), *p = a.tensor();
   const bool wide = a.i32();
   const int unit = a.i32();
   const Tensor* sq = a.maybe();
   const float eps = a.number(), limit = a.number(), slope = a.number(), shift = a.number();
+  const int few = a.left ? a.i32() : 0, steps = few > 1 ? few : 0;
   if (!a.done() || x->dim() != 2 || !bf16(*x) || !pieces(*x) || !packed16(*p, x->size(1)) || (unit && wide) || (unit > 1 && sq)) return none();
   const int64_t M = x->size(0), K = x->size(1), N = p->size(0) * 16;
   if (M < 1 || M > ROWS64_MAX_ROWS || N % (unit ? 128 : 64) || K % 1024 || !squares_fit(sq, M) || !fits(N) || !fits(K)) return none();
+  if (steps && (!unit || M > 8 || (steps != 4 && steps != 8 && steps != 16) || N / 2 % (64 * steps))) return none();
   const int64_t skew = M >= GATED_SKEW_MIN_ROWS ? ROW_SKEW : 0;
-  Tensor y = unit ? make_rows(*x, M, N / 2, skew) : make(*x, {M, N}, wide ? at::kFloat : at::kBFloat16);
+  Tensor y = steps  ? make(*x, {N / 2 / (64 * steps), steps, 64, 8}, at::kBFloat16)
+             : unit ? make_rows(*x, M, N / 2, skew)
+                    : make(*x, {M, N}, wide ? at::kFloat : at::kBFloat16);
   if (TS_REFUSED("gemm_rows64",
-                 ts_gemm_rows64_bf16(ptr(&y), ptr(x), ptr(p), M, N, K, x->stride(0), y.stride(0), unit, wide, ptr(sq), sq ? sq->size(1) : 0, eps, limit, slope,
-                                     shift, stream())))
+                 ts_gemm_rows64_bf16(ptr(&y), ptr(x), ptr(p), M, N, K, x->stride(0), steps ? N / 2 : y.stride(0), unit, wide, ptr(sq), sq ? sq->size(1) : 0,
+                                     eps, limit, slope, shift, few, stream())))
     return none();
   return wrap(y);
 }

@@ -31,7 +31,7 @@ int ts_gemm_whole_rope_bf16(void* q_out, const void* x, const void* w, int M, in
 int ts_gemm_glu_bf16(void* y, const void* x, const void* w, int M, int F, int K, int64_t ldx, int64_t ldw, int64_t ldy, int tile, int act,
                      float limit, float slope, float up_shift, hipStream_t stream);
 int ts_gemm_rows64_bf16(void* y, const void* x, const void* w16, int M, int N, int K, int64_t ldx, int64_t ldy, int glu, int out_f32,
-                        const void* ssq_in, int ssq_parts, float eps, float limit, float slope, float up_shift, hipStream_t stream);
+                        const void* ssq_in, int ssq_parts, float eps, float limit, float slope, float up_shift, int few, hipStream_t stream);
 int ts_gemm_rows64_group_bf16(int products, void* const* y, const void* const* x, const void* w16, const int* N, int M, int K, int64_t ldx,
                               hipStream_t stream);
 int ts_gemm_rows64_sliced_bf16(void* y, void* parts, const void* x, const void* w16, int M, int N, int K, int64_t ldx, int slices,

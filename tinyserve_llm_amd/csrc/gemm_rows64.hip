@@ -1,4 +1,4 @@
-// y[M, N] = e(f(x)[M, K] · W[N, K]^T) in bfloat16 for 17 to 128 rows of x and a wide W (the gate|up
+// y[M, N] = e(f(x)[M, K] · W[N, K]^T) in bfloat16 for 5 to 128 rows of x and a wide W (the gate|up
 // projection of a decode step of a few dozen requests), where time should go to reading W once.
 //
 // With so many rows the weight-streaming kernel of gemm_skinny.hip reads x from the second-level cache
@@ -22,6 +22,10 @@
 //         N / 2 rows below them, and y [M, N / 2] = silu(gate) * up
 // (The norm on the way in, which every workgroup would have to repeat for all of x, was tried in the
 // staging waves and costs more than the norm kernel it saves: 37 µs against 21 + 7 at 64 rows.)
+// Up to 32 rows (FEW) it serves a wide W, in the weight-streaming kernels' place, whose waves each load their own x for 16 to 64 rows of W, ask for
+// all of their W at once and then wait for all of it: 128,256 x 2,048, 8 rows 90 us there and 83 here, 16 rows 103 and 86, 32 rows 127 and 91;
+// 12,288 x 2,048, 5 rows 13.2 and 11.2; the gate of 16,384 x 2,048, 8 rows 14.8 and 13.4 (hip.rows64_few has more).
+//
 // W comes as the 16-row packed copy ([N / 16 tiles][K / 32 steps][64 lanes][8]); K is a multiple of
 // 1,024. A row of x meets W's k in ascending order in one accumulator, whatever the other rows are.
 //
@@ -60,6 +64,8 @@ struct Rows64Args {
   float eps;
   float limit, slope, up_shift;      // of the unit (GLU > 1)
   int slices;            // the reduction in this many slices (gridDim.y); more than one: y is float [slices][M][ldy]
+  int few;               // up to 32 rows whose sums are added up as the 16-row weight-streaming form does; more than 1: a gated product of up to 8 rows in
+                         // the order of a reader of so many steps (SkinnyArgs::x_packed8 of gemm_skinny.hip)
 };
 
 // Several products of the same rows and reduction in one launch, each with its x and its 32-bit y, their packed copies one behind the other:
@@ -79,13 +85,18 @@ struct Rows64GroupArgs : Rows64Args {
 // 64, the library's beyond 2.7e-7). A product of a few million numbers of W is a launch, a trip of x to LDS and as few workgroups as it has columns for
 // 64 each: five of them (2,048 columns four times and 64, K 2,048) took 18 us apart and take 10.5 here with 1 row, 20 and 10.7 with 8, 28 and 11.3 with
 // 32, 50 and 11.8 with 48.
-template <int GLU, typename OUT, int BLOCKS, typename ARGS>
+// FEW (up to 32 rows): a chunk's products are summed, then the chunks in ascending order: what a wave of the 16-row form makes of its share of
+// K and what becomes of the waves' sums, so that a product has the bits of that form, whichever of the two makes it.
+template <int GLU, typename OUT, int BLOCKS, typename ARGS, bool FEW = false>
 __global__ void __launch_bounds__(512) gemm_rows64_kernel(const ARGS a) {
   constexpr bool GROUP = std::is_same_v<ARGS, Rows64GroupArgs>;
+  constexpr bool SUMS = GROUP || FEW;
+  static_assert(!FEW || (!GROUP && BLOCKS <= 2), "few rows");
   static_assert(!GROUP || (GLU == 0 && std::is_same_v<OUT, float>), "products of a group are plain and 32-bit");
   // x as the B operands of the matrix instruction: [buffer][step][block of 16 rows][lane], lane r + 16 g
   // holding k = 8 g .. 8 g + 7 of row r (turned: sk_place)
   extern __shared__ __align__(16) uint4 xs_all[];
+  __shared__ float scale_s[FEW ? 16 * BLOCKS : 1];
   auto xs = [&](int buf, int step, int b) { return xs_all + (((size_t)buf * R64_CHUNK_STEPS + step) * BLOCKS + b) * TS_WAVE; };
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / TS_WAVE), lane = threadIdx.x & (TS_WAVE - 1);
   const int r = lane & 15, g = lane >> 4;
@@ -128,7 +139,38 @@ __global__ void __launch_bounds__(512) gemm_rows64_kernel(const ARGS a) {
     };
     uint4 A[LOADS], B[LOADS];
     ask(0, A);
+    // The parts of few rows' sums of squares: a lane takes every 64th, the lanes meet in a fixed tree. The first 256 parts are asked for here,
+    // behind the first chunk; they are added up while the compute waves have a chunk to go through.
+    constexpr int ROWS = FEW ? 4 * BLOCKS : 1, EARLY = 4;
+    const bool parts = FEW && a.ssq_in && a.ssq_parts > 1;
+    float early[ROWS][EARLY];
+    if (parts) {
+#pragma unroll
+      for (int i = 0; i < ROWS; ++i) {
+        const int m = min(sw * ROWS + i, a.M - 1);
+#pragma unroll
+        for (int q = 0; q < EARLY; ++q) early[i][q] = a.ssq_in[(int64_t)m * a.ssq_parts + min(lane + 64 * q, a.ssq_parts - 1)];
+      }
+    }
     for (int c = 0; c < nchunks; c += 2) {
+      if (parts && c + 2 >= nchunks) {
+        float sum[ROWS];
+#pragma unroll
+        for (int i = 0; i < ROWS; ++i) {
+          const int m = min(sw * ROWS + i, a.M - 1);
+          sum[i] = 0.f;
+#pragma unroll
+          for (int q = 0; q < EARLY; ++q) sum[i] += lane + 64 * q < a.ssq_parts ? early[i][q] : 0.f;
+          for (int q = lane + 64 * EARLY; q < a.ssq_parts; q += TS_WAVE) sum[i] += a.ssq_in[(int64_t)m * a.ssq_parts + q];
+        }
+#pragma unroll
+        for (int off = TS_WAVE / 2; off > 0; off >>= 1)
+#pragma unroll
+          for (int i = 0; i < ROWS; ++i) sum[i] += __shfl_xor(sum[i], off, TS_WAVE);
+#pragma unroll
+        for (int i = 0; i < ROWS; ++i)
+          if (lane == i) scale_s[sw * ROWS + i] = 1.0f / sqrtf(sum[i] / (float)a.K + a.eps);
+      }
       ask(c + 1, B);
       put(c, A);
       __syncthreads();          // chunk c is there (and chunk c - 1 has been used: its buffer is the next one's)
@@ -160,9 +202,10 @@ __global__ void __launch_bounds__(512) gemm_rows64_kernel(const ARGS a) {
   float4_t acc[BLOCKS];
 #pragma unroll
   for (int b = 0; b < BLOCKS; ++b) acc[b] = (float4_t){0.f, 0.f, 0.f, 0.f};
-  constexpr bool PAIRS = BLOCKS <= 4;                    // (more rows have no registers for it, and were the library's, which has no stretches)
-  float4_t total[GROUP ? BLOCKS : 1], held[GROUP && PAIRS ? BLOCKS : 1];
-  if constexpr (GROUP) {
+  constexpr int STRETCH = GROUP ? R64_STRETCH : R64_CHUNK_STEPS;
+  constexpr bool PAIRS = GROUP && BLOCKS <= 4;           // (more rows have no registers for it, and were the library's, which has no stretches)
+  float4_t total[SUMS ? BLOCKS : 1], held[PAIRS ? BLOCKS : 1];
+  if constexpr (SUMS) {
 #pragma unroll
     for (int b = 0; b < BLOCKS; ++b) total[b] = (float4_t){0.f, 0.f, 0.f, 0.f};
   }
@@ -175,7 +218,7 @@ __global__ void __launch_bounds__(512) gemm_rows64_kernel(const ARGS a) {
   float scale[BLOCKS];
 #pragma unroll
   for (int b = 0; b < BLOCKS; ++b) scale[b] = 1.f;
-  if (a.ssq_in) {
+  if (a.ssq_in && (!FEW || a.ssq_parts == 1)) {
 #pragma unroll
     for (int b = 0; b < BLOCKS; ++b) {
       const int m = 16 * b + r;
@@ -214,16 +257,18 @@ __global__ void __launch_bounds__(512) gemm_rows64_kernel(const ARGS a) {
 #pragma unroll
         for (int i = 0; i < PER; ++i) {
           const int sl = R64_CHUNK_STEPS * h + PER * q + i;
+          if (FEW && sl % STRETCH == 0) {              // (the last stretch's sums, which are there by now)
 #pragma unroll
-          for (int b = 0; b < BLOCKS; ++b) acc[b] = sk_mfma(wr[sl], xb[q & 1][i][b], GROUP && sl % R64_STRETCH == 0 ? (float4_t){0.f, 0.f, 0.f, 0.f} : acc[b]);
-          if constexpr (GROUP) {
-            if (sl % R64_STRETCH == R64_STRETCH - 1) {
+            for (int b = 0; b < BLOCKS; ++b) total[b] += acc[b];
+          }
 #pragma unroll
-              for (int b = 0; b < BLOCKS; ++b) {
-                if (!PAIRS) total[b] += acc[b];
-                else if (sl % (2 * R64_STRETCH) < R64_STRETCH) held[b] = acc[b];
-                else total[b] += held[b] + acc[b];
-              }
+          for (int b = 0; b < BLOCKS; ++b) acc[b] = sk_mfma(wr[sl], xb[q & 1][i][b], SUMS && sl % STRETCH == 0 ? (float4_t){0.f, 0.f, 0.f, 0.f} : acc[b]);
+          if (GROUP && sl % STRETCH == STRETCH - 1) {
+#pragma unroll
+            for (int b = 0; b < BLOCKS; ++b) {
+              if (!PAIRS) total[b] += acc[b];
+              else if (sl % (2 * STRETCH) < STRETCH) held[b] = acc[b];
+              else total[b] += held[b] + acc[b];
             }
           }
           if (decltype(more)::value) wr[sl] = load_once(wp + (int64_t)(base + R64_RING + sl) * 512);
@@ -236,7 +281,11 @@ __global__ void __launch_bounds__(512) gemm_rows64_kernel(const ARGS a) {
   int base = 0;
   for (; base + R64_RING < nsteps; base += R64_RING) ring(base, std::true_type{});
   ring(base, std::false_type{});
-  // acc[b][j] = sum over k of W[row 16 tile + 4 g + j, k] * x[16 b + r, k]
+  if constexpr (FEW) {
+#pragma unroll
+    for (int b = 0; b < BLOCKS; ++b) acc[b] = total[b] + acc[b];
+  }
+  // acc[b][j] (of a group total[b][j]) = sum over k of W[row 16 tile + 4 g + j, k] * x[16 b + r, k]
   if constexpr (GROUP) {
     float* const to = a.ys[which] + column + 4 * g;
 #pragma unroll
@@ -255,20 +304,35 @@ __global__ void __launch_bounds__(512) gemm_rows64_kernel(const ARGS a) {
   }
   OUT* y = (OUT*)a.y + (int64_t)slice * a.M * a.ldy;
   const int n0 = GLU ? (2 * blockIdx.x + wave) * 16 + 4 * g : tile * 16 + 4 * g;
+  const bool whole = FEW && a.ldy % 4 == 0 && !(((uintptr_t)a.y) & (4 * sizeof(OUT) - 1));      // a lane's four columns in one store (more rows gain nothing by it)
 #pragma unroll
   for (int b = 0; b < BLOCKS; ++b) {
     const int m = 16 * b + r;
     if (m >= a.M) continue;
-    float4_t u = {0.f, 0.f, 0.f, 0.f};
+    float4_t v = acc[b], u = {0.f, 0.f, 0.f, 0.f};
     if (GLU) u = ex[(wave * BLOCKS + b) * TS_WAVE + lane];
-    acc[b] *= scale[b];
-    u *= scale[b];
+    const float by = FEW && a.ssq_in && a.ssq_parts > 1 ? scale_s[m] : scale[b];
+    v *= by;
+    u *= by;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      float v = acc[b][j];
-      if constexpr (GLU == 1) v = sk_silu(v) * u[j];
-      if constexpr (GLU > 1) v = glu_capped(GLU - 1, v, u[j], a.limit, a.slope, a.up_shift);
-      Num<OUT>::st(y + (int64_t)m * a.ldy + n0 + j, v);
+      if constexpr (GLU == 1) v[j] = sk_silu(v[j]) * u[j];
+      if constexpr (GLU > 1) v[j] = glu_capped(GLU - 1, v[j], u[j], a.limit, a.slope, a.up_shift);
+    }
+    OUT* to = y + (int64_t)m * a.ldy + n0;
+    if constexpr (GLU && FEW && BLOCKS == 1) {
+      if (a.few > 1) {      // (the four columns are four neighbouring k of the reader's lane; the host has checked the widths)
+        const int S = a.few, w = n0 / (64 * S), in_wave = n0 - w * 64 * S, hf = in_wave / (32 * S), in_half = in_wave - hf * 32 * S;
+        to = y + (((int64_t)w * S + (in_half >> 5)) * 64 + m + 8 * hf + 16 * ((in_half & 31) >> 3)) * 8 + (n0 & 7);
+      }
+    }
+    if (!whole) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) Num<OUT>::st(to + j, v[j]);
+    } else if constexpr (sizeof(OUT) == 4) {
+      *(float4_t*)to = v;
+    } else {
+      *(uint2*)to = make_uint2(f2bf(v[0]) | ((uint32_t)f2bf(v[1]) << 16), f2bf(v[2]) | ((uint32_t)f2bf(v[3]) << 16));
     }
   }
 }
@@ -276,13 +340,19 @@ __global__ void __launch_bounds__(512) gemm_rows64_kernel(const ARGS a) {
 #define R64_MAX_ROWS 128
 
 // Blocks of 16 rows of x that a workgroup takes; two buffers of a chunk of them in LDS.
-static int r64_blocks(int M) { return M <= 32 ? 2 : M <= 64 ? 4 : M <= 96 ? 6 : 8; }
+static int r64_blocks(int M) { return M <= 16 ? 1 : M <= 32 ? 2 : M <= 64 ? 4 : M <= 96 ? 6 : 8; }
 static size_t r64_lds(int blocks) { return 2 * R64_CHUNK_STEPS * blocks * TS_WAVE * sizeof(uint4); }
 
 template <int GLU, typename OUT>
 static int r64_launch(const Rows64Args& a, hipStream_t stream) {
   const dim3 grid(a.N / 64, a.slices);
+  if (a.few) {
+    if (a.M <= 16) gemm_rows64_kernel<GLU, OUT, 1, Rows64Args, true><<<grid, 512, r64_lds(1), stream>>>(a);
+    else gemm_rows64_kernel<GLU, OUT, 2, Rows64Args, true><<<grid, 512, r64_lds(2), stream>>>(a);
+    return ts_check_launch();
+  }
   switch (r64_blocks(a.M)) {
+    case 1: gemm_rows64_kernel<GLU, OUT, 1, Rows64Args><<<grid, 512, r64_lds(1), stream>>>(a); break;
     case 2: gemm_rows64_kernel<GLU, OUT, 2, Rows64Args><<<grid, 512, r64_lds(2), stream>>>(a); break;
     case 4: gemm_rows64_kernel<GLU, OUT, 4, Rows64Args><<<grid, 512, r64_lds(4), stream>>>(a); break;
     case 6: gemm_rows64_kernel<GLU, OUT, 6, Rows64Args><<<grid, 512, r64_lds(6), stream>>>(a); break;
@@ -299,16 +369,19 @@ static bool r64_operands_ok(const void* x, const void* w16, int M, int N, int K,
 // x [M <= 128, K] (row stride ldx), w16: W [N, K] as its 16-row packed copy, y [M, N] or, with glu, [M, N / 2]
 // (row stride ldy; out_f32: 32-bit sums instead of bfloat16). N a multiple of 64 (128 with glu), K of 1,024.
 // ssq_in [M, ssq_parts] and eps: the prepared norm's scale per row (null: none). glu: 1 silu(gate) up, 1 + f the unit of form f
-// of glu_unit.h with limit, slope and up_shift.
+// of glu_unit.h with limit, slope and up_shift. few: 0, or up to 32 rows added up as the 16-row form does;
+// 4, 8 or 16 (glu, M <= 8, N / 2 a multiple of 64 few): y is the gated product in the order the 8-row form of so many steps reads its x.
 extern "C" int ts_gemm_rows64_bf16(void* y, const void* x, const void* w16, int M, int N, int K, int64_t ldx, int64_t ldy,
                                    int glu, int out_f32, const void* ssq_in, int ssq_parts, float eps, float limit, float slope,
-                                   float up_shift, hipStream_t stream) {
+                                   float up_shift, int few, hipStream_t stream) {
   if (M <= 0 || N <= 0) return TS_OK;
   if (N % (glu ? 128 : 64) || K % 1024 || !y || !r64_operands_ok(x, w16, M, N, K, ldx)) return TS_BAD_SHAPE;
   if (ldy < (glu ? N / 2 : N) || (((uintptr_t)y) & (out_f32 ? 3 : 1))) return TS_BAD_SHAPE;
   if (glu && out_f32) return TS_BAD_SHAPE;
+  if (few < 0 || (few && M > 32)) return TS_BAD_SHAPE;
+  if (few > 1 && (!glu || M > 8 || (few != 4 && few != 8 && few != 16) || (N / 2) % (64 * few) || (((uintptr_t)y) & 7))) return TS_BAD_SHAPE;
   if (ssq_in && (ssq_parts <= 0 || (((uintptr_t)ssq_in) & 3))) return TS_BAD_SHAPE;
-  Rows64Args a = {(const bf16_t*)x, (const bf16_t*)w16, y, M, N, K, ldx, ldy, (const float*)ssq_in, ssq_parts, eps, limit, slope, up_shift, 1};
+  Rows64Args a = {(const bf16_t*)x, (const bf16_t*)w16, y, M, N, K, ldx, ldy, (const float*)ssq_in, ssq_parts, eps, limit, slope, up_shift, 1, few};
   switch (glu) {
     case 0: return out_f32 ? r64_launch<0, float>(a, stream) : r64_launch<0, bf16_t>(a, stream);
     case 1: return r64_launch<1, bf16_t>(a, stream);
@@ -335,6 +408,7 @@ extern "C" int ts_gemm_rows64_group_bf16(int products, void* const* y, const voi
     if (tiles > (1 << 24)) return TS_TOO_LARGE;
   }
   switch (r64_blocks(M)) {
+    case 1: gemm_rows64_kernel<0, float, 1, Rows64GroupArgs><<<(unsigned)groups, 512, r64_lds(1), stream>>>(a); break;
     case 2: gemm_rows64_kernel<0, float, 2, Rows64GroupArgs><<<(unsigned)groups, 512, r64_lds(2), stream>>>(a); break;
     case 4: gemm_rows64_kernel<0, float, 4, Rows64GroupArgs><<<(unsigned)groups, 512, r64_lds(4), stream>>>(a); break;
     case 6: gemm_rows64_kernel<0, float, 6, Rows64GroupArgs><<<(unsigned)groups, 512, r64_lds(6), stream>>>(a); break;
@@ -437,7 +511,7 @@ extern "C" int ts_gemm_rows64_sliced_bf16(void* y, void* parts, const void* x, c
   } else if (!y || (((uintptr_t)y) & 7)) {
     return TS_BAD_SHAPE;
   }
-  Rows64Args a = {(const bf16_t*)x, (const bf16_t*)w16, parts, M, N, K, ldx, (int64_t)N, nullptr, 0, 0.f, 0.f, 0.f, 0.f, slices};
+  Rows64Args a = {(const bf16_t*)x, (const bf16_t*)w16, parts, M, N, K, ldx, (int64_t)N, nullptr, 0, 0.f, 0.f, 0.f, 0.f, slices, 0};
   const int rc = r64_launch<0, float>(a, stream);
   if (rc != TS_OK) return rc;
   const int threads = N / 4 >= R64_FINISH_THREADS ? R64_FINISH_THREADS : (N / 4 + TS_WAVE - 1) / TS_WAVE * TS_WAVE;
@@ -571,7 +645,7 @@ extern "C" int ts_gemm_rows64_sliced_rope_bf16(void* q_out, void* parts, const v
   if (ssq_in && (ssq_parts <= 0 || (((uintptr_t)ssq_in) & 3))) return TS_BAD_SHAPE;
   if (rotate && (!cos_sin || !positions)) return TS_BAD_SHAPE;
   if (k_cache && (!v_cache || !slots || (kp % 4) || (ks % 4) || (kh % 4) || (((uintptr_t)k_cache) & 7))) return TS_BAD_SHAPE;
-  Rows64Args a = {(const bf16_t*)x, (const bf16_t*)w16, parts, M, N, K, ldx, (int64_t)N, nullptr, 0, 0.f, 0.f, 0.f, 0.f, slices};
+  Rows64Args a = {(const bf16_t*)x, (const bf16_t*)w16, parts, M, N, K, ldx, (int64_t)N, nullptr, 0, 0.f, 0.f, 0.f, 0.f, slices, 0};
   const int rc = r64_launch<0, float>(a, stream);
   if (rc != TS_OK) return rc;
   Rows64RopeArgs f = {(const float*)parts, slices, M, N, K, (const float*)ssq_in, ssq_parts, eps, cos_sin, positions, slots,

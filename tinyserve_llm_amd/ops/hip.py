@@ -93,7 +93,7 @@ def _declare(lib: ctypes.CDLL) -> None:
         "ts_gemm_slices_bf16": [p, p, p, p, p, i, i, i, i64, i64, i, i, i, p, p, f, p],
         "ts_gemm_whole_bf16": [i, p, p, p, p, i, i, i64, i64, i, i, p],
         "ts_gemm_whole_rope_bf16": [p, p, p, i, i, i64, i64, p, p, p, p, p, i, i, i, i, i64, i64, i64, i64, i64, i64, i64, i, p],
-        "ts_gemm_rows64_bf16": [p, p, p, i, i, i, i64, i64, i, i, p, i, f, f, f, f, p],
+        "ts_gemm_rows64_bf16": [p, p, p, i, i, i, i64, i64, i, i, p, i, f, f, f, f, i, p],
         "ts_gemm_rows64_group_bf16": [i, p, p, p, p, i, i, i64, p],
         "ts_gemm_rows64_sliced_bf16": [p, p, p, p, i, i, i, i64, i, p, p, p, p, p, i64, p],
         "ts_gemm_rows64_sliced_rope_bf16": [p, p, p, p, i, i, i64, i, p, i, f, p, p, p, p, p, i, i, i, i, i, i64, i64, i64, i64, i64,
@@ -1286,8 +1286,7 @@ def gemm_skinny(x: torch.Tensor, weight: torch.Tensor, out_dtype: torch.dtype = 
     return (PackedRows8(out, M, N // 2, pack8_steps) if pack8_steps else out), res_out
 
 
-ROWS64_MIN_ROWS = 33         # fewer rows are the weight-streaming kernel's (gemm_skinny: 32 rows 16.6 µs against 17.7 here,
-                             # 48 rows 23.7 against 19.3, 64 rows 26.9 against 20.7 for a gate|up weight of 16,384 x 2,048),
+ROWS64_MIN_ROWS = 33         # fewer rows are this kernel's or the weight-streaming ones' (`rows64_few`),
 ROWS64_MAX_ROWS = 128        # rows of x the kernel takes (eight blocks of 16 in LDS): more are the matrix library's
 ROWS64_PLAIN_MAX_ROWS = 64   # a plain wide product (the head) of more rows is the library's too: 128 rows against the
                              # vocabulary matrix take 147 µs here and 125 there. What rides on the kernel pays for 65 to
@@ -1304,6 +1303,29 @@ def rows64_takes(rows: int, n: int, k: int, glu: bool = False) -> bool:
             and n % 64 == 0 and k % 1024 == 0)
 
 
+ROWS64_FEW_WIDTH = 8192      # rows of W beyond which few rows of x are this kernel's
+
+
+def rows64_few(rows: int, n: int, k: int, glu: bool = False) -> bool:
+    """Whether up to 32 rows of x against a weight [n, k] are `gemm_rows32`'s and not the weight-streaming kernels' or the library's. The sums have the
+    bits of the 16-row form's; up to 4 rows a plain product stays with the 8-row form, whose sums are nearer to 64 bits, and a gated one gains
+    nothing inside a step (1 row by itself 14.5 and 13.9, a step of 12 layers 579 and 585). Measured, µs, before and here,
+    k 2,048: the gate, n 16,384, 8 rows 14.8 and 13.4, 32 rows 17.1 and 14.0, n 8,192, 8 rows 10.4 and 9.4, 32 rows 12.5 and 10.0, n 4,096, 32 rows (left) 7.3 and 8.7; plain and 32-bit, n 128,256, 8 rows 90.9 and 83.1, 16 rows 103 and 86, 32 rows 127 and 91, n
+    12,288, 5 rows 13.2 and 11.2, 32 rows 16.6 and 13.3, n 8,192, 8 rows (left) 9.1 both, 32 rows 14.7 and 11.4, n 5,120, 8 rows (left) 8.1 and 8.0, 16
+    rows 8.9 and 8.0, 32 rows 12.5 and 9.7, n 4,096, 32 rows (left) 7.0 and 8.3. k 3,072: the gate, n 16,384, 8 rows 21.5 and 18.8, n 8,192, 8 rows (left) 12.3 and
+    12.8; plain, n 5,120, 24 rows (left) 14.0 and 13.4, n 8,192, 24 rows 19.5 and 15.9. k 4,096: plain, n 8,192, 8 rows (left) 15.8 and 16.6, 24 rows
+    (left) 16.9 and 20.4, n 16,384, 24 rows 34.0 and 27.0."""
+    if not 1 <= rows < ROWS64_MIN_ROWS or n % (128 if glu else 64) or k % 1024 or not 1024 <= k <= 4096:
+        return False
+    if rows <= 4:
+        return False
+    if glu:
+        return n > ROWS64_FEW_WIDTH or (n == ROWS64_FEW_WIDTH and k == 2048)
+    if rows <= SKINNY_FUSED_ROWS:
+        return n > ROWS64_FEW_WIDTH or (rows > 8 and n >= 5120 and k <= 3072)
+    return n >= (5120 if k <= 2048 else 8192 if k <= 3072 else ROWS64_FEW_WIDTH + 64) and n * k > SKINNY_WIDE_ELEMENTS
+
+
 def gemm_rows64(x: torch.Tensor, packed: torch.Tensor, out_dtype: torch.dtype = torch.bfloat16, *,
                 glu: bool = False, squares: torch.Tensor | None = None, eps: float = 0.0,
                 unit: "tuple[str, float, float, float] | None" = None) -> torch.Tensor:
@@ -1312,11 +1334,25 @@ def gemm_rows64(x: torch.Tensor, packed: torch.Tensor, out_dtype: torch.dtype = 
     rows then up rows and the result is silu(gate) * up, [M, N / 2]. With `squares` (and `eps`) x is
     the operand of a `PreparedNorm` and the rows' scales multiply the finished sums. `unit` (with `glu`, a plain
     x): (form, limit, slope, up_shift) of the unit of `capped_glu` in silu's place."""
+    return _shared_x(x, packed, out_dtype, glu, squares, eps, unit, 0, 0)
+
+
+def gemm_rows32(x: torch.Tensor, packed: torch.Tensor, out_dtype: torch.dtype = torch.bfloat16, *,
+                glu: bool = False, squares: torch.Tensor | None = None, eps: float = 0.0,
+                unit: "tuple[str, float, float, float] | None" = None, pack8_steps: int = 0) -> "torch.Tensor | PackedRows8":
+    """`gemm_rows64` of up to 32 rows whose sums have the bits of `gemm_skinny`'s (`rows64_few` says where it is the faster way). With `pack8_steps`
+    (and `glu`, up to 8 rows) the gated product comes back as a `PackedRows8` for a reader of that many steps."""
+    _need(x.dim() == 2 and x.shape[0] < ROWS64_MIN_ROWS, lambda: f"gemm_rows32 takes up to {ROWS64_MIN_ROWS - 1} rows, not {tuple(x.shape)}")
+    return _shared_x(x, packed, out_dtype, glu, squares, eps, unit, pack8_steps, pack8_steps or 1)
+
+
+def _shared_x(x: torch.Tensor, packed: torch.Tensor, out_dtype: torch.dtype, glu: bool, squares: torch.Tensor | None, eps: float,
+              unit: "tuple[str, float, float, float] | None", pack8_steps: int, few: int) -> "torch.Tensor | PackedRows8":
     if unit is None or (glu and unit[0] in GLU_ACTIVATIONS):
         out = _native().gemm_rows64(x, packed, out_dtype is torch.float32, _unit_code(glu, unit), squares, eps,
-                                    *((0.0, 0.0, 0.0) if unit is None else unit[1:])) if out_dtype in _DTYPE_CODE else None
+                                    *((0.0, 0.0, 0.0) if unit is None else unit[1:]), few) if out_dtype in _DTYPE_CODE else None
         if out is not None:
-            return out
+            return PackedRows8(out, x.shape[0], packed.shape[0] * 8, pack8_steps) if pack8_steps else out
     _gpu(x, packed)
     _need(x.dtype == torch.bfloat16 and packed.dtype == torch.bfloat16 and x.dim() == 2 and packed.dim() == 4
           and packed.shape[2:] == (64, 8) and packed.is_contiguous(), "gemm_rows64 takes bfloat16 x [M, K] and pack_weight(W)")
@@ -1330,12 +1366,17 @@ def gemm_rows64(x: torch.Tensor, packed: torch.Tensor, out_dtype: torch.dtype = 
     _need(out_dtype == torch.bfloat16 or (out_dtype == torch.float32 and not glu), "32-bit output comes without the gate")
     _check_squares(squares, M)
     _need(unit is None or (glu and squares is None and unit[0] in GLU_ACTIVATIONS), lambda: f"a unit {unit} comes with the gate and a plain x")
-    out = _gated_output(M, N // 2, x.device) if glu else torch.empty((M, N), dtype=out_dtype, device=x.device)
+    _need(not pack8_steps or (glu and M <= 8 and pack8_steps in (4, 8, 16) and (N // 2) % (64 * pack8_steps) == 0),
+          "packed rows come from a gated product of up to 8 rows whose width is whole waves of the reader")
+    if pack8_steps:
+        out = torch.empty(((N // 2) // (64 * pack8_steps), pack8_steps, 64, 8), dtype=torch.bfloat16, device=x.device)
+    else:
+        out = _gated_output(M, N // 2, x.device) if glu else torch.empty((M, N), dtype=out_dtype, device=x.device)
     _run("gemm_rows64", library().ts_gemm_rows64_bf16(
-        _ptr(out), _ptr(x), _ptr(packed), M, N, K, x.stride(0), out.stride(0), _unit_code(glu, unit), int(out_dtype == torch.float32),
-        _ptr(squares), 0 if squares is None else squares.shape[1], float(eps),
-        *((0.0, 0.0, 0.0) if unit is None else map(float, unit[1:])), _stream()))
-    return out
+        _ptr(out), _ptr(x), _ptr(packed), M, N, K, x.stride(0), N // 2 if pack8_steps else out.stride(0), _unit_code(glu, unit),
+        int(out_dtype == torch.float32), _ptr(squares), 0 if squares is None else squares.shape[1], float(eps),
+        *((0.0, 0.0, 0.0) if unit is None else map(float, unit[1:])), int(few), _stream()))
+    return PackedRows8(out, M, N // 2, pack8_steps) if pack8_steps else out
 
 
 ROWS64_PRODUCTS = 8            # products of one launch
@@ -2068,7 +2109,7 @@ def _library_serves(rows: int, n: int, k: int, packed16: bool, out_f32: bool) ->
     weight's 16-row copy is there: no kernel of this library takes it, and its rows are whole 16-byte pieces."""
     if k % 8 or n < 8 or skinny8_takes(rows, n, k) or _skinny_serves(rows, n, k):
         return False
-    return not (packed16 and (rows64_takes(rows, n, k) or (not out_f32 and n <= ROWS64_PLAIN_MAX_WIDTH and rows64_slices(rows, n, k))))
+    return not (packed16 and (rows64_takes(rows, n, k) or rows64_few(rows, n, k) or (not out_f32 and n <= ROWS64_PLAIN_MAX_WIDTH and rows64_slices(rows, n, k))))
 
 
 @functools.lru_cache(maxsize=4096)
@@ -2103,7 +2144,7 @@ def many_rows(x: torch.Tensor, weight: torch.Tensor, packed: "StreamingCopies | 
     if not (_dense_rows(x) and weight.is_contiguous() and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0):
         return True
     return not (skinny8_takes(rows, n, k) or _skinny_serves(rows, n, k)
-                or (packed is not None and packed.by16 is not None and rows64_takes(rows, n, k)))
+                or (packed is not None and packed.by16 is not None and (rows64_takes(rows, n, k) or rows64_few(rows, n, k))))
 
 
 def linear_bf16(x: torch.Tensor, weight: torch.Tensor, out_dtype: torch.dtype = torch.bfloat16,
@@ -2128,6 +2169,9 @@ def linear_bf16(x: torch.Tensor, weight: torch.Tensor, out_dtype: torch.dtype = 
     _need(x.dim() == 2 and weight.dim() == 2 and x.shape[1] == weight.shape[1],
           lambda: f"shapes {tuple(x.shape)} x {tuple(weight.shape)}^T")
     streams = _dense_rows(x) and weight.is_contiguous() and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0
+    if (streams and next_norm is None and packed is not None and packed.by16 is not None and out_dtype in (torch.bfloat16, torch.float32)
+            and rows64_few(x.shape[0], weight.shape[0], x.shape[1])):
+        return gemm_rows32(x, packed.by16, out_dtype)
     if streams and skinny8_takes(x.shape[0], weight.shape[0], x.shape[1]):
         return gemm_skinny8(x, weight, out_dtype, None if packed is None else packed.by8, next_norm=next_norm)
     if streams and _skinny_serves(x.shape[0], weight.shape[0], x.shape[1]):

@@ -117,6 +117,12 @@ def in_three_steps(mixer, x: torch.Tensor, ctx, mem, together: torch.Tensor | No
 PACKED_ROWS_MIN = 2      # rows from which a gated product is handed on in the 8-row form's order (one row is read whole anyway)
 
 
+def _pack8(rows: int, n: int, feeds: torch.Tensor | None) -> int:
+    """Steps of the reader whose order a gated product of `n` rows of W that feeds the weight `feeds` is handed on in, or 0: as a matrix."""
+    steps = hip.rows8_reader_steps(rows, feeds) if feeds is not None and PACKED_ROWS_MIN <= rows <= 8 else 0
+    return 0 if steps and (n // 2) % (64 * steps) else steps
+
+
 def few_rows_unit(x: torch.Tensor, weight: torch.Tensor, packed: hip.StreamingCopies | None, feeds: torch.Tensor,
                   unit: tuple[str, float, float, float]) -> "torch.Tensor | hip.PackedRows8 | None":
     """The gated unit (form, limit, slope, up_shift: `hip.capped_glu`) of few rows of x against W = [gate rows | up rows] by
@@ -131,12 +137,11 @@ def few_rows_unit(x: torch.Tensor, weight: torch.Tensor, packed: hip.StreamingCo
     by16 = None if packed is None else packed.by16
     if by16 is not None and hip.rows64_takes(rows, n, k) and n % 128 == 0:
         return hip.gemm_rows64(x, by16, glu=True, unit=unit)
+    if by16 is not None and hip.rows64_few(rows, n, k, True):
+        return hip.gemm_rows32(x, by16, glu=True, unit=unit, pack8_steps=_pack8(rows, n, feeds))
     if (hip.skinny_fuses(rows, k, False, True) and (rows <= hip.SKINNY_FUSED_ROWS or hip._skinny_serves(rows, n, k))
             and hip.few_rows_unit_pays(rows, n, k)):
-        pack8 = hip.rows8_reader_steps(rows, feeds) if PACKED_ROWS_MIN <= rows <= 8 else 0
-        if pack8 and (n // 2) % (64 * pack8):
-            pack8 = 0
-        return hip.gemm_skinny(x, weight, glu=True, packed=by16, pack8_steps=pack8, unit=unit)[0]
+        return hip.gemm_skinny(x, weight, glu=True, packed=by16, pack8_steps=_pack8(rows, n, feeds), unit=unit)[0]
     return None
 
 
@@ -185,9 +190,7 @@ def linear(x: "torch.Tensor | DeferredNorm | hip.PackedRows8 | hip.SplitAttentio
         return DeferredNorm(linear(x, weight, out_dtype, packed=packed), residual, then.weight, then.eps)
     by16 = None if packed is None else packed.by16
     rows = x.rows if isinstance(x, DeferredNorm) else x.shape[0]
-    pack8 = hip.rows8_reader_steps(rows, feeds) if glu and feeds is not None and PACKED_ROWS_MIN <= rows <= 8 else 0
-    if pack8 and (weight.shape[0] // 2) % (64 * pack8):
-        pack8 = 0
+    pack8 = _pack8(rows, weight.shape[0], feeds) if glu else 0
     if isinstance(x, DeferredNorm) and x.prepared is not None:
         d, op = x, x.prepared.operand
         if out_dtype in (None, torch.bfloat16) and _streams(op, weight, dense_rows=True) and not (glu and weight.shape[0] % 32):
@@ -195,6 +198,8 @@ def linear(x: "torch.Tensor | DeferredNorm | hip.PackedRows8 | hip.SplitAttentio
             wide = by16 is not None and hip.rows64_takes(rows, n, k, glu) and n % (128 if glu else 64) == 0
             if wide:
                 return hip.gemm_rows64(op, by16, glu=glu, squares=d.prepared.squares, eps=d.eps)
+            if by16 is not None and hip.rows64_few(rows, n, k, glu):
+                return hip.gemm_rows32(op, by16, glu=glu, squares=d.prepared.squares, eps=d.eps, pack8_steps=pack8)
             if (hip.skinny_fuses(rows, k, False, True) if glu else hip._skinny_serves(rows, n, k)):
                 return hip.gemm_skinny(op, weight, glu=glu, packed=by16, squares=d.prepared.squares, eps=d.eps,
                                        pack8_steps=pack8 if glu else 0)[0]
@@ -212,6 +217,8 @@ def linear(x: "torch.Tensor | DeferredNorm | hip.PackedRows8 | hip.SplitAttentio
         if (out_dtype in (None, torch.bfloat16) and by16 is not None and _streams(x, weight)
                 and hip.rows64_takes(x.shape[0], weight.shape[0], weight.shape[1], True) and weight.shape[0] % 128 == 0):
             return hip.gemm_rows64(x, by16, glu=True)
+        if out_dtype in (None, torch.bfloat16) and by16 is not None and _streams(x, weight) and hip.rows64_few(x.shape[0], *weight.shape, True):
+            return hip.gemm_rows32(x, by16, glu=True, pack8_steps=pack8)
         if (out_dtype in (None, torch.bfloat16) and _streams(x, weight) and weight.shape[0] % 32 == 0
                 and hip.skinny_fuses(x.shape[0], weight.shape[1], False, True)):
             return hip.gemm_skinny(x, weight, glu=True, packed=by16, pack8_steps=pack8)[0]

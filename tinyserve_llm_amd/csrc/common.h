@@ -36,6 +36,11 @@ template <typename V = uint4> __device__ __forceinline__ V load_once(const void*
   static_assert(sizeof(V) == 16, "16 bytes");
   return __builtin_bit_cast(V, __builtin_nontemporal_load((const stream_u32x4_t*)p));
 }
+// The same for what is written and not read again soon (a state, until the next step).
+template <typename V> __device__ __forceinline__ void store_once(void* p, const V& v) {
+  static_assert(sizeof(V) == 16, "16 bytes");
+  __builtin_nontemporal_store(__builtin_bit_cast(stream_u32x4_t, v), (stream_u32x4_t*)p);
+}
 
 // A kernel's arguments lie in memory that no cache holds when the kernel starts, and the compiler fetches them
 // as the code comes to need them: a long argument block is then waited for two or three times, a trip to

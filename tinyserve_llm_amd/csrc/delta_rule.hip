@@ -198,7 +198,8 @@ extern "C" int ts_delta_prepare(void* mixed, int out_dtype, float* units, float*
 // a column, each with every eighth four of its numbers, so that a column is read and written in whole cache lines; NQ =
 // np / 32 fours a lane. The next token's operands are fetched while one is worked on. A token's three sums (S^T k, S^T q and
 // k . q) are taken together from the state before it: o = exp(l) S^T q + (k . q) u. Requests of more than `up_to` tokens are
-// left out (0: none is).
+// left out (0: none is). The state goes by the caches, both ways: nothing reads it before the next step, which has put it out by then (a decode
+// step of 33 rows with two such mixers of 32 x 128 x 128 and two of 16 x 128 x 128 of the state-space kernel took 581 us through them and takes 560).
 template <typename T, int NQ, int RV>
 __global__ void __launch_bounds__(DL_THREADS)
 delta_step_kernel(float* __restrict__ out, const T* __restrict__ mixed, const float* __restrict__ units, const float* __restrict__ betas,
@@ -217,7 +218,7 @@ delta_step_kernel(float* __restrict__ out, const T* __restrict__ mixed, const fl
 #pragma unroll
   for (int rv = 0; rv < RV; ++rv)
 #pragma unroll
-    for (int i = 0; i < NQ; ++i) ss_load4(st + (int64_t)min(v0 + 32 * rv, vp - 1) * np + 32 * i, S[rv][i]);
+    for (int i = 0; i < NQ; ++i) *(float4*)S[rv][i] = load_once<float4>(st + (int64_t)min(v0 + 32 * rv, vp - 1) * np + 32 * i);
   float kn[NQ][4], qn[NQ][4], vn[RV], bn, ln, rkn, rqn;
   auto fetch = [&](int t) {
     const T* m = mixed + (int64_t)t * row;
@@ -285,7 +286,7 @@ delta_step_kernel(float* __restrict__ out, const T* __restrict__ mixed, const fl
   for (int rv = 0; rv < RV; ++rv)
     if (v0 + 32 * rv < vp) {
 #pragma unroll
-      for (int i = 0; i < NQ; ++i) ss_store4(st + (int64_t)(v0 + 32 * rv) * np + 32 * i, S[rv][i]);
+      for (int i = 0; i < NQ; ++i) store_once(st + (int64_t)(v0 + 32 * rv) * np + 32 * i, *(const float4*)S[rv][i]);
     }
 }
 

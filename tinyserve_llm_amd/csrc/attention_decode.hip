@@ -21,11 +21,18 @@
 // 2,560 keys take 137 µs instead of 122); the instance with a single step per wave has room for 8
 #define DEC_WAVES_FOR(HD, ONE) ((HD) > 64 && !(ONE) ? 4 : DEC_MAX_WAVES)
 
+// Bytes of keys and values that a launch walks from which they go by the caches: they are put out before the next step reads them again, and
+// what they put out are the weights' and the other kernels' lines. Decode steps of 12 layers of the 1B widths over 2,048 keys, through the
+// caches and past them: 64 rows (302 MB a layer) 1,415 and 1,379 us, 16 rows (75 MB) 833 and 811, 12 rows (57 MB) 789 and 770; 8 rows (38 MB) 685 and
+// 689, 8 rows over 500 keys (13 MB) 625 and 629.
+#define DEC_ONCE_BYTES (48ll << 20)
+
 // ONE: a wave has a single 32-key step (chunk = 32 waves); without the second buffer of the
 // general loop the kernel needs fewer registers and more workgroups share a compute unit
 // GENERAL: capped scores, weights in two terms (attention_mfma.h), and optionally a sink: one more in the
 // softmax's denominator, added where a token's chunks meet (here with one chunk, else in the combining kernel).
-template <int HD, bool ONE, bool GENERAL>
+// ONCE: keys and values by load_once (DEC_ONCE_BYTES).
+template <int HD, bool ONE, bool GENERAL, bool ONCE>
 __global__ void __launch_bounds__(DEC_WAVES_FOR(HD, ONE) * TS_WAVE)
 attn_decode_mfma_kernel(bf16_t* __restrict__ out, float* __restrict__ part_o, float* __restrict__ part_ml,
                         const bf16_t* __restrict__ q, const bf16_t* __restrict__ k_cache, const bf16_t* __restrict__ v_cache,
@@ -76,7 +83,7 @@ attn_decode_mfma_kernel(bf16_t* __restrict__ out, float* __restrict__ part_o, fl
   int kend = k0 + chunk;
   if (kend > pos + 1) kend = pos + 1;
   int kb = (k0 > (lo & ~31) ? k0 : (lo & ~31)) + 32 * wave;
-#define TS_LOAD(T, KB) load_tile<HD>(T, KB, r, g, lo, pos, kvh, table, pm, k_cache, v_cache, kp, ks, kh, vp, vh, vd)
+#define TS_LOAD(T, KB) load_tile<HD, ONCE>(T, KB, r, g, lo, pos, kvh, table, pm, k_cache, v_cache, kp, ks, kh, vp, vh, vd)
   // (the general variant: this row's head's penalty per position of distance, in the scores' units before scale2)
   const float slope = (GENERAL && slopes && r < G) ? slopes[kvh * G + r] * (1.44269504088896340736f / scale2) : 0.f;
 #define TS_USE(T, KB) use_tile_auto<HD, GENERAL>(T, KB, r, g, lo, pos, pos, lo, qreg, scale2, m, l, o, cap_in, cap_out, slope)
@@ -236,16 +243,19 @@ static int launch_decode(void* out, float* part_o, float* part_ml, const void* q
     while ((1 << page_shift) < page_size) ++page_shift;
   }
   dim3 grid(num_splits, nkv, num_tokens);
+  const int64_t reach = (int64_t)num_splits * chunk, keys = window > 0 && window < reach ? window : reach;
+  const bool once = (int64_t)num_tokens * nkv * hd * 4 * keys >= DEC_ONCE_BYTES;
   // capped: the cap's tanh takes the scale in and gives units of log2 out, and the softmax's own scale is 1
   const float log2e = 1.44269504088896340736f;
   const float cap_in = softcap > 0.f ? scale / softcap : 0.f, cap_out = softcap * log2e;
   const float scale2 = softcap > 0.f ? 1.0f : scale * log2e;
-#define TS_DEC2(HH, ON, GG)                                                                                     \
-  attn_decode_mfma_kernel<HH, ON, GG><<<grid, waves * TS_WAVE, smem, stream>>>(                                 \
+#define TS_DEC3(HH, ON, GG, NC)                                                                                 \
+  attn_decode_mfma_kernel<HH, ON, GG, NC><<<grid, waves * TS_WAVE, smem, stream>>>(                                 \
       (bf16_t*)out, part_o, part_ml, (const bf16_t*)q, (const bf16_t*)k_cache, (const bf16_t*)v_cache,          \
       block_tables, seq_of_token, positions, nh, G, page_size, page_shift, page_run, kp, ks, kh, vp, vh, vd, max_blocks,  \
       num_splits, chunk, scale2, window, cap_in, cap_out, sink, sinks, slopes, gate, gate_stride)
-#define TS_DEC1(HH, ON) if (general) TS_DEC2(HH, ON, true); else TS_DEC2(HH, ON, false)
+#define TS_DEC2(HH, ON, GG) if (once) TS_DEC3(HH, ON, GG, true); else TS_DEC3(HH, ON, GG, false)
+#define TS_DEC1(HH, ON) if (general) { TS_DEC2(HH, ON, true); } else { TS_DEC2(HH, ON, false); }
 #define TS_DEC(HH) if (chunk == 32 * waves) { TS_DEC1(HH, true); } else { TS_DEC1(HH, false); }
   switch (hd) {
     case 32: TS_DEC(32); break;
@@ -257,6 +267,7 @@ static int launch_decode(void* out, float* part_o, float* part_ml, const void* q
 #undef TS_DEC
 #undef TS_DEC1
 #undef TS_DEC2
+#undef TS_DEC3
   int rc = ts_check_launch();
   if (rc || num_splits == 1 || !combine) return rc;     // (combine 0: the caller's next kernel reads the parts itself)
   attn_decode_combine_kernel<<<num_tokens * nh, TS_WAVE, 0, stream>>>((bf16_t*)out, part_o, part_ml, positions, nh, hd,

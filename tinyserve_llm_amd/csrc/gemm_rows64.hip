@@ -83,8 +83,8 @@ struct Rows64GroupArgs : Rows64Args {
 // With a group's arguments the sums are added up in stretches of 128 of K, with up to 64 rows in pairs of them, so that they are as near to 64 bits as
 // those of the kernels for a product of its own, which share a reduction out to their waves (over 2,048: 0.9e-7 up to 8 rows, 1.0e-7 up to 32, 1.3e-7 up to
 // 64, the library's beyond 2.7e-7). A product of a few million numbers of W is a launch, a trip of x to LDS and as few workgroups as it has columns for
-// 64 each: five of them (2,048 columns four times and 64, K 2,048) took 18 us apart and take 10.5 here with 1 row, 20 and 10.7 with 8, 28 and 11.3 with
-// 32, 50 and 11.8 with 48.
+// 64 each: five of them (2,048 columns four times and 64, K 2,048) took 17.6 us apart and take 9.5 here with 1 row, 19.1 and 9.7 with 8, 26.5 and 11.1 with
+// 32, 50.0 and 12.0 with 48.
 // FEW (up to 32 rows): a chunk's products are summed, then the chunks in ascending order: what a wave of the 16-row form makes of its share of
 // K and what becomes of the waves' sums, so that a product has the bits of that form, whichever of the two makes it.
 template <int GLU, typename OUT, int BLOCKS, typename ARGS, bool FEW = false>

@@ -1412,9 +1412,9 @@ def rows64_slices(rows: int, n: int, k: int) -> int:
     narrow weight [n, k] into: the fewest that give every compute unit a workgroup of 64 rows of W
     (else the most the reduction allows); 0 where the kernel does not serve the shape or the weight
     is wide enough for `gemm_rows64` itself. Measured with the finishing kernel, against the library
-    followed by the norm kernel, for a down projection over 8,192 (14,336 at the widest): 9 rows 12.9
-    against 15.5 µs at a width of 2,048, 15.8 against 18.5 at 3,072, 27.0 against 31.1 at 4,096; 32 rows
-    14.1 against 18.9, 17.3 against 21.6, 27.5 against 38.3; 64 rows 15.5 against 22.0 + 7 at 2,048."""
+    followed by the norm kernel, for a down projection over 8,192 (14,336 at the widest): 9 rows 11.7
+    against 15.5 µs at a width of 2,048, 14.0 against 18.5 at 3,072, 23.6 against 31.1 at 4,096; 32 rows
+    12.3 against 18.9, 15.4 against 21.6, 24.6 against 38.3; 64 rows 14.2 against 22.0 + 7 at 2,048."""
     if not (ROWS64_SLICED_MIN_ROWS <= rows <= ROWS64_MAX_ROWS) or n % 64 or n >= ROWS64_MIN_WIDTH or k % ROWS64_SLICE_K:
         return 0
     return _filling_slices(n, k)
@@ -1899,7 +1899,8 @@ def gemm_whole(xs: "Sequence[torch.Tensor]", weights: "Sequence[torch.Tensor]", 
     return ys
 
 
-GROUP_FEW_ROWS = 64            # rows up to which a group goes to the kernel that streams W past x, beyond to whole tiles
+GROUP_FEW_ROWS = 64            # rows up to which a group goes to the kernel that streams W past x, beyond to whole tiles (up to 128 rows the first would be
+                               # the faster one still, which steps of so many tokens, bound by the host, do not show)
 GROUP_SURE_ROWS, GROUP_SURE_WIDTH, GROUP_MIN_ROWS = 9, 8192, 5      # two products of few rows: from these rows on, or, with so many columns, from those
 
 
@@ -1907,9 +1908,9 @@ GROUP_SURE_ROWS, GROUP_SURE_WIDTH, GROUP_MIN_ROWS = 9, 8192, 5      # two produc
 def group_plan(rows: int, widths: "tuple[int, ...]", k: int, packed: bool) -> int | None:
     """How `gemm_group` makes the products of `rows` rows against weights [width, k]: -1 by `gemm_rows64_group` (with `packed`: their packed copies are
     there), a tile of `gemm_whole`, or None: one by one, which may well be as fast. Measured, µs, one by one and together: widths 2,048 four times and 64, k
-    2,048: 1 row 18.4 and 11.1, 8 rows 20.4 and 11.1, 48 rows 50.5 and 12.7, 128 rows 43.0 and 14.6, 600 rows 62.5 and 30.5, 2,048 rows 109.6 and 85.3; 2,048
-    twice: 1 row (left) 7.3 and 8.9, 16 rows 10.0 and 9.3, 48 rows 17.2 and 9.5, 1,024 rows 29.0 and 23.0; 3,104 and 8,192: 4 rows (left) 13.4 and 13.1, 8 rows 14.1 and 13.2, 48
-    rows 24.0 and 14.8, 1,024 rows 62.6 and 53.3, 1,500 rows (left) 77.6 and 86.0."""
+    2,048: 1 row 17.6 and 9.5, 8 rows 19.1 and 9.7, 48 rows 50.0 and 12.0, 128 rows 50.4 and 18.0, 600 rows 66.5 and 32.9, 2,048 rows 109 and 83; 2,048 twice: 1 row (left) 7.4 and 8.5, 16 rows 10.4 and 8.8, 48 rows 21.0 and 11.4, 128 rows 22.5 and 18.1, 1,024
+    rows 37.3 and 24.6; 3,104 and 8,192: 4 rows (left: the 8-row form's sums are nearer to 64 bits) 13.4 and 11.3, 8 rows 14.0 and 11.3, 48
+    rows 20.9 and 13.0, 96 rows 27.9 and 19.8, 1,024 rows 63.1 and 54.3, 1,500 rows (left) 77.6 and 86.0."""
     if len(widths) < 2 or len(widths) > min(ROWS64_PRODUCTS, WHOLE_PRODUCTS):
         return None
     if rows <= GROUP_FEW_ROWS:

@@ -1289,11 +1289,10 @@ def gemm_skinny(x: torch.Tensor, weight: torch.Tensor, out_dtype: torch.dtype = 
 ROWS64_MIN_ROWS = 33         # fewer rows are this kernel's or the weight-streaming ones' (`rows64_few`),
 ROWS64_MAX_ROWS = 128        # rows of x the kernel takes (eight blocks of 16 in LDS): more are the matrix library's
 ROWS64_PLAIN_MAX_ROWS = 64   # a plain wide product (the head) of more rows is the library's too: 128 rows against the
-                             # vocabulary matrix take 147 µs here and 125 there. What rides on the kernel pays for 65 to
-                             # 128 rows: the gate (24.0 µs against 24.2 for the library and the gate kernel), and for the
-                             # narrow products in slices the finishing kernel (o 12.7 against 14.2 for the library and
-                             # the norm kernel, down 18.6 against 23.9, q|k|v with the rotation 18.1 against 20.4): a
-                             # decode step at batch 128 takes 2.99 ms instead of 3.20, at batch 96 2.47 instead of 2.76
+                             # vocabulary matrix take 136 µs here and 125 there. What rides on the kernel pays for 65 to
+                             # 128 rows: the gate (20.6 µs against 24.2 for the library and the gate kernel), and for the
+                             # narrow products in slices the finishing kernel (o 11.5 against 14.2 for the library and
+                             # the norm kernel, down 17.0 against 23.9, q|k|v with the rotation 18.1 against 20.4)
 ROWS64_MIN_WIDTH = 8192      # rows of W from which 64 of them a workgroup still give every compute unit one
 
 

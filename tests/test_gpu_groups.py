@@ -102,6 +102,13 @@ def test_the_rule_takes_what_was_measured_faster():
     assert hip.group_plan(48, (2048, 24), 2048, True) is None and hip.group_plan(48, lasts, 1536, True) is None and hip.group_plan(100, (2048, 20), 2048, True) is None
 
 
+@pytest.mark.parametrize("widths, k", [((2048, 2048), 5120), ((2048, 2048), 8192), ((1536, 1536), 8192), ((4096,) * 4, 5120), ((4096,) * 4, 6144), ((2048,) * 4 + (64,), 8192)])
+def test_products_that_go_in_slices_by_themselves_are_not_grouped(widths, k):
+    """Their reductions' shorter chains are nearer to 64 bits than a whole one, and faster."""
+    sliced = [rows for rows in range(129, 2049) if any(hip.slices_plan(rows, n, k, "f32") is not None for n in widths)]
+    assert len(sliced) > 200 and all(hip.group_plan(rows, widths, k, True) is None for rows in sliced)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [BF, torch.float32])
 @pytest.mark.parametrize("right", ["shifted_decay_recurrence", "retention"])

@@ -1909,7 +1909,8 @@ def group_plan(rows: int, widths: "tuple[int, ...]", k: int, packed: bool) -> in
     there), a tile of `gemm_whole`, or None: one by one, which may well be as fast. Measured, µs, one by one and together: widths 2,048 four times and 64, k
     2,048: 1 row 17.6 and 9.5, 8 rows 19.1 and 9.7, 48 rows 50.0 and 12.0, 128 rows 50.4 and 18.0, 600 rows 66.5 and 32.9, 2,048 rows 109 and 83; 2,048 twice: 1 row (left) 7.4 and 8.5, 16 rows 10.4 and 8.8, 48 rows 21.0 and 11.4, 128 rows 22.5 and 18.1, 1,024
     rows 37.3 and 24.6; 3,104 and 8,192: 4 rows (left: the 8-row form's sums are nearer to 64 bits) 13.4 and 11.3, 8 rows 14.0 and 11.3, 48
-    rows 20.9 and 13.0, 96 rows 27.9 and 19.8, 1,024 rows 63.1 and 54.3, 1,500 rows (left) 77.6 and 86.0."""
+    rows 20.9 and 13.0, 96 rows 27.9 and 19.8, 1,024 rows 63.1 and 54.3, 1,500 rows (left) 77.6 and 86.0. A group with a product that would go by
+    itself in slices (`slices_plan`) is left: 1,536 twice, k 8,192, 129 rows 31.7 and 52.9, errors 2.1e-7 and 5.7e-7."""
     if len(widths) < 2 or len(widths) > min(ROWS64_PRODUCTS, WHOLE_PRODUCTS):
         return None
     if rows <= GROUP_FEW_ROWS:
@@ -1917,12 +1918,13 @@ def group_plan(rows: int, widths: "tuple[int, ...]", k: int, packed: bool) -> in
         return -1 if packed and pays and k % 1024 == 0 and all(n % 16 == 0 for n in widths) else None
     if rows > WHOLE_MAX_ROWS or k % 64 or k < WHOLE_MIN_K or any(n % 8 for n in widths):
         return None
+    if any(slices_plan(rows, n, k, "f32") is not None for n in widths):      # (their sums are of shorter chains, and nearer to 64 bits)
+        return None
     us, tile = _whole_cost(rows, widths, k, "f32")
     apart = 0.0
     for n in widths:
-        taken = many_rows_plan(rows, n, k, "f32")
         alone = _whole_library(rows, n, k, "f32")
-        apart += min(alone, _whole_cost(rows, (n,), k, "f32")[0]) if taken is not None else alone
+        apart += alone if whole_plan(rows, n, k, "f32") is None else min(alone, _whole_cost(rows, (n,), k, "f32")[0])
     return tile if us < apart else None
 
 

@@ -109,6 +109,33 @@ def test_products_that_go_in_slices_by_themselves_are_not_grouped(widths, k):
     assert len(sliced) > 200 and all(hip.group_plan(rows, widths, k, True) is None for rows in sliced)
 
 
+def test_small_results_are_left_out_of_whole_tiles():
+    parts = hip.group_parts
+    for rows in (130, 600, 2048):
+        assert parts(rows, (2048,) * 4 + (64,), 2048, True) == (hip.group_plan(rows, (2048,) * 4, 2048, False), (4,))
+        assert parts(rows, (2048, 64), 2048, True) == (None, ()) and parts(rows, (2048, 64), 1024, True)[1] == ()
+    assert parts(129, (512, 1024, 1024), 2048, False)[1] == (0,) and parts(320, (512, 1024, 1024), 2048, False)[1] == ()
+    for rows in (65, 80, 128):
+        assert parts(rows, (2048,) * 4 + (64,), 2048, True) == parts(rows, (1024,) * 3, 2048, True) == (-1, ())
+        assert parts(rows, (1024,) * 3, 2048, False) == (None, ()) and parts(rows, (1024,) * 3, 4096, True) == (None, ())
+    assert parts(80, (3104, 8192), 2048, True) == (-1, ()) and parts(80, (3104, 8192), 2048, False) == (None, ())
+    assert parts(96, (3104, 8192), 2048, True) == (hip.group_plan(96, (3104, 8192), 2048, True), ())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [66, 88, 96, 129, 200, 330, 700])
+@pytest.mark.parametrize("widths, k", [((2048, 2048, 64), 2048), ((1536, 1536), 2048), ((1024, 1024, 1024), 3072), ((3104, 8192), 2048), ((512, 2048, 1024), 1536)])
+def test_no_product_of_a_group_of_many_rows_is_further_from_64_bits_than_by_itself(rows, widths, k):
+    """The mean error over a result's numbers varies by less than a tenth between one order of the sums and another that is as good."""
+    xs, ws = group(rows, widths, k)
+    copies = torch.cat([hip.pack_weight(w) for w in ws]) if k % 1024 == 0 else None
+    for packed in (copies, None):
+        ys = hip.gemm_group(xs, ws, packed)
+        for x, w, y in zip(xs, ws, ys or ()):
+            want = x.double() @ w.double().T
+            assert y.shape == want.shape and float((y.double() - want).norm()) <= 1.1 * float((hip.linear_bf16(x, w, torch.float32).double() - want).norm())
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [BF, torch.float32])
 @pytest.mark.parametrize("right", ["shifted_decay_recurrence", "retention"])

@@ -1898,14 +1898,29 @@ def gemm_whole(xs: "Sequence[torch.Tensor]", weights: "Sequence[torch.Tensor]", 
     return ys
 
 
-GROUP_FEW_ROWS = 64            # rows up to which a group goes to the kernel that streams W past x, beyond to whole tiles (up to 128 rows the first would be
-                               # the faster one still, which steps of so many tokens, bound by the host, do not show)
+GROUP_FEW_ROWS = 64            # rows up to which a group goes to the kernel that streams W past x, beyond to whole tiles where these are as exact (`group_parts`)
 GROUP_SURE_ROWS, GROUP_SURE_WIDTH, GROUP_MIN_ROWS = 9, 8192, 5      # two products of few rows: from these rows on, or, with so many columns, from those
+# products whose sums the matrix library may split into four chains: reductions beyond GROUP_CHAIN_K of results of at most GROUP_SPLIT_NUMBERS, and of up to
+# GROUP_SPLIT_ROWS rows and more than GROUP_SPLIT_WIDTH columns
+GROUP_CHAIN_K, GROUP_SPLIT_NUMBERS, GROUP_SPLIT_ROWS, GROUP_SPLIT_WIDTH = 1024, 1 << 17, 95, 2048
+GROUP_STREAM_K, GROUP_STREAM_MIN_WIDTH = 3072, 1024      # three products and more of 65 to 128 rows by the kernel that streams W: up to this k, from so many columns
+
+
+def _group_streams(rows: int, widths: "tuple[int, ...]", k: int) -> bool:
+    """Whether the kernel that streams W past x is the faster way to a group of up to 128 rows."""
+    if k % 1024 or any(n % 16 for n in widths):
+        return False
+    columns = sum(widths)
+    if rows <= GROUP_FEW_ROWS:
+        return len(widths) > 2 or rows >= GROUP_SURE_ROWS or (rows >= GROUP_MIN_ROWS and columns >= GROUP_SURE_WIDTH)
+    if len(widths) > 2:
+        return rows <= ROWS64_MAX_ROWS and (k < columns or (k <= GROUP_STREAM_K and columns >= GROUP_STREAM_MIN_WIDTH))
+    return rows <= ROWS64_MAX_ROWS and k < columns and (k <= 2048 or 4 * k <= 3 * columns)
 
 
 @functools.lru_cache(maxsize=4096)
 def group_plan(rows: int, widths: "tuple[int, ...]", k: int, packed: bool) -> int | None:
-    """How `gemm_group` makes the products of `rows` rows against weights [width, k]: -1 by `gemm_rows64_group` (with `packed`: their packed copies are
+    """The faster way to the products of `rows` rows against weights [width, k]: -1 by `gemm_rows64_group` (with `packed`: their packed copies are
     there), a tile of `gemm_whole`, or None: one by one, which may well be as fast. Measured, µs, one by one and together: widths 2,048 four times and 64, k
     2,048: 1 row 17.6 and 9.5, 8 rows 19.1 and 9.7, 48 rows 50.0 and 12.0, 128 rows 50.4 and 18.0, 600 rows 66.5 and 32.9, 2,048 rows 109 and 83; 2,048 twice: 1 row (left) 7.4 and 8.5, 16 rows 10.4 and 8.8, 48 rows 21.0 and 11.4, 128 rows 22.5 and 18.1, 1,024
     rows 37.3 and 24.6; 3,104 and 8,192: 4 rows (left: the 8-row form's sums are nearer to 64 bits) 13.4 and 11.3, 8 rows 14.0 and 11.3, 48
@@ -1914,8 +1929,7 @@ def group_plan(rows: int, widths: "tuple[int, ...]", k: int, packed: bool) -> in
     if len(widths) < 2 or len(widths) > min(ROWS64_PRODUCTS, WHOLE_PRODUCTS):
         return None
     if rows <= GROUP_FEW_ROWS:
-        pays = len(widths) > 2 or rows >= GROUP_SURE_ROWS or (rows >= GROUP_MIN_ROWS and sum(widths) >= GROUP_SURE_WIDTH)
-        return -1 if packed and pays and k % 1024 == 0 and all(n % 16 == 0 for n in widths) else None
+        return -1 if packed and _group_streams(rows, widths, k) else None
     if rows > WHOLE_MAX_ROWS or k % 64 or k < WHOLE_MIN_K or any(n % 8 for n in widths):
         return None
     if any(slices_plan(rows, n, k, "f32") is not None for n in widths):      # (their sums are of shorter chains, and nearer to 64 bits)
@@ -1928,23 +1942,54 @@ def group_plan(rows: int, widths: "tuple[int, ...]", k: int, packed: bool) -> in
     return tile if us < apart else None
 
 
+@functools.lru_cache(maxsize=4096)
+def group_parts(rows: int, widths: "tuple[int, ...]", k: int, packed: bool) -> "tuple[int | None, tuple[int, ...]]":
+    """(`group_plan` of the products made together, the places of those made by themselves): a product in whole tiles is one chain over all of k, and small
+    results are nearer to 64 bits by the library (of `rows` x 64 over 2,048 1.3e-7 and 2.7e-7, of 129 x 512 the same, of 320 x 512 2.7e-7 both, over 1,024
+    1.8e-7 both; where it splits follows from 1,000 measured results, GROUP_SPLIT_NUMBERS and GROUP_SPLIT_ROWS), or by the kernel that streams W (1.0e-7), which up
+    to 128 rows takes the whole group where it is the faster way, µs, one by one and together: 1,024 three times, k 2,048, 65 rows 24.8 and 12.7, 128 rows 25.4 and
+    16.2, k 4,096 (left) 36.0 and 27.9; 3,104 and 8,192, k 2,048, 80 rows 28.2 and 16.2; 1,024 twice, k 3,072 (left) 128 rows 15.6 and 21.9."""
+    plan = group_plan(rows, widths, k, packed)
+    if plan is None or plan < 0 or k <= GROUP_CHAIN_K:
+        return plan, ()
+    alone = tuple(i for i, n in enumerate(widths) if rows * n <= GROUP_SPLIT_NUMBERS or (rows <= GROUP_SPLIT_ROWS and n > GROUP_SPLIT_WIDTH))
+    if not alone:
+        return plan, ()
+    if packed and _group_streams(rows, widths, k):
+        return -1, ()
+    plan = group_plan(rows, tuple(n for i, n in enumerate(widths) if i not in alone), k, False)
+    return (None, ()) if plan is None else (plan, alone)
+
+
 def gemm_group(xs: "Sequence[torch.Tensor]", weights: "Sequence[torch.Tensor]", packed: torch.Tensor | None) -> "tuple[torch.Tensor, ...] | None":
-    """float32 x · weight^T of several bfloat16 products of the same rows and reduction in one launch, where that is the faster way (`group_plan`); None
-    where not, or where their operands are another way. `packed`: the `pack_weight` copies of all the weights, one behind the other, if they are kept."""
+    """float32 x · weight^T of several bfloat16 products of the same rows and reduction in one launch, where that is the faster way and as exact (`group_parts`);
+    None where not, or where their operands are another way. `packed`: the `pack_weight` copies of all the weights, one behind the other, if they are kept."""
     x, w = xs[0], weights[0]
     if _many_rows != "library" or x.dim() != 2 or not x.is_cuda:
         return None
     rows, k = x.shape
     widths = tuple([v.shape[0] for v in weights])
-    plan = group_plan(rows, widths, k, packed is not None)
+    plan, alone = group_parts(rows, widths, k, packed is not None)
     if rows == 0 or plan is None:
         return None
-    done = _native().gemm_slices(tuple(xs), tuple(weights), plan, packed if plan < 0 else None)
+    if alone:
+        ys = _group([t for i, t in enumerate(xs) if i not in alone], [t for i, t in enumerate(weights) if i not in alone], plan, None)
+        if ys is None or not all(t.shape == x.shape for t in xs):
+            return None
+        left = iter(ys)
+        return tuple([linear_bf16(xs[i], weights[i], torch.float32) if i in alone else next(left) for i in range(len(xs))])
+    return _group(xs, weights, plan, packed if plan < 0 else None)
+
+
+def _group(xs: "Sequence[torch.Tensor]", weights: "Sequence[torch.Tensor]", plan: int, packed: torch.Tensor | None) -> "tuple[torch.Tensor, ...] | None":
+    """The products in one launch by the way `plan` of `group_plan`; None where it does not take the operands."""
+    done = _native().gemm_slices(tuple(xs), tuple(weights), plan, packed)
     if done is not None:
         return done
+    x, w = xs[0], weights[0]
     if not all(t.shape == x.shape and t.stride() == x.stride() and v.stride() == w.stride() and whole_takes(t, v) for t, v in zip(xs, weights)):
         return None
-    return gemm_rows64_group(xs, packed, widths) if plan < 0 else gemm_whole(xs, weights, plan, torch.float32)
+    return gemm_whole(xs, weights, plan, torch.float32) if packed is None else gemm_rows64_group(xs, packed, [v.shape[0] for v in weights])
 
 
 WHOLE_MIN_STEPS = 3      # steps of 64 that a tile's reduction has at least

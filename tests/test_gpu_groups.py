@@ -109,12 +109,26 @@ def test_products_that_go_in_slices_by_themselves_are_not_grouped(widths, k):
     assert len(sliced) > 200 and all(hip.group_plan(rows, widths, k, True) is None for rows in sliced)
 
 
+@pytest.mark.parametrize("rows, widths, inside, outside", [
+    (9, (1024, 1024), 1024, 2048), (9, (2304, 768), 1024, 2048), (9, (64, 64), 1024, 2048), (16, (1024, 1024), 2048, 3072), (9, (2048, 2048), 3072, 4096), (48, (2048, 2048), 4096, 8192), (17, (4096, 4096), 8192, 9216), (1, (1024,) * 3, 2048, 3072),
+    (5, (1024,) * 3, 4096, 5120), (64, (2048,) * 4 + (64,), 8192, 9216), (16, (64,) * 3, 4096, 16384), (9, (4096, 64), 4096, 5120), (128, (2048, 2048), 3072, 4096), (200, (2048, 2048), 3072, 4096)])
+def test_groups_of_few_columns_are_left_over_long_reductions(rows, widths, inside, outside):
+    """A workgroup walks all of k, however few of them there are."""
+    assert hip.group_plan(rows, widths, inside, True) is not None and hip.group_plan(rows, widths, outside, True) is None
+
+
+def test_wide_groups_of_many_rows_promise_more_than_the_estimates_err_by():
+    for rows, k in ((1500, 1024), (1500, 2048), (1500, 4096)):
+        assert hip.group_plan(rows, (3104, 8192), k, True) is None
+    assert hip.group_plan(2048, (6144, 8192), 4096, True) is None and hip.group_plan(900, (3104, 8192), 4096, True) is not None
+
+
 def test_small_results_are_left_out_of_whole_tiles():
     parts = hip.group_parts
     for rows in (130, 600, 2048):
         assert parts(rows, (2048,) * 4 + (64,), 2048, True) == (hip.group_plan(rows, (2048,) * 4, 2048, False), (4,))
         assert parts(rows, (2048, 64), 2048, True) == (None, ()) and parts(rows, (2048, 64), 1024, True)[1] == ()
-    assert parts(129, (512, 1024, 1024), 2048, False)[1] == (0,) and parts(320, (512, 1024, 1024), 2048, False)[1] == ()
+    assert parts(129, (512, 2048, 1024), 2048, False)[1] == (0,) and parts(320, (512, 2048, 1024), 2048, False)[1] == ()
     for rows in (65, 80, 128):
         assert parts(rows, (2048,) * 4 + (64,), 2048, True) == parts(rows, (1024,) * 3, 2048, True) == (-1, ())
         assert parts(rows, (1024,) * 3, 2048, False) == (None, ()) and parts(rows, (1024,) * 3, 4096, True) == (None, ())

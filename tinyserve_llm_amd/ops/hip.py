@@ -1900,6 +1900,9 @@ def gemm_whole(xs: "Sequence[torch.Tensor]", weights: "Sequence[torch.Tensor]", 
 
 GROUP_FEW_ROWS = 64            # rows up to which a group goes to the kernel that streams W past x, beyond to whole tiles where these are as exact (`group_parts`)
 GROUP_SURE_ROWS, GROUP_SURE_WIDTH, GROUP_MIN_ROWS = 9, 8192, 5      # two products of few rows: from these rows on, or, with so many columns, from those
+GROUP_LONG_K = 4096            # three products and more: up to this k also where it is not below the columns (from 5 rows on)
+GROUP_EVEN_ROWS, GROUP_SHORT_K = 16, 2048      # two products over more than 1,024: from these rows on up to k columns; of fewer rows, up to this k, only from 2 k columns on
+GROUP_CHAIN_ROWS, GROUP_WIDE_SHARE = 256, 0.92      # whole tiles of up to so many rows only for k below the columns; the share of the time one by one, both as estimated, that wide groups promise
 # products whose sums the matrix library may split into four chains: reductions beyond GROUP_CHAIN_K of results of at most GROUP_SPLIT_NUMBERS, and of up to
 # GROUP_SPLIT_ROWS rows and more than GROUP_SPLIT_WIDTH columns
 GROUP_CHAIN_K, GROUP_SPLIT_NUMBERS, GROUP_SPLIT_ROWS, GROUP_SPLIT_WIDTH = 1024, 1 << 17, 95, 2048
@@ -1907,12 +1910,21 @@ GROUP_STREAM_K, GROUP_STREAM_MIN_WIDTH = 3072, 1024      # three products and mo
 
 
 def _group_streams(rows: int, widths: "tuple[int, ...]", k: int) -> bool:
-    """Whether the kernel that streams W past x is the faster way to a group of up to 128 rows."""
+    """Whether the kernel that streams W past x is the faster way to a group of up to 128 rows. A workgroup of it walks all of k for 64 columns, where what a
+    product has by itself cuts k into shares for its waves, or into slices: so a group of few columns over a long k is left. Measured at k 1,024 to 8,192
+    over 16 groups, µs, one by one and together: 1,024 twice, k 1,024, 9 rows 6.6 and 6.1, 48 rows 16.6 and 7.3, k 2,048, 9 rows (left) 8.2 and 8.5, 48 rows 16.6 and 11.1, k 4,096, 48 rows (left)
+    17.1 and 18.3; 64 twice, k 1,024, 9 rows 7.0 and 4.2; 2,048 twice, k 3,072, 9 rows 13.1 and 11.6, k 4,096, 16 rows 18.0 and 14.9, k 8,192 (left) 17 rows 25.6 and 27.5, 48 rows 30.3 and 33.9; 4,096 twice, k
+    8,192, 17 rows 35.5 and 33.5; 1,024 three times, k 3,072, 1 row (left) 10.5 and 11.0, 5 rows 11.6 and 11.4, k 4,096, 9 rows 21.3 and 14.0, k 8,192 (left) 5 rows
+    23.7 and 24.0; 2,304 and 768, k 2,048, 9 rows (left) 8.4 and 8.8; 2,048 four times and 64, k 8,192, 1 row 42.1 and 28.8, 48 rows 71.6 and 36.3.
+    Of 780 points it takes four are slower, by 1 to 3 % (4,096 twice, k 4,096, 5 rows 17.8 and 18.3)."""
     if k % 1024 or any(n % 16 for n in widths):
         return False
     columns = sum(widths)
     if rows <= GROUP_FEW_ROWS:
-        return len(widths) > 2 or rows >= GROUP_SURE_ROWS or (rows >= GROUP_MIN_ROWS and columns >= GROUP_SURE_WIDTH)
+        if len(widths) > 2:
+            return k < columns or (rows >= GROUP_MIN_ROWS and k <= GROUP_LONG_K)
+        return ((rows >= GROUP_SURE_ROWS or (rows >= GROUP_MIN_ROWS and columns >= GROUP_SURE_WIDTH))
+                and (k <= GROUP_CHAIN_K or (k <= columns if rows >= GROUP_EVEN_ROWS else k < columns and (k > GROUP_SHORT_K or 2 * k <= columns))))
     if len(widths) > 2:
         return rows <= ROWS64_MAX_ROWS and (k < columns or (k <= GROUP_STREAM_K and columns >= GROUP_STREAM_MIN_WIDTH))
     return rows <= ROWS64_MAX_ROWS and k < columns and (k <= 2048 or 4 * k <= 3 * columns)
@@ -1924,7 +1936,9 @@ def group_plan(rows: int, widths: "tuple[int, ...]", k: int, packed: bool) -> in
     there), a tile of `gemm_whole`, or None: one by one, which may well be as fast. Measured, µs, one by one and together: widths 2,048 four times and 64, k
     2,048: 1 row 17.6 and 9.5, 8 rows 19.1 and 9.7, 48 rows 50.0 and 12.0, 128 rows 50.4 and 18.0, 600 rows 66.5 and 32.9, 2,048 rows 109 and 83; 2,048 twice: 1 row (left) 7.4 and 8.5, 16 rows 10.4 and 8.8, 48 rows 21.0 and 11.4, 128 rows 22.5 and 18.1, 1,024
     rows 37.3 and 24.6; 3,104 and 8,192: 4 rows (left: the 8-row form's sums are nearer to 64 bits) 13.4 and 11.3, 8 rows 14.0 and 11.3, 48
-    rows 20.9 and 13.0, 96 rows 27.9 and 19.8, 1,024 rows 63.1 and 54.3, 1,500 rows (left) 77.6 and 86.0. A group with a product that would go by
+    rows 20.9 and 13.0, 96 rows 27.9 and 19.8, 1,024 rows 63.1 and 54.3, 1,500 rows (left) 77.6 and 86.0. Whole tiles over 1,100 points (65 to 2,600 rows, k 1,024 to
+    8,192): 2,048 twice, k 4,096, 129 rows (left) 29.5 and 30.6, 320 rows 43.3 and 31.9; with a width of 8,192, whose estimates err most, 0.77 of the time one by one on average and 2 of
+    167 slower, by 2 and 3 % (3,104 and 8,192, k 1,024, 1,500 rows, left, 53.5 and 56.3); without, 0.65 and none. A group with a product that would go by
     itself in slices (`slices_plan`) is left: 1,536 twice, k 8,192, 129 rows 31.7 and 52.9, errors 2.1e-7 and 5.7e-7."""
     if len(widths) < 2 or len(widths) > min(ROWS64_PRODUCTS, WHOLE_PRODUCTS):
         return None
@@ -1934,12 +1948,14 @@ def group_plan(rows: int, widths: "tuple[int, ...]", k: int, packed: bool) -> in
         return None
     if any(slices_plan(rows, n, k, "f32") is not None for n in widths):      # (their sums are of shorter chains, and nearer to 64 bits)
         return None
+    if rows <= GROUP_CHAIN_ROWS and k >= sum(widths) and not (len(widths) > 2 and k <= GROUP_LONG_K):
+        return None
     us, tile = _whole_cost(rows, widths, k, "f32")
     apart = 0.0
     for n in widths:
         alone = _whole_library(rows, n, k, "f32")
         apart += alone if whole_plan(rows, n, k, "f32") is None else min(alone, _whole_cost(rows, (n,), k, "f32")[0])
-    return tile if us < apart else None
+    return tile if us < (GROUP_WIDE_SHARE if max(widths) >= WHOLE_WIDE else 1.0) * apart else None
 
 
 @functools.lru_cache(maxsize=4096)

@@ -167,6 +167,16 @@ def test_whole_tiles_are_taken_where_they_were_the_faster_way():
     assert hip.many_rows_plan(1024, 2048, 8192, "f32") == hip.slices_plan(1024, 2048, 8192, "f32") != None      # noqa: E711 (a long reduction is cut as before)
 
 
+def test_wide_products_of_even_columns_are_the_library_s_where_it_was_as_fast():
+    for n in (8192, 10240, 12288, 12800):
+        for rows in range(129, 3073, 7):
+            assert all(hip.whole_plan(rows, n, k, "bf16") is None for k in (1024, 2048, 4096, 5120))
+            assert rows >= 960 or all(hip.whole_plan(rows, n, k, "f32") is None for k in (1024, 2048, 4096, 5120))
+    for rows, n, k, ending, taken in ((1280, 10304, 2048, "bf16", True), (1150, 12288, 2048, "bf16", False), (1514, 7168, 2048, "bf16", True), (999, 12288, 2048, "f32", False),
+                                      (1514, 10240, 2048, "f32", True), (800, 12352, 4096, "f32", False), (640, 12352, 4096, "f32", True)):
+        assert (hip.whole_plan(rows, n, k, ending) is not None) == taken
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("rows, n, k, out", [(720, 2048, 2048, torch.float32), (999, 12352, 2048, BF)])
 def test_linear_takes_them_by_the_module_and_by_the_general_function(rows, n, k, out, monkeypatch):

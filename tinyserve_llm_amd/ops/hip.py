@@ -1826,9 +1826,9 @@ WHOLE_TILES = {"bf16": ((2, 3.37, 0.894, 0.374, 0.555, 0.314, 0.124, 0.303), (1,
 # of W and of y
 WHOLE_LIBRARY = {"bf16": (6.10, 0.431, 1.371, 1.152, 0.418, 0.329), "f32": (5.25, 0.551, 1.564, 1.093, 0.432, 0.862)}
 # the share of that, both as estimated, up to which whole tiles are taken: of few rows (inside a pass bfloat16 products of 500 to 650 rows were 1 % of the
-# pass slower than timed by themselves), of more, and of many in 32 bits with a wide W
-WHOLE_FEW_SHARE, WHOLE_SHARE, WHOLE_WIDE_SHARE = 0.92, 0.98, 1.03
-WHOLE_FEW, WHOLE_MANY, WHOLE_WIDE = {"bf16": 960, "f32": 450}, 960, 8192
+# pass slower than timed by themselves) and of more; of many in 32 bits with a wide W of ragged columns, and of even ones, which the library's tiles divide
+WHOLE_FEW_SHARE, WHOLE_SHARE, WHOLE_RAGGED_SHARE, WHOLE_EVEN_SHARE = 0.92, 0.98, 1.03, 0.94
+WHOLE_FEW, WHOLE_MANY, WHOLE_WIDE, WHOLE_EVEN = {"bf16": 960, "f32": 450}, 960, 8192, 128
 WHOLE_MIN_ROWS, WHOLE_MAX_ROWS = 129, 3072      # fewer rows: the kernels that share x
 WHOLE_MIN_WIDTH, WHOLE_MAX_WIDTH, WHOLE_MIN_K = 2048, 12800, 1024
 
@@ -1852,14 +1852,25 @@ def _whole_library(rows: int, n: int, k: int, ending: str) -> float:
 @functools.lru_cache(maxsize=4096)
 def whole_plan(rows: int, n: int, k: int, ending: str) -> int | None:
     """The tile of `gemm_whole` for `rows` rows of x against a weight [n, k]; None where the matrix library may well be as fast. Both sides are estimates
-    fitted to 836 measured points with weights from memory (129 to 6,000 rows, n 256 to 16,384, k 256 to 5,120; 3 to 9 % root mean square within these limits). Of 530 of
-    them that lie within these limits and are not for slices, the rule takes 137, at 0.93 of the library's time on average; 7 of them are slower by more than 2 %, all in
-    bfloat16 and wide: n 8,192, k 2,048, 2,048 rows 52.5 and 56.8 µs the most. Library and here: bfloat16, n 12,352, k 2,048, 999 rows 58.4 and 50.6; 32 bits, the same
+    fitted to 836 measured points with weights from memory (129 to 6,000 rows, n 256 to 16,384, k 256 to 5,120; 3 to 9 % root mean square within these limits) and tried on 676
+    more (160 to 2,600 rows, n 6,144 to 14,336, k 2,048 and 4,096). A wide W whose columns are whole multiples of 128 is the library's in bfloat16, and in 32 bits below 960 rows: the
+    estimates promised 9 % on average at 103 such points, and 61 were no faster (library and here: 12,288 x 2,048, 1,150 rows 53.4 and 59.3, 8,192 x 2,048, 2,048 rows 52.5 and 56.8, 12,288 x 4,096, 800 rows 70.9 and 81.5), where ragged columns
+    cost the library a tenth. Of 1,154 points within these limits that are not for slices the rule takes 242, at 0.92 of the library's time in bfloat16 and 0.94 in 32 bits; 8 of them are slower by more than 2 %: bfloat16
+    7,168 x 2,048 and x 4,096, 2,048 rows, 52.9 and 56.6, 86.3 and 92.3, 32 bits 9,280 x 2,048 and x 4,096, 1,280 rows, 51.0 and 56.1, 89.9 and 98.9, and four by up to 5 %. Beyond 12,800 columns (14,336 and 16,384 measured) the estimates promise a gain at 45
+    points, and 21 of these are. Library and here: bfloat16, n 12,352, k 2,048, 999 rows 58.4 and 50.6; 32 bits, the same
     62.7 and 55.3, n 10,304, k 2,048, 2,048 rows 98.2 and 88.4, n 2,048, k 2,048, 720 rows 14.8 and 13.9, 257 rows (left to the library) 11.6 and 13.0."""
     if (not WHOLE_MIN_ROWS <= rows <= WHOLE_MAX_ROWS or not WHOLE_MIN_WIDTH <= n <= WHOLE_MAX_WIDTH or n % 8 or k % 64 or k < WHOLE_MIN_K):
         return None
+    share = WHOLE_SHARE
+    if n >= WHOLE_WIDE and n % WHOLE_EVEN == 0:
+        if ending == "bf16" or rows < WHOLE_MANY:
+            return None
+        share = WHOLE_EVEN_SHARE
+    elif rows < (WHOLE_MANY if n >= WHOLE_WIDE else WHOLE_FEW[ending]):
+        share = WHOLE_FEW_SHARE
+    elif n >= WHOLE_WIDE and ending == "f32":
+        share = WHOLE_RAGGED_SHARE
     us, tile = _whole_cost(rows, (n,), k, ending)
-    share = WHOLE_FEW_SHARE if rows < WHOLE_FEW[ending] else WHOLE_WIDE_SHARE if rows >= WHOLE_MANY and n >= WHOLE_WIDE and ending == "f32" else WHOLE_SHARE
     return tile if us < share * _whole_library(rows, n, k, ending) else None
 
 
@@ -1954,7 +1965,7 @@ def group_plan(rows: int, widths: "tuple[int, ...]", k: int, packed: bool) -> in
     apart = 0.0
     for n in widths:
         alone = _whole_library(rows, n, k, "f32")
-        apart += alone if whole_plan(rows, n, k, "f32") is None else min(alone, _whole_cost(rows, (n,), k, "f32")[0])
+        apart += alone if n < WHOLE_WIDE and whole_plan(rows, n, k, "f32") is None else min(alone, _whole_cost(rows, (n,), k, "f32")[0])
     return tile if us < (GROUP_WIDE_SHARE if max(widths) >= WHOLE_WIDE else 1.0) * apart else None
 
 

@@ -88,3 +88,12 @@ def test_the_rule_takes_what_was_measured_faster():
         assert not few(rows, n, k)
     for rows, n, k in ((1, 16384, 2048), (4, 16384, 4096), (8, 8192, 3072), (32, 8192, 3072), (16, 4096, 2048), (8, 16448, 2048), (33, 16384, 2048)):
         assert not few(rows, n, k, True)
+
+
+def test_the_gate_s_line_is_a_bound_on_the_reduction():
+    few = hip.rows64_few
+    for rows in (5, 16):
+        assert all(few(rows, 8192, k, True) for k in (1024, 2048)) and not any(few(rows, 8192, k, True) for k in (3072, 4096))
+        assert all(few(rows, 8320, k, True) for k in (1024, 2048, 3072, 4096)) and not any(few(rows, 8064, k, True) for k in (1024, 2048, 3072, 4096))
+    for rows in (17, 32):
+        assert few(rows, 8192, 2048, True) and not few(rows, 8192, 1024, True) and not few(rows, 11264, 1024, True) and few(rows, 16384, 1024, True)

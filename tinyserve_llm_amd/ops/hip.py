@@ -1302,24 +1302,30 @@ def rows64_takes(rows: int, n: int, k: int, glu: bool = False) -> bool:
             and n % 64 == 0 and k % 1024 == 0)
 
 
-ROWS64_FEW_WIDTH = 8192      # rows of W beyond which few rows of x are this kernel's
+ROWS64_FEW_WIDTH = 8192      # rows of W beyond which few rows of x are this kernel's, with the gate over reductions up to
+ROWS64_FEW_GATE_K = 2048     # this from so many on
+ROWS64_FEW_SHORT_K, ROWS64_FEW_SHORT_WIDTH = 1024, 16384      # and more than 16 rows over so short a reduction only from so many
 
 
 def rows64_few(rows: int, n: int, k: int, glu: bool = False) -> bool:
     """Whether up to 32 rows of x against a weight [n, k] are `gemm_rows32`'s and not the weight-streaming kernels' or the library's. The sums have the
     bits of the 16-row form's; up to 4 rows a plain product stays with the 8-row form, whose sums are nearer to 64 bits, and a gated one gains
     nothing inside a step (1 row by itself 14.5 and 13.9, a step of 12 layers 579 and 585). Measured, µs, before and here,
-    k 2,048: the gate, n 16,384, 8 rows 14.8 and 13.4, 32 rows 17.1 and 14.0, n 8,192, 8 rows 10.4 and 9.4, 32 rows 12.5 and 10.0, n 4,096, 32 rows (left) 7.3 and 8.7; plain and 32-bit, n 128,256, 8 rows 90.9 and 83.1, 16 rows 103 and 86, 32 rows 127 and 91, n
+    k 2,048: the gate, n 16,384, 8 rows 14.8 and 13.4, 32 rows 17.1 and 14.0, n 8,192, 8 rows 10.4 and 9.4, 32 rows 12.5 and 10.0, n 7,680 and 7,168 (left), 8 rows 8.4 and 8.7, 8.2
+    and 8.8, 32 rows 9.7 and 9.8, 9.3 and 9.8, n 4,096, 32 rows (left) 7.3 and 8.7; plain and 32-bit, n 128,256, 8 rows 90.9 and 83.1, 16 rows 103 and 86, 32 rows 127 and 91, n
     12,288, 5 rows 13.2 and 11.2, 32 rows 16.6 and 13.3, n 8,192, 8 rows (left) 9.1 both, 32 rows 14.7 and 11.4, n 5,120, 8 rows (left) 8.1 and 8.0, 16
     rows 8.9 and 8.0, 32 rows 12.5 and 9.7, n 4,096, 32 rows (left) 7.0 and 8.3. k 3,072: the gate, n 16,384, 8 rows 21.5 and 18.8, n 8,192, 8 rows (left) 12.3 and
-    12.8; plain, n 5,120, 24 rows (left) 14.0 and 13.4, n 8,192, 24 rows 19.5 and 15.9. k 4,096: plain, n 8,192, 8 rows (left) 15.8 and 16.6, 24 rows
+    12.8, n 8,320, 8 rows 17.1 and 11.9; k 1,024: the gate behind a prepared norm, n 8,192, 8 rows 7.5 and 6.5, 16 rows 6.9 and 6.4, 17 rows (left) 7.8 and 8.3, n 7,168, 16 rows (left) 5.7
+    and 6.3, n 11,264, 17 rows (left) 8.4 and 8.6, n 16,384, 17 rows 10.0 and 9.4; the gate alone, n 8,192, 8 rows 5.9 and 6.0, 16 rows 6.4 and 6.0, n 16,384, 5 rows 8.2 and 8.5, 16 rows 8.6 and 8.4. k 3,072: plain, n 5,120, 24 rows (left) 14.0 and 13.4, n 8,192, 24 rows 19.5 and 15.9. k 4,096: plain, n 8,192, 8 rows (left) 15.8 and 16.6, 24 rows
     (left) 16.9 and 20.4, n 16,384, 24 rows 34.0 and 27.0."""
     if not 1 <= rows < ROWS64_MIN_ROWS or n % (128 if glu else 64) or k % 1024 or not 1024 <= k <= 4096:
         return False
     if rows <= 4:
         return False
     if glu:
-        return n > ROWS64_FEW_WIDTH or (n == ROWS64_FEW_WIDTH and k == 2048)
+        if k <= ROWS64_FEW_SHORT_K and rows > SKINNY_FUSED_ROWS:
+            return n >= ROWS64_FEW_SHORT_WIDTH
+        return n >= ROWS64_FEW_WIDTH if k <= ROWS64_FEW_GATE_K else n > ROWS64_FEW_WIDTH
     if rows <= SKINNY_FUSED_ROWS:
         return n > ROWS64_FEW_WIDTH or (rows > 8 and n >= 5120 and k <= 3072)
     return n >= (5120 if k <= 2048 else 8192 if k <= 3072 else ROWS64_FEW_WIDTH + 64) and n * k > SKINNY_WIDE_ELEMENTS

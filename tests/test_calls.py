@@ -181,3 +181,16 @@ def test_a_group_of_products(stub):
     assert module.gemm_slices(many, ws, 0, None) is not None and called() and module.gemm_slices(many, ws, 0, packed) is None
     for other in (bf(6, 16, 64, 8), bf(5, 32, 64, 8), packed.float()):
         assert module.gemm_slices(xs, ws, 0, other) is None and called() == []
+
+
+def test_the_two_meanings_of_a_q_k_v_call_are_kept_apart(stub, monkeypatch):
+    """The module tells a packed weight from one as it is; neither general function takes the other's."""
+    module, answer, called = stub
+    monkeypatch.setattr(hip, "_native", lambda: module)
+    weight, packed, rest = bf(512, 1024), bf(32, 32, 64, 8), (torch.zeros(9, 64), ints(0, 1, 2), ints(0, 1, 2), *caches(), 4, 2, 64)
+    hip.qkv_rope_store_sliced(bf(3, 1024), packed, 2, *rest), hip.qkv_rope_store_whole(bf(3, 1024), weight, 2, *rest)
+    assert called() == ["ts_gemm_rows64_sliced_rope_bf16", "ts_gemm_whole_rope_bf16"]
+    for bad in (lambda: hip.qkv_rope_store_sliced(bf(3, 1024), weight, 2, *rest), lambda: hip.qkv_rope_store_whole(bf(3, 1024), packed, 2, *rest)):
+        with pytest.raises(hip.KernelError):
+            bad()
+    assert called() == []

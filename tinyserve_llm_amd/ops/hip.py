@@ -1579,8 +1579,9 @@ def qkv_rope_store_sliced(x: torch.Tensor, packed_rope: torch.Tensor, slices: in
     second kernel that adds the parts, rotates and writes the cache: q [tokens, nh, hd] comes back.
     `packed_rope` = pack_weight_rope(weight, head_dim). With `squares` (and `eps`) x is the operand of
     a `PreparedNorm` and the rows' scales multiply the finished sums."""
+    # (of a weight as it is the module makes `qkv_rope_store_whole`)
     q = _native().qkv_rope_store_sliced(x, packed_rope, slices, cos_sin, positions, slots, k_cache, v_cache, num_heads, num_kv_heads,
-                                        head_dim, eps, squares)
+                                        head_dim, eps, squares) if packed_rope.dim() == 4 else None
     if q is not None:
         return q
     _gpu(x, packed_rope, cos_sin, positions, slots, k_cache, v_cache)
@@ -2093,7 +2094,8 @@ def qkv_rope_store_whole(x: torch.Tensor, weight: torch.Tensor, tile: int, cos_s
                          k_cache: torch.Tensor | None, v_cache: torch.Tensor | None, num_heads: int, num_kv_heads: int, head_dim: int) -> torch.Tensor:
     """`rope_store(x · weight^T in bfloat16, ...)` for many rows of x in one kernel (gemm_whole.hip), whole heads of a multiple of 64;
     `tile` by its place in `WHOLE_ROPE_TILES`."""
-    q = _native().qkv_rope_store_sliced(x, weight, tile, cos_sin, positions, slots, k_cache, v_cache, num_heads, num_kv_heads, head_dim, 0.0, None)
+    q = _native().qkv_rope_store_sliced(x, weight, tile, cos_sin, positions, slots, k_cache, v_cache, num_heads, num_kv_heads, head_dim, 0.0,
+                                        None) if weight.dim() == 2 else None
     if q is not None:
         return q
     _gpu(x, weight, cos_sin, positions, slots, k_cache, v_cache)

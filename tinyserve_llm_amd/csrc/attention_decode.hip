@@ -21,17 +21,21 @@
 // 2,560 keys take 137 µs instead of 122); the instance with a single step per wave has room for 8
 #define DEC_WAVES_FOR(HD, ONE) ((HD) > 64 && !(ONE) ? 4 : DEC_MAX_WAVES)
 
-// Bytes of keys and values that a launch walks from which they go by the caches: they are put out before the next step reads them again, and
-// what they put out are the weights' and the other kernels' lines. Decode steps of 12 layers of the 1B widths over 2,048 keys, through the
-// caches and past them: 64 rows (302 MB a layer) 1,415 and 1,379 us, 16 rows (75 MB) 833 and 811, 12 rows (57 MB) 789 and 770; 8 rows (38 MB) 685 and
-// 689, 8 rows over 500 keys (13 MB) 625 and 629.
+// Bytes of keys and values, counted from what the tables have room for (from the window, where that is less), from which values go by the
+// caches: they are put out before the next step reads them again, and what they put out are the weights' and the other kernels' lines. Decode steps of
+// 12 layers of the 1B widths, through the caches and past them, us: over 2,048 keys 16 rows (67 MB a layer) 825 and 817, 64 rows 1,358 and 1,337, 96 rows 1,878 and 1,821, over 4,096
+// keys 48 rows 1,644 and 1,572, 64 rows 2,059 and 1,911, over 1,024 keys 24 rows 770 both, 96 rows 1,398 and 1,384; 8 layers of heads of 128 over 2,048 keys, 16 rows 873 and 852, 64 rows 1,633 and 1,533; below,
+// 8 rows over 2,048 keys (34 MB) 685 and 689, with the keys. With pages that all requests share as with their own: 64 rows over 2,048 keys, 7 of 9 pages shared, 1,096 and 1,081.
+// Keys too where a wave has a single step of heads up to 64 wide: 16 rows over 2,048 keys 819 and 806, 48 rows 1,193 and 1,181; in the loop over several steps, where half of each
+// line is asked for a second time, it has gone by then (20 rows over 3,072 keys 928 and 972, 96 rows over 1,024 keys 1,384 and 1,444). But not of pages that the next token's request
+// has too, which reads them at once (16 rows over 2,048 keys, 8 of 9 pages shared: 759 and 766).
 #define DEC_ONCE_BYTES (48ll << 20)
 
 // ONE: a wave has a single 32-key step (chunk = 32 waves); without the second buffer of the
 // general loop the kernel needs fewer registers and more workgroups share a compute unit
 // GENERAL: capped scores, weights in two terms (attention_mfma.h), and optionally a sink: one more in the
 // softmax's denominator, added where a token's chunks meet (here with one chunk, else in the combining kernel).
-// ONCE: keys and values by load_once (DEC_ONCE_BYTES).
+// ONCE: values by load_once, and some keys (DEC_ONCE_BYTES).
 template <int HD, bool ONE, bool GENERAL, bool ONCE>
 __global__ void __launch_bounds__(DEC_WAVES_FOR(HD, ONE) * TS_WAVE)
 attn_decode_mfma_kernel(bf16_t* __restrict__ out, float* __restrict__ part_o, float* __restrict__ part_ml,
@@ -55,8 +59,15 @@ attn_decode_mfma_kernel(bf16_t* __restrict__ out, float* __restrict__ part_o, fl
   const int r = lane & 15, g = lane >> 4;
   const int split = blockIdx.x, kvh = blockIdx.y, t = blockIdx.z;
   int pos = positions[t];
+  constexpr bool KEYS = ONCE && ONE && HD <= 64;
+  int next = t, next_seq = 0;                   // KEYS: the token after this one (before it, of the last), and its request
+  if constexpr (KEYS) {
+    next = t + 1 < (int)gridDim.z ? t + 1 : max(t - 1, 0);
+    next_seq = seq_of_token[next];
+  }
   int seq = seq_of_token[t];                    // (asked for with the position: one trip to memory, not one after the other;
   asm volatile("" : "+s"(pos), "+s"(seq));      //  left to itself the compiler fetches it when it has seen that the chunk is visible)
+  if constexpr (KEYS) asm volatile("" : "+s"(next_seq));
   const int lo = ts_first_key(pos, window);
   const int k0 = split * chunk;
   if (k0 > pos || k0 + chunk <= lo) return;     // nothing of this chunk is visible
@@ -83,15 +94,22 @@ attn_decode_mfma_kernel(bf16_t* __restrict__ out, float* __restrict__ part_o, fl
   int kend = k0 + chunk;
   if (kend > pos + 1) kend = pos + 1;
   int kb = (k0 > (lo & ~31) ? k0 : (lo & ~31)) + 32 * wave;
-#define TS_LOAD(T, KB) load_tile<HD, ONCE>(T, KB, r, g, lo, pos, kvh, table, pm, k_cache, v_cache, kp, ks, kh, vp, vh, vd)
+#define TS_LOAD_AS(KEYS_ONCE, T, KB) load_tile<HD, KEYS_ONCE, ONCE>(T, KB, r, g, lo, pos, kvh, table, pm, k_cache, v_cache, kp, ks, kh, vp, vh, vd)
+#define TS_LOAD(T, KB) TS_LOAD_AS(false, T, KB)
   // (the general variant: this row's head's penalty per position of distance, in the scores' units before scale2)
   const float slope = (GENERAL && slopes && r < G) ? slopes[kvh * G + r] * (1.44269504088896340736f / scale2) : 0.f;
 #define TS_USE(T, KB) use_tile_auto<HD, GENERAL>(T, KB, r, g, lo, pos, pos, lo, qreg, scale2, m, l, o, cap_in, cap_out, slope)
   if (ONE) {
     if (kb < kend) {
       KVTile<HD> A;
-      TS_LOAD(A, kb);
-      TS_USE(A, kb);
+      const int entry = pm.page(kb) >> page_run;      // (KEYS: of this step, whose page is looked up in any case)
+      if (KEYS && !(next != t && block_tables[(int64_t)next_seq * max_blocks + entry] == table[entry])) {
+        TS_LOAD_AS(KEYS, A, kb);      // (the products in both arms: where these meet the compiler waits for every load)
+        TS_USE(A, kb);
+      } else {
+        TS_LOAD(A, kb);
+        TS_USE(A, kb);
+      }
     }
   } else if (kb < kend) {
     // (the next step is asked for on every path, this step again where there is none: with a load that
@@ -112,6 +130,7 @@ attn_decode_mfma_kernel(bf16_t* __restrict__ out, float* __restrict__ part_o, fl
     }
   }
 #undef TS_LOAD
+#undef TS_LOAD_AS
 #undef TS_USE
   // ---- the waves meet
   l = row_sum(l);
@@ -243,7 +262,7 @@ static int launch_decode(void* out, float* part_o, float* part_ml, const void* q
     while ((1 << page_shift) < page_size) ++page_shift;
   }
   dim3 grid(num_splits, nkv, num_tokens);
-  const int64_t reach = (int64_t)num_splits * chunk, keys = window > 0 && window < reach ? window : reach;
+  const int64_t reach = (int64_t)num_splits * chunk, within = window < 0 ? -(int64_t)window : window, keys = within && within < reach ? within : reach;
   const bool once = (int64_t)num_tokens * nkv * hd * 4 * keys >= DEC_ONCE_BYTES;
   // capped: the cap's tanh takes the scale in and gives units of log2 out, and the softmax's own scale is 1
   const float log2e = 1.44269504088896340736f;

@@ -80,9 +80,9 @@ static __device__ __forceinline__ float row_sum(float x) {
 // operand registers. Every lane loads, whatever its keys, from an address inside the request's pages
 // (that of a visible key where its own is not), by the same instructions on every path: the compiler
 // can then count the loads under way and wait for a step's own only, while the next step's are in
-// flight. Keys outside [lo, pos] are masked by the softmax; values outside count as zeros (`vok`). ONCE: by load_once (of heads
-// wider than 64 the values only: 13 rows over 1,700 keys of 128 dimensions, a step of 8 layers 795 us, 801 with the keys too and with neither).
-template <int HD, bool ONCE>
+// flight. Keys outside [lo, pos] are masked by the softmax; values outside count as zeros (`vok`). KEYS, VALUES:
+// these by load_once.
+template <int HD, bool KEYS, bool VALUES>
 static __device__ __forceinline__ void load_tile(KVTile<HD>& T, int kb, int r, int g, int lo, int pos, int kvh,
                                                  const int32_t* __restrict__ table, const PageMath pm,
                                                  const bf16_t* __restrict__ k_cache, const bf16_t* __restrict__ v_cache,
@@ -116,9 +116,9 @@ static __device__ __forceinline__ void load_tile(KVTile<HD>& T, int kb, int r, i
 #pragma unroll
   for (int tau = 0; tau < 2; ++tau)
 #pragma unroll
-    for (int c = 0; c < NC; ++c) T.k[tau][c] = ONCE && HD <= 64 ? load_once(k_cache + koff[tau] + 32 * c) : *(const uint4*)(k_cache + koff[tau] + 32 * c);
+    for (int c = 0; c < NC; ++c) T.k[tau][c] = KEYS ? load_once(k_cache + koff[tau] + 32 * c) : *(const uint4*)(k_cache + koff[tau] + 32 * c);
 #pragma unroll
-  for (int db = 0; db < NDB; ++db) T.v[db] = ONCE ? load_once(v_cache + voff + (int64_t)(16 * db) * vd) : *(const uint4*)(v_cache + voff + (int64_t)(16 * db) * vd);
+  for (int db = 0; db < NDB; ++db) T.v[db] = VALUES ? load_once(v_cache + voff + (int64_t)(16 * db) * vd) : *(const uint4*)(v_cache + voff + (int64_t)(16 * db) * vd);
 }
 
 #define TS_LAZY_MAX 8.0f     // a row's reference maximum is raised when a score exceeds it by more than this (log2 units)

@@ -123,17 +123,56 @@ def test_wide_groups_of_many_rows_promise_more_than_the_estimates_err_by():
     assert hip.group_plan(2048, (6144, 8192), 4096, True) is None and hip.group_plan(900, (3104, 8192), 4096, True) is not None
 
 
-def test_small_results_are_left_out_of_whole_tiles():
+def test_small_results_go_along_in_chains_or_by_themselves():
     parts = hip.group_parts
-    for rows in (130, 600, 2048):
-        assert parts(rows, (2048,) * 4 + (64,), 2048, True) == (hip.group_plan(rows, (2048,) * 4, 2048, False), (4,))
-        assert parts(rows, (2048, 64), 2048, True) == (None, ()) and parts(rows, (2048, 64), 1024, True)[1] == ()
-    assert parts(129, (512, 2048, 1024), 2048, False)[1] == (0,) and parts(320, (512, 2048, 1024), 2048, False)[1] == ()
+    for rows in (130, 600, 1600):
+        assert parts(rows, (3072,) + (2048,) * 4 + (64, 32), 2048, True)[1:] == ((5, 6), ())
+        assert parts(rows, (2048, 64), 2048, True) == (None, (), ()) and parts(rows, (2048, 64), 1024, True)[1:] == ((), ())
+    assert parts(2048, (2048,) * 4 + (64,), 2048, True) == (hip.group_plan(2048, (2048,) * 4, 2048, False), (), (4,))
+    for rows in (129, 200, 330, 700, 1229, 2048):
+        for widths in ((512, 2048, 1024), (2048,) * 4 + (64,), (32, 2048, 2048)):
+            small = tuple(i for i, n in enumerate(widths) if rows * n <= 1 << 17)
+            assert parts(rows, widths, 2048, False)[1:] in ((small, ()), ((), small))
     for rows in (65, 80, 128):
-        assert parts(rows, (2048,) * 4 + (64,), 2048, True) == parts(rows, (1024,) * 3, 2048, True) == (-1, ())
-        assert parts(rows, (1024,) * 3, 2048, False) == (None, ()) and parts(rows, (1024,) * 3, 4096, True) == (None, ())
-    assert parts(80, (3104, 8192), 2048, True) == (-1, ()) and parts(80, (3104, 8192), 2048, False) == (None, ())
-    assert parts(96, (3104, 8192), 2048, True) == (hip.group_plan(96, (3104, 8192), 2048, True), ())
+        assert parts(rows, (2048,) * 4 + (64,), 2048, True) == parts(rows, (1024,) * 3, 2048, True) == (-1, (), ())
+        assert parts(rows, (1024,) * 3, 2048, False) == (None, (), ()) and parts(rows, (1024,) * 3, 4096, True) == (None, (), ())
+    assert parts(80, (3104, 8192), 2048, True) == (-1, (), ()) and parts(80, (3104, 8192), 2048, False) == (None, (), ())
+    assert parts(96, (3104, 8192), 2048, True) == (hip.group_plan(96, (3104, 8192), 2048, True), (), ())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tile", range(5))
+@pytest.mark.parametrize("rows, widths, k, chained", [(1, (8, 64), 768, (0,)), (130, (72, 264, 32), 832, (0, 2)), (300, (128, 64), 2048, (0, 1)), (257, (2048, 64), 1984, (1,))])
+def test_products_in_chains(tile, rows, widths, k, chained):
+    """A product cut into four is the four added up, bit for bit, and the others are what they were."""
+    xs, ws = group(rows, widths, k)
+    plain, got = hip.gemm_whole(xs, ws, tile, torch.float32), hip.gemm_whole(xs, ws, tile, torch.float32, chained)
+    ends = [0]
+    for i in range(4):
+        ends.append(ends[-1] + 64 * (k // 64 // 4 + (i < k // 64 % 4)))
+    for i, (x, w) in enumerate(zip(xs, ws)):
+        want = plain[i]
+        if i in chained:
+            parts = [hip.gemm_whole([x[:, a:b].contiguous()], [w[:, a:b].contiguous()], tile, torch.float32)[0] for a, b in zip(ends, ends[1:])]
+            want = ((parts[0] + parts[1]) + parts[2]) + parts[3]
+        assert torch.equal(got[i], want)
+    for bad in (lambda: hip.gemm_whole(xs, ws, tile, BF, chained), lambda: hip.gemm_whole(xs, ws, tile, torch.float32, (len(xs),)),
+                lambda: hip.gemm_whole([x[:, :704].contiguous() for x in xs], [w[:, :704].contiguous() for w in ws], tile, torch.float32, chained)):
+        with pytest.raises(hip.KernelError):
+            bad()
+
+
+@pytest.mark.gpu
+def test_a_group_with_small_results_by_the_module_and_by_the_general_function(monkeypatch):
+    import types
+    groups = [(300, (2048, 64, 2048, 32)), (2048, (2048, 2048, 64, 2048, 2048))]
+    assert [hip.group_parts(rows, widths, 2048, False)[1:] for rows, widths in groups] == [((1, 3), ()), ((), (2,))]
+    made = [group(rows, widths, 2048) for rows, widths in groups]
+    got = [hip.gemm_group(xs, ws, None) for xs, ws in made]
+    monkeypatch.setattr(hip, "_native", lambda: types.SimpleNamespace(gemm_slices=lambda *a: None, gemm_library=lambda *a: None))
+    for ys, (xs, ws) in zip(got, made):
+        assert all(torch.equal(a, b) for a, b in zip(ys, hip.gemm_group(xs, ws, None)))
+    assert torch.equal(got[1][2], hip.linear_bf16(made[1][0][2], made[1][1][2], torch.float32))
 
 
 @pytest.mark.gpu

@@ -239,7 +239,7 @@ bool packed16(const Tensor& p, int64_t K) {
 }
 
 // The products of a group (`gemm_group` of ops/hip.py), 32 bits on their way out: by the kernel that streams W past x where `packed` is given (the copies
-// of all the weights one behind the other), else in whole tiles.
+// of all the weights one behind the other), else in whole tiles (`tile`: and from its bit 8 on a bit for each product in chains).
 PyObject* group(PyObject* xs, PyObject* ws, const Tensor* packed, int tile) {
   constexpr Py_ssize_t most{8};
   if (!PyTuple_Check(xs) || !PyTuple_Check(ws)) return none();
@@ -269,7 +269,7 @@ PyObject* group(PyObject* xs, PyObject* ws, const Tensor* packed, int tile) {
   Tensor y[most];
   for (Py_ssize_t i = 0; i < n; ++i) y[i] = make(*x[0], {M, widths[i]}, at::kFloat), yp[i] = ptr(&y[i]);
   if (packed ? TS_REFUSED("gemm_rows64_group", ts_gemm_rows64_group_bf16(n, yp, xp, ptr(packed), widths, M, K, ldx, stream()))
-             : TS_REFUSED("gemm_whole", ts_gemm_whole_bf16(n, yp, xp, wp, widths, M, K, ldx, ldw, tile, 1, stream())))
+             : TS_REFUSED("gemm_whole", ts_gemm_whole_bf16(n, yp, xp, wp, widths, M, K, ldx, ldw, tile & 0xff, tile >> 8, 1, stream())))
     return none();
   PyObject* out = PyTuple_New(n);
   for (Py_ssize_t i = 0; out && i < n; ++i) PyTuple_SET_ITEM(out, i, wrap(y[i]));

@@ -24,7 +24,7 @@ int ts_gemm_library_bf16(void* y, const void* x, const void* w, int M, int N, in
 int ts_gemm_slices_bf16(void* y, void* sum, void* parts, const void* x, const void* w, int M, int N, int K, int64_t ldx, int64_t ldw, int tile,
                         int slices, int out_f32, const void* res, const void* norm_w, float eps, hipStream_t stream);
 int ts_gemm_whole_bf16(int products, void* const* y, const void* const* x, const void* const* w, const int* N, int M, int K, int64_t ldx, int64_t ldw,
-                       int tile, int out_f32, hipStream_t stream);
+                       int tile, int chained, int out_f32, hipStream_t stream);
 int ts_gemm_whole_rope_bf16(void* q_out, const void* x, const void* w, int M, int K, int64_t ldx, int64_t ldw, const float* cos_sin,
                             const int32_t* positions, const int32_t* slots, void* k_cache, void* v_cache, int nh, int nkv, int hd, int page_size,
                             int64_t kp, int64_t ks, int64_t kh, int64_t vp, int64_t vs, int64_t vh, int64_t vd, int tile, hipStream_t stream);

@@ -158,7 +158,7 @@ extern "C" int ts_gemm_slices_bf16(void* y, void* sum, void* parts, const void* 
                                    int tile, int slices, int out_f32, const void* res, const void* norm_w, float eps, hipStream_t stream) {
   if (M <= 0 || N <= 0) return TS_OK;
   if (K <= 0 || K % 64 || N % 8 || ldx < K || ldw < K || ldx % 8 || ldw % 8 || tile < 0 || tile > 4 || slices < 1 || slices > 64 || K / 64 / slices < TileProduct<64, 128, 1, 4, 3>::MIN_STEPS) return TS_BAD_SHAPE;
-  if (slices == 1 && !norm_w) return ts_gemm_whole_bf16(1, &y, &x, &w, &N, M, K, ldx, ldw, tile, out_f32, stream);
+  if (slices == 1 && !norm_w) return ts_gemm_whole_bf16(1, &y, &x, &w, &N, M, K, ldx, ldw, tile, 0, out_f32, stream);
   if (!x || !w || !y || !parts || (((uintptr_t)x | (uintptr_t)w | (uintptr_t)y | (uintptr_t)parts) & 15)) return TS_BAD_SHAPE;
   if ((int64_t)M * N >= (1ll << 40) || 256 * ldx * 2 >= (1ll << 31) || 256 * ldw * 2 >= (1ll << 31)) return TS_TOO_LARGE;      // (byte offsets from a tile's start)
   if (norm_w && (out_f32 || !sum || N > 8 * GS_THREADS * GS_HELD || (((uintptr_t)sum | (uintptr_t)res | (uintptr_t)norm_w) & 15))) return TS_BAD_SHAPE;

@@ -9,11 +9,16 @@
 #include "tile_product.h"
 
 #define GW_PRODUCTS 8           // products of one launch
+// A product's sums are one chain of its whole reduction, or GW_CHAINS of it, whose sums a tile adds up in memory: as near to 64 bits as the library's for
+// small results, which it splits (600 x 64 over 2,048: 1.3e-7, one chain 2.7e-7). A tile of so many chains begins as many times, and the launch begins with
+// these: 3,072, 2,048 four times, 64 and 32 columns over 2,048, the last two in chains, 320 rows 26.6 µs, with the two by the library 41.2, all in one chain each 25.3.
+#define GW_CHAINS 4
 
 struct WholeProduct {
   const bf16_t *x, *w;
   void* y;                      // [M, N], 32-bit or bfloat16
   int N, first;                 // columns, and its first tile of columns among those of all products
+  int chains;                   // that its reduction is cut into, one after the other, each added to y (32-bit)
 };
 struct WholeArgs {
   WholeProduct p[GW_PRODUCTS];
@@ -44,20 +49,38 @@ __global__ __launch_bounds__(WM * WN * TS_WAVE, 2) void gemm_whole_kernel(const 
     const int at = Tile::w_row(q);
     woff[q] = (uint32_t)(min(at, p.N - 1 - c0) * a.ldw * 2) + Tile::piece(at);
   }
-  float4_t acc[Tile::TN][Tile::TM];
-  Tile::run(lds, load_base(p.x + (int64_t)m0 * a.ldx), load_base(p.w + (int64_t)c0 * a.ldw), xoff, woff, a.steps, acc);
   const int lane = threadIdx.x % TS_WAVE, r = lane % 16, g = lane / 16, wm = wave_index() % WM, wn = wave_index() / WM;
+  float4_t acc[Tile::TN][Tile::TM];
+  if constexpr (WIDE) {
+    const int base = a.steps / p.chains, longer = a.steps % p.chains;      // (the first chains take a step more where they are uneven)
+    int64_t k0 = 0;
+#pragma unroll 1
+    for (int q = 0; q < p.chains; ++q) {
+      const int steps = base + (q < longer ? 1 : 0);
+      if (q) __syncthreads();      // every wave has read the chain before's last operands
+      Tile::run(lds, load_base(p.x + (int64_t)m0 * a.ldx + k0), load_base(p.w + (int64_t)c0 * a.ldw + k0), xoff, woff, steps, acc);
+      k0 += 64 * (int64_t)steps;
 #pragma unroll
-  for (int i = 0; i < Tile::TM; ++i) {
-    const int m = m0 + (wm * Tile::TM + i) * 16 + r;
-    const int64_t row = (int64_t)m * p.N;
-    if constexpr (WIDE) {
+      for (int i = 0; i < Tile::TM; ++i) {
+        const int m = m0 + (wm * Tile::TM + i) * 16 + r;
+        const int64_t row = (int64_t)m * p.N;
 #pragma unroll
-      for (int j = 0; j < Tile::TN; ++j) {
-        const int c = c0 + (wn * Tile::TN + j) * 16 + 4 * g;
-        if (m < a.M && c < p.N) *(float4_t*)((float*)p.y + row + c) = acc[j][i];
+        for (int j = 0; j < Tile::TN; ++j) {
+          const int c = c0 + (wn * Tile::TN + j) * 16 + 4 * g;
+          if (m < a.M && c < p.N) {
+            float4_t* const at = (float4_t*)((float*)p.y + row + c);
+            if (q) acc[j][i] += *at;
+            *at = acc[j][i];
+          }
+        }
       }
-    } else {
+    }
+  } else {
+    Tile::run(lds, load_base(p.x + (int64_t)m0 * a.ldx), load_base(p.w + (int64_t)c0 * a.ldw), xoff, woff, a.steps, acc);
+#pragma unroll
+    for (int i = 0; i < Tile::TM; ++i) {
+      const int m = m0 + (wm * Tile::TM + i) * 16 + r;
+      const int64_t row = (int64_t)m * p.N;
       // lane (r, g) holds columns 16 j + 4 g .. + 3 of row r: lanes g and g ^ 1 exchange so that each has eight in a row
 #pragma unroll
       for (int j = 0; j < Tile::TN; j += 2) {
@@ -92,16 +115,20 @@ static bool whole_operands_ok(const void* x, const void* w, int K, int64_t ldx, 
 
 // `products` of them in one launch (1 to 8), all of M rows and the reduction K: x[i] [M, K] and w[i] [N[i], K] bfloat16, 16-byte aligned, rows
 // ldx and ldw elements apart (multiples of 8), y[i] [M, N[i]] contiguous, 16-byte aligned, 32-bit or bfloat16; K a multiple of 64 of at least 3, N[i] of
-// 8. tile (rows of x by rows of W of a workgroup): 0 128 x 128, 1 128 x 256, 2 192 x 256, 3 256 x 256, 4 64 x 128.
+// 8. tile (rows of x by rows of W of a workgroup): 0 128 x 128, 1 128 x 256, 2 192 x 256, 3 256 x 256, 4 64 x 128. chained: a bit for each product whose
+// reduction is cut into GW_CHAINS chains (32-bit, K of 64 times 3 a chain).
 extern "C" int ts_gemm_whole_bf16(int products, void* const* y, const void* const* x, const void* const* w, const int* N, int M, int K, int64_t ldx,
-                                  int64_t ldw, int tile, int out_f32, hipStream_t stream) {
+                                  int64_t ldw, int tile, int chained, int out_f32, hipStream_t stream) {
   if (M <= 0) return TS_OK;
-  if (products < 1 || products > GW_PRODUCTS || !y || !x || !w || !N || tile < 0 || tile > 4) return TS_BAD_SHAPE;
+  if (products < 1 || products > GW_PRODUCTS || !y || !x || !w || !N || tile < 0 || tile > 4 || chained < 0 || chained >> products) return TS_BAD_SHAPE;
+  if (chained && (!out_f32 || K / 64 / GW_CHAINS < TileProduct<64, 128, 1, 4, 3>::MIN_STEPS)) return TS_BAD_SHAPE;
   WholeArgs a = {};
   a.products = products, a.M = M, a.steps = K / 64, a.ldx = ldx, a.ldw = ldw;
+  int at[2] = {0, __builtin_popcount(chained)};      // the next place of those in chains, which come first, and of the others
   for (int i = 0; i < products; ++i) {
     if (N[i] <= 0 || N[i] % 8 || !y[i] || ((uintptr_t)y[i] & 15) || !whole_operands_ok(x[i], w[i], K, ldx, ldw)) return TS_BAD_SHAPE;
-    a.p[i] = {(const bf16_t*)x[i], (const bf16_t*)w[i], y[i], N[i], 0};
+    const int in_chains = chained >> i & 1;
+    a.p[at[!in_chains]++] = {(const bf16_t*)x[i], (const bf16_t*)w[i], y[i], N[i], 0, in_chains ? GW_CHAINS : 1};
   }
   if (256 * ldx * 2 >= (1ll << 31) || 256 * ldw * 2 >= (1ll << 31)) return TS_TOO_LARGE;      // (byte offsets from a tile's start)
   switch (tile) {

@@ -91,7 +91,7 @@ def _declare(lib: ctypes.CDLL) -> None:
         "ts_gemm_skinny8_bf16": [p, p, p, i, i, i, i64, i64, i64, i, i, p, p, p, p, p, i, p, p, p, i, i, i, i, p],
         "ts_gemm_skinny8_act_bf16": [p, p, p, i, i, i, i64, i64, i64, i, i, p, i, p],
         "ts_gemm_slices_bf16": [p, p, p, p, p, i, i, i, i64, i64, i, i, i, p, p, f, p],
-        "ts_gemm_whole_bf16": [i, p, p, p, p, i, i, i64, i64, i, i, p],
+        "ts_gemm_whole_bf16": [i, p, p, p, p, i, i, i64, i64, i, i, i, p],
         "ts_gemm_whole_rope_bf16": [p, p, p, i, i, i64, i64, p, p, p, p, p, i, i, i, i, i64, i64, i64, i64, i64, i64, i64, i, p],
         "ts_gemm_rows64_bf16": [p, p, p, i, i, i, i64, i64, i, i, p, i, f, f, f, f, i, p],
         "ts_gemm_rows64_group_bf16": [i, p, p, p, p, i, i, i64, p],
@@ -1891,12 +1891,14 @@ def many_rows_plan(rows: int, n: int, k: int, ending: str) -> tuple[int, int] | 
     return plan
 
 
-WHOLE_PRODUCTS = 8                                                             # products of one launch
+WHOLE_PRODUCTS, WHOLE_CHAINS = 8, 4                                                             # products of one launch
 
 
-def gemm_whole(xs: "Sequence[torch.Tensor]", weights: "Sequence[torch.Tensor]", tile: int, out_dtype: torch.dtype = torch.bfloat16) -> "tuple[torch.Tensor, ...]":
+def gemm_whole(xs: "Sequence[torch.Tensor]", weights: "Sequence[torch.Tensor]", tile: int, out_dtype: torch.dtype = torch.bfloat16,
+               chained: "tuple[int, ...]" = ()) -> "tuple[torch.Tensor, ...]":
     """bfloat16 x [M, K] · weight [N, K]^T of up to 8 products of the same M, K and strides in one launch, each tile's reduction in one
-    workgroup (gemm_whole.hip); `tile` by its place in `SLICES_TILES`."""
+    workgroup (gemm_whole.hip); `tile` by its place in `SLICES_TILES`. `chained`: the places of the products (32-bit) whose reductions are four chains
+    of at least 192, added up in order."""
     _need(1 <= len(xs) == len(weights) <= WHOLE_PRODUCTS, lambda: f"{len(xs)} operands and {len(weights)} weights: one to {WHOLE_PRODUCTS} products")
     _gpu(*xs, *weights)
     _need(out_dtype in (torch.bfloat16, torch.float32), lambda: f"bfloat16 products come out as bfloat16 or float32, not {out_dtype}")
@@ -1907,13 +1909,19 @@ def gemm_whole(xs: "Sequence[torch.Tensor]", weights: "Sequence[torch.Tensor]", 
         _need(whole_takes(x, w), "products of whole tiles take bfloat16 operands with dense, 16-byte aligned rows, a reduction that is a "
               f"multiple of 64 from {64 * WHOLE_MIN_STEPS} on and widths that are multiples of 8")
     M, K = xs[0].shape
+    _need(not chained or (out_dtype is torch.float32 and K >= 64 * WHOLE_MIN_STEPS * WHOLE_CHAINS and all(0 <= i < len(xs) for i in chained)),
+          lambda: f"products {chained} of {len(xs)} in chains: 32-bit ones over {64 * WHOLE_MIN_STEPS * WHOLE_CHAINS} and more")
     ys = tuple(torch.empty((M, w.shape[0]), dtype=out_dtype, device=w.device) for w in weights)
     if M:
         n = len(ys)
         pointers = [(ctypes.c_void_p * n)(*(t.data_ptr() for t in ts)) for ts in (ys, xs, weights)]
         _run("gemm_whole", library().ts_gemm_whole_bf16(n, *pointers, (ctypes.c_int * n)(*(w.shape[0] for w in weights)), M, K, xs[0].stride(0),
-                                                        weights[0].stride(0), tile, int(out_dtype is torch.float32), _stream()))
+                                                        weights[0].stride(0), tile, _bits(chained), int(out_dtype is torch.float32), _stream()))
     return ys
+
+
+def _bits(places: "tuple[int, ...]") -> int:
+    return sum(1 << i for i in set(places))
 
 
 GROUP_FEW_ROWS = 64            # rows up to which a group goes to the kernel that streams W past x, beyond to whole tiles where these are as exact (`group_parts`)
@@ -1921,7 +1929,7 @@ GROUP_SURE_ROWS, GROUP_SURE_WIDTH, GROUP_MIN_ROWS = 9, 8192, 5      # two produc
 GROUP_LONG_K = 4096            # three products and more: up to this k also where it is not below the columns (from 5 rows on)
 GROUP_EVEN_ROWS, GROUP_SHORT_K = 16, 2048      # two products over more than 1,024: from these rows on up to k columns; of fewer rows, up to this k, only from 2 k columns on
 GROUP_CHAIN_ROWS, GROUP_WIDE_SHARE = 256, 0.92      # whole tiles of up to so many rows only for k below the columns; the share of the time one by one, both as estimated, that wide groups promise
-# products whose sums the matrix library may split into four chains: reductions beyond GROUP_CHAIN_K of results of at most GROUP_SPLIT_NUMBERS, and of up to
+# products whose sums the matrix library may split into chains: reductions beyond GROUP_CHAIN_K of results of at most GROUP_SPLIT_NUMBERS, and of up to
 # GROUP_SPLIT_ROWS rows and more than GROUP_SPLIT_WIDTH columns
 GROUP_CHAIN_K, GROUP_SPLIT_NUMBERS, GROUP_SPLIT_ROWS, GROUP_SPLIT_WIDTH = 1024, 1 << 17, 95, 2048
 GROUP_STREAM_K, GROUP_STREAM_MIN_WIDTH = 3072, 1024      # three products and more of 65 to 128 rows by the kernel that streams W: up to this k, from so many columns
@@ -1976,54 +1984,65 @@ def group_plan(rows: int, widths: "tuple[int, ...]", k: int, packed: bool) -> in
     return tile if us < (GROUP_WIDE_SHARE if max(widths) >= WHOLE_WIDE else 1.0) * apart else None
 
 
+GROUP_CHAINS_US = 5.0, 2.5      # what a tile's four chains add to a launch: fixed, and a thousand of k
+
+
 @functools.lru_cache(maxsize=4096)
-def group_parts(rows: int, widths: "tuple[int, ...]", k: int, packed: bool) -> "tuple[int | None, tuple[int, ...]]":
-    """(`group_plan` of the products made together, the places of those made by themselves): a product in whole tiles is one chain over all of k, and small
-    results are nearer to 64 bits by the library (of `rows` x 64 over 2,048 1.3e-7 and 2.7e-7, of 129 x 512 the same, of 320 x 512 2.7e-7 both, over 1,024
-    1.8e-7 both; where it splits follows from 1,000 measured results, GROUP_SPLIT_NUMBERS and GROUP_SPLIT_ROWS), or by the kernel that streams W (1.0e-7), which up
-    to 128 rows takes the whole group where it is the faster way, µs, one by one and together: 1,024 three times, k 2,048, 65 rows 24.8 and 12.7, 128 rows 25.4 and
-    16.2, k 4,096 (left) 36.0 and 27.9; 3,104 and 8,192, k 2,048, 80 rows 28.2 and 16.2; 1,024 twice, k 3,072 (left) 128 rows 15.6 and 21.9."""
+def group_parts(rows: int, widths: "tuple[int, ...]", k: int, packed: bool) -> "tuple[int | None, tuple[int, ...], tuple[int, ...]]":
+    """(`group_plan` of the products made together, the places of those of them that whole tiles make in four chains, the places of those made by themselves): a
+    product in whole tiles is one chain over all of k, and small results are nearer to 64 bits by the library (of `rows` x 64 over 2,048 1.3e-7 and
+    2.7e-7, of 129 x 512 the same, of 320 x 512 2.7e-7 both, over 1,024 1.8e-7 both; where it splits follows from 1,000 measured results, GROUP_SPLIT_NUMBERS and
+    GROUP_SPLIT_ROWS), or by the kernel that streams W (1.0e-7), which up to 128 rows takes the whole group where it is the faster way, µs, one by one and
+    together: 1,024 three times, k 2,048, 65 rows 24.8 and 12.7, 128 rows 25.4 and 16.2, k 4,096 (left) 36.0 and 27.9; 3,104 and 8,192, k 2,048, 80 rows 28.2
+    and 16.2; 1,024 twice, k 3,072 (left) 128 rows 15.6 and 21.9. Beyond, where two and more of the products are as near in one chain and pay together, the others
+    go along in chains or are the library's, by what both are estimated to take: 3,072, 2,048 four times, 64 and 32 over 2,048, the last two by the library and in chains,
+    130 rows 38.5 and 30.2, 1,600 rows 106.9 and 89.1; 2,048 four times and 64, 2,048 rows (by the library) 68.2 and 96.4."""
     plan = group_plan(rows, widths, k, packed)
     if plan is None or plan < 0 or k <= GROUP_CHAIN_K:
-        return plan, ()
-    alone = tuple(i for i, n in enumerate(widths) if rows * n <= GROUP_SPLIT_NUMBERS or (rows <= GROUP_SPLIT_ROWS and n > GROUP_SPLIT_WIDTH))
-    if not alone:
-        return plan, ()
+        return plan, (), ()
+    small = tuple(i for i, n in enumerate(widths) if rows * n <= GROUP_SPLIT_NUMBERS or (rows <= GROUP_SPLIT_ROWS and n > GROUP_SPLIT_WIDTH))
+    if not small:
+        return plan, (), ()
     if packed and _group_streams(rows, widths, k):
-        return -1, ()
-    plan = group_plan(rows, tuple(n for i, n in enumerate(widths) if i not in alone), k, False)
-    return (None, ()) if plan is None else (plan, alone)
+        return -1, (), ()
+    others = tuple(n for i, n in enumerate(widths) if i not in small)
+    plan = group_plan(rows, others, k, False)
+    if plan is None:
+        return None, (), ()
+    us, tile = _whole_cost(rows, widths, k, "f32")
+    apart = _whole_cost(rows, others, k, "f32")[0] + sum(_whole_library(rows, widths[i], k, "f32") for i in small)
+    return (tile, small, ()) if us + GROUP_CHAINS_US[0] + GROUP_CHAINS_US[1] * k / 1024 < apart else (plan, (), small)
 
 
 def gemm_group(xs: "Sequence[torch.Tensor]", weights: "Sequence[torch.Tensor]", packed: torch.Tensor | None) -> "tuple[torch.Tensor, ...] | None":
     """float32 x · weight^T of several bfloat16 products of the same rows and reduction in one launch, where that is the faster way and as exact (`group_parts`);
     None where not, or where their operands are another way. `packed`: the `pack_weight` copies of all the weights, one behind the other, if they are kept."""
-    x, w = xs[0], weights[0]
+    x = xs[0]
     if _many_rows != "library" or x.dim() != 2 or not x.is_cuda:
         return None
     rows, k = x.shape
-    widths = tuple([v.shape[0] for v in weights])
-    plan, alone = group_parts(rows, widths, k, packed is not None)
+    plan, chained, alone = group_parts(rows, tuple([v.shape[0] for v in weights]), k, packed is not None)
     if rows == 0 or plan is None:
         return None
-    if alone:
-        ys = _group([t for i, t in enumerate(xs) if i not in alone], [t for i, t in enumerate(weights) if i not in alone], plan, None)
-        if ys is None or not all(t.shape == x.shape for t in xs):
-            return None
-        left = iter(ys)
-        return tuple([linear_bf16(xs[i], weights[i], torch.float32) if i in alone else next(left) for i in range(len(xs))])
-    return _group(xs, weights, plan, packed if plan < 0 else None)
+    if not alone:
+        return _group(xs, weights, plan, chained, packed if plan < 0 else None)
+    ys = _group([t for i, t in enumerate(xs) if i not in alone], [t for i, t in enumerate(weights) if i not in alone], plan, (), None)
+    if ys is None or not all(t.shape == x.shape for t in xs):
+        return None
+    left = iter(ys)
+    return tuple([linear_bf16(xs[i], weights[i], torch.float32) if i in alone else next(left) for i in range(len(xs))])
 
 
-def _group(xs: "Sequence[torch.Tensor]", weights: "Sequence[torch.Tensor]", plan: int, packed: torch.Tensor | None) -> "tuple[torch.Tensor, ...] | None":
+def _group(xs: "Sequence[torch.Tensor]", weights: "Sequence[torch.Tensor]", plan: int, chained: "tuple[int, ...]",
+           packed: torch.Tensor | None) -> "tuple[torch.Tensor, ...] | None":
     """The products in one launch by the way `plan` of `group_plan`; None where it does not take the operands."""
-    done = _native().gemm_slices(tuple(xs), tuple(weights), plan, packed)
+    done = _native().gemm_slices(tuple(xs), tuple(weights), plan if not chained else plan | _bits(chained) << 8, packed)
     if done is not None:
         return done
     x, w = xs[0], weights[0]
     if not all(t.shape == x.shape and t.stride() == x.stride() and v.stride() == w.stride() and whole_takes(t, v) for t, v in zip(xs, weights)):
         return None
-    return gemm_whole(xs, weights, plan, torch.float32) if packed is None else gemm_rows64_group(xs, packed, [v.shape[0] for v in weights])
+    return gemm_whole(xs, weights, plan, torch.float32, chained) if packed is None else gemm_rows64_group(xs, packed, [v.shape[0] for v in weights])
 
 
 WHOLE_MIN_STEPS = 3      # steps of 64 that a tile's reduction has at least

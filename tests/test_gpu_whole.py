@@ -158,6 +158,11 @@ def test_the_rule_keeps_to_what_was_measured():
     assert plan(512, 3072, 2080) is None and plan(512, 1536, 128) is None
 
 
+def test_a_product_that_goes_in_slices_by_itself_is_left_apart():
+    sliced = [(rows, n, k) for n in (2048, 3072, 4096) for k in (5376, 6144, 8192) for rows in range(129, 2049, 13) if hip.slices_plan(rows, n, k, "bf16") is not None]
+    assert len(sliced) > 500 and all(hip.qkv_rope_whole_plan(*size) is None for size in sliced)
+
+
 def test_whole_tiles_are_taken_where_they_were_the_faster_way():
     for rows, n, k, ending, tile in ((999, 12352, 2048, "f32", (256, 256)), (2048, 10304, 2048, "f32", (192, 256)), (2048, 2048, 2048, "bf16", (128, 128)), (720, 2048, 2048, "f32", (64, 128))):
         plan, slices = hip.many_rows_plan(rows, n, k, ending)

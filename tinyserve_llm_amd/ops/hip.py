@@ -2057,7 +2057,7 @@ def whole_takes(x: torch.Tensor, weight: torch.Tensor) -> bool:
 # sizes, those of a step of 64 of K for a workgroup a compute unit (and for two, where it holds two), of a million numbers of W and of a million of the product
 WHOLE_ROPE_TILES = ((128, 128, 2, (3.97, 0.474, 0.748, 0.12, 1.17)), (128, 256, 1, (4.40, 0.723, 0.0, 0.06, 0.92)),
                     (192, 256, 1, (6.50, 0.906, 0.0, 0.0, 0.96)), (64, 128, 2, (3.15, 0.324, 0.537, 0.20, 0.84)))
-# what the product (by the matrix library or in slices) and the rotation's kernel take: fixed, a thousand of K, that times the root of the rows over 32,
+# what the product (the matrix library's: one in slices is left apart) and the rotation's kernel take: fixed, a thousand of K, that times the root of the rows over 32,
 # and a million products (of a thousand each), numbers of W and of the product
 WHOLE_ROPE_APART = (9.89, 1.506, 0.309, 1.233, 0.323, 1.167)
 WHOLE_ROPE_SHARE, WHOLE_ROPE_SURE_SHARE = 0.97, 0.9      # the share of that, both as estimated, up to which one kernel is taken; the second one up to
@@ -2075,7 +2075,7 @@ def qkv_rope_whole_plan(rows: int, n: int, k: int) -> int | None:
     shapes was: whole passes at 0.95 to 1.00 of their time). Apart and here: n 3,072, k 2,048 192 rows
     20.9 and 13.8, 513 rows 20.9 and 14.2, 1,024 rows 26.6 and 22.8, 2,048 rows 37.0 and 32.4, 3,000 rows 50.5 and 46.0; n 5,120, k 3,072
     192 rows (left apart) 32.3 and 27.8, 720 rows 39.9 and 34.4, 1,514 rows 59.5 and 49.4, 2,048 rows 72.4 and 59.6."""
-    if not WHOLE_ROPE_MIN_ROWS <= rows <= WHOLE_ROPE_MAX_ROWS or k % 64 or k < 64 * WHOLE_MIN_STEPS:
+    if not WHOLE_ROPE_MIN_ROWS <= rows <= WHOLE_ROPE_MAX_ROWS or k % 64 or k < 64 * WHOLE_MIN_STEPS or slices_plan(rows, n, k, "bf16") is not None:
         return None
     steps, costs = k // 64, []
     for bm, bn, held, (fixed, one, two, weight, out) in WHOLE_ROPE_TILES:

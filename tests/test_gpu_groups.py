@@ -23,7 +23,7 @@ def group(rows, widths, k, seed=0, skew=0):
 @pytest.mark.parametrize("rows", [1, 15, 16, 17, 63, 64, 65, 127, 128])
 @pytest.mark.parametrize("widths, k, skew", [([64, 16, 80, 32], 1024, 0), ([16], 2048, 8), ([48, 128, 2000, 64, 16, 16, 112, 64], 2048, 0)])
 def test_products_of_few_rows_in_one_launch(rows, widths, k, skew):
-    """32-bit sums of k products: 32 + (k / 128) roundings of stretches of 128 and of their sums, each at most 2^-24 of the sum of the products' sizes."""
+    """32-bit sums of k products: 128 + k / 128 roundings, those within a stretch of 128 and of the stretches' sums, each at most 2^-24 of the sum of the products' sizes."""
     xs, ws = group(rows, widths, k, skew=skew)
     ys = hip.gemm_rows64_group(xs, torch.cat([hip.pack_weight(w) for w in ws]), widths)
     for x, w, y in zip(xs, ws, ys):

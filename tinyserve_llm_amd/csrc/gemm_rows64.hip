@@ -27,7 +27,9 @@
 // 12,288 x 2,048, 5 rows 13.2 and 11.2; the gate of 16,384 x 2,048, 8 rows 14.8 and 13.4 (hip.rows64_few has more).
 //
 // W comes as the 16-row packed copy ([N / 16 tiles][K / 32 steps][64 lanes][8]); K is a multiple of
-// 1,024. A row of x meets W's k in ascending order in one accumulator, whatever the other rows are.
+// 1,024. A row of x meets W's k in ascending order, whatever the other rows are: in one accumulator over the
+// slice, or with FEW a chunk of 256 at a time, a group's a stretch of 128 at a time (in pairs of them up to 64
+// rows), the chunks' and stretches' sums added up in order.
 //
 // A narrow W (the o and down projections: 2,048 to 4,096 rows) has too few 64-row tiles to give every
 // compute unit a workgroup, so its reduction may be cut into slices (the grid's second dimension): the
@@ -47,6 +49,7 @@
                                   // 15.0 and 17.7, 90 rows 16.8 and 21.1, 128 rows 20.6 and 23.1; a head of 128,256 x 2,048, 64 rows 100.8 and 110.2;
                                   // in slices, with the finishing kernel, 2,048 x 8,192, 32 rows 12.6 and 14.0, 64 rows 14.0 and 14.8, 90 rows 15.6 and
                                   // 17.5, 3,072 x 3,072, 90 rows 16.6 and 19.9. (The ring alone 0.2 to 1.5 of it, the blocks 0.5 to 1.5, the caches the rest.)
+#define R64_SLICE_K (2 * R64_CHUNK_STEPS * 32)      // k that a slice has a multiple of: the staging waves take chunks two a turn, and meet the others at a barrier a chunk
 #define R64_STRETCH 4             // steps whose products a group's sums take together
 #define R64_STAGE_LOADS 8          // loads of a staging wave per chunk: two rows of its block each
 
@@ -77,7 +80,7 @@ struct Rows64GroupArgs : Rows64Args {
   float* ys[R64_PRODUCTS];             // [M, width]
 };
 
-// BLOCKS: blocks of 16 rows of x, 2, 4, 6 or 8 (beyond 64 rows the compute waves take a chunk's steps one at a time
+// BLOCKS: blocks of 16 rows of x, 1, 2, 4, 6 or 8 (beyond 64 rows the compute waves take a chunk's steps one at a time
 // instead of in pairs, for their registers' sake).
 // GLU: 0 none, 1 silu(gate) up, 1 + f the unit of form f of glu_unit.h.
 // With a group's arguments the sums are added up in stretches of 128 of K, with up to 64 rows in pairs of them, so that they are as near to 64 bits as
@@ -351,9 +354,15 @@ static int r64_launch(const Rows64Args& a, hipStream_t stream) {
     else gemm_rows64_kernel<GLU, OUT, 2, Rows64Args, true><<<grid, 512, r64_lds(2), stream>>>(a);
     return ts_check_launch();
   }
-  switch (r64_blocks(a.M)) {
-    case 1: gemm_rows64_kernel<GLU, OUT, 1, Rows64Args><<<grid, 512, r64_lds(1), stream>>>(a); break;
-    case 2: gemm_rows64_kernel<GLU, OUT, 2, Rows64Args><<<grid, 512, r64_lds(2), stream>>>(a); break;
+  // (fewer than 33 rows in this order of the sums are those of the products in slices, 32-bit and plain; others take four blocks for them)
+  if constexpr (GLU == 0 && std::is_same_v<OUT, float>) {
+    if (a.M <= 32) {
+      if (a.M <= 16) gemm_rows64_kernel<GLU, OUT, 1, Rows64Args><<<grid, 512, r64_lds(1), stream>>>(a);
+      else gemm_rows64_kernel<GLU, OUT, 2, Rows64Args><<<grid, 512, r64_lds(2), stream>>>(a);
+      return ts_check_launch();
+    }
+  }
+  switch (max(r64_blocks(a.M), 4)) {
     case 4: gemm_rows64_kernel<GLU, OUT, 4, Rows64Args><<<grid, 512, r64_lds(4), stream>>>(a); break;
     case 6: gemm_rows64_kernel<GLU, OUT, 6, Rows64Args><<<grid, 512, r64_lds(6), stream>>>(a); break;
     default: gemm_rows64_kernel<GLU, OUT, 8, Rows64Args><<<grid, 512, r64_lds(8), stream>>>(a);
@@ -501,7 +510,7 @@ extern "C" int ts_gemm_rows64_sliced_bf16(void* y, void* parts, const void* x, c
                                           int slices, const void* next_res, const void* next_nw, void* next_res_out,
                                           void* next_op, void* ssq_out, int64_t ld_op, hipStream_t stream) {
   if (M <= 0 || N <= 0) return TS_OK;
-  if (N % 64 || slices < 1 || slices > 64 || K % (512 * slices) || !parts || !r64_operands_ok(x, w16, M, N, K, ldx)) return TS_BAD_SHAPE;
+  if (N % 64 || slices < 1 || slices > 64 || K % (R64_SLICE_K * slices) || !parts || !r64_operands_ok(x, w16, M, N, K, ldx)) return TS_BAD_SHAPE;
   if (((uintptr_t)parts) & 15) return TS_BAD_SHAPE;
   Rows64FinishArgs f = {(const float*)parts, slices, M, N, (bf16_t*)y, (const bf16_t*)next_res, (const bf16_t*)next_nw,
                         (bf16_t*)next_res_out, (bf16_t*)next_op, (float*)ssq_out, ld_op};
@@ -640,7 +649,7 @@ extern "C" int ts_gemm_rows64_sliced_rope_bf16(void* q_out, void* parts, const v
   if (M <= 0) return TS_OK;
   if (nh <= 0 || nkv < 0 || hd <= 0 || hd % 32 || page_size <= 0) return TS_BAD_SHAPE;
   const int N = (nh + 2 * nkv) * hd;
-  if (N % 64 || slices < 1 || slices > 64 || K % (512 * slices) || !parts || !q_out || !r64_operands_ok(x, w16, M, N, K, ldx)) return TS_BAD_SHAPE;
+  if (N % 64 || slices < 1 || slices > 64 || K % (R64_SLICE_K * slices) || !parts || !q_out || !r64_operands_ok(x, w16, M, N, K, ldx)) return TS_BAD_SHAPE;
   if ((((uintptr_t)parts) & 15) || (((uintptr_t)q_out) & 7)) return TS_BAD_SHAPE;
   if (ssq_in && (ssq_parts <= 0 || (((uintptr_t)ssq_in) & 3))) return TS_BAD_SHAPE;
   if (rotate && (!cos_sin || !positions)) return TS_BAD_SHAPE;

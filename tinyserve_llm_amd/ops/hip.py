@@ -1407,7 +1407,7 @@ def gemm_rows64_group(xs: "Sequence[torch.Tensor]", packed: torch.Tensor, widths
     return ys
 
 
-ROWS64_SLICE_K = 512           # a slice of the reduction is a multiple of this (one turn of a compute wave's ring of W)
+ROWS64_SLICE_K = 512           # a slice of the reduction is a multiple of this (two chunks of x, which the staging waves take a turn)
 ROWS64_SLICED_MIN_ROWS = 5     # (fewer rows are the 8-row form's at any width; where the weight-streaming kernels serve a shape, they come first)
 ROWS64_WORKGROUPS = 192        # workgroups from which the chip's 256 compute units count as filled
 

@@ -180,10 +180,12 @@ class Mixer(Part):
     finishes_into_norm = False
     # True if forward() is 32-bit products of rows that follow from x alone, something between, and one product with the weight `o`, and the
     # mixer offers these apart, so that two mixers side by side share launches: `first_weights()` [(weight, its streaming copy or None)],
-    # `first_rows(x, ctx, mem)` the rows each of them multiplies, `between(sums, x, ctx, mem)` the last product's rows, `o` and `o_packed`. (`alone`: a
-    # mixer beside another leaves the copies that several products share to the pair.)
+    # `first_rows(x, ctx, mem)` the rows each of them multiplies, `between(sums, x, ctx, mem)` the last product's rows, `o` and `o_packed`.
     in_three = False
-    alone = True
+
+    def keep_product_copies(self) -> int:
+        """`keep_streaming_copies` of a mixer beside another, which keeps what several products share: a copy a weight."""
+        return self.keep_streaming_copies()
 
     def kv_spec(self) -> KVSpec | None:
         return None

@@ -97,7 +97,6 @@ class ShiftedDecayRecurrence(Mixer):
         self.o: torch.Tensor | None = None
         self.packed: dict[str, hip.StreamingCopies | None] = {}
         self.together: torch.Tensor | None = None      # the first products' packed copies, one behind the other
-        self.alone = True                              # (a mixer beside another leaves them to the pair)
 
     @property
     def size(self) -> int:
@@ -122,10 +121,13 @@ class ShiftedDecayRecurrence(Mixer):
         # (a long portion's chunks of 64 tokens each keep a state; the projections of GatedLinearAttention are wider than that)
         return max(super().widest_activation(), -(-self.size * self.head_dim // hip.SSD_CHUNK))
 
+    def keep_product_copies(self) -> int:
+        self.packed, self.together = {n: streaming_copy(getattr(self, n)) for n in ("r", "k", "v", "g", "o")}, None
+        return sum(c.nbytes() for c in self.packed.values() if c is not None)
+
     def keep_streaming_copies(self) -> int:
-        self.packed = {n: streaming_copy(getattr(self, n)) for n in ("r", "k", "v", "g", "o")}
-        held = sum(c.nbytes() for c in self.packed.values() if c is not None)
-        self.together, more = packed_together(self.first_weights()) if self.alone else (None, 0)
+        held = self.keep_product_copies()
+        self.together, more = packed_together(self.first_weights())
         return held + more
 
     @property

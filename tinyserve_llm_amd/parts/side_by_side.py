@@ -49,11 +49,9 @@ class SideBySide(Mixer):
         return max(self.left.widest_activation(), self.right.widest_activation())
 
     def keep_streaming_copies(self) -> int:
-        if self.in_threes:
-            self.right.alone = self.left.alone = False
-        held = self.left.keep_streaming_copies() + self.right.keep_streaming_copies()
         if not self.in_threes:
-            return held
+            return self.left.keep_streaming_copies() + self.right.keep_streaming_copies()
+        held = self.left.keep_product_copies() + self.right.keep_product_copies()
         self.first_together, first = packed_together(self.left.first_weights() + self.right.first_weights())
         self.last_together, last = packed_together([(m.o, m.o_packed) for m in (self.left, self.right)])
         return held + first + last

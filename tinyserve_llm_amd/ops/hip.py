@@ -1962,7 +1962,7 @@ def group_plan(rows: int, widths: "tuple[int, ...]", k: int, packed: bool) -> in
     there), a tile of `gemm_whole`, or None: one by one, which may well be as fast. Measured, µs, one by one and together: widths 2,048 four times and 64, k
     2,048: 1 row 17.6 and 9.5, 8 rows 19.1 and 9.7, 48 rows 50.0 and 12.0, 128 rows 50.4 and 18.0, 600 rows 66.5 and 32.9, 2,048 rows 109 and 83; 2,048 twice: 1 row (left) 7.4 and 8.5, 16 rows 10.4 and 8.8, 48 rows 21.0 and 11.4, 128 rows 22.5 and 18.1, 1,024
     rows 37.3 and 24.6; 3,104 and 8,192: 4 rows (left: the 8-row form's sums are nearer to 64 bits) 13.4 and 11.3, 8 rows 14.0 and 11.3, 48
-    rows 20.9 and 13.0, 96 rows 27.9 and 19.8, 1,024 rows 63.1 and 54.3, 1,500 rows (left) 77.6 and 86.0. Whole tiles over 1,100 points (65 to 2,600 rows, k 1,024 to
+    rows 20.9 and 13.0, 96 rows 27.9 and 19.8, 1,024 rows 63.1 and 54.3, 1,500 rows (left) 77.6 and 86.0. Whole tiles over 924 points (66 to 2,600 rows, k 1,024 to
     8,192): 2,048 twice, k 4,096, 129 rows (left) 29.5 and 30.6, 320 rows 43.3 and 31.9; with a width of 8,192, whose estimates err most, 0.77 of the time one by one on average and 2 of
     167 slower, by 2 and 3 % (3,104 and 8,192, k 1,024, 1,500 rows, left, 53.5 and 56.3); without, 0.65 and none. A group with a product that would go by
     itself in slices (`slices_plan`) is left: 1,536 twice, k 8,192, 129 rows 31.7 and 52.9, errors 2.1e-7 and 5.7e-7."""

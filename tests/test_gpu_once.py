@@ -1,5 +1,5 @@
-"""Decode attention over more keys and values than go through the caches (DEC_ONCE_BYTES of attention_decode.hip): a token's result is that of the
-same token in a step of few, whose keys go through them, whether its request's pages are its own or shared."""
+"""What goes by the caches in large steps has the results of smaller ones, where it goes through them: decode attention over many keys and values
+(DEC_ONCE_BYTES of attention_decode.hip), whether a request's pages are its own or shared, and experts' products (`hip.moe_weights_once`)."""
 
 from __future__ import annotations
 
@@ -56,3 +56,23 @@ def test_a_token_s_result_does_not_depend_on_how_its_keys_come(layout, hd, page,
     for first in range(0, TOKENS, 5):
         part = list(range(first, min(first + 5, TOKENS)))
         assert torch.equal(attend(part), everyone[part])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("experts, top, tokens", [(4, 1, 4), (4, 1, 5), (4, 2, 31), (4, 2, 32), (16, 4, 4), (16, 4, 5), (16, 4, 63), (16, 4, 64)])
+@pytest.mark.parametrize("n, k", [(48, 512), (131, 1120)])
+def test_an_expert_s_rows_do_not_depend_on_how_its_matrices_come(experts, top, tokens, n, k):
+    g = torch.Generator().manual_seed(experts + tokens + n)
+    ids = torch.stack([torch.randperm(experts, generator=g)[:top] for _ in range(tokens)]).to(I32).cuda()
+    x, w = torch.randn(tokens, k, generator=g).to(BF).cuda(), (torch.randn(experts, 2 * n, k, generator=g) * k ** -0.5).to(BF).cuda()
+    assert hip.moe_weights_once(tokens * top, experts) == (experts < tokens * top < 16 * experts)
+    for args in (dict(out_dtype=torch.float32), dict(out_dtype=BF, glu=(1.2, 1.702, 1.0)), dict(out_dtype=BF, activation="relu2")):
+        together = hip.moe_gemm(x, w, hip.moe_group(ids, experts), per_token=True, **args).view(tokens, top, -1)
+        for t in range(tokens):
+            assert not hip.moe_weights_once(top, experts)
+            assert torch.equal(hip.moe_gemm(x[t:t + 1], w, hip.moe_group(ids[t:t + 1].contiguous(), experts), per_token=True, **args), together[t])
+
+
+def test_experts_matrices_go_by_the_caches_between_a_pair_and_a_tile_an_expert():
+    once = hip.moe_weights_once
+    assert not once(16, 16) and once(17, 16) and once(255, 16) and not once(256, 16) and not once(4, 128) and once(384, 64)

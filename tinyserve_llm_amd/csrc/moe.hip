@@ -461,11 +461,12 @@ moe_gemm_mfma_kernel(TO* __restrict__ out, const bf16_t* __restrict__ x, const b
 // Tiles of 16 rows, for steps of few tokens, where the experts' matrices are streamed once and nothing else counts:
 // a workgroup takes a tile's rows by 16 columns (with GLU: 16 gate and 16 up columns), and its four waves take a
 // quarter of K each, eight k-steps' loads in flight at a time, so that a step with one token still has a thousand
-// waves asking for memory. A row's loads go out side by side (two take a cache line) and by the caches: with four steps, through the caches
-// and each step's row and columns in turn, a decode step with two layers of 16 experts of 2,048 and 1,024, four choices each, took 633 us with 6
-// tokens, 686 with 16, 866 with 48 and 949 with 64, and takes 603, 657, 822 and 930. The quarters' sums meet through LDS and are added in the waves' order: a row's result
+// waves asking for memory. A row's loads go out side by side (two take a cache line): the two products of 32 experts of 3,072 and 1,536 over four choices each took
+// with four steps and each step's row and columns in turn 106 us with 8 tokens and 377 with 128, and take 96 and 322. ONCE: W goes by the caches, which leaves them to the
+// weights of other layers (a decode step with two layers of 16 experts of 2,048 and 1,024 beside two without, 6 tokens 600 and 589 us, 16 669 and 647, 48 850 and 821) but asks for each
+// line twice: by themselves the products above take 110 and 398 so. The quarters' sums meet through LDS and are added in the waves' order: a row's result
 // depends on K alone, not on the tile or the batch it lands in.
-template <bool GLU, typename TO>
+template <bool GLU, typename TO, bool ONCE>
 __global__ void __launch_bounds__(MOE_THREADS)
 moe_gemm_stream_kernel(TO* __restrict__ out, const bf16_t* __restrict__ x, const bf16_t* __restrict__ w,
                        const int32_t* __restrict__ sorted, const int32_t* __restrict__ tiles, int src_div, int N, int K,
@@ -499,7 +500,7 @@ moe_gemm_stream_kernel(TO* __restrict__ out, const bf16_t* __restrict__ x, const
 #pragma unroll
     for (int t = 0; t < SETS; ++t)
 #pragma unroll
-      for (int d = 0; d < DEPTH; ++d) fw[t][d] = load_once<moe_u32x4>(wp[t] + 32 * (s + d));
+      for (int d = 0; d < DEPTH; ++d) fw[t][d] = ONCE ? load_once<moe_u32x4>(wp[t] + 32 * (s + d)) : *(const moe_u32x4*)(wp[t] + 32 * (s + d));
 #pragma unroll
     for (int d = 0; d < DEPTH; ++d) fx[d] = *(const moe_u32x4*)(xp + 32 * (s + d));
     __builtin_amdgcn_sched_barrier(0);
@@ -728,7 +729,7 @@ moe_gemm_lds_kernel(TO* __restrict__ out, const bf16_t* __restrict__ x, const bf
 
 extern "C" int ts_moe_gemm(void* out, int out_dtype, const void* x, int x_dtype, const void* w, const int32_t* sorted,
                            const int32_t* tiles, int max_tiles, int tile_rows, int src_div, int N, int K, int glu, float limit,
-                           float slope, float shift, int act, hipStream_t stream) {
+                           float slope, float shift, int act, int once, hipStream_t stream) {
   if (max_tiles <= 0) return TS_OK;
   if (act < 0 || act > 1 || (glu && act)) return TS_BAD_SHAPE;
   if (N <= 0 || K <= 0 || src_div <= 0 || (tile_rows != 16 && tile_rows != 64 && tile_rows != 128 && tile_rows != 256)) return TS_BAD_SHAPE;
@@ -758,8 +759,8 @@ extern "C" int ts_moe_gemm(void* out, int out_dtype, const void* x, int x_dtype,
       dim3 grid(max_tiles, (N + 15) / 16);
       if (grid.y > 65535) return TS_BAD_SHAPE;
 #define MOE_STREAM(GLU, TO) \
-      moe_gemm_stream_kernel<GLU, TO><<<grid, MOE_THREADS, 0, stream>>>((TO*)out, (const bf16_t*)x, (const bf16_t*)w, sorted, tiles, \
-                                                                        src_div, N, K, limit, slope, shift, act)
+      (once ? moe_gemm_stream_kernel<GLU, TO, true> : moe_gemm_stream_kernel<GLU, TO, false>)<<<grid, MOE_THREADS, 0, stream>>>( \
+          (TO*)out, (const bf16_t*)x, (const bf16_t*)w, sorted, tiles, src_div, N, K, limit, slope, shift, act)
       if (glu && out_dtype == 1) MOE_STREAM(true, bf16_t);
       else if (!glu && out_dtype == 0) MOE_STREAM(false, float);
       else if (!glu && out_dtype == 1) MOE_STREAM(false, bf16_t);

@@ -118,7 +118,7 @@ def _declare(lib: ctypes.CDLL) -> None:
         "ts_conv_state_update": [p, p, i64, p, p, i, i, i, i, p],
         "ts_moe_route": [p, p, p, i, p, p, i, i, i, i, f, i, i, i, p, i, i, p],
         "ts_moe_group": [p, p, p, i, i, i, i, p],
-        "ts_moe_gemm": [p, i, p, i, p, p, p, i, i, i, i, i, i, f, f, f, i, p],
+        "ts_moe_gemm": [p, i, p, i, p, p, p, i, i, i, i, i, i, f, f, f, i, i, p],
         "ts_segment_rmsnorm": [p, i, i64, p, i64, i, p, f, i, p],
         "ts_segment_rmsnorm_pair": [p, i64, i, i, p, i, i, p, f, p, i, i, i, p],
         "ts_latent_finish": [p, p, i, p, i64, i, i, i, i, i, p, p, f, p, f, p, p, i, i64, i64, p, i64, i64, i, p],
@@ -2893,6 +2893,14 @@ def moe_tile_rows(pairs: int, experts: int, dtype: torch.dtype, k_sizes: "tuple[
     return MOE_WIDE_TILE_ROWS if wide else MOE_TILE_ROWS
 
 
+def moe_weights_once(pairs: int, experts: int) -> bool:
+    """Whether the experts' matrices go by the caches where tiles have 16 rows: of more than a pair an expert and fewer than a tile. Past the caches the products
+    take longer by themselves (`moe_gemm_stream_kernel`), and a step is the shorter where other layers' weights stay in them: two layers of 16 experts, four choices each, beside
+    two without, µs a step through the caches and past them, 4 rows 600 and 607, 5 rows 590 and 582, 16 rows 669 and 647, 48 rows 850 and 821, 56 rows 869 and 844, 64 rows 926 and
+    928, 96 rows 1,116 and 1,134; eight layers of 16 experts of half the width, 64 rows (tokens a second) 49,060 and 47,310."""
+    return experts < pairs < MOE_TILE_ROWS * experts
+
+
 def moe_group(ids: torch.Tensor, experts: int, tile_rows: int = MOE_TILE_ROWS) -> ExpertTiles:
     """Groups the step's pairs by expert and cuts the groups into tiles of up to `tile_rows` rows. A pair whose choice is
     `experts` or beyond (an identity expert, which has no matrices) lands in no tile."""
@@ -2933,7 +2941,8 @@ def moe_gemm(x: torch.Tensor, weights: torch.Tensor, grouped: ExpertTiles, out_d
     _need(grouped.tile_rows < MOE_LDS_TILE_ROWS or x.shape[1] % 64 == 0, "tiles of 128 and 256 rows: a reduction that is a multiple of 64")
     _run("moe_gemm", library().ts_moe_gemm(_ptr(out), _code(out_dtype), _ptr(x), _code(x.dtype), _ptr(weights), _ptr(grouped.sorted),
                                            _ptr(grouped.tiles), grouped.tiles.shape[0], grouped.tile_rows, grouped.top if per_token else 1, n, x.shape[1],
-                                           int(glu is not None), float(limit), float(slope), float(shift), ACTIVATIONS[activation], _stream()))
+                                           int(glu is not None), float(limit), float(slope), float(shift), ACTIVATIONS[activation],
+                                           int(moe_weights_once(P, grouped.experts)), _stream()))
     return out
 
 

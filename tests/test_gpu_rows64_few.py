@@ -91,8 +91,9 @@ def test_the_rule_takes_what_was_measured_faster():
 
 def test_the_gate_s_line_is_a_bound_on_the_reduction():
     few = hip.rows64_few
-    for rows in (5, 16):
-        assert all(few(rows, 8192, k, True) for k in (1024, 2048)) and not any(few(rows, 8192, k, True) for k in (3072, 4096))
-        assert all(few(rows, 8320, k, True) for k in (1024, 2048, 3072, 4096)) and not any(few(rows, 8064, k, True) for k in (1024, 2048, 3072, 4096))
-    for rows in (17, 32):
-        assert few(rows, 8192, 2048, True) and not few(rows, 8192, 1024, True) and not few(rows, 11264, 1024, True) and few(rows, 16384, 1024, True)
+    for rows in (5, 8, 9, 16):
+        assert few(rows, 8192, 2048, True) and not few(rows, 8192, 3072, True) and not few(rows, 8192, 4096, True)
+        assert all(few(rows, 8320, k, True) for k in (2048, 3072, 4096)) and not any(few(rows, 8064, k, True) for k in (1024, 2048, 3072, 4096))
+    for rows, n, taken in ((5, 16384, False), (7, 28672, False), (8, 8192, False), (8, 16384, True), (9, 8192, True), (16, 8192, True), (17, 11264, False), (17, 16384, True), (32, 8192, False)):
+        assert few(rows, n, 1024, True) == taken
+    assert few(17, 8192, 2048, True) and few(32, 8192, 2048, True)

@@ -1304,7 +1304,7 @@ def rows64_takes(rows: int, n: int, k: int, glu: bool = False) -> bool:
 
 ROWS64_FEW_WIDTH = 8192      # rows of W beyond which few rows of x are this kernel's, with the gate over reductions up to
 ROWS64_FEW_GATE_K = 2048     # this from so many on
-ROWS64_FEW_SHORT_K, ROWS64_FEW_SHORT_WIDTH = 1024, 16384      # and more than 16 rows over so short a reduction only from so many
+ROWS64_FEW_SHORT_K, ROWS64_FEW_SHORT_WIDTH = 1024, 16384      # and 8 rows, and more than 16, over so short a reduction only from so many, fewer not at all
 
 
 def rows64_few(rows: int, n: int, k: int, glu: bool = False) -> bool:
@@ -1315,16 +1315,17 @@ def rows64_few(rows: int, n: int, k: int, glu: bool = False) -> bool:
     and 8.8, 32 rows 9.7 and 9.8, 9.3 and 9.8, n 4,096, 32 rows (left) 7.3 and 8.7; plain and 32-bit, n 128,256, 8 rows 90.9 and 83.1, 16 rows 103 and 86, 32 rows 127 and 91, n
     12,288, 5 rows 13.2 and 11.2, 32 rows 16.6 and 13.3, n 8,192, 8 rows (left) 9.1 both, 32 rows 14.7 and 11.4, n 5,120, 8 rows (left) 8.1 and 8.0, 16
     rows 8.9 and 8.0, 32 rows 12.5 and 9.7, n 4,096, 32 rows (left) 7.0 and 8.3. k 3,072: the gate, n 16,384, 8 rows 21.5 and 18.8, n 8,192, 8 rows (left) 12.3 and
-    12.8, n 8,320, 8 rows 17.1 and 11.9; k 1,024: the gate behind a prepared norm, n 8,192, 8 rows 7.5 and 6.5, 16 rows 6.9 and 6.4, 17 rows (left) 7.8 and 8.3, n 7,168, 16 rows (left) 5.7
-    and 6.3, n 11,264, 17 rows (left) 8.4 and 8.6, n 16,384, 17 rows 10.0 and 9.4; the gate alone, n 8,192, 8 rows 5.9 and 6.0, 16 rows 6.4 and 6.0, n 16,384, 5 rows 8.2 and 8.5, 16 rows 8.6 and 8.4. k 3,072: plain, n 5,120, 24 rows (left) 14.0 and 13.4, n 8,192, 24 rows 19.5 and 15.9. k 4,096: plain, n 8,192, 8 rows (left) 15.8 and 16.6, 24 rows
+    12.8, n 8,320, 8 rows 17.1 and 11.9; k 1,024: the gate behind a prepared norm, n 8,192, 16 rows 6.9 and 6.4, 17 rows (left) 7.8 and 8.3, n 7,168, 16 rows (left) 5.7
+    and 6.3, n 11,264, 17 rows (left) 8.4 and 8.6, n 16,384, 17 rows 10.0 and 9.4; the gate alone, n 8,192, 8 rows (left) 5.9 and 6.0, 16 rows 6.4 and 6.0, n 16,384, 8 rows 8.2 and 8.4, and inside a step of 16 layers
+    5 rows (left) 8.8 and 9.2, a step of 12 rows 589 and 541. k 3,072: plain, n 5,120, 24 rows (left) 14.0 and 13.4, n 8,192, 24 rows 19.5 and 15.9. k 4,096: plain, n 8,192, 8 rows (left) 15.8 and 16.6, 24 rows
     (left) 16.9 and 20.4, n 16,384, 24 rows 34.0 and 27.0."""
     if not 1 <= rows < ROWS64_MIN_ROWS or n % (128 if glu else 64) or k % 1024 or not 1024 <= k <= 4096:
         return False
     if rows <= 4:
         return False
     if glu:
-        if k <= ROWS64_FEW_SHORT_K and rows > SKINNY_FUSED_ROWS:
-            return n >= ROWS64_FEW_SHORT_WIDTH
+        if k <= ROWS64_FEW_SHORT_K and (rows <= 8 or rows > SKINNY_FUSED_ROWS):
+            return rows >= 8 and n >= ROWS64_FEW_SHORT_WIDTH
         return n >= ROWS64_FEW_WIDTH if k <= ROWS64_FEW_GATE_K else n > ROWS64_FEW_WIDTH
     if rows <= SKINNY_FUSED_ROWS:
         return n > ROWS64_FEW_WIDTH or (rows > 8 and n >= 5120 and k <= 3072)

@@ -11,6 +11,8 @@
 // current device's current stream.
 #include <Python.h>
 
+#include <vector>
+
 #include <ATen/core/Tensor.h>
 #include <ATen/ops/empty.h>
 #include <ATen/ops/empty_strided.h>
@@ -181,8 +183,60 @@ PyObject* rmsnorm(Args a) {      // x, weight, eps, residual, want_residual -> (
   return Py_BuildValue("(NN)", wrap(out), second);
 }
 
-PyObject* stream_post_norm(Args a) {      // x, a, post weight, scale, post eps, weight, eps, out code or -1 -> rows or None
-  const Tensor *x = a.tensor(), *b = a.tensor(), *post = a.tensor(), *scale = a.maybe();
+// A branch's rows in parts: a tuple (parts [count, n, width]) or (one, its factor, the other, its factor).
+struct Parts {
+  const float* p = nullptr;
+  int64_t stride = 0;
+  int count = 0, scaled = 0;
+  float fa = 1.f, fb = 1.f;
+};
+bool in_parts(const Args& a) { return a.left > 0 && PyTuple_Check(*a.at); }
+Parts row_parts(Args& a, int64_t n, int64_t width) {
+  PyObject* tuple = a.next();
+  std::vector<PyObject*> items;
+  for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(tuple); ++i) items.push_back(PyTuple_GET_ITEM(tuple, i));
+  Args in{items.data(), (Py_ssize_t)items.size()};
+  const bool one = in.left == 1;
+  const Tensor* p = in.tensor();
+  Parts parts;
+  if (one) {
+    a.bad |= !in.done() || !f32(*p) || p->dim() != 3 || p->size(1) != n || p->size(2) != width || !p->is_contiguous() || !fits(p->size(0)) || p->size(0) < 1;
+    if (!a.bad) parts = {typed<float>(p), n * width, (int)p->size(0)};
+    return parts;
+  }
+  const float fa = in.number();
+  const Tensor* second = in.tensor();
+  const float fb = in.number();
+  a.bad |= !in.done();
+  for (const Tensor* t : {p, second}) a.bad = a.bad || !f32(*t) || !matrix(*t, n, width) || !t->is_contiguous();
+  const int64_t apart = a.bad ? 0 : (char*)second->data_ptr() - (char*)p->data_ptr();
+  a.bad |= apart % 4 != 0;
+  if (!a.bad) parts = {typed<float>(p), apart / 4, 2, 1, fa, fb};
+  return parts;
+}
+
+PyObject* stream_post_norm(Args a) {      // x, a (or in parts), post weight, scale, post eps, weight, eps, out code or -1 -> rows or None
+  const Tensor* x = a.tensor();
+  if (in_parts(a)) {
+    if (a.bad || x->dim() != 2) return none();
+    const int64_t n = x->size(0), width = x->size(1);
+    const Parts b = row_parts(a, n, width);
+    const Tensor *post = a.tensor(), *scale = a.maybe();
+    const float post_eps = a.number();
+    const Tensor* w = a.maybe();
+    const float eps = a.number();
+    const int out_code = a.i32();
+    if (!a.done() || out_code < 0 || out_code > 1 || !f32(*x) || !x->is_contiguous() || !fits(n) || !fits(width)) return none();
+    for (const Tensor* v : {post, scale, w})
+      if (v && !vector(*v, at::kFloat, width)) return none();
+    Tensor out = make(*x, {n, width}, out_code ? at::kBFloat16 : at::kFloat);
+    if (TS_REFUSED("stream_post_norm",
+                   ts_stream_post_norm_parts(typed<float>(x), b.p, b.stride, b.count, b.scaled, b.fa, b.fb, typed<float>(post), typed<float>(scale), post_eps, ptr(&out),
+                                             out_code, typed<float>(w), eps, n, width, stream())))
+      return none();
+    return wrap(out);
+  }
+  const Tensor *b = a.tensor(), *post = a.tensor(), *scale = a.maybe();
   const float post_eps = a.number();
   const Tensor* w = a.maybe();
   const float eps = a.number();
@@ -200,8 +254,26 @@ PyObject* stream_post_norm(Args a) {      // x, a, post weight, scale, post eps,
   return wrap(out);
 }
 
-PyObject* stream_update_norm(Args a) {      // x, a, b, mult, weight, eps, out code -> rows (one norm, no bias, no picked rows)
-  const Tensor *x = a.tensor(), *b1 = a.maybe(), *b2 = a.maybe();
+PyObject* stream_update_norm(Args a) {      // x, a, b (or in parts), mult, weight, eps, out code -> rows (one norm, no bias, no picked rows)
+  const Tensor *x = a.tensor(), *b1 = a.maybe();
+  if (in_parts(a)) {
+    if (a.bad || x->dim() != 2) return none();
+    const int64_t n = x->size(0), width = x->size(1);
+    const Parts b = row_parts(a, n, width);
+    const float mult = a.number();
+    const Tensor* w = a.tensor();
+    const float eps = a.number();
+    const int out_code = a.i32();
+    if (!a.done() || out_code < 0 || out_code > 1 || !f32(*x) || !x->is_contiguous() || code(*w) < 0 || !vector(*w, w->scalar_type(), width)) return none();
+    if ((b1 && !(f32(*b1) && matrix(*b1, n, width) && b1->is_contiguous())) || !fits(n) || !fits(width)) return none();
+    Tensor out = make(*x, {n, width}, out_code ? at::kBFloat16 : at::kFloat);
+    if (TS_REFUSED("stream_update_norm",
+                   ts_stream_update_norm_parts(typed<float>(x), typed<float>(b1), b.p, b.stride, b.count, b.scaled, b.fa, b.fb, mult, ptr(&out), out_code, ptr(w),
+                                               code(*w), eps, n, width, stream())))
+      return none();
+    return wrap(out);
+  }
+  const Tensor* b2 = a.maybe();
   const float mult = a.number();
   const Tensor* w = a.tensor();
   const float eps = a.number();
@@ -276,7 +348,8 @@ PyObject* group(PyObject* xs, PyObject* ws, const Tensor* packed, int tile) {
   return out;
 }
 
-// x, weight, tile, slices, 32-bit out, residual, norm weight, eps -> y, or with a norm weight (norm, sum); or, with tuples of operands: operands,
+// x, weight, tile, slices, 32-bit out, residual, norm weight, eps -> y, or with a norm weight (norm, sum); x, weight, tile, slices, 32-bit out -> the slices'
+// parts; or, with tuples of operands: operands,
 // weights, tile, packed copies -> the products of a `group`
 PyObject* gemm_slices(Args a) {
   if (a.left == 4) {
@@ -285,17 +358,24 @@ PyObject* gemm_slices(Args a) {
     const Tensor* packed = a.maybe();
     return a.done() ? group(xs, ws, packed, tile) : none();
   }
+  const bool leave = a.left == 5;
   const Tensor *x = a.tensor(), *w = a.tensor();
   const int tile = a.i32(), slices = a.i32();
   const bool wide = a.i32();
-  const Tensor *res = a.maybe(), *nw = a.maybe();
-  const float eps = a.number();
+  const Tensor *res = leave ? nullptr : a.maybe(), *nw = leave ? nullptr : a.maybe();
+  const float eps = leave ? 0.f : a.number();
   if (!a.done() || x->dim() != 2 || w->dim() != 2 || !bf16(*x) || !bf16(*w) || x->size(1) != w->size(1) || !pieces(*x) || !pieces(*w)) return none();
   const int64_t M = x->size(0), K = x->size(1), N = w->size(0);
   if (!M || !N || !fits(M) || !fits(N) || !fits(K) || x->stride(0) < K || w->stride(0) < K || slices < 1 || slices > 64 || (res && !nw)) return none();
   if (nw && (wide || !vector(*nw, at::kBFloat16, N) || !aligned(*nw))) return none();
   if (res && !(bf16(*res) && matrix(*res, M, N) && res->is_contiguous() && aligned(*res))) return none();
   if (N % 8 || K % 64) return none();
+  if (leave) {
+    if (!wide) return none();
+    Tensor parts = make(*x, {slices, M, N}, at::kFloat);
+    if (TS_REFUSED("gemm_slices", ts_gemm_slices_parts_bf16(typed<float>(&parts), ptr(x), ptr(w), M, N, K, x->stride(0), w->stride(0), tile, slices, stream()))) return none();
+    return wrap(parts);
+  }
   Tensor parts, y = make(*x, {M, N}, wide ? at::kFloat : at::kBFloat16), sum;
   if (nw || slices > 1) parts = make(*x, {slices, M, N}, at::kFloat);
   if (nw) sum = make(*x, {M, N}, at::kBFloat16);

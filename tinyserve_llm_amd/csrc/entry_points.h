@@ -23,6 +23,8 @@ int ts_gemm_library_bf16(void* y, const void* x, const void* w, int M, int N, in
                          int tune, void* flush, size_t flush_bytes, hipStream_t stream);
 int ts_gemm_slices_bf16(void* y, void* sum, void* parts, const void* x, const void* w, int M, int N, int K, int64_t ldx, int64_t ldw, int tile,
                         int slices, int out_f32, const void* res, const void* norm_w, float eps, hipStream_t stream);
+int ts_gemm_slices_parts_bf16(float* parts, const void* x, const void* w, int M, int N, int K, int64_t ldx, int64_t ldw, int tile, int slices,
+                              hipStream_t stream);
 int ts_gemm_whole_bf16(int products, void* const* y, const void* const* x, const void* const* w, const int* N, int M, int K, int64_t ldx, int64_t ldw,
                        int tile, int chained, int out_f32, hipStream_t stream);
 int ts_gemm_whole_rope_bf16(void* q_out, const void* x, const void* w, int M, int K, int64_t ldx, int64_t ldw, const float* cos_sin,
@@ -66,6 +68,10 @@ int ts_paged_attention_prefill_general(void* out, const void* q, const void* k_c
                                        hipStream_t stream);
 int ts_stream_post_norm(float* x, const float* a, const float* post_w, const float* scale, float post_eps, void* h, int h_dtype,
                         const float* w, float eps, int num_rows, int width, hipStream_t stream);
+int ts_stream_post_norm_parts(float* x, const float* p, int64_t stride, int count, int scaled, float fa, float fb, const float* post_w, const float* scale,
+                              float post_eps, void* h, int h_dtype, const float* w, float eps, int num_rows, int width, hipStream_t stream);
+int ts_stream_update_norm_parts(float* x, const float* a, const float* p, int64_t stride, int count, int scaled, float fa, float fb, float mult, void* h,
+                                int h_dtype, const void* w, int w_dtype, float eps, int num_rows, int width, hipStream_t stream);
 int ts_stream_update_norm(float* x, const void* a, int a_dtype, const void* b, int b_dtype, const void* bias, int bias_dtype, float mult,
                           void* h1, void* h2, int h_dtype, const void* w1, const void* w2, int w_dtype, float eps, const int32_t* rows,
                           int num_rows, int width, hipStream_t stream);

@@ -149,6 +149,26 @@ static int launch_slices(SlicesArgs a, hipStream_t stream) {
   return ts_check_launch();
 }
 
+// The slices' parts of a product.
+static int slices_parts(float* parts, const void* x, const void* w, int M, int N, int K, int64_t ldx, int64_t ldw, int tile, int slices, hipStream_t stream) {
+  if (K <= 0 || K % 64 || N % 8 || ldx < K || ldw < K || ldx % 8 || ldw % 8 || tile < 0 || tile > 4 || slices < 1 || slices > 64 || K / 64 / slices < TileProduct<64, 128, 1, 4, 3>::MIN_STEPS) return TS_BAD_SHAPE;
+  if (!x || !w || !parts || (((uintptr_t)x | (uintptr_t)w | (uintptr_t)parts) & 15)) return TS_BAD_SHAPE;
+  if ((int64_t)M * N >= (1ll << 40) || 256 * ldx * 2 >= (1ll << 31) || 256 * ldw * 2 >= (1ll << 31)) return TS_TOO_LARGE;      // (byte offsets from a tile's start)
+  const SlicesArgs a = {parts, (const bf16_t*)x, (const bf16_t*)w, M, N, K / 64, slices, 0, 0, 0, 0, ldx, ldw};
+  switch (tile) {
+    case 0: return launch_slices<128, 128, 2, 2, 2>(a, stream);
+    case 1: return launch_slices<128, 256, 2, 4, 2>(a, stream);
+    case 2: return launch_slices<192, 256, 2, 4, 2>(a, stream);
+    case 3: return launch_slices<256, 256, 2, 4, 2>(a, stream);
+    default: return launch_slices<64, 128, 1, 4, 3>(a, stream);
+  }
+}
+
+template <bool WIDE> static int slices_finish(void* y, const void* parts, int64_t size, int slices, hipStream_t stream) {
+  slices_finish_kernel<WIDE><<<(unsigned)((size / 4 + GS_THREADS - 1) / GS_THREADS), GS_THREADS, 0, stream>>>(y, (const float*)parts, size, slices);
+  return ts_check_launch();
+}
+
 // x [M, K] and w [N, K] bfloat16, 16-byte aligned, rows ldx and ldw elements apart (multiples of 8); K a multiple of 64 with at
 // least 3 steps of 64 a slice, N a multiple of 8. parts: float32 [slices][M][N], scratch that the call fills and reads. tile (rows of x by
 // rows of W of a workgroup): 0 128 x 128, 1 128 x 256, 2 192 x 256, 3 256 x 256, 4 64 x 128. y [M, N] contiguous, 32-bit or bfloat16; or, with
@@ -157,25 +177,27 @@ static int launch_slices(SlicesArgs a, hipStream_t stream) {
 extern "C" int ts_gemm_slices_bf16(void* y, void* sum, void* parts, const void* x, const void* w, int M, int N, int K, int64_t ldx, int64_t ldw,
                                    int tile, int slices, int out_f32, const void* res, const void* norm_w, float eps, hipStream_t stream) {
   if (M <= 0 || N <= 0) return TS_OK;
-  if (K <= 0 || K % 64 || N % 8 || ldx < K || ldw < K || ldx % 8 || ldw % 8 || tile < 0 || tile > 4 || slices < 1 || slices > 64 || K / 64 / slices < TileProduct<64, 128, 1, 4, 3>::MIN_STEPS) return TS_BAD_SHAPE;
   if (slices == 1 && !norm_w) return ts_gemm_whole_bf16(1, &y, &x, &w, &N, M, K, ldx, ldw, tile, 0, out_f32, stream);
-  if (!x || !w || !y || !parts || (((uintptr_t)x | (uintptr_t)w | (uintptr_t)y | (uintptr_t)parts) & 15)) return TS_BAD_SHAPE;
-  if ((int64_t)M * N >= (1ll << 40) || 256 * ldx * 2 >= (1ll << 31) || 256 * ldw * 2 >= (1ll << 31)) return TS_TOO_LARGE;      // (byte offsets from a tile's start)
+  if (!y || ((uintptr_t)y & 15)) return TS_BAD_SHAPE;
   if (norm_w && (out_f32 || !sum || N > 8 * GS_THREADS * GS_HELD || (((uintptr_t)sum | (uintptr_t)res | (uintptr_t)norm_w) & 15))) return TS_BAD_SHAPE;
-  const SlicesArgs a = {(float*)parts, (const bf16_t*)x, (const bf16_t*)w, M, N, K / 64, slices, 0, 0, 0, 0, ldx, ldw};
-  int rc;
-  switch (tile) {
-    case 0: rc = launch_slices<128, 128, 2, 2, 2>(a, stream); break;
-    case 1: rc = launch_slices<128, 256, 2, 4, 2>(a, stream); break;
-    case 2: rc = launch_slices<192, 256, 2, 4, 2>(a, stream); break;
-    case 3: rc = launch_slices<256, 256, 2, 4, 2>(a, stream); break;
-    default: rc = launch_slices<64, 128, 1, 4, 3>(a, stream);
-  }
+  const int rc = slices_parts((float*)parts, x, w, M, N, K, ldx, ldw, tile, slices, stream);
   if (rc != TS_OK) return rc;
   const int64_t size = (int64_t)M * N;
-  const unsigned blocks = (unsigned)((size / 4 + GS_THREADS - 1) / GS_THREADS);
-  if (norm_w) slices_norm_kernel<<<M, GS_THREADS, 0, stream>>>((bf16_t*)y, (bf16_t*)sum, (const float*)parts, (const bf16_t*)res, (const bf16_t*)norm_w, size, slices, N, eps);
-  else if (out_f32) slices_finish_kernel<true><<<blocks, GS_THREADS, 0, stream>>>(y, (const float*)parts, size, slices);
-  else slices_finish_kernel<false><<<blocks, GS_THREADS, 0, stream>>>(y, (const float*)parts, size, slices);
+  if (out_f32 && !norm_w) return slices_finish<true>(y, parts, size, slices, stream);
+  if (!norm_w) return slices_finish<false>(y, parts, size, slices, stream);
+  slices_norm_kernel<<<M, GS_THREADS, 0, stream>>>((bf16_t*)y, (bf16_t*)sum, (const float*)parts, (const bf16_t*)res, (const bf16_t*)norm_w, size, slices, N, eps);
   return ts_check_launch();
+}
+
+// The parts alone, float32 [slices][M][N], for a kernel that adds them up where it takes the rows (residual_stream.hip).
+extern "C" int ts_gemm_slices_parts_bf16(float* parts, const void* x, const void* w, int M, int N, int K, int64_t ldx, int64_t ldw, int tile, int slices,
+                                         hipStream_t stream) {
+  return M <= 0 || N <= 0 ? TS_OK : slices_parts(parts, x, w, M, N, K, ldx, ldw, tile, slices, stream);
+}
+
+// y: the sum of such parts of `size` numbers each (a multiple of 4), as ts_gemm_slices_bf16 stores it in 32 bits
+extern "C" int ts_slices_sum(float* y, const float* parts, int64_t size, int slices, hipStream_t stream) {
+  if (size <= 0) return TS_OK;
+  if (!y || !parts || size % 4 || slices < 1 || (((uintptr_t)y | (uintptr_t)parts) & 15)) return TS_BAD_SHAPE;
+  return slices_finish<true>(y, parts, size, slices, stream);
 }

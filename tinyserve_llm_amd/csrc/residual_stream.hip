@@ -85,22 +85,58 @@ stream_update_norm_kernel(float* __restrict__ x, const void* __restrict__ a, int
   }
 }
 
+// A branch's rows that are still to be added up: `count` parts of their shape, `stride` elements apart, the first one first
+// (a product in slices), or fa * the first + fb * the second (two mixers side by side). The stream's kernels add them where they
+// take the rows: as a kernel of its own the sum cost a launch and the rows' trip through memory and back (2,048 rows of 2,048, what makes the
+// sum and the stream's kernel apart and together: two slices 8.7 + 11.7 and 14.5 us, two mixers' sum 9.7 + 11.7 and 14.5).
+struct RowParts {
+  const float* p;
+  int64_t stride;
+  int count;
+  float fa, fb;
+};
+// HELD elements of a row from element `at` on, every RS_THREADS-th: P parts are asked for together (PAIR: the two that have factors), in the order that
+// `slices_finish_kernel` and `scaled_sum_kernel` add them.
+template <int P, bool PAIR, int HELD>
+static __device__ __forceinline__ void rs_parts_sum(float (&v)[HELD], const RowParts& parts, int64_t row, int width) {
+  for (int s0 = 0; s0 < parts.count; s0 += P) {
+    float part[P][HELD];
+#pragma unroll
+    for (int k = 0; k < P; ++k)
+#pragma unroll
+      for (int j = 0; j < HELD; ++j) {
+        const int i = min(threadIdx.x + j * RS_THREADS, width - 1);
+        part[k][j] = parts.p[min(s0 + k, parts.count - 1) * parts.stride + row + i];
+      }
+#pragma unroll
+    for (int j = 0; j < HELD; ++j) {
+      if constexpr (PAIR) {
+        v[j] = fmaf(parts.fb, part[1][j], parts.fa * part[0][j]);
+      } else {
+#pragma unroll
+        for (int k = 0; k < P; ++k) v[j] = s0 + k == 0 ? part[k][j] : s0 + k < parts.count ? v[j] + part[k][j] : v[j];
+      }
+    }
+  }
+}
+
 // The same for rows of up to RS_THREADS * HELD elements whose branches are 32-bit and whose norms' weights, bias and
 // outputs share the type H: every load of the row goes out before the first is used (no branch on a storage type
 // or on whether an operand is there stands between two loads: an operand that is not there is read from another of
 // its shape and counts times 0), and the updated row stays in registers between the sum of squares and the scaling.
+// With P, b is in parts, P of them asked for together.
 #define RS_HELD 16
-template <typename H, typename W, int HELD, bool NORMS>
+template <typename H, typename W, int HELD, bool NORMS, int P = 0, bool PAIR = false>
 __global__ void __launch_bounds__(RS_THREADS)
 stream_update_norm_held_kernel(float* __restrict__ x, const float* __restrict__ a, const float* __restrict__ b,
                                const H* __restrict__ bias, float mult, H* __restrict__ h1, H* __restrict__ h2,
                                const W* __restrict__ w1, const W* __restrict__ w2, float eps,
-                               const int32_t* __restrict__ rows, int width) {
+                               const int32_t* __restrict__ rows, int width, const RowParts parts = {}) {
   __shared__ float scratch[RS_THREADS / TS_WAVE];
   const int64_t r = blockIdx.x;
   const int64_t t = rows ? rows[r] : r;
   float* xr = x + t * width;
-  const bool update = a || b || bias, bias_on = bias;
+  const bool update = P || a || b || bias, bias_on = bias;
   // an operand that is not there is read from another of its size (the row itself; a norm's weight) and not used
   const float* ar = (a ? a : x) + t * width;
   const float* br = (b ? b : x) + t * width;
@@ -113,19 +149,20 @@ stream_update_norm_held_kernel(float* __restrict__ x, const float* __restrict__ 
     const int i = min(threadIdx.x + j * RS_THREADS, width - 1);     // (a lane beyond the row reads its last element, and stores nothing)
     v[j] = xr[i];
     va[j] = ar[i];
-    vb[j] = br[i];
+    if constexpr (!P) vb[j] = br[i];
     vbias[j] = Num<H>::ld(bs + i);
     if constexpr (NORMS) {
       wva[j] = Num<W>::ld(wa + i);
       wvb[j] = Num<W>::ld(wb + i);
     }
   }
+  if constexpr (P > 0) rs_parts_sum<P, PAIR>(vb, parts, t * width, width);
   float squares = 0.f;
 #pragma unroll
   for (int j = 0; j < HELD; ++j) {
     const int i = threadIdx.x + j * RS_THREADS;
     // x + mult * (a + b + bias), the sum of the branches first
-    const float add = (a ? va[j] : 0.f) + (b ? vb[j] : 0.f) + (bias_on ? vbias[j] : 0.f);
+    const float add = (a ? va[j] : 0.f) + (P || b ? vb[j] : 0.f) + (bias_on ? vbias[j] : 0.f);
     v[j] = update ? fmaf(mult, add, v[j]) : v[j];
     if (update && i < width) xr[i] = v[j];
     squares = i < width ? fmaf(v[j], v[j], squares) : squares;
@@ -178,12 +215,36 @@ extern "C" int ts_stream_update_norm(float* x, const void* a, int a_dtype, const
   return ts_check_launch();
 }
 
+static bool row_parts_ok(const float* p, int64_t stride, int count, int scaled) { return p && (stride || count == 1) && count >= 1 && (!scaled || count == 2); }
+
+// `ts_stream_update_norm` of x += mult * (a + b) and one norm, b in `count` parts, `stride` elements apart (with `scaled`: fa * the first + fb * the
+// second); a 32-bit or null, the norm's weight 32-bit or of its rows' type, rows of up to 4,096.
+extern "C" int ts_stream_update_norm_parts(float* x, const float* a, const float* p, int64_t stride, int count, int scaled, float fa, float fb, float mult, void* h,
+                                           int h_dtype, const void* w, int w_dtype, float eps, int num_rows, int width, hipStream_t stream) {
+  if (num_rows <= 0) return TS_OK;
+  if (width <= 0 || width > RS_THREADS * RS_HELD || !x || !h || !w || !row_parts_ok(p, stride, count, scaled)) return TS_BAD_SHAPE;
+  if ((h_dtype | w_dtype) & ~1 || (w_dtype == 1 && h_dtype == 0)) return TS_BAD_DTYPE;
+  const RowParts parts = {p, stride, count, fa, fb};
+#define RS_PARTS(H, W, HELD, P, PAIR) \
+  stream_update_norm_held_kernel<H, W, HELD, true, P, PAIR><<<num_rows, RS_THREADS, 0, stream>>>(x, a, nullptr, nullptr, mult, (H*)h, nullptr, (const W*)w, nullptr, \
+                                                                                                 eps, nullptr, width, parts)
+#define RS_PARTS_P(H, W, HELD) \
+  if (scaled) { RS_PARTS(H, W, HELD, 2, true); } else if (count <= 2) { RS_PARTS(H, W, HELD, 2, false); } else { RS_PARTS(H, W, HELD, 4, false); }
+#define RS_PARTS_H(H, W) \
+  if (width <= RS_THREADS * 4) { RS_PARTS_P(H, W, 4); } else if (width <= RS_THREADS * 8) { RS_PARTS_P(H, W, 8); } else { RS_PARTS_P(H, W, RS_HELD); }
+  if (h_dtype == 0) { RS_PARTS_H(float, float) } else if (w_dtype == 0) { RS_PARTS_H(bf16_t, float) } else { RS_PARTS_H(bf16_t, bf16_t) }
+#undef RS_PARTS_H
+#undef RS_PARTS_P
+#undef RS_PARTS
+  return ts_check_launch();
+}
+
 // out[t] = [x[t] + a[t] + b[t] | y[t]] (a, b: what branches have left pending, may be absent), rounded to out's storage
 // type: the stream after its sum beside other rows of its width, as a projection's operand. Nothing is written back.
-template <typename TO, bool BY4>
+template <typename TO, bool BY4, bool PARTS = false>
 __global__ void __launch_bounds__(RS_THREADS)
 stream_join_kernel(TO* __restrict__ out, const float* __restrict__ x, const void* __restrict__ a, int a_code,
-                   const void* __restrict__ b, int b_code, const float* __restrict__ y, int64_t items, int width) {
+                   const void* __restrict__ b, int b_code, const float* __restrict__ y, int64_t items, int width, const RowParts parts = {}) {
   for (int64_t idx = (int64_t)blockIdx.x * RS_THREADS + threadIdx.x; idx < items; idx += (int64_t)gridDim.x * RS_THREADS) {
     constexpr int N = BY4 ? 4 : 1;
     const int64_t at = idx * N, t = at / width;
@@ -193,8 +254,16 @@ stream_join_kernel(TO* __restrict__ out, const float* __restrict__ x, const void
       const float4 s = *(const float4*)(x + at), o = *(const float4*)(y + at);
       float4 add = make_float4(0.f, 0.f, 0.f, 0.f);
       if (a) add = *(const float4*)((const float*)a + at);
-      if (b) {
-        const float4 c = *(const float4*)((const float*)b + at);
+      if (PARTS || b) {
+        float4 c;
+        if constexpr (PARTS) {
+          for (int s = 0; s < parts.count; ++s) {
+            const float4 p = *(const float4*)(parts.p + s * parts.stride + at);
+            c = s == 0 ? p : make_float4(c.x + p.x, c.y + p.y, c.z + p.z, c.w + p.w);
+          }
+        } else {
+          c = *(const float4*)((const float*)b + at);
+        }
         add.x += c.x; add.y += c.y; add.z += c.z; add.w += c.w;
       }
       v[0] = s.x + add.x; v[1] = s.y + add.y; v[2] = s.z + add.z; v[3] = s.w + add.w;
@@ -233,6 +302,20 @@ extern "C" int ts_stream_join(void* out, int out_dtype, const float* x, const vo
   if (out_dtype == 0) { if (by4) RS_JOIN(float, true); else RS_JOIN(float, false); }
   else { if (by4) RS_JOIN(bf16_t, true); else RS_JOIN(bf16_t, false); }
 #undef RS_JOIN
+  return ts_check_launch();
+}
+
+// `ts_stream_join` with a 32-bit or null and b in `count` parts, `stride` elements apart; everything in whole 16-byte pieces.
+extern "C" int ts_stream_join_parts(void* out, int out_dtype, const float* x, const float* a, const float* p, int64_t stride, int count, const float* y, int num_rows,
+                                    int width, hipStream_t stream) {
+  if (num_rows <= 0) return TS_OK;
+  if (width <= 0 || width % 4 || stride % 4 || !x || !y || !row_parts_ok(p, stride, count, 0)) return TS_BAD_SHAPE;
+  if (((uintptr_t)out | (uintptr_t)x | (uintptr_t)a | (uintptr_t)p | (uintptr_t)y) & 15) return TS_BAD_SHAPE;
+  if (out_dtype & ~1) return TS_BAD_DTYPE;
+  const RowParts parts = {p, stride, count, 1.f, 1.f};
+  const int64_t items = (int64_t)num_rows * width / 4, blocks = min((items + RS_THREADS - 1) / RS_THREADS, (int64_t)16384);
+  if (out_dtype == 0) stream_join_kernel<float, true, true><<<(unsigned)blocks, RS_THREADS, 0, stream>>>((float*)out, x, a, 0, nullptr, 0, y, items, width, parts);
+  else stream_join_kernel<bf16_t, true, true><<<(unsigned)blocks, RS_THREADS, 0, stream>>>((bf16_t*)out, x, a, 0, nullptr, 0, y, items, width, parts);
   return ts_check_launch();
 }
 
@@ -341,12 +424,13 @@ stream_post_norm_kernel(float* __restrict__ x, const float* __restrict__ a, cons
 
 // The same for rows of up to RS_THREADS * HELD elements: every load of the row, the branch and the weights goes out before
 // the first is used, and the row stays in registers between the sums of squares and the scalings (a lane beyond the row
-// reads the row's last element and stores nothing). The sums are taken by the same tree over the same lanes' parts.
-template <typename H, int HELD>
+// reads the row's last element and stores nothing). The sums are taken by the same tree over the same lanes' parts. With P, the
+// branch is in parts, P of them asked for together.
+template <typename H, int HELD, int P = 0, bool PAIR = false>
 __global__ void __launch_bounds__(RS_THREADS)
 stream_post_norm_held_kernel(float* __restrict__ x, const float* __restrict__ a, const float* __restrict__ post_w,
                              const float* __restrict__ scale, float post_eps, H* __restrict__ h, const float* __restrict__ w,
-                             float eps, int width) {
+                             float eps, int width, const RowParts parts = {}) {
   __shared__ float scratch[RS_THREADS / TS_WAVE];
   const int64_t r = blockIdx.x;
   float* xr = x + r * width;
@@ -358,11 +442,12 @@ stream_post_norm_held_kernel(float* __restrict__ x, const float* __restrict__ a,
   for (int j = 0; j < HELD; ++j) {
     const int i = min(threadIdx.x + j * RS_THREADS, width - 1);
     v[j] = xr[i];
-    va[j] = ar[i];
+    if constexpr (!P) va[j] = ar[i];
     pw[j] = post_w[i];
     ps[j] = sc[i];
     nw[j] = wn[i];
   }
+  if constexpr (P > 0) rs_parts_sum<P, PAIR>(va, parts, r * width, width);
   float squares = 0.f;
 #pragma unroll
   for (int j = 0; j < HELD; ++j) squares = threadIdx.x + j * RS_THREADS < width ? fmaf(va[j], va[j], squares) : squares;
@@ -405,6 +490,26 @@ extern "C" int ts_stream_post_norm(float* x, const float* a, const float* post_w
     return ts_check_launch();
   }
   stream_post_norm_kernel<<<num_rows, RS_THREADS, 0, stream>>>(x, a, post_w, scale, post_eps, h, h_dtype, w, eps, width);
+  return ts_check_launch();
+}
+
+// `ts_stream_post_norm` of a branch in `count` parts, `stride` elements apart (with `scaled`: fa * the first + fb * the second); rows of up to 4,096.
+extern "C" int ts_stream_post_norm_parts(float* x, const float* p, int64_t stride, int count, int scaled, float fa, float fb, const float* post_w, const float* scale,
+                                         float post_eps, void* h, int h_dtype, const float* w, float eps, int num_rows, int width, hipStream_t stream) {
+  if (num_rows <= 0) return TS_OK;
+  if (width <= 0 || width > RS_THREADS * RS_HELD || !x || !post_w || !row_parts_ok(p, stride, count, scaled)) return TS_BAD_SHAPE;
+  if (h_dtype & ~1) return TS_BAD_DTYPE;
+  const RowParts parts = {p, stride, count, fa, fb};
+#define RS_POST(H, HELD, P, PAIR) \
+  stream_post_norm_held_kernel<H, HELD, P, PAIR><<<num_rows, RS_THREADS, 0, stream>>>(x, nullptr, post_w, scale, post_eps, (H*)h, w, eps, width, parts)
+#define RS_POST_P(H, HELD) \
+  if (scaled) { RS_POST(H, HELD, 2, true); } else if (count <= 2) { RS_POST(H, HELD, 2, false); } else { RS_POST(H, HELD, 4, false); }
+#define RS_POST_H(H) \
+  if (width <= RS_THREADS * 4) { RS_POST_P(H, 4); } else if (width <= RS_THREADS * 8) { RS_POST_P(H, 8); } else { RS_POST_P(H, RS_HELD); }
+  if (h_dtype == 0) { RS_POST_H(float) } else { RS_POST_H(bf16_t) }
+#undef RS_POST_H
+#undef RS_POST_P
+#undef RS_POST
   return ts_check_launch();
 }
 

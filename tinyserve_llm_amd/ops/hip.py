@@ -154,6 +154,11 @@ def _declare(lib: ctypes.CDLL) -> None:
         "ts_token_shift": [p, p, i, p, p, i64, p, p, p, i, i, i, p],
         "ts_token_shift_keep": [p, i64, p, i, p, p, i, i, p],
         "ts_stream_post_norm": [p, p, p, p, f, p, i, p, f, i, i, p],
+        "ts_stream_post_norm_parts": [p, p, i64, i, i, f, f, p, p, f, p, i, p, f, i, i, p],
+        "ts_stream_update_norm_parts": [p, p, p, i64, i, i, f, f, f, p, i, p, i, f, i, i, p],
+        "ts_stream_join_parts": [p, i, p, p, p, i64, i, p, i, i, p],
+        "ts_gemm_slices_parts_bf16": [p, p, p, i, i, i, i64, i64, i, i, p],
+        "ts_slices_sum": [p, p, i64, i, p],
         "ts_scaled_sum": [p, p, f, p, f, i64, p],
         "ts_gather_gate": [p, i, p, p, i, i64, i, p, i, i, i, p],
         "ts_qkv_prepare": [p, p, i, i, i, i, i, p, p, f, p, i, p],
@@ -2301,6 +2306,20 @@ def linear_bf16(x: torch.Tensor, weight: torch.Tensor, out_dtype: torch.dtype = 
     return gemm_library(x, weight, out_dtype)
 
 
+def linear_parts(x: torch.Tensor, weight: torch.Tensor, packed: StreamingCopies | None = None) -> RowParts | None:
+    """float32 x · weight^T left in its slices' parts, where `linear_bf16` would give the product to the slices and add the parts up; None where not."""
+    if not isinstance(x, torch.Tensor) or _many_rows != "library" or _library_tuning is not None or x.dim() != 2 or weight.shape[0] > STREAM_PARTS_MAX_WIDTH:
+        return None
+    rows, k = x.shape
+    if not _library_serves(rows, weight.shape[0], k, packed is not None and packed.by16 is not None, True):
+        return None
+    plan = many_rows_plan(rows, weight.shape[0], k, "f32")
+    if plan is None or plan[1] < 2:
+        return None
+    parts = _native().gemm_slices(x, weight, *plan, True)
+    return None if parts is None else RowParts(parts)
+
+
 def gemm_library_init() -> None:
     """Makes the matrix library's handle and workspace on the current device. Steps that are recorded
     into graphs need it done beforehand (the runner does it when it is made)."""
@@ -2415,20 +2434,52 @@ def embedding_stream(table: torch.Tensor, ids: torch.Tensor) -> torch.Tensor:
     return out
 
 
-def stream_update_norm(x: torch.Tensor, a: torch.Tensor | None = None, b: torch.Tensor | None = None,
+STREAM_PARTS_MAX_WIDTH = 4096      # rows whose parts the stream's kernels add up as they take them
+
+
+class RowParts:
+    """float32 rows [tokens, width] that are still to be added up: `parts` [count, tokens, width], the first one first, or, with `factors` = (fa, fb),
+    fa * parts[0] + fb * parts[1] of a pair of such rows. The stream's kernels take them as they are; `rows()` adds them up by a kernel of its own."""
+
+    def __init__(self, parts: "torch.Tensor | tuple[torch.Tensor, torch.Tensor]", factors: "tuple[float, float] | None" = None) -> None:
+        self.parts, self.factors = parts, factors
+
+    @property
+    def shape(self) -> torch.Size:
+        return self.parts[0].shape
+
+    def rows(self) -> torch.Tensor:
+        if self.factors is not None:
+            return scaled_sum(self.parts[0], self.factors[0], self.parts[1], self.factors[1])
+        _gpu(self.parts)
+        y = torch.empty(self.shape, dtype=torch.float32, device=self.parts.device)
+        _run("slices_sum", library().ts_slices_sum(_ptr(y), _ptr(self.parts), y.numel(), self.parts.shape[0], _stream()))
+        return y
+
+    def operands(self) -> tuple:
+        """As the library's own module takes them."""
+        return (self.parts,) if self.factors is None else (self.parts[0], self.factors[0], self.parts[1], self.factors[1])
+
+
+def added_up(rows: "torch.Tensor | RowParts | None") -> torch.Tensor | None:
+    return rows.rows() if isinstance(rows, RowParts) else rows
+
+
+def stream_update_norm(x: torch.Tensor, a: torch.Tensor | None = None, b: "torch.Tensor | RowParts | None" = None,
                        bias: torch.Tensor | None = None, mult: float = 1.0,
                        weights: "tuple[torch.Tensor | None, torch.Tensor | None]" = (None, None), eps: float = 0.0,
                        rows: torch.Tensor | None = None, out_dtype: torch.dtype = torch.float32
                        ) -> "tuple[torch.Tensor | None, torch.Tensor | None]":
     """The float32 stream x [tokens, width] takes x += mult * (a + b + bias) in place (a, b: what
-    parallel branches made, float32 or bfloat16, either may be None; bias [width] goes to every row), and
+    parallel branches made, float32 or bfloat16, either may be None, b possibly in parts; bias [width] goes to every row), and
     for each given weight norm(x) * weight of the updated rows comes back in `out_dtype` (both norms
     share the row's mean square). With `rows` (int32) nothing is updated and only those rows are
     normalised, in that order."""
     if rows is None and bias is None and weights[0] is not None and weights[1] is None and out_dtype in _DTYPE_CODE:
-        out = _native().stream_update_norm(x, a, b, mult, weights[0], eps, _DTYPE_CODE[out_dtype])
+        out = _native().stream_update_norm(x, a, b.operands() if isinstance(b, RowParts) else b, mult, weights[0], eps, _DTYPE_CODE[out_dtype])
         if out is not None:
             return out, None
+    b = added_up(b)
     _gpu(x, a, b, bias, rows, *weights)
     _need(x.dtype == torch.float32 and x.dim() == 2 and x.is_contiguous(), "the stream must be contiguous float32 [tokens, width]")
     tokens, width = x.shape
@@ -2451,15 +2502,26 @@ def stream_update_norm(x: torch.Tensor, a: torch.Tensor | None = None, b: torch.
     return outs[0], outs[1]
 
 
-def stream_join(x: torch.Tensor, a: torch.Tensor | None, b: torch.Tensor | None, y: torch.Tensor, out_dtype: torch.dtype) -> torch.Tensor:
+def stream_join(x: torch.Tensor, a: torch.Tensor | None, b: "torch.Tensor | RowParts | None", y: torch.Tensor, out_dtype: torch.dtype) -> torch.Tensor:
     """[x + a + b | y] row by row as `out_dtype` [tokens, 2 width]: the float32 stream x after its pending sum (a, b float32
-    or bfloat16, either may be None) beside float32 rows y of the same width. Nothing is written back."""
-    _gpu(x, a, b, y)
+    or bfloat16, either may be None, b possibly in parts) beside float32 rows y of the same width. Nothing is written back."""
+    parts = None
+    if isinstance(b, RowParts):
+        whole = b.factors is None and x.dim() == 2 and x.shape[1] % 4 == 0 and (a is None or a.dtype == torch.float32)
+        if whole and b.parts.shape[1:] == x.shape and b.parts.is_contiguous() and not any(t is not None and t.data_ptr() % 16 for t in (x, a, b.parts, y)):
+            b, parts = None, b.parts
+        else:
+            b = b.rows()
+    _gpu(x, a, b, y, parts)
     for name, t in (("x", x), ("y", y)):
         _need(t.dtype == torch.float32 and t.dim() == 2 and t.is_contiguous() and t.shape == x.shape, lambda: f"{name} must be contiguous float32 [tokens, width]")
     for name, t in (("a", a), ("b", b)):
         _need(t is None or (t.shape == x.shape and t.is_contiguous()), lambda: f"{name} must match the stream")
     out = torch.empty((x.shape[0], 2 * x.shape[1]), dtype=out_dtype, device=x.device)
+    if parts is not None:
+        _run("stream_join", library().ts_stream_join_parts(_ptr(out), _code(out_dtype), _ptr(x), _ptr(a), _ptr(parts), x.numel(), parts.shape[0], _ptr(y),
+                                                           x.shape[0], x.shape[1], _stream()))
+        return out
     _run("stream_join", library().ts_stream_join(_ptr(out), _code(out_dtype), _ptr(x), _ptr(a), 0 if a is None else _code(a.dtype), _ptr(b),
                                                  0 if b is None else _code(b.dtype), _ptr(y), x.shape[0], x.shape[1], _stream()))
     return out
@@ -3460,15 +3522,16 @@ def token_shift_keep(kept: torch.Tensor, h: torch.Tensor, ctx) -> None:
                                                            _ptr(ctx.state_slots), ctx.state_slots.shape[0], h.shape[1], _stream()))
 
 
-def stream_post_norm(x: torch.Tensor, a: torch.Tensor, post_weight: torch.Tensor, scale: torch.Tensor | None, post_eps: float,
+def stream_post_norm(x: torch.Tensor, a: "torch.Tensor | RowParts", post_weight: torch.Tensor, scale: torch.Tensor | None, post_eps: float,
                      weight: torch.Tensor | None = None, eps: float = 0.0, out_dtype: torch.dtype | None = None) -> torch.Tensor | None:
     """The float32 stream x [tokens, width] takes x += a / sqrt(mean(a^2) + post_eps) * post_weight * scale in place (a
-    float32, what a branch has made; `scale` float32 [width] or None). With `out_dtype`, the updated rows come back in
+    float32, what a branch has made, possibly in parts; `scale` float32 [width] or None). With `out_dtype`, the updated rows come back in
     that type: normalised and times `weight` (x / sqrt(mean(x^2) + eps) * weight), or as they are if `weight` is None."""
     if out_dtype in _DTYPE_CODE:
-        out = _native().stream_post_norm(x, a, post_weight, scale, post_eps, weight, eps, _DTYPE_CODE[out_dtype])
+        out = _native().stream_post_norm(x, a.operands() if isinstance(a, RowParts) else a, post_weight, scale, post_eps, weight, eps, _DTYPE_CODE[out_dtype])
         if out is not None:
             return out
+    a = added_up(a)
     _gpu(x, a, post_weight, scale, weight)
     _need(x.dtype == torch.float32 and x.dim() == 2 and x.is_contiguous() and a.dtype == torch.float32 and a.shape == x.shape and a.is_contiguous(),
           "the stream and the branch's rows must be contiguous float32 [tokens, width]")

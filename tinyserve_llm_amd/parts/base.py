@@ -178,6 +178,8 @@ class Mixer(Part):
     # True if forward() takes `then=` (a request of the norm that follows: Norm.request), hands it to
     # the `linear()` call that makes its result, and returns what that call returns
     finishes_into_norm = False
+    # True if forward() takes `parts=True` from a caller that takes its rows into a 32-bit stream, and may then return them in parts (`hip.RowParts`)
+    leaves_parts = False
     # True if forward() is 32-bit products of rows that follow from x alone, something between, and one product with the weight `o`, and the
     # mixer offers these apart, so that two mixers side by side share launches: `first_weights()` [(weight, its streaming copy or None)],
     # `first_rows(x, ctx, mem)` the rows each of them multiplies, `between(sums, x, ctx, mem)` the last product's rows, `o` and `o_packed`.
@@ -200,6 +202,7 @@ class Mixer(Part):
 class FeedForward(Part):
     takes_deferred_norm = False    # as for Mixer
     finishes_into_norm = False     # as for Mixer
+    leaves_parts = False           # as for Mixer
 
     def forward(self, x: torch.Tensor, ctx: StepContext) -> torch.Tensor:
         raise NotImplementedError

@@ -101,6 +101,11 @@ def pre_norm_block(layer: Layer, hidden, residual: torch.Tensor | None, ctx: Ste
     return x, residual
 
 
+def _into_stream(part, *args):
+    """What a part makes of `args`, for a 32-bit stream: possibly still in parts."""
+    return part.forward(*args, **({"parts": True} if getattr(part, "leaves_parts", False) else {}))
+
+
 def keeps_stream(fn):
     """Declares that an arrangement takes a `parts.stream.ResidualStream` as `hidden` (with `residual`
     None) and returns one: a model whose residual stream is 32-bit is made of such arrangements."""
@@ -146,8 +151,8 @@ def parallel_one_norm_block(layer: Layer, hidden, residual, ctx: StepContext, me
     if not isinstance(hidden, ResidualStream) or residual is not None:
         raise TypeError("this arrangement runs on a 32-bit residual stream (ModelSpec.residual_dtype = 'float32')")
     x, h = hidden.take(layer.norms["norm1"])
-    a = layer.mixer.forward(h, ctx, mem)
-    return ResidualStream(x, a, layer.feed_forward.forward(h, ctx)), None
+    a = _into_stream(layer.mixer, h, ctx, mem)
+    return ResidualStream(x, a, _into_stream(layer.feed_forward, h, ctx)), None
 
 
 @register("block", "sandwich")
@@ -163,13 +168,13 @@ def sandwich_block(layer: Layer, hidden, residual, ctx: StepContext, mem: LayerM
         raise TypeError("the sandwich arrangement runs on a 32-bit residual stream (ModelSpec.residual_dtype = 'float32')")
     norms = layer.norms
     x, h = hidden.take(norms["norm1"], out_dtype=norms["norm1"].weight.dtype)
-    stream = ResidualStream(x, layer.mixer.forward(h, ctx, mem), post=norms["norm1b"])
+    stream = ResidualStream(x, _into_stream(layer.mixer, h, ctx, mem), post=norms["norm1b"])
     if "norm2" not in norms:
         if layer.feed_forward.forward(None, ctx) is not None:
             raise KeyError("a sandwich layer with a feed-forward names the norms 'norm2' and 'norm2b'")
         return stream, None
     x, h = stream.take(norms["norm2"], out_dtype=norms["norm2"].weight.dtype)
-    return ResidualStream(x, layer.feed_forward.forward(h, ctx), post=norms["norm2b"]), None
+    return ResidualStream(x, _into_stream(layer.feed_forward, h, ctx), post=norms["norm2b"]), None
 
 
 @register("block", "pre_norm_stream")
@@ -184,13 +189,13 @@ def pre_norm_stream_block(layer: Layer, hidden, residual, ctx: StepContext, mem:
         raise TypeError("this arrangement runs on a 32-bit residual stream (ModelSpec.residual_dtype = 'float32')")
     norms = layer.norms
     x, h = hidden.take(norms["norm1"])
-    stream = ResidualStream(x, layer.mixer.forward(h, ctx, mem))
+    stream = ResidualStream(x, _into_stream(layer.mixer, h, ctx, mem))
     if "norm2" not in norms:
         if layer.feed_forward.forward(None, ctx) is not None:
             raise KeyError("a layer with a feed-forward names the norm 'norm2'")
         return stream, None
     x, h = stream.take(norms["norm2"])
-    return ResidualStream(x, layer.feed_forward.forward(h, ctx)), None
+    return ResidualStream(x, _into_stream(layer.feed_forward, h, ctx)), None
 
 
 @register("block", "post_norm_stream")
@@ -206,13 +211,13 @@ def post_norm_stream_block(layer: Layer, hidden, residual, ctx: StepContext, mem
         raise TypeError("this arrangement runs on a 32-bit residual stream (ModelSpec.residual_dtype = 'float32')")
     norms = layer.norms
     x, rows = hidden.rows_as(norms["norm1"].weight.dtype)
-    stream = ResidualStream(x, layer.mixer.forward(rows, ctx, mem), post=norms["norm1"])
+    stream = ResidualStream(x, _into_stream(layer.mixer, rows, ctx, mem), post=norms["norm1"])
     if "norm2" not in norms:
         if layer.feed_forward.forward(None, ctx) is not None:
             raise KeyError("a layer with a feed-forward names the norm 'norm2'")
         return stream, None
     x, rows = stream.rows_as(norms["norm2"].weight.dtype)
-    return ResidualStream(x, layer.feed_forward.forward(rows, ctx), post=norms["norm2"]), None
+    return ResidualStream(x, _into_stream(layer.feed_forward, rows, ctx), post=norms["norm2"]), None
 
 
 @register("block", "sandwich_scaled")
@@ -229,10 +234,10 @@ def sandwich_scaled_block(layer: Layer, hidden, residual, ctx: StepContext, mem:
         raise TypeError("this arrangement runs on a 32-bit residual stream (ModelSpec.residual_dtype = 'float32')")
     norms = layer.norms
     x, h = hidden.take(norms["norm1"])
-    stream = ResidualStream(x, layer.mixer.forward(h, ctx, mem), post=norms["norm1b"], scale=norms["scale1"].weight32)
+    stream = ResidualStream(x, _into_stream(layer.mixer, h, ctx, mem), post=norms["norm1b"], scale=norms["scale1"].weight32)
     if "norm2" in norms:
         x, h = stream.take(norms["norm2"])
-        stream = ResidualStream(x, layer.feed_forward.forward(h, ctx), post=norms["norm2b"], scale=norms["scale2"].weight32)
+        stream = ResidualStream(x, _into_stream(layer.feed_forward, h, ctx), post=norms["norm2b"], scale=norms["scale2"].weight32)
     elif layer.feed_forward.forward(None, ctx) is not None:
         raise KeyError("a layer with a feed-forward names the norms 'norm2', 'norm2b' and 'scale2'")
     for part in layer.token_inputs.values():

@@ -95,6 +95,7 @@ class CappedGLU(FeedForward):
     through the sigmoid; "gelu_tanh": through gelu in its tanh form."""
 
     graph_safe = True
+    leaves_parts = True
 
     def __init__(self, hidden_size: int, intermediate_size: int, limit: float = 0.0, slope: float = 1.702,
                  up_shift: float = 1.0, activation: str = "sigmoid") -> None:
@@ -116,7 +117,7 @@ class CappedGLU(FeedForward):
         self.gate_up_packed, self.down_packed = streaming_copy(self.gate_up), streaming_copy(self.down)
         return sum(c.nbytes() for c in (self.gate_up_packed, self.down_packed) if c is not None)
 
-    def forward(self, x: torch.Tensor, ctx: StepContext) -> torch.Tensor:
+    def forward(self, x: torch.Tensor, ctx: StepContext, parts: bool = False) -> "torch.Tensor | hip.RowParts":
         unit = few_rows_unit(x, self.gate_up, self.gate_up_packed, self.down, (self.activation, self.limit, self.slope, self.up_shift))
         if unit is None and (hip.many_rows_products() == "library" and x.is_cuda and hip.glu_takes(x, self.gate_up)
                              and hip.many_rows(x, self.gate_up, self.gate_up_packed)
@@ -126,7 +127,8 @@ class CappedGLU(FeedForward):
         if unit is None:
             sums = linear(x, self.gate_up, out_dtype=torch.float32, packed=self.gate_up_packed)
             unit = hip.capped_glu(sums, self.limit, self.slope, self.up_shift, x.dtype, activation=self.activation)
-        return linear(unit, self.down, out_dtype=torch.float32, packed=self.down_packed)
+        down = hip.linear_parts(unit, self.down, self.down_packed) if parts else None
+        return down if down is not None else linear(unit, self.down, out_dtype=torch.float32, packed=self.down_packed)
 
 
 @register("feed_forward", "none")

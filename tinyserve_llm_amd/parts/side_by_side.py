@@ -15,6 +15,8 @@ from tinyserve_llm_amd.parts.linear import packed_together, products
 
 @register("mixer", "side_by_side")
 class SideBySide(Mixer):
+    leaves_parts = True
+
     def __init__(self, left: PartSpec, right: PartSpec, left_scale: float = 1.0, right_scale: float = 1.0) -> None:
         self.left, self.right = make("mixer", left), make("mixer", right)
         self.left_scale, self.right_scale = float(left_scale), float(right_scale)
@@ -56,7 +58,7 @@ class SideBySide(Mixer):
         self.last_together, last = packed_together([(m.o, m.o_packed) for m in (self.left, self.right)])
         return held + first + last
 
-    def forward(self, x: torch.Tensor, ctx: StepContext, mem: LayerMemory) -> torch.Tensor:
+    def forward(self, x: torch.Tensor, ctx: StepContext, mem: LayerMemory, parts: bool = False) -> "torch.Tensor | hip.RowParts":
         if not self.in_threes:
             a = self.left.forward(x, ctx, mem)
             b = self.right.forward(x, ctx, mem)
@@ -66,4 +68,5 @@ class SideBySide(Mixer):
             at = len(pairs[0][1])
             lasts = [m.between(part, x, ctx, mem) for m, part in ((self.left, sums[:at]), (self.right, sums[at:]))]
             a, b = products([(rows, m.o, m.o_packed) for m, rows in zip((self.left, self.right), lasts)], self.last_together)
-        return hip.scaled_sum(a, self.left_scale, b, self.right_scale)
+        sides = hip.RowParts((a, b), (self.left_scale, self.right_scale))
+        return sides if parts else sides.rows()

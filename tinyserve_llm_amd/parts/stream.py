@@ -19,7 +19,8 @@ class ResidualStream:
     that goes to every token: a bias that the last projection of a branch left to the sum, or a vector that
     is added to the stream itself. With `post` (a norm; then only `a` is
     pending and `mult` is 1) the pending update is x += post(a), or x += post(a) * scale with `scale`
-    (float32 [hidden], a learned factor per channel; with an RMS norm as `post` only)."""
+    (float32 [hidden], a learned factor per channel; with an RMS norm as `post` only). `a`, or `b` beside it, may still be
+    in parts (`hip.RowParts`): the kernels of RMS norms add them up where they take the rows."""
 
     def __init__(self, x: torch.Tensor, a: torch.Tensor | None = None, b: torch.Tensor | None = None,
                  bias: torch.Tensor | None = None, mult: float = 1.0, post=None, scale: torch.Tensor | None = None) -> None:
@@ -29,6 +30,8 @@ class ResidualStream:
             raise ValueError("a norm after a branch goes with that branch's rows alone")
         if scale is not None and not hasattr(post, "weight32"):
             raise ValueError("a scale per channel rides on the kernel of an RMS norm after the branch")
+        if isinstance(a, hip.RowParts) and b is not None:
+            a, b = (a.rows() if isinstance(b, hip.RowParts) else b), (b if isinstance(b, hip.RowParts) else a)
         self.x, self.a, self.b, self.bias, self.mult, self.post, self.scale = x, a, b, bias, mult, post, scale
 
     def _apply_post(self, weight: torch.Tensor | None = None, eps: float = 0.0, out_dtype: torch.dtype | None = None):
@@ -42,7 +45,7 @@ class ResidualStream:
             out = hip.stream_post_norm(self.x, self.a, self.post.weight32, self.scale, self.post.eps, weight, eps, out_dtype)
             self.a = self.post = self.scale = None
             return out
-        self.a, self.post = self.post(self.a)[0], None
+        self.a, self.post = self.post(hip.added_up(self.a))[0], None
         return None
 
     def joined_with(self, other: torch.Tensor, dtype: torch.dtype) -> torch.Tensor:
@@ -51,7 +54,12 @@ class ResidualStream:
         self._apply_post()
         if self.bias is not None or self.mult != 1.0:
             self.settle()
-        return hip.stream_join(self.x, self.a, self.b, other, dtype)
+        a, b = self._branches()
+        return hip.stream_join(self.x, a, b, other, dtype)
+
+    def _branches(self):
+        """(a, b) as the stream's kernels take them: only b in parts."""
+        return (None, self.a) if isinstance(self.a, hip.RowParts) else (self.a, self.b)
 
     def rows_as(self, dtype: torch.dtype) -> "tuple[torch.Tensor, torch.Tensor]":
         """Does the pending sum and returns (x, x in `dtype`): the stream's rows as a projection's operand."""
@@ -67,6 +75,8 @@ class ResidualStream:
         if no norm is). Norms that work element by element (they have `elementwise()`: alpha, w, b of
         tanh(alpha x) w + b) ride in the kernel that sums; any other norm gets the settled stream."""
         fused = norm is None or hasattr(norm, "elementwise")
+        if fused and (self.post is None or hasattr(self.post, "elementwise")):
+            self.a, self.b = hip.added_up(self.a), hip.added_up(self.b)
         if fused and (self.post is None or hasattr(self.post, "elementwise")) and self.b is None and self.bias is None \
                 and self.mult == 1.0:
             post = self.post.elementwise() if self.post is not None else None
@@ -98,8 +108,8 @@ class ResidualStream:
         """Does the pending sum; returns (x, norm(x) * weights[0], norm(x) * weights[1]) with None for a
         weight not given, the norms in `out_dtype`."""
         self._apply_post()
-        a, b, bias = self.a, self.b, self.bias
-        if a is None and b is not None and bias is None:
+        (a, b), bias = self._branches(), self.bias
+        if a is None and isinstance(b, torch.Tensor) and bias is None:
             a, b = b, None
         h1, h2 = (None, None)
         if self.pending or weights[0] is not None or weights[1] is not None:

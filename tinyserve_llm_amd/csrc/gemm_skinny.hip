@@ -970,6 +970,61 @@ gemm_skinny8_kernel(const SkinnyArgs a) {
   }
 }
 
+// The same product of a matrix of very many rows (the head's vocabulary), by workgroups that stay: each takes every gridDim.x-th tile of 8 rows of W,
+// with the next tile's W on its way, past the caches, while this one's waves meet, and keeps its x. Sixteen thousand workgroups of 32 KB each came and
+// went at the rate the chip starts them, which follows its clock: 128,256 x 2,048 took 83 us in a decode step and 88 to 100 behind the products of a
+// prompt, whose power holds the clock down (timed apart 91.7 us, 79.1 here; 128,256 x 3,072 130.3 and 122.9). The sums are those of the kernel above, bit for bit. W as its packed copy, no norm behind.
+#define SK8_STAY_GRID 256       // one a compute unit, two tiles each under way (512 and more: 5 to 7 us slower)
+#define SK8_STAY_TILES 4096     // tiles from which they stay: with fewer a workgroup takes no more than two or three
+template <int STEPS, typename OUT>
+__global__ void __launch_bounds__(512)
+gemm_skinny8_stay_kernel(const SkinnyArgs a) {
+  __shared__ __align__(16) float smem[2][8 * 256];
+  const int nwaves = blockDim.x / TS_WAVE, tiles = a.N / 8;
+  const int wave = wave_index(), lane = threadIdx.x & (TS_WAVE - 1);
+  const int r = lane & 15, g = lane >> 4, row = r & 7, half = r >> 3;
+  const int kbeg = wave * (2 * STEPS * SK_KSTEP) + half * (STEPS * SK_KSTEP) + 8 * g;
+  const bf16_t* xrow = a.x_packed8 ? a.x + ((int64_t)wave * STEPS * 64 + lane) * 8 : a.x + (int64_t)(row < a.M ? row : 0) * a.ldx + kbeg;
+  const int xstep = a.x_packed8 ? 512 : SK_KSTEP;
+  const int64_t tile_size = (int64_t)nwaves * STEPS * 512;
+  const bf16_t* blk = a.w + (wave * STEPS * 64 + lane) * 8;
+  uint4 xb[STEPS], w0[STEPS], w1[STEPS];
+#pragma unroll
+  for (int s = 0; s < STEPS; ++s) xb[s] = *(const uint4*)(xrow + s * xstep);
+#pragma unroll
+  for (int s = 0; s < STEPS; ++s) w0[s] = load_once(blk + blockIdx.x * tile_size + s * 512);
+  const int m = lane >> 3, nl = lane & 7;
+  int turn = 0;
+  // one tile: the next one's loads (the last one's again, never read), this one's products, then a wave in turn adds the waves' sums
+  auto take = [&](int tile, uint4 (&now)[STEPS], uint4 (&next)[STEPS]) {
+    const int after = tile + (int)gridDim.x < tiles ? tile + (int)gridDim.x : tile;
+#pragma unroll
+    for (int s = 0; s < STEPS; ++s) next[s] = load_once(blk + after * tile_size + s * 512);
+    __builtin_amdgcn_sched_barrier(0);
+    float4_t acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < STEPS; ++s) acc = sk_mfma(now[s], xb[s], acc);
+    float* sums = smem[turn & 1];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) sums[wave * 256 + r * 16 + 4 * g + j] = acc[j];
+    __syncthreads();      // (one a tile: a half is written again two tiles on, behind the next meeting)
+    if (wave == turn % nwaves) {
+      float sum = 0.f;
+      for (int wv = 0; wv < nwaves; ++wv) sum += sums[wv * 256 + m * 16 + nl] + sums[wv * 256 + (m + 8) * 16 + nl + 8];
+      if (m < a.M) {
+        OUT* dst = (OUT*)a.y + (int64_t)m * a.ldy + 8 * tile + nl;
+        if constexpr (sizeof(OUT) == 4) *dst = sum;
+        else *dst = (bf16_t)sk_round(sum);
+      }
+    }
+    ++turn;
+  };
+  for (int tile = blockIdx.x; tile < tiles; tile += 2 * gridDim.x) {
+    take(tile, w0, w1);
+    if (tile + (int)gridDim.x < tiles) take(tile + gridDim.x, w1, w0);
+  }
+}
+
 template <typename OUT, bool NEXT = false>
 static int sk8_dispatch(const SkinnyArgs& a, hipStream_t stream) {
   // a wave covers 64 STEPS of k; 8 waves where the reduction allows it, never more than 16
@@ -988,6 +1043,13 @@ static int sk8_dispatch(const SkinnyArgs& a, hipStream_t stream) {
       return ts_check_launch();
     } else {
       return TS_BAD_SHAPE;
+    }
+  }
+  if constexpr (!NEXT) {
+    if (a.packed && !a.ssq_parts && a.N / 8 >= SK8_STAY_TILES && steps <= 8) {
+      if (steps == 4) gemm_skinny8_stay_kernel<4, OUT><<<SK8_STAY_GRID, block, 0, stream>>>(a);
+      else gemm_skinny8_stay_kernel<8, OUT><<<SK8_STAY_GRID, block, 0, stream>>>(a);
+      return ts_check_launch();
     }
   }
   if (steps == 4) gemm_skinny8_kernel<4, 512, OUT, NEXT><<<grid, block, smem, stream>>>(a);

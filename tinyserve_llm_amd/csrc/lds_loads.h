@@ -19,6 +19,11 @@ static __device__ __forceinline__ void load_to_lds(__amdgpu_buffer_rsrc_t rsrc, 
   __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_ptr_t)(uintptr_t)lds, 16, (int)voffset, (int)soffset, 0, 0);
 }
 
+// The same for what is read once: the caches do not put other lines out for it
+static __device__ __forceinline__ void load_to_lds_once(__amdgpu_buffer_rsrc_t rsrc, uint32_t lds, uint32_t voffset, uint32_t soffset) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_ptr_t)(uintptr_t)lds, 16, (int)voffset, (int)soffset, 0, 2);
+}
+
 // The same with an address of its own for every lane's 16 bytes (rows gathered from anywhere)
 static __device__ __forceinline__ void row_to_lds(const void* src, uint32_t lds) {
   __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src, (lds_ptr_t)(uintptr_t)lds, 16, 0, 0);

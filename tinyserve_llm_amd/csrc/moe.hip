@@ -535,6 +535,114 @@ moe_gemm_stream_kernel(TO* __restrict__ out, const bf16_t* __restrict__ x, const
   moe_store4(orow + c0, y, N - c0);
 }
 
+// The same sums, bit for bit, for reductions of whole lines (K a multiple of 256): a load of the kernel above takes 64 bytes of each of 16 rows, half a line,
+// and past the caches the other half is a line fetched again. Here 64 of k at a time go from memory straight into LDS, 8 rows of 128 bytes a load, pieces turned
+// by (row / 2) % 8 against bank conflicts; a wave has MOE_LINES of them there, its own, and waits for nobody. Without the gate a workgroup takes 32 columns.
+// Both products of 16 experts over 2,048, 2 x 1,024 and back over 1,024, past the caches, the kernel above and here: 4 tokens of four choices 36.6 and 20.8 us, 16
+// tokens 46.6 and 42.1, 48 tokens 55.2 and 45.5 (W at 4.4 TB/s), 64 tokens, some experts in two tiles, 91 and 61; through the caches 48 tokens 52.7 and 51.1.
+#define MOE_LINES 3
+template <bool GLU, typename TO, bool ONCE>
+__global__ void __launch_bounds__(MOE_THREADS)
+moe_gemm_lines_kernel(TO* __restrict__ out, const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, const int32_t* __restrict__ sorted,
+                      const int32_t* __restrict__ tiles, int src_div, int N, int K, float limit, float slope, float shift, int act) {
+  constexpr int WAVES = MOE_THREADS / TS_WAVE, R = MOE_LINES, STAGE = 3 * 2048;      // a stage: 16 rows of W twice, 16 rows of x, 64 of k
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[WAVES * R * STAGE];
+  __shared__ moe_f32x4 part_s[WAVES - 1][2][TS_WAVE];
+  const int tile = blockIdx.x;
+  const int rows = tiles[3 * tile + 2];
+  if (rows == 0) return;
+  const int e = tiles[3 * tile], first = tiles[3 * tile + 1];
+  const int wave = wave_index(), lane = threadIdx.x & (TS_WAVE - 1);
+  const int r = lane & 15, g = lane >> 4;
+  const int n0 = blockIdx.y * (GLU ? 16 : 32);
+  const int stages = K / 256, k0 = wave * (K / 4);
+  const bf16_t* we = w + ((int64_t)e * (GLU ? 2 : 1) * N + n0) * K + k0;
+  const __amdgpu_buffer_rsrc_t rsrc[2] = {load_base(we), load_base(GLU ? we + (int64_t)N * K : we)};
+  const uint32_t turned[2] = {(uint32_t)((lane % 8) ^ (lane / 16)) * 16, (uint32_t)((lane % 8) ^ (4 + lane / 16)) * 16};      // of rows lane / 8 and 8 + lane / 8
+  uint32_t woff[2][2];
+  int pair_at[2];
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    const int at = 8 * q + lane / 8;
+    pair_at[q] = sorted[first + min(at, rows - 1)];
+#pragma unroll
+    for (int t = 0; t < 2; ++t) woff[t][q] = (uint32_t)(min(GLU ? at : 16 * t + at, N - 1 - n0) * (int64_t)K * 2) + turned[q];
+  }
+  const uint32_t mine = (uint32_t)(uintptr_t)(lds_ptr_t)lds + wave * R * STAGE;
+  auto fetch_w = [&](int stage, uint32_t slot) {
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        if constexpr (ONCE) load_to_lds_once(rsrc[t], mine + slot + (2 * t + q) * 1024, woff[t][q], (uint32_t)stage * 128);
+        else load_to_lds(rsrc[t], mine + slot + (2 * t + q) * 1024, woff[t][q], (uint32_t)stage * 128);
+      }
+  };
+  const int ahead = min(R, stages);
+  for (int s = 0; s < ahead; ++s) fetch_w(s, s * STAGE);
+  __builtin_amdgcn_sched_barrier(0);
+  const bf16_t* xp[2];
+#pragma unroll
+  for (int q = 0; q < 2; ++q) xp[q] = x + (int64_t)(pair_at[q] / src_div) * K + k0 + turned[q] / 2;
+  auto fetch_x = [&](int stage, uint32_t slot) {
+#pragma unroll
+    for (int q = 0; q < 2; ++q) row_to_lds(xp[q] + stage * 64, mine + slot + (4 + q) * 1024);
+  };
+  for (int s = 0; s < ahead; ++s) fetch_x(s, s * STAGE);
+  const int pair = sorted[first + min(r, rows - 1)];
+  __builtin_amdgcn_sched_barrier(0);
+  moe_f32x4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+  const uint32_t rd = (uint32_t)(r * 128 + (g ^ (r >> 1)) * 16);
+  uint32_t slot = 0;
+  for (int s = 0; s < stages; ++s) {
+    // what has been asked for behind this stage: first the stages' rows of x behind their rows of W, and the pair's number, later whole stages
+    const int behind = s < R ? 2 * (ahead - 1 - s) + 1 + 6 * min(s, stages - ahead) : 6 * min(R - 1, stages - 1 - s);
+    if (behind >= 12) wait_for<12>();
+    else if (behind >= 8) wait_for<8>();
+    else if (behind >= 6) wait_for<6>();
+    else if (behind >= 4) wait_for<4>();
+    else if (behind >= 2) wait_for<2>();
+    else wait_for<0>();
+    __builtin_amdgcn_sched_barrier(0);
+    const unsigned char* from = lds + wave * R * STAGE + slot;
+    u32x4_t fw[2][2], fx[2];
+#pragma unroll
+    for (int d = 0; d < 2; ++d) {
+#pragma unroll
+      for (int t = 0; t < 2; ++t) fw[t][d] = *(const u32x4_t*)(from + t * 2048 + (rd ^ (64 * d)));
+      fx[d] = *(const u32x4_t*)(from + 4096 + (rd ^ (64 * d)));
+    }
+#pragma unroll
+    for (int d = 0; d < 2; ++d)
+#pragma unroll
+      for (int t = 0; t < 2; ++t) acc[t] = mfma32v(fw[t][d], fx[d], acc[t]);
+    __builtin_amdgcn_sched_barrier(0);      // (its operands have been read: the stage's place may be filled)
+    if (s + R < stages) fetch_w(s + R, slot), fetch_x(s + R, slot);
+    slot = slot == (R - 1) * STAGE ? 0 : slot + STAGE;
+  }
+  if (wave > 0) part_s[wave - 1][0][lane] = acc[0], part_s[wave - 1][1][lane] = acc[1];
+  __syncthreads();
+  if (wave > 0) return;
+#pragma unroll
+  for (int v = 0; v < WAVES - 1; ++v) acc[0] += part_s[v][0][lane], acc[1] += part_s[v][1][lane];
+  // lane (r, g): row r of the tile, columns n0 + 4 g .. + 3 (and 16 further on)
+  if (r >= rows) return;
+  TO* orow = out + (int64_t)pair * N;
+  float y[4];
+  if constexpr (GLU) {
+#pragma unroll
+    for (int c = 0; c < 4; ++c) y[c] = moe_unit(acc[0][c], acc[1][c], limit, slope, shift);
+    moe_store4(orow + n0 + 4 * g, y, N - n0 - 4 * g);
+  } else {
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+#pragma unroll
+      for (int c = 0; c < 4; ++c) y[c] = moe_act(acc[t][c], act);
+      moe_store4(orow + n0 + 16 * t + 4 * g, y, N - n0 - 16 * t - 4 * g);
+    }
+  }
+}
+
 // Steps of 64 of k in a stretch of the tiles of 128 rows (a whole number of stretches).
 static __device__ __forceinline__ int moe_stretch(int K) { return K >= 512 && K % 256 == 0 ? K / 256 : K / 64; }
 
@@ -753,6 +861,18 @@ extern "C" int ts_moe_gemm(void* out, int out_dtype, const void* x, int x_dtype,
     if (tile_rows == 16) {
       dim3 grid(max_tiles, (N + 15) / 16);
       if (grid.y > 65535) return TS_BAD_SHAPE;
+      if (K % 256 == 0 && K <= (1 << 22)) {                 // (byte offsets within 32 rows of W)
+        if (!glu) grid.y = (N + 31) / 32;
+#define MOE_BY_LINES(GLU, TO) \
+        (once ? moe_gemm_lines_kernel<GLU, TO, true> : moe_gemm_lines_kernel<GLU, TO, false>)<<<grid, MOE_THREADS, 0, stream>>>( \
+            (TO*)out, (const bf16_t*)x, (const bf16_t*)w, sorted, tiles, src_div, N, K, limit, slope, shift, act)
+        if (glu && out_dtype == 1) MOE_BY_LINES(true, bf16_t);
+        else if (!glu && out_dtype == 0) MOE_BY_LINES(false, float);
+        else if (!glu && out_dtype == 1) MOE_BY_LINES(false, bf16_t);
+        else return TS_BAD_DTYPE;
+#undef MOE_BY_LINES
+        return ts_check_launch();
+      }
 #define MOE_STREAM(GLU, TO) \
       (once ? moe_gemm_stream_kernel<GLU, TO, true> : moe_gemm_stream_kernel<GLU, TO, false>)<<<grid, MOE_THREADS, 0, stream>>>( \
           (TO*)out, (const bf16_t*)x, (const bf16_t*)w, sorted, tiles, src_div, N, K, limit, slope, shift, act)

@@ -1,0 +1,37 @@
+"""A step of one token a request through the decay states' own kernel: the bits of the kernel that walks requests of any length."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from tinyserve_llm_amd.ops import hip
+
+F32 = torch.float32
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("form,bonus", [("sigmoid_root", False), ("double_exponent", True), ("double_exponent", False)])
+@pytest.mark.parametrize("dim,vdim", [(64, 64), (64, 128), (64, 192), (64, 256), (128, 64), (128, 128), (128, 256), (128, 512), (128, 320)])
+@pytest.mark.parametrize("requests,heads", [(1, 1), (5, 3), (48, 2)])
+def test_one_token_a_request(requests, heads, dim, vdim, form, bonus):
+    g = torch.Generator(device="cuda").manual_seed(requests + dim + vdim)
+
+    def r(*shape):
+        return torch.randn(*shape, generator=g, device="cuda")
+    fused = r(requests, 2 * heads * dim + heads * vdim + 4)      # (rows that lie apart, as columns of one product)
+    q, k, v = fused[:, :heads * dim], fused[:, heads * dim:2 * heads * dim], fused[:, 2 * heads * dim:-4]
+    z, z_bias = r(requests, heads * dim) * 3, r(heads * dim)
+    if requests == 1:
+        z[0, :2] = torch.tensor([100.0, -100.0])
+    state = r(requests + 2, heads * dim * vdim + 8)
+    slots = torch.randperm(requests + 2, generator=g, device="cuda")[:requests].to(torch.int32)
+    cu = torch.arange(requests + 1, dtype=torch.int32, device="cuda")
+    made = []
+    for longest in (1, 2):      # (2: the walk)
+        kept = state.clone()
+        o = hip.decay_scan(q, k, v, z, z_bias, kept, cu, slots, heads, dim, vdim, form=form, tau=16.0, q_scale=dim ** -0.5,
+                           bonus=state[0, :heads * dim].clone().view(heads, dim) if bonus else None, longest=longest)
+        made.append((o, kept))
+    assert torch.equal(made[0][0], made[1][0]) and torch.equal(made[0][1], made[1][1])
+    assert not torch.equal(made[0][1], state)

@@ -14,6 +14,7 @@
 //     written back at the end. A column's sum runs over the rows in an order that the sizes alone fix. Heads of more
 //     than 256 dimensions, and sizes or places that are no whole 16-byte pieces, take a kernel that fetches element
 //     by element, with 4 columns a wave.
+//   * `ts_decay_step`: the same for steps of one token a request, decays included, bit for bit.
 //   * `ts_token_shift`: x_s[t] = h[t] + (h[t-1] - h[t]) mu_s for several mixes s at once, h[t-1] of a request's first
 //     token of the step being the row its state slot keeps (zeros for a new request); `ts_token_shift_keep` then
 //     leaves each request's last row of the step in its slot.
@@ -422,6 +423,142 @@ extern "C" int ts_decay_scan(float* out, const float* q, int64_t q_stride, const
   }
 #undef DS_LAUNCH
 #undef DS_ARGS
+  return ts_check_launch();
+}
+
+// A token a request (a decode step): what bounds it is the state's way in and out. A workgroup takes VC = 4 LPR columns of a head, a wave some of the shares
+// (four rows each, SHARES of them), a lane four columns side by side, so that a load takes whole lines of up to a kilobyte; the token's rows are asked for ahead of the
+// state, and its decays are made here while that is on its way. The shares' sums meet in the same tree as above, and the decays are those of the kernel below: the
+// same bits. 48 requests, 8 heads of 128 x 256 and 32 of 64 x 64, with the decays' kernel: 30.0 -> 20.6 us (4.9 TB/s) and
+// 19.4 -> 10.1; one request 15.1 -> 4.9 and 9.7 -> 3.3.
+template <int SHARES, int LPR, int WAVES, bool READ_FIRST>
+__global__ void __launch_bounds__(WAVES * TS_WAVE)
+decay_step_kernel(float* __restrict__ out, const float* __restrict__ q, int64_t q_stride, const float* __restrict__ k, int64_t k_stride,
+                  const float* __restrict__ v, int64_t v_stride, const float* __restrict__ z, int64_t z_stride, const float* __restrict__ z_bias,
+                  const float* __restrict__ bonus, float* __restrict__ state, int64_t state_stride, const int32_t* __restrict__ cu_seqlens,
+                  const int32_t* __restrict__ state_slots, int heads, int vdim, float q_scale, int form, float inv_tau) {
+  constexpr int DIM = 4 * SHARES, VC = 4 * LPR, GPW = TS_WAVE / LPR, PASSES = SHARES / (GPW * WAVES), THREADS = WAVES * TS_WAVE;
+  static_assert(SHARES == GPW * WAVES * PASSES, "whole passes of the waves over the shares");
+  __shared__ __attribute__((aligned(16))) float q_s[DIM], k_s[DIM], w_s[DIM], u_s[READ_FIRST ? DIM : 4];
+  __shared__ __attribute__((aligned(16))) float o_s[WAVES][VC];
+  const int seq = blockIdx.x, h = blockIdx.y, v0 = blockIdx.z * VC;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / TS_WAVE), lane = threadIdx.x & (TS_WAVE - 1);
+  const int t = cu_seqlens[seq];
+  if (cu_seqlens[seq + 1] != t + 1) return;
+  // the token's rows, a number a thread, ahead of the state
+  constexpr int PER = (DIM + THREADS - 1) / THREADS;
+  float qr[PER], kr[PER], zr[PER], br[PER], ur[PER];
+#pragma unroll
+  for (int i = 0; i < PER; ++i) {
+    const int d = min((int)threadIdx.x + i * THREADS, DIM - 1);
+    qr[i] = q[(int64_t)t * q_stride + h * DIM + d], kr[i] = k[(int64_t)t * k_stride + h * DIM + d], zr[i] = z[(int64_t)t * z_stride + h * DIM + d];
+    br[i] = z_bias[h * DIM + d];
+    if constexpr (READ_FIRST) ur[i] = bonus[h * DIM + d];
+  }
+  const int c = 4 * (lane % LPR), gi = lane / LPR;
+  const float4 vv = *(const float4*)(v + (int64_t)t * v_stride + (int64_t)h * vdim + v0 + c);
+  __builtin_amdgcn_sched_barrier(0);
+  float* st = state + (int64_t)state_slots[seq] * state_stride + (int64_t)h * DIM * vdim + v0 + c;
+  float4 S[PASSES][4];
+#pragma unroll
+  for (int p = 0; p < PASSES; ++p)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) S[p][j] = load_once<float4>(st + (int64_t)(4 * ((wave * PASSES + p) * GPW + gi) + j) * vdim);
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int i = 0; i < PER; ++i) {
+    const int d = threadIdx.x + i * THREADS;
+    if (d < DIM) {
+      q_s[d] = qr[i] * q_scale, k_s[d] = kr[i], w_s[d] = ds_decay(zr[i] + br[i], form, inv_tau);
+      if constexpr (READ_FIRST) u_s[d] = ur[i];
+    }
+  }
+  __syncthreads();
+  const float vc[4] = {vv.x, vv.y, vv.z, vv.w};
+  float o[PASSES][4];
+#pragma unroll
+  for (int p = 0; p < PASSES; ++p) {
+    const int d0 = 4 * ((wave * PASSES + p) * GPW + gi);
+    const float4 q4 = *(const float4*)(q_s + d0), k4 = *(const float4*)(k_s + d0), w4 = *(const float4*)(w_s + d0);
+    const float qq[4] = {q4.x, q4.y, q4.z, q4.w}, kk[4] = {k4.x, k4.y, k4.z, k4.w}, ww[4] = {w4.x, w4.y, w4.z, w4.w};
+    float uu[4] = {0.f, 0.f, 0.f, 0.f};
+    if constexpr (READ_FIRST) {
+      const float4 u4 = *(const float4*)(u_s + d0);
+      uu[0] = u4.x, uu[1] = u4.y, uu[2] = u4.z, uu[3] = u4.w;
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o[p][e] = 0.f;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      float s[4] = {S[p][j].x, S[p][j].y, S[p][j].z, S[p][j].w};
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float kv = kk[j] * vc[e];
+        if constexpr (READ_FIRST) {
+          o[p][e] = fmaf(fmaf(uu[j], kv, s[e]), qq[j], o[p][e]);
+          s[e] = fmaf(ww[j], s[e], kv);
+        } else {
+          s[e] = fmaf(ww[j], s[e], kv);
+          o[p][e] = fmaf(s[e], qq[j], o[p][e]);
+        }
+      }
+      store_once(st + (int64_t)(d0 + j) * vdim, make_float4(s[0], s[1], s[2], s[3]));
+    }
+  }
+  // the shares' sums, neighbours first: those of a pass side by side in the wave, the passes', the waves'
+#pragma unroll
+  for (int p = 0; p < PASSES; ++p)
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+      for (int off = LPR; off < TS_WAVE; off <<= 1) o[p][e] += __shfl_xor(o[p][e], off, TS_WAVE);
+#pragma unroll
+  for (int span = 1; span < PASSES; span <<= 1)
+#pragma unroll
+    for (int p = 0; p < PASSES; p += 2 * span)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o[p][e] += o[p + span][e];
+  if (gi == 0) *(float4*)&o_s[wave][c] = make_float4(o[0][0], o[0][1], o[0][2], o[0][3]);
+  __syncthreads();
+  if (threadIdx.x >= VC) return;
+  float sum[WAVES];
+#pragma unroll
+  for (int w = 0; w < WAVES; ++w) sum[w] = o_s[w][threadIdx.x];
+#pragma unroll
+  for (int span = 1; span < WAVES; span <<= 1)
+#pragma unroll
+    for (int w = 0; w < WAVES; w += 2 * span) sum[w] += sum[w + span];
+  out[((int64_t)t * heads + h) * vdim + v0 + threadIdx.x] = sum[0];
+}
+
+// A step of one token a request (requests that feed another number are left as they are): heads of 64 or 128 dimensions, values of whole 64s, everything in
+// whole 16-byte pieces; the decays from z and z_bias [heads dim] as ts_decay_factors makes them.
+extern "C" int ts_decay_step(float* out, const float* q, int64_t q_stride, const float* k, int64_t k_stride, const float* v, int64_t v_stride, const float* z,
+                             int64_t z_stride, const float* z_bias, const float* bonus, float* state, int64_t state_stride, const int32_t* cu_seqlens,
+                             const int32_t* state_slots, int num_seqs, int heads, int dim, int vdim, float q_scale, int form, float tau, hipStream_t stream) {
+  if (num_seqs <= 0) return TS_OK;
+  if (heads <= 0 || heads > 65535 || (dim != 64 && dim != 128) || vdim <= 0 || vdim % 64 || vdim / 64 > 65535 || state_stride < (int64_t)heads * dim * vdim ||
+      (form != 0 && form != 1) || !(tau > 0.f))
+    return TS_BAD_SHAPE;
+  if (((v_stride | state_stride) & 3) || (((uintptr_t)v | (uintptr_t)state) & 15)) return TS_BAD_SHAPE;
+#define DS_STEP(SHARES, LPR, WAVES) \
+  do { \
+    const dim3 grid(num_seqs, heads, vdim / (4 * LPR)); \
+    if (bonus) decay_step_kernel<SHARES, LPR, WAVES, true><<<grid, WAVES * TS_WAVE, 0, stream>>>(DS_STEP_ARGS); \
+    else decay_step_kernel<SHARES, LPR, WAVES, false><<<grid, WAVES * TS_WAVE, 0, stream>>>(DS_STEP_ARGS); \
+  } while (0)
+#define DS_STEP_ARGS out, q, q_stride, k, k_stride, v, v_stride, z, z_stride, z_bias, bonus, state, state_stride, cu_seqlens, state_slots, heads, vdim, q_scale, form, 1.0f / tau
+  if (dim == 128) {
+    if (vdim % 256 == 0) DS_STEP(32, 64, 8);
+    else if (vdim % 128 == 0) DS_STEP(32, 32, 4);
+    else DS_STEP(32, 16, 4);
+  } else {
+    if (vdim % 256 == 0) DS_STEP(16, 64, 4);
+    else if (vdim % 128 == 0) DS_STEP(16, 32, 4);
+    else DS_STEP(16, 16, 4);
+  }
+#undef DS_STEP
+#undef DS_STEP_ARGS
   return ts_check_launch();
 }
 

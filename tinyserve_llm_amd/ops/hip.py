@@ -159,6 +159,7 @@ def _declare(lib: ctypes.CDLL) -> None:
         "ts_stream_join_parts": [p, i, p, p, p, i64, i, p, i, i, p],
         "ts_gemm_slices_parts_bf16": [p, p, p, i, i, i, i64, i64, i, i, p],
         "ts_slices_sum": [p, p, i64, i, p],
+        "ts_decay_step": [p, p, i64, p, i64, p, i64, p, i64, p, p, p, i64, p, p, i, i, i, i, f, i, f, p],
         "ts_scaled_sum": [p, p, f, p, f, i64, p],
         "ts_gather_gate": [p, i, p, p, i, i64, i, p, i, i, i, p],
         "ts_qkv_prepare": [p, p, i, i, i, i, i, p, p, f, p, i, p],
@@ -3427,6 +3428,7 @@ DECAY_FULL_WORKGROUPS = 512      # workgroups of four waves from which a step ke
 # walk at every head size.
 DECAY_CHUNKS_FROM = 768
 DECAY_CHUNK_DIMS = (32, 64, 128)
+DECAY_STEP_DIMS = (64, 128)      # heads whose decode steps have a kernel of their own
 DECAY_WIDE_UP_TO = 4             # tokens of a step's longest portion up to which a wave owns 64 value columns instead of 16
 
 
@@ -3477,6 +3479,12 @@ def decay_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, z: torch.Tenso
             return out
         at_most = DECAY_CHUNKS_FROM - 1
         longest = max(n for n in (b - a for a, b in zip(ctx.host_cu_seqlens, ctx.host_cu_seqlens[1:])) if n <= at_most)
+    if (longest == 1 and T == S and dim in DECAY_STEP_DIMS and vdim % 64 == 0 and v.stride(0) % 4 == 0 and state.stride(0) % 4 == 0
+            and v.data_ptr() % 16 == 0 and state.data_ptr() % 16 == 0):
+        _run("decay_step", library().ts_decay_step(
+            _ptr(out), _ptr(q), q.stride(0), _ptr(k), k.stride(0), _ptr(v), v.stride(0), _ptr(z), z.stride(0), _ptr(z_bias), _ptr(bonus), _ptr(state),
+            state.stride(0), _ptr(cu_seqlens), _ptr(state_slots), S, heads, dim, vdim, float(q_scale), DECAY_FORMS[form], float(tau), _stream()))
+        return out
     w = torch.empty((T, heads * dim), dtype=torch.float32, device=q.device)
     _run("decay_factors", library().ts_decay_factors(_ptr(w), _ptr(z), z.stride(0), _ptr(z_bias), T, heads * dim, DECAY_FORMS[form], float(tau), _stream()))
     wide = longest is not None and longest <= DECAY_WIDE_UP_TO and vdim >= 64

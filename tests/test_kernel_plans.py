@@ -149,6 +149,18 @@ def test_gated_products_take_the_unit_along_where_that_is_faster():
     assert hip.glu_pays(256, 16384, 2048, 4) and hip.glu_pays(2048, 16384, 2048, 4) and hip.glu_pays(512, 8192, 2048, 4)
 
 
+def test_a_tile_just_passed_costs_the_library_a_whole_one():
+    """Products of 129 to 256 rows, both ways timed with the weights in memory: the gated ones (rows, n, k), and those into a norm by slices."""
+    along = [(129, 16384, 2048), (190, 16384, 2048), (129, 16384, 3072), (160, 16384, 4096), (129, 12288, 2048), (160, 24576, 2048), (129, 28672, 2048)]
+    apart = [(129, 2048, 2048), (160, 8192, 2048), (129, 10240, 2560), (160, 20480, 2560), (129, 22016, 4096), (160, 27648, 5120)]
+    assert [hip.glu_pays(*c) for c in along] == [True] * len(along) and [hip.glu_pays(*c) for c in apart] == [False] * len(apart)
+    assert not hip.glu_pays(129, 16384, 2048, 4), "32-bit branches are as they were"
+    for rows, n, k in ((129, 1024, 2048), (190, 2048, 2048), (129, 2048, 3072), (256, 2560, 2560), (160, 3072, 3072), (190, 3072, 2048)):
+        assert hip.slices_plan(rows, n, k, "norm") is not None and hip.slices_plan(rows, n, k, "norm")[1] > 2, (rows, n, k)
+    for rows, n, k, ending in ((225, 3072, 2048, "norm"), (190, 4096, 2048, "norm"), (256, 3072, 3072, "norm"), (190, 2048, 2048, "bf16"), (300, 2048, 2048, "norm")):
+        assert hip.slices_plan(rows, n, k, ending) is None, (rows, n, k)
+
+
 def test_units_of_few_rows_ride_along_where_that_is_faster():
     along = [(1, 1024, 512), (8, 2048, 1024), (1, 4096, 2048), (8, 16384, 2048), (16, 2048, 2048), (4, 8192, 3072), (8, 28672, 4096), (16, 28672, 4096), (1, 8192, 4096)]
     apart = [(1, 1024, 2560), (8, 1024, 3072), (4, 2048, 3072), (1, 1024, 4096), (16, 1024, 4096), (8, 4096, 4096), (4, 28672, 4096), (1, 16384, 4096)]

@@ -1702,14 +1702,16 @@ def glu_pays(rows: int, n: int, k: int, branch_bytes: int = 2) -> bool:
     they are, where the library cuts the reduction and has smaller tiles; what it saves is a launch and the branches' trip
     through memory. Both sides are estimated as they measured, in µs, with the weights coming from memory: here the plan's
     rounds; there 11 (10 for 32-bit branches, whose reading is counted apart) beside the longer of the weight's reading at
-    6.5 TB/s and the full tiles' products at 1 / 1.15 of the rate here, and the branches' trip at 3 TB/s. Over 589 points (1 to 2,048 rows, n
+    6.5 TB/s and the full tiles' products at 1 / 1.15 of the rate here (129 to 255 rows: those of 256, which its time hardly falls below: n 16,384, k 2,048
+    129 rows 30.8 apart and 23.8 here, 256 rows 34.8 and 26.2; k 3,072 36.9 and 33.9, 46.9 and 37.8; n 12,288, k 2,048 29.7 and 22.0, 32.2 and 24.1; n 10,240,
+    k 2,560 129 rows 25.7 and 26.0), and the branches' trip at 3 TB/s. Over 674 points (1 to 2,048 rows, n
     1,024 to 28,672, k 512 to 8,192) what this takes is at most 1.05 times the slower route's time where it errs; more often it errs by
-    leaving a gain, where a tile's height has just been passed (n 16,384, apart and here: k 2,048 129 to 161 rows 30 and 24, 257 to 316 36 and
-    33, 513 to 531 48 and 41, 1,025 to 1,175 88 and 79; k 3,072 129 to 212 39 and 35, 513 to 608 67 and 59, 1,025 to 1,298 123 and 114, but 257 to
+    leaving a gain, where a tile's height has just been passed (n 16,384, apart and here: k 2,048 257 to 316 rows 36 and
+    33, 513 to 531 48 and 41, 1,025 to 1,175 88 and 79; k 3,072 513 to 608 67 and 59, 1,025 to 1,298 123 and 114, but 257 to
     378 46 and 49). Apart and
-    here: F = n / 2 of 8,192, k 3,072: 17 rows 25 and 34, 160 rows 39 and 36, 320 rows 47 and 50, 2,048 rows 171 and 151; F 1,024, k 8,192: 16 rows 15
+    here: F = n / 2 of 8,192, k 3,072: 17 rows 25 and 34, 320 rows 47 and 50, 2,048 rows 171 and 151; F 1,024, k 8,192: 16 rows 15
     and 64, 1,024 rows 54 and 70, 2,048 rows 78 and 77; F 1,536, k 576: 1 row 8.9 and 7.6, 1,024 rows 15.8 and 9.2."""
-    full = 60 * rows * n / (256 * 256 * COMPUTE_UNITS) * k / 2048
+    full = 60 * (256 if 128 < rows < 256 and branch_bytes == 2 else rows) * n / (256 * 256 * COMPUTE_UNITS) * k / 2048
     apart = (11 if branch_bytes == 2 else 10) + max(2 * n * k / 6.5e6, 1.15 * full) + rows * n * (branch_bytes + 1) / 3e6
     return 1.5 + glu_plan(rows, n)[1] * k / 2048 < apart
 
@@ -1747,6 +1749,7 @@ SLICES_TILES = ((128, 128, (8.0, 0.42, 1.28, 0.16), (10.8, 0.45, 1.23, 0.15)),
 SLICES_LIBRARY = {"bf16": (4.7, 0.33, 1.24, 1.16, 0.55, 0.10), "f32": (3.9, 0.29, 1.46, 1.07, 0.63, 0.57), "norm": (7.7, 0.25, 1.20, 1.15, 0.61, 1.58)}
 # the share of the library's time, both as estimated, up to which the slices are taken: two of them in each tile, and more
 SLICES_TWO_SHARE, SLICES_SHARE = (0.95, 0.92, 0.91, 0.80, 0.80), 0.94
+SLICES_NORM_FEW_ROWS, SLICES_NORM_FEW_SHARE = 256, 1.02      # the same of more than two slices with the norm, up to so many rows
 SLICES_MIN_ROWS, SLICES_MAX_ROWS = 129, 2048       # fewer rows: the kernels that share x; more: whole reductions fill the chip
 SLICES_MIN_WIDTH, SLICES_MAX_WIDTH = 1024, 4096    # columns (wider: whole reductions fill the chip as well)
 SLICES_MAX, SLICES_MIN_STEPS = 16, 3               # slices, and steps of 64 in each
@@ -1762,9 +1765,12 @@ def slices_plan(rows: int, n: int, k: int, ending: str) -> tuple[int, int] | Non
     128 (513 rows, n 1,536, k 8,192 estimated 26.9, measured 35.0, the library 30.5), so these have to promise more. Over 4,536
     points (28 numbers of rows, 6 of n, 9 of k, the three endings) the rule takes 1,912, at 0.77 of the other way's time on average; 4 of them are
     slower by more than 2 %: 257 rows, n 3,072, k 8,192 31.5 and 34.8, 1,501 rows, n 4,096, k 4,096 with the norm 67.4 and 69.6, k 5,120 67.9 and 69.6.
+    With the norm and up to 256 rows the slices measure better than estimated, so more than two of them are taken up to 1.02 of the library's
+    estimate: 36 points measured 0.77 to 1.00 of its time (129 rows and 256, library and here: n 2,048, k 2,048 12.3 and 11.8, 13.4 and 13.4; k 3,072
+    19.1 and 14.8, 19.1 and 16.8; n 2,560, k 2,560 18.6 and 15.7, 20.6 and 18.9; n 3,072, k 3,072 129 and 190 rows 20.6 and 18.0, 22.5 and 19.3), and one call
+    on the host takes 6 less than the library's and the norm's.
     n 2,048, library and here: k 8,192 160 rows 26.6 and 19.2, 512 rows 34.1 and 29.9, 1,024 rows 53.4 and 44.7, with the norm 1,514
-    rows 66.5 and 61.9; k 4,096 with the norm 300 rows 25.2 and 20.4, 2,048 rows 50.0 and 49.9; k 2,048 160 rows 9.6 and 11.3, with the norm
-    12.8 and 13.4."""
+    rows 66.5 and 61.9; k 4,096 with the norm 300 rows 25.2 and 20.4, 2,048 rows 50.0 and 49.9; k 2,048 160 rows 9.6 and 11.3."""
     if not SLICES_MIN_ROWS <= rows <= SLICES_MAX_ROWS or not SLICES_MIN_WIDTH <= n <= SLICES_MAX_WIDTH or n % 8 or k % 64 or k < 2048:
         return None
     steps, best = k // 64, None
@@ -1780,7 +1786,8 @@ def slices_plan(rows: int, n: int, k: int, ending: str) -> tuple[int, int] | Non
     us, tile, slices = best
     fixed, chain, rooted, work, weight, out = SLICES_LIBRARY[ending]
     library = fixed + (chain + rooted * math.sqrt(rows) / 32) * k / 1024 + (work * rows * n * k * 1e-3 + weight * n * k + out * rows * n) * 1e-6
-    return (tile, slices) if us < (SLICES_TWO_SHARE[tile] if slices == 2 else SLICES_SHARE) * library else None
+    share = SLICES_TWO_SHARE[tile] if slices == 2 else SLICES_NORM_FEW_SHARE if ending == "norm" and rows <= SLICES_NORM_FEW_ROWS else SLICES_SHARE
+    return (tile, slices) if us < share * library else None
 
 
 def slices_takes(x: torch.Tensor, weight: torch.Tensor) -> bool:

@@ -194,3 +194,23 @@ def test_the_two_meanings_of_a_q_k_v_call_are_kept_apart(stub, monkeypatch):
         with pytest.raises(hip.KernelError):
             bad()
     assert called() == []
+
+
+def test_calls_of_few_rows_reach_the_kernels_that_stream_the_copies(stub):
+    """The forms of three calls that lead to another kernel: no slices, and the 8-row form's copy."""
+    module, answer, called = stub
+    rope = lambda slices, heads=4: (bf(3, 1024), bf(32, 32, 64, 8), slices, torch.zeros(9, 64), ints(0, 1, 2), ints(0, 1, 2), *caches(), heads, 2, 64, 1e-5, torch.zeros(3, 2))
+    into = lambda res=bf(3, 64), nw=bf(64): (bf(3, 1024), bf(4, 32, 64, 8), 0, res, nw)
+    few = lambda x=bf(8, 1024), p=bf(4, 4, 4, 64, 8), unit=0, squares=None: (x, p, True, unit, squares, 0.0, 0.0, 0.0, 0.0)
+    for call, plain, refused, launcher, shape in (
+            (module.qkv_rope_store_sliced, rope(0), [rope(-1), rope(0, 5)], "ts_gemm_skinny_rope_bf16", (3, 4, 64)),
+            (module.gemm_rows64_sliced, into(), [into(None, None), into(bf(3, 32)), into(nw=bf(32))], "ts_gemm_skinny_bf16", (3, 64)),
+            (module.gemm_rows64, few(), [few(bf(9, 1024)), few(bf(8, 1032)), few(unit=1), few(squares=torch.zeros(8, 1)), few(p=bf(4, 4, 4, 64, 8).float())],
+             "ts_gemm_skinny8_bf16", (8, 32))):
+        y = call(*plain)
+        y = y[0] if isinstance(y, tuple) else y
+        assert called()[-1] == launcher and tuple(y.shape) == shape
+        assert [call(*args) for args in refused] == [None] * len(refused) and called() == []
+        answer(launcher, BAD_SHAPE)
+        assert call(*plain) is None and called()[-1] == launcher
+        answer(launcher, OK)

@@ -402,6 +402,17 @@ PyObject* gemm_glu(Args a) {      // x, weight, tile, form's number, limit, slop
 
 bool squares_fit(const Tensor* s, int64_t rows) { return !s || (f32(*s) && s->dim() == 2 && s->size(0) == rows && s->size(1) >= 1 && s->is_contiguous()); }
 
+// What gemm_rows64 makes of up to 8 rows of x and the copy that the 8-row form reads (five-dimensional; its steps are those that the caller found for the reduction).
+PyObject* rows8(const Tensor& x, const Tensor& p, bool wide) {
+  const int64_t M = x.size(0), K = x.size(1), N = p.size(0) * 8;
+  if (M < 1 || M > 8 || !bf16(p) || p.size(1) * p.size(2) * 64 != K || p.size(3) != 64 || p.size(4) != 8 || !p.is_contiguous() || !fits(N) || !fits(K)) return none();
+  Tensor y = make(x, {M, N}, wide ? at::kFloat : at::kBFloat16);
+  if (TS_REFUSED("gemm_skinny8", ts_gemm_skinny8_bf16(ptr(&y), ptr(&x), ptr(&p), M, N, K, x.stride(0), K, N, wide ? 0 : 1, 1, nullptr, nullptr, nullptr, nullptr, nullptr,
+                                                      0, nullptr, nullptr, nullptr, 0, 0, 0, 0, stream())))
+    return none();
+  return wrap(y);
+}
+
 PyObject* gemm_rows64(Args a) {      // x, packed, 32-bit out, unit's number (0: none), squares, eps, limit, slope, up_shift, `few` of the launcher if it is there -> y
   const Tensor *x = a.tensor(), *p = a.tensor();
   const bool wide = a.i32();
@@ -409,6 +420,7 @@ PyObject* gemm_rows64(Args a) {      // x, packed, 32-bit out, unit's number (0:
   const Tensor* sq = a.maybe();
   const float eps = a.number(), limit = a.number(), slope = a.number(), shift = a.number();
   const int few = a.left ? a.i32() : 0, steps = few > 1 ? few : 0;
+  if (a.done() && p->dim() == 5) return unit || sq || few || x->dim() != 2 || !bf16(*x) || !pieces(*x) ? none() : rows8(*x, *p, wide);
   if (!a.done() || x->dim() != 2 || !bf16(*x) || !pieces(*x) || !packed16(*p, x->size(1)) || (unit && wide) || (unit > 1 && sq)) return none();
   const int64_t M = x->size(0), K = x->size(1), N = p->size(0) * 16;
   if (M < 1 || M > ROWS64_MAX_ROWS || N % (unit ? 128 : 64) || K % 1024 || !squares_fit(sq, M) || !fits(N) || !fits(K)) return none();
@@ -424,15 +436,28 @@ PyObject* gemm_rows64(Args a) {      // x, packed, 32-bit out, unit's number (0:
   return wrap(y);
 }
 
-PyObject* gemm_rows64_sliced(Args a) {      // x, packed, slices, residual, norm weight -> y, or with a weight (sum, operand, squares)
+PyObject* gemm_rows64_sliced(Args a) {      // x, packed, slices (0: whole, by the kernel that streams the copy; with a weight), residual, norm weight -> y, or with a weight (sum, operand, squares)
   const Tensor *x = a.tensor(), *p = a.tensor();
   const int slices = a.i32();
   const Tensor *res = a.maybe(), *nw = a.maybe();
   if (!a.done() || x->dim() != 2 || !bf16(*x) || !pieces(*x) || !packed16(*p, x->size(1)) || (res && !nw)) return none();
   const int64_t M = x->size(0), K = x->size(1), N = p->size(0) * 16;
-  if (M < 1 || M > ROWS64_MAX_ROWS || N % 64 || slices < 1 || slices > 64 || K % (ROWS64_SLICE_K * slices) || !fits(N) || !fits(K)) return none();
+  if (M < 1 || M > ROWS64_MAX_ROWS || !fits(N) || !fits(K) || (!slices && !nw)) return none();
+  if (slices && (N % 64 || slices < 1 || slices > 64 || K % (ROWS64_SLICE_K * slices))) return none();
   if (nw && !vector(*nw, at::kBFloat16, N)) return none();
   if (res && !(bf16(*res) && matrix(*res, M, N) && res->is_contiguous())) return none();
+  if (!slices) {
+    if (x->stride(0) < K || !aligned(*p)) return none();
+    const int64_t tiles = [&] {
+      Unlocked unlocked;
+      return ts_skinny_tiles(M, N, K);
+    }();
+    Tensor sum = make(*x, {M, N}, at::kBFloat16), operand = make(*x, {M, N}, at::kBFloat16), squares = make(*x, {M, tiles}, at::kFloat);
+    if (TS_REFUSED("gemm_skinny", ts_gemm_skinny_bf16(nullptr, ptr(x), ptr(p), nullptr, nullptr, nullptr, M, N, K, x->stride(0), K, N, 0.f, 0, 0, 1, 1, nullptr, 0,
+                                                      ptr(res), ptr(nw), ptr(&sum), ptr(&operand), ptr(&squares), 0, 0.f, 0.f, 0.f, stream())))
+      return none();
+    return Py_BuildValue("(NNN)", wrap(sum), wrap(operand), wrap(squares));
+  }
   Tensor parts = make(*x, {slices, M, N}, at::kFloat);
   if (!nw) {
     Tensor y = make(*x, {M, N}, at::kBFloat16);
@@ -510,11 +535,21 @@ PyObject* qkv_rope_store_sliced(Args a) {
   }
   if (!packed16(*p, K) || !aligned(*p)) return none();
   const int64_t N = p->size(0) * 16;
-  if (N != (nh + 2 * (int64_t)nkv) * hd || M < 1 || M > ROWS64_MAX_ROWS || N % 64 || slices < 1 || slices > 64 || K % (ROWS64_SLICE_K * slices)) return none();
+  if (N != (nh + 2 * (int64_t)nkv) * hd || M < 1 || M > ROWS64_MAX_ROWS) return none();
+  if (slices && (N % 64 || slices < 1 || slices > 64 || K % (ROWS64_SLICE_K * slices))) return none();
   if (!vector(*pos, at::kInt, M) || !squares_fit(sq, M) || !fits(N) || !fits(K)) return none();
   if (table && !(f32(*table) && table->dim() == 2 && table->size(1) == hd && table->is_contiguous())) return none();
   if (!s.take(M, at::kBFloat16, nkv, hd, hd)) return none();
-  Tensor parts = make(*x, {slices, M, N}, at::kFloat), q = make(*x, {M, nh, hd}, at::kBFloat16);
+  Tensor q = make(*x, {M, nh, hd}, at::kBFloat16);
+  if (!slices) {      // whole, by the kernel that streams the copy
+    if (TS_REFUSED("qkv_rope_store",
+                   ts_gemm_skinny_rope_bf16(ptr(&q), ptr(x), ptr(p), nullptr, nullptr, nullptr, M, K, x->stride(0), K, eps, sq ? 2 : 0, 1, typed<float>(table),
+                                            typed<int32_t>(pos), typed<int32_t>(s.slots), ptr(s.k), ptr(s.v), nh, nkv, hd, table != nullptr, s.page, s.ks[0],
+                                            s.ks[1], s.ks[2], s.vs[0], s.vs[1], s.vs[2], s.vs[3], ptr(sq), sq ? sq->size(1) : 0, stream())))
+      return none();
+    return wrap(q);
+  }
+  Tensor parts = make(*x, {slices, M, N}, at::kFloat);
   if (TS_REFUSED("qkv_rope_store_sliced",
                  ts_gemm_rows64_sliced_rope_bf16(ptr(&q), ptr(&parts), ptr(x), ptr(p), M, K, x->stride(0), slices, ptr(sq), sq ? sq->size(1) : 0, eps,
                                                  typed<float>(table), typed<int32_t>(pos), typed<int32_t>(s.slots), ptr(s.k), ptr(s.v), nh, nkv, hd, table !=

@@ -39,6 +39,19 @@ int ts_gemm_rows64_group_bf16(int products, void* const* y, const void* const* x
 int ts_gemm_rows64_sliced_bf16(void* y, void* parts, const void* x, const void* w16, int M, int N, int K, int64_t ldx, int slices,
                                const void* next_res, const void* next_nw, void* next_res_out, void* next_op, void* ssq_out, int64_t ld_op,
                                hipStream_t stream);
+int ts_gemm_skinny8_bf16(void* y, const void* x, const void* w, int M, int N, int K, int64_t ldx, int64_t ldw, int64_t ldy, int out_dtype, int packed,
+                         const void* next_res, const void* next_nw, void* next_res_out, void* next_op, void* ssq_out, int x_packed8, const float* comb_o,
+                         const float* comb_ml, const int32_t* comb_pos, int comb_splits, int comb_chunk, int comb_window, int comb_hd,
+                         hipStream_t stream);
+int ts_skinny_tiles(int M, int N, int K);
+int ts_gemm_skinny_bf16(void* y, const void* x, const void* w, const void* res, const void* nw, void* res_out, int M, int N, int K, int64_t ldx, int64_t ldw,
+                        int64_t ldy, float eps, int mode, int glu, int out_dtype, int packed, const void* ssq_in, int ssq_parts, const void* next_res,
+                        const void* next_nw, void* next_res_out, void* next_op, void* ssq_out, int y_pack8, float limit, float slope, float up_shift,
+                        hipStream_t stream);
+int ts_gemm_skinny_rope_bf16(void* q_out, const void* x, const void* w, const void* res, const void* nw, void* res_out, int M, int K, int64_t ldx,
+                             int64_t ldw, float eps, int mode, int packed, const float* cos_sin, const int32_t* positions, const int32_t* slots,
+                             void* k_cache, void* v_cache, int nh, int nkv, int hd, int rotate, int page_size, int64_t kp, int64_t ks, int64_t kh,
+                             int64_t vp, int64_t vs, int64_t vh, int64_t vd, const void* ssq_in, int ssq_parts, hipStream_t stream);
 int ts_gemm_rows64_sliced_rope_bf16(void* q_out, void* parts, const void* x, const void* w16, int M, int K, int64_t ldx, int slices,
                                     const void* ssq_in, int ssq_parts, float eps, const float* cos_sin, const int32_t* positions,
                                     const int32_t* slots, void* k_cache, void* v_cache, int nh, int nkv, int hd, int rotate, int page_size,

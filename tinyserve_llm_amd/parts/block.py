@@ -62,9 +62,9 @@ def first_norm_of(layer: Layer) -> Norm | None:
     return layer.norms[name] if name else None
 
 
-def _through(part, norm: Norm, x, residual, run, following: Norm | None):
-    """One branch of a pre-norm arrangement: `norm` applied to (x, residual), then `part` (`run` calls
-    its forward). `x` may be `norm` itself in deferred form (then `residual` is None). The norm is
+def _through(part, norm: Norm, x, residual, args: tuple, following: Norm | None):
+    """One branch of a pre-norm arrangement: `norm` applied to (x, residual), then `part` (`args`: what
+    its forward takes behind x). `x` may be `norm` itself in deferred form (then `residual` is None). The norm is
     handed to the part deferred if the part takes it so; the part is asked to finish into
     `following` if it can and that norm takes requests. Returns (the part's output or `following`
     deferred, the residual stream after `norm`'s sum)."""
@@ -78,7 +78,8 @@ def _through(part, norm: Norm, x, residual, run, following: Norm | None):
     # the stream after this norm's sum: known now, or once the part's first projection has run
     request = following.request(pending if pending is not None else residual) \
         if following is not None and part.finishes_into_norm else None
-    out = run(pending if pending is not None else x, request) if request is not None else run(pending if pending is not None else x)
+    operand = pending if pending is not None else x
+    out = part.forward(operand, *args) if request is None else part.forward(operand, *args, then=request)
     if pending is not None:
         residual = pending.residual_out
     return out, residual
@@ -90,12 +91,10 @@ def _through(part, norm: Norm, x, residual, run, following: Norm | None):
 def pre_norm_block(layer: Layer, hidden, residual: torch.Tensor | None, ctx: StepContext, mem: LayerMemory,
                    following: Norm | None = None) -> tuple[torch.Tensor, torch.Tensor | None]:
     mixer_norm, ff_norm = layer.norms["mixer_norm"], layer.norms["ff_norm"]
-    x, residual = _through(layer.mixer, mixer_norm, hidden, residual,
-                           lambda x, then=None: layer.mixer.forward(x, ctx, mem, **({"then": then} if then else {})), ff_norm)
+    x, residual = _through(layer.mixer, mixer_norm, hidden, residual, (ctx, mem), ff_norm)
     if ff_norm.made_for(x):
         residual = None                      # the sum is inside the deferred norm
-    x, residual = _through(layer.feed_forward, ff_norm, x, residual,
-                           lambda x, then=None: layer.feed_forward.forward(x, ctx, **({"then": then} if then else {})), following)
+    x, residual = _through(layer.feed_forward, ff_norm, x, residual, (ctx,), following)
     if following is not None and following.made_for(x):
         residual = None
     return x, residual

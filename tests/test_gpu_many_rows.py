@@ -337,6 +337,23 @@ def test_products_per_head_are_the_same_bits_whatever_the_tokens(tokens, x_type,
     assert torch.all((out[picked].double().cpu() - want).abs() <= bound + 1e-30)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("x_type, y_type", [(torch.float32, torch.float32), (torch.float32, BF), (BF, BF)])
+@pytest.mark.parametrize("heads, k, n", [(5, 72, 100), (32, 256, 64), (64, 64, 62), (130, 128, 192)])
+@pytest.mark.parametrize("tokens", [1, 16, 17, 33])
+def test_products_per_head_of_few_tokens_share_out_the_columns(tokens, x_type, y_type, heads, k, n):
+    """A block of 16 tokens a workgroup and 16 columns a wave (up to 384 workgroups, and any number of them up to 16 tokens), with a gate: the bits of
+    the same rows among 700, whose waves take all 64 columns; nothing beside them."""
+    g = torch.Generator().manual_seed(tokens + heads)
+    x = torch.randn(700, heads, k, generator=g).to(x_type).cuda()
+    w = (torch.randn(heads, n, k, generator=g) * k ** -0.5).to(BF).cuda().transpose(1, 2)
+    gate = torch.randn(700, heads * n, generator=g).cuda()
+    whole, few = (torch.full((m + 1, heads, n + 4), 7.0, dtype=y_type, device="cuda") for m in (700, tokens))
+    hip.heads_gemm(x, w, whole[:700, :, :n], gate)
+    hip.heads_gemm(x[:tokens], w, few[:tokens, :, :n], gate[:tokens])
+    assert torch.equal(few[:tokens], whole[:tokens]) and torch.all(few[tokens] == 7.0) and torch.all(few[:, :, n:] == 7.0)
+
+
 def test_the_blocks_of_tokens_a_wave_takes_are_blocks_that_have_tokens():
     """Sizes that were measured on both sides of the rule's lines (latent_mfma.hip): few tokens of many heads keep one block a wave."""
     blocks = hip.library().ts_heads_gemm_blocks

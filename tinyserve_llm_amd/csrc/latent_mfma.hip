@@ -578,25 +578,28 @@ extern "C" int ts_paged_attention_latent_tiles(void* out, int out_dtype, const f
 #define HM_TOKENS 64
 #define HM_COLS 64
 
-template <int RT, typename TX, typename TO>
+// BLOCKS 0: a workgroup takes one block of 16 tokens, and its waves 16 of the 64 columns each (with few tokens most waves had no token and the one
+// that had them read the matrix by itself; which is better by the rule of ts_heads_gemm_few).
+template <int BLOCKS, typename TX, typename TO>
 __global__ void __launch_bounds__(LM_THREADS)
 heads_gemm_mfma_kernel(TO* __restrict__ y, int64_t y_token, int64_t y_head, const TX* __restrict__ x, int64_t x_token,
                        int64_t x_head, const bf16_t* __restrict__ w, int64_t w_head, int64_t w_n, int num_tokens, int N, int K,
                        const float* __restrict__ gate, int64_t gate_token) {
+  constexpr int RT = BLOCKS ? BLOCKS : 1, NB = BLOCKS ? HM_COLS / 16 : 1;      // blocks of 16 tokens and of 16 columns of a wave
   const int wave = wave_index(), lane = threadIdx.x & (TS_WAVE - 1);
   const int r = lane & 15, g = lane >> 4;
-  const int h = blockIdx.y, n0 = blockIdx.z * HM_COLS;
-  const int t0 = RT * (blockIdx.x * HM_TOKENS + 16 * wave);
+  const int h = blockIdx.y, n0 = blockIdx.z * HM_COLS + (BLOCKS ? 0 : 16 * wave);
+  const int t0 = BLOCKS ? RT * (blockIdx.x * HM_TOKENS + 16 * wave) : 16 * blockIdx.x;
   const TX* xrow[RT];
 #pragma unroll
   for (int rt = 0; rt < RT; ++rt) xrow[rt] = x + (int64_t)min(t0 + 16 * rt + r, num_tokens - 1) * x_token + (int64_t)h * x_head;
   const bf16_t* wh = w + (int64_t)h * w_head;
-  float4_t acc[RT][HM_COLS / 16];
+  float4_t acc[RT][NB];
 #pragma unroll
   for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
-    for (int nb = 0; nb < HM_COLS / 16; ++nb) acc[rt][nb] = (float4_t){0.f, 0.f, 0.f, 0.f};
-#pragma unroll 4
+    for (int nb = 0; nb < NB; ++nb) acc[rt][nb] = (float4_t){0.f, 0.f, 0.f, 0.f};
+#pragma unroll(BLOCKS ? 4 : 8)
   for (int k0 = 0; k0 < K; k0 += 32) {
     const int k = k0 + 8 * g, kc = min(k, K - 8);
     uint4 b[RT];
@@ -611,7 +614,7 @@ heads_gemm_mfma_kernel(TO* __restrict__ y, int64_t y_token, int64_t y_head, cons
       if (k >= K) b[rt] = make_uint4(0, 0, 0, 0);
     }
 #pragma unroll
-    for (int nb = 0; nb < HM_COLS / 16; ++nb) {
+    for (int nb = 0; nb < NB; ++nb) {
       const int n = min(n0 + 16 * nb + r, N - 1);
       const uint4 a = *(const uint4*)(wh + (int64_t)n * w_n + kc);
 #pragma unroll
@@ -634,16 +637,16 @@ heads_gemm_mfma_kernel(TO* __restrict__ y, int64_t y_token, int64_t y_head, cons
       else *(uint2*)yrow = make_uint2(pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3]));
     };
     __shared__ __attribute__((aligned(16))) float4_t turn[LM_WAVES][16][HM_COLS / 4 + 1];
-    const bool turned = RT > 1 || (sizeof(TO) == 4 && num_tokens >= HM_TOKENS);
+    const bool turned = RT > 1 || (BLOCKS && sizeof(TO) == 4 && num_tokens >= HM_TOKENS);
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) {
       if (!turned) {
 #pragma unroll
-        for (int nb = 0; nb < HM_COLS / 16; ++nb) put(t0 + 16 * rt + r, n0 + 16 * nb + 4 * g, acc[rt][nb]);
+        for (int nb = 0; nb < NB; ++nb) put(t0 + 16 * rt + r, n0 + 16 * nb + 4 * g, acc[rt][nb]);
         continue;
       }
 #pragma unroll
-      for (int nb = 0; nb < HM_COLS / 16; ++nb) turn[wave][r][4 * nb + g] = acc[rt][nb];
+      for (int nb = 0; nb < NB; ++nb) turn[wave][r][4 * nb + g] = acc[rt][nb];
       __builtin_amdgcn_wave_barrier();
 #pragma unroll
       for (int i = 0; i < 4; ++i) put(t0 + 16 * rt + 4 * i + g, n0 + 4 * r, turn[wave][4 * i + g][r]);
@@ -657,7 +660,7 @@ heads_gemm_mfma_kernel(TO* __restrict__ y, int64_t y_token, int64_t y_head, cons
     if (t >= num_tokens) continue;
     TO* yrow = y + (int64_t)t * y_token + (int64_t)h * y_head;
 #pragma unroll
-  for (int nb = 0; nb < HM_COLS / 16; ++nb)
+  for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const int n = n0 + 16 * nb + 4 * g + j;
@@ -679,6 +682,15 @@ extern "C" int ts_heads_gemm_blocks(int num_tokens, int heads, int N, int K, int
   return groups >= 2048 || (groups >= 1024 && x_dtype == 1) ? 4 : 2;
 }
 
+// Whether a workgroup of one block of tokens a wave is better made one of 16 tokens whose waves share out the columns: where these are few workgroups,
+// or one to a head's 64 columns. us, before and so: 8 tokens, 32 heads, K 256 by 64, bfloat16 rows 5.9 and 3.3, K 64 by 256, 32-bit rows 3.3 and 2.5,
+// 128 heads of 512 by 128 12.1 and 6.8, 16 tokens of 128 by 512, 32-bit 11.7 and 8.2. From so many workgroups on each reads the matrix again for too few
+// tokens: K 64 by 256, 32 heads, 48 tokens (384 of them) 3.7 and 3.4, 64 tokens (512, left) 3.8 and 3.9; 16 heads of 128 by 512, 33 tokens (384)
+// 5.0 and 5.1, 65 tokens (640, left) 5.6 and 6.6; 128 heads of 128 by 512, 17 tokens (2,048, left) 11.8 and 14.0; K 256 by 64, 200 tokens (416, left) 7.5 and 5.9.
+static bool ts_heads_gemm_few(int num_tokens, int heads, int N) {
+  return num_tokens <= 16 || (int64_t)((num_tokens + 15) / 16) * heads * ((N + HM_COLS - 1) / HM_COLS) <= 384;
+}
+
 // w: bfloat16 [heads][N][K] with K along memory (stride w_n between rows, a multiple of 8; K a multiple of 8);
 // x rows 16-byte aligned.
 extern "C" int ts_heads_gemm_mfma(void* y, int y_dtype, int64_t y_token, int64_t y_head, const void* x, int x_dtype,
@@ -689,14 +701,17 @@ extern "C" int ts_heads_gemm_mfma(void* y, int y_dtype, int64_t y_token, int64_t
   if (heads <= 0 || heads > 65535 || N <= 0 || K < 8 || K % 8 || w_n % 8 || w_head % 8 || ((uintptr_t)w & 15) ||
       ((uintptr_t)x & 15) || (x_token * x_size) % 16 || (x_head * x_size) % 16 || (N + HM_COLS - 1) / HM_COLS > 65535)
     return TS_BAD_SHAPE;
-  const int blocks = ts_heads_gemm_blocks(num_tokens, heads, N, K, x_dtype);
-  const dim3 grid((num_tokens + blocks * HM_TOKENS - 1) / (blocks * HM_TOKENS), heads, (N + HM_COLS - 1) / HM_COLS);
+  int blocks = ts_heads_gemm_blocks(num_tokens, heads, N, K, x_dtype);
+  if (blocks == 1 && ts_heads_gemm_few(num_tokens, heads, N)) blocks = 0;
+  const int tokens = blocks ? blocks * HM_TOKENS : 16;
+  const dim3 grid((num_tokens + tokens - 1) / tokens, heads, (N + HM_COLS - 1) / HM_COLS);
 #define HM_GO(RT, TX, TO) \
   heads_gemm_mfma_kernel<RT, TX, TO><<<grid, LM_THREADS, 0, stream>>>((TO*)y, y_token, y_head, (const TX*)x, x_token, x_head, \
       (const bf16_t*)w, w_head, w_n, num_tokens, N, K, gate, gate_token)
 #define HM_LAUNCH(TX, TO) \
   do { \
-    if (blocks == 1) HM_GO(1, TX, TO); \
+    if (blocks == 0) HM_GO(0, TX, TO); \
+    else if (blocks == 1) HM_GO(1, TX, TO); \
     else if (blocks == 2) HM_GO(2, TX, TO); \
     else HM_GO(4, TX, TO); \
   } while (0)

@@ -35,3 +35,29 @@ def test_one_token_a_request(requests, heads, dim, vdim, form, bonus):
         made.append((o, kept))
     assert torch.equal(made[0][0], made[1][0]) and torch.equal(made[0][1], made[1][1])
     assert not torch.equal(made[0][1], state)
+
+
+@pytest.mark.parametrize("form,bonus", [("sigmoid_root", False), ("double_exponent", True)])
+@pytest.mark.parametrize("out_dtype", [torch.bfloat16, F32])
+@pytest.mark.parametrize("dim,vdim,shared,takes", [(64, 64, True, True), (64, 128, False, True), (64, 256, None, True), (128, 64, False, True), (128, 128, True, True),
+                                                   (128, 256, False, True), (128, 512, False, False), (128, 192, True, False)])
+@pytest.mark.parametrize("requests,heads", [(1, 1), (7, 3), (48, 2)])
+def test_one_token_a_request_with_the_heads_norm_and_gate(requests, heads, dim, vdim, shared, takes, out_dtype, form, bonus):
+    """The finishing kernel's bits of the sums that are left without it; weights of all heads, shared and none, rows of the gate that lie apart."""
+    g = torch.Generator(device="cuda").manual_seed(requests + dim + vdim)
+
+    def r(*shape):
+        return torch.randn(*shape, generator=g, device="cuda")
+    q, k, v, z, z_bias = r(requests, heads * dim), r(requests, heads * dim), r(requests, heads * vdim), r(requests, heads * dim) * 3, r(heads * dim)
+    gate = r(requests, heads * vdim + 8)[:, 4:-4] * 4
+    weight = None if shared is None else r(vdim if shared else heads * vdim)
+    state = r(requests + 2, heads * dim * vdim)
+    slots = torch.randperm(requests + 2, generator=g, device="cuda")[:requests].to(torch.int32)
+    cu = torch.arange(requests + 1, dtype=torch.int32, device="cuda")
+    kw = dict(form=form, tau=16.0, q_scale=dim ** -0.5, bonus=r(heads, dim) if bonus else None, longest=1)
+    kept, other = state.clone(), state.clone()
+    assert hip._decay_step_finishes(weight, gate, 1e-6, out_dtype, requests, heads, vdim) == takes
+    got = hip.decay_scan(q, k, v, z, z_bias, kept, cu, slots, heads, dim, vdim, finish=(weight, gate, 1e-6, out_dtype), **kw)
+    o = hip.decay_scan(q, k, v, z, z_bias, other, cu, slots, heads, dim, vdim, **kw)
+    want = hip.mlstm_finish(o, weight, gate, heads, vdim, 1e-6, out_dtype, silu_gate=True)
+    assert torch.equal(got, want) and torch.equal(kept, other)

@@ -430,13 +430,22 @@ extern "C" int ts_decay_scan(float* out, const float* q, int64_t q_stride, const
 // (four rows each, SHARES of them), a lane four columns side by side, so that a load takes whole lines of up to a kilobyte; the token's rows are asked for ahead of the
 // state, and its decays are made here while that is on its way. The shares' sums meet in the same tree as above, and the decays are those of the kernel below: the
 // same bits. 48 requests, 8 heads of 128 x 256 and 32 of 64 x 64, with the decays' kernel: 30.0 -> 20.6 us (4.9 TB/s) and
-// 19.4 -> 10.1; one request 15.1 -> 4.9 and 9.7 -> 3.3.
+// 19.4 -> 10.1; one request 15.1 -> 4.9 and 9.7 -> 3.3. A workgroup that has all of a head's columns may also finish them (DecayFinish): the norm's sum in
+// the tree of mlstm_finish_fours_kernel and its gate, asked for ahead of the state as well, in place of that kernel's launch (four of them in a step of 48
+// requests: 790 -> 784 us).
+struct DecayFinish {
+  void* out;                    // [tokens, heads vdim]; null: the sums go out as they are
+  const float *weight, *gate;   // as of ts_mlstm_finish
+  int64_t gate_stride;
+  float eps;
+  int weight_head, silu_gate, bf16;
+};
 template <int SHARES, int LPR, int WAVES, bool READ_FIRST>
 __global__ void __launch_bounds__(WAVES * TS_WAVE)
 decay_step_kernel(float* __restrict__ out, const float* __restrict__ q, int64_t q_stride, const float* __restrict__ k, int64_t k_stride,
                   const float* __restrict__ v, int64_t v_stride, const float* __restrict__ z, int64_t z_stride, const float* __restrict__ z_bias,
                   const float* __restrict__ bonus, float* __restrict__ state, int64_t state_stride, const int32_t* __restrict__ cu_seqlens,
-                  const int32_t* __restrict__ state_slots, int heads, int vdim, float q_scale, int form, float inv_tau) {
+                  const int32_t* __restrict__ state_slots, int heads, int vdim, float q_scale, int form, float inv_tau, const DecayFinish fin) {
   constexpr int DIM = 4 * SHARES, VC = 4 * LPR, GPW = TS_WAVE / LPR, PASSES = SHARES / (GPW * WAVES), THREADS = WAVES * TS_WAVE;
   static_assert(SHARES == GPW * WAVES * PASSES, "whole passes of the waves over the shares");
   __shared__ __attribute__((aligned(16))) float q_s[DIM], k_s[DIM], w_s[DIM], u_s[READ_FIRST ? DIM : 4];
@@ -457,6 +466,11 @@ decay_step_kernel(float* __restrict__ out, const float* __restrict__ q, int64_t 
   }
   const int c = 4 * (lane % LPR), gi = lane / LPR;
   const float4 vv = *(const float4*)(v + (int64_t)t * v_stride + (int64_t)h * vdim + v0 + c);
+  float4 gate = make_float4(0.f, 0.f, 0.f, 0.f), weight = make_float4(1.f, 1.f, 1.f, 1.f);
+  if (fin.out && wave == 0) {
+    gate = *(const float4*)(fin.gate + (int64_t)t * fin.gate_stride + (int64_t)h * vdim + c);
+    if (fin.weight) weight = *(const float4*)(fin.weight + (int64_t)h * fin.weight_head + c);
+  }
   __builtin_amdgcn_sched_barrier(0);
   float* st = state + (int64_t)state_slots[seq] * state_stride + (int64_t)h * DIM * vdim + v0 + c;
   float4 S[PASSES][4];
@@ -520,23 +534,53 @@ decay_step_kernel(float* __restrict__ out, const float* __restrict__ q, int64_t 
       for (int e = 0; e < 4; ++e) o[p][e] += o[p + span][e];
   if (gi == 0) *(float4*)&o_s[wave][c] = make_float4(o[0][0], o[0][1], o[0][2], o[0][3]);
   __syncthreads();
-  if (threadIdx.x >= VC) return;
+  const bool mine = threadIdx.x < VC;
   float sum[WAVES];
 #pragma unroll
-  for (int w = 0; w < WAVES; ++w) sum[w] = o_s[w][threadIdx.x];
+  for (int w = 0; w < WAVES; ++w) sum[w] = mine ? o_s[w][threadIdx.x] : 0.f;
 #pragma unroll
   for (int span = 1; span < WAVES; span <<= 1)
 #pragma unroll
     for (int w = 0; w < WAVES; w += 2 * span) sum[w] += sum[w + span];
-  out[((int64_t)t * heads + h) * vdim + v0 + threadIdx.x] = sum[0];
+  if (!fin.out) {
+    if (mine) out[((int64_t)t * heads + h) * vdim + v0 + threadIdx.x] = sum[0];
+    return;
+  }
+  // the head's norm and gate, four columns a lane of the first wave
+  if (mine) o_s[0][threadIdx.x] = sum[0];      // (no other thread reads the column before the barrier)
+  __syncthreads();
+  if (threadIdx.x >= LPR) return;
+  const float4 x = *(const float4*)&o_s[0][c];
+  float squares = fmaf(x.x, x.x, fmaf(x.y, x.y, fmaf(x.z, x.z, x.w * x.w)));
+#pragma unroll
+  for (int off = LPR / 2; off > 0; off >>= 1) squares += __shfl_xor(squares, off, TS_WAVE);
+  const float inv = 1.0f / sqrtf(squares / (float)vdim + fin.eps);
+  auto one = [&](float xv, float gv, float wv) {
+    const float s = 1.0f / (1.0f + expf(-gv));
+    return xv * inv * wv * (fin.silu_gate ? gv * s : s);
+  };
+  const float y[4] = {one(x.x, gate.x, weight.x), one(x.y, gate.y, weight.y), one(x.z, gate.z, weight.z), one(x.w, gate.w, weight.w)};
+  const int64_t at = ((int64_t)t * heads + h) * vdim + c;
+  if (fin.bf16)
+    *(uint2*)((bf16_t*)fin.out + at) = make_uint2((uint32_t)f2bf(y[0]) | ((uint32_t)f2bf(y[1]) << 16), (uint32_t)f2bf(y[2]) | ((uint32_t)f2bf(y[3]) << 16));
+  else
+    *(float4*)((float*)fin.out + at) = make_float4(y[0], y[1], y[2], y[3]);
 }
 
 // A step of one token a request (requests that feed another number are left as they are): heads of 64 or 128 dimensions, values of whole 64s, everything in
-// whole 16-byte pieces; the decays from z and z_bias [heads dim] as ts_decay_factors makes them.
+// whole 16-byte pieces; the decays from z and z_bias [heads dim] as ts_decay_factors makes them. With `finished` (heads of 64, 128 or 256 value columns)
+// what ts_mlstm_finish makes of the sums goes there, and no sums are left.
 extern "C" int ts_decay_step(float* out, const float* q, int64_t q_stride, const float* k, int64_t k_stride, const float* v, int64_t v_stride, const float* z,
                              int64_t z_stride, const float* z_bias, const float* bonus, float* state, int64_t state_stride, const int32_t* cu_seqlens,
-                             const int32_t* state_slots, int num_seqs, int heads, int dim, int vdim, float q_scale, int form, float tau, hipStream_t stream) {
+                             const int32_t* state_slots, int num_seqs, int heads, int dim, int vdim, float q_scale, int form, float tau, void* finished,
+                             int out_dtype, const float* weight, const float* gate, int64_t gate_stride, float eps, int weight_head, int silu_gate,
+                             hipStream_t stream) {
   if (num_seqs <= 0) return TS_OK;
+  if (finished && ((vdim != 64 && vdim != 128 && vdim != 256) || !gate || gate_stride % 4 || (weight_head != 0 && weight_head != vdim) ||
+                   (((uintptr_t)finished | (uintptr_t)gate | (uintptr_t)weight) & 15)))
+    return TS_BAD_SHAPE;
+  if (finished && out_dtype != 0 && out_dtype != 1) return TS_BAD_DTYPE;
+  const DecayFinish fin = {finished, weight, gate, gate_stride, eps, weight_head, silu_gate, out_dtype == 1};
   if (heads <= 0 || heads > 65535 || (dim != 64 && dim != 128) || vdim <= 0 || vdim % 64 || vdim / 64 > 65535 || state_stride < (int64_t)heads * dim * vdim ||
       (form != 0 && form != 1) || !(tau > 0.f))
     return TS_BAD_SHAPE;
@@ -547,7 +591,7 @@ extern "C" int ts_decay_step(float* out, const float* q, int64_t q_stride, const
     if (bonus) decay_step_kernel<SHARES, LPR, WAVES, true><<<grid, WAVES * TS_WAVE, 0, stream>>>(DS_STEP_ARGS); \
     else decay_step_kernel<SHARES, LPR, WAVES, false><<<grid, WAVES * TS_WAVE, 0, stream>>>(DS_STEP_ARGS); \
   } while (0)
-#define DS_STEP_ARGS out, q, q_stride, k, k_stride, v, v_stride, z, z_stride, z_bias, bonus, state, state_stride, cu_seqlens, state_slots, heads, vdim, q_scale, form, 1.0f / tau
+#define DS_STEP_ARGS out, q, q_stride, k, k_stride, v, v_stride, z, z_stride, z_bias, bonus, state, state_stride, cu_seqlens, state_slots, heads, vdim, q_scale, form, 1.0f / tau, fin
   if (dim == 128) {
     if (vdim % 256 == 0) DS_STEP(32, 64, 8);
     else if (vdim % 128 == 0) DS_STEP(32, 32, 4);

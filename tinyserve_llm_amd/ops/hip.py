@@ -159,7 +159,7 @@ def _declare(lib: ctypes.CDLL) -> None:
         "ts_stream_join_parts": [p, i, p, p, p, i64, i, p, i, i, p],
         "ts_gemm_slices_parts_bf16": [p, p, p, i, i, i, i64, i64, i, i, p],
         "ts_slices_sum": [p, p, i64, i, p],
-        "ts_decay_step": [p, p, i64, p, i64, p, i64, p, i64, p, p, p, i64, p, p, i, i, i, i, f, i, f, p],
+        "ts_decay_step": [p, p, i64, p, i64, p, i64, p, i64, p, p, p, i64, p, p, i, i, i, i, f, i, f, p, i, p, p, i64, f, i, i, p],
         "ts_scaled_sum": [p, p, f, p, f, i64, p],
         "ts_gather_gate": [p, i, p, p, i, i64, i, p, i, i, i, p],
         "ts_qkv_prepare": [p, p, i, i, i, i, i, p, p, f, p, i, p],
@@ -3462,7 +3462,8 @@ DECAY_WIDE_UP_TO = 4             # tokens of a step's longest portion up to whic
 
 def decay_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, z: torch.Tensor, z_bias: torch.Tensor, state: torch.Tensor,
                cu_seqlens: torch.Tensor, state_slots: torch.Tensor, heads: int, dim: int, vdim: int, *, form: str, tau: float = 1.0,
-               q_scale: float = 1.0, bonus: torch.Tensor | None = None, longest: int | None = None, ctx=None) -> torch.Tensor:
+               q_scale: float = 1.0, bonus: torch.Tensor | None = None, longest: int | None = None, ctx=None,
+               finish: "tuple[torch.Tensor | None, torch.Tensor, float, torch.dtype] | None" = None) -> torch.Tensor:
     """Linear attention with a decay per key channel over a packed step. q, k, z float32 [tokens, heads dim] and v
     float32 [tokens, heads vdim] are views whose rows may lie apart (columns of fused projections); z_bias float32
     [heads dim]. The decays are w = sigmoid(z + z_bias)^(1 / tau) (`form` "sigmoid_root") or exp(-exp(z + z_bias))
@@ -3473,7 +3474,10 @@ def decay_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, z: torch.Tenso
     fewer, wider slices of the value columns (the result is the same bit for bit). With `ctx` (the packed step's context, whose
     requests these are) requests that feed at least `DECAY_CHUNKS_FROM` tokens are worked in chunks on the matrix cores where
     the sizes allow it (`decay_chunks_take`): the same sums in another order, no further from 64 bits, so a request's rows then depend on how
-    its tokens are cut into steps."""
+    its tokens are cut into steps. With `finish` = (weight or None, gate, eps, out_dtype) what `mlstm_finish` (with a silu gate) makes of o comes back; a
+    step of one token a request makes it in the same kernel where a workgroup has whole heads."""
+    def finished(o: torch.Tensor) -> torch.Tensor:
+        return o if finish is None else mlstm_finish(o, finish[0], finish[1], heads, vdim, finish[2], finish[3], silu_gate=True)
     _gpu(q, k, v, z, z_bias, state, cu_seqlens, state_slots, bonus)
     T = q.shape[0]
     _need(form in DECAY_FORMS, lambda: f"form {form!r}: one of {sorted(DECAY_FORMS)}")
@@ -3504,15 +3508,19 @@ def decay_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, z: torch.Tenso
             state.stride(0), _ptr(chunks), _ptr(chunk_cu), _ptr(state_slots), _ptr(buf), _ptr(totals), _ptr(logs), C, S, heads, dim, vdim, float(q_scale),
             DECAY_FORMS[form], float(tau), _stream()))
         if _all_in_chunks(ctx, DECAY_CHUNKS_FROM):
-            return out
+            return finished(out)
         at_most = DECAY_CHUNKS_FROM - 1
         longest = max(n for n in (b - a for a, b in zip(ctx.host_cu_seqlens, ctx.host_cu_seqlens[1:])) if n <= at_most)
     if (longest == 1 and T == S and dim in DECAY_STEP_DIMS and vdim % 64 == 0 and v.stride(0) % 4 == 0 and state.stride(0) % 4 == 0
             and v.data_ptr() % 16 == 0 and state.data_ptr() % 16 == 0):
+        whole = finish is not None and _decay_step_finishes(*finish, T, heads, vdim)
+        weight, gate, eps, out_dtype = finish if whole else (None, None, 0.0, torch.float32)
+        gated = torch.empty((T, heads * vdim), dtype=out_dtype, device=q.device) if whole else None
         _run("decay_step", library().ts_decay_step(
             _ptr(out), _ptr(q), q.stride(0), _ptr(k), k.stride(0), _ptr(v), v.stride(0), _ptr(z), z.stride(0), _ptr(z_bias), _ptr(bonus), _ptr(state),
-            state.stride(0), _ptr(cu_seqlens), _ptr(state_slots), S, heads, dim, vdim, float(q_scale), DECAY_FORMS[form], float(tau), _stream()))
-        return out
+            state.stride(0), _ptr(cu_seqlens), _ptr(state_slots), S, heads, dim, vdim, float(q_scale), DECAY_FORMS[form], float(tau), _ptr(gated), _code(out_dtype),
+            _ptr(weight), _ptr(gate), _check_gate(gate, T, heads * vdim), float(eps), vdim if weight is not None and weight.shape[0] == heads * vdim else 0, 1, _stream()))
+        return gated if whole else finished(out)
     w = torch.empty((T, heads * dim), dtype=torch.float32, device=q.device)
     _run("decay_factors", library().ts_decay_factors(_ptr(w), _ptr(z), z.stride(0), _ptr(z_bias), T, heads * dim, DECAY_FORMS[form], float(tau), _stream()))
     wide = longest is not None and longest <= DECAY_WIDE_UP_TO and vdim >= 64
@@ -3524,7 +3532,15 @@ def decay_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, z: torch.Tenso
         _ptr(out), _ptr(q), q.stride(0), _ptr(k), k.stride(0), _ptr(v), v.stride(0), _ptr(w), w.stride(0), _ptr(bonus),
         _ptr(state), state.stride(0), _ptr(cu_seqlens), _ptr(state_slots), S, heads, dim, vdim, float(q_scale), int(bonus is not None),
         waves, int(wide), at_most, _stream()))
-    return out
+    return finished(out)
+
+
+def _decay_step_finishes(weight: torch.Tensor | None, gate: torch.Tensor, eps: float, out_dtype: torch.dtype, tokens: int, heads: int, vdim: int) -> bool:
+    """Whether the decay states' step kernel takes the heads' norm and gate along: a workgroup has all of a head's columns, everything in whole 16-byte pieces."""
+    return (vdim in (64, 128, 256) and out_dtype in _DTYPE_CODE and gate.is_cuda and gate.dtype == torch.float32 and gate.shape == (tokens, heads * vdim)
+            and gate.stride(1) == 1 and gate.stride(0) >= heads * vdim and gate.stride(0) % 4 == 0 and gate.data_ptr() % 16 == 0
+            and (weight is None or (weight.is_cuda and weight.dtype == torch.float32 and weight.shape in ((heads * vdim,), (vdim,)) and weight.is_contiguous()
+                                    and weight.data_ptr() % 16 == 0)))
 
 
 def decay_chunks_take(dim: int, vdim: int, state: torch.Tensor, bonus: torch.Tensor | None, rows: "tuple[torch.Tensor, ...]") -> bool:

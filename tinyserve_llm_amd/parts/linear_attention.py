@@ -67,11 +67,10 @@ class GatedLinearAttention(Mixer):
         H, K, V = self.num_heads, self.key_size, self.out_size
         proj = linear(x, self.proj, out_dtype=torch.float32, packed=self.proj_packed)
         z = linear(linear(x, self.decay_down), self.decay_up, out_dtype=torch.float32)
-        o = hip.decay_scan(proj[:, :K], proj[:, K:2 * K], proj[:, 2 * K:2 * K + V], z, self.decay_bias, mem.state, ctx.cu_seqlens,
-                           ctx.state_slots, H, self.head_dim, self.value_dim, form="sigmoid_root", tau=self.tau,
-                           q_scale=float(self.head_dim) ** -0.5, longest=ctx.max_query_len,
-                           ctx=ctx if x.dtype == torch.bfloat16 else None)
-        gated = hip.mlstm_finish(o, self.norm, proj[:, 2 * K + V:], H, self.value_dim, self.norm_eps, x.dtype, silu_gate=True)
+        gated = hip.decay_scan(proj[:, :K], proj[:, K:2 * K], proj[:, 2 * K:2 * K + V], z, self.decay_bias, mem.state, ctx.cu_seqlens,
+                               ctx.state_slots, H, self.head_dim, self.value_dim, form="sigmoid_root", tau=self.tau,
+                               q_scale=float(self.head_dim) ** -0.5, longest=ctx.max_query_len,
+                               ctx=ctx if x.dtype == torch.bfloat16 else None, finish=(self.norm, proj[:, 2 * K + V:], self.norm_eps, x.dtype))
         return linear(gated, self.o, out_dtype=torch.float32, packed=self.o_packed)
 
 
@@ -147,9 +146,9 @@ class ShiftedDecayRecurrence(Mixer):
         H, D = self.num_heads, self.head_dim
         r, k, v, g, low = sums
         z = linear(hip.bias_activation(low, None, "tanh", x.dtype), self.decay_up, out_dtype=torch.float32)
-        o = hip.decay_scan(r, k, v, z, self.decay_bias, mem.state, ctx.cu_seqlens, ctx.state_slots, H, D, D,
-                           form="double_exponent", bonus=self.bonus, longest=ctx.max_query_len, ctx=ctx if x.dtype == torch.bfloat16 else None)
-        return hip.mlstm_finish(o, self.norm, g, H, D, self.norm_eps, x.dtype, silu_gate=True)
+        return hip.decay_scan(r, k, v, z, self.decay_bias, mem.state, ctx.cu_seqlens, ctx.state_slots, H, D, D,
+                              form="double_exponent", bonus=self.bonus, longest=ctx.max_query_len, ctx=ctx if x.dtype == torch.bfloat16 else None,
+                              finish=(self.norm, g, self.norm_eps, x.dtype))
 
     def forward(self, x: torch.Tensor, ctx: StepContext, mem: LayerMemory) -> torch.Tensor:
         return in_three_steps(self, x, ctx, mem, self.together)

@@ -320,6 +320,26 @@ def test_token_shift_of_enough_pieces(n, width, mixes):
     test_token_shift_in_whole_pieces(torch.bfloat16, n, width, mixes)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("lengths,width", [([1], 70), ([1] * 48, 2048), ([1] * 299, 2056), ([1, 1, 3], 264), ([1, 0, 2], 72)])
+def test_token_shift_keeps_the_rows_of_a_decode_step(dtype, lengths, width):
+    """One launch for a step of one token a request (up to 614,400 numbers), two for others: the bits of the two calls, other slots as they were."""
+    from types import SimpleNamespace
+    h = hip()
+    n, requests = sum(lengths), len(lengths)
+    mu, state = torch.rand(5, width, device=DEV), torch.randn(requests + 2, width + 3, device=DEV)
+    x, _ = rounded(torch.randn(n, width), dtype)
+    ints = lambda t: torch.tensor(t, dtype=torch.int32, device=DEV)
+    cu = [sum(lengths[:i]) for i in range(requests + 1)]
+    ctx = SimpleNamespace(cu_seqlens=ints(cu), seq_of_token=ints([i for i, m in enumerate(lengths) for _ in range(m)]), num_seqs=requests,
+                          max_query_len=max(lengths), state_slots=torch.randperm(requests + 2, device=DEV)[:requests].int())
+    one, two = state.clone(), state.clone()
+    got = h.token_shift(x, mu, one[:, 3:], ctx, keep=True)
+    want = h.token_shift(x, mu, two[:, 3:], ctx)
+    h.token_shift_keep(two[:, 3:], x, ctx)
+    assert torch.equal(got, want) and torch.equal(one, two) and not torch.equal(one, state)
+
+
 @pytest.mark.parametrize("shared", [True, False])
 def test_heads_norm_weight_and_silu_gate(shared):
     h = hip()

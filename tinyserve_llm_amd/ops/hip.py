@@ -151,7 +151,7 @@ def _declare(lib: ctypes.CDLL) -> None:
         "ts_decay_scan": [p, p, i64, p, i64, p, i64, p, i64, p, p, i64, p, p, i, i, i, i, f, i, i, i, i, p],
         "ts_decay_chunks": [p, p, i64, p, i64, p, i64, p, i64, p, p, p, i64, p, p, p, p, p, p, i, i, i, i, i, f, i, f, p],
         "ts_decay_factors": [p, p, i64, p, i, i, i, f, p],
-        "ts_token_shift": [p, p, i, p, p, i64, p, p, p, i, i, i, p],
+        "ts_token_shift": [p, p, i, p, p, i64, p, p, p, i, i, i, i, p],
         "ts_token_shift_keep": [p, i64, p, i, p, p, i, i, p],
         "ts_stream_post_norm": [p, p, p, p, f, p, i, p, f, i, i, p],
         "ts_stream_post_norm_parts": [p, p, i64, i, i, f, f, p, p, f, p, i, p, f, i, i, p],
@@ -3549,19 +3549,25 @@ def decay_chunks_take(dim: int, vdim: int, state: torch.Tensor, bonus: torch.Ten
             and (bonus is None or bonus.data_ptr() % 16 == 0) and all(max(t.stride(0), t.shape[1]) <= 1 << 23 for t in rows))
 
 
-def token_shift(h: torch.Tensor, mu: torch.Tensor, kept: torch.Tensor, ctx) -> torch.Tensor:
+SHIFT_KEEP_MAX = 76800 * 8       # numbers of a step beyond which its shift goes by 16-byte pieces, which keep nothing
+
+
+def token_shift(h: torch.Tensor, mu: torch.Tensor, kept: torch.Tensor, ctx, keep: bool = False) -> torch.Tensor:
     """out[s, t] = h[t] + (h[t - 1] - h[t]) * mu[s] for every mix s (mu float32 [mixes, width]); for a request's first
     token of the step h[t - 1] is the row that `kept` (float32 [slots, width], a view whose rows may lie apart) holds
     at the request's state slot. Returns [mixes, tokens, width] of h's type. `token_shift_keep` leaves the step's last
-    rows in `kept` afterwards."""
+    rows in `kept` afterwards; with `keep` that is done here, by the same kernel where the step feeds one token a request."""
     _gpu(h, mu, kept)
     T, W = h.shape
     _need(h.dim() == 2 and h.is_contiguous(), "h must be contiguous [tokens, width]")
     _need(mu.dtype == torch.float32 and mu.dim() == 2 and mu.shape[1] == W and mu.is_contiguous(), "mu must be float32 [mixes, width]")
     _need(kept.dtype == torch.float32 and kept.dim() == 2 and kept.shape[1] == W and kept.stride(1) == 1, "the kept rows must be float32 [slots, width]")
     out = torch.empty((mu.shape[0], T, W), dtype=h.dtype, device=h.device)
+    alone = keep and ctx.max_query_len == 1 and T == ctx.num_seqs and T * W <= SHIFT_KEEP_MAX
     _run("token_shift", library().ts_token_shift(_ptr(out), _ptr(h), _code(h.dtype), _ptr(mu), _ptr(kept), kept.stride(0), _ptr(ctx.cu_seqlens),
-                                                 _ptr(ctx.seq_of_token), _ptr(ctx.state_slots), T, W, mu.shape[0], _stream()))
+                                                 _ptr(ctx.seq_of_token), _ptr(ctx.state_slots), T, W, mu.shape[0], int(alone), _stream()))
+    if keep and not alone:
+        token_shift_keep(kept, h, ctx)
     return out
 
 

@@ -138,9 +138,7 @@ class ShiftedDecayRecurrence(Mixer):
 
     def first_rows(self, x: torch.Tensor, ctx: StepContext, mem: LayerMemory) -> list[torch.Tensor]:
         kept = mem.state[:, self.size * self.head_dim:]
-        mixes = hip.token_shift(x, self.mu, kept, ctx)
-        hip.token_shift_keep(kept, x, ctx)
-        return list(mixes)
+        return list(hip.token_shift(x, self.mu, kept, ctx, keep=True))
 
     def between(self, sums: list[torch.Tensor], x: torch.Tensor, ctx: StepContext, mem: LayerMemory) -> torch.Tensor:
         H, D = self.num_heads, self.head_dim

@@ -63,3 +63,31 @@ def test_a_product_in_slices_leaves_its_parts(rows, n, k):
     if parts is not None:
         assert torch.equal(parts.rows(), hip.linear_bf16(x, w, F32))
     assert hip.linear_parts(x[:, ::2], w[:, : k // 2]) is None      # (rows that are not dense)
+
+
+@pytest.mark.parametrize("top,identity,shared", [(1, False, None), (2, True, "gated"), (4, True, "plain"), (4, False, "gated"), (5, True, None), (9, True, "plain")])
+@pytest.mark.parametrize("n,width", [(1, 64), (7, 1028), (48, 2048), (130, 2052), (3, 4096), (2, 4100)])
+def test_experts_rows_are_added_up_where_the_stream_takes_them(n, width, top, identity, shared):
+    g = torch.Generator(device="cuda").manual_seed(n + width + top)
+
+    def r(*shape):
+        return torch.randn(*shape, generator=g, device="cuda")
+    ids = torch.randint(0, 6, (n, top), generator=g, device="cuda", dtype=torch.int32)
+    pairs = r(n * top, width)
+    if identity:
+        pairs[ids.view(-1) >= 4] = float("nan")      # (an identity expert's pairs are in no tile)
+    x, post, scale, w = r(n, width), r(width), r(width), r(width)
+    for kind in (BF, F32):      # (a 32-bit input of identity experts is added up before)
+        left = hip.ExpertRows(pairs, r(n, top), r(n, width) if shared else None, (ids, 4, r(n, width).to(kind)) if identity else None, r(n, 1) if shared == "gated" else None)
+        for out_dtype, weight, sc in ((BF, w, scale), (F32, w, None), (BF, None, None), (None, None, scale)):
+            got, want = x.clone(), x.clone()
+            rows = hip.stream_post_norm(got, left, post, sc, 1e-5, weight, 1e-6, out_dtype)
+            rows_want = hip.stream_post_norm(want, left.rows(), post, sc, 1e-5, weight, 1e-6, out_dtype)
+            assert torch.equal(got, want) and (rows is None) == (rows_want is None) and (rows is None or torch.equal(rows, rows_want))
+    assert not torch.isnan(left.rows()).any()
+    norm = RMSNorm(width, 1e-5)
+    norm.bind({"weight": w.to(BF)})
+    for one, other in ((left, None), (None, left), (x, left)):
+        got, rows = ResidualStream(x.clone(), one, other).take(norm)
+        want, rows_want = ResidualStream(x.clone(), hip.added_up(one), hip.added_up(other)).take(norm)
+        assert torch.equal(got, want) and torch.equal(rows, rows_want)

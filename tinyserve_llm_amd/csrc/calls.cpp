@@ -215,10 +215,44 @@ Parts row_parts(Args& a, int64_t n, int64_t width) {
   return parts;
 }
 
-PyObject* stream_post_norm(Args a) {      // x, a (or in parts), post weight, scale, post eps, weight, eps, out code or -1 -> rows or None
+// A branch's rows as experts have left them: a tuple (rows, weights, shared, its gate, chosen experts, experts with matrices, input), as moe_combine of
+// ops/hip.py takes them.
+PyObject* post_norm_of_experts(const Tensor* x, Args& a) {
+  PyObject* tuple = a.next();
+  PyObject* items[7];
+  for (int i = 0; i < 7; ++i) items[i] = PyTuple_GET_ITEM(tuple, i);
+  Args in{items, 7};
+  const Tensor *rows = in.tensor(), *weights = in.tensor(), *shared = in.maybe(), *gate = in.maybe(), *ids = in.maybe();
+  const int real = in.i32();
+  const Tensor* input = in.maybe();
+  const Tensor *post = a.tensor(), *scale = a.maybe();
+  const float post_eps = a.number();
+  const Tensor* w = a.maybe();
+  const float eps = a.number();
+  const int out_code = a.i32();
+  if (!in.done() || !a.done() || out_code < 0 || out_code > 1 || !f32(*x) || !x->is_contiguous() || weights->dim() != 2) return none();
+  const int64_t n = x->size(0), width = x->size(1), top = weights->size(1);
+  if (!f32(*weights) || weights->size(0) != n || !weights->is_contiguous() || top < 1 || !fits(n * top) || !fits(width)) return none();
+  if (!f32(*rows) || !matrix(*rows, n * top, width) || !rows->is_contiguous()) return none();
+  if (shared && !(f32(*shared) && matrix(*shared, n, width) && shared->is_contiguous())) return none();
+  if (gate && !(shared && f32(*gate) && gate->numel() == n && gate->is_contiguous())) return none();
+  if (ids && !(input && is(*ids, at::kInt) && matrix(*ids, n, top) && ids->is_contiguous() && bf16(*input) && matrix(*input, n, width) && input->is_contiguous())) return none();
+  for (const Tensor* v : {post, scale, w})
+    if (v && !vector(*v, at::kFloat, width)) return none();
+  Tensor out = make(*x, {n, width}, out_code ? at::kBFloat16 : at::kFloat);
+  if (TS_REFUSED("stream_post_norm",
+                 ts_stream_post_norm_experts(typed<float>(x), typed<float>(rows), typed<float>(weights), typed<float>(shared), top, typed<int32_t>(ids), real, ptr(input),
+                                             typed<float>(gate), typed<float>(post), typed<float>(scale), post_eps, ptr(&out), out_code, typed<float>(w), eps, n, width,
+                                             stream())))
+    return none();
+  return wrap(out);
+}
+
+PyObject* stream_post_norm(Args a) {      // x, a (or in parts, or as experts left it), post weight, scale, post eps, weight, eps, out code or -1 -> rows or None
   const Tensor* x = a.tensor();
   if (in_parts(a)) {
     if (a.bad || x->dim() != 2) return none();
+    if (PyTuple_GET_SIZE(*a.at) == 7) return post_norm_of_experts(x, a);
     const int64_t n = x->size(0), width = x->size(1);
     const Parts b = row_parts(a, n, width);
     const Tensor *post = a.tensor(), *scale = a.maybe();

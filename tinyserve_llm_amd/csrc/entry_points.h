@@ -83,6 +83,9 @@ int ts_stream_post_norm(float* x, const float* a, const float* post_w, const flo
                         const float* w, float eps, int num_rows, int width, hipStream_t stream);
 int ts_stream_post_norm_parts(float* x, const float* p, int64_t stride, int count, int scaled, float fa, float fb, const float* post_w, const float* scale,
                               float post_eps, void* h, int h_dtype, const float* w, float eps, int num_rows, int width, hipStream_t stream);
+int ts_stream_post_norm_experts(float* x, const float* rows, const float* weights, const float* shared, int top, const int32_t* ids, int real, const void* input,
+                                const float* gate, const float* post_w, const float* scale, float post_eps, void* h, int h_dtype, const float* w, float eps,
+                                int num_rows, int width, hipStream_t stream);
 int ts_stream_update_norm_parts(float* x, const float* a, const float* p, int64_t stride, int count, int scaled, float fa, float fb, float mult, void* h,
                                 int h_dtype, const void* w, int w_dtype, float eps, int num_rows, int width, hipStream_t stream);
 int ts_stream_update_norm(float* x, const void* a, int a_dtype, const void* b, int b_dtype, const void* bias, int bias_dtype, float mult,

@@ -2490,8 +2490,24 @@ class RowParts:
         return (self.parts,) if self.factors is None else (self.parts[0], self.factors[0], self.parts[1], self.factors[1])
 
 
-def added_up(rows: "torch.Tensor | RowParts | None") -> torch.Tensor | None:
-    return rows.rows() if isinstance(rows, RowParts) else rows
+class ExpertRows:
+    """float32 rows [tokens, width] as experts have left them, still to be added up: the operands of `moe_combine`. `stream_post_norm` takes them as they
+    are; `rows()` adds them up by a kernel of its own."""
+
+    def __init__(self, rows: torch.Tensor, weights: torch.Tensor, shared: torch.Tensor | None = None,
+                 identity: "tuple[torch.Tensor, int, torch.Tensor] | None" = None, shared_gate: torch.Tensor | None = None) -> None:
+        self.pairs, self.weights, self.shared, self.identity, self.shared_gate = rows, weights, shared, identity, shared_gate
+
+    def rows(self) -> torch.Tensor:
+        return moe_combine(self.pairs, self.weights, self.shared, identity=self.identity, shared_gate=self.shared_gate)
+
+    def operands(self) -> tuple:
+        """As the library's own module takes them."""
+        return (self.pairs, self.weights, self.shared, self.shared_gate, *(self.identity or (None, 0, None)))
+
+
+def added_up(rows: "torch.Tensor | RowParts | ExpertRows | None") -> torch.Tensor | None:
+    return rows.rows() if isinstance(rows, (RowParts, ExpertRows)) else rows
 
 
 def stream_update_norm(x: torch.Tensor, a: torch.Tensor | None = None, b: "torch.Tensor | RowParts | None" = None,
@@ -3580,13 +3596,13 @@ def token_shift_keep(kept: torch.Tensor, h: torch.Tensor, ctx) -> None:
                                                            _ptr(ctx.state_slots), ctx.state_slots.shape[0], h.shape[1], _stream()))
 
 
-def stream_post_norm(x: torch.Tensor, a: "torch.Tensor | RowParts", post_weight: torch.Tensor, scale: torch.Tensor | None, post_eps: float,
+def stream_post_norm(x: torch.Tensor, a: "torch.Tensor | RowParts | ExpertRows", post_weight: torch.Tensor, scale: torch.Tensor | None, post_eps: float,
                      weight: torch.Tensor | None = None, eps: float = 0.0, out_dtype: torch.dtype | None = None) -> torch.Tensor | None:
     """The float32 stream x [tokens, width] takes x += a / sqrt(mean(a^2) + post_eps) * post_weight * scale in place (a
-    float32, what a branch has made, possibly in parts; `scale` float32 [width] or None). With `out_dtype`, the updated rows come back in
+    float32, what a branch has made, possibly in parts or as experts have left it; `scale` float32 [width] or None). With `out_dtype`, the updated rows come back in
     that type: normalised and times `weight` (x / sqrt(mean(x^2) + eps) * weight), or as they are if `weight` is None."""
     if out_dtype in _DTYPE_CODE:
-        out = _native().stream_post_norm(x, a.operands() if isinstance(a, RowParts) else a, post_weight, scale, post_eps, weight, eps, _DTYPE_CODE[out_dtype])
+        out = _native().stream_post_norm(x, a.operands() if isinstance(a, (RowParts, ExpertRows)) else a, post_weight, scale, post_eps, weight, eps, _DTYPE_CODE[out_dtype])
         if out is not None:
             return out
     a = added_up(a)

@@ -29,6 +29,7 @@ class RoutedExperts(FeedForward):
     chosen."""
 
     graph_safe = True
+    leaves_parts = True
 
     def __init__(self, hidden_size: int, num_experts: int, top: int, intermediate_size: int, limit: float = 0.0,
                  slope: float = 1.702, up_shift: float = 1.0, router_scale: float = 1.0, normalize: bool = True,
@@ -80,7 +81,7 @@ class RoutedExperts(FeedForward):
     def keep_streaming_copies(self) -> int:
         return self.shared.keep_streaming_copies() if self.shared is not None else 0
 
-    def forward(self, x: torch.Tensor, ctx: StepContext) -> torch.Tensor:
+    def forward(self, x: torch.Tensor, ctx: StepContext, parts: bool = False) -> "torch.Tensor | hip.ExpertRows":
         routed = hip.moe_route(x, self.router, self.correction, self.top, self.router_scale, self.normalize,
                                softmax_all=self.scoring == "softmax_all", extras=int(self.shared_gate), groups=self.groups)
         experts, weights = routed[0], routed[1]
@@ -89,8 +90,8 @@ class RoutedExperts(FeedForward):
         unit = hip.moe_gemm(x, self.gate_up, grouped, x.dtype, per_token=True, glu=(self.limit, self.slope, self.up_shift))
         rows = hip.moe_gemm(unit, self.down, grouped, torch.float32, per_token=False)
         shared = self.shared.forward(x, ctx) if self.shared is not None else None
-        return hip.moe_combine(rows, weights, shared, identity=(experts, self.num_experts, x) if self.identity else None,
-                               shared_gate=routed[2] if self.shared_gate else None)
+        left = hip.ExpertRows(rows, weights, shared, (experts, self.num_experts, x) if self.identity else None, routed[2] if self.shared_gate else None)
+        return left if parts else left.rows()
 
 
 @register("feed_forward", "routed_dense_experts")

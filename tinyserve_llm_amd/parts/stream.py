@@ -20,7 +20,8 @@ class ResidualStream:
     is added to the stream itself. With `post` (a norm; then only `a` is
     pending and `mult` is 1) the pending update is x += post(a), or x += post(a) * scale with `scale`
     (float32 [hidden], a learned factor per channel; with an RMS norm as `post` only). `a`, or `b` beside it, may still be
-    in parts (`hip.RowParts`): the kernels of RMS norms add them up where they take the rows."""
+    in parts (`hip.RowParts`): the kernels of RMS norms add them up where they take the rows. Rows as experts have left them
+    (`hip.ExpertRows`) stay so where an RMS norm is `post`."""
 
     def __init__(self, x: torch.Tensor, a: torch.Tensor | None = None, b: torch.Tensor | None = None,
                  bias: torch.Tensor | None = None, mult: float = 1.0, post=None, scale: torch.Tensor | None = None) -> None:
@@ -30,6 +31,10 @@ class ResidualStream:
             raise ValueError("a norm after a branch goes with that branch's rows alone")
         if scale is not None and not hasattr(post, "weight32"):
             raise ValueError("a scale per channel rides on the kernel of an RMS norm after the branch")
+        if isinstance(a, hip.ExpertRows) and not hasattr(post, "weight32"):
+            a = a.rows()
+        if isinstance(b, hip.ExpertRows):
+            b = b.rows()
         if isinstance(a, hip.RowParts) and b is not None:
             a, b = (a.rows() if isinstance(b, hip.RowParts) else b), (b if isinstance(b, hip.RowParts) else a)
         self.x, self.a, self.b, self.bias, self.mult, self.post, self.scale = x, a, b, bias, mult, post, scale

@@ -91,6 +91,22 @@ def test_a_projection_has_the_bits_of_the_product_and_the_rotation(tile, heads, 
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("heads, kv, dim", [(38, 5, 64), (14, 5, 128), (48, 9, 64)])
+@pytest.mark.parametrize("rows", [1921, 2048, 2200])
+def test_the_second_tile_is_narrow_or_wide_with_the_same_bits(rows, heads, kv, dim):
+    """3,072 columns in 256 workgroups of 192 columns (1,921 and 2,048 rows) and in wide ones (2,200 rows); 4,224 columns in wide ones."""
+    n, k, page = (heads + 2 * kv) * dim, 256, 32
+    assert (-(-rows // 128) * -(-n // 192) <= hip.COMPUTE_UNITS) == (n == 3072 and rows < 2200)
+    x, w = operands(rows, n, k)
+    pages = -(-(rows + 700) // page)
+    table, pos, slots = torch.randn(rows, dim, device="cuda"), torch.arange(rows, dtype=I32, device="cuda"), places(rows, "beside", pages * page)
+    got_kv, want_kv = caches(pages, page, kv, dim, True), caches(pages, page, kv, dim, True)
+    q = hip.qkv_rope_store_whole(x, w, 1, table, pos, slots, *got_kv, heads, kv, dim)
+    want = hip.rope_store(hip.gemm_whole([x], [w], 0)[0], table, pos, slots, *want_kv, heads, kv, dim)
+    assert torch.equal(q, want) and torch.equal(got_kv[0], want_kv[0]) and torch.equal(got_kv[1], want_kv[1])
+
+
+@pytest.mark.gpu
 def test_the_module_and_the_general_function_give_the_same_and_refuse_the_same(monkeypatch):
     x, w = operands(300, 4 * 64, 256)
     table, pos, slots = torch.randn(400, 64, device="cuda"), torch.arange(300, dtype=I32, device="cuda"), torch.arange(300, dtype=I32, device="cuda")

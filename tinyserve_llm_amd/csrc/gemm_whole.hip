@@ -4,7 +4,7 @@
 //
 // What bounds it: from some 800 rows on the matrix cores, at the 1.6 to 1.9 GHz that their power leaves them; at fewer rows the chain of a tile's steps, of
 // which each waits for LDS (0.3 µs a step of 64 x 128, whose products take 0.11). Measured with W coming from memory: q|k|v of 32 heads of 64 beside 8 + 8,
-// K 2,048, 192 rows 13.8 µs, 513 rows 14.2, 1,024 rows 22.8, 2,048 rows 32.4; the library's product and `rope_store` took 20.9, 20.9, 26.6
+// K 2,048, 192 rows 13.8 µs, 513 rows 14.2, 1,024 rows 22.8, 2,048 rows 30.0; the library's product and `rope_store` took 20.9, 20.9, 26.6
 // and 37.0. The rotation's kernel read and wrote what the product had just written, and was a launch of its own.
 #include "tile_product.h"
 
@@ -13,6 +13,7 @@
 // small results, which it splits (600 x 64 over 2,048: 1.3e-7, one chain 2.7e-7). A tile of so many chains begins as many times, and the launch begins with
 // these: 3,072, 2,048 four times, 64 and 32 columns over 2,048, the last two in chains, 320 rows 26.6 µs, with the two by the library 41.2, all in one chain each 25.3.
 #define GW_CHAINS 4
+#define GW_COMPUTE_UNITS 256
 
 struct WholeProduct {
   const bf16_t *x, *w;
@@ -154,21 +155,22 @@ struct WholeRopeArgs {
   int64_t kp, ks, kh, vp, vs, vh, vd;
 };
 
-// A wave's 64 columns of the tile are 32 dimensions of a head's first half and the 32 that turn with them, hd / 2 further on (W's rows are
+// A wave's columns of the tile are units of 16 HT dimensions of a head's first half and those that turn with them, hd / 2 further on (W's rows are
 // fetched in that order), so that a pair meets in a lane; with values, whose pages are transposed, the lanes exchange through LDS, which
 // is free by then. The product is rounded as it would be stored, turned and stored as `rope_store` does it.
-template <int BM, int BN, int WM, int WN, int XN>
+template <int BM, int BN, int WM, int WN, int XN, int HT>
 __global__ __launch_bounds__(WM * WN * TS_WAVE, 2) void gemm_whole_rope_kernel(const WholeRopeArgs a) {
   using Tile = TileProduct<BM, BN, WM, WN, XN>;
   constexpr int PASSES = (Tile::TM + 3) / 4, TP = Tile::TM / PASSES, TOKENS = TP * 16;      // a wave's values go at most 64 tokens at a time
   constexpr int SPAN = TOKENS + 8;                              // numbers between two dimensions of the values in LDS
-  static_assert(Tile::TN == 4 && Tile::TM % PASSES == 0, "a wave has 64 columns, and passes of as many tokens each");
-  static_assert(WM * WN * 64 * SPAN * 2 <= Tile::LDS, "the values' way through LDS");
+  constexpr int UNIT = 32 * HT, UNITS = Tile::TN / (2 * HT);    // columns of a unit, and units of a wave
+  static_assert(Tile::TN % (2 * HT) == 0 && Tile::TM % PASSES == 0, "a wave has whole units, and passes of as many tokens each");
+  static_assert(WM * WN * UNIT * SPAN * 2 <= Tile::LDS, "the values' way through LDS");
   __shared__ __attribute__((aligned(1024))) unsigned char lds[Tile::LDS];
   const int item = blockIdx.x % 8 * a.per_die + blockIdx.x / 8;
   if (item >= a.items) return;
-  const int m0 = item % a.row_tiles * BM, u0 = item / a.row_tiles * (BN / 64);      // first row, and first unit of 64 columns
-  const int units = a.N / 64, per_head = a.hd / 64, half = a.hd / 2;
+  const int m0 = item % a.row_tiles * BM, u0 = item / a.row_tiles * (BN / UNIT);      // first row, and first unit
+  const int units = a.N / UNIT, per_head = a.hd / UNIT, half = a.hd / 2;
   uint32_t xoff[Tile::NX], woff[Tile::NW];
 #pragma unroll
   for (int q = 0; q < Tile::NX; ++q) {
@@ -177,12 +179,11 @@ __global__ __launch_bounds__(WM * WN * TS_WAVE, 2) void gemm_whole_rope_kernel(c
   }
 #pragma unroll
   for (int q = 0; q < Tile::NW; ++q) {
-    const int at = Tile::w_row(q), u = min(u0 + at / 64, units - 1), in = at % 64;
-    const int row = u / per_head * a.hd + u % per_head * 32 + in % 32 + (in >= 32 ? half : 0);
+    const int at = Tile::w_row(q), u = min(u0 + at / UNIT, units - 1), in = at % UNIT;
+    const int row = u / per_head * a.hd + u % per_head * (UNIT / 2) + in % (UNIT / 2) + (in >= UNIT / 2 ? half : 0);
     woff[q] = (uint32_t)(row * a.ldw * 2) + Tile::piece(at);
   }
   const int lane = threadIdx.x % TS_WAVE, r = lane % 16, g = lane / 16, wave = wave_index(), wm = wave % WM, wn = wave / WM;
-  const int u = u0 + wn, head = u / per_head, d0 = u % per_head * 32;      // this wave's head, and the first of its dimensions in the first half
   const int first = m0 + wm * Tile::TM * 16;
   int position[Tile::TM], slot[Tile::TM];
 #pragma unroll
@@ -194,124 +195,136 @@ __global__ __launch_bounds__(WM * WN * TS_WAVE, 2) void gemm_whole_rope_kernel(c
   float4_t acc[Tile::TN][Tile::TM];
   Tile::run(lds, load_base(a.x + (int64_t)m0 * a.ldx), load_base(a.w), xoff, woff, a.steps, acc);
   const int values = (a.nh + a.nkv) * per_head;      // the first unit of the values
-  if (a.k_cache && u0 + BN / 64 > values) __syncthreads();      // every wave has read its last operands: LDS is free
-  if (u >= units || (head >= a.nh && !a.k_cache)) return;
+  if (a.k_cache && u0 + BN / UNIT > values) __syncthreads();      // every wave has read its last operands: LDS is free
   auto page_of = [&](int s) { return a.page_shift >= 0 ? s >> a.page_shift : s / a.page_size; };
-  if (u < values) {
+  bf16_t* turn = (bf16_t*)lds + wave * (UNIT * SPAN);
 #pragma unroll
-    for (int i = 0; i < Tile::TM; ++i) {
-      const int m = first + 16 * i + r;
-      uint32_t p[2][2][2];      // [half][tile of the half][pair]
+  for (int w = 0; w < UNITS; ++w) {
+    const int u = u0 + wn * UNITS + w, head = u / per_head, d0 = u % per_head * (UNIT / 2);      // the unit's head, and the first of its dimensions in the first half
+    if (u >= units || (head >= a.nh && !a.k_cache)) return;
+    if (u < values) {
 #pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        float y[2][4];
+      for (int i = 0; i < Tile::TM; ++i) {
+        const int m = first + 16 * i + r;
+        uint32_t p[2][HT][2];      // [half][tile of the half][pair]
 #pragma unroll
-        for (int h = 0; h < 2; ++h)
+        for (int j = 0; j < HT; ++j) {
+          float y[2][4];
 #pragma unroll
-          for (int e = 0; e < 2; ++e) {
-            const uint32_t both = pack_bf16(acc[2 * h + j][i][2 * e], acc[2 * h + j][i][2 * e + 1]);      // as the product would be stored
-            y[h][2 * e] = __uint_as_float(both << 16), y[h][2 * e + 1] = __uint_as_float(both & 0xffff0000u);
+          for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+              const float4_t& at = acc[(2 * w + h) * HT + j][i];
+              const uint32_t both = pack_bf16(at[2 * e], at[2 * e + 1]);      // as the product would be stored
+              y[h][2 * e] = __uint_as_float(both << 16), y[h][2 * e + 1] = __uint_as_float(both & 0xffff0000u);
+            }
+          if (a.cos_sin) {
+            const float* at = a.cos_sin + (int64_t)position[i] * a.hd + d0 + 16 * j + 4 * g;
+            const float4 c = *(const float4*)at, s = *(const float4*)(at + half);
+            const float cs[4] = {c.x, c.y, c.z, c.w}, sn[4] = {s.x, s.y, s.z, s.w};
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              const float y1 = fmaf(y[0][e], cs[e], -(y[1][e] * sn[e])), y2 = fmaf(y[1][e], cs[e], y[0][e] * sn[e]);      // (as rope_store's are compiled)
+              y[0][e] = y1, y[1][e] = y2;
+            }
           }
-        if (a.cos_sin) {
-          const float* at = a.cos_sin + (int64_t)position[i] * a.hd + d0 + 16 * j + 4 * g;
-          const float4 c = *(const float4*)at, s = *(const float4*)(at + half);
-          const float cs[4] = {c.x, c.y, c.z, c.w}, sn[4] = {s.x, s.y, s.z, s.w};
 #pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const float y1 = fmaf(y[0][e], cs[e], -(y[1][e] * sn[e])), y2 = fmaf(y[1][e], cs[e], y[0][e] * sn[e]);      // (as rope_store's are compiled)
-            y[0][e] = y1, y[1][e] = y2;
+          for (int h = 0; h < 2; ++h) p[h][j][0] = pack_bf16(y[h][0], y[h][1]), p[h][j][1] = pack_bf16(y[h][2], y[h][3]);
+        }
+        bf16_t* dst = nullptr;
+        if (m < a.M) {
+          if (head < a.nh) {
+            dst = a.q_out + ((int64_t)m * a.nh + head) * a.hd;
+          } else if (slot[i] >= 0) {
+            const int page = page_of(slot[i]);
+            dst = a.k_cache + (int64_t)page * a.kp + (int64_t)(slot[i] - page * a.page_size) * a.ks + (int64_t)(head - a.nh) * a.kh;
           }
         }
+        // lane (r, g) holds four dimensions of each of two tiles (of one half; of both, where a half is one tile): lanes g and g ^ 1 exchange
+        // so that each has eight in a row
 #pragma unroll
-        for (int h = 0; h < 2; ++h) p[h][j][0] = pack_bf16(y[h][0], y[h][1]), p[h][j][1] = pack_bf16(y[h][2], y[h][3]);
-      }
-      bf16_t* dst = nullptr;
-      if (m < a.M) {
-        if (head < a.nh) {
-          dst = a.q_out + ((int64_t)m * a.nh + head) * a.hd;
-        } else if (slot[i] >= 0) {
-          const int page = page_of(slot[i]);
-          dst = a.k_cache + (int64_t)page * a.kp + (int64_t)(slot[i] - page * a.page_size) * a.ks + (int64_t)(head - a.nh) * a.kh;
+        for (int h = 0; h < HT; ++h) {
+          const uint32_t(&one)[2] = HT == 2 ? p[h][0] : p[0][0], (&other)[2] = HT == 2 ? p[h][HT - 1] : p[1][0];
+          const auto lo = __builtin_amdgcn_permlane16_swap(one[0], other[0], false, false);
+          const auto hi = __builtin_amdgcn_permlane16_swap(one[1], other[1], false, false);
+          const int at = HT == 2 ? h * half + (g & 1) * 16 : (g & 1) * half;
+          if (dst) *(u32x4_t*)(dst + at + d0 + (g >> 1) * 8) = (u32x4_t){lo[0], hi[0], lo[1], hi[1]};
         }
       }
-      // lane (r, g) holds four dimensions of each of two tiles: lanes g and g ^ 1 exchange so that each has eight in a row
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const auto lo = __builtin_amdgcn_permlane16_swap(p[h][0][0], p[h][1][0], false, false);
-        const auto hi = __builtin_amdgcn_permlane16_swap(p[h][0][1], p[h][1][1], false, false);
-        if (dst) *(u32x4_t*)(dst + h * half + d0 + (g & 1) * 16 + (g >> 1) * 8) = (u32x4_t){lo[0], hi[0], lo[1], hi[1]};
-      }
+      continue;
     }
-    return;
-  }
-  // ---- values: [dimension of the wave's 64][token] in LDS, then eight slots a store wherever eight tokens of this wave have slots in a row
-  // that begin at a multiple of eight, a store a token for the others
-  bf16_t* turn = (bf16_t*)lds + wave * (64 * SPAN);
-  bf16_t* const base = a.v_cache + (int64_t)(head - a.nh - a.nkv) * a.vh;
-  auto dimension = [&](int d) { return d0 + d % 32 + (d >= 32 ? half : 0); };
+    // ---- values: [dimension of the unit][token] in LDS, then eight slots a store wherever eight tokens of this wave have slots in a row
+    // that begin at a multiple of eight, a store a token for the others
+    bf16_t* const base = a.v_cache + (int64_t)(head - a.nh - a.nkv) * a.vh;
+    auto dimension = [&](int d) { return d0 + d % (UNIT / 2) + (d >= UNIT / 2 ? half : 0); };
 #pragma unroll
-  for (int pass = 0; pass < PASSES; ++pass) {
-    const int begin0 = first + pass * TOKENS;
-    if (pass) wave_sync();      // the pass before has been read
+    for (int pass = 0; pass < PASSES; ++pass) {
+      const int begin0 = first + pass * TOKENS;
+      if (w || pass) wave_sync();      // the unit or pass before has been read
 #pragma unroll
-    for (int i = 0; i < TP; ++i)
+      for (int i = 0; i < TP; ++i)
 #pragma unroll
-      for (int j = 0; j < Tile::TN; ++j)
+        for (int j = 0; j < 2 * HT; ++j)
 #pragma unroll
-        for (int e = 0; e < 4; e += 2) {
-          const uint32_t both = pack_bf16(acc[j][pass * TP + i][e], acc[j][pass * TP + i][e + 1]);
-          turn[(16 * j + 4 * g + e) * SPAN + 16 * i + r] = (bf16_t)both;
-          turn[(16 * j + 4 * g + e + 1) * SPAN + 16 * i + r] = (bf16_t)(both >> 16);
-        }
-    wave_sync();
-    const int mine = lane < TOKENS && begin0 + lane < a.M ? a.slots[begin0 + lane] : -1, in_run = mine & 7, begin = lane - in_run;
-    bool whole = a.runs && mine >= 0 && begin >= 0 && begin + 7 < TOKENS;
-#pragma unroll
-    for (int k = 0; k < 8; ++k) whole = (__shfl(mine, (begin + k) & (TS_WAVE - 1), TS_WAVE) == mine - in_run + k) & whole;
-    const uint64_t runs = __ballot(whole && in_run == 0), singles = __ballot(mine >= 0 && !whole);
-    if (runs) {
-      // eight lanes take the runs, eight dimensions at a time (so that a dimension's runs leave together)
-      uint64_t left = runs;
-      for (int k = 0; k < lane % 8; ++k) left &= left - 1;
-      const int t = left ? __builtin_ctzll(left) : -1, s0 = __shfl(mine, t & (TS_WAVE - 1), TS_WAVE), page = page_of(s0);
-      bf16_t* const to = base + (int64_t)page * a.vp + (s0 - page * a.page_size);
-      const bool in_pieces = !(runs & ~0x0101010101010101ull);
-      if (t >= 0) {
-#pragma unroll
-        for (int q = 0; q < 8; ++q) {
-          const int d = lane / 8 + 8 * q;
-          const bf16_t* from = turn + d * SPAN + t;
-          u32x4_t v;
-          if (in_pieces) {
-            v = *(const u32x4_t*)from;
-          } else {
-#pragma unroll
-            for (int k = 0; k < 4; ++k) v[k] = (uint32_t)from[2 * k] | ((uint32_t)from[2 * k + 1] << 16);
+          for (int e = 0; e < 4; e += 2) {
+            const float4_t& at = acc[2 * HT * w + j][pass * TP + i];
+            const uint32_t both = pack_bf16(at[e], at[e + 1]);
+            turn[(16 * j + 4 * g + e) * SPAN + 16 * i + r] = (bf16_t)both;
+            turn[(16 * j + 4 * g + e + 1) * SPAN + 16 * i + r] = (bf16_t)(both >> 16);
           }
-          *(u32x4_t*)(to + (int64_t)dimension(d) * a.vd) = v;
+      wave_sync();
+      const int mine = lane < TOKENS && begin0 + lane < a.M ? a.slots[begin0 + lane] : -1, in_run = mine & 7, begin = lane - in_run;
+      bool whole = a.runs && mine >= 0 && begin >= 0 && begin + 7 < TOKENS;
+#pragma unroll
+      for (int k = 0; k < 8; ++k) whole = (__shfl(mine, (begin + k) & (TS_WAVE - 1), TS_WAVE) == mine - in_run + k) & whole;
+      const uint64_t runs = __ballot(whole && in_run == 0), singles = __ballot(mine >= 0 && !whole);
+      if (runs) {
+        // eight lanes take the runs, eight dimensions at a time (so that a dimension's runs leave together)
+        uint64_t left = runs;
+        for (int k = 0; k < lane % 8; ++k) left &= left - 1;
+        const int t = left ? __builtin_ctzll(left) : -1, s0 = __shfl(mine, t & (TS_WAVE - 1), TS_WAVE), page = page_of(s0);
+        bf16_t* const to = base + (int64_t)page * a.vp + (s0 - page * a.page_size);
+        const bool in_pieces = !(runs & ~0x0101010101010101ull);
+        if (t >= 0) {
+#pragma unroll
+          for (int q = 0; q < UNIT / 8; ++q) {
+            const int d = lane / 8 + 8 * q;
+            const bf16_t* from = turn + d * SPAN + t;
+            u32x4_t v;
+            if (in_pieces) {
+              v = *(const u32x4_t*)from;
+            } else {
+#pragma unroll
+              for (int k = 0; k < 4; ++k) v[k] = (uint32_t)from[2 * k] | ((uint32_t)from[2 * k + 1] << 16);
+            }
+            *(u32x4_t*)(to + (int64_t)dimension(d) * a.vd) = v;
+          }
         }
       }
-    }
-    for (uint64_t left = singles; left; left &= left - 1) {
-      const int t = __builtin_ctzll(left), s = __builtin_amdgcn_readlane(mine, t), page = page_of(s);
-      base[(int64_t)page * a.vp + (int64_t)(s - page * a.page_size) * a.vs + (int64_t)dimension(lane) * a.vd] = turn[lane * SPAN + t];
+      for (uint64_t left = singles; left; left &= left - 1) {
+        const int t = __builtin_ctzll(left), s = __builtin_amdgcn_readlane(mine, t), page = page_of(s);
+        if (UNIT == TS_WAVE || lane < UNIT)
+          base[(int64_t)page * a.vp + (int64_t)(s - page * a.page_size) * a.vs + (int64_t)dimension(lane) * a.vd] = turn[lane * SPAN + t];
+      }
     }
   }
 }
 
-template <int BM, int BN, int WM, int WN, int XN>
+template <int BM, int BN, int WM, int WN, int XN, int HT = 2>
 static int launch_whole_rope(WholeRopeArgs a, hipStream_t stream) {
   a.row_tiles = (a.M + BM - 1) / BM;
   const int64_t items = (int64_t)a.row_tiles * ((a.N + BN - 1) / BN);
   if (items > (1 << 24)) return TS_TOO_LARGE;
   a.items = (int)items, a.per_die = (a.items + 7) / 8;
-  gemm_whole_rope_kernel<BM, BN, WM, WN, XN><<<8 * a.per_die, WM * WN * TS_WAVE, 0, stream>>>(a);
+  gemm_whole_rope_kernel<BM, BN, WM, WN, XN, HT><<<8 * a.per_die, WM * WN * TS_WAVE, 0, stream>>>(a);
   return ts_check_launch();
 }
 
 // `ts_rope_store` of x [M, K] · w [(nh + 2 nkv) hd, K]^T (operands as for ts_gemm_whole_bf16) rounded to bfloat16, whole heads turned by the
 // table or, with cos_sin null, none; hd a multiple of 64, the table, q_out, the key cache and its strides in whole 16-byte pieces. tile (rows of x
-// by rows of W of a workgroup): 0 128 x 128, 1 128 x 256, 2 192 x 256, 3 64 x 128.
+// by rows of W of a workgroup): 0 128 x 128, 1 128 x 256, or x 192 where that is no more than a workgroup a compute unit either (the same bits: 3,072 columns
+// over 2,048, 2,048 rows 192 workgroups of 32.7 us and 256 of 30.0, 1,400 rows 32.1 and 28.4; 5,120 over 3,072, 1,024 rows 46.9 and 41.5, 1,280 rows,
+// 270 of them (left) 47.3 and 70.1; of two rounds either way, 1,700 rows (left) 78.1 and 78.3), 2 192 x 256, 3 64 x 128.
 extern "C" int ts_gemm_whole_rope_bf16(void* q_out, const void* x, const void* w, int M, int K, int64_t ldx, int64_t ldw, const float* cos_sin,
                                        const int32_t* positions, const int32_t* slots, void* k_cache, void* v_cache, int nh, int nkv, int hd, int page_size,
                                        int64_t kp, int64_t ks, int64_t kh, int64_t vp, int64_t vs, int64_t vh, int64_t vd, int tile, hipStream_t stream) {
@@ -326,7 +339,9 @@ extern "C" int ts_gemm_whole_rope_bf16(void* q_out, const void* x, const void* w
   a.runs = vs == 1 && page_size % 8 == 0 && vp % 8 == 0 && vh % 8 == 0 && vd % 8 == 0 && !((uintptr_t)v_cache & 15);
   switch (tile) {
     case 0: return launch_whole_rope<128, 128, 2, 2, 2>(a, stream);
-    case 1: return launch_whole_rope<128, 256, 2, 4, 2>(a, stream);
+    case 1:
+      if ((int64_t)((M + 127) / 128) * ((N + 191) / 192) <= GW_COMPUTE_UNITS) return launch_whole_rope<128, 192, 4, 2, 2, 1>(a, stream);
+      return launch_whole_rope<128, 256, 2, 4, 2>(a, stream);
     case 2: return launch_whole_rope<192, 256, 2, 4, 2>(a, stream);
     default: return launch_whole_rope<64, 128, 2, 2, 3>(a, stream);
   }

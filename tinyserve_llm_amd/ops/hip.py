@@ -2092,6 +2092,7 @@ def whole_takes(x: torch.Tensor, weight: torch.Tensor) -> bool:
 # sizes, those of a step of 64 of K for a workgroup a compute unit (and for two, where it holds two), of a million numbers of W and of a million of the product
 WHOLE_ROPE_TILES = ((128, 128, 2, (3.97, 0.474, 0.748, 0.12, 1.17)), (128, 256, 1, (4.40, 0.723, 0.0, 0.06, 0.92)),
                     (192, 256, 1, (6.50, 0.906, 0.0, 0.0, 0.96)), (64, 128, 2, (3.15, 0.324, 0.537, 0.20, 0.84)))
+WHOLE_ROPE_NARROW = (128, 192, 1, (5.2, 0.65, 0.0, 0.06, 0.60))      # what the second one is where its workgroups are no more than the compute units
 # what the product (the matrix library's: one in slices is left apart) and the rotation's kernel take: fixed, a thousand of K, that times the root of the rows over 32,
 # and a million products (of a thousand each), numbers of W and of the product
 WHOLE_ROPE_APART = (9.89, 1.506, 0.309, 1.233, 0.323, 1.167)
@@ -2107,13 +2108,17 @@ def qkv_rope_whole_plan(rows: int, n: int, k: int) -> int | None:
     5,120; 5 to 10 % root mean square here, 7 % there). Of these the rule takes 152, at 0.80 of the other way's time on average; 4 of them are
     slower by more than 2 %: n 5,120, k 3,072 513 rows 32.1 and 32.9 µs, 3,000 rows 96.0 and 101.3, n 7,168, k 5,120 2,300 rows 151.3 and 157.7, n 12,288, k 4,096 1,280
     rows 116.6 and 119.2 (inside a pass, where the library's choices are made among a few timed runs, none of 34 sizes of these two Llama
-    shapes was: whole passes at 0.95 to 1.00 of their time). Apart and here: n 3,072, k 2,048 192 rows
-    20.9 and 13.8, 513 rows 20.9 and 14.2, 1,024 rows 26.6 and 22.8, 2,048 rows 37.0 and 32.4, 3,000 rows 50.5 and 46.0; n 5,120, k 3,072
-    192 rows (left apart) 32.3 and 27.8, 720 rows 39.9 and 34.4, 1,514 rows 59.5 and 49.4, 2,048 rows 72.4 and 59.6."""
+    shapes was: whole passes at 0.95 to 1.00 of their time). The narrow form of the second tile was fitted to 18 points and adds 16 of 220 tried,
+    at 0.84 to 0.96. Apart and here: n 3,072, k 2,048 192 rows
+    20.9 and 13.8, 513 rows 20.9 and 14.2, 1,024 rows 26.6 and 22.8, 1,400 rows 33.9 and 29.7, 2,048 rows 37.0 and 30.0, 3,000 rows 50.5 and 46.0; n 5,120, k 3,072
+    192 rows (left apart) 32.3 and 27.8, 720 rows 39.9 and 34.4, 999 rows 47.9 and 42.5, 1,514 rows 59.5 and 49.4, 2,048 rows 72.4 and 59.6."""
     if not WHOLE_ROPE_MIN_ROWS <= rows <= WHOLE_ROPE_MAX_ROWS or k % 64 or k < 64 * WHOLE_MIN_STEPS or slices_plan(rows, n, k, "bf16") is not None:
         return None
     steps, costs = k // 64, []
-    for bm, bn, held, (fixed, one, two, weight, out) in WHOLE_ROPE_TILES:
+    for place, tile in enumerate(WHOLE_ROPE_TILES):
+        if place == 1 and -(-rows // 128) * -(-n // 192) <= COMPUTE_UNITS:
+            tile = WHOLE_ROPE_NARROW
+        bm, bn, held, (fixed, one, two, weight, out) = tile
         rounds = -(-(-(-rows // bm) * -(-n // bn)) // COMPUTE_UNITS)
         chain = one * (rounds % 2) + two * (rounds // 2) if held == 2 else one * rounds
         costs.append(fixed + steps * chain + (weight * k + out * rows) * n * 1e-6)

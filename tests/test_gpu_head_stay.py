@@ -25,3 +25,23 @@ def test_workgroups_that_stay_add_up_as_those_of_a_tile_each(rows, n, k, out_dty
     assert torch.equal(got, hip.gemm_skinny8(hip.pack_rows8(x, hip.skinny8_steps(k)), w, out_dtype, packed))
     want = x.double() @ w[-64:].double().t()
     torch.testing.assert_close(got[:, -64:].double(), want, rtol=2e-5 if out_dtype is torch.float32 else 2.0 ** -8, atol=1e-4 * k ** 0.5)
+
+
+@pytest.mark.parametrize("rows", [1, 3, 4, 5, 8, 16, 17, 32, 33, 64, 65, 130])
+@pytest.mark.parametrize("n,k", [(32832, 2048), (128256, 1024), (32768, 8192), (2048, 1024), (40000, 96)])
+def test_capped_logits_have_the_bits_of_the_product_and_the_cap(rows, n, k):
+    """By the kernel that makes the product where it caps its sums itself, by a kernel of its own elsewhere."""
+    from tinyserve_llm_amd.parts.ends import ProjectionHead
+    g = torch.Generator(device="cuda").manual_seed(rows + n)
+    x, w = torch.randn(rows, k, generator=g, device="cuda").to(BF), (torch.randn(n, k, generator=g, device="cuda") * 4 * k ** -0.5).to(BF)
+    x[0, 3], w[5] = 0.0, 0.0
+    if rows > 1:
+        x[1] *= 1e3      # (sums far beyond the cap)
+    head = ProjectionHead(n, k, softcap=20.0)
+    head.bind({"weight": w})
+    head.keep_streaming_copies()
+    want = hip.soft_cap(hip.linear_bf16(x, w, torch.float32, head.weight_packed), 20.0)
+    got = head.forward(x)
+    assert torch.equal(got, want) and float(got.abs().max()) <= 20.0
+    taken = hip.capped_product(x, w, head.weight_packed, 20.0) is not None
+    assert taken == (n > 8192 and ((rows <= 4 and k in (1024, 2048)) or (5 <= rows <= 32 and k in (1024, 2048) and hip.rows64_few(rows, n, k)) or (k <= 4096 and hip.rows64_takes(rows, n, k))))

@@ -437,24 +437,24 @@ PyObject* gemm_glu(Args a) {      // x, weight, tile, form's number, limit, slop
 bool squares_fit(const Tensor* s, int64_t rows) { return !s || (f32(*s) && s->dim() == 2 && s->size(0) == rows && s->size(1) >= 1 && s->is_contiguous()); }
 
 // What gemm_rows64 makes of up to 8 rows of x and the copy that the 8-row form reads (five-dimensional; its steps are those that the caller found for the reduction).
-PyObject* rows8(const Tensor& x, const Tensor& p, bool wide) {
+PyObject* rows8(const Tensor& x, const Tensor& p, bool wide, float cap) {
   const int64_t M = x.size(0), K = x.size(1), N = p.size(0) * 8;
   if (M < 1 || M > 8 || !bf16(p) || p.size(1) * p.size(2) * 64 != K || p.size(3) != 64 || p.size(4) != 8 || !p.is_contiguous() || !fits(N) || !fits(K)) return none();
   Tensor y = make(x, {M, N}, wide ? at::kFloat : at::kBFloat16);
   if (TS_REFUSED("gemm_skinny8", ts_gemm_skinny8_bf16(ptr(&y), ptr(&x), ptr(&p), M, N, K, x.stride(0), K, N, wide ? 0 : 1, 1, nullptr, nullptr, nullptr, nullptr, nullptr,
-                                                      0, nullptr, nullptr, nullptr, 0, 0, 0, 0, stream())))
+                                                      0, nullptr, nullptr, nullptr, 0, 0, 0, 0, cap, stream())))
     return none();
   return wrap(y);
 }
 
-PyObject* gemm_rows64(Args a) {      // x, packed, 32-bit out, unit's number (0: none), squares, eps, limit, slope, up_shift, `few` of the launcher if it is there -> y
+PyObject* gemm_rows64(Args a) {      // x, packed, 32-bit out, unit's number (0: none), squares, eps, limit (0: none; without a unit the sums' cap), slope, up_shift, `few` of the launcher if it is there -> y
   const Tensor *x = a.tensor(), *p = a.tensor();
   const bool wide = a.i32();
   const int unit = a.i32();
   const Tensor* sq = a.maybe();
   const float eps = a.number(), limit = a.number(), slope = a.number(), shift = a.number();
   const int few = a.left ? a.i32() : 0, steps = few > 1 ? few : 0;
-  if (a.done() && p->dim() == 5) return unit || sq || few || x->dim() != 2 || !bf16(*x) || !pieces(*x) ? none() : rows8(*x, *p, wide);
+  if (a.done() && p->dim() == 5) return unit || sq || few || x->dim() != 2 || !bf16(*x) || !pieces(*x) ? none() : rows8(*x, *p, wide, limit);
   if (!a.done() || x->dim() != 2 || !bf16(*x) || !pieces(*x) || !packed16(*p, x->size(1)) || (unit && wide) || (unit > 1 && sq)) return none();
   const int64_t M = x->size(0), K = x->size(1), N = p->size(0) * 16;
   if (M < 1 || M > ROWS64_MAX_ROWS || N % (unit ? 128 : 64) || K % 1024 || !squares_fit(sq, M) || !fits(N) || !fits(K)) return none();

@@ -41,7 +41,7 @@ int ts_gemm_rows64_sliced_bf16(void* y, void* parts, const void* x, const void* 
                                hipStream_t stream);
 int ts_gemm_skinny8_bf16(void* y, const void* x, const void* w, int M, int N, int K, int64_t ldx, int64_t ldw, int64_t ldy, int out_dtype, int packed,
                          const void* next_res, const void* next_nw, void* next_res_out, void* next_op, void* ssq_out, int x_packed8, const float* comb_o,
-                         const float* comb_ml, const int32_t* comb_pos, int comb_splits, int comb_chunk, int comb_window, int comb_hd,
+                         const float* comb_ml, const int32_t* comb_pos, int comb_splits, int comb_chunk, int comb_window, int comb_hd, float cap,
                          hipStream_t stream);
 int ts_skinny_tiles(int M, int N, int K);
 int ts_gemm_skinny_bf16(void* y, const void* x, const void* w, const void* res, const void* nw, void* res_out, int M, int N, int K, int64_t ldx, int64_t ldw,

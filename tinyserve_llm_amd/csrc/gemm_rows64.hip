@@ -65,7 +65,7 @@ struct Rows64Args {
   const float* ssq_in;
   int ssq_parts;
   float eps;
-  float limit, slope, up_shift;      // of the unit (GLU > 1)
+  float limit, slope, up_shift;      // of the unit (GLU > 1); of a plain 32-bit product: limit > 0 caps the sums, limit tanh(sum / limit), as soft_cap_kernel does
   int slices;            // the reduction in this many slices (gridDim.y); more than one: y is float [slices][M][ldy]
   int few;               // up to 32 rows whose sums are added up as the 16-row weight-streaming form does; more than 1: a gated product of up to 8 rows in
                          // the order of a reader of so many steps (SkinnyArgs::x_packed8 of gemm_skinny.hip)
@@ -317,6 +317,13 @@ __global__ void __launch_bounds__(512) gemm_rows64_kernel(const ARGS a) {
     const float by = FEW && a.ssq_in && a.ssq_parts > 1 ? scale_s[m] : scale[b];
     v *= by;
     u *= by;
+    if constexpr (GLU == 0 && sizeof(OUT) == 4) {
+      if (a.limit > 0.f) {
+        const float inv = 1.0f / a.limit;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[j] = a.limit * tanhf(v[j] * inv);
+      }
+    }
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       if constexpr (GLU == 1) v[j] = sk_silu(v[j]) * u[j];

@@ -55,7 +55,7 @@ struct SkinnyArgs {
   // sees. Its operands travel in fields that the 8-row form leaves unused otherwise, so that the block of arguments
   // which every kernel of this file fetches stays as short as it is (see SkinnyParts).
   int64_t ldx, ldw, ldy;
-  float eps;
+  float eps;            // (of a plain product of the 8-row form: the cap of its 32-bit sums, 0: none)
   // MODE_PREP: sums of squares [M, ssq_parts] of the rows of h + res, in parts (K is their width)
   const float* ssq_in;
   int ssq_parts;
@@ -1013,7 +1013,7 @@ gemm_skinny8_stay_kernel(const SkinnyArgs a) {
       for (int wv = 0; wv < nwaves; ++wv) sum += sums[wv * 256 + m * 16 + nl] + sums[wv * 256 + (m + 8) * 16 + nl + 8];
       if (m < a.M) {
         OUT* dst = (OUT*)a.y + (int64_t)m * a.ldy + 8 * tile + nl;
-        if constexpr (sizeof(OUT) == 4) *dst = sum;
+        if constexpr (sizeof(OUT) == 4) *dst = a.eps > 0.f ? a.eps * tanhf(sum * (1.0f / a.eps)) : sum;      // (capped as soft_cap_kernel does it)
         else *dst = (bf16_t)sk_round(sum);
       }
     }
@@ -1051,6 +1051,7 @@ static int sk8_dispatch(const SkinnyArgs& a, hipStream_t stream) {
       else gemm_skinny8_stay_kernel<8, OUT><<<SK8_STAY_GRID, block, 0, stream>>>(a);
       return ts_check_launch();
     }
+    if (a.eps > 0.f) return TS_BAD_SHAPE;
   }
   if (steps == 4) gemm_skinny8_kernel<4, 512, OUT, NEXT><<<grid, block, smem, stream>>>(a);
   else if (steps == 8) gemm_skinny8_kernel<8, 512, OUT, NEXT><<<grid, block, smem, stream>>>(a);
@@ -1074,13 +1075,15 @@ static bool sk_next_ok(const void* next_res, const void* next_nw, const void* ne
 // y is not written: next_res_out, next_op [M, N] and ssq_out [M, (N + 7) / 8] are. x_packed8: x is given in
 // the order the lanes read it (SkinnyArgs::x_packed8; K / 8 16-byte pieces of 64 lanes, whatever M), ldx unused.
 // comb_o (x null, M = 1, bfloat16 out, K a multiple of 256 up to 2,048): x is made on the way in from the split-key
-// attention kernel's parts (SkinnyParts; comb_hd a multiple of 32 that divides K, up to 16 chunks).
+// attention kernel's parts (SkinnyParts; comb_hd a multiple of 32 that divides K, up to 16 chunks). cap > 0 (32-bit out, by the workgroups that stay
+// only): y = cap tanh(sum / cap).
 extern "C" int ts_gemm_skinny8_bf16(void* y, const void* x, const void* w, int M, int N, int K, int64_t ldx, int64_t ldw,
                                     int64_t ldy, int out_dtype, int packed, const void* next_res, const void* next_nw,
                                     void* next_res_out, void* next_op, void* ssq_out, int x_packed8, const float* comb_o,
                                     const float* comb_ml, const int32_t* comb_pos, int comb_splits, int comb_chunk,
-                                    int comb_window, int comb_hd, hipStream_t stream) {
+                                    int comb_window, int comb_hd, float cap, hipStream_t stream) {
   if (M <= 0 || N <= 0) return TS_OK;
+  if (cap > 0.f && (next_nw || comb_o || out_dtype != 0)) return TS_BAD_SHAPE;
   if (comb_o) {
     if (x || x_packed8 || M != 1 || out_dtype != 1 || !comb_ml || !comb_pos || comb_splits < 1 || comb_splits > SK_COMB_CHUNKS ||
         comb_chunk <= 0 || comb_hd <= 0 || comb_hd % 32 || K % comb_hd || K % 256 || K > 2048 ||
@@ -1093,6 +1096,7 @@ extern "C" int ts_gemm_skinny8_bf16(void* y, const void* x, const void* w, int M
   SkinnyArgs a = {};
   a.x = (const bf16_t*)x; a.w = (const bf16_t*)w; a.y = y; a.M = M; a.N = N; a.K = K; a.ldx = ldx; a.ldw = ldw; a.ldy = ldy;
   a.packed = packed;
+  a.eps = cap > 0.f ? cap : 0.f;
   a.x_packed8 = x_packed8 != 0;
   if (comb_o) {                                         // (see SkinnyParts)
     a.x_packed8 = 2;

@@ -88,7 +88,7 @@ def _declare(lib: ctypes.CDLL) -> None:
         "ts_gemm_library_choices": [p, i],
         "ts_paged_attention_prefill": [p, p, p, p, p, p, p, p, i, i, i, i, i, i, i, i64, i64, i64, i64, i64, i64, i, f, i, i, i, i, i, p, p, i, p],
         "ts_gemm_skinny_bf16": [p, p, p, p, p, p, i, i, i, i64, i64, i64, f, i, i, i, i, p, i, p, p, p, p, p, i, f, f, f, p],
-        "ts_gemm_skinny8_bf16": [p, p, p, i, i, i, i64, i64, i64, i, i, p, p, p, p, p, i, p, p, p, i, i, i, i, p],
+        "ts_gemm_skinny8_bf16": [p, p, p, i, i, i, i64, i64, i64, i, i, p, p, p, p, p, i, p, p, p, i, i, i, i, f, p],
         "ts_gemm_skinny8_act_bf16": [p, p, p, i, i, i, i64, i64, i64, i, i, p, i, p],
         "ts_gemm_slices_bf16": [p, p, p, p, p, i, i, i, i64, i64, i, i, i, p, p, f, p],
         "ts_gemm_whole_bf16": [i, p, p, p, p, i, i, i64, i64, i, i, i, p],
@@ -1173,12 +1173,12 @@ def gemm_skinny8(x: "torch.Tensor | PackedRows8 | SplitAttention", weight: torch
         _run("gemm_skinny8", library().ts_gemm_skinny8_bf16(
             None, x_arg, _ptr(weight if packed8 is None else packed8), M, N, K, ldx, weight.stride(0), N, 1,
             int(packed8 is not None), _ptr(residual), _ptr(nw), _ptr(prepared.summed), _ptr(prepared.operand),
-            _ptr(prepared.squares), int(x_packed), *comb, _stream()))
+            _ptr(prepared.squares), int(x_packed), *comb, 0.0, _stream()))
         return prepared
     out = torch.empty((M, N), dtype=out_dtype, device=xt.device)
     _run("gemm_skinny8", library().ts_gemm_skinny8_bf16(
         _ptr(out), x_arg, _ptr(weight if packed8 is None else packed8), M, N, K, ldx, weight.stride(0),
-        out.stride(0), _code(out_dtype), int(packed8 is not None), None, None, None, None, None, int(x_packed), *comb, _stream()))
+        out.stride(0), _code(out_dtype), int(packed8 is not None), None, None, None, None, None, int(x_packed), *comb, 0.0, _stream()))
     return out
 
 
@@ -2338,6 +2338,22 @@ def linear_bf16(x: torch.Tensor, weight: torch.Tensor, out_dtype: torch.dtype = 
     if plan is not None and slices_takes(x, weight):
         return gemm_slices(x, weight, *plan, out_dtype)
     return gemm_library(x, weight, out_dtype)
+
+
+def capped_product(x: torch.Tensor, weight: torch.Tensor, packed: StreamingCopies | None, cap: float) -> torch.Tensor | None:
+    """cap tanh(x · weight^T / cap) in float32, the bits of `soft_cap` of that product, by the kernel `linear_bf16` gives the product to where that
+    caps its sums on their way out (the ones that read a wide weight's copies: the shared-x kernel and the 8-row form's workgroups that stay); None where not."""
+    if packed is None or not (x.is_cuda and x.dim() == 2 and weight.dim() == 2 and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and _dense_rows(x)
+                              and weight.is_contiguous() and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0 and x.shape[1] == weight.shape[1] and cap > 0):
+        return None
+    rows, (n, k) = x.shape[0], weight.shape
+    few = rows64_few(rows, n, k)
+    if packed.by16 is not None and packed.by16.shape[0] * 16 == n and (few or rows64_takes(rows, n, k)):
+        return _native().gemm_rows64(x, packed.by16, True, 0, None, 0.0, cap, 0.0, 0.0, int(few))
+    steps = skinny8_steps(k)
+    if packed.by8 is not None and not few and skinny8_takes(rows, n, k) and steps and packed.by8.shape == (n // 8, k // (64 * steps), steps, 64, 8) and n % 8 == 0:
+        return _native().gemm_rows64(x, packed.by8, True, 0, None, 0.0, cap, 0.0, 0.0)
+    return None
 
 
 def linear_parts(x: torch.Tensor, weight: torch.Tensor, packed: StreamingCopies | None = None) -> RowParts | None:

@@ -95,5 +95,8 @@ class ProjectionHead(Head):
         return 0 if self.weight_packed is None else self.weight_packed.nbytes()
 
     def forward(self, rows: torch.Tensor) -> torch.Tensor:
+        capped = hip.capped_product(rows, self.weight, self.weight_packed, self.softcap) if self.softcap else None
+        if capped is not None:
+            return capped
         logits = linear(rows, self.weight, out_dtype=torch.float32, packed=self.weight_packed)
         return hip.soft_cap(logits, self.softcap) if self.softcap else logits

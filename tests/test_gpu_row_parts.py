@@ -65,6 +65,21 @@ def test_a_product_in_slices_leaves_its_parts(rows, n, k):
     assert hip.linear_parts(x[:, ::2], w[:, : k // 2]) is None      # (rows that are not dense)
 
 
+@pytest.mark.parametrize("rows,n,k,taken", [(300, 2048, 4096, True), (999, 2048, 4096, True), (1000, 1024, 4096, True), (700, 2048, 4096, False), (999, 2048, 2048, False),
+                                            (128, 2048, 4096, False), (2048, 2048, 8192, True)])
+def test_a_product_leaves_parts_sooner_for_a_norm_that_adds_them(rows, n, k, taken):
+    """Against 64 bits: chains of at most k numbers, their bfloat16 products exact in 32 bits, and no further from it than the product made whole."""
+    g = torch.Generator(device="cuda").manual_seed(rows)
+    x, w = torch.randn(rows, k, generator=g, device="cuda").to(BF), torch.randn(n, k, generator=g, device="cuda").to(BF)
+    parts = hip.linear_parts(x, w, sooner=True)
+    assert (parts is not None) == taken
+    if taken:
+        want, size = x.double() @ w.double().t(), x.double().abs() @ w.double().abs().t()
+        off = (parts.rows().double() - want).abs()
+        assert bool((off <= k * 2.0 ** -24 * size).all())
+        assert float(off.norm()) <= 1.1 * float((hip.linear_bf16(x, w, F32).double() - want).norm())
+
+
 @pytest.mark.parametrize("top,identity,shared", [(1, False, None), (2, True, "gated"), (4, True, "plain"), (4, False, "gated"), (5, True, None), (9, True, "plain")])
 @pytest.mark.parametrize("n,width", [(1, 64), (7, 1028), (48, 2048), (130, 2052), (3, 4096), (2, 4100)])
 def test_experts_rows_are_added_up_where_the_stream_takes_them(n, width, top, identity, shared):

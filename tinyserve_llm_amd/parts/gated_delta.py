@@ -22,6 +22,7 @@ from tinyserve_llm_amd.parts.linear import linear, streaming_copy
 @register("mixer", "gated_delta")
 class GatedDelta(Mixer):
     graph_safe = True
+    leaves_parts = True
 
     def __init__(self, hidden_size: int, num_heads: int, groups: int, head_dim: int, value_dim: int, conv_taps: int, norm_eps: float) -> None:
         self.sizes = hip.SsdSizes(num_heads, value_dim, groups, head_dim, conv_taps)
@@ -66,10 +67,11 @@ class GatedDelta(Mixer):
         self.proj_packed, self.o_packed = streaming_copy(self.proj), streaming_copy(self.o)
         return sum(c.nbytes() for c in (self.proj_packed, self.o_packed) if c is not None)
 
-    def forward(self, x: torch.Tensor, ctx: StepContext, mem: LayerMemory) -> torch.Tensor:
+    def forward(self, x: torch.Tensor, ctx: StepContext, mem: LayerMemory, parts: bool = False) -> "torch.Tensor | hip.RowParts":
         z = self.sizes
         proj = linear(x, self.proj, out_dtype=torch.float32, packed=self.proj_packed)
         rows = hip.delta_prepare(proj, self._conv, self.dt_bias, self.a_log, mem.state, ctx, z, x.dtype)
         o = hip.delta_scan(rows, mem.state, ctx, z)
         gated = hip.mlstm_finish(o, self.norm, proj[:, :z.inner], z.heads, z.vdim, self.norm_eps, x.dtype, silu_gate=True)
-        return linear(gated, self.o, out_dtype=torch.float32, packed=self.o_packed)
+        out = hip.linear_parts(gated, self.o, self.o_packed, sooner=True) if parts else None
+        return out if out is not None else linear(gated, self.o, out_dtype=torch.float32, packed=self.o_packed)

@@ -1,0 +1,54 @@
+"""A step's decoding tokens and prompts attended to in one launch: the bits of the two launches."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from tinyserve_llm_amd.ops import hip
+
+BF, I32 = torch.bfloat16, torch.int32
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("extra", ["plain", "cap", "sinks", "gate", "window", "chunks"])
+@pytest.mark.parametrize("heads,kv,dim", [(8, 2, 64), (3, 1, 64), (16, 1, 64), (6, 2, 128), (4, 4, 128)])
+@pytest.mark.parametrize("rt,waves,chunk,dwaves,lead,page", [(1, 4, 128, 4, 33, 64), (1, 4, 256, 8, 1, 32), (1, 8, 256, 8, 5, 256), (2, 4, 256, 8, 33, 96),
+                                                             (1, 4, 256, 4, 5, 256), (1, 8, 512, 8, 33, 32), (2, 4, 1024, 8, 1, 256)])
+def test_one_launch_has_the_bits_of_two(rt, waves, chunk, dwaves, lead, page, heads, kv, dim, extra):
+    if dim == 128 and chunk != 32 * dwaves:
+        chunk, dwaves = chunk // 2, 4          # (wide heads decode in up to four waves where a wave has several steps)
+    g = torch.Generator().manual_seed(lead + heads + chunk)
+    prompts = [70, 1, 33]
+    lengths = [int(n) for n in torch.randint(1, 700, (lead,), generator=g)]
+    lengths[0] = 700
+    starts = [n - 1 for n in lengths] + [0, 5, 64]
+    ends = lengths + [s + n for s, n in zip(starts[lead:], prompts)]
+    per = [-(-n // page) for n in ends]
+    pages, width = sum(per) + 1, max(per)
+    tables, at, order = torch.zeros(len(ends), width, dtype=I32), 0, torch.randperm(pages, generator=g)
+    for i, n in enumerate(per):
+        tables[i, :n] = order[at:at + n]
+        at += n
+    tables = tables.cuda()
+    k = torch.randn(pages, kv, page, dim, generator=g).to(BF).cuda().permute(0, 2, 1, 3)
+    v = torch.randn(pages, kv, dim, page, generator=g).to(BF).cuda().permute(0, 3, 1, 2)
+    total = lead + sum(prompts)
+    q = torch.randn(total, heads, dim, generator=g).to(BF).cuda()
+    seq = torch.tensor(list(range(lead)) + [lead + i for i, n in enumerate(prompts) for _ in range(n)], dtype=I32).cuda()
+    pos = torch.tensor(starts[:lead] + [s + j for s, n in zip(starts[lead:], prompts) for j in range(n)], dtype=I32).cuda()
+    cu = list(range(lead + 1))
+    for n in prompts:
+        cu.append(cu[-1] + n)
+    tile = rt * waves * (16 // (heads // kv))
+    tiles = torch.tensor(hip.attention_tiles(cu, starts, tile, lead), dtype=I32).view(-1, 2).cuda()
+    window = {"window": 100, "chunks": -96}.get(extra, 0)
+    more = dict(softcap=30.0 if extra == "cap" else 0.0, sink=False, sinks=torch.randn(heads, generator=g).cuda() if extra == "sinks" else None, slopes=None,
+                gate=torch.randn(total, heads * dim, generator=g).cuda() if extra == "gate" else None)
+    one = hip._native().attention_step(q, k, v, tables, seq, pos, tiles, dim ** -0.5, window, *more.values(), 1, lead, chunk, dwaves, tile, waves, 1, 0, lead)
+    two = torch.zeros_like(q)
+    hip.paged_attention_prefill(q, k, v, tables, seq, pos, tiles, dim ** -0.5, window, tile, two, waves=waves, first_token=lead, **more)
+    if more["gate"] is not None:
+        more["gate"] = more["gate"][:lead]
+    hip.paged_attention_decode(q[:lead], k, v, tables, seq[:lead], pos[:lead], dim ** -0.5, window, chunk, dwaves, two[:lead], **more)
+    assert torch.equal(one, two)

@@ -25,6 +25,7 @@
 // one head's keys sit on as few dies as possible: with eight heads (or a multiple) each die works
 // on heads of its own and reads their keys from memory once.
 #include <type_traits>
+#include "attention_decode.h"
 #include "lds_loads.h"
 
 #define PRE_MAX_WAVES 8
@@ -324,6 +325,36 @@ prefill_tile(PrefillLds<HD, WHOLE>& lds, int tile, int kvh, bf16_t* __restrict__
     }
 }
 
+// Workgroup `block` of `blocks`, the kernel's own or the first ones of the kernel below.
+template <int HD, int RT, int PRE_WAVES, bool WHOLE, bool GENERAL>
+static __device__ __forceinline__ void
+prefill_block(PrefillLds<HD, WHOLE>& lds, int block, int blocks, bf16_t* __restrict__ out, const bf16_t* __restrict__ q, const bf16_t* __restrict__ k_cache,
+                         const bf16_t* __restrict__ v_cache, const int32_t* __restrict__ block_tables,
+                         const int32_t* __restrict__ seq_of_token, const int32_t* __restrict__ positions,
+                         const int32_t* __restrict__ tiles, int num_tiles, int nh, int group, int dies_per_group,
+                         int heads_per_group, int page_size, int page_shift, int page_run, int64_t kp, int64_t ks, int64_t kh,
+                         int64_t vp, int64_t vh, int64_t vd, int max_blocks, float scale2, int window,
+                         float* __restrict__ part_o, float* __restrict__ part_ml, int num_splits, int chunk,
+                         float cap_in, float cap_out, int sink, const float* __restrict__ sinks,
+                         const float* __restrict__ slopes, const float* __restrict__ gate, int64_t gate_stride) {
+  // die = workgroup index mod 8. The dies form `groups` groups of `dies_per_group`, the heads as
+  // many groups of `heads_per_group`; a group's (tile, head) pairs go round its dies, long tiles first.
+  // A die's workgroups go round its 32 compute units. Where two of them fit a unit, those of a short prompt run all at once, and
+  // every other round takes its tiles in the opposite order, so that the unit with the longest walk of one round has the
+  // shortest of the next (heads of 64: 1,024 tokens 18.2 and now 16.0 µs, 2,048 33.8 and 32.3; of 128 with eight waves, one
+  // workgroup a unit, 46.0 and 54.2: longest first there).
+  constexpr bool PAIRS = PRE_WAVES == 4 ? RT * HD <= 256 : HD <= 64;
+  const int die = block % 8, place = block / 8, round = place / 32;
+  const int turn = PAIRS && round % 2 ? 32 * round + min(32 * round + 32, blocks / 8) - 1 - place : place;
+  const int item = turn * dies_per_group + die % dies_per_group;
+  if (item >= num_tiles * heads_per_group) return;
+  const int tile = num_tiles - 1 - item / heads_per_group;
+  const int kvh = (die / dies_per_group) * heads_per_group + item % heads_per_group;
+  prefill_tile<HD, RT, PRE_WAVES, WHOLE, GENERAL>(lds, tile, kvh, out, q, k_cache, v_cache, block_tables, seq_of_token, positions, tiles, nh,
+                       group, page_size, page_shift, page_run, kp, ks, kh, vp, vh, vd, max_blocks, scale2, window, part_o, part_ml,
+                       num_splits, chunk, blockIdx.y, cap_in, cap_out, sink, sinks, slopes, gate, gate_stride);
+}
+
 template <int HD, int RT, int PRE_WAVES, bool WHOLE, bool GENERAL>
 __global__ void __launch_bounds__(PRE_WAVES * TS_WAVE)
 attn_prefill_mfma_kernel(bf16_t* __restrict__ out, const bf16_t* __restrict__ q, const bf16_t* __restrict__ k_cache,
@@ -336,22 +367,36 @@ attn_prefill_mfma_kernel(bf16_t* __restrict__ out, const bf16_t* __restrict__ q,
                          float cap_in, float cap_out, int sink, const float* __restrict__ sinks,
                          const float* __restrict__ slopes, const float* __restrict__ gate, int64_t gate_stride) {
   __shared__ __attribute__((aligned(1024))) PrefillLds<HD, WHOLE> lds;
-  // die = workgroup index mod 8. The dies form `groups` groups of `dies_per_group`, the heads as
-  // many groups of `heads_per_group`; a group's (tile, head) pairs go round its dies, long tiles first.
-  // A die's workgroups go round its 32 compute units. Where two of them fit a unit, those of a short prompt run all at once, and
-  // every other round takes its tiles in the opposite order, so that the unit with the longest walk of one round has the
-  // shortest of the next (heads of 64: 1,024 tokens 18.2 and now 16.0 µs, 2,048 33.8 and 32.3; of 128 with eight waves, one
-  // workgroup a unit, 46.0 and 54.2: longest first there).
-  constexpr bool PAIRS = PRE_WAVES == 4 ? RT * HD <= 256 : HD <= 64;
-  const int die = blockIdx.x % 8, place = blockIdx.x / 8, round = place / 32;
-  const int turn = PAIRS && round % 2 ? 32 * round + min(32 * round + 32, (int)gridDim.x / 8) - 1 - place : place;
-  const int item = turn * dies_per_group + die % dies_per_group;
-  if (item >= num_tiles * heads_per_group) return;
-  const int tile = num_tiles - 1 - item / heads_per_group;
-  const int kvh = (die / dies_per_group) * heads_per_group + item % heads_per_group;
-  prefill_tile<HD, RT, PRE_WAVES, WHOLE, GENERAL>(lds, tile, kvh, out, q, k_cache, v_cache, block_tables, seq_of_token, positions, tiles, nh,
-                       group, page_size, page_shift, page_run, kp, ks, kh, vp, vh, vd, max_blocks, scale2, window, part_o, part_ml,
-                       num_splits, chunk, blockIdx.y, cap_in, cap_out, sink, sinks, slopes, gate, gate_stride);
+  prefill_block<HD, RT, PRE_WAVES, WHOLE, GENERAL>(lds, blockIdx.x, gridDim.x, out, q, k_cache, v_cache, block_tables, seq_of_token, positions, tiles, num_tiles, nh,
+                                                   group, dies_per_group, heads_per_group, page_size, page_shift, page_run, kp, ks, kh, vp, vh, vd, max_blocks,
+                                                   scale2, window, part_o, part_ml, num_splits, chunk, cap_in, cap_out, sink, sinks, slopes, gate, gate_stride);
+}
+
+// A step of decoding tokens beside prompts in one launch: the prompts' workgroups first, then one per (decoding token, key/value head, chunk of keys), as
+// attention_decode.hip has them. The ones multiply and take LDS, the others wait for memory, and side by side they take
+// little more than the longer of the two, where two launches follow each other. The bits are those of the two launches. us, two launches and one (the combining kernel's
+// counted with both): 24 heads of 128, 13 requests of up to 1,700 keys beside prompts of 751 and 750 tokens 48.6 and 41.8, beside 300 tokens 35.1 and 25.4; 32
+// heads of 64, 8 requests of 500 beside 64 tokens 13.2 and 8.8, 32 of 1,000 beside 300 21.0 and 16.5, 64 of 2,000 beside 200 50.0 and 43.1, beside 2,000 67.2
+// and 64.9; capped, 24 of 900 beside 700 29.1 and 20.2. (Both kinds of workgroup in turn: 58.8 where this order takes 38.9, 8 of 2,000 beside 2,000; two streams, which
+// meet in two events: 10 to 15 us more than one launch after the other.)
+template <int HD, int RT, int PRE_WAVES, bool ONE, bool GENERAL, bool ONCE>
+__global__ void __launch_bounds__(PRE_WAVES * TS_WAVE)
+attn_step_kernel(const DecodeArgs d, const int32_t* __restrict__ tiles, int num_tiles, int group, int dies_per_group, int heads_per_group, int prefill_blocks,
+                 int decode_waves, int tokens) {
+  __shared__ __attribute__((aligned(1024))) PrefillLds<HD, true> lds;
+  const int block = blockIdx.x;
+  if (block < prefill_blocks) {
+    prefill_block<HD, RT, PRE_WAVES, true, GENERAL>(lds, block, prefill_blocks, d.out, d.q, d.k_cache, d.v_cache, d.block_tables, d.seq_of_token, d.positions, tiles,
+                                                    num_tiles, d.nh, group, dies_per_group, heads_per_group, d.page_size, d.page_shift, d.page_run, d.kp, d.ks, d.kh,
+                                                    d.vp, d.vh, d.vd, d.max_blocks, d.scale2, d.window, nullptr, nullptr, 1, 0, d.cap_in, d.cap_out, d.sink, d.sinks,
+                                                    d.slopes, d.gate, d.gate_stride);
+    return;
+  }
+  const int id = block - prefill_blocks, split = id % d.num_splits, rest = id / d.num_splits, heads = d.nh / d.G;
+  decode_chunk<HD, ONE, GENERAL, ONCE, true>((float*)&lds, decode_waves, split, rest % heads, rest / heads, tokens, d.out, d.part_o, d.part_ml, d.q, d.k_cache,
+                                              d.v_cache, d.block_tables, d.seq_of_token, d.positions, d.nh, d.G, d.page_size, d.page_shift, d.page_run, d.kp, d.ks,
+                                              d.kh, d.vp, d.vh, d.vd, d.max_blocks, d.num_splits, d.chunk, d.scale2, d.window, d.cap_in, d.cap_out, d.sink, d.sinks,
+                                              d.slopes, d.gate, d.gate_stride);
 }
 
 // Keys: rows dense in head_dim, strides kp/ks/kh (page, slot, head). Values: transposed pages,
@@ -471,4 +516,56 @@ extern "C" int ts_paged_attention_prefill_general(void* out, const void* q, cons
                         nkv, hd, page_size, kp, ks, kh, vp, vh, vd, max_blocks, scale, window, first_token, num_tokens,
                         num_splits, chunk, part_o, part_ml, page_run, true, softcap, sink || sinks, sinks, slopes, gate, gate_stride,
                         stream);
+}
+
+// The decoding tokens 0 .. num_tokens - 1 and the tiles' tokens of a step in one launch (attn_step_kernel), then the decoding tokens' chunks combined: what
+// ts_paged_attention_decode[_general] and ts_paged_attention_prefill[_general] make of these operands, for pages of whole 32-key steps, heads of 64 (plain or
+// general) or 128 (plain) and prompts that are not split.
+extern "C" int ts_paged_attention_step(void* out, float* part_o, float* part_ml, const void* q, const void* k_cache, const void* v_cache,
+                                       const int32_t* block_tables, const int32_t* seq_of_token, const int32_t* positions, int num_tokens, int num_splits,
+                                       int chunk, int decode_waves, const int32_t* tiles, int num_tiles, int tile_tokens, int waves, int nh, int nkv, int hd,
+                                       int page_size, int64_t kp, int64_t ks, int64_t kh, int64_t vp, int64_t vh, int64_t vd, int max_blocks, float scale,
+                                       int window, int page_run, int general, float softcap, int sink, const float* sinks, const float* slopes,
+                                       const float* gate, int64_t gate_stride, hipStream_t stream) {
+  if (num_tokens <= 0 || num_tiles <= 0 || nkv <= 0 || nh % nkv || nh / nkv > 16 || page_size <= 0 || page_size % 32 || max_blocks <= 0 || page_run < 0 || page_run > 16)
+    return TS_BAD_SHAPE;
+  if (!(hd == 64 || (hd == 128 && !general)) || softcap < 0.f || (!general && (softcap > 0.f || sink || sinks || slopes || gate))) return TS_BAD_SHAPE;
+  if (gate && gate_stride < (int64_t)nh * hd && -gate_stride < nh) return TS_BAD_SHAPE;
+  if (decode_waves < 1 || decode_waves > DEC_WAVES_FOR(hd, chunk == 32 * decode_waves) || chunk <= 0 || chunk % (32 * decode_waves) || num_splits < 1 || num_splits > 1024 || (num_splits > 1 && (!part_o || !part_ml)))
+    return TS_BAD_SHAPE;
+  const int G = nh / nkv;
+  if ((waves != 4 && waves != 8) || decode_waves < waves) return TS_BAD_SHAPE;      // (a workgroup's waves all have chunks to walk)
+  const int per_wave = waves * (16 / G), rt = tile_tokens / per_wave, group = G | ((16 / G) << 8) | (((255 + G) / G) << 16);
+  if (tile_tokens != rt * per_wave || !(rt == 1 || (rt == 2 && waves == 4))) return TS_BAD_SHAPE;
+  if ((size_t)decode_waves * (32 + G * hd) * sizeof(float) > (hd == 64 ? sizeof(PrefillLds<64, true>) : sizeof(PrefillLds<128, true>))) return TS_BAD_SHAPE;
+  if ((kp | ks | kh | vp | vh | vd) % 8 || ((((uintptr_t)q) | ((uintptr_t)k_cache) | ((uintptr_t)v_cache)) & 15)) return TS_BAD_SHAPE;
+  int groups = 8;                                   // gcd(nkv, 8)
+  while (nkv % groups) groups /= 2;
+  const int dies_per_group = 8 / groups, heads_per_group = nkv / groups;
+  const int64_t turns = ((int64_t)num_tiles * heads_per_group + dies_per_group - 1) / dies_per_group, all = 8 * turns + (int64_t)num_tokens * nkv * num_splits;
+  if (all > 0x7fffffff) return TS_BAD_SHAPE;
+  int page_shift = -1;
+  if ((page_size & (page_size - 1)) == 0) page_shift = __builtin_ctz(page_size);
+  const float log2e = 1.44269504088896340736f;
+  const bool capped = softcap > 0.f;
+  const DecodeArgs d = {(bf16_t*)out, part_o, part_ml, (const bf16_t*)q, (const bf16_t*)k_cache, (const bf16_t*)v_cache, block_tables, seq_of_token, positions, nh, G,
+                        page_size, page_shift, page_run, kp, ks, kh, vp, vh, vd, max_blocks, num_splits, chunk, capped ? 1.0f : scale * log2e, window,
+                        capped ? scale / softcap : 0.f, softcap * log2e, sink || sinks, sinks, slopes, gate, gate_stride};
+  const int64_t reach = (int64_t)num_splits * chunk, within = window < 0 ? -(int64_t)window : window, keys = within && within < reach ? within : reach;
+  const bool once = (int64_t)num_tokens * nkv * hd * 4 * keys >= DEC_ONCE_BYTES;
+#define TS_STEP(HH, RR, WW, ON, GG, NC) \
+  attn_step_kernel<HH, RR, WW, ON, GG, NC><<<(unsigned)all, WW * TS_WAVE, 0, stream>>>(d, tiles, num_tiles, group, dies_per_group, heads_per_group, (int)(8 * turns), decode_waves, num_tokens)
+#define TS_STEP_N(HH, RR, WW, ON, GG) if (once) { TS_STEP(HH, RR, WW, ON, GG, true); } else { TS_STEP(HH, RR, WW, ON, GG, false); }
+#define TS_STEP_O(HH, RR, WW, GG) if (chunk == 32 * decode_waves) { TS_STEP_N(HH, RR, WW, true, GG) } else { TS_STEP_N(HH, RR, WW, false, GG) }
+#define TS_STEP_W(HH, GG) \
+  if (rt == 2) { TS_STEP_O(HH, 2, 4, GG) } else if (waves == 4) { TS_STEP_O(HH, 1, 4, GG) } else { TS_STEP_O(HH, 1, 8, GG) }
+  if (hd == 128) { TS_STEP_W(128, false) } else if (general) { TS_STEP_W(64, true) } else { TS_STEP_W(64, false) }
+#undef TS_STEP_W
+#undef TS_STEP_O
+#undef TS_STEP_N
+#undef TS_STEP
+  const int rc = ts_check_launch();
+  if (rc || num_splits == 1) return rc;
+  return ts_launch_attention_combine(out, part_o, part_ml, positions, num_tokens, nh, hd, num_splits, chunk, window, stream, general ? (sink || sinks) : 0,
+                                     general ? sinks : nullptr, gate, gate_stride);
 }

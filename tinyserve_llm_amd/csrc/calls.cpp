@@ -680,6 +680,13 @@ PyObject* attention_step(Args a) {
   const int32_t *tb = typed<int32_t>(tables), *sq = typed<int32_t>(seq), *ps = typed<int32_t>(pos), *tl = typed<int32_t>(tiles);
   const int64_t k0 = k->stride(0), k1 = k->stride(1), k2 = k->stride(2), v0 = v->stride(0), v2 = v->stride(2), v3 = v->stride(3);
   const float *sk = typed<float>(sinks), *sl = typed<float>(slopes), *gt = typed<float>(gate);
+  // both in one launch (attn_step_kernel), unless the decoding part's chunks are for fewer waves than the prompts' tiles (24 heads of 128, 64 requests of 2,048
+  // keys for four waves beside 1,500 tokens for eight: 111 us in two launches, 125 in one)
+  if (lead && splits == 1 && first == lead && page % 32 == 0 && dwaves >= waves && (hd == 64 || (hd == 128 && !general)) && tile_tokens <= 2 * per_wave &&
+      !TS_REFUSED("paged_attention_step",
+                  ts_paged_attention_step(ptr(&out), dpof, dpmf, ptr(q), ptr(k), ptr(v), tb, sq, ps, lead, dsplits, dchunk, dwaves, tl, tiles->size(0), tile_tokens, waves,
+                                          nh, nkv, hd, page, k0, k1, k2, v0, v2, v3, blocks, scale, window, run, general, softcap, sink, sk, sl, gt, gstride, stream())))
+    return wrap(out);
   if (lead && general) {
     if (TS_REFUSED("paged_attention_decode_general",
                    ts_paged_attention_decode_general(ptr(&out), dpof, dpmf, ptr(q), ptr(k), ptr(v), tb, sq, ps, lead, nh, nkv, hd, page, k0, k1, k2, v0, v2, v3, blocks,

@@ -56,6 +56,11 @@ int ts_gemm_rows64_sliced_rope_bf16(void* q_out, void* parts, const void* x, con
                                     const void* ssq_in, int ssq_parts, float eps, const float* cos_sin, const int32_t* positions,
                                     const int32_t* slots, void* k_cache, void* v_cache, int nh, int nkv, int hd, int rotate, int page_size,
                                     int64_t kp, int64_t ks, int64_t kh, int64_t vp, int64_t vs, int64_t vh, int64_t vd, hipStream_t stream);
+int ts_paged_attention_step(void* out, float* part_o, float* part_ml, const void* q, const void* k_cache, const void* v_cache, const int32_t* block_tables,
+                            const int32_t* seq_of_token, const int32_t* positions, int num_tokens, int num_splits, int chunk, int decode_waves,
+                            const int32_t* tiles, int num_tiles, int tile_tokens, int waves, int nh, int nkv, int hd, int page_size, int64_t kp, int64_t ks,
+                            int64_t kh, int64_t vp, int64_t vh, int64_t vd, int max_blocks, float scale, int window, int page_run, int general, float softcap,
+                            int sink, const float* sinks, const float* slopes, const float* gate, int64_t gate_stride, hipStream_t stream);
 int ts_paged_attention_decode(void* out, float* part_o, float* part_ml, const void* q, const void* k_cache, const void* v_cache,
                               const int32_t* block_tables, const int32_t* seq_of_token, const int32_t* positions, int num_tokens, int nh,
                               int nkv, int hd, int page_size, int64_t kp, int64_t ks, int64_t kh, int64_t vp, int64_t vh, int64_t vd,

@@ -37,6 +37,18 @@ def test_several_products_of_one_launch(tile, over):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("tile, rows, n", [(1, 1000, 6144), (1, 1000, 6152), (1, 1200, 8192), (1, 127, 8), (2, 768, 10304), (2, 769, 10304), (2, 1792, 9280), (2, 193, 200),
+                                           (3, 1000, 12288), (3, 1000, 12296), (3, 2048, 4160), (3, 257, 184)])
+def test_tiles_are_narrow_or_wide_with_the_same_bits(tile, rows, n):
+    """Up to and past the last width that 192 columns take no more rounds of the chip for, in one round and in two; a tile's sums are those of tiles of
+    128 x 128, whole and in each slice."""
+    x, w = operands(rows, n, 448, x_skew=8)
+    for out in (torch.float32, BF):
+        assert torch.equal(hip.gemm_whole([x], [w], tile, out)[0], hip.gemm_whole([x], [w], 0, out)[0])
+    assert torch.equal(hip.gemm_slices(x, w, tile, 2, torch.float32), hip.gemm_slices(x, w, 0, 2, torch.float32))
+
+
+@pytest.mark.gpu
 def test_what_the_whole_tiles_do_not_take_is_refused():
     x, w = operands(130, 64, 256)
     for bad in (lambda: hip.gemm_whole([x] * 9, [w] * 9, 0), lambda: hip.gemm_whole([x, x[:129]], [w, w], 0), lambda: hip.gemm_whole([x], [w[:, :192]], 0),

@@ -155,11 +155,15 @@ static int slices_parts(float* parts, const void* x, const void* w, int M, int N
   if (!x || !w || !parts || (((uintptr_t)x | (uintptr_t)w | (uintptr_t)parts) & 15)) return TS_BAD_SHAPE;
   if ((int64_t)M * N >= (1ll << 40) || 256 * ldx * 2 >= (1ll << 31) || 256 * ldw * 2 >= (1ll << 31)) return TS_TOO_LARGE;      // (byte offsets from a tile's start)
   const SlicesArgs a = {parts, (const bf16_t*)x, (const bf16_t*)w, M, N, K / 64, slices, 0, 0, 0, 0, ldx, ldw};
+  auto narrow = [&](int bm) {
+    const int64_t rows = (int64_t)((M + bm - 1) / bm) * slices;
+    return tiles_go_narrow(rows * ((N + 255) / 256), rows * ((N + 191) / 192), bm);
+  };
   switch (tile) {
     case 0: return launch_slices<128, 128, 2, 2, 2>(a, stream);
-    case 1: return launch_slices<128, 256, 2, 4, 2>(a, stream);
-    case 2: return launch_slices<192, 256, 2, 4, 2>(a, stream);
-    case 3: return launch_slices<256, 256, 2, 4, 2>(a, stream);
+    case 1: return narrow(128) ? launch_slices<128, 192, 4, 2, 2>(a, stream) : launch_slices<128, 256, 2, 4, 2>(a, stream);
+    case 2: return narrow(192) ? launch_slices<192, 192, 4, 2, 2>(a, stream) : launch_slices<192, 256, 2, 4, 2>(a, stream);
+    case 3: return narrow(256) ? launch_slices<256, 192, 4, 2, 2>(a, stream) : launch_slices<256, 256, 2, 4, 2>(a, stream);
     default: return launch_slices<64, 128, 1, 4, 3>(a, stream);
   }
 }
@@ -171,7 +175,8 @@ template <bool WIDE> static int slices_finish(void* y, const void* parts, int64_
 
 // x [M, K] and w [N, K] bfloat16, 16-byte aligned, rows ldx and ldw elements apart (multiples of 8); K a multiple of 64 with at
 // least 3 steps of 64 a slice, N a multiple of 8. parts: float32 [slices][M][N], scratch that the call fills and reads. tile (rows of x by
-// rows of W of a workgroup): 0 128 x 128, 1 128 x 256, 2 192 x 256, 3 256 x 256, 4 64 x 128. y [M, N] contiguous, 32-bit or bfloat16; or, with
+// rows of W of a workgroup): 0 128 x 128, 1 128 x 256, 2 192 x 256, 3 256 x 256, 4 64 x 128; 192 columns
+// for 256 by `tiles_go_narrow`. y [M, N] contiguous, 32-bit or bfloat16; or, with
 // norm_w [N]: y the norm of (the product in bfloat16 plus res [M, N], which may be null), sum [M, N] that sum; N at most 8,192. One slice without
 // a norm needs no parts (null): its workgroups store y themselves (gemm_whole.hip).
 extern "C" int ts_gemm_slices_bf16(void* y, void* sum, void* parts, const void* x, const void* w, int M, int N, int K, int64_t ldx, int64_t ldw,

@@ -13,7 +13,6 @@
 // small results, which it splits (600 x 64 over 2,048: 1.3e-7, one chain 2.7e-7). A tile of so many chains begins as many times, and the launch begins with
 // these: 3,072, 2,048 four times, 64 and 32 columns over 2,048, the last two in chains, 320 rows 26.6 µs, with the two by the library 41.2, all in one chain each 25.3.
 #define GW_CHAINS 4
-#define GW_COMPUTE_UNITS 256
 
 struct WholeProduct {
   const bf16_t *x, *w;
@@ -109,6 +108,13 @@ static int launch_whole(WholeArgs a, bool wide, hipStream_t stream) {
   return ts_check_launch();
 }
 
+static bool narrow(const WholeArgs& a, int bm) {
+  int64_t wide = 0, narrow = 0;
+  for (int i = 0; i < a.products; ++i) wide += (a.p[i].N + 255) / 256, narrow += (a.p[i].N + 191) / 192;
+  const int64_t rows = (a.M + bm - 1) / bm;
+  return tiles_go_narrow(rows * wide, rows * narrow, bm);
+}
+
 static bool whole_operands_ok(const void* x, const void* w, int K, int64_t ldx, int64_t ldw) {
   return x && w && !(((uintptr_t)x | (uintptr_t)w) & 15) && K > 0 && K % 64 == 0 && K / 64 >= TileProduct<64, 128, 1, 4, 3>::MIN_STEPS && ldx >= K && ldw >= K &&
          ldx % 8 == 0 && ldw % 8 == 0;
@@ -116,7 +122,7 @@ static bool whole_operands_ok(const void* x, const void* w, int K, int64_t ldx, 
 
 // `products` of them in one launch (1 to 8), all of M rows and the reduction K: x[i] [M, K] and w[i] [N[i], K] bfloat16, 16-byte aligned, rows
 // ldx and ldw elements apart (multiples of 8), y[i] [M, N[i]] contiguous, 16-byte aligned, 32-bit or bfloat16; K a multiple of 64 of at least 3, N[i] of
-// 8. tile (rows of x by rows of W of a workgroup): 0 128 x 128, 1 128 x 256, 2 192 x 256, 3 256 x 256, 4 64 x 128. chained: a bit for each product whose
+// 8. tile (rows of x by rows of W of a workgroup): 0 128 x 128, 1 128 x 256, 2 192 x 256, 3 256 x 256, 4 64 x 128; 192 columns for 256 by `tiles_go_narrow`. chained: a bit for each product whose
 // reduction is cut into GW_CHAINS chains (32-bit, K of 64 times 3 a chain).
 extern "C" int ts_gemm_whole_bf16(int products, void* const* y, const void* const* x, const void* const* w, const int* N, int M, int K, int64_t ldx,
                                   int64_t ldw, int tile, int chained, int out_f32, hipStream_t stream) {
@@ -134,9 +140,9 @@ extern "C" int ts_gemm_whole_bf16(int products, void* const* y, const void* cons
   if (256 * ldx * 2 >= (1ll << 31) || 256 * ldw * 2 >= (1ll << 31)) return TS_TOO_LARGE;      // (byte offsets from a tile's start)
   switch (tile) {
     case 0: return launch_whole<128, 128, 2, 2, 2>(a, out_f32, stream);
-    case 1: return launch_whole<128, 256, 2, 4, 2>(a, out_f32, stream);
-    case 2: return launch_whole<192, 256, 2, 4, 2>(a, out_f32, stream);
-    case 3: return launch_whole<256, 256, 2, 4, 2>(a, out_f32, stream);
+    case 1: return narrow(a, 128) ? launch_whole<128, 192, 4, 2, 2>(a, out_f32, stream) : launch_whole<128, 256, 2, 4, 2>(a, out_f32, stream);
+    case 2: return narrow(a, 192) ? launch_whole<192, 192, 4, 2, 2>(a, out_f32, stream) : launch_whole<192, 256, 2, 4, 2>(a, out_f32, stream);
+    case 3: return narrow(a, 256) ? launch_whole<256, 192, 4, 2, 2>(a, out_f32, stream) : launch_whole<256, 256, 2, 4, 2>(a, out_f32, stream);
     default: return launch_whole<64, 128, 1, 4, 3>(a, out_f32, stream);
   }
 }
@@ -340,7 +346,7 @@ extern "C" int ts_gemm_whole_rope_bf16(void* q_out, const void* x, const void* w
   switch (tile) {
     case 0: return launch_whole_rope<128, 128, 2, 2, 2>(a, stream);
     case 1:
-      if ((int64_t)((M + 127) / 128) * ((N + 191) / 192) <= GW_COMPUTE_UNITS) return launch_whole_rope<128, 192, 4, 2, 2, 1>(a, stream);
+      if ((int64_t)((M + 127) / 128) * ((N + 191) / 192) <= COMPUTE_UNITS) return launch_whole_rope<128, 192, 4, 2, 2, 1>(a, stream);
       return launch_whole_rope<128, 256, 2, 4, 2>(a, stream);
     case 2: return launch_whole_rope<192, 256, 2, 4, 2>(a, stream);
     default: return launch_whole_rope<64, 128, 2, 2, 3>(a, stream);

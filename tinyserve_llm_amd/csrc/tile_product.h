@@ -7,6 +7,19 @@
 #pragma once
 #include "lds_loads.h"
 
+#define COMPUTE_UNITS 256
+
+// Whether tiles of `bm` rows (128, 192 or 256) are 192 columns wide instead of 256: where the chip, which holds one a compute unit, takes as many rounds for them. A step
+// costs what its products do and a third of a microsecond, and a tile's sums are the same bits. us by 256 and by 192 columns: whole, 32-bit, over 2,048, 256 rows, 1,000 x
+// 11,296 (180 and 236 tiles) 54.0 and 46.2, 2,048 x 10,304 (328 and 432) 103 and 90; 192 rows, 768 x 10,304 (164 and 216) 42.8 and 36.7, 1,792 x 9,280 (370 and 490)
+// 85.6 and 73.6; 128 rows, 1,000 x 6,144 (192 and 256) 33.6 and 30.7, but in one round only (1,200 x 8,192, 320 and 430, 55.5 and 56.4). A round more: 1,024 x
+// 12,352 (196 and 260) 54.7 and 77.4. In two slices with the norm, 192 rows, 1,514 x 3,072 over 8,192 (192 and 256) 86.6 and
+// 84.1, over 3,072 51.5 and 46.4; 256 rows, 2,048 x 3,072 over 8,192 (192 and 256) 106.0 and 101.6. (224 columns in tiles of 256 rows: 54.2 where 256 take 54.0.)
+static inline bool tiles_go_narrow(int64_t wide, int64_t narrow, int bm) {
+  const int64_t rounds = (wide + COMPUTE_UNITS - 1) / COMPUTE_UNITS;
+  return narrow <= rounds * COMPUTE_UNITS && (bm > 128 || rounds == 1);
+}
+
 template <int BM, int BN, int WM, int WN, int XN> struct TileProduct {
   static constexpr int WAVES = WM * WN, TM = BM / WM / 16, TN = BN / WN / 16;
   static constexpr int NX = BM / 8 / WAVES, NW = BN / 8 / WAVES;      // kilobytes of a step that a wave fetches

@@ -52,3 +52,26 @@ def test_one_launch_has_the_bits_of_two(rt, waves, chunk, dwaves, lead, page, he
         more["gate"] = more["gate"][:lead]
     hip.paged_attention_decode(q[:lead], k, v, tables, seq[:lead], pos[:lead], dim ** -0.5, window, chunk, dwaves, two[:lead], **more)
     assert torch.equal(one, two)
+
+
+@pytest.mark.parametrize("splits", [1, 2, 7, 8, 9, 16, 17, 70])
+@pytest.mark.parametrize("heads,dim", [(3, 64), (2, 96), (5, 128), (2, 32)])
+@pytest.mark.parametrize("window", [0, 40, -64])
+def test_chunks_are_combined_whatever_the_ones_without_a_visible_key_hold(splits, heads, dim, window):
+    """Against 64 bits: a bfloat16 rounding (2^-8 with room for the 32-bit sums' own error, which is splits + 3 roundings of 2^-22 of the terms' sizes)."""
+    g, chunk = torch.Generator().manual_seed(100 * splits + dim), 32
+    positions = [0, 31, 32, splits * chunk // 2, splits * chunk - 1, splits * chunk - 33]
+    positions = torch.tensor([min(max(p, 0), splits * chunk - 1) for p in positions], dtype=I32)
+    tokens = len(positions)
+    o, ml = torch.randn(tokens, heads, splits, dim, generator=g), torch.rand(tokens, heads, splits, 2, generator=g) * 3 + 0.1
+    want, size = torch.empty(tokens, heads, dim, dtype=torch.float64), torch.empty(tokens, heads, dim, dtype=torch.float64)
+    for t, p in enumerate(positions.tolist()):
+        first = max(p - window + 1, 0) if window > 0 else p // -window * -window if window else 0
+        seen = slice(first // chunk, p // chunk + 1)
+        w = torch.exp2(ml[t, :, seen, 0].double())
+        total = (ml[t, :, seen, 1].double() * w).sum(1)[:, None]
+        want[t], size[t] = (o[t, :, seen].double() * w[..., None]).sum(1) / total, (o[t, :, seen].double().abs() * w[..., None]).sum(1) / total
+        hidden = [s for s in range(splits) if not seen.start <= s < seen.stop]
+        o[t, :, hidden], ml[t, :, hidden] = float("nan"), float("nan")
+    got = hip.SplitAttention(o.cuda(), ml.cuda(), positions.cuda(), chunk, window).combined().view(tokens, heads, dim).cpu().double()
+    assert bool(((got - want).abs() <= 2.0 ** -8 * want.abs() + (splits + 3) * 2.0 ** -22 * size).all())

@@ -158,12 +158,13 @@ def linear(x: "torch.Tensor | DeferredNorm | hip.PackedRows8 | hip.SplitAttentio
     still in its chunks' parts): the 8-row form adds the parts up on its way in where it can, the combining
     kernel does otherwise."""
     if type(x) is torch.Tensor and then is not None and packed is not None and packed.by16 is not None and out_dtype is None and not glu and x.dim() == 2:
-        # the commonest way of a step of a few dozen rows, whose conditions the module looks at itself (with the module's ways into the cache and into
-        # the norm of up to 32 rows a prompt over 12 layers, which the host bounds: 32 tokens 1118 -> 733 µs, 48 947 -> 719; 90, the kernels' 828, 856 -> 828)
+        # the commonest way of a step of a few dozen rows (with the module's ways into the cache and into the norm of up to 32 rows a prompt over 12
+        # layers, which the host bounds: 32 tokens 1118 -> 733 µs, 48 947 -> 719; 90, the kernels' 828, 856 -> 828)
         slices = hip._sliced_route(x.shape[0], *weight.shape) if x.is_cuda and weight.dtype == torch.bfloat16 and weight.is_contiguous() else 0
-        done = hip._native().gemm_rows64_sliced(x, packed.by16, slices, then.residual(), then.weight) if slices else None
-        if done is not None:
-            return DeferredNorm(None, None, then.weight, then.eps, hip.PreparedNorm(*done))
+        residual = then.residual() if slices else None
+        if (slices and x.dtype == torch.bfloat16 and hip._dense_rows(x) and x.data_ptr() % 16 == 0 and then.weight.dtype == torch.bfloat16
+                and (residual is None or (residual.is_contiguous() and residual.dtype == torch.bfloat16))):
+            return DeferredNorm(None, None, then.weight, then.eps, hip.gemm_rows64_sliced(x, packed.by16, slices, next_norm=(residual, then.weight)))
     if isinstance(x, hip.SplitAttention):
         residual = then.residual() if then is not None else None
         if (not glu and out_dtype in (None, torch.bfloat16) and hip.split_attention_fuses(x.shape[0], weight)

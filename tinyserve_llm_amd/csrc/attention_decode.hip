@@ -13,6 +13,7 @@
 // normalises and writes the output itself. Otherwise a chunk's unnormalised output with its running
 // max and sum goes to a 32-bit workspace, and a second kernel combines the chunks of a token in
 // ascending order. Chunk boundaries are multiples of the chunk size counted from position 0.
+// (The chunk's walk is attention_decode.h's, which a step with prompts beside the decoding tokens takes too: attn_step_kernel in attention_prefill.hip.)
 #include "attention_decode.h"
 
 template <int HD, bool ONE, bool GENERAL, bool ONCE>

@@ -6,7 +6,7 @@
 // what is gained is the trip of the product through memory and the launch that read it again. Measured with the weights
 // coming from memory, against the library's product followed by the unit's kernel: 2,048 rows 120 µs against 134 (bfloat16
 // product) and 171 (32-bit product: 125 with relu, 135 with the sigmoid), 999 rows 63 against 71, 512 rows 36 against 46,
-// 160 rows 24 against 31 (which hip.glu_pays leaves to the product all the same).
+// 160 rows 24 against 31.
 //
 // The tile is the one whose rounds of one workgroup a compute unit cost least (hip.glu_plan): a round of 256 x 256 is the chip's best
 // rate, and other heights fill the last round where that one would not. F 8,192, weights from memory, in tiles of 256, 192 and

@@ -8,7 +8,7 @@
 //   * `ts_embedding_dyt_stream`: token rows of the table times a scale, through a norm, into the stream.
 // alpha, w and b are 32-bit; alpha is read from device memory, so a recorded step needs no host value.
 // The hyperbolic tangent is taken as 1 - 2 / (exp(2 z) + 1) with the 32-bit library exponential.
-#include "glu_unit.h"
+#include "common.h"
 
 #define DT_THREADS 256
 
@@ -164,12 +164,16 @@ extern "C" int ts_embedding_dyt_stream(float* out, const void* table, int dtype,
   return ts_check_launch();
 }
 
-// What the gate passes: 0 g sigmoid(slope g), 1 relu, 2 gelu in its tanh form, 3 as 0 by the library's exponential.
-static __device__ __forceinline__ float dt_gate(float g, float slope, int act) { return glu_gate(act + GLU_SIGMOID, g, slope); }
+// What the gate passes: 0 g sigmoid(slope g), 1 relu, 2 gelu in its tanh form.
+static __device__ __forceinline__ float dt_gate(float g, float slope, int act) {
+  if (act == 1) return fmaxf(g, 0.f);
+  if (act == 2) return 0.5f * g * (1.0f + tanhf(0.7978845608028654f * (g + 0.044715f * g * g * g)));
+  return g / (1.0f + expf(-slope * g));
+}
 
 // The capped gated unit between the two projections of a feed-forward: from a row [gate | up] of 32-bit (or
 // stored) sums, g = min(gate, limit), u = clamp(up, -limit, limit), y = act(g) (u + up_shift) with act(g) = g sigmoid(slope g) (act 0),
-// max(g, 0) (1), gelu in its tanh form (2) or as 0 by the library's exponential (3). limit <= 0: no cap. Rows may be picked through `row_stride` (a row of the operand may be wider than 2 ff).
+// max(g, 0) (1) or gelu in its tanh form (2). limit <= 0: no cap. Rows may be picked through `row_stride` (a row of the operand may be wider than 2 ff).
 __global__ void __launch_bounds__(DT_THREADS)
 capped_glu_kernel(void* __restrict__ out, int out_code, const void* __restrict__ gate_up, int in_code, int64_t row_stride,
                   int ff, float limit, float slope, float up_shift, int64_t total, int act) {
@@ -212,7 +216,7 @@ capped_glu_fours_kernel(TO* __restrict__ out, const float* __restrict__ gate_up,
 extern "C" int ts_capped_glu(void* out, int out_dtype, const void* gate_up, int in_dtype, int64_t row_stride, int n, int ff,
                              float limit, float slope, float up_shift, int act, hipStream_t stream) {
   if (n <= 0) return TS_OK;
-  if (ff <= 0 || row_stride < 2 * (int64_t)ff || act < 0 || act > GLU_SIGMOID_LIBRARY - GLU_SIGMOID) return TS_BAD_SHAPE;
+  if (ff <= 0 || row_stride < 2 * (int64_t)ff || act < 0 || act > 2) return TS_BAD_SHAPE;
   if ((out_dtype | in_dtype) & ~1) return TS_BAD_DTYPE;
   const int64_t total = (int64_t)n * ff;
   const int64_t blocks = (total + DT_THREADS - 1) / DT_THREADS;

@@ -212,7 +212,6 @@ static int launch_glu(GluArgs a, int act, hipStream_t stream) {
   switch (act) {
     case GLU_SILU_ROUNDED: gemm_glu_kernel<BM, BN, WM, WN, GLU_SILU_ROUNDED><<<grid, WM * WN * TS_WAVE, 0, stream>>>(a); break;
     case GLU_SIGMOID: gemm_glu_kernel<BM, BN, WM, WN, GLU_SIGMOID><<<grid, WM * WN * TS_WAVE, 0, stream>>>(a); break;
-    case GLU_SIGMOID_LIBRARY: gemm_glu_kernel<BM, BN, WM, WN, GLU_SIGMOID_LIBRARY><<<grid, WM * WN * TS_WAVE, 0, stream>>>(a); break;
     case GLU_RELU: gemm_glu_kernel<BM, BN, WM, WN, GLU_RELU><<<grid, WM * WN * TS_WAVE, 0, stream>>>(a); break;
     default: gemm_glu_kernel<BM, BN, WM, WN, GLU_GELU><<<grid, WM * WN * TS_WAVE, 0, stream>>>(a);
   }
@@ -222,11 +221,11 @@ static int launch_glu(GluArgs a, int act, hipStream_t stream) {
 // x [M, K], w [2 F, K], y [M, F] bfloat16, 16-byte aligned, rows ldx, ldw, ldy elements apart (multiples of 8); K a
 // multiple of 64, F of 8. tile: rows of x by rows of W of a workgroup, 0 256 x 256, 1 192 x 256, 2 128 x 128,
 // 3 128 x 256. act: 0 silu(gate) up with both branches rounded to bfloat16 first (limit, slope and up_shift
-// unused); 1 to 4: the capped unit from the 32-bit sums with the gate through that form of glu_unit.h.
+// unused); 1, 2, 3: the capped unit from the 32-bit sums with the gate through a sigmoid of slope, relu or gelu's tanh form.
 extern "C" int ts_gemm_glu_bf16(void* y, const void* x, const void* w, int M, int F, int K, int64_t ldx, int64_t ldw, int64_t ldy,
                                 int tile, int act, float limit, float slope, float up_shift, hipStream_t stream) {
   if (M <= 0 || F <= 0) return TS_OK;
-  if (K <= 0 || K % 64 || F % 8 || ldx < K || ldw < K || ldy < F || ldx % 8 || ldw % 8 || ldy % 8 || act < 0 || act > GLU_SIGMOID_LIBRARY || tile < 0 || tile > 3) return TS_BAD_SHAPE;
+  if (K <= 0 || K % 64 || F % 8 || ldx < K || ldw < K || ldy < F || ldx % 8 || ldw % 8 || ldy % 8 || act < 0 || act > 3 || tile < 0 || tile > 3) return TS_BAD_SHAPE;
   if (((uintptr_t)x | (uintptr_t)w | (uintptr_t)y) & 15) return TS_BAD_SHAPE;
   if (!x || !w || !y || 2 * (int64_t)F * ldw * 2 >= (1ll << 31) || 256 * ldx * 2 >= (1ll << 31)) return TS_TOO_LARGE;   // (byte offsets from a tile's start)
   const GluArgs a = {(bf16_t*)y, (const bf16_t*)x, (const bf16_t*)w, M, F, K, 0, 0, 0, ldx, ldw, ldy, limit, slope, up_shift};

@@ -404,7 +404,6 @@ extern "C" int ts_gemm_rows64_bf16(void* y, const void* x, const void* w16, int 
     case 1 + GLU_SIGMOID: return r64_launch<1 + GLU_SIGMOID, bf16_t>(a, stream);
     case 1 + GLU_RELU: return r64_launch<1 + GLU_RELU, bf16_t>(a, stream);
     case 1 + GLU_GELU: return r64_launch<1 + GLU_GELU, bf16_t>(a, stream);
-    case 1 + GLU_SIGMOID_LIBRARY: return r64_launch<1 + GLU_SIGMOID_LIBRARY, bf16_t>(a, stream);
   }
   return TS_BAD_SHAPE;
 }

@@ -1173,7 +1173,7 @@ extern "C" int ts_gemm_skinny_bf16(void* y, const void* x, const void* w, const 
     if (mode == MODE_PLAIN) return sk_dispatch<MODE_PLAIN, EPI_NEXT, bf16_t>(a, stream);
     return sk_dispatch<MODE_PREP, EPI_NEXT, bf16_t>(a, stream);
   }
-  if (!y || ldy < (glu ? N / 2 : N) || glu < 0 || glu > 1 + GLU_SIGMOID_LIBRARY) return TS_BAD_SHAPE;
+  if (!y || ldy < (glu ? N / 2 : N) || glu < 0 || glu > 1 + GLU_GELU) return TS_BAD_SHAPE;
   if (glu > 1) {
     if (out_dtype != 1 || mode != MODE_PLAIN) return TS_BAD_DTYPE;
     a.nh = glu - 1, a.nkv = __builtin_bit_cast(int, limit), a.hd = __builtin_bit_cast(int, slope), a.rotate = __builtin_bit_cast(int, up_shift);

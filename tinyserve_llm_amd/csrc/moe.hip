@@ -22,7 +22,6 @@
 //     has no matrices, `ts_moe_group` leaves its pairs out of every tile, and its row is the token's input itself.
 // float32 runs 32-bit multiply-adds; bfloat16 operands go through the matrix cores with 32-bit sums.
 #include <type_traits>
-#include "glu_unit.h"
 #include "lds_loads.h"
 
 #define MOE_THREADS 256
@@ -294,7 +293,13 @@ static __device__ __forceinline__ float moe_act(float s, int act) {
   return s;
 }
 
-static __device__ __forceinline__ float moe_unit(float g, float u, float limit, float slope, float shift) { return glu_capped(GLU_SIGMOID_LIBRARY, g, u, limit, slope, shift); }
+static __device__ __forceinline__ float moe_unit(float g, float u, float limit, float slope, float shift) {
+  if (limit > 0.f) {
+    g = fminf(g, limit);
+    u = fminf(fmaxf(u, -limit), limit);
+  }
+  return g / (1.0f + expf(-slope * g)) * (u + shift);
+}
 
 // Plain 32-bit multiply-adds: a tile of up to 16 rows by 64 columns a workgroup; thread (column, row quarter).
 template <typename TX, typename TO>

@@ -1688,7 +1688,7 @@ def gemm_tiled(x: torch.Tensor, weight: torch.Tensor, glu: bool = False,
     return y
 
 
-GLU_FORMS = {"silu_rounded": 0, "sigmoid": 1, "relu": 2, "gelu_tanh": 3, "sigmoid_library": 4}
+GLU_FORMS = {"silu_rounded": 0, "sigmoid": 1, "relu": 2, "gelu_tanh": 3}
 
 
 def glu_takes(x: torch.Tensor, weight: torch.Tensor) -> bool:
@@ -2857,7 +2857,7 @@ def embedding_dyt_stream(table: torch.Tensor, ids: torch.Tensor, scale: float = 
     return out
 
 
-GLU_ACTIVATIONS = {"sigmoid": 0, "relu": 1, "gelu_tanh": 2, "sigmoid_library": 3}      # (the last for what comes between routers)
+GLU_ACTIVATIONS = {"sigmoid": 0, "relu": 1, "gelu_tanh": 2}
 
 
 def capped_glu(gate_up: torch.Tensor, limit: float, slope: float, up_shift: float, out_dtype: torch.dtype,

@@ -99,9 +99,8 @@ class CappedGLU(FeedForward):
 
     def __init__(self, hidden_size: int, intermediate_size: int, limit: float = 0.0, slope: float = 1.702,
                  up_shift: float = 1.0, activation: str = "sigmoid") -> None:
-        known = [name for name in hip.GLU_ACTIVATIONS if name != "sigmoid_library"]
-        if activation not in known:
-            raise ValueError(f"activation {activation!r}: one of {sorted(known)} ('sigmoid': g sigmoid(slope g))")
+        if activation not in hip.GLU_ACTIVATIONS:
+            raise ValueError(f"activation {activation!r}: one of {sorted(hip.GLU_ACTIVATIONS)} ('sigmoid': g sigmoid(slope g))")
         self.activation = activation
         self.hidden_size, self.intermediate_size = hidden_size, intermediate_size
         self.limit, self.slope, self.up_shift = limit, slope, up_shift

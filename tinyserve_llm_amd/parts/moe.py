@@ -51,8 +51,6 @@ class RoutedExperts(FeedForward):
         self.limit, self.slope, self.up_shift = limit, slope, up_shift
         self.router_scale, self.normalize, self.has_correction = router_scale, normalize, correction
         self.shared = CappedGLU(hidden_size=hidden_size, **shared) if shared is not None else None
-        if self.shared is not None and self.shared.activation == "sigmoid":
-            self.shared.activation = "sigmoid_library"      # (the experts' own: what a next router reads keeps its last bits)
         self.router: torch.Tensor | None = None
         self.correction: torch.Tensor | None = None
         self.gate_up: torch.Tensor | None = None

@@ -2,10 +2,13 @@
 
 from __future__ import annotations
 
+from types import SimpleNamespace
+
 import pytest
 import torch
 
 from tinyserve_llm_amd.ops import hip
+from tinyserve_llm_amd.parts.gated_delta import GatedDelta
 from tinyserve_llm_amd.parts.norm import RMSNorm
 from tinyserve_llm_amd.parts.stream import ResidualStream
 
@@ -65,19 +68,19 @@ def test_a_product_in_slices_leaves_its_parts(rows, n, k):
     assert hip.linear_parts(x[:, ::2], w[:, : k // 2]) is None      # (rows that are not dense)
 
 
-@pytest.mark.parametrize("rows,n,k,taken", [(300, 2048, 4096, True), (999, 2048, 4096, True), (1000, 1024, 4096, True), (700, 2048, 4096, False), (999, 2048, 2048, False),
-                                            (128, 2048, 4096, False), (2048, 2048, 8192, True)])
-def test_a_product_leaves_parts_sooner_for_a_norm_that_adds_them(rows, n, k, taken):
-    """Against 64 bits: chains of at most k numbers, their bfloat16 products exact in 32 bits, and no further from it than the product made whole."""
+@pytest.mark.parametrize("rows", [300, 999, 1280, 2048])
+def test_a_part_that_leaves_parts_leaves_those_of_its_own_rows(rows, monkeypatch):
+    """The delta rule's output projection (4,096 into 2,048): in parts only where the product made whole is in the same slices, so the bits are those of its rows."""
     g = torch.Generator(device="cuda").manual_seed(rows)
-    x, w = torch.randn(rows, k, generator=g, device="cuda").to(BF), torch.randn(n, k, generator=g, device="cuda").to(BF)
-    parts = hip.linear_parts(x, w, sooner=True)
-    assert (parts is not None) == taken
-    if taken:
-        want, size = x.double() @ w.double().t(), x.double().abs() @ w.double().abs().t()
-        off = (parts.rows().double() - want).abs()
-        assert bool((off <= k * 2.0 ** -24 * size).all())
-        assert float(off.norm()) <= 1.1 * float((hip.linear_bf16(x, w, F32).double() - want).norm())
+    mixer = GatedDelta(hidden_size=2048, num_heads=32, groups=16, head_dim=128, value_dim=128, conv_taps=4, norm_eps=1e-5)
+    mixer.proj = torch.randn(64, 2048, generator=g, device="cuda").to(BF)
+    mixer.o = torch.randn(2048, 4096, generator=g, device="cuda").to(BF)
+    gated = torch.randn(rows, 4096, generator=g, device="cuda").to(BF)
+    for name, made in (("delta_prepare", None), ("delta_scan", None), ("mlstm_finish", gated)):
+        monkeypatch.setattr(hip, name, lambda *args, _made=made, **options: _made)
+    memory = SimpleNamespace(state=None)
+    x = torch.randn(rows, 2048, generator=g, device="cuda").to(BF)
+    assert torch.equal(hip.added_up(mixer.forward(x, None, memory, parts=True)), mixer.forward(x, None, memory))
 
 
 @pytest.mark.parametrize("top,identity,shared", [(1, False, None), (2, True, "gated"), (4, True, "plain"), (4, False, "gated"), (5, True, None), (9, True, "plain")])

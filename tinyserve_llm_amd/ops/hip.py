@@ -1771,7 +1771,6 @@ SLICES_LIBRARY = {"bf16": (4.7, 0.33, 1.24, 1.16, 0.55, 0.10), "f32": (3.9, 0.29
 # the share of the library's time, both as estimated, up to which the slices are taken: two of them in each tile, and more
 SLICES_TWO_SHARE, SLICES_SHARE = (0.95, 0.92, 0.91, 0.80, 0.80), 0.94
 SLICES_NORM_FEW_ROWS, SLICES_NORM_FEW_SHARE = 256, 1.02      # the same of more than two slices with the norm, up to so many rows
-SLICES_PARTS_SHARE, SLICES_PARTS_MIN_K = 1.09, 3072          # the same where a norm's kernel adds the parts up (`parts_plan`)
 SLICES_MIN_ROWS, SLICES_MAX_ROWS = 129, 2048       # fewer rows: the kernels that share x; more: whole reductions fill the chip
 SLICES_MIN_WIDTH, SLICES_MAX_WIDTH = 1024, 4096    # columns (wider: whole reductions fill the chip as well)
 SLICES_MAX, SLICES_MIN_STEPS = 16, 3               # slices, and steps of 64 in each
@@ -1793,27 +1792,6 @@ def slices_plan(rows: int, n: int, k: int, ending: str) -> tuple[int, int] | Non
     on the host takes 6 less than the library's and the norm's.
     n 2,048, library and here: k 8,192 160 rows 26.6 and 19.2, 512 rows 34.1 and 29.9, 1,024 rows 53.4 and 44.7, with the norm 1,514
     rows 66.5 and 61.9; k 4,096 with the norm 300 rows 25.2 and 20.4, 2,048 rows 50.0 and 49.9; k 2,048 160 rows 9.6 and 11.3."""
-    found = _slices_estimate(rows, n, k, ending)
-    if found is None:
-        return None
-    us, tile, slices, library = found
-    share = SLICES_TWO_SHARE[tile] if slices == 2 else SLICES_NORM_FEW_SHARE if ending == "norm" and rows <= SLICES_NORM_FEW_ROWS else SLICES_SHARE
-    return (tile, slices) if us < share * library else None
-
-
-@functools.lru_cache(maxsize=4096)
-def parts_plan(rows: int, n: int, k: int) -> tuple[int, int] | None:
-    """The same of a 32-bit product whose parts a norm's kernel adds up on its way into the stream (`linear_parts`): no kernel of their own does, and so
-    slices are taken up to SLICES_PARTS_SHARE of the library's estimate, over reductions from SLICES_PARTS_MIN_K on. Product and norm, whole and in parts, us: n
-    2,048, k 4,096 300 rows 26.5 and 20.5, 999 rows 39.1 and 32.7, 1,280 rows 43.5 and 38.5, 1,500 rows 46.2 and 45.0, 2,048 rows 56.0 and 51.9, but (left) 513 rows
-    28.8 and 24.6, 700 rows 30.3 and 32.2; n 3,072, k 3,072 300 rows 24.5 and 22.6, 1,280 rows 46.8 and 44.8, (left) 2,048 rows 60.7 and 65.0; k 2,048 (left) 999 rows
-    21.5 and 23.7."""
-    found = _slices_estimate(rows, n, k, "f32") if k >= SLICES_PARTS_MIN_K else None
-    return found[1:3] if found is not None and found[0] < SLICES_PARTS_SHARE * found[3] else None
-
-
-def _slices_estimate(rows: int, n: int, k: int, ending: str) -> tuple[float, int, int, float] | None:
-    """(us of the fastest slices as estimated, their tile, their number, us of the library); None out of the sizes' range."""
     if not SLICES_MIN_ROWS <= rows <= SLICES_MAX_ROWS or not SLICES_MIN_WIDTH <= n <= SLICES_MAX_WIDTH or n % 8 or k % 64 or k < 2048:
         return None
     steps, best = k // 64, None
@@ -1826,8 +1804,11 @@ def _slices_estimate(rows: int, n: int, k: int, ending: str) -> tuple[float, int
                 best = (us, tile, slices)
     if best is None:
         return None
+    us, tile, slices = best
     fixed, chain, rooted, work, weight, out = SLICES_LIBRARY[ending]
-    return *best, fixed + (chain + rooted * math.sqrt(rows) / 32) * k / 1024 + (work * rows * n * k * 1e-3 + weight * n * k + out * rows * n) * 1e-6
+    library = fixed + (chain + rooted * math.sqrt(rows) / 32) * k / 1024 + (work * rows * n * k * 1e-3 + weight * n * k + out * rows * n) * 1e-6
+    share = SLICES_TWO_SHARE[tile] if slices == 2 else SLICES_NORM_FEW_SHARE if ending == "norm" and rows <= SLICES_NORM_FEW_ROWS else SLICES_SHARE
+    return (tile, slices) if us < share * library else None
 
 
 def slices_takes(x: torch.Tensor, weight: torch.Tensor) -> bool:
@@ -2375,17 +2356,14 @@ def capped_product(x: torch.Tensor, weight: torch.Tensor, packed: StreamingCopie
     return None
 
 
-def linear_parts(x: torch.Tensor, weight: torch.Tensor, packed: StreamingCopies | None = None, sooner: bool = False) -> RowParts | None:
-    """float32 x · weight^T left in its slices' parts, where `linear_bf16` would give the product to the slices and add the parts up, or, with `sooner`
-    (for a caller whose rows a norm's kernel takes, and whose sums may come in shorter chains), where parts are the faster way then; None where not."""
+def linear_parts(x: torch.Tensor, weight: torch.Tensor, packed: StreamingCopies | None = None) -> RowParts | None:
+    """float32 x · weight^T left in its slices' parts, where `linear_bf16` would give the product to the slices and add the parts up; None where not."""
     if not isinstance(x, torch.Tensor) or _many_rows != "library" or _library_tuning is not None or x.dim() != 2 or weight.shape[0] > STREAM_PARTS_MAX_WIDTH:
         return None
     rows, k = x.shape
     if not _library_serves(rows, weight.shape[0], k, packed is not None and packed.by16 is not None, True):
         return None
     plan = many_rows_plan(rows, weight.shape[0], k, "f32")
-    if sooner and (plan is None or plan[1] < 2):
-        plan = parts_plan(rows, weight.shape[0], k)
     if plan is None or plan[1] < 2:
         return None
     parts = _native().gemm_slices(x, weight, *plan, True)

@@ -73,5 +73,5 @@ class GatedDelta(Mixer):
         rows = hip.delta_prepare(proj, self._conv, self.dt_bias, self.a_log, mem.state, ctx, z, x.dtype)
         o = hip.delta_scan(rows, mem.state, ctx, z)
         gated = hip.mlstm_finish(o, self.norm, proj[:, :z.inner], z.heads, z.vdim, self.norm_eps, x.dtype, silu_gate=True)
-        out = hip.linear_parts(gated, self.o, self.o_packed, sooner=True) if parts else None
+        out = hip.linear_parts(gated, self.o, self.o_packed) if parts else None
         return out if out is not None else linear(gated, self.o, out_dtype=torch.float32, packed=self.o_packed)

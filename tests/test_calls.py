@@ -214,3 +214,43 @@ def test_calls_of_few_rows_reach_the_kernels_that_stream_the_copies(stub):
         answer(launcher, BAD_SHAPE)
         assert call(*plain) is None and called()[-1] == launcher
         answer(launcher, OK)
+
+
+def test_the_general_functions_of_few_rows_take_what_they_say(stub, monkeypatch):
+    """What the module's forms that share a name would take of another function's operands, or without a look at the weight that a copy is of."""
+    module, _, called = stub
+    monkeypatch.setattr(hip, "_native", lambda: module)
+    x, w, w512, p16, p16q, p8 = bf(3, 1024), bf(64, 1024), bf(512, 1024), bf(4, 32, 64, 8), bf(32, 32, 64, 8), bf(8, 4, 4, 64, 8)
+    rope = (torch.zeros(9, 64), ints(0, 1, 2), ints(0, 1, 2), *caches(), 4, 2, 64)
+    away = lambda t: torch.empty_like(t, device="meta")
+    into = dict(packed=p16, next_norm=(None, bf(64)))
+    for good, launcher in ((lambda: hip.gemm_rows64(x, p16), "ts_gemm_rows64_bf16"), (lambda: hip.gemm_rows64_sliced(x, p16, 2), "ts_gemm_rows64_sliced_bf16"),
+                           (lambda: hip.qkv_rope_store_sliced(x, p16q, 2, *rope), "ts_gemm_rows64_sliced_rope_bf16"),
+                           (lambda: hip.gemm_skinny8(x, w, BF, p8), "ts_gemm_skinny8_bf16"), (lambda: hip.gemm_skinny(x, w, **into), "ts_gemm_skinny_bf16"),
+                           (lambda: hip.qkv_rope_store(x, w512, *rope, packed=p16q), "ts_gemm_skinny_rope_bf16"),
+                           (lambda: hip.stream_update_norm(torch.zeros(3, 64), None, hip.RowParts(torch.zeros(2, 3, 64)), weights=(bf(64), None), out_dtype=BF), "ts_stream_update_norm_parts"),
+                           (lambda: hip.stream_post_norm(torch.zeros(3, 64), hip.RowParts(torch.zeros(2, 3, 64)), torch.zeros(64), None, 1e-6, out_dtype=BF), "ts_stream_post_norm_parts")):
+        good()
+        assert called()[-1] == launcher
+    for bad in (lambda: hip.gemm_rows64(x, p8), lambda: hip.gemm_rows32(x, p8), lambda: hip.gemm_rows64_sliced(x, p16, 0, next_norm=(None, bf(64))),
+                lambda: hip.qkv_rope_store_sliced(x, p16q, 0, *rope), lambda: hip.gemm_skinny8(x, away(w), BF, p8), lambda: hip.gemm_skinny8(x, bf(64), BF, p8),
+                lambda: hip.gemm_skinny(x, away(w), **into), lambda: hip.gemm_skinny(x, w, unit=("sigmoid", 0.0, 1.0, 0.0), **into),
+                lambda: hip.qkv_rope_store(x, away(w512), *rope, packed=p16q),
+                lambda: hip.stream_update_norm(torch.zeros(3, 64), None, (torch.zeros(2, 3, 64),), weights=(bf(64), None), out_dtype=BF),
+                lambda: hip.stream_post_norm(torch.zeros(3, 64), (torch.zeros(2, 3, 64),), torch.zeros(64), None, 1e-6, out_dtype=BF)):
+        with pytest.raises((hip.KernelError, AttributeError)):      # (a tuple is no tensor)
+            bad()
+        assert called() == []
+    plain = lambda copy: module.gemm_rows64(x, copy, True, 0, None, 0.0, 0.0, 0.0, 0.0)
+    assert plain(p8) is not None and called() == ["ts_gemm_skinny8_bf16"]
+    assert plain(bf(8, 2, 8, 64, 8)) is None and plain(bf(8, 1, 16, 64, 8)) is None and called() == []      # (copies for a reader of other steps)
+
+
+@pytest.mark.parametrize("k", [256, 512, 1024, 2048, 2304, 4096, 8192, 1024 * 16, 1024 * 17, 96, 5120])
+def test_the_steps_of_the_8_row_form_are_the_same_on_both_sides(stub, k):
+    module, _, called = stub
+    steps = hip.skinny8_steps(k)
+    for tried in (4, 8, 16):
+        taken = k % (64 * tried) == 0 and module.gemm_rows64(bf(1, k), bf(1, k // (64 * tried), tried, 64, 8), True, 0, None, 0.0, 0.0, 0.0, 0.0) is not None
+        assert taken == (tried == steps)
+    called()

@@ -436,10 +436,12 @@ PyObject* gemm_glu(Args a) {      // x, weight, tile, form's number, limit, slop
 
 bool squares_fit(const Tensor* s, int64_t rows) { return !s || (f32(*s) && s->dim() == 2 && s->size(0) == rows && s->size(1) >= 1 && s->is_contiguous()); }
 
-// What gemm_rows64 makes of up to 8 rows of x and the copy that the 8-row form reads (five-dimensional; its steps are those that the caller found for the reduction).
+// What gemm_rows64 makes of up to 8 rows of x and the copy that the 8-row form reads (five-dimensional: hip.pack_weight8).
 PyObject* rows8(const Tensor& x, const Tensor& p, bool wide, float cap) {
   const int64_t M = x.size(0), K = x.size(1), N = p.size(0) * 8;
-  if (M < 1 || M > 8 || !bf16(p) || p.size(1) * p.size(2) * 64 != K || p.size(3) != 64 || p.size(4) != 8 || !p.is_contiguous() || !fits(N) || !fits(K)) return none();
+  if (M < 1 || M > 8 || !fits(N) || !fits(K) || !bf16(p) || p.size(2) != ts_skinny8_steps(K) || p.size(1) * p.size(2) * 64 != K || p.size(3) != 64 || p.size(4) != 8 ||
+      !p.is_contiguous())
+    return none();
   Tensor y = make(x, {M, N}, wide ? at::kFloat : at::kBFloat16);
   if (TS_REFUSED("gemm_skinny8", ts_gemm_skinny8_bf16(ptr(&y), ptr(&x), ptr(&p), M, N, K, x.stride(0), K, N, wide ? 0 : 1, 1, nullptr, nullptr, nullptr, nullptr, nullptr,
                                                       0, nullptr, nullptr, nullptr, 0, 0, 0, 0, cap, stream())))

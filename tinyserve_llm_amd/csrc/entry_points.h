@@ -105,3 +105,11 @@ int ts_qkv_finish(void* q_out, void* k_cache, void* v_cache, const void* qkv, co
 int ts_mlstm_finish(void* out, int out_dtype, const float* o, const float* weight, const float* gate, int64_t gate_stride, int num_tokens,
                     int heads, int vdim, float eps, int weight_head, int silu_gate, hipStream_t stream);
 }
+
+// 32-wide steps of k that a wave of the 8-row form takes for a reduction of K (it covers 64 of k in each): the fewest that fit 8 waves, else 16 in up to
+// 16 waves; 0: it does not serve K.
+static inline int ts_skinny8_steps(int K) {
+  for (int steps : {4, 8, 16})
+    if (K % (64 * steps) == 0 && K / (64 * steps) <= 8) return steps;
+  return K % 1024 == 0 && K / 1024 <= 16 ? 16 : 0;
+}

@@ -1027,11 +1027,7 @@ gemm_skinny8_stay_kernel(const SkinnyArgs a) {
 
 template <typename OUT, bool NEXT = false>
 static int sk8_dispatch(const SkinnyArgs& a, hipStream_t stream) {
-  // a wave covers 64 STEPS of k; 8 waves where the reduction allows it, never more than 16
-  int steps = 0;
-  for (int cand : {4, 8, 16})
-    if (!steps && a.K % (64 * cand) == 0 && a.K / (64 * cand) <= 8) steps = cand;
-  if (!steps && a.K % 1024 == 0 && a.K / 1024 <= 16) steps = 16;
+  const int steps = ts_skinny8_steps(a.K);
   if (!steps) return TS_BAD_SHAPE;
   const int nwaves = a.K / (64 * steps);
   dim3 grid((a.N + 7) / 8), block(nwaves * TS_WAVE);

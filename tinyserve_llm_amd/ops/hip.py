@@ -1127,7 +1127,8 @@ def gemm_skinny8(x: "torch.Tensor | PackedRows8 | SplitAttention", weight: torch
     x_packed = isinstance(x, PackedRows8)
     split = x if isinstance(x, SplitAttention) else None
     xt = x.data if x_packed else x.parts if split is not None else x
-    if packed8 is not None and next_norm is None and xt is x and x.dim() == 2 and x.shape[0] <= SKINNY8_MAX_ROWS and out_dtype in (torch.bfloat16, torch.float32):
+    if (packed8 is not None and next_norm is None and xt is x and x.dim() == 2 and weight.dim() == 2 and weight.device == x.device
+            and x.shape[0] <= SKINNY8_MAX_ROWS and out_dtype in (torch.bfloat16, torch.float32)):
         n, k = weight.shape
         steps = skinny8_steps(k)
         if (steps and n % 8 == 0 and packed8.shape == (n // 8, k // (64 * steps), steps, 64, 8) and x.shape[1] == k and weight.dtype == torch.bfloat16
@@ -1243,8 +1244,8 @@ def gemm_skinny(x: torch.Tensor, weight: torch.Tensor, out_dtype: torch.dtype = 
     With `pack8_steps` (and `glu`, up to 8 rows) the gated product comes back as a `PackedRows8` for a
     reader of that many steps. `unit` (with `glu` and a plain x): (form, limit, slope, up_shift) of the unit of
     `capped_glu` in silu's place."""
-    if (next_norm is not None and packed is not None and norm_weight is None and residual is None and squares is None and not glu and out_dtype is torch.bfloat16
-            and next_norm[1] is not None and x.dim() == 2 and packed.dim() == 4 and weight.shape == (packed.shape[0] * 16, x.shape[1])
+    if (next_norm is not None and packed is not None and norm_weight is None and residual is None and squares is None and not glu and unit is None
+            and out_dtype is torch.bfloat16 and next_norm[1] is not None and x.dim() == 2 and packed.dim() == 4 and weight.device == x.device and weight.shape == (packed.shape[0] * 16, x.shape[1])
             and skinny_fuses(*x.shape, False, False) and weight.dtype == torch.bfloat16 and weight.is_contiguous() and weight.data_ptr() % 16 == 0):
         done = _native().gemm_rows64_sliced(x, packed, 0, *next_norm)
         if done is not None:
@@ -1374,7 +1375,7 @@ def gemm_rows32(x: torch.Tensor, packed: torch.Tensor, out_dtype: torch.dtype = 
 
 def _shared_x(x: torch.Tensor, packed: torch.Tensor, out_dtype: torch.dtype, glu: bool, squares: torch.Tensor | None, eps: float,
               unit: "tuple[str, float, float, float] | None", pack8_steps: int, few: int) -> "torch.Tensor | PackedRows8":
-    if unit is None or (glu and unit[0] in GLU_ACTIVATIONS):
+    if packed.dim() == 4 and (unit is None or (glu and unit[0] in GLU_ACTIVATIONS)):      # (of a copy of five dimensions the module makes `gemm_skinny8`)
         out = _native().gemm_rows64(x, packed, out_dtype is torch.float32, _unit_code(glu, unit), squares, eps,
                                     *((0.0, 0.0, 0.0) if unit is None else unit[1:]), few) if out_dtype in _DTYPE_CODE else None
         if out is not None:
@@ -1460,7 +1461,8 @@ def gemm_rows64_sliced(x: torch.Tensor, packed: torch.Tensor, slices: int, next_
     parts a second kernel adds in ascending order. With `next_norm` = (residual or None, weight of the
     norm that follows) the product is not stored: a `PreparedNorm` comes back."""
     residual, nw = (None, None) if next_norm is None else next_norm
-    done = _native().gemm_rows64_sliced(x, packed, slices, residual, nw) if next_norm is None or nw is not None else None
+    # (without slices the module makes `gemm_skinny`)
+    done = _native().gemm_rows64_sliced(x, packed, slices, residual, nw) if slices > 0 and (next_norm is None or nw is not None) else None
     if done is not None:
         return done if next_norm is None else PreparedNorm(*done)
     _gpu(x, packed)
@@ -1528,8 +1530,8 @@ def qkv_rope_store(x: torch.Tensor, weight: torch.Tensor, cos_sin: torch.Tensor 
     that copy."""
     if packed is not None and norm_weight is None and residual is None:
         q = None      # (the module's way: 4 µs on the host instead of 20, which bound prompts of 17 to 64 tokens)
-        if weight.dtype == torch.bfloat16 and weight.shape == ((num_heads + 2 * num_kv_heads) * head_dim, x.shape[-1]) and weight.is_contiguous() \
-                and weight.data_ptr() % 16 == 0 and packed.dim() == 4:
+        if weight.dtype == torch.bfloat16 and weight.device == x.device and weight.shape == ((num_heads + 2 * num_kv_heads) * head_dim, x.shape[-1]) \
+                and weight.is_contiguous() and weight.data_ptr() % 16 == 0 and packed.dim() == 4:
             q = _native().qkv_rope_store_sliced(x, packed, 0, cos_sin, positions, slots, k_cache, v_cache, num_heads, num_kv_heads, head_dim, eps, squares)
         if q is not None:
             return q, None
@@ -1607,9 +1609,9 @@ def qkv_rope_store_sliced(x: torch.Tensor, packed_rope: torch.Tensor, slices: in
     second kernel that adds the parts, rotates and writes the cache: q [tokens, nh, hd] comes back.
     `packed_rope` = pack_weight_rope(weight, head_dim). With `squares` (and `eps`) x is the operand of
     a `PreparedNorm` and the rows' scales multiply the finished sums."""
-    # (of a weight as it is the module makes `qkv_rope_store_whole`)
+    # (of a weight as it is the module makes `qkv_rope_store_whole`, without slices `qkv_rope_store`)
     q = _native().qkv_rope_store_sliced(x, packed_rope, slices, cos_sin, positions, slots, k_cache, v_cache, num_heads, num_kv_heads,
-                                        head_dim, eps, squares) if packed_rope.dim() == 4 else None
+                                        head_dim, eps, squares) if packed_rope.dim() == 4 and slices > 0 else None
     if q is not None:
         return q
     _gpu(x, packed_rope, cos_sin, positions, slots, k_cache, v_cache)
@@ -2541,7 +2543,7 @@ def stream_update_norm(x: torch.Tensor, a: torch.Tensor | None = None, b: "torch
     for each given weight norm(x) * weight of the updated rows comes back in `out_dtype` (both norms
     share the row's mean square). With `rows` (int32) nothing is updated and only those rows are
     normalised, in that order."""
-    if rows is None and bias is None and weights[0] is not None and weights[1] is None and out_dtype in _DTYPE_CODE:
+    if rows is None and bias is None and weights[0] is not None and weights[1] is None and out_dtype in _DTYPE_CODE and not isinstance(b, tuple):
         out = _native().stream_update_norm(x, a, b.operands() if isinstance(b, RowParts) else b, mult, weights[0], eps, _DTYPE_CODE[out_dtype])
         if out is not None:
             return out, None
@@ -3622,7 +3624,7 @@ def stream_post_norm(x: torch.Tensor, a: "torch.Tensor | RowParts | ExpertRows",
     """The float32 stream x [tokens, width] takes x += a / sqrt(mean(a^2) + post_eps) * post_weight * scale in place (a
     float32, what a branch has made, possibly in parts or as experts have left it; `scale` float32 [width] or None). With `out_dtype`, the updated rows come back in
     that type: normalised and times `weight` (x / sqrt(mean(x^2) + eps) * weight), or as they are if `weight` is None."""
-    if out_dtype in _DTYPE_CODE:
+    if out_dtype in _DTYPE_CODE and not isinstance(a, tuple):      # (a tuple is how the module is told of parts)
         out = _native().stream_post_norm(x, a.operands() if isinstance(a, (RowParts, ExpertRows)) else a, post_weight, scale, post_eps, weight, eps, _DTYPE_CODE[out_dtype])
         if out is not None:
             return out

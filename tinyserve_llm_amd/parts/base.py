@@ -109,6 +109,12 @@ class Part:
     # can be recorded into a HIP graph and replayed with new inputs.
     graph_safe = False
 
+    def __init_subclass__(cls, **options) -> None:
+        """`leaves_parts` (of mixers and feed-forwards) is said of a forward(): a class with one of its own says it anew, or is asked for no parts."""
+        super().__init_subclass__(**options)
+        if "forward" in vars(cls) and "leaves_parts" not in vars(cls) and hasattr(cls, "leaves_parts"):
+            cls.leaves_parts = False
+
     def param_specs(self) -> dict[str, ParamSpec]:
         return {}
 

@@ -61,3 +61,26 @@ def test_one_token_a_request_with_the_heads_norm_and_gate(requests, heads, dim, 
     o = hip.decay_scan(q, k, v, z, z_bias, other, cu, slots, heads, dim, vdim, **kw)
     want = hip.mlstm_finish(o, weight, gate, heads, vdim, 1e-6, out_dtype, silu_gate=True)
     assert torch.equal(got, want) and torch.equal(kept, other)
+
+
+@pytest.mark.parametrize("finish", [False, True])
+def test_a_portion_in_chunks_beside_requests_that_feed_nothing(finish):
+    """As many tokens as requests, and one the most of those that are not in chunks, but no step of a token a request. The bound: a number is a sum of some
+    dim + 64 products beside what the state's 32-bit numbers carry; the norm divides by a root that is no less than the eps's."""
+    from tests.test_gpu_fanotar import step_context
+    least, dim = hip.DECAY_CHUNKS_FROM, 64
+    lengths = [least, 1] + [0] * (least - 1)
+    tokens = requests = sum(lengths)
+    assert len(lengths) == requests
+    g = torch.Generator(device="cuda").manual_seed(3)
+    q, k, v, z, gate = (torch.randn(tokens, dim, generator=g, device="cuda") for _ in range(5))
+    z_bias, start = torch.randn(dim, generator=g, device="cuda"), torch.randn(requests, dim * dim, generator=g, device="cuda")
+    cu = torch.tensor([0, least] + [tokens] * requests, dtype=torch.int32, device="cuda")[:requests + 1]
+    slots, made = torch.arange(requests, dtype=torch.int32, device="cuda"), []
+    for ctx in (step_context([[0]] * requests, 4096, [0] * requests, lengths, slots=list(range(requests))), None):
+        state = start.clone()
+        o = hip.decay_scan(q, k, v, z, z_bias, state, cu, slots, 1, dim, dim, form="sigmoid_root", tau=16.0, q_scale=dim ** -0.5, longest=least, ctx=ctx,
+                           finish=(None, gate, 1.0, F32) if finish else None)
+        made.append((o, state))
+    for got, want in zip(*made):
+        torch.testing.assert_close(got, want, atol=4 * (dim + 64) * 2.0 ** -24 * float(want.abs().max()), rtol=1e-4)

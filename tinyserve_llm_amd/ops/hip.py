@@ -3550,7 +3550,8 @@ def decay_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, z: torch.Tenso
             return finished(out)
         at_most = DECAY_CHUNKS_FROM - 1
         longest = max(n for n in (b - a for a, b in zip(ctx.host_cu_seqlens, ctx.host_cu_seqlens[1:])) if n <= at_most)
-    if (longest == 1 and T == S and dim in DECAY_STEP_DIMS and vdim % 64 == 0 and v.stride(0) % 4 == 0 and state.stride(0) % 4 == 0
+    # (a token of every request: with portions in chunks the number of tokens does not say so, as a request may feed none)
+    if (longest == 1 and T == S and at_most == 0x7fffffff and dim in DECAY_STEP_DIMS and vdim % 64 == 0 and v.stride(0) % 4 == 0 and state.stride(0) % 4 == 0
             and v.data_ptr() % 16 == 0 and state.data_ptr() % 16 == 0):
         whole = finish is not None and _decay_step_finishes(*finish, T, heads, vdim)
         weight, gate, eps, out_dtype = finish if whole else (None, None, 0.0, torch.float32)

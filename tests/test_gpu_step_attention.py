@@ -75,3 +75,17 @@ def test_chunks_are_combined_whatever_the_ones_without_a_visible_key_hold(splits
         o[t, :, hidden], ml[t, :, hidden] = float("nan"), float("nan")
     got = hip.SplitAttention(o.cuda(), ml.cuda(), positions.cuda(), chunk, window).combined().view(tokens, heads, dim).cpu().double()
     assert bool(((got - want).abs() <= 2.0 ** -8 * want.abs() + (splits + 3) * 2.0 ** -22 * size).all())
+
+
+@pytest.mark.parametrize("splits", [1, 2, 4, 5, 8, 9, 12, 16])
+@pytest.mark.parametrize("heads,dim", [(3, 64), (5, 128), (2, 256), (2, 32)])
+@pytest.mark.parametrize("window", [0, 40, 200, -64])
+def test_few_chunks_have_the_bits_of_the_kernel_for_many(splits, heads, dim, window):
+    """The same chunks with more behind them that no token sees go to the kernel that takes any number of them."""
+    g, chunk = torch.Generator(device="cuda").manual_seed(splits + dim), 32
+    positions = torch.arange(0, splits * chunk, 13, dtype=I32, device="cuda")
+    tokens = len(positions)
+    o, ml = torch.randn(tokens, heads, splits, dim, generator=g, device="cuda"), torch.rand(tokens, heads, splits, 2, generator=g, device="cuda") * 9 + 0.1
+    beyond = lambda t: torch.cat([t, t.new_full((tokens, heads, 17 - splits, t.shape[3]), float("nan"))], 2)
+    few, many = (hip.SplitAttention(a, b, positions, chunk, window).combined() for a, b in ((o, ml), (beyond(o), beyond(ml))))
+    assert torch.equal(few, many)

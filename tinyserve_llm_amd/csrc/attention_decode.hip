@@ -73,39 +73,52 @@ attn_decode_combine_kernel(bf16_t* __restrict__ out, const float* __restrict__ p
   }
 }
 
+// What output dimension `d` has of chunks s0 to s1, up to MOST of them, whose (m, l) and parts are all asked for before the first is used (the last one's
+// again for those that there are fewer): the sums are those above, in their order.
+template <int MOST>
+static __device__ __forceinline__ float
+combine_few(const float* __restrict__ part_o, const float* __restrict__ part_ml, int64_t th, int s0, int s1, int num_splits, int hd, int d, float* sink) {
+  const int lane = threadIdx.x % TS_WAVE;
+  const float* const po = part_o + th * num_splits * hd + min(d, hd - 1);
+  float v[MOST];
+#pragma unroll
+  for (int k = 0; k < MOST; ++k) v[k] = po[min(s0 + k, s1) * hd];
+  const float* const ml = part_ml + 2 * (th * num_splits + min(s0 + lane, s1));
+  const bool visible = s0 + lane <= s1;
+  const float m = ml[0], l = ml[1];
+  const float M = wave_max(visible ? m : -INFINITY);
+  const float w = visible ? fast_exp2(m - M) : 0.f;
+  float L = wave_sum(visible ? l * w : 0.f);
+  if (sink) L += fast_exp2(*sink - M);
+  const float inv = 1.0f / L;
+  float acc = 0.f;
+#pragma unroll
+  for (int k = 0; k < MOST; ++k) {
+    const float ws = __shfl(w, k, TS_WAVE);
+    if (s0 + k <= s1) acc = fmaf(v[k], ws, acc);
+  }
+  return acc * inv;
+}
+
 // The same of up to MOST chunks, a thread an output dimension: the kernel is a chain of trips to memory (the position, the chunks' (m, l), their parts, which other
-// dies have just written), so all of them are asked for at once, also of chunks that turn out to hold no visible key, whose numbers are not used. The
-// sums are those above, in their order. us with the launch, chain and at once: 32
-// heads of 64, 8 tokens of 8 chunks 3.27 and 2.76, 20 of 12 4.59 and 3.24, 64 of 8 4.67 and 3.52, 300 of 8 9.87 and 6.97; 24 of 128, 13 tokens of 7 chunks 4.04 and 2.98.
+// dies have just written), so all that a token's visible chunks have left is asked for at once when its position is there, and no more of it (of up to
+// four of them with a quarter of the loads). us, chain and here, with every chunk visible and with one: 32 heads of 64, 8 tokens of 8 chunks 3.14 and 2.50, 2.62 and 2.16, 64 of 8
+// 4.95 and 4.32, 3.44 and 3.00, 64 of 12 5.88 and 5.16, 3.32 and 2.90, 300 of 8 13.3 and 11.2, 6.42 and 4.86; 32 of 128, 64 of 16 11.7 and 9.84, 3.70 and 3.08, 24 of 128, 8 of 8 2.98 and
+// 2.23, 2.70 and 2.16. (The position asked for along with the parts of every chunk there is: no faster with all visible, 10.5 with one of the 16.)
 template <int MOST>
 __global__ void __launch_bounds__(4 * TS_WAVE)
 attn_decode_combine_few_kernel(bf16_t* __restrict__ out, const float* __restrict__ part_o, const float* __restrict__ part_ml, const int32_t* __restrict__ positions,
                                int nh, int hd, int num_splits, int chunk, int window, int sink, const float* __restrict__ sinks, const float* __restrict__ gate,
                                int64_t gate_stride) {
-  const int t = blockIdx.x / nh, lane = threadIdx.x % TS_WAVE, d = threadIdx.x;
+  const int t = blockIdx.x / nh, d = threadIdx.x;
   const int64_t th = blockIdx.x;
-  const float* po = part_o + th * num_splits * hd + min(d, hd - 1);
-  float v[MOST];
-#pragma unroll
-  for (int s = 0; s < MOST; ++s) v[s] = po[min(s, num_splits - 1) * hd];
-  const float* const ml = part_ml + 2 * (th * num_splits + min(lane, num_splits - 1));
-  const float m = ml[0], l = ml[1];
   const int pos = positions[t], lo = ts_first_key(pos, window);
-  const int s0 = min(lo / chunk, num_splits - 1), s1 = min(pos / chunk, num_splits - 1);  // the last chunk is open-ended
-  const bool visible = lane >= s0 && lane <= s1;
-  const float M = wave_max(visible ? m : -INFINITY);
-  const float w = visible ? fast_exp2(m - M) : 0.f;
-  float L = wave_sum(visible ? l * w : 0.f);
+  const int s0 = min(lo / chunk, num_splits - 1), s1 = max(min(pos / chunk, num_splits - 1), s0);  // the last chunk is open-ended
   // the sink's score is 0, or its head's learned one
-  if (sink) L += fast_exp2((sinks ? sinks[blockIdx.x % nh] * 1.44269504088896340736f : 0.f) - M);
-  const float inv = 1.0f / L;
-  float acc = 0.f;
-#pragma unroll
-  for (int s = 0; s < MOST; ++s) {
-    const float ws = __shfl(w, s, TS_WAVE);
-    if (s >= s0 && s <= s1) acc = fmaf(v[s], ws, acc);
-  }
-  if (d < hd) out[th * hd + d] = f2bf(acc * inv * ts_out_gate(gate, gate_stride, t, blockIdx.x % nh, hd, d));
+  float score = sink && sinks ? sinks[blockIdx.x % nh] * 1.44269504088896340736f : 0.f;
+  const float y = s1 - s0 < 4 ? combine_few<4>(part_o, part_ml, th, s0, s1, num_splits, hd, d, sink ? &score : nullptr)
+                              : combine_few<MOST>(part_o, part_ml, th, s0, s1, num_splits, hd, d, sink ? &score : nullptr);
+  if (d < hd) out[th * hd + d] = f2bf(y * ts_out_gate(gate, gate_stride, t, blockIdx.x % nh, hd, d));
 }
 
 // The combining kernel alone: out [tokens, nh, hd] bfloat16 from the parts that ts_paged_attention_decode leaves

@@ -975,7 +975,15 @@ gemm_skinny8_kernel(const SkinnyArgs a) {
 // went at the rate the chip starts them, which follows its clock: 128,256 x 2,048 took 83 us in a decode step and 88 to 100 behind the products of a
 // prompt, whose power holds the clock down (timed apart 91.7 us, 79.1 here; 128,256 x 3,072 130.3 and 122.9). The sums are those of the kernel above, bit for bit. W as its packed copy, no norm behind.
 #define SK8_STAY_GRID 256       // one a compute unit, two tiles each under way (512 and more: 5 to 7 us slower)
-#define SK8_STAY_TILES 4096     // tiles from which they stay: with fewer a workgroup takes no more than two or three
+// From which sizes on they stay: a workgroup has 16 bytes of W under way for each k, too few for the memory's latency below 1,792, and has to take some 16 tiles for its start
+// and end to weigh little. One row, W from memory, us, a tile each and staying: k 256, 128,256 rows of W (left) 12.8 and 26.5; k 1,024 (left) 32,768 12.9 and 16.8,
+// 128,256 44.8 and 56.8; k 1,536 (left) 32,768 18.7 and 19.4, 65,536 35.0 both, 262,144 132 and 128, four rows 133 and 139; k 1,792 32,768 20.8 and 20.3, 65,536 39.4 and 36.2; k 2,048
+// 16,384 (left) 12.5 and 13.0, 24,576 (left) 18.2 and 17.8, 32,768 23.8 and 22.6, 65,536 44.0 and 41.1, 128,256 86.2 and 80.1; k 3,072 16,384 (left) 18.6 both, 32,768 33.7 and 32.3; k 3,584
+// 32,768 38.7 and 37.9; k 4,096 32,768 (left) 46.1 and 47.6, 65,536 (left) 90.6 and 88.2, four rows 87.8 and 90.2, 98,304 139.6 and 130.6, four rows 137.0 and 134.3.
+extern "C" int ts_skinny8_stays(int N, int K) {
+  const int steps = ts_skinny8_steps(K);
+  return K >= 1792 && (steps == 4 || steps == 8) && N / 8 >= (K <= 3584 ? 4096 : 12288);
+}
 template <int STEPS, typename OUT>
 __global__ void __launch_bounds__(512)
 gemm_skinny8_stay_kernel(const SkinnyArgs a) {
@@ -1042,7 +1050,7 @@ static int sk8_dispatch(const SkinnyArgs& a, hipStream_t stream) {
     }
   }
   if constexpr (!NEXT) {
-    if (a.packed && !a.ssq_parts && a.N / 8 >= SK8_STAY_TILES && steps <= 8) {
+    if (a.packed && !a.ssq_parts && ts_skinny8_stays(a.N, a.K)) {
       if (steps == 4) gemm_skinny8_stay_kernel<4, OUT><<<SK8_STAY_GRID, block, 0, stream>>>(a);
       else gemm_skinny8_stay_kernel<8, OUT><<<SK8_STAY_GRID, block, 0, stream>>>(a);
       return ts_check_launch();

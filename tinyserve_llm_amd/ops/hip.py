@@ -89,6 +89,7 @@ def _declare(lib: ctypes.CDLL) -> None:
         "ts_paged_attention_prefill": [p, p, p, p, p, p, p, p, i, i, i, i, i, i, i, i64, i64, i64, i64, i64, i64, i, f, i, i, i, i, i, p, p, i, p],
         "ts_gemm_skinny_bf16": [p, p, p, p, p, p, i, i, i, i64, i64, i64, f, i, i, i, i, p, i, p, p, p, p, p, i, f, f, f, p],
         "ts_gemm_skinny8_bf16": [p, p, p, i, i, i, i64, i64, i64, i, i, p, p, p, p, p, i, p, p, p, i, i, i, i, f, p],
+        "ts_skinny8_stays": [i, i],
         "ts_gemm_skinny8_act_bf16": [p, p, p, i, i, i, i64, i64, i64, i, i, p, i, p],
         "ts_gemm_slices_bf16": [p, p, p, p, p, i, i, i, i64, i64, i, i, i, p, p, f, p],
         "ts_gemm_whole_bf16": [i, p, p, p, p, i, i, i64, i64, i, i, i, p],
@@ -1042,6 +1043,12 @@ def skinny8_steps(k: int) -> int:
     return 16 if k % 1024 == 0 and k // 1024 <= 16 else 0
 
 
+@functools.lru_cache(maxsize=256)
+def skinny8_stays(n: int, k: int) -> bool:
+    """Whether the 8-row form's workgroups stay for a weight [n, k] whose copy it reads: those that may cap their sums."""
+    return bool(library().ts_skinny8_stays(n, k))
+
+
 def skinny8_takes(rows: int, n: int, k: int) -> bool:
     """Whether `linear_bf16` gives the product to the 8-row form. Every workgroup reads all rows of x
     for its 8 rows of W, twice as much of x per byte of W as the 16-row form: with 8 rows of x and a
@@ -1117,13 +1124,14 @@ def pack_weight8(weight: torch.Tensor) -> torch.Tensor:
 
 
 def gemm_skinny8(x: "torch.Tensor | PackedRows8 | SplitAttention", weight: torch.Tensor, out_dtype: torch.dtype = torch.bfloat16,
-                 packed8: torch.Tensor | None = None, next_norm=None) -> "torch.Tensor | PreparedNorm":
+                 packed8: torch.Tensor | None = None, next_norm=None, cap: float = 0.0) -> "torch.Tensor | PreparedNorm":
     """bfloat16 x [M <= 8, K] · weight [N, K]^T by the weight-streaming kernel's 8-row form (a matrix
     instruction multiplies 8 rows of W by 8 rows of x over 64 k; a workgroup owns 8 rows of W).
     x may come as a `PackedRows8` made for this K. With `packed8` (= pack_weight8(weight)) the kernel
     reads that copy. With `next_norm` = (residual or None, weight of the norm that follows) the product
     is not stored: a `PreparedNorm` comes back. x may also be a `SplitAttention` that `split_attention_fuses`
-    allows: the kernel then adds up the chunks' parts on its way in (bfloat16 out)."""
+    allows: the kernel then adds up the chunks' parts on its way in (bfloat16 out). `cap` > 0 (32-bit, where `skinny8_stays`): cap tanh(. / cap)
+    of the sums, as `soft_cap` makes it."""
     x_packed = isinstance(x, PackedRows8)
     split = x if isinstance(x, SplitAttention) else None
     xt = x.data if x_packed else x.parts if split is not None else x
@@ -1133,7 +1141,7 @@ def gemm_skinny8(x: "torch.Tensor | PackedRows8 | SplitAttention", weight: torch
         steps = skinny8_steps(k)
         if (steps and n % 8 == 0 and packed8.shape == (n // 8, k // (64 * steps), steps, 64, 8) and x.shape[1] == k and weight.dtype == torch.bfloat16
                 and weight.is_contiguous() and weight.data_ptr() % 16 == 0 and packed8.data_ptr() % 16 == 0):
-            y = _native().gemm_rows64(x, packed8, out_dtype is torch.float32, 0, None, 0.0, 0.0, 0.0, 0.0)
+            y = _native().gemm_rows64(x, packed8, out_dtype is torch.float32, 0, None, 0.0, cap, 0.0, 0.0)
             if y is not None:
                 return y
     _gpu(xt, weight, packed8)
@@ -1168,6 +1176,8 @@ def gemm_skinny8(x: "torch.Tensor | PackedRows8 | SplitAttention", weight: torch
         _need(packed8.dtype == torch.bfloat16 and packed8.shape == (-(-N // 8), K // (64 * steps), steps, 64, 8)
               and packed8.is_contiguous() and packed8.data_ptr() % 16 == 0 and N % 8 == 0,
               lambda: f"the packed copy does not belong to a weight of {N} x {K}")
+    _need(cap == 0.0 or (cap > 0 and next_norm is None and out_dtype == torch.float32 and packed8 is not None and skinny8_stays(N, K)),
+          "a cap comes with 32-bit sums of the workgroups that stay")
     if next_norm is not None:
         _need(out_dtype == torch.bfloat16, "a prepared norm comes with bfloat16")
         prepared, residual, nw = _next_norm_outputs(xt, N, -(-N // 8), next_norm, rows=M)
@@ -1179,7 +1189,7 @@ def gemm_skinny8(x: "torch.Tensor | PackedRows8 | SplitAttention", weight: torch
     out = torch.empty((M, N), dtype=out_dtype, device=xt.device)
     _run("gemm_skinny8", library().ts_gemm_skinny8_bf16(
         _ptr(out), x_arg, _ptr(weight if packed8 is None else packed8), M, N, K, ldx, weight.stride(0),
-        out.stride(0), _code(out_dtype), int(packed8 is not None), None, None, None, None, None, int(x_packed), *comb, 0.0, _stream()))
+        out.stride(0), _code(out_dtype), int(packed8 is not None), None, None, None, None, None, int(x_packed), *comb, float(cap), _stream()))
     return out
 
 
@@ -1355,29 +1365,31 @@ def rows64_few(rows: int, n: int, k: int, glu: bool = False) -> bool:
 
 def gemm_rows64(x: torch.Tensor, packed: torch.Tensor, out_dtype: torch.dtype = torch.bfloat16, *,
                 glu: bool = False, squares: torch.Tensor | None = None, eps: float = 0.0,
-                unit: "tuple[str, float, float, float] | None" = None) -> torch.Tensor:
+                unit: "tuple[str, float, float, float] | None" = None, cap: float = 0.0) -> torch.Tensor:
     """bfloat16 e(x [M <= 128, K] · W [N, K]^T) for a wide W given as `packed` = pack_weight(W), by the
     kernel that shares x among 64 rows of W through LDS (gemm_rows64.hip). With `glu`, W holds gate
     rows then up rows and the result is silu(gate) * up, [M, N / 2]. With `squares` (and `eps`) x is
     the operand of a `PreparedNorm` and the rows' scales multiply the finished sums. `unit` (with `glu`, a plain
-    x): (form, limit, slope, up_shift) of the unit of `capped_glu` in silu's place."""
-    return _shared_x(x, packed, out_dtype, glu, squares, eps, unit, 0, 0)
+    x): (form, limit, slope, up_shift) of the unit of `capped_glu` in silu's place. `cap` > 0 (32-bit, without the gate): cap tanh(. / cap) of the sums, as
+    `soft_cap` makes it."""
+    return _shared_x(x, packed, out_dtype, glu, squares, eps, unit, 0, 0, cap)
 
 
 def gemm_rows32(x: torch.Tensor, packed: torch.Tensor, out_dtype: torch.dtype = torch.bfloat16, *,
                 glu: bool = False, squares: torch.Tensor | None = None, eps: float = 0.0,
-                unit: "tuple[str, float, float, float] | None" = None, pack8_steps: int = 0) -> "torch.Tensor | PackedRows8":
+                unit: "tuple[str, float, float, float] | None" = None, pack8_steps: int = 0, cap: float = 0.0) -> "torch.Tensor | PackedRows8":
     """`gemm_rows64` of up to 32 rows whose sums have the bits of `gemm_skinny`'s (`rows64_few` says where it is the faster way). With `pack8_steps`
     (and `glu`, up to 8 rows) the gated product comes back as a `PackedRows8` for a reader of that many steps."""
     _need(x.dim() == 2 and x.shape[0] < ROWS64_MIN_ROWS, lambda: f"gemm_rows32 takes up to {ROWS64_MIN_ROWS - 1} rows, not {tuple(x.shape)}")
-    return _shared_x(x, packed, out_dtype, glu, squares, eps, unit, pack8_steps, pack8_steps or 1)
+    return _shared_x(x, packed, out_dtype, glu, squares, eps, unit, pack8_steps, pack8_steps or 1, cap)
 
 
 def _shared_x(x: torch.Tensor, packed: torch.Tensor, out_dtype: torch.dtype, glu: bool, squares: torch.Tensor | None, eps: float,
-              unit: "tuple[str, float, float, float] | None", pack8_steps: int, few: int) -> "torch.Tensor | PackedRows8":
+              unit: "tuple[str, float, float, float] | None", pack8_steps: int, few: int, cap: float) -> "torch.Tensor | PackedRows8":
+    _need(cap == 0.0 or (cap > 0 and not glu and out_dtype == torch.float32), "a cap comes with 32-bit sums without the gate")
     if packed.dim() == 4 and (unit is None or (glu and unit[0] in GLU_ACTIVATIONS)):      # (of a copy of five dimensions the module makes `gemm_skinny8`)
         out = _native().gemm_rows64(x, packed, out_dtype is torch.float32, _unit_code(glu, unit), squares, eps,
-                                    *((0.0, 0.0, 0.0) if unit is None else unit[1:]), few) if out_dtype in _DTYPE_CODE else None
+                                    *((cap, 0.0, 0.0) if unit is None else unit[1:]), few) if out_dtype in _DTYPE_CODE else None
         if out is not None:
             return PackedRows8(out, x.shape[0], packed.shape[0] * 8, pack8_steps) if pack8_steps else out
     _gpu(x, packed)
@@ -1402,7 +1414,7 @@ def _shared_x(x: torch.Tensor, packed: torch.Tensor, out_dtype: torch.dtype, glu
     _run("gemm_rows64", library().ts_gemm_rows64_bf16(
         _ptr(out), _ptr(x), _ptr(packed), M, N, K, x.stride(0), N // 2 if pack8_steps else out.stride(0), _unit_code(glu, unit),
         int(out_dtype == torch.float32), _ptr(squares), 0 if squares is None else squares.shape[1], float(eps),
-        *((0.0, 0.0, 0.0) if unit is None else map(float, unit[1:])), int(few), _stream()))
+        *((float(cap), 0.0, 0.0) if unit is None else map(float, unit[1:])), int(few), _stream()))
     return PackedRows8(out, M, N // 2, pack8_steps) if pack8_steps else out
 
 
@@ -2351,10 +2363,9 @@ def capped_product(x: torch.Tensor, weight: torch.Tensor, packed: StreamingCopie
     rows, (n, k) = x.shape[0], weight.shape
     few = rows64_few(rows, n, k)
     if packed.by16 is not None and packed.by16.shape[0] * 16 == n and (few or rows64_takes(rows, n, k)):
-        return _native().gemm_rows64(x, packed.by16, True, 0, None, 0.0, cap, 0.0, 0.0, int(few))
-    steps = skinny8_steps(k)
-    if packed.by8 is not None and not few and skinny8_takes(rows, n, k) and steps and packed.by8.shape == (n // 8, k // (64 * steps), steps, 64, 8) and n % 8 == 0:
-        return _native().gemm_rows64(x, packed.by8, True, 0, None, 0.0, cap, 0.0, 0.0)
+        return (gemm_rows32 if few else gemm_rows64)(x, packed.by16, torch.float32, cap=cap)
+    if packed.by8 is not None and not few and n % 8 == 0 and skinny8_takes(rows, n, k) and skinny8_stays(n, k):
+        return gemm_skinny8(x, weight, torch.float32, packed.by8, cap=cap)
     return None
 
 

@@ -254,3 +254,20 @@ def test_calls_go_to_the_current_stream_and_can_be_recorded():
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("place", [0, 1])
+def test_a_projection_into_a_norm_has_one_route(place, monkeypatch):
+    """`linear` with a request asks `hip.linear_into_norm` and nothing beside it: what that leaves (here a weight that begins between two 16-byte pieces, and
+    nothing is launched) is the general way's."""
+    from tinyserve_llm_amd.parts.linear import DeferredNorm, NormRequest, linear, streaming_copy
+    whole = torch.zeros(2048 * 8192 + 8, dtype=torch.bfloat16, device="cuda")
+    weight = whole[place:place + 2048 * 8192].view(2048, 8192)
+    packed = streaming_copy(whole[:2048 * 8192].view(2048, 8192))
+    x, then = torch.zeros(48, 8192, dtype=torch.bfloat16, device="cuda"), NormRequest(torch.ones(2048, dtype=torch.bfloat16, device="cuda"), 1e-5, None)
+    asked, made = [], torch.zeros(48, 2048, dtype=torch.bfloat16, device="cuda")
+    prepared = hip.PreparedNorm(made, made, torch.ones(48, 1, device="cuda"))
+    for name, answer in (("gemm_rows64_sliced", prepared), ("linear_through_norm", None), ("linear_bf16", made)):
+        monkeypatch.setattr(hip, name, lambda *args, _name=name, _answer=answer, **options: asked.append(_name) or _answer)
+    assert isinstance(linear(x, weight, packed=packed, then=then), DeferredNorm)
+    assert asked == (["linear_through_norm", "linear_bf16"] if place else ["gemm_rows64_sliced"])

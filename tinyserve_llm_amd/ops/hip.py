@@ -1473,10 +1473,10 @@ def gemm_rows64_sliced(x: torch.Tensor, packed: torch.Tensor, slices: int, next_
     parts a second kernel adds in ascending order. With `next_norm` = (residual or None, weight of the
     norm that follows) the product is not stored: a `PreparedNorm` comes back."""
     residual, nw = (None, None) if next_norm is None else next_norm
-    # (without slices the module makes `gemm_skinny`)
-    done = _native().gemm_rows64_sliced(x, packed, slices, residual, nw) if slices > 0 and (next_norm is None or nw is not None) else None
-    if done is not None:
-        return done if next_norm is None else PreparedNorm(*done)
+    if slices > 0 and (next_norm is None or nw is not None):      # (without slices the module makes `gemm_skinny`)
+        done = _native().gemm_rows64_sliced(x, packed, slices, residual, nw)
+        if done is not None:
+            return done if next_norm is None else PreparedNorm(*done)
     _gpu(x, packed)
     _need(x.dtype == torch.bfloat16 and packed.dtype == torch.bfloat16 and x.dim() == 2 and packed.dim() == 4
           and packed.shape[2:] == (64, 8) and packed.is_contiguous(), "gemm_rows64_sliced takes bfloat16 x [M, K] and pack_weight(W)")
@@ -1503,7 +1503,10 @@ def gemm_rows64_sliced(x: torch.Tensor, packed: torch.Tensor, slices: int, next_
 def _dense_rows(x: torch.Tensor) -> bool:
     """Whether the rows of a matrix are dense and begin at multiples of 16 bytes (they may lie further
     apart than they are long)."""
-    return x.dim() == 2 and x.stride(1) == 1 and x.stride(0) % 8 == 0 and x.stride(0) >= x.shape[1]
+    if x.dim() != 2:
+        return False
+    apart, step = x.stride()
+    return step == 1 and apart % 8 == 0 and apart >= x.shape[1]
 
 
 def qkv_rope_max_rows(k: int, norm: bool = False) -> int:
@@ -2227,7 +2230,9 @@ def _next_norm_route(x: "torch.Tensor | PackedRows8", weight: torch.Tensor, pack
     if not (x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and x.is_cuda and x.dim() == 2 and weight.dim() == 2
             and _dense_rows(x) and weight.is_contiguous() and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0):
         return 0
-    rows, (n, k) = x.shape[0], weight.shape
+    (rows, width), (n, k) = x.shape, weight.shape
+    if width != k:
+        return 0
     return _sliced_serves(rows, n, k, packed) or (-1 if skinny8_takes(rows, n, k) or _skinny_serves(rows, n, k) else 0)
 
 
@@ -2240,7 +2245,7 @@ def linear_into_norm(x: "torch.Tensor | PackedRows8", weight: torch.Tensor, pack
     """x · weight^T finished into `next_norm` = (residual or None, weight of the norm that follows) by the kernel that
     `linear_bf16` gives such a product to; None where that kernel leaves no prepared norm."""
     route = _next_norm_route(x, weight, packed)
-    if route > 0 and x.shape[1] == weight.shape[1]:
+    if route > 0:
         return gemm_rows64_sliced(x, packed.by16, route, next_norm=next_norm)
     return linear_bf16(x, weight, torch.bfloat16, packed, next_norm=next_norm) if route else None
 

@@ -66,7 +66,7 @@ class NormRequest:
 def _streams(x: torch.Tensor, weight: torch.Tensor, dense_rows: bool = False) -> bool:
     """Whether the weight-streaming kernels take these operands; `dense_rows`: x need not be
     contiguous as long as its rows are (a prepared norm's operand, whose rows may lie further apart)."""
-    rows_ok = (x.stride(1) == 1 and x.stride(0) % 8 == 0 and x.stride(0) >= x.shape[1]) if dense_rows and x.dim() == 2 else x.is_contiguous()
+    rows_ok = hip._dense_rows(x) if dense_rows and x.dim() == 2 else x.is_contiguous()
     return (x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and x.is_cuda and rows_ok
             and weight.is_contiguous() and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0)
 
@@ -145,6 +145,26 @@ def few_rows_unit(x: torch.Tensor, weight: torch.Tensor, packed: hip.StreamingCo
     return None
 
 
+def _into_norm(x: "torch.Tensor | DeferredNorm | hip.PackedRows8", weight: torch.Tensor, out_dtype: torch.dtype | None, glu: bool,
+               packed: hip.StreamingCopies | None, then: NormRequest) -> DeferredNorm:
+    """`linear` with a request of the norm that follows."""
+    if glu:
+        raise ValueError("a gated projection does not finish into a norm")
+    residual = then.residual()
+    if isinstance(x, DeferredNorm):
+        x = x.materialize()
+    if (out_dtype in (None, torch.bfloat16) and then.weight.dtype == torch.bfloat16
+            and (residual is None or (residual.is_contiguous() and residual.dtype == torch.bfloat16))):
+        prepared = hip.linear_into_norm(x, weight, packed, (residual, then.weight))
+        if prepared is not None:
+            return DeferredNorm(None, None, then.weight, then.eps, prepared)
+        if x.is_cuda:
+            done = hip.linear_through_norm(x, weight, packed, residual, then.weight, then.eps)
+            if done is not None:
+                return DeferredNorm(None, None, then.weight, then.eps, done=done)
+    return DeferredNorm(linear(x, weight, out_dtype, packed=packed), residual, then.weight, then.eps)
+
+
 def linear(x: "torch.Tensor | DeferredNorm | hip.PackedRows8 | hip.SplitAttention", weight: torch.Tensor, out_dtype: torch.dtype | None = None,
            glu: bool = False, packed: hip.StreamingCopies | None = None,
            then: NormRequest | None = None, feeds: torch.Tensor | None = None) -> "torch.Tensor | DeferredNorm | hip.PackedRows8":
@@ -157,14 +177,8 @@ def linear(x: "torch.Tensor | DeferredNorm | hip.PackedRows8 | hip.SplitAttentio
     handed to `linear` with that weight and to nothing else. x may be a `hip.SplitAttention` (an attention output
     still in its chunks' parts): the 8-row form adds the parts up on its way in where it can, the combining
     kernel does otherwise."""
-    if type(x) is torch.Tensor and then is not None and packed is not None and packed.by16 is not None and out_dtype is None and not glu and x.dim() == 2:
-        # the commonest way of a step of a few dozen rows (with the module's ways into the cache and into the norm of up to 32 rows a prompt over 12
-        # layers, which the host bounds: 32 tokens 1118 -> 733 µs, 48 947 -> 719; 90, the kernels' 828, 856 -> 828)
-        slices = hip._sliced_route(x.shape[0], *weight.shape) if x.is_cuda and weight.dtype == torch.bfloat16 and weight.is_contiguous() else 0
-        residual = then.residual() if slices else None
-        if (slices and x.dtype == torch.bfloat16 and hip._dense_rows(x) and x.data_ptr() % 16 == 0 and then.weight.dtype == torch.bfloat16
-                and (residual is None or (residual.is_contiguous() and residual.dtype == torch.bfloat16))):
-            return DeferredNorm(None, None, then.weight, then.eps, hip.gemm_rows64_sliced(x, packed.by16, slices, next_norm=(residual, then.weight)))
+    if then is not None and type(x) is torch.Tensor:      # (first: a step of a few dozen rows waits for the host)
+        return _into_norm(x, weight, out_dtype, glu, packed, then)
     if isinstance(x, hip.SplitAttention):
         residual = then.residual() if then is not None else None
         if (not glu and out_dtype in (None, torch.bfloat16) and hip.split_attention_fuses(x.shape[0], weight)
@@ -181,21 +195,7 @@ def linear(x: "torch.Tensor | DeferredNorm | hip.PackedRows8 | hip.SplitAttentio
     if isinstance(x, hip.PackedRows8) and then is None:
         return hip.linear_bf16(x, weight, out_dtype or torch.bfloat16, packed)
     if then is not None:
-        if glu:
-            raise ValueError("a gated projection does not finish into a norm")
-        residual = then.residual()
-        if isinstance(x, DeferredNorm):
-            x = x.materialize()
-        if (out_dtype in (None, torch.bfloat16) and then.weight.dtype == torch.bfloat16
-                and (residual is None or (residual.is_contiguous() and residual.dtype == torch.bfloat16))):
-            prepared = hip.linear_into_norm(x, weight, packed, (residual, then.weight))
-            if prepared is not None:
-                return DeferredNorm(None, None, then.weight, then.eps, prepared)
-            if x.is_cuda:
-                done = hip.linear_through_norm(x, weight, packed, residual, then.weight, then.eps)
-                if done is not None:
-                    return DeferredNorm(None, None, then.weight, then.eps, done=done)
-        return DeferredNorm(linear(x, weight, out_dtype, packed=packed), residual, then.weight, then.eps)
+        return _into_norm(x, weight, out_dtype, glu, packed, then)
     by16 = None if packed is None else packed.by16
     rows = x.rows if isinstance(x, DeferredNorm) else x.shape[0]
     pack8 = _pack8(rows, weight.shape[0], feeds) if glu else 0

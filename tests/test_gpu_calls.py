@@ -256,6 +256,7 @@ def test_calls_go_to_the_current_stream_and_can_be_recorded():
         assert torch.equal(got, want)
 
 
+@pytest.mark.gpu
 @pytest.mark.parametrize("place", [0, 1])
 def test_a_projection_into_a_norm_has_one_route(place, monkeypatch):
     """`linear` with a request asks `hip.linear_into_norm` and nothing beside it: what that leaves (here a weight that begins between two 16-byte pieces, and

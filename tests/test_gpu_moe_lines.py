@@ -1,5 +1,5 @@
 """The experts' products of narrow tiles by whole lines (`moe_gemm_lines_kernel`): reductions of one stage to many, columns that end inside a
-workgroup's, tiles of 1 to 16 rows, against 64 bits, and a row's bits whatever its batch."""
+workgroup's, tiles of 1 to 16 rows, against 64 bits, a row's bits whatever its batch, and those of the kernel for other reductions."""
 
 from __future__ import annotations
 
@@ -11,6 +11,10 @@ from tinyserve_llm_amd.ops import hip
 BF, F32 = torch.bfloat16, torch.float32
 pytestmark = pytest.mark.gpu
 E = 5
+
+
+def present(experts):
+    return [p for p, e in enumerate(experts) if e < E]
 
 
 @pytest.mark.parametrize("once", [False, True])
@@ -39,6 +43,11 @@ def test_products_by_lines(monkeypatch, tokens, n, k, once):
         want = w[e, :n].double() @ rows[p].double()
         torch.testing.assert_close(plain[p].double(), want, rtol=1e-5, atol=2e-6 * k ** 0.5)
         torch.testing.assert_close(squared[p].double(), want.clamp(min=0.0) ** 2, rtol=2.0 ** -8, atol=1e-4)
+    # a step of zeros behind each quarter of the reduction makes it the other kernel's, whose sums are the same, bit for bit
+    spread = lambda t: torch.nn.functional.pad(t.reshape(*t.shape[:-1], 4, k // 4), (0, 32)).flatten(-2).contiguous()
+    assert (k + 128) % 256
+    assert torch.equal(gated[present(flat)], hip.moe_gemm(spread(x), spread(w), grouped, BF, per_token=True, glu=(5.0, 1.0, 0.5))[present(flat)])
+    assert torch.equal(plain[present(flat)], hip.moe_gemm(spread(rows), spread(w[:, :n]), grouped, F32, per_token=False)[present(flat)])
     # a token by itself: the same bits
     alone = hip.moe_group(ids[-1:].contiguous(), E)
     last = hip.moe_gemm(x[-1:].contiguous(), w, alone, BF, per_token=True, glu=(5.0, 1.0, 0.5))

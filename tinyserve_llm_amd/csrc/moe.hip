@@ -458,7 +458,8 @@ moe_gemm_mfma_kernel(TO* __restrict__ out, const bf16_t* __restrict__ x, const b
   }
 }
 
-// Tiles of 16 rows, for steps of few tokens, where the experts' matrices are streamed once and nothing else counts:
+// Tiles of 16 rows, for steps of few tokens, where the experts' matrices are streamed once and nothing else counts, over reductions that are no multiple of 256 (the
+// kernel below takes those; the figures here are from when this one took all):
 // a workgroup takes a tile's rows by 16 columns (with GLU: 16 gate and 16 up columns), and its four waves take a
 // quarter of K each, eight k-steps' loads in flight at a time, so that a step with one token still has a thousand
 // waves asking for memory. A row's loads go out side by side (two take a cache line): the two products of 32 experts of 3,072 and 1,536 over four choices each took
@@ -540,7 +541,7 @@ moe_gemm_stream_kernel(TO* __restrict__ out, const bf16_t* __restrict__ x, const
   moe_store4(orow + c0, y, N - c0);
 }
 
-// The same sums, bit for bit, for reductions of whole lines (K a multiple of 256): a load of the kernel above takes 64 bytes of each of 16 rows, half a line,
+// The same sums, bit for bit (a quarter's steps in turn, then the quarters), for reductions of whole lines (K a multiple of 256): a load of the kernel above takes 64 bytes of each of 16 rows, half a line,
 // and past the caches the other half is a line fetched again. Here 64 of k at a time go from memory straight into LDS, 8 rows of 128 bytes a load, pieces turned
 // by (row / 2) % 8 against bank conflicts; a wave has MOE_LINES of them there, its own, and waits for nobody. Without the gate a workgroup takes 32 columns.
 // Both products of 16 experts over 2,048, 2 x 1,024 and back over 1,024, past the caches, the kernel above and here: 4 tokens of four choices 36.6 and 20.8 us, 16

@@ -3041,10 +3041,12 @@ def moe_tile_rows(pairs: int, experts: int, dtype: torch.dtype, k_sizes: "tuple[
 
 
 def moe_weights_once(pairs: int, experts: int) -> bool:
-    """Whether the experts' matrices go by the caches where tiles have 16 rows: of more than a pair an expert and fewer than a tile. Past the caches the products
-    take longer by themselves (`moe_gemm_stream_kernel`), and a step is the shorter where other layers' weights stay in them: two layers of 16 experts, four choices each, beside
-    two without, µs a step through the caches and past them, 4 rows 600 and 607, 5 rows 590 and 582, 16 rows 669 and 647, 48 rows 850 and 821, 56 rows 869 and 844, 64 rows 926 and
-    928, 96 rows 1,116 and 1,134; eight layers of 16 experts of half the width, 64 rows (tokens a second) 49,060 and 47,310."""
+    """Whether the experts' matrices go by the caches where tiles have 16 rows: of more than a pair an expert and fewer than a tile. Other layers' weights stay in the
+    caches then. Two layers of 16 experts, four choices each, beside two without, µs a step through the caches and past them, by the kernel of reductions of whole 256s
+    (`moe_gemm_lines_kernel`, which is the faster past them by itself too): 4 rows (left) 517 and 511, 5 rows 535 and 508, 16 rows 618 and 585, 48 rows 783 and 738, 56 rows 811 and 774, 64 rows
+    (left) 847 and 826, 80 rows (left) 995 and 985. The lines are those of the kernel for other reductions (`moe_gemm_stream_kernel`), which takes longer past the caches by itself: the same
+    steps by that kernel, 4 rows 600 and 607, 5 rows 590 and 582, 16 rows 669 and 647, 48 rows 850 and 821, 64 rows 926 and 928, 96 rows 1,116 and 1,134; eight layers of 16 experts of half the
+    width, 64 rows (tokens a second) 49,060 and 47,310."""
     return experts < pairs < MOE_TILE_ROWS * experts
 
 

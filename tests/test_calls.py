@@ -140,6 +140,27 @@ def test_a_step_whose_decoding_part_has_run_is_not_made_again(stub, softcap):
     answer(prefill, OK)
 
 
+@pytest.mark.parametrize("softcap", [0.0, 20.0])
+def test_a_step_of_decoding_tokens_and_prompts_is_one_launch_or_two(stub, softcap):
+    module, answer, called = stub
+    general = "_general" if softcap else ""
+    both, decode, prefill = "ts_paged_attention_step", f"ts_paged_attention_decode{general}", f"ts_paged_attention_prefill{general}"
+    change = lambda **other: [other.get(f"a{i}", a) for i, a in enumerate(step(2, softcap))]
+    wide = dict(a16=128, a17=4)      # (chunks for as many waves as the prompts' tiles have)
+    assert module.attention_step(*change(**wide)) is not None and called() == [both]
+    for rc in (BAD_DTYPE, BAD_SHAPE, TOO_LARGE):
+        answer(both, rc)
+        assert module.attention_step(*change(**wide)) is not None and called() == [both, decode, prefill]
+    answer(both, LAUNCH_FAILED)
+    with pytest.raises(hip.KernelError, match=f"paged_attention_step: {re.escape(hip._ERRORS[LAUNCH_FAILED])}"):
+        module.attention_step(*change(**wide))
+    assert called() == [both]
+    answer(both, OK)
+    # fewer waves than a tile's, tiles of four rows of 16 a wave, prompts in parts
+    for other in (dict(a16=64, a17=2), dict(wide, a18=128), dict(wide, a20=2, a21=64)):
+        assert module.attention_step(*change(**other)) is not None and called() == [decode, prefill]
+
+
 def test_a_stream_is_updated_by_one_launch(stub, monkeypatch):
     module, answer, called = stub
     monkeypatch.setattr(hip, "_native", lambda: module)

@@ -557,10 +557,13 @@ extern "C" int ts_paged_attention_step(void* out, float* part_o, float* part_ml,
   attn_step_kernel<HH, RR, WW, ON, GG, NC><<<(unsigned)all, WW * TS_WAVE, 0, stream>>>(d, tiles, num_tiles, group, dies_per_group, heads_per_group, (int)(8 * turns), decode_waves, num_tokens)
 #define TS_STEP_N(HH, RR, WW, ON, GG) if (once) { TS_STEP(HH, RR, WW, ON, GG, true); } else { TS_STEP(HH, RR, WW, ON, GG, false); }
 #define TS_STEP_O(HH, RR, WW, GG) if (chunk == 32 * decode_waves) { TS_STEP_N(HH, RR, WW, true, GG) } else { TS_STEP_N(HH, RR, WW, false, GG) }
-#define TS_STEP_W(HH, GG) \
-  if (rt == 2) { TS_STEP_O(HH, 2, 4, GG) } else if (waves == 4) { TS_STEP_O(HH, 1, 4, GG) } else { TS_STEP_O(HH, 1, 8, GG) }
-  if (hd == 128) { TS_STEP_W(128, false) } else if (general) { TS_STEP_W(64, true) } else { TS_STEP_W(64, false) }
+#define TS_STEP_1(HH, RR, WW, GG) TS_STEP_N(HH, RR, WW, true, GG)
+#define TS_STEP_W(HH, GG, EIGHT) \
+  if (rt == 2) { TS_STEP_O(HH, 2, 4, GG) } else if (waves == 4) { TS_STEP_O(HH, 1, 4, GG) } else { EIGHT(HH, 1, 8, GG) }
+  // (eight waves of wide heads have a single step each: DEC_WAVES_FOR)
+  if (hd == 128) { TS_STEP_W(128, false, TS_STEP_1) } else if (general) { TS_STEP_W(64, true, TS_STEP_O) } else { TS_STEP_W(64, false, TS_STEP_O) }
 #undef TS_STEP_W
+#undef TS_STEP_1
 #undef TS_STEP_O
 #undef TS_STEP_N
 #undef TS_STEP

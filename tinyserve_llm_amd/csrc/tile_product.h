@@ -15,6 +15,8 @@
 // 85.6 and 73.6; 128 rows, 1,000 x 6,144 (192 and 256) 33.6 and 30.7, but in one round only (1,200 x 8,192, 320 and 430, 55.5 and 56.4). A round more: 1,024 x
 // 12,352 (196 and 260) 54.7 and 77.4. In two slices with the norm, 192 rows, 1,514 x 3,072 over 8,192 (192 and 256) 86.6 and
 // 84.1, over 3,072 51.5 and 46.4; 256 rows, 2,048 x 3,072 over 8,192 (192 and 256) 106.0 and 101.6. (224 columns in tiles of 256 rows: 54.2 where 256 take 54.0.)
+// The plans that choose between tiles, and between these and the library (whole_plan, slices_plan, group_plan of ops/hip.py), cost 256 columns: where tiles go narrow a product
+// takes 2 to 15 % less than they count on, so they leave gains there that they do not see. (qkv_rope_whole_plan knows its narrow tile.)
 static inline bool tiles_go_narrow(int64_t wide, int64_t narrow, int bm) {
   const int64_t rounds = (wide + COMPUTE_UNITS - 1) / COMPUTE_UNITS;
   return narrow <= rounds * COMPUTE_UNITS && (bm > 128 || rounds == 1);

@@ -1916,7 +1916,7 @@ def whole_plan(rows: int, n: int, k: int, ending: str) -> int | None:
     estimates promised 9 % on average at 103 such points, and 61 were no faster (library and here: 12,288 x 2,048, 1,150 rows 53.4 and 59.3, 8,192 x 2,048, 2,048 rows 52.5 and 56.8, 12,288 x 4,096, 800 rows 70.9 and 81.5), where ragged columns
     cost the library a tenth. Of 1,154 points within these limits that are not for slices the rule takes 242, at 0.92 of the library's time in bfloat16 and 0.94 in 32 bits; 8 of them are slower by more than 2 %: bfloat16
     7,168 x 2,048 and x 4,096, 2,048 rows, 52.9 and 56.6, 86.3 and 92.3, 32 bits 9,280 x 2,048 and x 4,096, 1,280 rows, 51.0 and 56.1, 89.9 and 98.9, and four by up to 5 %. Beyond 12,800 columns (14,336 and 16,384 measured) the estimates promise a gain at 45
-    points, and 21 of these are. Library and here: bfloat16, n 12,352, k 2,048, 999 rows 58.4 and 50.6; 32 bits, the same
+    points, and 21 of these are. The points are from before tiles 192 columns wide (`tiles_go_narrow` of tile_product.h), which the estimates do not know. Library and here: bfloat16, n 12,352, k 2,048, 999 rows 58.4 and 50.6; 32 bits, the same
     62.7 and 55.3, n 10,304, k 2,048, 2,048 rows 98.2 and 88.4, n 2,048, k 2,048, 720 rows 14.8 and 13.9, 257 rows (left to the library) 11.6 and 13.0."""
     if (not WHOLE_MIN_ROWS <= rows <= WHOLE_MAX_ROWS or not WHOLE_MIN_WIDTH <= n <= WHOLE_MAX_WIDTH or n % 8 or k % 64 or k < WHOLE_MIN_K):
         return None

@@ -255,7 +255,8 @@ def test_the_general_functions_of_few_rows_take_what_they_say(stub, monkeypatch)
         assert called()[-1] == launcher
     for bad in (lambda: hip.gemm_rows64(x, p8), lambda: hip.gemm_rows32(x, p8), lambda: hip.gemm_rows64_sliced(x, p16, 0, next_norm=(None, bf(64))),
                 lambda: hip.qkv_rope_store_sliced(x, p16q, 0, *rope), lambda: hip.gemm_skinny8(x, away(w), BF, p8), lambda: hip.gemm_skinny8(x, bf(64), BF, p8),
-                lambda: hip.gemm_skinny(x, away(w), **into), lambda: hip.gemm_skinny(x, w, unit=("sigmoid", 0.0, 1.0, 0.0), **into),
+                lambda: hip.gemm_skinny8(x, w, F32, p8, cap=-1.0), lambda: hip.gemm_skinny8(x, w, F32, p8, cap=float("nan")), lambda: hip.gemm_rows64(x, p16, F32, cap=-1.0),
+                lambda: hip.gemm_rows64(x, p16, cap=1.0), lambda: hip.gemm_skinny(x, away(w), **into), lambda: hip.gemm_skinny(x, w, unit=("sigmoid", 0.0, 1.0, 0.0), **into),
                 lambda: hip.qkv_rope_store(x, away(w512), *rope, packed=p16q),
                 lambda: hip.stream_update_norm(torch.zeros(3, 64), None, (torch.zeros(2, 3, 64),), weights=(bf(64), None), out_dtype=BF),
                 lambda: hip.stream_post_norm(torch.zeros(3, 64), (torch.zeros(2, 3, 64),), torch.zeros(64), None, 1e-6, out_dtype=BF)):

@@ -1136,7 +1136,7 @@ def gemm_skinny8(x: "torch.Tensor | PackedRows8 | SplitAttention", weight: torch
     split = x if isinstance(x, SplitAttention) else None
     xt = x.data if x_packed else x.parts if split is not None else x
     if (packed8 is not None and next_norm is None and xt is x and x.dim() == 2 and weight.dim() == 2 and weight.device == x.device
-            and x.shape[0] <= SKINNY8_MAX_ROWS and out_dtype in (torch.bfloat16, torch.float32)):
+            and x.shape[0] <= SKINNY8_MAX_ROWS and out_dtype in (torch.bfloat16, torch.float32) and cap >= 0.0):
         n, k = weight.shape
         steps = skinny8_steps(k)
         if (steps and n % 8 == 0 and packed8.shape == (n // 8, k // (64 * steps), steps, 64, 8) and x.shape[1] == k and weight.dtype == torch.bfloat16
